@@ -119,8 +119,9 @@ __global__ __launch_bounds__(THREADS) void rms_fwd_bf16_kernel(bf16_t *__restric
     const int blk = xcd_remap(blockIdx.x, nblk);
     const int slab = blk / strips, strip = blk - slab * strips;
     const int lc = threadIdx.x % LPR, row0 = threadIdx.x / LPR;
-    const int col = (strip * LPR + lc) * VEC;
-    const bool col_ok = col < S;
+    const LaneCols mine = lane_cols<VEC>((strip * LPR + lc) * VEC, S);
+    const int col = mine.col;
+    const bool col_ok = mine.ok;
     const size_t base = (size_t)slab * C * S + col;
     float acc[1][VEC];
 #pragma unroll
@@ -198,8 +199,9 @@ __global__ __launch_bounds__(THREADS) void rms_bwd_bf16_kernel(bf16_t *dx, float
     const int blk = xcd_remap(blockIdx.x, nblk);
     const int slab = blk / strips, strip = blk - slab * strips;
     const int lc = threadIdx.x % LPR, row0 = threadIdx.x / LPR;
-    const int col = (strip * LPR + lc) * VEC;
-    const bool col_ok = col < S;
+    const LaneCols mine = lane_cols<VEC>((strip * LPR + lc) * VEC, S);
+    const int col = mine.col;
+    const bool col_ok = mine.ok;
     const size_t base = (size_t)slab * C * S + col;
     float *part = dw_part + (size_t)blk * C;
     float acc[2][VEC];
@@ -209,12 +211,11 @@ __global__ __launch_bounds__(THREADS) void rms_bwd_bf16_kernel(bf16_t *dx, float
     auto row_out = [&](int c, const float (&xr)[VEC], const float (&dyr)[VEC], float wc, const float (&rr)[VEC],
                        const float (&dotn)[VEC]) {
         float o[VEC];
-        float p = 0.f;
+        float p = own_sum<VEC>(mine, [&](int j) { return (dyr[j] * xr[j]) * rr[j]; });
 #pragma unroll
         for (int j = 0; j < VEC; j++) {
             if (variant == 0) o[j] = ((dyr[j] - xr[j] * dotn[j]) * rr[j]) * wc;
             else o[j] = (dyr[j] * wc) * rr[j] - (xr[j] * dotn[j]) * rr[j];
-            p += (dyr[j] * xr[j]) * rr[j];
         }
         if (col_ok) {
             // res != NULL: the backward residual rides along, dx = rmsnorm_bwd + res, and dx2 = alpha2 * dx if asked
@@ -333,7 +334,7 @@ __global__ __launch_bounds__(BT) void rope_bf16_kernel(bf16_t *q_out, bf16_t *k_
                                                        const float *__restrict__ sin_t, float sgn, size_t total) {
     const size_t idx = (size_t)blockIdx.x * BT + threadIdx.x;
     if (idx >= total) return;
-    const int cols = S / VEC;
+    const int cols = (S + VEC - 1) / VEC;
     const int cg = (int)(idx % cols);
     size_t pr = idx / cols;
     const int half = hd >> 1;
@@ -345,6 +346,15 @@ __global__ __launch_bounds__(BT) void rope_bf16_kernel(bf16_t *q_out, bf16_t *k_
     const size_t row = (pr / half) * hd + 2 * i;
     const int s = cg * VEC;
     const size_t o0 = row * S + s;
+    if (VEC > 1 && s + VEC > S) {        // the short last group of a row of any length
+        for (int j = 0; j < S - s; j++) {
+            const float a = bf_to_f(in[o0 + j]), b = bf_to_f(in[o0 + S + j]);
+            const float c = cos_t[(size_t)i * S + s + j], sj = sin_t[(size_t)i * S + s + j] * sgn;
+            out[o0 + j] = (bf16_t)f_to_bf(a * c - b * sj);
+            out[o0 + S + j] = (bf16_t)f_to_bf(a * sj + b * c);
+        }
+        return;
+    }
     float v0[VEC], v1[VEC], c[VEC], sn[VEC], r0[VEC], r1[VEC];
     ldb<VEC, true>(v0, in + o0);
     ldb<VEC, true>(v1, in + o0 + S);
@@ -375,8 +385,9 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_fwd_bf16_kernel(
     if (blk >= nq) { blk -= nq; in = k; out = k_out; w = wk; }
     const int slab = blk / strips, strip = blk - slab * strips;
     const int lc = threadIdx.x % LPR, p0 = threadIdx.x / LPR;
-    const int col = (strip * LPR + lc) * VEC;
-    const bool col_ok = col < S;
+    const LaneCols mine = lane_cols<VEC>((strip * LPR + lc) * VEC, S);
+    const int col = mine.col;
+    const bool col_ok = mine.ok;
     const int half = hd >> 1;
     const size_t base = (size_t)slab * hd * S + col;
     typename RawT<VEC>::type r0[CAP], r1[CAP];
@@ -446,8 +457,9 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_bwd_bf16_kernel(
     if (blk >= nq) { blk -= nq; gin = dk_out; xin = k; out = dk; w = wk; }
     const int slab = blk / strips, strip = blk - slab * strips;
     const int lc = threadIdx.x % LPR, p0 = threadIdx.x / LPR;
-    const int col = (strip * LPR + lc) * VEC;
-    const bool col_ok = col < S;
+    const LaneCols mine = lane_cols<VEC>((strip * LPR + lc) * VEC, S);
+    const int col = mine.col;
+    const bool col_ok = mine.ok;
     const int half = hd >> 1;
     const size_t base = (size_t)slab * hd * S + col;
     typename RawT<VEC>::type rx0[CAP], rx1[CAP], rg0[CAP], rg1[CAP];
@@ -519,7 +531,8 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_bwd_bf16_kernel(
             unpack<VEC>(x0, rx0[kk]);
             unpack<VEC>(x1, rx1[kk]);
             unrotate(kk, rp, d0, d1);
-            float s0 = 0.f, s1 = 0.f;
+            float s0 = own_sum<VEC>(mine, [&](int j) { return (d0[j] * x0[j]) * rr[j]; });
+            float s1 = own_sum<VEC>(mine, [&](int j) { return (d1[j] * x1[j]) * rr[j]; });
 #pragma unroll
             for (int j = 0; j < VEC; j++) {
                 if (variant == 0) {
@@ -529,8 +542,6 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_bwd_bf16_kernel(
                     o0[j] = (d0[j] * w0[kk]) * rr[j] - (x0[j] * dotn[j]) * rr[j];
                     o1[j] = (d1[j] * w1[kk]) * rr[j] - (x1[j] * dotn[j]) * rr[j];
                 }
-                s0 += (d0[j] * x0[j]) * rr[j];
-                s1 += (d1[j] * x1[j]) * rr[j];
             }
             if (col_ok) {
                 stb<VEC>(out + base + (size_t)(2 * rp) * S, o0);
@@ -551,20 +562,23 @@ struct QkBf {
 };
 
 // Widest strip whose row pairs fit the (packed) register tile: 16 lanes x 8 columns = 256-byte row segments first;
-// 64-byte segments run at little more than half the rate.  One-column lanes (ragged S, unaligned pointers) hold
-// at most four pairs.
-bool pick_qk_bf(int hd, bool vec_ok, bool backward, QkBf &cfg) {
+// 64-byte segments run at little more than half the rate.  One-column lanes (rows of fewer than eight columns, in-place
+// calls whose short last group of columns would be shared by two workgroups) hold at most four pairs.
+bool pick_qk_bf(int hd, int S, bool in_place, bool backward, QkBf &cfg) {
     const int half = hd / 2;
-    if (!vec_ok) {
-        cfg = QkBf{1, 64, 1024, 4};
-        return half <= 64;
+    auto fits = [&](int lpr, int threads, int cap) {
+        cfg = QkBf{8, lpr, threads, cap};
+        return (threads / lpr) * cap >= half && (!in_place || tail_in_strip(S, lpr * 8, 8));
+    };
+    if (S >= 8) {
+        const int thr = backward ? 512 : 256;
+        for (int lpr : {16, 8, 4})
+            for (int cap : {1, 2, 4})
+                if (fits(lpr, thr, cap)) return true;
+        if (fits(4, 1024, 2)) return true;
     }
-    const int thr = backward ? 512 : 256;
-    for (int lpr : {16, 8, 4})
-        for (int cap : {1, 2, 4})
-            if ((thr / lpr) * cap >= half) { cfg = QkBf{8, lpr, thr, cap}; return true; }
-    if (512 >= half) { cfg = QkBf{8, 4, 1024, 2}; return true; }
-    return false;
+    cfg = QkBf{1, 64, 1024, 4};
+    return half <= 64;
 }
 
 #define QKBF_CASE(KERNEL, V, L, T, CP, grid, ...)                                                                    \
@@ -598,11 +612,17 @@ int qk_shape(const char *who, int heads, int kv_heads, int hd, int S, int batch)
 struct BfCfg {
     int vec, lpr, threads, cap;
 };
+// One column per lane: rows of fewer than eight columns, and in-place calls whose short last group of columns would be
+// shared by two workgroups (lane_cols in tile.h).
+constexpr BfCfg BF_SCALAR = {1, 64, 256, 0};
+BfCfg bf_tile_for_alias(const BfCfg &c, bool in_place, int S) {
+    return in_place && !tail_in_strip(S, c.lpr * c.vec, c.vec) ? BF_SCALAR : c;
+}
 
 // 8-column lanes when the rows allow 128-bit accesses; rows in (packed) registers when one workgroup can hold
 // them, else two sweeps.  The rms_lpr / rms_threads knobs override the strip width and workgroup size.
 BfCfg pick_bf(int C, bool vec_ok, int S, int batch) {
-    if (!vec_ok) return BfCfg{1, 64, 256, 0};
+    if (!vec_ok) return BF_SCALAR;
     // 128-byte strips (8 lanes x 8 columns) once they still give every compute unit a workgroup
     const long strips8 = (long)ceil_div((size_t)S, 64) * batch;
     int lpr = g_ctx.rms_lpr == 8 || (!g_ctx.rms_lpr && strips8 >= (g_ctx.num_cu > 0 ? g_ctx.num_cu : 256)) ? 8 : 4;
@@ -741,7 +761,7 @@ MI355_API int mi355_rmsnorm_fwd_bf16_dev(uint16_t *y, const uint16_t *x, const f
     if (!mi355_ready("rmsnorm_fwd_bf16")) return -1;
     if (!y || !x || !w) return mi355_fail("rmsnorm_fwd_bf16: NULL pointer");
     if (C <= 0 || S <= 0 || batch <= 0) return mi355_fail("rmsnorm_fwd_bf16: bad shape C=%d S=%d batch=%d", C, S, batch);
-    const bool vec_ok = S % 8 == 0 && aligned16(x) && aligned16(y);
+    const bool vec_ok = S >= 8;
     // tall shapes whose strips would leave compute units idle split the channel axis over clusters of workgroups,
     // as the fp32 op does (norm_cluster.h); in place the single-workgroup tile is used
     const ClusterPlan cp = y == x ? NO_CLUSTER : plan_cluster_bf(C, S, batch, vec_ok);
@@ -754,7 +774,7 @@ MI355_API int mi355_rmsnorm_fwd_bf16_dev(uint16_t *y, const uint16_t *x, const f
         LAUNCH_OK("rmsnorm_fwd_bf16");
         return 0;
     }
-    const BfCfg cfg = pick_bf(C, vec_ok, S, batch);
+    const BfCfg cfg = bf_tile_for_alias(pick_bf(C, vec_ok, S, batch), y == x, S);
     const int strips = (int)ceil_div((size_t)S, (size_t)cfg.lpr * cfg.vec);
     const int nblk = strips * batch;
     BF_DISPATCH(rms_fwd_bf16_kernel, cfg, nblk, y, x, w, C, S, strips, nblk, eps, 1.0f / (float)C);
@@ -769,7 +789,7 @@ MI355_API int mi355_rmsnorm_bwd_bf16_dev(uint16_t *dx, float *dw, const uint16_t
     if (C <= 0 || S <= 0 || batch <= 0) return mi355_fail("rmsnorm_bwd_bf16: bad shape C=%d S=%d batch=%d", C, S, batch);
     if (variant != 0 && variant != 1) return mi355_fail("rmsnorm_bwd_bf16: variant must be 0 or 1");
     if (dx == x) return mi355_fail("rmsnorm_bwd_bf16: dx must not alias x (dx may alias dy)");      // as the fp32 op
-    const bool vec_ok = S % 8 == 0 && aligned16(x) && aligned16(dy) && aligned16(dx);
+    const bool vec_ok = S >= 8;
     const ClusterPlan cp = dx == dy ? NO_CLUSTER : plan_cluster_bf(C, S, batch, vec_ok);
     if (cp.csplit) {
         if (!mi355_exchange(&g_bf_cluster_ws)) return -1;
@@ -784,7 +804,7 @@ MI355_API int mi355_rmsnorm_bwd_bf16_dev(uint16_t *dx, float *dw, const uint16_t
         if (mi355_dw_submit(dw, part, nrows, C)) return -1;
         return mi355_dw_op_end();
     }
-    const BfCfg cfg = pick_bf(C, vec_ok, S, batch);
+    const BfCfg cfg = bf_tile_for_alias(pick_bf(C, vec_ok, S, batch), dx == dy, S);
     const int strips = (int)ceil_div((size_t)S, (size_t)cfg.lpr * cfg.vec);
     const int nblk = strips * batch;
     float *part = mi355_dw_partials((size_t)nblk * C, dw, nullptr);
@@ -806,7 +826,7 @@ MI355_API int mi355_residual_rmsnorm_fwd_bf16_dev(uint16_t *y, uint16_t *yn, con
     if (C <= 0 || S <= 0 || batch <= 0)
         return mi355_fail("residual_rmsnorm_fwd_bf16: bad shape C=%d S=%d batch=%d", C, S, batch);
     if (yn == y || yn == a || yn == b) return mi355_fail("residual_rmsnorm_fwd_bf16: yn must not alias y, a or b");
-    const bool vec_ok = S % 8 == 0 && aligned16(y) && aligned16(yn) && aligned16(a) && aligned16(b);
+    const bool vec_ok = S >= 8;
     const ClusterPlan cp = (y == a || y == b) ? NO_CLUSTER : plan_cluster_bf(C, S, batch, vec_ok);
     if (cp.csplit) {
         if (!mi355_exchange(&g_bf_cluster_ws)) return -1;
@@ -838,9 +858,9 @@ MI355_API int mi355_rmsnorm_bwd_residual_bf16_dev(uint16_t *dx, uint16_t *dx_sca
     if (dx_scaled && (dx_scaled == dx || dx_scaled == dy || dx_scaled == x || dx_scaled == res))
         return mi355_fail("rmsnorm_bwd_residual_bf16: dx_scaled must not alias another operand");
     if (dx == x) return mi355_fail("rmsnorm_bwd_residual_bf16: dx must not alias x (dx may alias res or dy)");
-    const bool vec_ok = S % 8 == 0 && aligned16(x) && aligned16(dy) && aligned16(dx) && aligned16(res) &&
-                        (!dx_scaled || aligned16(dx_scaled));
-    const ClusterPlan cp = dx == dy ? NO_CLUSTER : plan_cluster_bf(C, S, batch, vec_ok);
+    const bool vec_ok = S >= 8;
+    const bool apart = dx != res || tail_in_strip(S, CL_LPR * StoreBf16::VEC, StoreBf16::VEC);
+    const ClusterPlan cp = dx == dy || !apart ? NO_CLUSTER : plan_cluster_bf(C, S, batch, vec_ok);
     if (cp.csplit) {
         if (!mi355_exchange(&g_bf_cluster_ws)) return -1;
         const int nrows = cp.nblk / cp.csplit;
@@ -857,7 +877,7 @@ MI355_API int mi355_rmsnorm_bwd_residual_bf16_dev(uint16_t *dx, uint16_t *dx_sca
         if (mi355_dw_submit(dw, part, nrows, C)) return -1;
         return mi355_dw_op_end();
     }
-    const BfCfg cfg = pick_bf(C, vec_ok, S, batch);
+    const BfCfg cfg = bf_tile_for_alias(pick_bf(C, vec_ok, S, batch), dx == dy || dx == res, S);
     const int strips = (int)ceil_div((size_t)S, (size_t)cfg.lpr * cfg.vec);
     const int nblk = strips * batch;
     float *part = mi355_dw_partials((size_t)nblk * C, dw, nullptr);
@@ -877,13 +897,9 @@ MI355_API int mi355_rope_bf16_dev(uint16_t *q_out, uint16_t *k_out, const uint16
     if (!cos_dev || !sin_dev || (heads > 0 && (!q_out || !q_in)) || (kv_heads > 0 && (!k_out || !k_in)))
         return mi355_fail("rope_bf16: NULL pointer");
     if (dir != 1 && dir != -1) return mi355_fail("rope_bf16: dir must be +1 or -1");
-    const bool vec = S % 8 == 0 && aligned16(cos_dev) && aligned16(sin_dev) &&
-                     (heads == 0 || (aligned16(q_in) && aligned16(q_out))) &&
-                     (kv_heads == 0 || (aligned16(k_in) && aligned16(k_out)));
     const size_t pair_rows = (size_t)batch * (heads + kv_heads) * (hd / 2);
-    const size_t total = pair_rows * (size_t)(vec ? S / 8 : S);
-    if (vec) hipLaunchKernelGGL(rope_bf16_kernel<8>, dim3(blocks_for(total)), dim3(BT), 0, g_ctx.stream, q_out, k_out, q_in, k_in, heads, kv_heads, hd, S, batch, cos_dev, sin_dev, (float)dir, total);
-    else hipLaunchKernelGGL(rope_bf16_kernel<1>, dim3(blocks_for(total)), dim3(BT), 0, g_ctx.stream, q_out, k_out, q_in, k_in, heads, kv_heads, hd, S, batch, cos_dev, sin_dev, (float)dir, total);
+    const size_t total = pair_rows * ceil_div((size_t)S, 8);
+    hipLaunchKernelGGL(rope_bf16_kernel<8>, dim3(blocks_for(total)), dim3(BT), 0, g_ctx.stream, q_out, k_out, q_in, k_in, heads, kv_heads, hd, S, batch, cos_dev, sin_dev, (float)dir, total);
     LAUNCH_OK("rope_bf16");
     return 0;
 }
@@ -895,11 +911,8 @@ MI355_API int mi355_qknorm_rope_fwd_bf16_dev(uint16_t *q_out, uint16_t *k_out, c
     if (qk_shape("qknorm_rope_fwd_bf16", heads, kv_heads, hd, S, batch)) return -1;
     if (!cos_dev || !sin_dev || (heads > 0 && (!q_out || !q || !wq)) || (kv_heads > 0 && (!k_out || !k || !wk)))
         return mi355_fail("qknorm_rope_fwd_bf16: NULL pointer");
-    const bool vec_ok = S % 8 == 0 && aligned16(cos_dev) && aligned16(sin_dev) &&
-                        (heads == 0 || (aligned16(q) && aligned16(q_out))) &&
-                        (kv_heads == 0 || (aligned16(k) && aligned16(k_out)));
     QkBf cfg;
-    if (!pick_qk_bf(hd, vec_ok, false, cfg))
+    if (!pick_qk_bf(hd, S, q_out == q || k_out == k, false, cfg))
         return mi355_fail("qknorm_rope_fwd_bf16: head size %d does not fit the register tile for this layout", hd);
     const int strips = (int)ceil_div((size_t)S, (size_t)cfg.lpr * cfg.vec);
     const int nq = batch * heads * strips, nk = batch * kv_heads * strips;
@@ -920,11 +933,8 @@ MI355_API int mi355_qknorm_rope_bwd_bf16_dev(uint16_t *dq, uint16_t *dk, float *
     if (!cos_dev || !sin_dev || (heads > 0 && (!dq || !dwq || !dq_out || !q || !wq)) ||
         (kv_heads > 0 && (!dk || !dwk || !dk_out || !k || !wk)))
         return mi355_fail("qknorm_rope_bwd_bf16: NULL pointer");
-    const bool vec_ok = S % 8 == 0 && aligned16(cos_dev) && aligned16(sin_dev) &&
-                        (heads == 0 || (aligned16(q) && aligned16(dq) && aligned16(dq_out))) &&
-                        (kv_heads == 0 || (aligned16(k) && aligned16(dk) && aligned16(dk_out)));
     QkBf cfg;
-    if (!pick_qk_bf(hd, vec_ok, true, cfg))
+    if (!pick_qk_bf(hd, S, dq == dq_out || dk == dk_out, true, cfg))
         return mi355_fail("qknorm_rope_bwd_bf16: head size %d does not fit the register tile for this layout", hd);
     const int strips = (int)ceil_div((size_t)S, (size_t)cfg.lpr * cfg.vec);
     const int nq = batch * heads * strips, nk = batch * kv_heads * strips;

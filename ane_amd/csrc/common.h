@@ -13,6 +13,10 @@
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v2f __attribute__((ext_vector_type(2)));
 typedef int v4i __attribute__((ext_vector_type(4)));
+// the same 16 bytes at any 4-byte boundary: global memory accesses need no more (the instruction is the one of the
+// aligned access), so rows of any length and tensors at any element keep 128-bit accesses.  Not for LDS, where an
+// unaligned 16-byte access is taken apart.
+typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4)));
 
 // -------------------------------------------------------------------------------------------
 // Host-side context (context.hip)
@@ -95,14 +99,14 @@ __device__ __forceinline__ int xcd_remap(int bid, int n) {
     return xcd * q + (xcd < r ? xcd : r) + idx;
 }
 
-__device__ __forceinline__ v4f ld4(const float *p) { return *reinterpret_cast<const v4f *>(p); }
-__device__ __forceinline__ void st4(float *p, v4f v) { *reinterpret_cast<v4f *>(p) = v; }
+__device__ __forceinline__ v4f ld4(const float *p) { return *reinterpret_cast<const v4f_any *>(p); }
+__device__ __forceinline__ void st4(float *p, v4f v) { *reinterpret_cast<v4f_any *>(p) = v; }
 // streaming store: output is not re-read by this kernel, keep it out of the way of the inputs
 __device__ __forceinline__ void st4_nt(float *p, v4f v) {
-    __builtin_nontemporal_store(v, reinterpret_cast<v4f *>(p));
+    __builtin_nontemporal_store(v, reinterpret_cast<v4f_any *>(p));
 }
 __device__ __forceinline__ v4f ld4_nt(const float *p) {
-    return __builtin_nontemporal_load(reinterpret_cast<const v4f *>(p));
+    return __builtin_nontemporal_load(reinterpret_cast<const v4f_any *>(p));
 }
 
 // Value of lane (l ^ M) of a wave64, through the cheapest path measured for each distance: a DPP quad permute inside

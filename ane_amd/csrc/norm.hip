@@ -30,8 +30,9 @@ __global__ __launch_bounds__(THREADS) void rms_fwd_kernel(float *__restrict__ y,
     const int blk = xcd_remap(blockIdx.x, nblk);
     const int slab = blk / strips, strip = blk - slab * strips;
     const int lc = threadIdx.x % LPR, row0 = threadIdx.x / LPR;
-    const int col = strip * W + lc * VEC;
-    const bool col_ok = col < S;
+    const LaneCols mine = lane_cols<VEC>(strip * W + lc * VEC, S);
+    const int col = mine.col;
+    const bool col_ok = mine.ok;
     const size_t base = (size_t)slab * C * S + col;
     const float *xs = x + base;
     float *ys = y + base;
@@ -114,8 +115,9 @@ __device__ __forceinline__ void rms_bwd_body(float *dx, float *__restrict__ dw_p
     const int blk = xcd_remap(blockIdx.x, nblk);
     const int slab = blk / strips, strip = blk - slab * strips;
     const int lc = threadIdx.x % LPR, row0 = threadIdx.x / LPR;
-    const int col = strip * W + lc * VEC;
-    const bool col_ok = col < S;
+    const LaneCols mine = lane_cols<VEC>(strip * W + lc * VEC, S);
+    const int col = mine.col;
+    const bool col_ok = mine.ok;
     const size_t base = (size_t)slab * C * S + col;
     const float *xs = x + base, *dys = dy + base;
     float *dxs = dx + base;
@@ -137,12 +139,11 @@ __device__ __forceinline__ void rms_bwd_body(float *dx, float *__restrict__ dw_p
     auto row_out = [&](int c, const float (&xr)[VEC], const float (&dyr)[VEC], float wc, const float (&rr)[VEC],
                        const float (&dotn)[VEC], const float (&rs)[VEC]) {
         float o[VEC];
-        float p = 0.f;
+        float p = own_sum<VEC>(mine, [&](int j) { return (dyr[j] * xr[j]) * rr[j]; });
 #pragma unroll
         for (int j = 0; j < VEC; j++) {
             if (variant == 0) o[j] = ((dyr[j] - xr[j] * dotn[j]) * rr[j]) * wc;
             else o[j] = (dyr[j] * wc) * rr[j] - (xr[j] * dotn[j]) * rr[j];
-            p += (dyr[j] * xr[j]) * rr[j];
             if constexpr (RES) o[j] = o[j] + rs[j];
         }
         if (col_ok) stv_nt<VEC>(dxs + (size_t)c * S, o);
@@ -262,8 +263,9 @@ __global__ __launch_bounds__(THREADS) void res_rms_fwd_kernel(float *y, float *_
     const int blk = xcd_remap(blockIdx.x, nblk);
     const int slab = blk / strips, strip = blk - slab * strips;
     const int lc = threadIdx.x % LPR, row0 = threadIdx.x / LPR;
-    const int col = strip * W + lc * VEC;
-    const bool col_ok = col < S;
+    const LaneCols mine = lane_cols<VEC>(strip * W + lc * VEC, S);
+    const int col = mine.col;
+    const bool col_ok = mine.ok;
     const size_t base = (size_t)slab * C * S + col;
     float acc[1][VEC];
 #pragma unroll
@@ -342,6 +344,12 @@ __global__ __launch_bounds__(THREADS) void res_rms_fwd_kernel(float *y, float *_
 struct NormCfg {
     int vec, lpr, threads, cap;
 };
+// One column per lane: rows of fewer than four columns, and in-place calls whose short last group of columns would be
+// shared by two workgroups (lane_cols in tile.h).
+constexpr NormCfg SCALAR_TILE = {1, 64, 256, 0};
+NormCfg tile_for_alias(const NormCfg &c, bool in_place, int S) {
+    return in_place && !tail_in_strip(S, c.lpr * c.vec, c.vec) ? SCALAR_TILE : c;
+}
 
 // The tiles that are instantiated (NORM_DISPATCH below has one case per entry): vec*1000000 + lpr*10000 + (threads/256)*100 + cap.
 constexpr int NORM_KEYS[] = {1640100, 4160100, 4160108, 4160116, 4160200, 4160208, 4160216, 4160400, 4160408,
@@ -359,7 +367,7 @@ bool norm_tile_exists(const NormCfg &c) {
 NormCfg pick_cfg(int C, int S, int batch, bool vec_ok, int max_cap, int max_cap_1024, int lpr_knob, int thr_knob,
                  bool backward) {
     NormCfg best{};
-    if (!vec_ok) return NormCfg{1, 64, 256, 0};
+    if (!vec_ok) return SCALAR_TILE;
     if (!lpr_knob && !thr_knob && C >= 512) {
         // Tall tensors, measured on MI355X at C=1024 and 16x256 columns with operands cold in HBM: forward, 64-byte strips in registers of a 16-wave workgroup
         // 9.6 us; backward, the single-pass register tile with 8 waves 13.9 us, with 4 waves 16.3 us, a two-sweep
@@ -521,7 +529,8 @@ void launch_bwd_cluster(const ClusterPlan &cp, float *dx, float *part, const flo
 // Host-only: which tile an entry point would run for a shape, and whether that tile exists.
 MI355_API int mi355_rmsnorm_tile(int op, int C, int S, int batch, int aligned, int *tile5) {
     if (op < 0 || op > 2 || C <= 0 || S <= 0 || batch <= 0) return mi355_fail("rmsnorm_tile: bad arguments");
-    const bool vec_ok = aligned && S % 4 == 0;
+    (void)aligned;                           // 128-bit accesses work at any float
+    const bool vec_ok = S >= 4;
     // the single-workgroup tile is also what an in-place call of a clustered shape runs: it has to exist either way
     const NormCfg cfg = plan_tile(op, C, S, batch, vec_ok);
     if (!norm_tile_exists(cfg)) return mi355_fail("rmsnorm: no kernel for tile key %d", norm_key(cfg));
@@ -540,7 +549,7 @@ MI355_API int mi355_rmsnorm_fwd_dev(float *y, const float *x, const float *w, in
     if (!mi355_ready("rmsnorm_fwd")) return -1;
     if (!y || !x || !w) return mi355_fail("rmsnorm_fwd: NULL pointer");
     if (C <= 0 || S <= 0 || batch <= 0) return mi355_fail("rmsnorm_fwd: bad shape C=%d S=%d batch=%d", C, S, batch);
-    const bool vec_ok = (S % 4 == 0) && aligned16(x) && aligned16(y);
+    const bool vec_ok = S >= 4;
     // in place the single-workgroup tile is used, for the reason given in mi355_rmsnorm_bwd_dev
     const ClusterPlan cp = y == x ? NO_CLUSTER : plan_cluster(C, S, batch, vec_ok, 8);
     if (cp.csplit) {
@@ -549,7 +558,7 @@ MI355_API int mi355_rmsnorm_fwd_dev(float *y, const float *x, const float *w, in
         LAUNCH_OK("rmsnorm_fwd");
         return 0;
     }
-    NormCfg cfg = plan_tile(0, C, S, batch, vec_ok);
+    const NormCfg cfg = tile_for_alias(plan_tile(0, C, S, batch, vec_ok), y == x, S);
     NORM_DISPATCH(launch_fwd, cfg, y, x, w, C, S, batch, eps);
     LAUNCH_OK("rmsnorm_fwd");
     return 0;
@@ -562,7 +571,7 @@ MI355_API int mi355_rmsnorm_bwd_dev(float *dx, float *dw, const float *dy, const
     if (C <= 0 || S <= 0 || batch <= 0) return mi355_fail("rmsnorm_bwd: bad shape C=%d S=%d batch=%d", C, S, batch);
     if (variant != 0 && variant != 1) return mi355_fail("rmsnorm_bwd: variant must be 0 or 1");
     if (dx == x) return mi355_fail("rmsnorm_bwd: dx must not alias x (dx may alias dy)");
-    const bool vec_ok = (S % 4 == 0) && aligned16(x) && aligned16(dy) && aligned16(dx);
+    const bool vec_ok = S >= 4;
     // in place on dy the single-workgroup tile is used: a cluster member that has to recompute another member's
     // sums (its bounded wait expired) would read rows that their owner has already overwritten
     const ClusterPlan cp = dx == dy ? NO_CLUSTER : plan_cluster(C, S, batch, vec_ok, 4);
@@ -576,7 +585,7 @@ MI355_API int mi355_rmsnorm_bwd_dev(float *dx, float *dw, const float *dy, const
         if (mi355_dw_submit(dw, part, nrows, C)) return -1;
         return mi355_dw_op_end();
     }
-    NormCfg cfg = plan_tile(1, C, S, batch, vec_ok);
+    const NormCfg cfg = tile_for_alias(plan_tile(1, C, S, batch, vec_ok), dx == dy, S);
     const int strips = (int)ceil_div((size_t)S, (size_t)cfg.lpr * cfg.vec);
     const int nblk = strips * batch;
     float *part = mi355_dw_partials((size_t)nblk * C, dw, nullptr);
@@ -598,9 +607,9 @@ MI355_API int mi355_rmsnorm_bwd_residual_dev(float *dx, float *dx_scaled, float 
     if (dx_scaled && (dx_scaled == dx || dx_scaled == dy || dx_scaled == x || dx_scaled == res))
         return mi355_fail("rmsnorm_bwd_residual: dx_scaled must not alias another operand");
     if (dx == x) return mi355_fail("rmsnorm_bwd_residual: dx must not alias x (dx may alias res or dy)");
-    const bool vec_ok = (S % 4 == 0) && aligned16(x) && aligned16(dy) && aligned16(dx) && aligned16(res) &&
-                        (!dx_scaled || aligned16(dx_scaled));
-    const ClusterPlan cp = dx == dy ? NO_CLUSTER : plan_cluster(C, S, batch, vec_ok, 4, 2);
+    const bool vec_ok = S >= 4;
+    const bool apart = dx != res || tail_in_strip(S, CL_LPR * StoreF32::VEC, StoreF32::VEC);
+    const ClusterPlan cp = dx == dy || !apart ? NO_CLUSTER : plan_cluster(C, S, batch, vec_ok, 4, 2);
     if (cp.csplit) {
         if (!cluster_ws_ready()) return -1;
         const int nrows = cp.nblk / cp.csplit;
@@ -611,7 +620,7 @@ MI355_API int mi355_rmsnorm_bwd_residual_dev(float *dx, float *dx_scaled, float 
         if (mi355_dw_submit(dw, part, nrows, C)) return -1;
         return mi355_dw_op_end();
     }
-    NormCfg cfg = plan_tile(2, C, S, batch, vec_ok);
+    const NormCfg cfg = tile_for_alias(plan_tile(2, C, S, batch, vec_ok), dx == dy || dx == res, S);
     const int strips = (int)ceil_div((size_t)S, (size_t)cfg.lpr * cfg.vec);
     const int nblk = strips * batch;
     float *part = mi355_dw_partials((size_t)nblk * C, dw, nullptr);
@@ -629,10 +638,10 @@ MI355_API int mi355_residual_rmsnorm_fwd_dev(float *y, float *yn, const float *a
     if (C <= 0 || S <= 0 || batch <= 0)
         return mi355_fail("residual_rmsnorm_fwd: bad shape C=%d S=%d batch=%d", C, S, batch);
     if (yn == y || yn == a || yn == b) return mi355_fail("residual_rmsnorm_fwd: yn must not alias y, a or b");
-    const bool vec_ok = (S % 4 == 0) && aligned16(y) && aligned16(yn) && aligned16(a) && aligned16(b);
+    const bool vec_ok = S >= 4, in_place = y == a || y == b;
     const float invC = 1.0f / (float)C;
     // in place (y over a or b) the single-workgroup tile is used, for the reason given in mi355_rmsnorm_bwd_dev
-    const ClusterPlan cp = (y == a || y == b) ? NO_CLUSTER : plan_cluster(C, S, batch, vec_ok, 8);
+    const ClusterPlan cp = in_place ? NO_CLUSTER : plan_cluster(C, S, batch, vec_ok, 8);
     if (cp.csplit) {
         if (!cluster_ws_ready()) return -1;
         launch_fwd_cluster<true>(cp, yn, y, a, b, alpha, w, C, S, eps);
@@ -646,14 +655,24 @@ MI355_API int mi355_residual_rmsnorm_fwd_dev(float *y, float *yn, const float *a
                            g_ctx.stream, y, yn, a, b, alpha, w, C, S, strips, strips * batch, eps, invC);        \
     } while (0)
     const long strips8 = (long)ceil_div((size_t)S, 32) * batch;
-    if (!vec_ok) RES_RMS(1, 64, 256, 0);
+    NormCfg cfg = SCALAR_TILE;
+    if (!vec_ok) cfg = SCALAR_TILE;
     else if (C > 512 && C <= 1024 && strips8 >= (g_ctx.num_cu > 0 ? g_ctx.num_cu : 256) && !g_ctx.rms_threads)
-        RES_RMS(4, 8, 1024, 8);
-    else if (C <= 128) RES_RMS(4, 16, 256, 8);
-    else if (C <= 512 && g_ctx.rms_threads != 1024) RES_RMS(4, 4, 256, 8);
-    else if (C <= 2048 && g_ctx.rms_threads != 256) RES_RMS(4, 4, 1024, 8);
-    else if (C <= 1024) RES_RMS(4, 4, 256, 16);
-    else RES_RMS(4, 8, 1024, 0);
+        cfg = NormCfg{4, 8, 1024, 8};
+    else if (C <= 128) cfg = NormCfg{4, 16, 256, 8};
+    else if (C <= 512 && g_ctx.rms_threads != 1024) cfg = NormCfg{4, 4, 256, 8};
+    else if (C <= 2048 && g_ctx.rms_threads != 256) cfg = NormCfg{4, 4, 1024, 8};
+    else if (C <= 1024) cfg = NormCfg{4, 4, 256, 16};
+    else cfg = NormCfg{4, 8, 1024, 0};
+    switch (norm_key(tile_for_alias(cfg, in_place, S))) {
+        case 4080408: RES_RMS(4, 8, 1024, 8); break;
+        case 4160108: RES_RMS(4, 16, 256, 8); break;
+        case 4040108: RES_RMS(4, 4, 256, 8); break;
+        case 4040408: RES_RMS(4, 4, 1024, 8); break;
+        case 4040116: RES_RMS(4, 4, 256, 16); break;
+        case 4080400: RES_RMS(4, 8, 1024, 0); break;
+        default: RES_RMS(1, 64, 256, 0); break;
+    }
 #undef RES_RMS
     LAUNCH_OK("residual_rmsnorm_fwd");
     return 0;

@@ -60,7 +60,7 @@ struct StoreBf16 {
     static constexpr int VEC = 8;
     static __device__ __forceinline__ Raw load_nt(const T *p) { return ld_raw<VEC, true>(p); }
     static __device__ __forceinline__ Raw load(const T *p) { return ld_raw<VEC, false>(p); }
-    static __device__ __forceinline__ void store_nt(T *p, Raw r) { __builtin_nontemporal_store(r, reinterpret_cast<v4u *>(p)); }
+    static __device__ __forceinline__ void store_nt(T *p, Raw r) { __builtin_nontemporal_store(r, reinterpret_cast<v4u_any *>(p)); }
     static __device__ __forceinline__ void widen(float (&v)[VEC], const Raw &r) { unpack<VEC>(v, r); }
     static __device__ __forceinline__ Raw pack(const float (&v)[VEC]) {
         Raw r;
@@ -195,8 +195,9 @@ __global__ __launch_bounds__(THREADS) void rms_fwd_cluster_kernel(typename ST::T
     __shared__ int failed;
     const ClusterGeo g = cluster_geo(nblk, csplit, strips);
     const int lc = threadIdx.x % CL_LPR, row0 = threadIdx.x / CL_LPR;
-    const int col = g.strip * W + lc * VEC;
-    const bool col_ok = col < S;
+    const LaneCols mine = lane_cols<VEC>(g.strip * W + lc * VEC, S);
+    const int col = mine.col;
+    const bool col_ok = mine.ok;
     const size_t slab_base = (size_t)g.slab * C * S + col;
     if (threadIdx.x == 0) failed = 0;
     unsigned my_tag, want_tag[cluster_fetches<THREADS, 1, VEC>()];
@@ -312,8 +313,9 @@ __global__ __launch_bounds__(THREADS) void rms_bwd_cluster_kernel(typename ST::T
     __shared__ int failed;
     const ClusterGeo g = cluster_geo(nblk, csplit, strips);
     const int lc = threadIdx.x % CL_LPR, row0 = threadIdx.x / CL_LPR;
-    const int col = g.strip * W + lc * VEC;
-    const bool col_ok = col < S;
+    const LaneCols mine = lane_cols<VEC>(g.strip * W + lc * VEC, S);
+    const int col = mine.col;
+    const bool col_ok = mine.ok;
     const size_t slab_base = (size_t)g.slab * C * S + col;
     if (threadIdx.x == 0) failed = 0;
     unsigned my_tag, want_tag[cluster_fetches<THREADS, 2, VEC>()];
@@ -411,7 +413,13 @@ __global__ __launch_bounds__(THREADS) void rms_bwd_cluster_kernel(typename ST::T
             for (int j = 0; j < VEC; j++) {
                 if (variant == 0) o[j] = ((dv[j] - xv[j] * dotn[j]) * rr[j]) * wv[k];
                 else o[j] = (dv[j] * wv[k]) * rr[j] - (xv[j] * dotn[j]) * rr[j];
-                p += (dv[j] * xv[j]) * rr[j];
+            }
+            auto dw_term = [&](int j) { return (dv[j] * xv[j]) * rr[j]; };
+            if constexpr (EXACT) {
+#pragma unroll
+                for (int j = 0; j < VEC; j++) p += dw_term(j);
+            } else {
+                p = own_sum<VEC>(mine, dw_term);
             }
             if constexpr (RES) {
                 float rv[VEC];

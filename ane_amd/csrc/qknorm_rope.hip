@@ -30,8 +30,9 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_fwd_kernel(
     else { blk -= nq; in = k; out = k_out; w = wk; }
     const int slab = blk / strips, strip = blk - slab * strips;
     const int lc = threadIdx.x % LPR, p0 = threadIdx.x / LPR;
-    const int col = strip * W + lc * 4;
-    const bool col_ok = col < S;
+    const LaneCols mine = lane_cols<4>(strip * W + lc * 4, S);
+    const int col = mine.col;
+    const bool col_ok = mine.ok;
     const int half = hd >> 1;
     const size_t base = (size_t)slab * hd * S + col;
 
@@ -98,8 +99,9 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_bwd_kernel(
     else { blk -= nq; gin = dk_out; xin = k; out = dk; w = wk; }
     const int slab = blk / strips, strip = blk - slab * strips;
     const int lc = threadIdx.x % LPR, p0 = threadIdx.x / LPR;
-    const int col = strip * W + lc * 4;
-    const bool col_ok = col < S;
+    const LaneCols mine = lane_cols<4>(strip * W + lc * 4, S);
+    const int col = mine.col;
+    const bool col_ok = mine.ok;
     const int half = hd >> 1;
     const size_t base = (size_t)slab * hd * S + col;
 
@@ -159,8 +161,8 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_bwd_kernel(
                 st4_nt(po + S, o1);
             }
             const v4f t0 = (d0[kk] * x0[kk]) * rr, t1 = (d1[kk] * x1[kk]) * rr;
-            float s0 = ((t0[0] + t0[1]) + t0[2]) + t0[3];
-            float s1 = ((t1[0] + t1[1]) + t1[2]) + t1[3];
+            float s0 = own_sum<4>(mine, [&](int j) { return t0[j]; });
+            float s1 = own_sum<4>(mine, [&](int j) { return t1[j]; });
             s0 = group_sum<LPR>(s0);
             s1 = group_sum<LPR>(s1);
             if (lc == 0) {
@@ -179,13 +181,16 @@ struct QkCfg {
     int lpr, threads, cap;
 };
 
-// widest strip whose row pairs fit the register tile (at most 4 pairs per lane: 8 would spill)
-bool pick_qk(int hd, QkCfg &cfg, bool backward) {
+// Widest strip whose row pairs fit the register tile (at most 4 pairs per lane: 8 would spill).  In place the short
+// last group of columns of a row and its neighbour must lie in one strip (lane_cols in tile.h).
+bool pick_qk(int hd, int S, bool in_place, QkCfg &cfg, bool backward) {
     const int half = hd / 2;
+    if (S < 4) return false;
     const int lprs[3] = {16, 8, 4};
     const int thr = g_ctx.qk_threads == 256 || g_ctx.qk_threads == 512 ? g_ctx.qk_threads : (backward ? QK_THREADS_BWD : QK_THREADS_FWD);
     for (int lpr : lprs) {
         if (g_ctx.qk_lpr && g_ctx.qk_lpr != lpr) continue;
+        if (in_place && !tail_in_strip(S, lpr * 4, 4)) continue;
         const int pps = thr / lpr;
         const int caps[3] = {1, 2, 4};
         for (int cap : caps)
@@ -236,10 +241,7 @@ MI355_API int mi355_qknorm_rope_fwd_dev(float *q_out, float *k_out, const float 
     if (!cos_dev || !sin_dev || (heads > 0 && (!q_out || !q || !wq)) || (kv_heads > 0 && (!k_out || !k || !wk)))
         return mi355_fail("qknorm_rope_fwd: NULL pointer");
     QkCfg cfg;
-    const bool vec_ok = (S % 4 == 0) && aligned16(cos_dev) && aligned16(sin_dev) &&
-                        (heads == 0 || (aligned16(q) && aligned16(q_out))) &&
-                        (kv_heads == 0 || (aligned16(k) && aligned16(k_out)));
-    if (!vec_ok || !pick_qk(hd, cfg, false)) {
+    if (!pick_qk(hd, S, q_out == q || k_out == k, cfg, false)) {
         // unfused composition: per-head norm (heads folded into the batch), then the rotation in place
         if (heads > 0 && mi355_rmsnorm_fwd_dev(q_out, q, wq, hd, S, batch * heads, eps)) return -1;
         if (kv_heads > 0 && mi355_rmsnorm_fwd_dev(k_out, k, wk, hd, S, batch * kv_heads, eps)) return -1;
@@ -264,10 +266,7 @@ MI355_API int mi355_qknorm_rope_bwd_dev(float *dq, float *dk, float *dwq, float 
         (kv_heads > 0 && (!dk || !dwk || !dk_out || !k || !wk)))
         return mi355_fail("qknorm_rope_bwd: NULL pointer");
     QkCfg cfg;
-    const bool vec_ok = (S % 4 == 0) && aligned16(cos_dev) && aligned16(sin_dev) &&
-                        (heads == 0 || (aligned16(q) && aligned16(dq) && aligned16(dq_out))) &&
-                        (kv_heads == 0 || (aligned16(k) && aligned16(dk) && aligned16(dk_out)));
-    if (!vec_ok || !pick_qk(hd, cfg, true)) {
+    if (!pick_qk(hd, S, dq == dq_out || dk == dk_out, cfg, true)) {
         // unfused composition: inverse rotation into dq/dk, then the per-head norm backward in place
         if (mi355_rope_dev(dq, dk, dq_out, dk_out, heads, kv_heads, hd, S, batch, cos_dev, sin_dev, -1)) return -1;
         if (heads > 0 && mi355_rmsnorm_bwd_dev(dq, dwq, dq, q, wq, hd, S, batch * heads, eps, variant)) return -1;

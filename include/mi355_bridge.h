@@ -130,8 +130,8 @@ int mi355_softmax_ce_bf16_dev(uint16_t *dlogits, float *loss_dev, const uint16_t
                               int V, int S, float grad_scale);
 int mi355_rope_bf16_dev(uint16_t *q_out, uint16_t *k_out, const uint16_t *q_in, const uint16_t *k_in, int heads,
                         int kv_heads, int hd, int S, int batch, const float *cos_dev, const float *sin_dev, int dir);
-/* The head size must fit the register tile: hd <= 1024 with rows of a multiple of 8 columns and 16-byte aligned
- * pointers, hd <= 128 otherwise (the fp32 entry points have no such limit). */
+/* The head size must fit the register tile: hd <= 1024 with rows of at least 8 columns (in place: of a multiple of 8),
+ * hd <= 128 otherwise (the fp32 entry points have no such limit). */
 int mi355_qknorm_rope_fwd_bf16_dev(uint16_t *q_out, uint16_t *k_out, const uint16_t *q, const uint16_t *k,
                                    const float *wq, const float *wk, int heads, int kv_heads, int hd, int S, int batch,
                                    const float *cos_dev, const float *sin_dev, float eps);
@@ -185,8 +185,8 @@ int mi355_rmsnorm_bwd_dev(float *dx, float *dw, const float *dy, const float *x,
                           int C, int S, int batch, float eps, int variant);
 
 /* Introspection, host-only (needs no GPU): the register tile that the RMSNorm entry points choose for a shape —
- * op 0 = mi355_rmsnorm_fwd_dev, 1 = mi355_rmsnorm_bwd_dev, 2 = mi355_rmsnorm_bwd_residual_dev; aligned != 0 means
- * 16-byte aligned tensors.  tile5 (may be NULL) receives {columns per lane, lanes per row piece, threads per
+ * op 0 = mi355_rmsnorm_fwd_dev, 1 = mi355_rmsnorm_bwd_dev, 2 = mi355_rmsnorm_bwd_residual_dev; `aligned` is without
+ * effect (128-bit accesses start at any float).  tile5 (may be NULL) receives {columns per lane, lanes per row piece, threads per
  * workgroup, rows per lane held in registers (0 = rows are read twice), workgroups that share the rows of one strip
  * (0 = one workgroup owns all C rows; 2, 4 or 8 = the clustered kernels, which out-of-place calls of tall shapes
  * run)}.  0, or -1 if no kernel exists for the choice (a defect: the entry point would fail the same way). */
