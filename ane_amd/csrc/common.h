@@ -35,7 +35,7 @@ struct Mi355Ctx {
     int scatter_cols;          // ordered scatter-add with the columns of dE dealt out to the workgroups: 0 = where it pays,
                                // 1 = whenever the shape allows, -1 = never
     int rms_cluster;           // channel split of the clustered RMSNorm: 0 = per shape, -1 = never, 2/4/8 = forced
-    int ce_resident;           // one-launch softmax-CE: 0 = where it pays, 1 = whenever the shape allows, -1 = never
+    int ce_resident;           // one-launch softmax-CE: -1 = never, otherwise whenever the shape allows
     int rms_cluster_spin;      // its bounded wait in ticks of the 100 MHz clock: 0 = 2 ms, negative = do not wait at all
     int xch_take_nothing;      // test mode of those kernels: 1 = no partner's value is taken, present or not, so every
                                // workgroup goes the way of an expired wait

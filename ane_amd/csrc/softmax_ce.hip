@@ -49,12 +49,13 @@ __device__ __forceinline__ void ld_cols_nt(float (&r)[VEC], const float *p) {
 // bfloat16 logits (the optional bf16-storage variant): four columns = one 64-bit access; widened to fp32 here,
 // so everything below is the same arithmetic for both storage types.
 typedef unsigned int v2u __attribute__((ext_vector_type(2)));
+typedef unsigned int v2u_any __attribute__((ext_vector_type(2), aligned(2)));     // at any bfloat16 element
 __device__ __forceinline__ float bf_widen(unsigned bits16) { return bf_to_f(bits16); }
 __device__ __forceinline__ unsigned bf_narrow(float f) { return f_to_bf(f); }      // round to nearest even; NaN stays NaN
 template <int VEC>
 __device__ __forceinline__ void ld_cols(float (&r)[VEC], const uint16_t *p) {
     if constexpr (VEC == 4) {
-        const v2u w = *reinterpret_cast<const v2u *>(p);
+        const v2u w = *reinterpret_cast<const v2u_any *>(p);
         r[0] = bf_widen(w[0] & 0xffffu); r[1] = bf_widen(w[0] >> 16);
         r[2] = bf_widen(w[1] & 0xffffu); r[3] = bf_widen(w[1] >> 16);
     } else {
@@ -64,7 +65,7 @@ __device__ __forceinline__ void ld_cols(float (&r)[VEC], const uint16_t *p) {
 template <int VEC>
 __device__ __forceinline__ void ld_cols_nt(float (&r)[VEC], const uint16_t *p) {
     if constexpr (VEC == 4) {
-        const v2u w = __builtin_nontemporal_load(reinterpret_cast<const v2u *>(p));
+        const v2u w = __builtin_nontemporal_load(reinterpret_cast<const v2u_any *>(p));
         r[0] = bf_widen(w[0] & 0xffffu); r[1] = bf_widen(w[0] >> 16);
         r[2] = bf_widen(w[1] & 0xffffu); r[3] = bf_widen(w[1] >> 16);
     } else {
@@ -86,7 +87,7 @@ template <int VEC>
 __device__ __forceinline__ void st_cols(uint16_t *p, const float (&o)[VEC]) {
     if constexpr (VEC == 4) {
         v2u w = {bf_narrow(o[0]) | (bf_narrow(o[1]) << 16), bf_narrow(o[2]) | (bf_narrow(o[3]) << 16)};
-        __builtin_nontemporal_store(w, reinterpret_cast<v2u *>(p));
+        __builtin_nontemporal_store(w, reinterpret_cast<v2u_any *>(p));
     } else {
         *p = (uint16_t)bf_narrow(o[0]);
     }
@@ -354,8 +355,8 @@ __global__ __launch_bounds__(256) void nll_grad_kernel(float *dlogits, const flo
 // with ONE workgroup of 1024 threads per compute unit can read most rows once: a workgroup owns a block of rows of
 // one 64-column strip (256-byte row pieces), keeps its last 16 row steps in registers and the 9 before them in LDS
 // (25 of the 38 steps of the Qwen3 vocabulary; all of them for 32000 rows, and for bfloat16 storage, whose rows take
-// half the space), and reads only the remainder a second time.  Measured at [151936][256]: 69 us against 84 us for
-// the three launches (bfloat16: 61 against 99).  The (max, sum exp) partials of the workgroups of a strip (its members)
+// half the space), and reads only the remainder a second time.  Measured at [151936][256]: 66 us against 83 us for
+// the three launches (bfloat16: 49 against 88).  The (max, sum exp) partials of the workgroups of a strip (its members)
 // are exchanged through tagged 8-byte slots as in the clustered RMSNorm (norm_cluster.h): one relaxed agent-scope
 // atomic {fp32 value, launch tag} per slot, a launch counter per workgroup number, nothing to clear, a bounded
 // wait.  A member whose wait for a partner expires recomputes that partner's partial from memory with the same
@@ -384,25 +385,31 @@ struct CeXch {
 struct CrF32 {
     typedef float T;
     typedef v4f Raw;
-    static constexpr int K_REG = 16, K_LDS = 9;
+    static constexpr int K_REG = 16, K_LDS = 9;        // of the largest variant
     static __device__ __forceinline__ Raw ld(const T *p) { return ld4(p); }
     static __device__ __forceinline__ Raw ld_nt(const T *p) { return ld4_nt(p); }
     static __device__ __forceinline__ Raw ninf() { Raw r = {-INFINITY, -INFINITY, -INFINITY, -INFINITY}; return r; }
     static __device__ __forceinline__ float at(const Raw &r, int j) { return r[j]; }
-    static __device__ __forceinline__ void st_nt(T *p, const float (&o)[4]) { Raw r = {o[0], o[1], o[2], o[3]}; st4_nt(p, r); }
+    template <bool NT>
+    static __device__ __forceinline__ void st(T *p, const float (&o)[4]) {
+        const Raw r = {o[0], o[1], o[2], o[3]};
+        if constexpr (NT) st4_nt(p, r); else st4(p, r);
+    }
     static __device__ __forceinline__ void forget(Raw &) {}
 };
 struct CrBf16 {
     typedef uint16_t T;
     typedef v2u Raw;
-    static constexpr int K_REG = 32, K_LDS = 18;
-    static __device__ __forceinline__ Raw ld(const T *p) { return *reinterpret_cast<const v2u *>(p); }
-    static __device__ __forceinline__ Raw ld_nt(const T *p) { return __builtin_nontemporal_load(reinterpret_cast<const v2u *>(p)); }
+    static constexpr int K_REG = 32, K_LDS = 18;       // of the largest variant
+    static __device__ __forceinline__ Raw ld(const T *p) { return *reinterpret_cast<const v2u_any *>(p); }
+    static __device__ __forceinline__ Raw ld_nt(const T *p) { return __builtin_nontemporal_load(reinterpret_cast<const v2u_any *>(p)); }
     static __device__ __forceinline__ Raw ninf() { Raw r = {0xff80ff80u, 0xff80ff80u}; return r; }
     static __device__ __forceinline__ float at(const Raw &r, int j) { return bf_to_f((j & 1) ? r[j >> 1] >> 16 : r[j >> 1] & 0xffffu); }
-    static __device__ __forceinline__ void st_nt(T *p, const float (&o)[4]) {
-        Raw r = {f2_to_bf2(o[0], o[1]), f2_to_bf2(o[2], o[3])};
-        __builtin_nontemporal_store(r, reinterpret_cast<v2u *>(p));
+    template <bool NT>
+    static __device__ __forceinline__ void st(T *p, const float (&o)[4]) {
+        const Raw r = {f2_to_bf2(o[0], o[1]), f2_to_bf2(o[2], o[3])};
+        if constexpr (NT) __builtin_nontemporal_store(r, reinterpret_cast<v2u_any *>(p));
+        else *reinterpret_cast<v2u_any *>(p) = r;
     }
     // Tells the compiler nothing about the words' contents from here on, so that the widened copies made for the
     // first pass are dropped instead of being kept alive for the second (they would double the register rows).
@@ -415,8 +422,31 @@ struct CrBf16 {
 template <typename T>
 struct CrGeo {
     const T *logits;
-    int V, S, strips, csplit, Rm, K;   // Rm rows per member, K = ceil(Rm / CR_RPS) row steps
+    int V, S, strips, sw, csplit, Rm;      // sw columns per strip, Rm rows per member
 };
+// The columns of lane lc of a strip (lane_cols in tile.h: the short last group of a row of any length takes its
+// neighbour's columns again).  The partials of a strip are kept by slot, four per lane: slot 4*lc + j is column col + j
+// and counts once, where j >= dup.
+__device__ __forceinline__ LaneCols cr_cols(int strip, int sw, int lc, int S) {
+    LaneCols l = lane_cols<4>(strip * sw + lc * 4, S);
+    l.ok = l.ok && lc * 4 < sw;
+    if (!l.ok) l.col = lane_cols<4>(strip * sw, S).col;      // no columns: reads along with lane 0, stores nothing
+    return l;
+}
+// The rows of member p: R of them from v_lo, in K steps of CR_RPS rows.  A lane has its row of every step but the last,
+// and of that one if row0 is below `last`.
+struct CrRows {
+    int v_lo, K, last;
+};
+template <typename T>
+__device__ __forceinline__ CrRows cr_rows(const CrGeo<T> &g, int p) {
+    CrRows r;
+    r.v_lo = p * g.Rm;
+    const int R = max(0, min(g.V, r.v_lo + g.Rm) - r.v_lo);
+    r.K = (R + CR_RPS - 1) / CR_RPS;
+    r.last = R - (r.K - 1) * CR_RPS;
+    return r;
+}
 
 // (m, l) <- (m, l) merged with N more values: the online-softmax step
 template <int N>
@@ -433,67 +463,55 @@ __device__ __forceinline__ void online_update(float &m, float &l, const float (&
         m = nm;
     }
 }
-__device__ __forceinline__ void merge_pair(float &m, float &l, float m1, float l1) {
-    const float nm = fmaxf(m, m1);
-    if (nm > -INFINITY) {
-        l = l * exp_neg(m - nm) + l1 * exp_neg(m1 - nm);
-        m = nm;
-    }
+// Sixteen (max, sum) pairs per column, [16][CR_P] in LDS -> their merge, in the quad of threads 4c .. 4c+3 of column c
+// (waves 0 to 3): the maximum first, then every sum rescaled to it and added in a fixed order.  A pair without rows is
+// (-inf, 0); exp_neg of the NaN that -inf - -inf gives is zero (its fmax drops the NaN).
+constexpr int CR_P = CR_W + 16;              // row pitch: the four threads of a quad read four rows of a column
+__device__ __forceinline__ void cr_merge16(const float (*wm)[CR_P], const float (*wl)[CR_P], float &M, float &L) {
+    const int c = threadIdx.x >> 2, q = threadIdx.x & 3;
+    float mm[CR_NW / 4];
+    M = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < CR_NW / 4; i++) { mm[i] = wm[q + 4 * i][c]; M = fmaxf(M, mm[i]); }
+    M = fmaxf(M, lane_xor<1>(M));
+    M = fmaxf(M, lane_xor<2>(M));
+    L = 0.f;
+#pragma unroll
+    for (int i = 0; i < CR_NW / 4; i++) L += wl[q + 4 * i][c] * exp_neg(mm[i] - M);
+    L += lane_xor<1>(L);
+    L += lane_xor<2>(L);
 }
 
-// Sixteen (max, sum) pairs of one column -> their merge: the maximum, then the sums rescaled to it (sixteen
-// independent exponentials) and added in order.
-__device__ __forceinline__ void cr_merge16(const float (*wm)[CR_W], const float (*wl)[CR_W], int c, float &M, float &L) {
-    float mm[CR_NW];
-    float mx = -INFINITY;
-#pragma unroll
-    for (int w = 0; w < CR_NW; w++) { mm[w] = wm[w][c]; mx = fmaxf(mx, mm[w]); }
-    float acc = 0.f;
-#pragma unroll
-    for (int w = 0; w < CR_NW; w++) acc += wl[w][c] * exp_neg(mm[w] - mx);     // an empty part has sum 0
-    M = mx;
-    L = acc;
-}
-
-// The (max, sum exp) partial of member p of a strip over its rows, for the 64 columns of the strip: valid in
-// threads 0..63 (thread t = column t) on return.  Of a member's K row steps the last K_REG are the register rows,
-// the K_LDS before them the LDS rows, and the first kL = K - K_REG - K_LDS the rows that are read twice.  A lane
-// folds its rows into its running (max, sum) four at a time, in row order: the rows before the register rows, then
-// the register rows.  KEEP: this workgroup's own rows; the loads run ahead of the arithmetic.
-// Otherwise nothing is kept: one column and one
-// group of four rows at a time, the same operations on the same values in the same order (same bits) in a handful
-// of registers, because the caller's own rows stay live in theirs.
-template <typename ST, bool KEEP, bool NT = false>
-__device__ __forceinline__ void cr_member_partial(const CrGeo<typename ST::T> &g, int strip, int p, typename ST::Raw (&xr)[ST::K_REG],
+// The (max, sum exp) partial of member p of a strip over its rows, for the 64 slots of the strip: valid in the quad of
+// threads 4c .. 4c+3 of slot c on return.  Of a member's K row steps the last K_REG are the register rows, the K_LDS
+// before them the LDS rows, and the first kL = K - K_REG - K_LDS the rows that are read twice.  A lane folds its rows
+// into its running (max, sum) four at a time, in row order: the rows before the register rows, then the register rows.
+// KEEP: this workgroup's own rows; the loads run ahead of the arithmetic.  Every condition on a step is the same for the
+// whole workgroup (scalar branches); a lane without a row in the last step reads the member's last row and its value
+// is replaced when it is folded.
+// Otherwise nothing is kept: one column and one group of four rows at a time, the same operations on the same values
+// in the same order (same bits) in a handful of registers, because the caller's own rows stay live in theirs.
+template <typename ST, int K_REG, int K_LDS, bool KEEP, bool NT>
+__device__ __forceinline__ void cr_member_partial(const CrGeo<typename ST::T> &g, int strip, int p, typename ST::Raw (&xr)[K_REG],
                                                   typename ST::Raw (*lrow)[CR_THREADS],
-                                                  float (*wm)[CR_W], float (*wl)[CR_W], float &Mout, float &Lout) {
+                                                  float (*wm)[CR_P], float (*wl)[CR_P], float &Mout, float &Lout) {
     typedef typename ST::Raw Raw;
-    constexpr int K_REG = ST::K_REG, K_LDS = ST::K_LDS;
     static_assert(K_REG % CR_SUB == 0, "the register rows fold four at a time");
     const int lc = threadIdx.x & 15, row0 = threadIdx.x >> 4, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int v_lo = p * g.Rm;
-    constexpr int rs = CR_RPS;                                    // rows between a lane's consecutive rows
-    // this lane holds the member's rows row0 + rs*k; they exist while rs*k < lim
-    const int lim = min(g.V, v_lo + g.Rm) - v_lo - row0;
-    const int kR = max(0, g.K - K_REG), kL = max(0, kR - K_LDS);
-    // a row piece = (uniform address of row v_lo + rs*k of the strip) + (this lane's fixed 32-bit offset)
-    const typename ST::T *base = g.logits + ((size_t)v_lo * g.S + (size_t)strip * CR_W);
-    const unsigned loff = (unsigned)row0 * (unsigned)g.S + (unsigned)lc * 4u;
-    const size_t step = (size_t)rs * g.S;
+    const LaneCols mine = cr_cols(strip, g.sw, lc, g.S);
+    const CrRows r = cr_rows(g, p);
+    const int K = r.K, kR = max(0, K - K_REG), kL = max(0, kR - K_LDS);
+    const int mineK = row0 < r.last ? K : K - 1;                  // steps in which this lane has a row
+    // a row piece = (uniform address of row v_lo + 64k) + (this lane's fixed 32-bit offset)
+    const typename ST::T *base = g.logits + (size_t)r.v_lo * g.S;
+    const unsigned loff = (unsigned)row0 * (unsigned)g.S + (unsigned)mine.col;
+    const unsigned loff_last = (unsigned)min(row0, max(r.last - 1, 0)) * (unsigned)g.S + (unsigned)mine.col;
+    const size_t step = (size_t)CR_RPS * g.S;
     const Raw ninf = ST::ninf();
     float m[4], l[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) { m[j] = -INFINITY; l[j] = 0.f; }
     if constexpr (KEEP) {
-        // rows that stay on the chip may be read past the cache (they are not read again); the others stay cached
-        auto loadg = [&](Raw (&t)[CR_SUB], int k0) {
-#pragma unroll
-            for (int u = 0; u < CR_SUB; u++) {
-                const int k = k0 + u;
-                if (k < kR && rs * k < lim) t[u] = (NT && k >= kL) ? ST::ld_nt(base + k * step + loff) : ST::ld(base + k * step + loff);
-                else t[u] = ninf;
-            }
-        };
         auto foldg = [&](const Raw (&t)[CR_SUB]) {
 #pragma unroll
             for (int j = 0; j < 4; j++) {
@@ -503,19 +521,34 @@ __device__ __forceinline__ void cr_member_partial(const CrGeo<typename ST::T> &g
                 online_update<CR_SUB>(m[j], l[j], x4);
             }
         };
-        auto keepg = [&](const Raw (&t)[CR_SUB], int k0) {
-#pragma unroll
-            for (int u = 0; u < CR_SUB; u++)
-                if (k0 + u >= kL && k0 + u < kR) lrow[k0 + u - kL][threadIdx.x] = t[u];
-        };
         // the register rows are asked for first and folded last: they are in flight while the other rows stream
-        // through two groups of four
+        // through two groups of four.  (Rows that stay on the chip may be read past the cache.)
 #pragma unroll
         for (int i = 0; i < K_REG; i++) {
             const int k = kR + i;
-            xr[i] = rs * k < lim ? (NT ? ST::ld_nt(base + k * step + loff) : ST::ld(base + k * step + loff)) : ninf;
+            if (k < K) {
+                const typename ST::T *a = base + k * step + (k == K - 1 ? loff_last : loff);
+                xr[i] = NT ? ST::ld_nt(a) : ST::ld(a);
+            }
         }
-        {
+        if (K_LDS > 0 && kR > 0) {
+            auto loadg = [&](Raw (&t)[CR_SUB], int k0) {
+#pragma unroll
+                for (int u = 0; u < CR_SUB; u++) {
+                    const int k = k0 + u;
+                    if (k < kR) {
+                        const typename ST::T *a = base + k * step + loff;
+                        t[u] = (NT && k >= kL) ? ST::ld_nt(a) : ST::ld(a);
+                    } else {
+                        t[u] = ninf;
+                    }
+                }
+            };
+            auto keepg = [&](const Raw (&t)[CR_SUB], int k0) {
+#pragma unroll
+                for (int u = 0; u < CR_SUB; u++)
+                    if (k0 + u >= kL && k0 + u < kR) lrow[k0 + u - kL][threadIdx.x] = t[u];
+            };
             Raw ta[CR_SUB], tb[CR_SUB];
             loadg(ta, 0);
             loadg(tb, CR_SUB);
@@ -532,18 +565,23 @@ __device__ __forceinline__ void cr_member_partial(const CrGeo<typename ST::T> &g
         }
 #pragma unroll
         for (int c = 0; c < K_REG / CR_SUB; c++) {
-            // (a member with fewer row steps than registers for them: the groups past its last step hold nothing,
-            // and folding nothing leaves (max, sum) as they are: skipped, for the exponentials' sake)
-            if (kR + c * CR_SUB >= g.K) continue;
-            Raw t[CR_SUB];
+            const int k0 = kR + c * CR_SUB;
+            if (k0 < K) {                                         // groups past the last step hold nothing
+                Raw t[CR_SUB];
 #pragma unroll
-            for (int u = 0; u < CR_SUB; u++) t[u] = xr[c * CR_SUB + u];
-            foldg(t);
+                for (int u = 0; u < CR_SUB; u++) t[u] = xr[c * CR_SUB + u];
+                if (k0 + CR_SUB >= K) {
+#pragma unroll
+                    for (int u = 0; u < CR_SUB; u++)
+                        if (k0 + u >= mineK) t[u] = ninf;
+                }
+                foldg(t);
+            }
         }
 #pragma unroll
         for (int i = 0; i < K_REG; i++) ST::forget(xr[i]);
     } else {
-#pragma unroll
+#pragma unroll 1
         for (int j = 0; j < 4; j++) {
             float mj = -INFINITY, lj = 0.f;
             auto part = [&](int kbeg, int kend) {
@@ -553,74 +591,80 @@ __device__ __forceinline__ void cr_member_partial(const CrGeo<typename ST::T> &g
 #pragma unroll
                     for (int u = 0; u < CR_SUB; u++) {
                         const int k = k0 + u;
-                        x4[u] = (k < kend && rs * k < lim) ? ld_one(base + k * step + loff + j) : -INFINITY;
+                        x4[u] = k < min(kend, mineK) ? ld_one(base + k * step + loff + j) : -INFINITY;
                     }
                     online_update<CR_SUB>(mj, lj, x4);
                 }
             };
             part(0, kR);
-            part(kR, kR + K_REG);
-            m[j] = mj;
-            l[j] = lj;
-            __builtin_amdgcn_sched_barrier(0);
+            part(kR, K);
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                if (q == j) { m[q] = mj; l[q] = lj; }
         }
     }
-    // the four row groups of a wave, then the sixteen waves in order
+    // the four row groups of a wave (their maximum, then the rescaled sums), then the sixteen waves
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-        merge_pair(m[j], l[j], lane_xor<16>(m[j]), lane_xor<16>(l[j]));
-        merge_pair(m[j], l[j], lane_xor<32>(m[j]), lane_xor<32>(l[j]));
+        float M = fmaxf(m[j], lane_xor<16>(m[j]));
+        M = fmaxf(M, lane_xor<32>(M));
+        float L = l[j] * exp_neg(m[j] - M);
+        L += lane_xor<16>(L);
+        L += lane_xor<32>(L);
+        m[j] = M;
+        l[j] = L;
     }
     if (lane < 16) {
 #pragma unroll
         for (int j = 0; j < 4; j++) { wm[wave][lc * 4 + j] = m[j]; wl[wave][lc * 4 + j] = l[j]; }
     }
     __syncthreads();
-    if (threadIdx.x < CR_W) cr_merge16(wm, wl, threadIdx.x, Mout, Lout);
+    if (threadIdx.x < 4 * CR_W) cr_merge16(wm, wl, Mout, Lout);
     __syncthreads();
 }
 
-constexpr int CR_MPG = CR_MAX_SPLIT / CR_NW;     // members per group of 64 threads (thread = group, column)
+constexpr int CR_MPG = CR_MAX_SPLIT / CR_NW;     // members per group of 64 threads (thread = group, slot)
 
-// The members' partials, four members per thread (pm, pl: member grp * mpg + q of column c) -> the strip's column
-// maxima and sums: the maximum first, then every member's sum rescaled to it and added in a fixed order (within the
-// sixteen groups, then the groups); valid in threads 0..63 on return.
-__device__ __forceinline__ void cr_merge_members(const float (&pm)[CR_MPG], const float (&pl)[CR_MPG], float (*wm)[CR_W],
-                                                 float (*wl)[CR_W], float &Mout, float &Lout) {
+// The members' partials, four members per thread (pm, pl: member grp * mpg + q of slot c) -> the strip's column maxima
+// and the reciprocals of its sums, in fM and fInv (valid after the barrier): first within the sixteen groups, then the
+// groups.
+__device__ __forceinline__ void cr_merge_members(const float (&pm)[CR_MPG], const float (&pl)[CR_MPG], float (*wm)[CR_P],
+                                                 float (*wl)[CR_P], float *fM, float *fInv) {
     const int c = threadIdx.x & 63, grp = threadIdx.x >> 6;
     float M = pm[0];
 #pragma unroll
     for (int q = 1; q < CR_MPG; q++) M = fmaxf(M, pm[q]);
-    wm[grp][c] = M;
-    __syncthreads();
-#pragma unroll
-    for (int w = 0; w < CR_NW; w++) M = fmaxf(M, wm[w][c]);
     float L = 0.f;
 #pragma unroll
-    for (int q = 0; q < CR_MPG; q++) L += pl[q] * exp_neg(pm[q] - M);      // a member that is absent has sum 0
+    for (int q = 0; q < CR_MPG; q++) L += pl[q] * exp_neg(pm[q] - M);      // a member that is absent is (-inf, 0)
+    wm[grp][c] = M;
     wl[grp][c] = L;
     __syncthreads();
-    if (threadIdx.x < CR_W) {
-        L = wl[0][threadIdx.x];
-#pragma unroll
-        for (int w = 1; w < CR_NW; w++) L += wl[w][threadIdx.x];
-        Mout = M;
-        Lout = L;
+    if (threadIdx.x < 4 * CR_W) {
+        cr_merge16(wm, wl, M, L);
+        if ((threadIdx.x & 3) == 0) { fM[threadIdx.x >> 2] = M; fInv[threadIdx.x >> 2] = 1.0f / L; }
     }
     __syncthreads();
 }
 
-// Sum over the strip's columns of -log(p[target] + 1e-10), by wave 0 (every lane of it ends with the sum).
+// The target of the column of slot threadIdx.x < 64 of a strip; -1 where the slot has no column of its own or the target
+// is out of range.
 template <typename T>
-__device__ __forceinline__ float cr_strip_loss(const CrGeo<T> &g, int strip, const int32_t *targets, float M, float inv) {
-    const int t = strip * CR_W + threadIdx.x;
-    const int tg = targets[t];
-    float loss = 0.f;
-    if (tg >= 0 && tg < g.V) {
-        const float p = exp_neg(ld_one(g.logits + (size_t)tg * g.S + t) - M) * inv;
-        loss = -logf(p + 1e-10f);
-    }
-    return wave_sum_far_first(loss);
+__device__ __forceinline__ int cr_slot_target(const CrGeo<T> &g, int strip, const int32_t *targets) {
+    const LaneCols mine = cr_cols(strip, g.sw, threadIdx.x >> 2, g.S);
+    if (!mine.ok || (int)(threadIdx.x & 3) < mine.dup) return -1;
+    const int tg = targets[mine.col + (threadIdx.x & 3)];
+    return tg < g.V ? tg : -1;
+}
+template <typename T>
+__device__ __forceinline__ float cr_slot_logit(const CrGeo<T> &g, int strip, int tg) {
+    if (tg < 0) return 0.f;
+    return ld_one(g.logits + (size_t)tg * g.S + cr_cols(strip, g.sw, threadIdx.x >> 2, g.S).col + (threadIdx.x & 3));
+}
+// Sum over the strip's columns of -log(p[target] + 1e-10), by wave 0 (every lane of it ends with the sum).
+__device__ __forceinline__ float cr_strip_loss(int tg, float logit, float M, float inv) {
+    const float p = exp_neg(logit - M) * inv;
+    return wave_sum_far_first(tg >= 0 ? -logf(p + 1e-10f) : 0.f);
 }
 
 // One bounded wait for a tagged slot.  false: the tag did not arrive within spin_ticks.
@@ -636,24 +680,31 @@ __device__ __forceinline__ bool cr_wait_slot(const unsigned long long *sp, unsig
 
 // grid: strips * csplit workgroups, all resident at once (one per compute unit).  Workgroup b: strip b % strips,
 // member b / strips, so that the workgroups that read the pieces of one row are neighbours in time.
-template <typename ST, bool NT>
+// K_REG, K_LDS: row steps kept in registers and in LDS.  The variants for few steps are not there for their registers:
+// the code of a step is written out once for each, 60 KB (fp32) and 83 KB (bfloat16) for the largest, and a launch that
+// runs through it once per wave waits for instructions: with one row step per workgroup ([1000][256]) a launch took
+// 12.8 us, 4.8 of them before its partial was ready.
+// NT: rows are read and written past the caches where their pieces are whole 128-byte lines; where two strips share
+// the lines at their border the caches have to put the pieces together ([151936][200] fp32 102 us past them, 77 with
+// them; [151936][256] 68 and 94).
+template <typename ST, int K_REG, int K_LDS, bool NT>
 __global__ __launch_bounds__(CR_THREADS) void ce_resident_kernel(typename ST::T *__restrict__ dlogits,
                                                                  const typename ST::T *__restrict__ logits,
                                                                  const int32_t *__restrict__ targets, int V, int S,
-                                                                 int strips, int csplit, int Rm, int K, float invS,
+                                                                 int strips, int sw, int csplit, int Rm, float invS,
                                                                  float grad_scale, float *__restrict__ loss_out, CeXch ws,
                                                                  int spin_ticks, int take_nothing) {
     typedef typename ST::Raw Raw;
-    constexpr int K_REG = ST::K_REG, K_LDS = ST::K_LDS;
-    __shared__ Raw lrow[K_LDS][CR_THREADS];
-    __shared__ float wm[CR_NW][CR_W], wl[CR_NW][CR_W];
+    __shared__ Raw lrow[K_LDS > 0 ? K_LDS : 1][K_LDS > 0 ? CR_THREADS : 1];
+    __shared__ float wm[CR_NW][CR_P], wl[CR_NW][CR_P];
     __shared__ float fb[2][CR_W];                  // one member's partial on its way to the threads that hold it
     __shared__ float fM[CR_W], fInv[CR_W];
     __shared__ float strip_loss[CR_MAX_STRIPS];
-    __shared__ unsigned want[CR_MAX_SPLIT], want_leader[CR_MAX_STRIPS];
-    __shared__ int failed[CR_MAX_SPLIT];
-    __shared__ int any_failed;
+    __shared__ unsigned want[CR_MAX_SPLIT];
+    __shared__ int failed[CR_MAX_SPLIT], failed_loss[CR_MAX_STRIPS];
+    __shared__ int any_failed, any_failed_loss;
     const int tid = threadIdx.x;
+    auto rows_of = [&]() { return (Raw (*)[CR_THREADS])lrow; };
     // Workgroups are dealt to the eight XCDs in turn.  The workgroups that read the pieces of one row run at the
     // same time and, where the split allows, on one XCD, so that each L2 sees whole rows.
     int strip = blockIdx.x % strips, me = blockIdx.x / strips;
@@ -663,26 +714,28 @@ __global__ __launch_bounds__(CR_THREADS) void ce_resident_kernel(typename ST::T 
         me = xcd + 8 * (q / strips);
     }
     const int b = me * strips + strip;           // the workgroup number that owns slots and counter
-    const CrGeo<typename ST::T> g = {logits, V, S, strips, csplit, Rm, K};
-    if (tid < csplit) { want[tid] = ws.cnt[tid * strips + strip] + 1u; failed[tid] = 0; }
-    if (tid < strips) want_leader[tid] = ws.cnt[tid] + 1u;          // member 0 of strip s is workgroup s
-    if (tid == 0) any_failed = 0;
+    const CrGeo<typename ST::T> g = {logits, V, S, strips, sw, csplit, Rm};
+    // the launch tags and the leader's targets are asked for ahead of the rows and wanted only after them
+    const unsigned t_mem = tid < csplit ? ws.cnt[tid * strips + strip] + 1u : 0u;
+    const unsigned t_lead = tid < strips ? ws.cnt[tid] + 1u : 0u;   // member 0 of strip s is workgroup s
     const unsigned my_tag = ws.cnt[b] + 1u;
-    __syncthreads();
+    const int my_tgt = me == 0 && tid < CR_W ? cr_slot_target(g, strip, targets) : -1;
 
     // ---- pass 1: this member's rows, kept; its partial published
     Raw xr[K_REG];
     float Mp = -INFINITY, Lp = 0.f;
-    cr_member_partial<ST, true, NT>(g, strip, me, xr, lrow, wm, wl, Mp, Lp);
-    if (tid < CR_W) {
-        unsigned long long *mine = ws.slots + (size_t)b * CR_STRIDE;
-        __hip_atomic_store(mine + tid, ((unsigned long long)my_tag << 32) | __float_as_uint(Mp), __ATOMIC_RELAXED,
+    cr_member_partial<ST, K_REG, K_LDS, true, NT>(g, strip, me, xr, rows_of(), wm, wl, Mp, Lp);
+    if (tid < 4 * CR_W && (tid & 3) < 2)
+        __hip_atomic_store(ws.slots + (size_t)b * CR_STRIDE + (tid & 3) * CR_W + (tid >> 2),
+                           ((unsigned long long)my_tag << 32) | __float_as_uint((tid & 3) ? Lp : Mp), __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(mine + CR_W + tid, ((unsigned long long)my_tag << 32) | __float_as_uint(Lp), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-    }
-    // ---- every member's partial.  Thread (group, column) fetches the (max, sum) slots of the group's members for
-    // its column: eight slots.  The loads of a round go out together, so a round costs one trip to the memory side
+    if (tid < csplit) { want[tid] = t_mem; failed[tid] = 0; }
+    if (tid < strips) failed_loss[tid] = 0;
+    if (tid == 0) any_failed = any_failed_loss = 0;
+    const float my_logit = cr_slot_logit(g, strip, my_tgt);         // (in flight while the partners' partials are awaited)
+    __syncthreads();
+    // ---- every member's partial.  Thread (group, slot) fetches the (max, sum) slots of the group's members for
+    // its slot: eight of them.  The loads of a round go out together, so a round costs one trip to the memory side
     // however many of the eight are still missing.
     const int mc = tid & 63, mgrp = tid >> 6;
     const int mpg = (csplit + CR_NW - 1) / CR_NW;                      // members per group, at most CR_MPG
@@ -733,155 +786,142 @@ __global__ __launch_bounds__(CR_THREADS) void ce_resident_kernel(typename ST::T 
             }
         }
     }
+    // one member's partial from memory, into the threads that hold it
+    auto recompute = [&](int s2, int p, float (&qm)[CR_MPG], float (&ql)[CR_MPG]) {
+        float M2 = -INFINITY, L2 = 0.f;
+        cr_member_partial<ST, K_REG, K_LDS, false, NT>(g, s2, p, xr, rows_of(), wm, wl, M2, L2);
+        if (tid < 4 * CR_W && (tid & 3) == 0) { fb[0][tid >> 2] = M2; fb[1][tid >> 2] = L2; }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < CR_MPG; q++)
+            if (q < mpg && mgrp * mpg + q == p) { qm[q] = fb[0][mc]; ql[q] = fb[1][mc]; }
+        __syncthreads();
+    };
     __syncthreads();
     if (any_failed) {                                                // the same for every thread: read after the barrier
         if (tid == 0) atomicAdd(ws.fallbacks, 1);
-        for (int p = 0; p < csplit; p++) {
-            if (failed[p]) {
-                float M2 = -INFINITY, L2 = 0.f;
-                cr_member_partial<ST, false>(g, strip, p, xr, lrow, wm, wl, M2, L2);
-                if (tid < CR_W) { fb[0][tid] = M2; fb[1][tid] = L2; }
-                __syncthreads();
-#pragma unroll
-                for (int q = 0; q < CR_MPG; q++)
-                    if (q < mpg && mgrp * mpg + q == p) { pm[q] = fb[0][mc]; pl[q] = fb[1][mc]; }
-                __syncthreads();
-            }
+        for (int p = 0; p < csplit; p++)
+            if (failed[p]) recompute(strip, p, pm, pl);
+    }
+    cr_merge_members(pm, pl, wm, wl, fM, fInv);
+    // ---- the loss: a strip's leader forms the strip's term; wave 0 of workgroup 0 adds the terms in order, before its
+    // rows (behind them its loads would queue after the workgroup's stores, 2 us at the end of the launch)
+    if (tid < CR_W && me == 0) {
+        const float ls = cr_strip_loss(my_tgt, my_logit, fM[tid], fInv[tid]);
+        if (tid == 0)
+            __hip_atomic_store(ws.slots + (size_t)b * CR_STRIDE + CR_LOSS_SLOT,
+                               ((unsigned long long)my_tag << 32) | __float_as_uint(ls), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        if (strip == 0) {
+            float val = ls;
+            bool late = false;
+            if (tid > 0 && tid < strips)
+                late = take_nothing || !cr_wait_slot(ws.slots + (size_t)tid * CR_STRIDE + CR_LOSS_SLOT, t_lead, spin_ticks, val);
+            if (tid < strips) strip_loss[tid] = val;
+            if (late) { failed_loss[tid] = 1; any_failed_loss = 1; }
+            float total = 0.f;
+            for (int s2 = 0; s2 < strips; s2++) total += __shfl(val, s2, 64);
+            if (tid == 0) *loss_out = total / (float)S;              // (written again below if a term was late)
         }
     }
-    float Mc = 0.f, Lc = 1.f;
-    cr_merge_members(pm, pl, wm, wl, Mc, Lc);
-    if (tid < CR_W) {
-        const float inv = 1.0f / Lc;
-        fM[tid] = Mc;
-        fInv[tid] = inv;
-        if (me == 0) {                                               // the strip's leader also forms its loss term
-            const float ls = cr_strip_loss(g, strip, targets, Mc, inv);
-            if (tid == 0) {
-                strip_loss[strip] = ls;
-                __hip_atomic_store(ws.slots + (size_t)b * CR_STRIDE + CR_LOSS_SLOT,
-                                   ((unsigned long long)my_tag << 32) | __float_as_uint(ls), __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-            }
-        }
-    }
-    __syncthreads();
 
     // ---- pass 2: dlogits = (exp(l - M) / L - onehot) / S * grad_scale
     {
         const int lc = tid & 15;
         int row0 = tid >> 4;
         asm volatile("" : "+v"(row0));     // the row masks are formed again here instead of being kept from pass 1
-        const int v_lo = me * Rm;
-        constexpr int rs = CR_RPS;
-        const int lim = min(V, v_lo + Rm) - v_lo - row0;           // this lane's rows row0 + rs*k exist while rs*k < lim
-        const int kR = max(0, K - K_REG), kL = max(0, kR - K_LDS);
-        const typename ST::T *src = logits + ((size_t)v_lo * S + (size_t)strip * CR_W);
-        typename ST::T *dst = dlogits + ((size_t)v_lo * S + (size_t)strip * CR_W);
-        const unsigned loff = (unsigned)row0 * (unsigned)S + (unsigned)lc * 4u;
-        const size_t step = (size_t)rs * S;
+        const LaneCols mine = cr_cols(strip, sw, lc, S);
+        const CrRows r = cr_rows(g, me);
+        const int K = r.K, kR = max(0, K - K_REG), kL = max(0, kR - K_LDS);
+        const int mineK = !mine.ok ? 0 : row0 < r.last ? K : K - 1;      // steps in which this lane has a row to write
+        const typename ST::T *src = logits + (size_t)r.v_lo * S;
+        typename ST::T *dst = dlogits + (size_t)r.v_lo * S;
+        const unsigned loff = (unsigned)row0 * (unsigned)S + (unsigned)mine.col;
+        const size_t step = (size_t)CR_RPS * S;
         float M[4], inv[4], sc[4];
-        int tk[4];                         // the target's row is this lane's row 64k when tk == 64k
+        int tk[4];                         // the target's row is this lane's row of step k when tk == 64k
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             M[j] = fM[lc * 4 + j];
             inv[j] = fInv[lc * 4 + j];
-            const int tg = targets[strip * CR_W + lc * 4 + j];
+            const int tg = targets[mine.col + j];
             const bool ok = tg >= 0 && tg < V;
-            tk[j] = ok ? tg - v_lo - row0 : -1;
+            tk[j] = ok ? tg - r.v_lo - row0 : -1;
             sc[j] = ok ? invS : 1.0f;      // an out-of-range target leaves the column unscaled (stories_cpu_ops.h:98)
         }
         auto emit = [&](int k, const Raw &x) {
+            if (k >= mineK) return;
             float o[4];
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 float pj = exp_neg(ST::at(x, j) - M[j]) * inv[j];
-                if (tk[j] == rs * k) pj -= 1.0f;
-                pj = pj * sc[j];
-                if (grad_scale != 1.0f) pj = pj * grad_scale;
-                o[j] = pj;
+                if (tk[j] == CR_RPS * k) pj -= 1.0f;
+                o[j] = (pj * sc[j]) * grad_scale;
             }
-            ST::st_nt(dst + k * step + loff, o);
+            ST::template st<NT>(dst + k * step + loff, o);
         };
         // the rows read a second time run up to sixteen ahead of their use, in the registers that the register
         // rows leave as they are written out
         auto loadg = [&](Raw (&t)[CR_SUB], int k0) {
 #pragma unroll
             for (int u = 0; u < CR_SUB; u++)
-                if (k0 + u < kL && rs * (k0 + u) < lim) t[u] = ST::ld_nt(src + (k0 + u) * step + loff);
+                if (k0 + u < kL) t[u] = NT ? ST::ld_nt(src + (k0 + u) * step + loff) : ST::ld(src + (k0 + u) * step + loff);
         };
         auto emitg = [&](const Raw (&t)[CR_SUB], int k0) {
 #pragma unroll
             for (int u = 0; u < CR_SUB; u++)
-                if (k0 + u < kL && rs * (k0 + u) < lim) emit(k0 + u, t[u]);
+                if (k0 + u < kL) emit(k0 + u, t[u]);
         };
         Raw t0[CR_SUB], t1[CR_SUB], t2[CR_SUB], t3[CR_SUB];
-        loadg(t0, 0);
+        if constexpr (K_LDS > 0) loadg(t0, 0);
 #pragma unroll
         for (int i = 0; i < K_REG; i++) {
-            if (rs * (kR + i) < lim) emit(kR + i, xr[i]);
+            if (kR + i < K) emit(kR + i, xr[i]);
             __builtin_amdgcn_sched_barrier(0);       // one row at a time: the scheduler would otherwise hold them all
         }
-        loadg(t1, CR_SUB);
-        loadg(t2, 2 * CR_SUB);
-        loadg(t3, 3 * CR_SUB);
-#pragma unroll
-        for (int i = 0; i < K_LDS; i++) {
-            if (kL + i < kR && rs * (kL + i) < lim) emit(kL + i, lrow[i][tid]);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        for (int k0 = 0; k0 < kL; k0 += 4 * CR_SUB) {
-            emitg(t0, k0);
-            loadg(t0, k0 + 4 * CR_SUB);
-            emitg(t1, k0 + CR_SUB);
-            loadg(t1, k0 + 5 * CR_SUB);
-            emitg(t2, k0 + 2 * CR_SUB);
-            loadg(t2, k0 + 6 * CR_SUB);
-            emitg(t3, k0 + 3 * CR_SUB);
-            loadg(t3, k0 + 7 * CR_SUB);
+        if constexpr (K_LDS > 0) {
+            loadg(t1, CR_SUB);
+            loadg(t2, 2 * CR_SUB);
+            loadg(t3, 3 * CR_SUB);
+#pragma unroll 1
+            for (int i = 0; i < kR - kL; i++) emit(kL + i, rows_of()[i][tid]);
+            for (int k0 = 0; k0 < kL; k0 += 4 * CR_SUB) {
+                emitg(t0, k0);
+                loadg(t0, k0 + 4 * CR_SUB);
+                emitg(t1, k0 + CR_SUB);
+                loadg(t1, k0 + 5 * CR_SUB);
+                emitg(t2, k0 + 2 * CR_SUB);
+                loadg(t2, k0 + 6 * CR_SUB);
+                emitg(t3, k0 + 3 * CR_SUB);
+                loadg(t3, k0 + 7 * CR_SUB);
+            }
         }
     }
 
-    // ---- the loss: workgroup 0 adds the strips' terms in order; by now the other leaders have long published
+    // a strip's loss term that did not arrive: from memory, the same way
     if (b == 0) {
         __syncthreads();
-        if (tid < strips) failed[tid] = 0;
-        __syncthreads();
-        if (tid > 0 && tid < strips) {
-            float val = 0.f;
-            if (take_nothing || !cr_wait_slot(ws.slots + (size_t)tid * CR_STRIDE + CR_LOSS_SLOT, want_leader[tid], spin_ticks, val))
-                failed[tid] = 1;
-            strip_loss[tid] = val;
-        }
-        __syncthreads();
-        for (int s2 = 1; s2 < strips; s2++) {
-            if (failed[s2]) {                                        // that strip's loss term from memory, the same way
-                float qm[CR_MPG], ql[CR_MPG];
+        if (any_failed_loss) {
+            for (int s2 = 1; s2 < strips; s2++) {
+                if (failed_loss[s2]) {
+                    float qm[CR_MPG], ql[CR_MPG];
 #pragma unroll
-                for (int q = 0; q < CR_MPG; q++) { qm[q] = -INFINITY; ql[q] = 0.f; }
-                for (int p = 0; p < csplit; p++) {
-                    float M2 = -INFINITY, L2 = 0.f;
-                    cr_member_partial<ST, false>(g, s2, p, xr, lrow, wm, wl, M2, L2);
-                    if (tid < CR_W) { fb[0][tid] = M2; fb[1][tid] = L2; }
-                    __syncthreads();
-#pragma unroll
-                    for (int q = 0; q < CR_MPG; q++)
-                        if (q < mpg && mgrp * mpg + q == p) { qm[q] = fb[0][mc]; ql[q] = fb[1][mc]; }
+                    for (int q = 0; q < CR_MPG; q++) { qm[q] = -INFINITY; ql[q] = 0.f; }
+                    for (int p = 0; p < csplit; p++) recompute(s2, p, qm, ql);
+                    cr_merge_members(qm, ql, wm, wl, fM, fInv);
+                    if (tid < CR_W) {
+                        const int tg = cr_slot_target(g, s2, targets);
+                        const float ls = cr_strip_loss(tg, cr_slot_logit(g, s2, tg), fM[tid], fInv[tid]);
+                        if (tid == 0) strip_loss[s2] = ls;
+                    }
                     __syncthreads();
                 }
-                float M3 = 0.f, L3 = 1.f;
-                cr_merge_members(qm, ql, wm, wl, M3, L3);
-                if (tid < CR_W) {
-                    const float ls = cr_strip_loss(g, s2, targets, M3, 1.0f / L3);
-                    if (tid == 0) strip_loss[s2] = ls;
-                }
-                __syncthreads();
             }
-        }
-        if (tid == 0) {
-            float total = 0.f;
-            for (int s2 = 0; s2 < strips; s2++) total += strip_loss[s2];
-            *loss_out = total / (float)S;
+            if (tid == 0) {
+                float total = 0.f;
+                for (int s2 = 0; s2 < strips; s2++) total += strip_loss[s2];
+                *loss_out = total / (float)S;
+            }
         }
     }
     if (tid == 0) ws.cnt[b] = my_tag;
@@ -921,22 +961,21 @@ int ce_run(const char *who, T *dlogits, float *loss_dev, const T *logits, const 
     if (!mi355_ready(who)) return -1;
     if (!dlogits || !loss_dev || !logits || !targets) return mi355_fail("%s: NULL pointer", who);
     if (V <= 0 || S <= 0) return mi355_fail("%s: bad shape V=%d S=%d", who, V, S);
-    // Rows per workgroup: one to six 64-row register tiles, chosen so that the workgroups of a column strip fill the
-    // compute units evenly (at least 1.75 per unit, and the last round of them as full as possible); ties go to
-    // the larger block, which leaves fewer partials to merge.  At V = 151936 on 256 units: 320 rows, 475
-    // workgroups (87 us for the op; 256 rows and 594 workgroups: 91 us; 384 rows and 396: 97 us).
     {
-        // The one-launch form: whole 64-column strips, a lane's four columns in one aligned access, out of place (a
-        // member that recomputes a partner's partial reads the partner's logits), and a vocabulary for which it
-        // pays (ce_resident: 0 = V >= 4096, 1 = any V, -1 = never).  One workgroup per compute unit at most, so that
-        // all of them are resident at once.
+        // The one-launch form: rows of 4 to 1024 columns, split into strips of at most 64, out of place (a member that
+        // recomputes a partner's partial reads the partner's logits).  One workgroup per compute unit at most, so that
+        // all of them are resident at once.  Measured against the three launches, us: fp32 [1000][256] 8.6 against 20
+        // (12 with one column per lane), [32000][256] 18.3 against 27, [151936][256] 65.7 against 83, [32000][1000] 71
+        // against 88; bfloat16 [32000][200] 15.3 against 31.6, [151936][256] 49 against 88.  Only a single strip of a
+        // large vocabulary, which occupies 64 of the compute units, is close: fp32 [151936][63] 42 against 38.
         typedef typename std::conditional<std::is_same<T, float>::value, CrF32, CrBf16>::type ST;
         const int cu = g_ctx.num_cu > 0 ? g_ctx.num_cu : 256;
-        const int strips_r = S / CR_W;
-        const uintptr_t amask = 4 * sizeof(T) - 1;
+        const int strips_r = (int)ceil_div((size_t)S, (size_t)CR_W);
+        // rows of whole 128-byte lines: strips of 64 columns past the caches; other rows: strips of equal width
+        const bool lines = ((size_t)S * sizeof(T)) % 128 == 0;
+        const int sw = lines ? CR_W : 4 * (int)ceil_div((size_t)S, 4 * (size_t)strips_r);
         unsigned char *base = (g_ctx.device >= 0 && g_ctx.device < CE_MAX_DEVICES) ? g_scratch_ptr[g_ctx.device] : nullptr;
-        if (g_ctx.ce_resident >= 0 && base && S % CR_W == 0 && strips_r <= CR_MAX_STRIPS && (const void *)dlogits != (const void *)logits &&
-            (((uintptr_t)logits | (uintptr_t)dlogits) & amask) == 0 && (V >= 4096 || g_ctx.ce_resident > 0)) {
+        if (g_ctx.ce_resident >= 0 && base && S >= 4 && strips_r <= CR_MAX_STRIPS && (const void *)dlogits != (const void *)logits) {
             const int csplit = cu / strips_r < CR_MAX_SPLIT ? cu / strips_r : CR_MAX_SPLIT;
             const int Rm = csplit > 0 ? (int)ceil_div((size_t)V, (size_t)csplit) : 0;
             const int K = (int)ceil_div((size_t)Rm, (size_t)CR_RPS);
@@ -945,15 +984,25 @@ int ce_run(const char *who, T *dlogits, float *loss_dev, const T *logits, const 
                 xch.slots = (unsigned long long *)(base + CE_SCRATCH_BYTES);
                 xch.cnt = (unsigned *)(base + CE_SCRATCH_BYTES + (size_t)CR_MAX_WG * CR_STRIDE * 8);
                 xch.fallbacks = (int *)(base + CE_SCRATCH_BYTES + (size_t)CR_MAX_WG * CR_STRIDE * 8 + (size_t)CR_MAX_WG * 4);
-                hipLaunchKernelGGL((ce_resident_kernel<ST, true>), dim3((unsigned)(csplit * strips_r)), dim3(CR_THREADS), 0,
-                                   g_ctx.stream, dlogits, logits, targets, V, S, strips_r, csplit, Rm, K, 1.0f / (float)S,
-                                   grad_scale, loss_dev, xch, mi355_exchange_spin_ticks() < 0 ? 0 : mi355_exchange_spin_ticks(),
-                                   g_ctx.xch_take_nothing > 0 ? 1 : 0);
+                auto launch = [&](auto kernel) {
+                    const int spin = mi355_exchange_spin_ticks();
+                    hipLaunchKernelGGL(kernel, dim3((unsigned)(csplit * strips_r)), dim3(CR_THREADS), 0, g_ctx.stream, dlogits,
+                                       logits, targets, V, S, strips_r, sw, csplit, Rm, 1.0f / (float)S, grad_scale, loss_dev,
+                                       xch, spin < 0 ? 0 : spin, g_ctx.xch_take_nothing > 0 ? 1 : 0);
+                };
+                if (K <= 8) { if (lines) launch(ce_resident_kernel<ST, 8, 0, true>); else launch(ce_resident_kernel<ST, 8, 0, false>); }
+                else if (K <= 16) { if (lines) launch(ce_resident_kernel<ST, 16, 0, true>); else launch(ce_resident_kernel<ST, 16, 0, false>); }
+                else if (lines) launch(ce_resident_kernel<ST, ST::K_REG, ST::K_LDS, true>);
+                else launch(ce_resident_kernel<ST, ST::K_REG, ST::K_LDS, false>);
                 LAUNCH_OK("softmax_ce (one launch)");
                 return 0;
             }
         }
     }
+    // Rows per workgroup: one to six 64-row register tiles, chosen so that the workgroups of a column strip fill the
+    // compute units evenly (at least 1.75 per unit, and the last round of them as full as possible); ties go to
+    // the larger block, which leaves fewer partials to merge.  At V = 151936 on 256 units: 320 rows, 475
+    // workgroups (87 us for the op; 256 rows and 594 workgroups: 91 us; 384 rows and 396: 97 us).
     int rpb = g_ctx.ce_rows;
     if (rpb <= 0) {
         const int cu = g_ctx.num_cu > 0 ? g_ctx.num_cu : 256;
@@ -985,9 +1034,10 @@ int ce_run(const char *who, T *dlogits, float *loss_dev, const T *logits, const 
         }
     }
     const int nblk2 = (int)ceil_div((size_t)V, (size_t)rpb2);
-    // four columns per lane: 16 bytes of fp32, 8 bytes of bf16
-    const uintptr_t mask = 4 * sizeof(T) - 1;
-    const bool vec_ok = (S % 4 == 0) && (((uintptr_t)logits | (uintptr_t)dlogits) & mask) == 0;
+    // Four columns per lane where the matrix is large enough to fill the chip with the quarter of the lanes and a row is
+    // wide enough for the 256 columns of a wave: [16384][256] 22.1 us so against 18.8 with one column per lane,
+    // [32000][256] 27.0 against 28.8, [32000][500] 50 against 66.
+    const bool vec_ok = S % 4 == 0 && S >= 160 && (size_t)V * S >= 6000000;
     const int vec = vec_ok ? 4 : 1;
     const int strips = (int)ceil_div((size_t)S, (size_t)64 * vec);
     if (strips > 65535) return mi355_fail("%s: S too large", who);
@@ -1060,7 +1110,7 @@ MI355_API int mi355_softmax_cols_dev(float *probs, const float *logits, int V, i
     if (V <= 0 || S <= 0) return mi355_fail("softmax_cols: bad shape V=%d S=%d", V, S);
     const int rpb = 4 * CE_TILE_ROWS;
     const int nblk = (int)ceil_div((size_t)V, (size_t)rpb);
-    const bool vec_ok = (S % 4 == 0) && aligned16(logits) && aligned16(probs);
+    const bool vec_ok = S % 4 == 0;
     const int vec = vec_ok ? 4 : 1;
     const int strips = (int)ceil_div((size_t)S, (size_t)64 * vec);
     if (strips > 65535) return mi355_fail("softmax_cols: S too large");
@@ -1091,7 +1141,7 @@ MI355_API int mi355_nll_from_probs_dev(float *dlogits, float *loss_dev, const fl
     const size_t n = (size_t)V * S;
     hipLaunchKernelGGL(nll_loss_kernel, dim3(1), dim3(CE_THREADS), 0, g_ctx.stream, loss_dev, probs, targets, V, S);
     LAUNCH_OK("nll_from_probs loss");
-    const bool vec_ok = (S % 4 == 0) && aligned16(probs) && aligned16(dlogits);
+    const bool vec_ok = S % 4 == 0;
     if (vec_ok)
         hipLaunchKernelGGL(nll_grad_kernel<4>, dim3((unsigned)ceil_div(n / 4, 256)), dim3(256), 0, g_ctx.stream, dlogits,
                            probs, targets, V, S, n, 1.0f / (float)S);

@@ -65,7 +65,7 @@ size_t mi355_workspace_size(void);
  * 0 = a multiple of 128 bytes that rotates from one allocation to the next, 1..8 = always (value-1)*128),
  * "rms_cluster" (channel split of the RMSNorm over cooperating workgroups: -1 = never, and mi355_int8_scale_dev and
  * mi355_int8_quantize_dynamic_dev then run as two launches each; 2/4/8 = forced),
- * "ce_resident" (one-launch softmax-CE: 1 = for any V, -1 = never), "rms_cluster_spin" (how long a workgroup of those
+ * "ce_resident" (one-launch softmax-CE: -1 = never), "rms_cluster_spin" (how long a workgroup of those
  * kernels and of mi355_int8_scale_dev waits for a partner's partial result before it computes it itself, in ticks
  * of 10 ns: 0 = 2 ms; -1 = do not wait), "xch_take_nothing" (1: those kernels take no partner's value at
  * all, present or not, so every workgroup goes the way of an expired wait).  The last two settings are for tests: the
@@ -298,12 +298,12 @@ int mi355_embed_scatter_add_form(int V, int D, int S, int batch, int aligned);
  * dlogits = (softmax - onehot) * (1/S) * grad_scale; *loss_dev = mean_t -logf(p[tgt]+1e-10f).
  * A target outside [0,V) contributes no loss and leaves its column as the unscaled softmax
  * (stories_cpu_ops.h:98).  dlogits may alias logits.
- * Logits with S a multiple of 64 (at most 1024), V >= 4096, 16-byte aligned and not in place run as ONE launch
+ * Logits of 4 to 1024 columns that are not overwritten in place run as ONE launch
  * that keeps the logits in registers and LDS between the two passes (one workgroup per compute unit; partial
  * sums exchanged inside the launch through a device array of the library, bounded wait as for the RMSNorm); every
  * other call runs as three launches that read the logits twice.  Both forms are deterministic; they sum in
- * different orders, so their results differ in the last bits.  Tuning knob "ce_resident": 0 = as described,
- * 1 = the one-launch form for any V, -1 = never. */
+ * different orders, so their results differ in the last bits.  Tuning knob "ce_resident": 0 or 1 = as described,
+ * -1 = never the one-launch form. */
 int mi355_softmax_ce_dev(float *dlogits, float *loss_dev, const float *logits,
                          const int32_t *targets, int V, int S, float grad_scale);
 
