@@ -138,7 +138,6 @@ MI355_API int mi355_init(void) {
 
 void mi355_free_caches(void);   // rope tables, host drop-in staging (other translation units)
 void mi355_dw_free(void);       // queued weight-gradient reductions and their arena
-void mi355_blas_free(void);     // rocBLAS handle of mi355_sgemm_dev
 void mi355_ckpt_free(void);     // pinned staging buffer of the checkpoint reader/writer
 void mi355_graph_shutdown(void);  // capture stream
 
@@ -147,7 +146,6 @@ MI355_API void mi355_shutdown(void) {
     (void)hipDeviceSynchronize();
     mi355_free_caches();
     mi355_dw_free();
-    mi355_blas_free();
     mi355_ckpt_free();
     mi355_graph_shutdown();
     if (g_xch.slots) (void)hipFree(g_xch.slots);

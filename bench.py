@@ -795,7 +795,7 @@ def bench_aux(br, args):
                                                              0, 0, 0, heads, kvh, hd, S, B, cosd, sind))
                  for j, t in enumerate(trip)],
         3 * 2 * nq + 4 * nq + 2 * kb, len(trip))
-    # classifier products on the compact vocabulary (train.m:490-508), fp32 through rocBLAS: flops, not bytes
+    # classifier products on the compact vocabulary (train.m:490-508), fp32: flops, not bytes
     xf, dyc = A((D, S)), A((D, S))
     br.check(br.lib.mi355_fill_normal_dev(xf.ptr, xf.size, 60, 0.0, 1.0))
     logit, dlog = A((CV, S)), A((CV, S))

@@ -404,7 +404,7 @@ int mi355_attn_grads_finish_dev(float *dq, float *dk, float *dv, const void *dq_
  * the classifier products training/training_dynamic/train.m:490-491 (logits), :501-502 (dy), :507-508 (gcembed +=)
  * and the weight-gradient products :577-581, :613, :681-685.  Same argument order and meaning as the cblas call
  * without the layout argument (always row-major); trans flags take 0/1 or CblasNoTrans/CblasTrans (111/112).
- * Runs on the bridge stream through rocBLAS, which is opened on the first call. */
+ * fp32 products and sums on the matrix cores, deterministic (K slices are added in order). */
 int mi355_sgemm_dev(int trans_a, int trans_b, int M, int N, int K, float alpha, const float *A, int lda,
                     const float *B, int ldb, float beta, float *C, int ldc);
 
