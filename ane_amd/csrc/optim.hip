@@ -9,6 +9,7 @@
 #include "common.h"
 
 #include <math.h>
+#include <algorithm>
 
 namespace {
 
@@ -105,49 +106,90 @@ __global__ __launch_bounds__(OPT_THREADS) void adam_kernel(float *__restrict__ w
     }
 }
 
-// ---- several tensors per launch: blockIdx.y selects the tensor ----
-constexpr int MT_MAX = 16;
+// ---- many tensors per launch ----
+// The blocks of all tensors of a launch are numbered through: tensor i owns the blocks first[i] .. first[i + 1] - 1.
+// A grid of (blocks of the largest tensor) x (tensors) is mostly empty workgroups where sizes differ: the 110 M
+// parameters of 12 layers and an embedding started 460 000 workgroups for 108 000 that had work.
+constexpr int MT_MAX = 64;                  // 3.1 KB of kernel arguments (4 KB is the most a launch takes)
+constexpr int SQ_V4 = 8;                    // 128-bit loads of a lane of the norm, all in flight together
+struct MtFirst {
+    unsigned first[MT_MAX];                 // 2^32 - 1 behind the last tensor
+};
 struct MtSumsq {
+    MtFirst blk;
     const float *g[MT_MAX];
     size_t n[MT_MAX];
 };
 struct MtAdam {
+    MtFirst blk;
     float *w[MT_MAX], *g[MT_MAX], *m[MT_MAX], *v[MT_MAX];
     size_t n[MT_MAX];
     float wd[MT_MAX];
 };
 
-// partials laid out [tensor][gridDim.x]; every tensor uses the same fixed grid, so the sum is deterministic
-__global__ __launch_bounds__(OPT_THREADS) void sumsq_partial_mt_kernel(float *__restrict__ part, MtSumsq a, float pre) {
+// The tensor that owns a block: two rounds of eight comparisons on scalar registers, two trips to the scalar cache
+// (a search by halves would be six dependent trips ahead of the first load of data).
+__device__ __forceinline__ int mt_owner(const MtFirst &f, unsigned block) {
+    int g = 0;
+#pragma unroll
+    for (int j = 1; j < MT_MAX / 8; j++) g += block >= f.first[8 * j] ? 1 : 0;
+    int i = 0;
+#pragma unroll
+    for (int j = 1; j < 8; j++) i += block >= f.first[8 * g + j] ? 1 : 0;
+    return 8 * g + i;
+}
+
+// One partial per block, in block order.  Bound by the read of g (110 M floats: 438 MB).  The loads are ordinary ones,
+// so that the end of g is in the 256 MB last-level cache when the update, which walks the blocks from the last to the
+// first, asks for it.  Norm + clip + update of the 110 M parameters (109 tensors, 3.5 GB besides the norm's read):
+// 748 us with one launch per 16 tensors of (largest tensor) x (tensors) blocks and a sum after each, 707 with the
+// blocks numbered through, 700 with the update backwards, 650 with these loads not marked as streaming.  Which elements a block sums depends on the sizes alone, so the sum is
+// deterministic.
+__global__ __launch_bounds__(OPT_THREADS) void sumsq_partial_mt_kernel(float *__restrict__ part, MtSumsq a, float pre,
+                                                                       int rounds) {
     __shared__ float red[OPT_THREADS / 64];
-    const float *__restrict__ g = a.g[blockIdx.y];
-    const size_t n = a.n[blockIdx.y], n4 = n / 4;
+    const int ti = mt_owner(a.blk, blockIdx.x);
+    const float *__restrict__ g = a.g[ti];
+    const size_t n = a.n[ti], n4 = n / 4;
+    size_t i0 = (size_t)(blockIdx.x - a.blk.first[ti]) * rounds * (OPT_THREADS * SQ_V4) + threadIdx.x;
     float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
-    const size_t tid = (size_t)blockIdx.x * OPT_THREADS + threadIdx.x;
-    const size_t stride = (size_t)gridDim.x * OPT_THREADS;
-    for (size_t i = tid; i < n4; i += stride) {
-        v4f v = ld4_nt(g + 4 * i) * pre;
-        s0 += v.x * v.x; s1 += v.y * v.y; s2 += v.z * v.z; s3 += v.w * v.w;
+    for (int r = 0; r < rounds; r++, i0 += OPT_THREADS * SQ_V4) {
+        v4f v[SQ_V4];
+#pragma unroll
+        for (int k = 0; k < SQ_V4; k++) {
+            const size_t i = i0 + (size_t)k * OPT_THREADS;
+            v[k] = i < n4 ? ld4(g + 4 * i) : v4f{0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll
+        for (int k = 0; k < SQ_V4; k++) {
+            const v4f t = v[k] * pre;
+            s0 += t.x * t.x; s1 += t.y * t.y; s2 += t.z * t.z; s3 += t.w * t.w;
+        }
+#pragma unroll
+        for (int k = 0; k < SQ_V4; k++)
+            if (i0 + (size_t)k * OPT_THREADS == n4)              // the lane behind the last whole group
+                for (size_t j = 4 * n4; j < n; j++) { const float t = g[j] * pre; s0 += t * t; }
     }
-    if (blockIdx.x == 0)
-        for (size_t i = n4 * 4 + threadIdx.x; i < n; i += OPT_THREADS) { float t = g[i] * pre; s0 += t * t; }
     float s = (s0 + s1) + (s2 + s3);
     s = wave_sum_far_first(s);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
     __syncthreads();
-    if (threadIdx.x == 0) part[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+    if (threadIdx.x == 0) part[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
+// Bound by its eight streams (16 B read, 16 B written per parameter with ZERO, at the 5.6 TB/s of a copy).  1024-thread
+// workgroups 705 us, plain stores 725, g read and cleared with ordinary accesses 698 (norm + clip + update, against 650).
 template <bool ZERO>
 __global__ __launch_bounds__(OPT_THREADS) void adam_mt_kernel(MtAdam a, float lr, float b1, float b2, float eps,
                                                               float bc1, float bc2, float scale1,
                                                               const float *__restrict__ scale2_p) {
-    const size_t n = a.n[blockIdx.y], n4 = n / 4;
-    const size_t i = (size_t)blockIdx.x * OPT_THREADS + threadIdx.x;
-    if (i >= n4 && !(blockIdx.x == 0 && threadIdx.x < n - n4 * 4)) return;
-    float *__restrict__ w = a.w[blockIdx.y], *__restrict__ g = a.g[blockIdx.y];
-    float *__restrict__ m = a.m[blockIdx.y], *__restrict__ v = a.v[blockIdx.y];
-    const float wd = a.wd[blockIdx.y];
+    const unsigned block = gridDim.x - 1 - blockIdx.x;
+    const int ti = mt_owner(a.blk, block);
+    const size_t n = a.n[ti], n4 = n / 4;
+    const size_t i = (size_t)(block - a.blk.first[ti]) * OPT_THREADS + threadIdx.x;
+    float *__restrict__ w = a.w[ti], *__restrict__ g = a.g[ti];
+    float *__restrict__ m = a.m[ti], *__restrict__ v = a.v[ti];
+    const float wd = a.wd[ti];
     const float scale2 = scale2_p ? *scale2_p : 1.0f;
     const float omb1 = 1.0f - b1, omb2 = 1.0f - b2;
     if (i < n4) {
@@ -163,13 +205,29 @@ __global__ __launch_bounds__(OPT_THREADS) void adam_mt_kernel(MtAdam a, float lr
         st4_nt(m + 4 * i, mv);
         st4_nt(v + 4 * i, vv);
         if (ZERO) { const v4f z4 = {0.f, 0.f, 0.f, 0.f}; st4_nt(g + 4 * i, z4); }
+    } else if (i == n4) {
+        for (size_t k = 4 * n4; k < n; k++) {                    // fewer than four are left
+            const float gg = (g[k] * scale1) * scale2;
+            adam1(w[k], m[k], v[k], gg, lr, b1, b2, omb1, omb2, eps, wd, bc1, bc2);
+            if (ZERO) g[k] = 0.f;
+        }
     }
-    if (blockIdx.x == 0 && threadIdx.x < n - n4 * 4) {
-        const size_t k = n4 * 4 + threadIdx.x;
-        float gg = (g[k] * scale1) * scale2;
-        adam1(w[k], m[k], v[k], gg, lr, b1, b2, omb1, omb2, eps, wd, bc1, bc2);
-        if (ZERO) g[k] = 0.f;
+}
+
+// The block table of the first tensors of a list, `per` 128-bit groups to a block (one more group where a tensor ends
+// within one): as many as one launch holds (MT_MAX, and fewer than 2^32 threads).  Returns how many; `blocks`: theirs.
+int mt_blocks(MtFirst &f, unsigned &blocks, const size_t *n, int count, size_t per) {
+    size_t total = 0;
+    int k = 0;
+    for (; k < count && k < MT_MAX; k++) {
+        const size_t more = ceil_div(ceil_div(n[k], (size_t)4), per);
+        if (total + more >= ((size_t)1 << 32) / OPT_THREADS) break;
+        f.first[k] = (unsigned)total;
+        total += more;
     }
+    for (int i = k; i < MT_MAX; i++) f.first[i] = 0xffffffffu;
+    blocks = (unsigned)total;
+    return k;
 }
 
 }   // namespace
@@ -180,20 +238,26 @@ MI355_API int mi355_sumsq_accum_multi_dev(float *acc_dev, const float *const *g,
     if (!acc_dev || !g || !n || count <= 0) return mi355_fail("sumsq_accum_multi: bad arguments");
     for (int i = 0; i < count; i++)
         if (!g[i] || n[i] == 0 || !aligned16(g[i])) return mi355_fail("sumsq_accum_multi: tensor %d is NULL, empty or not 16-byte aligned", i);
-    for (int i0 = 0; i0 < count; i0 += MT_MAX) {
-        const int k = count - i0 < MT_MAX ? count - i0 : MT_MAX;
+    // from 134 M elements on a block takes several rounds, so that the partials stay near 64 KB
+    size_t all = 0, total = 0, done = 0;
+    for (int i = 0; i < count; i++) all += n[i] / 4;
+    const int rounds = (int)std::min<size_t>(ceil_div(all + 1, (size_t)OPT_THREADS * SQ_V4 * 16384), 1u << 30);
+    const size_t per = (size_t)OPT_THREADS * SQ_V4 * rounds;
+    for (int i = 0; i < count; i++) total += ceil_div(ceil_div(n[i], (size_t)4), per);
+    float *part = (float *)mi355_ws(total * sizeof(float));
+    if (!part) return -1;
+    for (int i0 = 0, k = 0; i0 < count; i0 += k) {
         MtSumsq a = {};
-        size_t nmax = 0;
-        for (int i = 0; i < k; i++) { a.g[i] = g[i0 + i]; a.n[i] = n[i0 + i]; if (n[i0 + i] > nmax) nmax = n[i0 + i]; }
-        size_t blocks = ceil_div(nmax / 4 + 1, (size_t)OPT_THREADS * 4);
-        if (blocks > 1024) blocks = 1024;
-        float *part = (float *)mi355_ws((size_t)k * blocks * sizeof(float));
-        if (!part) return -1;
-        hipLaunchKernelGGL(sumsq_partial_mt_kernel, dim3((unsigned)blocks, (unsigned)k), dim3(OPT_THREADS), 0, g_ctx.stream,
-                           part, a, pre_scale);
-        hipLaunchKernelGGL(sumsq_final_kernel, dim3(1), dim3(1024), 0, g_ctx.stream, acc_dev, part, (int)(k * blocks));
-        LAUNCH_OK("sumsq_accum_multi");
+        unsigned blocks;
+        k = mt_blocks(a.blk, blocks, n + i0, count - i0, per);
+        if (!k) return mi355_fail("sumsq_accum_multi: tensor %d is too large for one launch", i0);
+        for (int i = 0; i < k; i++) { a.g[i] = g[i0 + i]; a.n[i] = n[i0 + i]; }
+        hipLaunchKernelGGL(sumsq_partial_mt_kernel, dim3(blocks), dim3(OPT_THREADS), 0, g_ctx.stream, part + done, a, pre_scale,
+                           rounds);
+        done += blocks;
     }
+    hipLaunchKernelGGL(sumsq_final_kernel, dim3(1), dim3(1024), 0, g_ctx.stream, acc_dev, part, (int)total);
+    LAUNCH_OK("sumsq_accum_multi");
     return 0;
 }
 
@@ -207,16 +271,16 @@ MI355_API int mi355_adam_update_multi_dev(float *const *w, float *const *g, floa
             !aligned16(v[i]))
             return mi355_fail("adam_update_multi: tensor %d is NULL, empty or not 16-byte aligned", i);
     const float bc1 = 1.0f - powf(b1, (float)t), bc2 = 1.0f - powf(b2, (float)t);
-    for (int i0 = 0; i0 < count; i0 += MT_MAX) {
-        const int k = count - i0 < MT_MAX ? count - i0 : MT_MAX;
+    for (int i0 = 0, k = 0; i0 < count; i0 += k) {
         MtAdam a = {};
-        size_t nmax = 0;
+        unsigned blocks;
+        k = mt_blocks(a.blk, blocks, n + i0, count - i0, OPT_THREADS);
+        if (!k) return mi355_fail("adam_update_multi: tensor %d is too large for one launch", i0);
+        const dim3 grid(blocks);
         for (int i = 0; i < k; i++) {
             a.w[i] = w[i0 + i]; a.g[i] = g[i0 + i]; a.m[i] = m[i0 + i]; a.v[i] = v[i0 + i];
             a.n[i] = n[i0 + i]; a.wd[i] = wd[i0 + i];
-            if (n[i0 + i] > nmax) nmax = n[i0 + i];
         }
-        const dim3 grid((unsigned)ceil_div(nmax / 4 + 1, (size_t)OPT_THREADS), (unsigned)k);
         if (zero_grad)
             hipLaunchKernelGGL((adam_mt_kernel<true>), grid, dim3(OPT_THREADS), 0, g_ctx.stream, a, lr, b1, b2, eps, bc1,
                                bc2, scale1, scale2_dev);
