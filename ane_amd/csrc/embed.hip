@@ -849,50 +849,67 @@ MI355_API int mi355_embed_gather_dev(float *x, const float *E, const int32_t *id
 
 // Which form takes an input of N positions and row width D.  Both forms give the same bits, so the choice is only a
 // matter of time, and what decides it is how the ids repeat: the column form pays one small access to dE per
-// (token, block of 8192 positions) and workgroup, the row form a token-major copy of dx whatever the ids are.  Ids of
-// text repeat (config 2: 4621 pairs in 16384 positions) and the column form is the default; for ids that hardly
-// repeat (drawn uniformly from a large vocabulary) it is up to twice as slow.  The ids are on the device, so the
-// library learns from the previous call: the last kernel of either form leaves its number of runs in a word of
-// pinned host memory, and the next call of the same N and D compares it with the number at which the two forms
-// cost the same (fitted to measurements: column form 10 + 2.5 per block + 4.9 ns per pair, row form
-// 24 + 1.4e-6 N D, in us).  The row form reports distinct tokens, not pairs; how many pairs a token makes is taken
-// from the last time both forms saw this shape (1.2, config 2's figure, until then), so that a steady input settles
-// on one form instead of alternating.
+// (token, block of 8192 positions) and workgroup, the row form a token-major copy of dx whatever the ids are, and beyond
+// 16384 positions (or a vocabulary of 2^18) the library sort.  Ids of text repeat (16384 Zipf-distributed ids of a
+// vocabulary of 32000: 4621 pairs); ids that hardly repeat (drawn uniformly from a large vocabulary) take up to twice as
+// long in columns.  The ids are on the device, so the library learns from the previous call of the same N and D: the last
+// kernel of either form leaves its number of runs in a word of pinned host memory, and the next call compares it with the
+// number at which the two forms cost the same.  Fitted to measurements, in us:
+//   up to 16384 positions  columns 10 + 2.5 per block + 4.9 ns per pair   rows 24 + 1.4e-6 N D
+//   with the library sort  columns  5 + 1.2e-6 N D + 5.0 ns per pair      rows 54 + 2.8e-6 N D
+// (20480 to 65536 positions, D = 768 and 1024, 14 % to 97 % pairs: [1000 x 40][1024] of 151936 Zipf-distributed ids 106
+// against 175, drawn uniformly 227 against 198).  Before the first report whole sequences of up to 16384 positions take
+// the columns, everything else the rows.  The row form reports distinct tokens, not pairs; how many pairs a token makes
+// is taken from the last time both forms saw this shape (1.2 until then), so that a steady input settles on one form
+// instead of alternating.
 namespace {
+constexpr int REPORT_WORDS = 8;                // of 8 bytes, a shape's own by its N and D: programs alternate between shapes
+constexpr int COLS_MAX_N = 65536;              // as far as the two lines above are measured
 unsigned long long *g_report = nullptr;        // pinned, written by the device
 unsigned long long *g_report_dev = nullptr;
 int g_cols_runs = 0, g_cols_N = 0, g_cols_D = 0;   // the column form's last report
 double g_pairs_per_token = 1.2;
 
-unsigned long long *scatter_report_word(void) {
+int report_word_of(int N, int D) { return (int)((((unsigned)N * 2654435761u) ^ ((unsigned)D * 2246822519u)) >> 29); }
+static_assert(REPORT_WORDS == 8, "the three top bits of the product");
+
+// The device address of a shape's word, NULL where there is none (its fields hold 20 bits).
+unsigned long long *scatter_report_word(int N, int D) {
     if (!g_report && !g_ctx.capturing) {
         void *h = nullptr, *d = nullptr;
-        if (hipHostMalloc(&h, 64, hipHostMallocMapped) == hipSuccess && hipHostGetDevicePointer(&d, h, 0) == hipSuccess) {
+        if (hipHostMalloc(&h, REPORT_WORDS * 8, hipHostMallocMapped) == hipSuccess &&
+            hipHostGetDevicePointer(&d, h, 0) == hipSuccess) {
             g_report = (unsigned long long *)h;
             g_report_dev = (unsigned long long *)d;
-            *(volatile unsigned long long *)g_report = 0ull;
+            for (int i = 0; i < REPORT_WORDS; i++) ((volatile unsigned long long *)g_report)[i] = 0ull;
         } else {
             if (h) (void)hipHostFree(h);
             (void)hipGetLastError();
         }
     }
-    return g_report_dev;
+    return g_report_dev && N < (1 << 20) && D < (1 << 20) ? g_report_dev + report_word_of(N, D) : nullptr;
 }
 
-// 1: columns of dE owned by workgroups, -1: token-major copy and row sums.  `cols_ok`: the column form can take the call.
-int scatter_form(int N, int D, bool cols_ok, bool rows_recordable) {
+// 1: columns of dE owned by workgroups, -1: token-major copy and row sums.  `cols_ok`: the column form can take the call;
+// `whole`: its sequences are a multiple of four positions and 16-byte aligned; `rows_recordable`: the row form sorts the
+// ids itself (the library sort is slower and cannot be recorded).
+int scatter_form(int N, int D, bool cols_ok, bool whole, bool rows_recordable) {
     if (!cols_ok) return -1;
+    if (g_ctx.capturing && !rows_recordable) return whole ? 1 : -1;
     if (g_ctx.scatter_cols > 0) return 1;
-    if (g_ctx.capturing && !rows_recordable) return 1;
     const int cu = g_ctx.num_cu > 0 ? g_ctx.num_cu : 256;
-    if (N > SMALL_N || (int)ceil_div((size_t)D, cols_per_workgroup(D)) > cu) return -1;
-    if (N <= COL_SMALL || !g_report) return 1;
-    const unsigned long long w = *(volatile unsigned long long *)g_report;
+    if (N > COLS_MAX_N || (int)ceil_div((size_t)D, cols_per_workgroup(D)) > cu) return -1;
+    if (N <= COL_SMALL) return 1;
+    const int unknown = whole && N <= SMALL_N ? 1 : -1;
+    if (!g_report) return unknown;
+    const unsigned long long w = ((volatile unsigned long long *)g_report)[report_word_of(N, D)];
     const int form = (int)(w >> 60), rD = (int)((w >> 40) & 0xfffffu), rN = (int)((w >> 20) & 0xfffffu);
     const int runs = (int)(w & 0xfffffu);
-    if (form == 0 || rN != N || rD != D) return 1;
+    if (form == 0 || rN != N || rD != D) return unknown;
     const int nblk = (int)ceil_div((size_t)N, CB);
-    const double even = std::max((14.0 - 2.5 * nblk + 1.4e-6 * (double)N * D) / 4.9e-3, 0.30 * N);
+    const double nd = (double)N * D;
+    const double even = rows_recordable ? std::max((14.0 - 2.5 * nblk + 1.4e-6 * nd) / 4.9e-3, 0.30 * N)
+                                        : (49.0 + 1.6e-6 * nd) / 5.0e-3;
     if (form == 1) {
         g_cols_runs = runs; g_cols_N = N; g_cols_D = D;
         return runs <= 1.08 * even ? 1 : -1;
@@ -914,9 +931,8 @@ MI355_API int mi355_embed_scatter_add_form(int V, int D, int S, int batch, int a
     if (!mi355_ready("embed_scatter_add_form")) return 0;
     if (V <= 0 || D <= 0 || S <= 0 || batch <= 0 || (size_t)batch * S > (size_t)1 << 30) return 0;
     const int N = batch * S;
-    const bool cols_ok = !g_ctx.scatter_tree && g_ctx.scatter_cols >= 0 && ((S % 4 == 0 && aligned) || N <= COL_SMALL) &&
-                         V < (1 << (32 - CB_BITS));
-    return scatter_form(N, D, cols_ok, N <= SMALL_N && key_bits(V) + POS_BITS <= 32);
+    const bool cols_ok = !g_ctx.scatter_tree && g_ctx.scatter_cols >= 0 && V < (1 << (32 - CB_BITS));
+    return scatter_form(N, D, cols_ok, S % 4 == 0 && aligned, N <= SMALL_N && key_bits(V) + POS_BITS <= 32);
 }
 
 MI355_API int mi355_embed_scatter_add_dev(float *dE, const float *dx, const int32_t *ids, int V, int D, int S,
@@ -932,11 +948,10 @@ MI355_API int mi355_embed_scatter_add_dev(float *dE, const float *dx, const int3
     // Two forms with the same bits (embed_cols.h says what each costs).  Columns of dE owned by workgroups: dx is
     // read where it lies, nothing is copied; chosen where one round of workgroups covers D and the positions are few
     // enough that the small accesses to dE (one per token and workgroup) do not outweigh the copy.
-    const bool cols_ok = !g_ctx.scatter_tree && g_ctx.scatter_cols >= 0 &&
-                         ((S % 4 == 0 && aligned16(dx)) || N <= COL_SMALL) && V < (1 << (32 - CB_BITS));
+    const bool cols_ok = !g_ctx.scatter_tree && g_ctx.scatter_cols >= 0 && V < (1 << (32 - CB_BITS));
     // (the column form also while a graph is recorded, for inputs whose row form would call the library sort, which cannot be)
-    unsigned long long *report = scatter_report_word();
-    if (scatter_form(N, D, cols_ok, N <= SMALL_N && key_bits(V) + POS_BITS <= 32) > 0)
+    unsigned long long *report = scatter_report_word(N, D);
+    if (scatter_form(N, D, cols_ok, S % 4 == 0 && aligned16(dx), N <= SMALL_N && key_bits(V) + POS_BITS <= 32) > 0)
         return scatter_add_cols(dE, dx, ids, V, D, S, N, report);
     const int bits = key_bits(V);
     const bool small = N <= SMALL_N && bits + POS_BITS <= 32;

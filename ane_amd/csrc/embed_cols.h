@@ -209,7 +209,11 @@ __device__ __forceinline__ float long_chain(float acc, const float *xc, int star
 template <int K>
 struct __attribute__((packed, aligned(4))) ColVec { float f[K]; };
 
-template <int K, bool FULL>                                     // FULL: D is a multiple of K, every workgroup has K columns
+// FULL: D is a multiple of K, every workgroup has K columns.  ANY: sequences of any length, dx at any 4-byte boundary: a
+// group of four positions that runs into the next sequence is read one by one (by a lane or two of a wave: at D = 768
+// 16351 positions in sequences of 197 take 47 us, the row form 63; 16384 in sequences of 256 take 44); without it S is a
+// multiple of 4 and dx 16-byte aligned.
+template <int K, bool FULL, bool ANY>
 __global__ __launch_bounds__(1024) void col_sum_kernel(float *dE, const float *__restrict__ dx,
                                                        const v2u *__restrict__ tasks,
                                                        const unsigned long long *__restrict__ cnt,
@@ -247,9 +251,19 @@ __global__ __launch_bounds__(1024) void col_sum_kernel(float *dE, const float *_
         for (int q = 0; q < COL_PPT / 4; q++) {
             const int p = p0 + 4 * q < N ? p0 + 4 * q : 0;       // (past the end: any address; the values are not used)
             const int b = p / S, s = p - b * S;
+            if (!ANY || s + 4 <= S) {
 #pragma unroll
-            for (int d = 0; d < K; d++)
-                o.px[d][q] = ld4_nt(dx + ((size_t)b * D + d0 + (d < kv ? d : 0)) * S + s);
+                for (int d = 0; d < K; d++)
+                    o.px[d][q] = ld4_nt(dx + ((size_t)b * D + d0 + (d < kv ? d : 0)) * S + s);
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const int pj = p + j < N ? p + j : 0, bj = pj / S;
+                    const float *src = dx + ((size_t)bj * D + d0) * S + (pj - bj * S);
+#pragma unroll
+                    for (int d = 0; d < K; d++) o.px[d][q][j] = src[(size_t)(d < kv ? d : 0) * S];
+                }
+            }
         }
         const unsigned *rp = reinterpret_cast<const unsigned *>(rk + (size_t)blk * CB + COL_PPT * t);
 #pragma unroll
@@ -499,8 +513,7 @@ __global__ __launch_bounds__(1024) void col_sum_small_kernel(float *dE, const fl
 // 148 KB of LDS, the most a workgroup can hold of a block of 8192 positions).
 int cols_per_workgroup(int D) { return D > 768 ? 4 : D > 512 ? 3 : D > 256 ? 2 : 1; }
 
-// Launches the kernels of the column form.  The caller has checked: V < 2^(32 - CB_BITS) and, beyond COL_SMALL
-// positions, S a multiple of 4 and dx 16-byte aligned.
+// Launches the kernels of the column form.  The caller has checked V < 2^(32 - CB_BITS).
 int scatter_add_cols(float *dE, const float *dx, const int32_t *ids, int V, int D, int S, int N,
                      unsigned long long *report) {
     const int K = cols_per_workgroup(D);
@@ -537,14 +550,16 @@ int scatter_add_cols(float *dE, const float *dx, const int32_t *ids, int V, int 
     hipLaunchKernelGGL(block_rank_kernel, dim3((unsigned)ceil_div((size_t)N, 64)), dim3(1024), 0, g_ctx.stream, rk, tasks,
                        cnt, sorted_chunks, ids, N, V, nchunks);
     LAUNCH_OK("embed_scatter_add plan");
-#define COL_LAUNCH(KK)                                                                                              \
-    case KK:                                                                                                        \
-        if (D % KK == 0)                                                                                            \
-            hipLaunchKernelGGL((col_sum_kernel<KK, true>), grid, dim3(1024), 0, g_ctx.stream, dE, dx, tasks, cnt, rk, N, D, \
-                               S, nblk, report);                                                                    \
-        else                                                                                                        \
-            hipLaunchKernelGGL((col_sum_kernel<KK, false>), grid, dim3(1024), 0, g_ctx.stream, dE, dx, tasks, cnt, rk, N, D, \
-                               S, nblk, report);                                                                    \
+    const bool any = S % 4 != 0 || !aligned16(dx);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(1024), 0, g_ctx.stream, dE, dx, tasks, cnt, rk, N, D, S, nblk, report);
+    };
+#define COL_LAUNCH(KK)                                                     \
+    case KK:                                                               \
+        if (D % KK == 0 && !any) launch(col_sum_kernel<KK, true, false>);  \
+        else if (D % KK == 0) launch(col_sum_kernel<KK, true, true>);      \
+        else if (!any) launch(col_sum_kernel<KK, false, false>);           \
+        else launch(col_sum_kernel<KK, false, true>);                      \
         break;
     switch (K) {
         COL_LAUNCH(1) COL_LAUNCH(2) COL_LAUNCH(3) COL_LAUNCH(4)

@@ -277,14 +277,14 @@ int mi355_embed_gather_dev(float *x, const float *E, const int32_t *ids, int V, 
  * training/training_dynamic/cpu_ops.h:158-164.  dE[ids[b][t]][d] += dx[b][d][t], each (row, d) sum
  * taken in ascending (b, t) order starting from the value already in dE, so the result is
  * bit-identical to the reference loop and run-to-run deterministic.  Ids outside [0,V) are skipped.
- * Two forms give the same bits: up to 16384 positions (S a multiple of 4, V < 2^19, D within one round of workgroups)
- * every workgroup owns a few columns of dE and reads its rows of dx in place; otherwise dx is first copied
- * token-major and summed row by row (the "scatter_cols" knob names a form).  The first form costs by the number of
- * distinct (token, block of 8192 positions) pairs and is the default; every call leaves that number in a word of
- * pinned host memory, and the next call with the same number of positions and D takes the second form if the ids
- * repeated too little for the first (and returns when they repeat again): same bits, only the time differs.
- * While a graph is recorded, inputs beyond 16384 positions take the first form too (the library sort of the second
- * cannot be recorded). */
+ * Two forms give the same bits (V < 2^19, D within one round of workgroups): every workgroup owns a few columns of dE and
+ * reads its rows of dx in place, or dx is copied token-major and summed row by row (the "scatter_cols" knob names a form).
+ * The first form costs by the number of distinct (token, block of 8192 positions) pairs; every call leaves that number in
+ * a word of pinned host memory, and the next call with the same number of positions and D (up to 65536) takes the form
+ * that it makes the faster: same bits, only the time differs.  Without such a word the first form is taken up to 16384
+ * positions in sequences of a multiple of 4 (of any length up to 512 positions), else the second.
+ * While a graph is recorded, inputs beyond 16384 positions (S a multiple of 4, dx 16-byte aligned) take the first form too
+ * (the library sort of the second cannot be recorded). */
 int mi355_embed_scatter_add_dev(float *dE, const float *dx, const int32_t *ids, int V, int D,
                                 int S, int batch);
 /* Which form the next mi355_embed_scatter_add_dev call of this shape would take under the current knobs and the last
