@@ -4,6 +4,9 @@
 // logits = cembed . x_final (training/training_dynamic/train.m:490-491), dy = cembed^T . dlogits (:501-502),
 // gcembed += dlogits . x_final^T (:507-508), and the dW products of each layer (:577-581, :613, :681-685).
 //
+// Large products go through the bfloat16 matrix instruction, each fp32 value as a sum of three (gemm_split.h); the kernel
+// in this file takes the others.
+//
 // fp32 products on the fp32 matrix instruction (v_mfma_f32_16x16x4_f32: fp32 products and sums, 157 TFLOP/s on the
 // chip).  An instruction takes 32 cycles of its SIMD for two registers of operands, so neither LDS nor memory is close to
 // its limit and what counts is that every SIMD has an instruction to issue all the time: tiles that divide the output
@@ -21,7 +24,9 @@
 //                 pitch puts into different quarters of the banks).
 // The instruction takes k from the lane's quarter; which k that is may be chosen as long as both operands agree: of the
 // four instructions of a step, number s multiplies k = s, 4 + s, 8 + s and 12 + s.
-#include "common.h"
+#include "tile.h"
+
+#include <type_traits>
 
 namespace {
 
@@ -223,6 +228,8 @@ __global__ __launch_bounds__(G_THREADS) void sgemm_kernel(const float *__restric
     }
 }
 
+#include "gemm_split.h"
+
 // C = alpha * sum_s part[s] + beta * C, s ascending
 __global__ __launch_bounds__(256) void slice_sum_kernel(float *C, int ldc, const float *__restrict__ part, int slices, int M,
                                                         int N, float alpha, float beta) {
@@ -243,34 +250,48 @@ int trans_flag(int t) {
 }
 
 struct GemmPlan {
-    int bm, bn, slices, k_slice;
+    int split, bm, bn, slices, k_slice;      // split: the kernel of gemm_split.h
 };
 
-// The tile and the number of K slices with the least estimated time.  A compute unit multiplies 0.48 MFLOP a microsecond
-// on these tiles (123 TFLOP/s on the chip, measured at 4096^3 with every tile size) when two or more workgroups share
-// it; with one, whose waves wait at their barriers, three quarters of that.  What is left to choose is how evenly the
-// output divides: [24573][1024] . [1024][256] takes 109 us in 768 tiles of 128 x 64, 115 in 1536 of 64 x 64.  Slices cost
-// their partial products' way through memory and a launch; they pay where the output has few tiles ([1024][24573] .
-// [24573][256]: 118 us in 16 slices of 64 tiles, 200 us in 4).  Only the smallest tile holds the old values of C through
-// its loop (beta != 0: [24573][256] . [256][1024] 129 us against 135 in tiles of 128 x 64).
-GemmPlan plan_gemm(int M, int N, int K, bool reads_c) {
+// The kernel, tile and number of K slices with the least estimated time.
+// Split kernel: a workgroup has a compute unit to itself and takes 2.5 us a step of 32 and 4 us around them (4 more where
+// it reads C).  fp32 kernel: a compute unit multiplies 0.48 MFLOP a microsecond (123 TFLOP/s on the chip, measured at
+// 4096^3 with every tile size) when two or more workgroups share it; with one, whose waves wait at their barriers, three
+// quarters of that.  Slices cost their partial products' way through memory and a launch; they pay where the output has
+// few tiles.  Measured, split kernel against fp32 kernel, us, and relative error of either against 64 bits:
+//   [24573][1024] . [1024][256]      86 / 109    5.0e-7 / 5.7e-7    (the library that stood here first: 121, 5.7e-7)
+//   [1024][24573] . [24573][256]     80 / 118    5.0e-7 / 10e-7     (144, 5.2e-7)
+//   [24573][256] . [256][1024] +=    90 / 129    2.6e-7 / 2.9e-7    (271, 2.9e-7)
+//   [9001][768] . [768][197]         39 / 49     2.6e-7 / 5.0e-7    [768][9001] . [9001][197]  34 / 44   2.8e-7 / 4.3e-7
+//   [768][768] . [768][256]          18 / 11     2.0e-7 / 2.3e-7    [2000][32] . [32][768]     7.6 / 5   1.2e-7 / 1.0e-7
+// The large tiles lose where the output has few of them, and the estimate leaves those to the fp32 kernel, of whose tiles
+// only the smallest holds the old values of C through its loop.
+GemmPlan plan_gemm(int M, int N, int K, bool reads_c, int lda, int ldb) {
     const int cus = g_ctx.num_cu > 0 ? g_ctx.num_cu : 256;
-    const int tile[3][2] = {{128, 64}, {64, 128}, {64, 64}};
-    GemmPlan best = {64, 64, 1, K};
+    struct Tile { int split, bm, bn; };
+    const Tile tile[5] = {{0, 128, 64}, {0, 64, 128}, {0, 64, 64}, {1, 128, 256}, {1, 256, 128}};
+    GemmPlan best = {0, 64, 64, 1, K};
     double best_us = -1.0;
-    for (const auto &t : tile) {
-        const double tiles = (double)ceil_div((size_t)M, (size_t)t[0]) * (double)ceil_div((size_t)N, (size_t)t[1]);
+    const bool can = lda < (1 << 22) && ldb < (1 << 22);        // (32-bit offsets of the lanes)
+    for (const Tile &t : tile) {
+        if (t.split ? g_ctx.gemm_split < 0 || !can : g_ctx.gemm_split > 0 && can) continue;
+        if (t.split && g_ctx.gemm_split > 0 && t.bm != 128 * g_ctx.gemm_split) continue;
+        const int step = t.split ? SK : GK;
+        const double tiles = (double)ceil_div((size_t)M, (size_t)t.bm) * (double)ceil_div((size_t)N, (size_t)t.bn);
         for (int want = 1; want <= 64; want++) {
             if (g_ctx.gemm_splitk && want != (K >= 2 * g_ctx.gemm_splitk ? g_ctx.gemm_splitk : 1)) continue;
-            const int k_slice = (int)ceil_div(ceil_div((size_t)K, (size_t)want), GK) * GK;
+            const int k_slice = (int)ceil_div(ceil_div((size_t)K, (size_t)want), (size_t)step) * step;
             const int slices = (int)ceil_div((size_t)K, (size_t)k_slice);
             if (want > 1 && !g_ctx.gemm_splitk && (k_slice < 128 || (double)slices * M * N > 64e6)) break;
             const double per_cu = tiles * slices / cus;
             const double rounds = per_cu <= 1.0 ? 1.0 : (double)(long)(per_cu + 0.999999);
-            double us = rounds * t[0] * t[1] * (double)k_slice * 2.0 / 0.48e6 * (per_cu <= 1.0 ? 1.33 : 1.0);
-            if (reads_c && slices == 1 && t[0] * t[1] > 64 * 64) us *= 1.05;
+            const double mflop = (double)t.bm * t.bn * k_slice * 2.0e-6;
+            double us;
+            if (t.split) us = rounds * (4.0 + 2.5 * (k_slice / SK)) + (reads_c && slices == 1 ? rounds * 4.0 : 0.0);
+            else us = rounds * mflop / 0.48 * (per_cu <= 1.0 ? 1.33 : 1.0);
+            if (!t.split && reads_c && slices == 1 && t.bm * t.bn > 64 * 64) us *= 1.05;
             if (slices > 1) us += 5.0 + (double)slices * M * N * 8.0 / 5e6;
-            if (best_us < 0.0 || us < best_us) { best_us = us; best = GemmPlan{t[0], t[1], slices, k_slice}; }
+            if (best_us < 0.0 || us < best_us) { best_us = us; best = GemmPlan{t.split, t.bm, t.bn, slices, k_slice}; }
         }
     }
     return best;
@@ -289,31 +310,43 @@ MI355_API int mi355_sgemm_dev(int trans_a, int trans_b, int M, int N, int K, flo
     // row-major leading dimensions: A is M x K (or K x M when transposed), B is K x N (or N x K), C is M x N
     if (lda < (ta ? M : K) || ldb < (tb ? K : N) || ldc < N)
         return mi355_fail("sgemm: leading dimension too small (lda=%d ldb=%d ldc=%d)", lda, ldb, ldc);
-    const GemmPlan p = plan_gemm(M, N, K, beta != 0.f);
+    const GemmPlan p = plan_gemm(M, N, K, beta != 0.f, lda, ldb);
     float *part = nullptr;
     if (p.slices > 1) {
         part = (float *)mi355_ws((size_t)p.slices * M * N * sizeof(float));
         if (!part) return -1;
     }
     const int tiles_n = (int)ceil_div((size_t)N, (size_t)p.bn), tiles = (int)ceil_div((size_t)M, (size_t)p.bm) * tiles_n;
-    auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned)tiles * p.slices), dim3(G_THREADS), 0, g_ctx.stream, A, lda, B, ldb, C, ldc, M,
-                           N, K, p.k_slice, tiles_n, tiles, alpha, beta, part);
+    // alpha == 0 reads neither operand (cblas semantics): a product over nothing
+    const int k_all = alpha != 0.f ? K : 0;
+    auto launch = [&](auto kernel, int threads) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)tiles * p.slices), dim3(threads), 0, g_ctx.stream, A, lda, B, ldb, C, ldc, M, N,
+                           k_all, p.k_slice, tiles_n, tiles, alpha, beta, part);
     };
 #define GEMM_CASE(BM, BN, WM, WN)                                                                                     \
     case (BM) * 1000 + (BN):                                                                                          \
-        if (!ta && !tb) launch(sgemm_kernel<BM, BN, WM, WN, false, false>);                                           \
-        else if (!ta) launch(sgemm_kernel<BM, BN, WM, WN, false, true>);                                              \
-        else if (!tb) launch(sgemm_kernel<BM, BN, WM, WN, true, false>);                                              \
-        else launch(sgemm_kernel<BM, BN, WM, WN, true, true>);                                                        \
+        if (!ta && !tb) launch(sgemm_kernel<BM, BN, WM, WN, false, false>, G_THREADS);                                \
+        else if (!ta) launch(sgemm_kernel<BM, BN, WM, WN, false, true>, G_THREADS);                                   \
+        else if (!tb) launch(sgemm_kernel<BM, BN, WM, WN, true, false>, G_THREADS);                                   \
+        else launch(sgemm_kernel<BM, BN, WM, WN, true, true>, G_THREADS);                                             \
+        break;
+#define SPLIT_CASE(BM, BN)                                                                                            \
+    case (BM) * 1000 + (BN):                                                                                          \
+        if (!ta && !tb) launch(sgemm_split_kernel<BM, BN, false, false>, S_THREADS);                              \
+        else if (!ta) launch(sgemm_split_kernel<BM, BN, false, true>, S_THREADS);                                 \
+        else if (!tb) launch(sgemm_split_kernel<BM, BN, true, false>, S_THREADS);                                 \
+        else launch(sgemm_split_kernel<BM, BN, true, true>, S_THREADS);                                           \
         break;
     switch (p.bm * 1000 + p.bn) {
         GEMM_CASE(64, 128, 32, 64)
         GEMM_CASE(128, 64, 64, 32)
         GEMM_CASE(64, 64, 32, 32)
+        SPLIT_CASE(128, 256)
+        SPLIT_CASE(256, 128)
         default: return mi355_fail("sgemm: no kernel for a tile of %d x %d", p.bm, p.bn);
     }
 #undef GEMM_CASE
+#undef SPLIT_CASE
     LAUNCH_OK("sgemm");
     if (part) {
         hipLaunchKernelGGL(slice_sum_kernel, dim3((unsigned)ceil_div((size_t)M * N, 256)), dim3(256), 0, g_ctx.stream, C, ldc,

@@ -56,7 +56,8 @@ size_t mi355_workspace_size(void);
  * "rms_lpr" (lanes per strip row, 4/8/16) and "rms_threads" (256/512/1024) of the RMSNorm tiles, "qk_lpr" and
  * "qk_threads" (256/512) of the QK-norm + RoPE tiles, "ew_unroll" (accesses per lane of the streaming ops, 1/2/4),
  * "ce_rows" / "ce_rows2" (rows of logits per workgroup in the first / second pass of softmax-CE),
- * "gemm_splitk" (K slices of mi355_sgemm_dev; 1 = never split),
+ * "gemm_splitk" (K slices of mi355_sgemm_dev; 1 = never split), "gemm_split" (its kernel that multiplies fp32 values as
+ * sums of three bfloat16 values: 0 = where it pays, -1 = never, 1 / 2 = always, in tiles of 128 x 256 / 256 x 128),
  * "scatter_tree" (1: mi355_embed_scatter_add_dev sums long segments by a fixed tree instead of the reference's
  * sequential order: still deterministic and within 1e-5 of each row's scale, faster, no longer bit-identical to
  * the CPU loop), "scatter_cols" (the form of mi355_embed_scatter_add_dev in which every workgroup owns a few columns

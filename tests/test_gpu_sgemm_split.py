@@ -1,0 +1,89 @@
+"""mi355_sgemm_dev through the bfloat16 matrix instruction, fp32 values as sums of three: tile edges in every transpose case,
+and the values that such a sum cannot hold, which have to give what the fp32 instruction gives."""
+import numpy as np
+import pytest
+
+import helpers as H
+
+pytestmark = pytest.mark.gpu
+
+
+def product(br, knob, A, B, ta, tb, alpha=1.0, beta=0.0, C0=None, off=0):
+    """(M, N, K of the operands as stored) -> C; every matrix starts `off` floats behind an aligned address."""
+    M, K = A.shape[::-1] if ta else A.shape
+    N = B.shape[0] if tb else B.shape[1]
+    put = lambda a: br.DevArray.from_numpy(np.concatenate([np.zeros(off, np.float32), a.ravel()]))
+    ad, bd, cd = put(A), put(B), put(np.full((M, N), np.nan, np.float32) if C0 is None else C0)
+    br.tune("gemm_split", knob)
+    try:
+        br.check(br.lib.mi355_sgemm_dev(ta, tb, M, N, K, alpha, ad.ptr + 4 * off, A.shape[1], bd.ptr + 4 * off, B.shape[1],
+                                        beta, cd.ptr + 4 * off, N))
+        return cd.numpy()[off:].reshape(M, N)
+    finally:
+        br.tune("gemm_split", 0)
+
+
+@pytest.mark.parametrize("knob", [1, 2])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (0, 1), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (127, 257, 31), (129, 255, 33), (256, 256, 64), (300, 130, 97), (70, 3, 700)])
+def test_split_tile_edges(br, M, N, K, ta, tb, knob):
+    print("[case] sgemm split M=%d N=%d K=%d ta=%d tb=%d knob=%d" % (M, N, K, ta, tb, knob), flush=True)
+    A = H.normal(600, (K, M) if ta else (M, K)); B = H.normal(601, (N, K) if tb else (K, N)); C0 = H.normal(602, (M, N))
+    A64, B64 = A.astype(np.float64), B.astype(np.float64)
+    ref = (A64.T if ta else A64) @ (B64.T if tb else B64)
+    mag = np.abs(A64.T if ta else A64) @ np.abs(B64.T if tb else B64)
+    for alpha, beta in ((1.0, 0.0), (-0.75, 1.5)):
+        got = product(br, knob, A, B, ta, tb, alpha, beta, None if beta == 0.0 else C0, off=1).astype(np.float64)
+        want = alpha * ref + beta * C0
+        # six instructions per 32 values of k, each within 2^-23 of the sum of magnitudes (rounded or cut off), slices added
+        # the same way; what is left out of a product is below 3 x 2^-26 of it; three more operations on the result
+        bound = (6 * (K // 32 + 2) + 1) * 2.0 ** -23 * abs(alpha) * mag + 3 * 2.0 ** -24 * (np.abs(want) + abs(beta) * np.abs(C0))
+        assert np.all(np.abs(got - want) <= bound)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (0, 1), (1, 1)])
+def test_split_gives_infinities_and_nans_of_fp32(br, ta, tb):
+    M, N, K = 300, 300, 70
+    A = H.normal(610, (M, K)); B = H.normal(611, (K, N))
+    A[3, 5] = np.inf; A[140, 69] = -np.inf; A[141, 0] = np.nan
+    A[7, 1] = np.finfo(np.float32).max          # rounds to an infinity in 8 bits
+    B[64, 260] = np.inf; B[1, 17] = 0.0; B[5, 4] = 0.0
+    As, Bs = np.ascontiguousarray(A.T if ta else A), np.ascontiguousarray(B.T if tb else B)
+    want = product(br, -1, As, Bs, ta, tb)
+    for knob in (1, 2):
+        got = product(br, knob, As, Bs, ta, tb)
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+        assert np.array_equal(np.sign(got[np.isinf(got)]), np.sign(want[np.isinf(want)]))
+        ok = np.isfinite(want)
+        with np.errstate(invalid="ignore"):
+            mag = np.abs(A[:, None, :].astype(np.float64) * B.T[None, :, :]).sum(-1)
+        assert np.all(np.abs(got[ok].astype(np.float64) - want[ok]) <= (K + 20) * 2.0 ** -23 * mag[ok])
+
+
+@pytest.mark.parametrize("scale", [2.0 ** -95, 2.0 ** -108, 2.0 ** -113, 2.0 ** -120])
+def test_split_keeps_values_near_the_smallest(br, scale):
+    """Values whose last 8 bits are no bfloat16 any more, and some whose last bits are its smallest ones."""
+    M, N, K = 130, 260, 64
+    A = (H.normal(620, (M, K)).astype(np.float64) * scale).astype(np.float32)
+    A[:, 0] = np.float32(scale * (1 + 2.0 ** -9 + 2.0 ** -17))
+    A[100:, :] = 0                              # rows that hold these values alone
+    A[100:, 0] = np.float32(2.0 ** -115 * (1 + 2.0 ** -9 + 2.0 ** -17))
+    B = H.normal(621, (K, N))
+    ref = A.astype(np.float64) @ B.astype(np.float64); mag = np.abs(A.astype(np.float64)) @ np.abs(B.astype(np.float64))
+    for knob in (1, 2):
+        got = product(br, knob, A, B, 0, 0).astype(np.float64)
+        assert np.all(np.abs(got - ref) <= (K + 1) * 2.0 ** -23 * mag + K * 2.0 ** -149)
+
+
+def test_alpha_zero_reads_no_operand(br):
+    A = np.full((40, 300), np.nan, np.float32); B = np.full((300, 50), np.inf, np.float32); C0 = H.normal(630, (40, 50))
+    for knob in (-1, 1):
+        assert np.array_equal(product(br, knob, A, B, 0, 0, alpha=0.0, beta=2.0, C0=C0), 2.0 * C0)
+        assert not np.any(product(br, knob, A, B, 0, 0, alpha=0.0))
+
+
+@pytest.fixture(scope="module")
+def br():
+    import ane_amd.bridge as b
+    b.init()
+    return b
