@@ -67,3 +67,28 @@ def test_form_is_learned_from_the_last_call_of_the_shape(br, B, S):
     assert form() == -1
     call(text)
     assert form() == 1
+
+
+def test_graph_records_a_short_sequence_of_any_length_into_a_large_vocabulary(br):
+    """Up to 512 positions the plan and the sums are one launch, which takes any length; the row form of so large a
+    vocabulary would call the library sort, which cannot be recorded."""
+    L = br.lib
+    V, D, B, S = 300000, 8, 2, 197
+    ids = H.zipf_ids(15, B * S, V).astype(np.int32).reshape(B, S)
+    dx = H.normal(16, (B, D, S)); dE0 = H.normal(17, (V, D))
+    dEd, idd, dxd = br.DevArray.from_numpy(dE0), br.DevArray.from_numpy(ids), br.DevArray.from_numpy(dx)
+    br.sync()
+    br.check(L.mi355_graph_begin())
+    got = L.mi355_embed_scatter_add_dev(dEd.ptr, dxd.ptr, idd.ptr, V, D, S, B)
+    why = br.last_error()
+    g = L.mi355_graph_end()
+    try:
+        assert got == 0 and g, why
+        want = dE0
+        for _ in range(3):
+            br.check(L.mi355_graph_launch(g))
+            want = O.embed_backward(want, dx, ids)
+            br.sync()
+            assert dEd.numpy().tobytes() == want.tobytes()
+    finally:
+        if g: L.mi355_graph_free(g)
