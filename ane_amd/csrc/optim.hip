@@ -143,8 +143,8 @@ __device__ __forceinline__ int mt_owner(const MtFirst &f, unsigned block) {
 // so that the end of g is in the 256 MB last-level cache when the update, which walks the blocks from the last to the
 // first, asks for it.  Norm + clip + update of the 110 M parameters (109 tensors, 3.5 GB besides the norm's read):
 // 748 us with one launch per 16 tensors of (largest tensor) x (tensors) blocks and a sum after each, 707 with the
-// blocks numbered through, 700 with the update backwards, 650 with these loads not marked as streaming.  Which elements a block sums depends on the sizes alone, so the sum is
-// deterministic.
+// blocks numbered through, 700 with the update backwards, 650 with these loads not marked as streaming.  Which elements
+// a block sums depends on the sizes alone, so the sum is deterministic.
 __global__ __launch_bounds__(OPT_THREADS) void sumsq_partial_mt_kernel(float *__restrict__ part, MtSumsq a, float pre,
                                                                        int rounds) {
     __shared__ float red[OPT_THREADS / 64];

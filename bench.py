@@ -45,7 +45,7 @@ OP_KERNELS = {
     "residual_rmsnorm_fwd": [("rms_fwd_cluster_kernel<StoreF32, 4, 1024, true, true>", 1.0)],
     "rmsnorm_bwd_residual": [("rms_bwd_cluster_kernel<StoreF32, 4, 1024, true, false>", 1.0)],
     "scale_copy": [("axpby_kernel<1, 1>", 1.0)],
-    "softmax_ce": [("ce_resident_kernel<CrF32, true>", 1.0)],
+    "softmax_ce": [("ce_resident_kernel<CrF32, 16, 9, true>", 1.0)],
     "int8_scale": [("absmax_scale_kernel", 1.0)],
     "int8_quant": [("quant_kernel<1>", 1.0)],
     "int8_dequant": [("dequant_kernel<1>", 1.0)],
@@ -54,7 +54,7 @@ OP_KERNELS = {
 # the three launches of the ordered scatter-add in its column form and in its row form, and
 # the gather
 EMBED_KERNELS = {
-    "scatter_cols": [("chunk_sort_blk_kernel", 1.0), ("block_rank_kernel", 1.0), ("col_sum_kernel<3, true>", 1.0)],
+    "scatter_cols": [("chunk_sort_blk_kernel", 1.0), ("block_rank_kernel", 1.0), ("col_sum_kernel<3, true, false>", 1.0)],
     "scatter_rows": [("chunk_sort_kernel", 1.0), ("rank_transpose_kernel", 1.0), ("seg_sum_kernel<false>", 1.0)],
     "gather": [("gather_kernel<true>", 1.0)],
 }
