@@ -18,16 +18,23 @@ namespace {
 constexpr int ST_THREADS = 256;
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+typedef _Float16 h8_any __attribute__((ext_vector_type(8), aligned(2)));      // at any fp16 element of global memory
 
 // ---- rectangle converts: one lane = 8 contiguous elements of one row ----
+// Bound by their bytes.  Rows of any length (>= 8) and pitch, at any element: the last lane of a row takes the row's last
+// 8 elements, some of them its neighbour's too, and stores the same values; a rectangle without gaps is one row.  With one
+// element per lane where a row was no multiple of 8 or off a 16-byte boundary: [8192][1001] to fp16 15.6 us (now 11.0),
+// [24576][1001] from fp16 63.0 (32.3).  Lanes are numbered in 32 bits (a launch holds no more).
+__device__ __forceinline__ size_t last_whole(size_t c, size_t n, size_t cols) { return c + n <= cols ? c : cols - n; }
+
 __global__ __launch_bounds__(ST_THREADS) void cvt_f32_f16_v8(_Float16 *__restrict__ dst, size_t dst_ld,
                                                              const float *__restrict__ src, size_t src_ld,
-                                                             size_t colg, size_t total) {
-    const size_t i = (size_t)blockIdx.x * ST_THREADS + threadIdx.x;
+                                                             unsigned colg, size_t cols, size_t total) {
+    const unsigned i = blockIdx.x * ST_THREADS + threadIdx.x;
     if (i >= total) return;
-    const size_t r = i / colg, g = i - r * colg;
-    const float *s = src + r * src_ld + 8 * g;
+    const unsigned r = i / colg;
+    const size_t c = last_whole((size_t)8 * (i - r * colg), 8, cols);
+    const float *s = src + r * src_ld + c;
     const v4f a = ld4_nt(s), b = ld4_nt(s + 4);
     h8 o;
 #pragma unroll
@@ -35,23 +42,24 @@ __global__ __launch_bounds__(ST_THREADS) void cvt_f32_f16_v8(_Float16 *__restric
         o[j] = (_Float16)a[j];       // round to nearest even, overflow to infinity, subnormals kept
         o[4 + j] = (_Float16)b[j];
     }
-    __builtin_nontemporal_store(o, reinterpret_cast<h8 *>(dst + r * dst_ld + 8 * g));
+    __builtin_nontemporal_store(o, reinterpret_cast<h8_any *>(dst + r * dst_ld + c));
 }
 
 __global__ __launch_bounds__(ST_THREADS) void cvt_f16_f32_v8(float *__restrict__ dst, size_t dst_ld,
                                                              const _Float16 *__restrict__ src, size_t src_ld,
-                                                             size_t colg, size_t total) {
-    const size_t i = (size_t)blockIdx.x * ST_THREADS + threadIdx.x;
+                                                             unsigned colg, size_t cols, size_t total) {
+    const unsigned i = blockIdx.x * ST_THREADS + threadIdx.x;
     if (i >= total) return;
-    const size_t r = i / colg, g = i - r * colg;
-    const h8 v = __builtin_nontemporal_load(reinterpret_cast<const h8 *>(src + r * src_ld + 8 * g));
+    const unsigned r = i / colg;
+    const size_t c = last_whole((size_t)8 * (i - r * colg), 8, cols);
+    const h8 v = __builtin_nontemporal_load(reinterpret_cast<const h8_any *>(src + r * src_ld + c));
     v4f a, b;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         a[j] = (float)v[j];
         b[j] = (float)v[4 + j];
     }
-    float *d = dst + r * dst_ld + 8 * g;
+    float *d = dst + r * dst_ld + c;
     st4_nt(d, a);
     st4_nt(d + 4, b);
 }
@@ -81,7 +89,7 @@ __device__ __forceinline__ void load_cols(float (&o)[VEC], const T *p) {
         o[0] = (float)p[0];
     } else if constexpr (sizeof(T) == 2) {
         static_assert(VEC == 8, "fp16 rows are read 8 columns at a time");
-        const h8 v = __builtin_nontemporal_load(reinterpret_cast<const h8 *>(p));
+        const h8 v = __builtin_nontemporal_load(reinterpret_cast<const h8_any *>(p));
 #pragma unroll
         for (int j = 0; j < 8; j++) o[j] = (float)v[j];
     } else {
@@ -120,42 +128,43 @@ __device__ __forceinline__ void store_cols(float *p, const float (&o)[VEC]) {
     }
 }
 
-// One lane = one interleaved row pair (2i, 2i+1) of one output head x VEC columns.
-// Pair rows are numbered Q heads first, then K heads, then V heads.
+// One lane = one interleaved row pair (2i, 2i+1) of one output head x VEC columns (rows of any length >= VEC: the last
+// lane of a row as in the converts, so not in place where S % VEC != 0: a neighbour in another wave could read what this
+// lane has rotated; one column per lane there).  [8][2048][1001] fp16 in: 89.4 us with one column per lane, now 50.1;
+// [16][2048][250] 48.1 and 26.9.  Pair rows are numbered Q heads first, then K heads, then V heads.
 template <typename T, int VEC>
 __global__ __launch_bounds__(ST_THREADS) void attn_grads_finish_kernel(
     float *dq, float *__restrict__ dk, float *__restrict__ dv, const T *qf, const T *__restrict__ kf,
     const T *__restrict__ vf, size_t sq, size_t sk, size_t sv, int heads, int kv_heads, int ratio, int hd, int S,
     int batch, const float *__restrict__ cos_t, const float *__restrict__ sin_t, size_t total) {
-    const size_t idx = (size_t)blockIdx.x * ST_THREADS + threadIdx.x;
+    const unsigned idx = blockIdx.x * ST_THREADS + threadIdx.x;
     if (idx >= total) return;
-    const int colg = S / VEC;
-    const int cg = (int)(idx % colg);
-    size_t pr = idx / colg;
-    const int half = hd >> 1;
-    const int s = cg * VEC;
-    const size_t q_rows = (size_t)batch * heads * half, kv_rows = (size_t)batch * kv_heads * half;
+    const unsigned colg = ((unsigned)S + VEC - 1) / VEC;
+    unsigned pr = idx / colg;
+    const unsigned half = (unsigned)hd >> 1;
+    const int s = (int)last_whole((size_t)(idx - pr * colg) * VEC, VEC, S);
+    const unsigned q_rows = (unsigned)batch * heads * half, kv_rows = (unsigned)batch * kv_heads * half;
 
     float r0[VEC], r1[VEC];
     float *out;
     int i;
     bool rotate;
     if (pr < q_rows) {
-        i = (int)(pr % half);
-        const size_t bh = pr / half;                 // b*heads + h
-        const size_t b = bh / heads, h = bh - b * heads;
+        const unsigned bh = pr / half;               // b*heads + h
+        i = (int)(pr - bh * half);
+        const size_t b = bh / (unsigned)heads, h = bh - b * heads;
         const T *in = qf + b * sq + (h * hd + 2 * i) * (size_t)S + s;
         load_cols<T, VEC>(r0, in);
         load_cols<T, VEC>(r1, in + S);
-        out = dq + (bh * hd + 2 * i) * (size_t)S + s;
+        out = dq + ((size_t)bh * hd + 2 * i) * (size_t)S + s;
         rotate = true;
     } else {
         pr -= q_rows;
         const bool is_k = pr < kv_rows;
         if (!is_k) pr -= kv_rows;
-        i = (int)(pr % half);
-        const size_t bh = pr / half;                 // b*kv_heads + kv
-        const size_t b = bh / kv_heads, kv = bh - b * kv_heads;
+        const unsigned bh = pr / half;               // b*kv_heads + kv
+        i = (int)(pr - bh * half);
+        const size_t b = bh / (unsigned)kv_heads, kv = bh - b * kv_heads;
         const T *in = (is_k ? kf + b * sk : vf + b * sv) + ((kv * ratio) * hd + 2 * i) * (size_t)S + s;
 #pragma unroll
         for (int j = 0; j < VEC; j++) r0[j] = r1[j] = 0.f;
@@ -169,7 +178,7 @@ __global__ __launch_bounds__(ST_THREADS) void attn_grads_finish_kernel(
                 r1[j] += a1[j];
             }
         }
-        out = (is_k ? dk : dv) + (bh * hd + 2 * i) * (size_t)S + s;
+        out = (is_k ? dk : dv) + ((size_t)bh * hd + 2 * i) * (size_t)S + s;
         rotate = is_k;
     }
     if (rotate && cos_t) {
@@ -206,11 +215,11 @@ MI355_API int mi355_cvt_f32_f16_dev(uint16_t *dst, size_t dst_ld, const float *s
                                     size_t cols) {
     if (cvt_args("cvt_f32_f16", dst, src, dst_ld, src_ld, rows, cols)) return -1;
     _Float16 *d = reinterpret_cast<_Float16 *>(dst);
-    const bool vec = cols % 8 == 0 && dst_ld % 8 == 0 && src_ld % 4 == 0 && aligned16(dst) && aligned16(src);
-    if (vec) {
-        const size_t colg = cols / 8, total = rows * colg;
+    if (dst_ld == cols && src_ld == cols) { cols *= rows; rows = 1; }       // no gaps: one row
+    if (cols >= 8) {
+        const size_t colg = ceil_div(cols, (size_t)8), total = rows * colg;
         hipLaunchKernelGGL(cvt_f32_f16_v8, dim3((unsigned)ceil_div(total, ST_THREADS)), dim3(ST_THREADS), 0,
-                           g_ctx.stream, d, dst_ld, src, src_ld, colg, total);
+                           g_ctx.stream, d, dst_ld, src, src_ld, (unsigned)colg, cols, total);
     } else {
         const size_t total = rows * cols;
         hipLaunchKernelGGL(cvt_f32_f16_v1, dim3((unsigned)ceil_div(total, ST_THREADS)), dim3(ST_THREADS), 0,
@@ -224,11 +233,11 @@ MI355_API int mi355_cvt_f16_f32_dev(float *dst, size_t dst_ld, const uint16_t *s
                                     size_t cols) {
     if (cvt_args("cvt_f16_f32", dst, src, dst_ld, src_ld, rows, cols)) return -1;
     const _Float16 *s = reinterpret_cast<const _Float16 *>(src);
-    const bool vec = cols % 8 == 0 && dst_ld % 4 == 0 && src_ld % 8 == 0 && aligned16(dst) && aligned16(src);
-    if (vec) {
-        const size_t colg = cols / 8, total = rows * colg;
+    if (dst_ld == cols && src_ld == cols) { cols *= rows; rows = 1; }       // no gaps: one row
+    if (cols >= 8) {
+        const size_t colg = ceil_div(cols, (size_t)8), total = rows * colg;
         hipLaunchKernelGGL(cvt_f16_f32_v8, dim3((unsigned)ceil_div(total, ST_THREADS)), dim3(ST_THREADS), 0,
-                           g_ctx.stream, dst, dst_ld, s, src_ld, colg, total);
+                           g_ctx.stream, dst, dst_ld, s, src_ld, (unsigned)colg, cols, total);
     } else {
         const size_t total = rows * cols;
         hipLaunchKernelGGL(cvt_f16_f32_v1, dim3((unsigned)ceil_div(total, ST_THREADS)), dim3(ST_THREADS), 0,
@@ -257,26 +266,20 @@ MI355_API int mi355_attn_grads_finish_dev(float *dq, float *dk, float *dv, const
         return mi355_fail("attn_grads_finish: sequence stride below heads*hd*S = %zu", full);
     const int ratio = heads / kv_heads;
     const size_t pair_rows = (size_t)batch * (heads + 2 * kv_heads) * (hd / 2);
-    const bool out_al = aligned16(dq) && aligned16(dk) && aligned16(dv);
-    const bool tab_al = !cos_dev || (aligned16(cos_dev) && aligned16(sin_dev));
-    const bool in_al = aligned16(dq_full) && aligned16(dk_full) && aligned16(dv_full);
+    const bool in_place = (const void *)dq == dq_full || (const void *)dk == dk_full || (const void *)dv == dv_full;
 #define FINISH(T, VEC)                                                                                               \
     do {                                                                                                             \
-        const size_t total = pair_rows * (size_t)(S / (VEC));                                                        \
+        const size_t total = pair_rows * ceil_div((size_t)S, (size_t)(VEC));                                         \
         hipLaunchKernelGGL((attn_grads_finish_kernel<T, VEC>), dim3((unsigned)ceil_div(total, ST_THREADS)),          \
                            dim3(ST_THREADS), 0, g_ctx.stream, dq, dk, dv, (const T *)dq_full, (const T *)dk_full,    \
                            (const T *)dv_full, q_stride, k_stride, v_stride, heads, kv_heads, ratio, hd, S, batch,   \
                            cos_dev, sin_dev, total);                                                                 \
     } while (0)
     if (in_f16) {
-        const bool vec = S % 8 == 0 && out_al && tab_al && in_al && q_stride % 8 == 0 && k_stride % 8 == 0 &&
-                         v_stride % 8 == 0;
-        if (vec) FINISH(_Float16, 8);
+        if (S % 8 == 0 || (S > 8 && !in_place)) FINISH(_Float16, 8);
         else FINISH(_Float16, 1);
     } else {
-        const bool vec = S % 4 == 0 && out_al && tab_al && in_al && q_stride % 4 == 0 && k_stride % 4 == 0 &&
-                         v_stride % 4 == 0;
-        if (vec) FINISH(float, 4);
+        if (S % 4 == 0 || (S > 4 && !in_place)) FINISH(float, 4);
         else FINISH(float, 1);
     }
 #undef FINISH
