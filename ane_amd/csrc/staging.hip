@@ -13,18 +13,25 @@
 // lane reads its fp16 (or fp32) inputs once and writes the three fp32 results once.
 #include "common.h"
 
+#include <algorithm>
+
 namespace {
 
 constexpr int ST_THREADS = 256;
+constexpr size_t ST_LANES = (size_t)1 << 31;   // of one launch
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+typedef _Float16 h4_any __attribute__((ext_vector_type(4), aligned(2)));
 typedef _Float16 h8_any __attribute__((ext_vector_type(8), aligned(2)));      // at any fp16 element of global memory
 
-// ---- rectangle converts: one lane = 8 contiguous elements of one row ----
-// Bound by their bytes.  Rows of any length (>= 8) and pitch, at any element: the last lane of a row takes the row's last
-// 8 elements, some of them its neighbour's too, and stores the same values; a rectangle without gaps is one row.  With one
+// ---- rectangle converts: one lane = 16 bytes of the result (8 fp16 or 4 fp32 elements of one row) ----
+// Bound by their bytes.  Every store instruction of a wave writes whole lines: with two 16-byte stores 32 bytes apart per
+// lane [49152][256] from fp16 took 16.7 us, with one 14.6 (75 MB: 5.2 TB/s).
+// Rows of any length (at least a lane's elements) and pitch, at any element: the last lane of a row takes the row's last
+// whole group, some of it its neighbour's too, and stores the same values; a rectangle without gaps is one row.  With one
 // element per lane where a row was no multiple of 8 or off a 16-byte boundary: [8192][1001] to fp16 15.6 us (now 11.0),
-// [24576][1001] from fp16 63.0 (32.3).  Lanes are numbered in 32 bits (a launch holds no more).
+// [24576][1001] from fp16 63.0 (26.7).  Lanes are numbered in 32 bits (a launch holds no more).
 __device__ __forceinline__ size_t last_whole(size_t c, size_t n, size_t cols) { return c + n <= cols ? c : cols - n; }
 
 __global__ __launch_bounds__(ST_THREADS) void cvt_f32_f16_v8(_Float16 *__restrict__ dst, size_t dst_ld,
@@ -45,23 +52,19 @@ __global__ __launch_bounds__(ST_THREADS) void cvt_f32_f16_v8(_Float16 *__restric
     __builtin_nontemporal_store(o, reinterpret_cast<h8_any *>(dst + r * dst_ld + c));
 }
 
-__global__ __launch_bounds__(ST_THREADS) void cvt_f16_f32_v8(float *__restrict__ dst, size_t dst_ld,
+__global__ __launch_bounds__(ST_THREADS) void cvt_f16_f32_v4(float *__restrict__ dst, size_t dst_ld,
                                                              const _Float16 *__restrict__ src, size_t src_ld,
                                                              unsigned colg, size_t cols, size_t total) {
     const unsigned i = blockIdx.x * ST_THREADS + threadIdx.x;
     if (i >= total) return;
     const unsigned r = i / colg;
-    const size_t c = last_whole((size_t)8 * (i - r * colg), 8, cols);
-    const h8 v = __builtin_nontemporal_load(reinterpret_cast<const h8_any *>(src + r * src_ld + c));
-    v4f a, b;
+    const size_t c = last_whole((size_t)4 * (i - r * colg), 4, cols);
+    const h4 v = __builtin_nontemporal_load(reinterpret_cast<const h4_any *>(src + r * src_ld + c));
+    v4f a;
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        a[j] = (float)v[j];
-        b[j] = (float)v[4 + j];
-    }
+    for (int j = 0; j < 4; j++) a[j] = (float)v[j];
     float *d = dst + r * dst_ld + c;
     st4_nt(d, a);
-    st4_nt(d + 4, b);
 }
 
 __global__ __launch_bounds__(ST_THREADS) void cvt_f32_f16_v1(_Float16 *__restrict__ dst, size_t dst_ld,
@@ -88,10 +91,10 @@ __device__ __forceinline__ void load_cols(float (&o)[VEC], const T *p) {
     if constexpr (VEC == 1) {
         o[0] = (float)p[0];
     } else if constexpr (sizeof(T) == 2) {
-        static_assert(VEC == 8, "fp16 rows are read 8 columns at a time");
-        const h8 v = __builtin_nontemporal_load(reinterpret_cast<const h8_any *>(p));
+        static_assert(VEC == 4, "fp16 rows are read 4 columns at a time");
+        const h4 v = __builtin_nontemporal_load(reinterpret_cast<const h4_any *>(p));
 #pragma unroll
-        for (int j = 0; j < 8; j++) o[j] = (float)v[j];
+        for (int j = 0; j < 4; j++) o[j] = (float)v[j];
     } else {
         static_assert(VEC == 4, "fp32 rows are read 4 columns at a time");
         const v4f v = ld4_nt(reinterpret_cast<const float *>(p));
@@ -130,8 +133,9 @@ __device__ __forceinline__ void store_cols(float *p, const float (&o)[VEC]) {
 
 // One lane = one interleaved row pair (2i, 2i+1) of one output head x VEC columns (rows of any length >= VEC: the last
 // lane of a row as in the converts, so not in place where S % VEC != 0: a neighbour in another wave could read what this
-// lane has rotated; one column per lane there).  [8][2048][1001] fp16 in: 89.4 us with one column per lane, now 50.1;
-// [16][2048][250] 48.1 and 26.9.  Pair rows are numbered Q heads first, then K heads, then V heads.
+// lane has rotated; one column per lane there).  [8][2048][1001] fp16 in: 89.4 us with one column per lane, now 45.2.
+// Four columns per lane for fp16 too, whose stores are then whole lines: [16][2048][256] 22.4 us (117 MB: 5.2 TB/s)
+// against 25.2 with eight, [16][2048][250] 24.6 against 26.9 (48.1 with one).  Pair rows are numbered Q heads first, then K heads, then V heads.
 template <typename T, int VEC>
 __global__ __launch_bounds__(ST_THREADS) void attn_grads_finish_kernel(
     float *dq, float *__restrict__ dk, float *__restrict__ dv, const T *qf, const T *__restrict__ kf,
@@ -234,14 +238,21 @@ MI355_API int mi355_cvt_f16_f32_dev(float *dst, size_t dst_ld, const uint16_t *s
     if (cvt_args("cvt_f16_f32", dst, src, dst_ld, src_ld, rows, cols)) return -1;
     const _Float16 *s = reinterpret_cast<const _Float16 *>(src);
     if (dst_ld == cols && src_ld == cols) { cols *= rows; rows = 1; }       // no gaps: one row
-    if (cols >= 8) {
-        const size_t colg = ceil_div(cols, (size_t)8), total = rows * colg;
-        hipLaunchKernelGGL(cvt_f16_f32_v8, dim3((unsigned)ceil_div(total, ST_THREADS)), dim3(ST_THREADS), 0,
-                           g_ctx.stream, dst, dst_ld, s, src_ld, (unsigned)colg, cols, total);
-    } else {
-        const size_t total = rows * cols;
-        hipLaunchKernelGGL(cvt_f16_f32_v1, dim3((unsigned)ceil_div(total, ST_THREADS)), dim3(ST_THREADS), 0,
-                           g_ctx.stream, dst, dst_ld, s, src_ld, cols, total);
+    // (pieces of what one launch can number, for rectangles of more than 8 G elements)
+    for (size_t c0 = 0; c0 < cols; c0 += 4 * ST_LANES) {
+        const size_t n = std::min(cols - c0, 4 * ST_LANES), colg = n >= 4 ? ceil_div(n, (size_t)4) : n;
+        const size_t per = ST_LANES / colg;
+        for (size_t r0 = 0; r0 < rows; r0 += per) {
+            const size_t total = std::min(rows - r0, per) * colg;
+            const dim3 grid((unsigned)ceil_div(total, ST_THREADS));
+            float *d = dst + r0 * dst_ld + c0;
+            const _Float16 *from = s + r0 * src_ld + c0;
+            if (n >= 4)
+                hipLaunchKernelGGL(cvt_f16_f32_v4, grid, dim3(ST_THREADS), 0, g_ctx.stream, d, dst_ld, from, src_ld,
+                                   (unsigned)colg, n, total);
+            else
+                hipLaunchKernelGGL(cvt_f16_f32_v1, grid, dim3(ST_THREADS), 0, g_ctx.stream, d, dst_ld, from, src_ld, n, total);
+        }
     }
     LAUNCH_OK("cvt_f16_f32");
     return 0;
@@ -265,18 +276,24 @@ MI355_API int mi355_attn_grads_finish_dev(float *dq, float *dk, float *dv, const
     if (q_stride < full || k_stride < full || v_stride < full)
         return mi355_fail("attn_grads_finish: sequence stride below heads*hd*S = %zu", full);
     const int ratio = heads / kv_heads;
-    const size_t pair_rows = (size_t)batch * (heads + 2 * kv_heads) * (hd / 2);
     const bool in_place = (const void *)dq == dq_full || (const void *)dk == dk_full || (const void *)dv == dv_full;
+    const size_t pairs = (size_t)(heads + 2 * kv_heads) * (hd / 2);        // of one sequence
+    auto launch = [&](auto kernel, auto *q, auto *k, auto *v, int vec) {
+        const size_t lanes = pairs * ceil_div((size_t)S, (size_t)vec);
+        const int per = (int)std::min<size_t>(std::max<size_t>(ST_LANES / lanes, 1), (size_t)batch);   // sequences of one launch
+        const size_t kv_full = (size_t)kv_heads * hd * S;
+        for (int b = 0; b < batch; b += std::min(per, batch - b)) {
+            const int n = std::min(per, batch - b);
+            hipLaunchKernelGGL(kernel, dim3((unsigned)ceil_div(lanes * n, ST_THREADS)), dim3(ST_THREADS), 0, g_ctx.stream,
+                               dq + b * full, dk + b * kv_full, dv + b * kv_full, q + b * q_stride, k + b * k_stride,
+                               v + b * v_stride, q_stride, k_stride, v_stride, heads, kv_heads, ratio, hd, S, n, cos_dev,
+                               sin_dev, lanes * n);
+        }
+    };
 #define FINISH(T, VEC)                                                                                               \
-    do {                                                                                                             \
-        const size_t total = pair_rows * ceil_div((size_t)S, (size_t)(VEC));                                         \
-        hipLaunchKernelGGL((attn_grads_finish_kernel<T, VEC>), dim3((unsigned)ceil_div(total, ST_THREADS)),          \
-                           dim3(ST_THREADS), 0, g_ctx.stream, dq, dk, dv, (const T *)dq_full, (const T *)dk_full,    \
-                           (const T *)dv_full, q_stride, k_stride, v_stride, heads, kv_heads, ratio, hd, S, batch,   \
-                           cos_dev, sin_dev, total);                                                                 \
-    } while (0)
+    launch(attn_grads_finish_kernel<T, VEC>, (const T *)dq_full, (const T *)dk_full, (const T *)dv_full, VEC)
     if (in_f16) {
-        if (S % 8 == 0 || (S > 8 && !in_place)) FINISH(_Float16, 8);
+        if (S % 4 == 0 || (S > 4 && !in_place)) FINISH(_Float16, 4);
         else FINISH(_Float16, 1);
     } else {
         if (S % 4 == 0 || (S > 4 && !in_place)) FINISH(float, 4);
