@@ -183,19 +183,18 @@ __device__ __forceinline__ float wave_sum_far_first(float v) {
 }
 
 // exp(d) for d <= 0 through the hardware exp2: the product d*log2(e) is carried in two floats
-// so the result keeps ~1 ulp for |d| up to ~100 (a single-float product loses |d|*2^-24).
+// so the result keeps ~1 ulp for |d| up to ~100 (a single-float product loses |d|*2^-24).  A NaN stays one: the clamp is
+// IEEE 754-2019's maximum (v_maximum3_f32), where fmaxf would take the bound in its place.
 __device__ __forceinline__ float exp_neg(float d) {
     const float L2E_HI = 1.44269502162933349609375f;      // float(log2 e)
     const float L2E_LO = 1.925963033500011e-08f;          // log2 e - L2E_HI
-    d = fmaxf(d, -200.0f);                                // exp2 of the product is already 0 there; keeps -inf finite
+    d = __builtin_elementwise_maximum(d, -200.0f);        // exp2 of the product is already 0 there; keeps -inf finite
     float hi = d * L2E_HI;
     float lo = __builtin_fmaf(d, L2E_HI, -hi) + d * L2E_LO;
     float e = __builtin_amdgcn_exp2f(hi);
     return __builtin_fmaf(e, lo * 0.693147180559945f, e);
 }
 
-// exp(d) for d <= 0 with a single-float product: relative error up to |d| * 6e-8.  Used where the
+// exp(d) for d <= 0 with a single-float product: relative error up to |d| * 6e-8; 0 for -inf, NaN for NaN.  Used where the
 // values are only summed (terms with large |d| are negligible there).
-__device__ __forceinline__ float exp_neg_fast(float d) {
-    return __builtin_amdgcn_exp2f(fmaxf(d, -200.0f) * 1.44269502162933349609375f);
-}
+__device__ __forceinline__ float exp_neg_fast(float d) { return __builtin_amdgcn_exp2f(d * 1.44269502162933349609375f); }

@@ -93,6 +93,12 @@ __device__ __forceinline__ void st_cols(uint16_t *p, const float (&o)[VEC]) {
     }
 }
 
+// Maximum of a (max, sum exp) pair before it has seen a value above: a finite number, so that what follows needs no case for
+// a part that is empty or all -inf (its sum is 0) or holds NaNs only (a maximum does not see them, x - max is one and the
+// sum keeps it).  A column with a NaN, with +inf (inf - inf) or of -inf alone (0 / 0) ends as NaNs, loss and gradient, as in
+// the sequential loop.
+constexpr float NO_MAX = -3.402823466e+38f;
+
 // grid: (row blocks, column strips of 64*VEC)
 template <int VEC, typename T>
 __global__ __launch_bounds__(CE_THREADS) void ce_partial_kernel(float *__restrict__ pm, float *__restrict__ pl,
@@ -107,7 +113,7 @@ __global__ __launch_bounds__(CE_THREADS) void ce_partial_kernel(float *__restric
 
     float m[VEC], l[VEC];
 #pragma unroll
-    for (int j = 0; j < VEC; j++) { m[j] = -INFINITY; l[j] = 0.f; }
+    for (int j = 0; j < VEC; j++) { m[j] = NO_MAX; l[j] = 0.f; }
 
     for (int base = v_lo; base < v_hi; base += CE_TILE_ROWS) {
         float x[CE_CAP][VEC];
@@ -126,13 +132,11 @@ __global__ __launch_bounds__(CE_THREADS) void ce_partial_kernel(float *__restric
 #pragma unroll
             for (int k = 1; k < CE_CAP; k++) tm = fmaxf(tm, x[k][j]);
             const float nm = fmaxf(m[j], tm);
-            if (nm > -INFINITY) {
-                float s = 0.f;
+            float s = 0.f;
 #pragma unroll
-                for (int k = 0; k < CE_CAP; k++) s += exp_neg_fast(x[k][j] - nm);   // exp(-inf) = 0 for masked rows
-                l[j] = l[j] * exp_neg(m[j] - nm) + s;
-                m[j] = nm;
-            }
+            for (int k = 0; k < CE_CAP; k++) s += exp_neg_fast(x[k][j] - nm);   // exp(-inf) = 0 for masked rows
+            l[j] = l[j] * exp_neg(m[j] - nm) + s;
+            m[j] = nm;
         }
     }
 #pragma unroll
@@ -146,10 +150,7 @@ __global__ __launch_bounds__(CE_THREADS) void ce_partial_kernel(float *__restric
             for (int w = 1; w < CE_WAVES; w++) M = fmaxf(M, sm[w][lane * VEC + j]);
             float L = 0.f;
 #pragma unroll
-            for (int w = 0; w < CE_WAVES; w++) {
-                const float mw = sm[w][lane * VEC + j];
-                if (mw > -INFINITY) L += sl[w][lane * VEC + j] * exp_neg(mw - M);
-            }
+            for (int w = 0; w < CE_WAVES; w++) L += sl[w][lane * VEC + j] * exp_neg(sm[w][lane * VEC + j] - M);
             pm[(size_t)blockIdx.x * S + col + j] = M;
             pl[(size_t)blockIdx.x * S + col + j] = L;
         }
@@ -171,23 +172,21 @@ __global__ __launch_bounds__(1024) void ce_combine_kernel(float *__restrict__ co
     __shared__ float sm[CB_GROUPS][CB_COLS], sl[CB_GROUPS][CB_COLS];
     const int cl = threadIdx.x % CB_COLS, g = threadIdx.x / CB_COLS;
     const int t = blockIdx.x * CB_COLS + cl;
-    float m = -INFINITY, l = 0.f;
+    float m = NO_MAX, l = 0.f;
     if (t < S)
         for (int r0 = g; r0 < nblk; r0 += CB_GROUPS * 4) {
             float mr[4], lr[4];
 #pragma unroll
             for (int u = 0; u < 4; u++) {     // four independent loads in flight
                 const int r = r0 + CB_GROUPS * u;
-                mr[u] = r < nblk ? pm[(size_t)r * S + t] : -INFINITY;
+                mr[u] = r < nblk ? pm[(size_t)r * S + t] : NO_MAX;
                 lr[u] = r < nblk ? pl[(size_t)r * S + t] : 0.f;
             }
 #pragma unroll
             for (int u = 0; u < 4; u++) {
                 const float nm = fmaxf(m, mr[u]);
-                if (nm > -INFINITY) {
-                    l = l * exp_neg(m - nm) + lr[u] * exp_neg(mr[u] - nm);
-                    m = nm;
-                }
+                l = l * exp_neg(m - nm) + lr[u] * exp_neg(mr[u] - nm);
+                m = nm;
             }
         }
     sm[g][cl] = m;
@@ -197,10 +196,8 @@ __global__ __launch_bounds__(1024) void ce_combine_kernel(float *__restrict__ co
         if (g < half) {
             const float m0 = sm[g][cl], m1 = sm[g + half][cl];
             const float nm = fmaxf(m0, m1);
-            if (nm > -INFINITY) {
-                sl[g][cl] = sl[g][cl] * exp_neg(m0 - nm) + sl[g + half][cl] * exp_neg(m1 - nm);
-                sm[g][cl] = nm;
-            }
+            sl[g][cl] = sl[g][cl] * exp_neg(m0 - nm) + sl[g + half][cl] * exp_neg(m1 - nm);
+            sm[g][cl] = nm;
         }
         __syncthreads();
     }
@@ -455,22 +452,20 @@ __device__ __forceinline__ void online_update(float &m, float &l, const float (&
 #pragma unroll
     for (int k = 1; k < N; k++) tm = fmaxf(tm, x[k]);
     const float nm = fmaxf(m, tm);
-    if (nm > -INFINITY) {
-        float s = 0.f;
+    float s = 0.f;
 #pragma unroll
-        for (int k = 0; k < N; k++) s += exp_neg_fast(x[k] - nm);     // exp(-inf) = 0 for masked rows
-        l = l * exp_neg(m - nm) + s;
-        m = nm;
-    }
+    for (int k = 0; k < N; k++) s += exp_neg_fast(x[k] - nm);        // exp(-inf) = 0 for masked rows
+    l = l * exp_neg(m - nm) + s;
+    m = nm;
 }
 // Sixteen (max, sum) pairs per column, [16][CR_P] in LDS -> their merge, in the quad of threads 4c .. 4c+3 of column c
 // (waves 0 to 3): the maximum first, then every sum rescaled to it and added in a fixed order.  A pair without rows is
-// (-inf, 0); exp_neg of the NaN that -inf - -inf gives is zero (its fmax drops the NaN).
+// (NO_MAX, 0).
 constexpr int CR_P = CR_W + 16;              // row pitch: the four threads of a quad read four rows of a column
 __device__ __forceinline__ void cr_merge16(const float (*wm)[CR_P], const float (*wl)[CR_P], float &M, float &L) {
     const int c = threadIdx.x >> 2, q = threadIdx.x & 3;
     float mm[CR_NW / 4];
-    M = -INFINITY;
+    M = NO_MAX;
 #pragma unroll
     for (int i = 0; i < CR_NW / 4; i++) { mm[i] = wm[q + 4 * i][c]; M = fmaxf(M, mm[i]); }
     M = fmaxf(M, lane_xor<1>(M));
@@ -510,7 +505,7 @@ __device__ __forceinline__ void cr_member_partial(const CrGeo<typename ST::T> &g
     const Raw ninf = ST::ninf();
     float m[4], l[4];
 #pragma unroll
-    for (int j = 0; j < 4; j++) { m[j] = -INFINITY; l[j] = 0.f; }
+    for (int j = 0; j < 4; j++) { m[j] = NO_MAX; l[j] = 0.f; }
     if constexpr (KEEP) {
         auto foldg = [&](const Raw (&t)[CR_SUB]) {
 #pragma unroll
@@ -519,6 +514,8 @@ __device__ __forceinline__ void cr_member_partial(const CrGeo<typename ST::T> &g
 #pragma unroll
                 for (int u = 0; u < CR_SUB; u++) x4[u] = ST::at(t[u], j);
                 online_update<CR_SUB>(m[j], l[j], x4);
+                // a column at a time: the four in step take 13 registers more than there are ([151936][256] 73 us)
+                asm volatile("" : "+v"(m[j]), "+v"(l[j]));
             }
         };
         // the register rows are asked for first and folded last: they are in flight while the other rows stream
@@ -583,7 +580,7 @@ __device__ __forceinline__ void cr_member_partial(const CrGeo<typename ST::T> &g
     } else {
 #pragma unroll 1
         for (int j = 0; j < 4; j++) {
-            float mj = -INFINITY, lj = 0.f;
+            float mj = NO_MAX, lj = 0.f;
             auto part = [&](int kbeg, int kend) {
 #pragma unroll 1
                 for (int k0 = kbeg; k0 < kend; k0 += CR_SUB) {
@@ -636,7 +633,7 @@ __device__ __forceinline__ void cr_merge_members(const float (&pm)[CR_MPG], cons
     for (int q = 1; q < CR_MPG; q++) M = fmaxf(M, pm[q]);
     float L = 0.f;
 #pragma unroll
-    for (int q = 0; q < CR_MPG; q++) L += pl[q] * exp_neg(pm[q] - M);      // a member that is absent is (-inf, 0)
+    for (int q = 0; q < CR_MPG; q++) L += pl[q] * exp_neg(pm[q] - M);      // a member that is absent has sum 0
     wm[grp][c] = M;
     wl[grp][c] = L;
     __syncthreads();
@@ -723,7 +720,7 @@ __global__ __launch_bounds__(CR_THREADS) void ce_resident_kernel(typename ST::T 
 
     // ---- pass 1: this member's rows, kept; its partial published
     Raw xr[K_REG];
-    float Mp = -INFINITY, Lp = 0.f;
+    float Mp = NO_MAX, Lp = 0.f;
     cr_member_partial<ST, K_REG, K_LDS, true, NT>(g, strip, me, xr, rows_of(), wm, wl, Mp, Lp);
     if (tid < 4 * CR_W && (tid & 3) < 2)
         __hip_atomic_store(ws.slots + (size_t)b * CR_STRIDE + (tid & 3) * CR_W + (tid >> 2),
@@ -744,7 +741,7 @@ __global__ __launch_bounds__(CR_THREADS) void ce_resident_kernel(typename ST::T 
         unsigned pend = 0;
 #pragma unroll
         for (int q = 0; q < CR_MPG; q++) {
-            pm[q] = -INFINITY;
+            pm[q] = NO_MAX;
             pl[q] = 0.f;
             if (q < mpg && mgrp * mpg + q < csplit) pend |= 3u << (2 * q);
         }
@@ -788,7 +785,7 @@ __global__ __launch_bounds__(CR_THREADS) void ce_resident_kernel(typename ST::T 
     }
     // one member's partial from memory, into the threads that hold it
     auto recompute = [&](int s2, int p, float (&qm)[CR_MPG], float (&ql)[CR_MPG]) {
-        float M2 = -INFINITY, L2 = 0.f;
+        float M2 = NO_MAX, L2 = 0.f;
         cr_member_partial<ST, K_REG, K_LDS, false, NT>(g, s2, p, xr, rows_of(), wm, wl, M2, L2);
         if (tid < 4 * CR_W && (tid & 3) == 0) { fb[0][tid >> 2] = M2; fb[1][tid >> 2] = L2; }
         __syncthreads();
@@ -906,7 +903,7 @@ __global__ __launch_bounds__(CR_THREADS) void ce_resident_kernel(typename ST::T 
                 if (failed_loss[s2]) {
                     float qm[CR_MPG], ql[CR_MPG];
 #pragma unroll
-                    for (int q = 0; q < CR_MPG; q++) { qm[q] = -INFINITY; ql[q] = 0.f; }
+                    for (int q = 0; q < CR_MPG; q++) { qm[q] = NO_MAX; ql[q] = 0.f; }
                     for (int p = 0; p < csplit; p++) recompute(s2, p, qm, ql);
                     cr_merge_members(qm, ql, wm, wl, fM, fInv);
                     if (tid < CR_W) {

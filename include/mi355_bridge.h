@@ -299,6 +299,7 @@ int mi355_embed_scatter_add_form(int V, int D, int S, int batch, int aligned);
  * dlogits = (softmax - onehot) * (1/S) * grad_scale; *loss_dev = mean_t -logf(p[tgt]+1e-10f).
  * A target outside [0,V) contributes no loss and leaves its column as the unscaled softmax
  * (stories_cpu_ops.h:98).  dlogits may alias logits.
+ * A column that holds a NaN or +inf, or -inf alone, is NaN throughout, and so is the loss that counts it.
  * Logits of 4 to 1024 columns that are not overwritten in place run as ONE launch
  * that keeps the logits in registers and LDS between the two passes (one workgroup per compute unit; partial
  * sums exchanged inside the launch through a device array of the library, bounded wait as for the RMSNorm); every
