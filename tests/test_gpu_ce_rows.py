@@ -1,6 +1,6 @@
 """The one-launch softmax cross-entropy on rows of any length and every number of row steps: row counts around the
 variants' limits (8 and 16 steps of 64 rows in each of the members, and the LDS rows beyond), strips that do not divide the
-row, short last groups, rows of whole 128-byte lines and others."""
+row, short last groups, rows of whole 128-byte lines and others, tensors that start within a line."""
 import numpy as np
 import pytest
 
@@ -10,13 +10,15 @@ import oracle as O
 pytestmark = pytest.mark.gpu
 
 
-def run(br, logits, tgt, bf16, scale):
+def run(br, logits, tgt, bf16, scale, off=0):
+    """off: elements between the start of an allocation and the tensor, on both sides"""
     dt = np.uint16 if bf16 else np.float32
-    ld = br.DevArray.from_numpy(O.cvt_f32_bf16(logits) if bf16 else logits)
-    td, dl, loss = br.DevArray.from_numpy(tgt), br.DevArray(logits.shape, dt), br.DevArray(1)
-    fn = br.lib.mi355_softmax_ce_bf16_dev if bf16 else br.lib.mi355_softmax_ce_dev
-    br.check(fn(dl.ptr, loss.ptr, ld.ptr, td.ptr, logits.shape[0], logits.shape[1], scale))
-    return loss.numpy().tobytes(), dl.numpy()
+    raw = O.cvt_f32_bf16(logits) if bf16 else logits
+    ld = br.DevArray.from_numpy(np.concatenate([np.zeros(off, dt), raw.ravel()]))
+    td, dl, loss = br.DevArray.from_numpy(tgt), br.DevArray(off + logits.size, dt), br.DevArray(1)
+    fn, at = br.lib.mi355_softmax_ce_bf16_dev if bf16 else br.lib.mi355_softmax_ce_dev, off * dt().itemsize
+    br.check(fn(dl.ptr + at, loss.ptr, ld.ptr + at, td.ptr, logits.shape[0], logits.shape[1], scale))
+    return loss.numpy().tobytes(), dl.numpy()[off:].reshape(logits.shape)
 
 
 # 64 members at S = 197 and 52, 51 at S = 300, 16 at S = 1000: 64 * 512 = 32768 rows are the last that fit 8 steps, 65536 the
@@ -46,3 +48,18 @@ def test_one_launch_on_rows_of_any_length(br, V, S, bf16):
     finally:
         br.tune("xch_take_nothing", 0)
     assert loss2 == loss and dl2.tobytes() == dl.tobytes()
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("V,S", [(9000, 256), (70000, 128)])
+def test_rows_of_whole_lines_at_any_element(br, V, S, bf16):
+    """The same bits wherever the tensors start: past the caches on a line or half a line, through them elsewhere."""
+    logits = H.normal(402, (V, S), 0, 2.0)
+    tgt = np.random.default_rng(403).integers(0, V, S).astype(np.int32)
+    loss, dl = run(br, logits, tgt, bf16, 1.0)
+    rl, rd = O.cross_entropy(O.cvt_bf16_f32(O.cvt_f32_bf16(logits)) if bf16 else logits, tgt, 1.0)
+    assert H.rel_err(O.cvt_bf16_f32(dl) if bf16 else dl, rd) <= (5e-3 if bf16 else 1e-5)
+    assert abs(float(np.frombuffer(loss, np.float32)[0]) - rl) <= 1e-5 * abs(rl)
+    for off in (1, 4, 16, 64):
+        loss2, dl2 = run(br, logits, tgt, bf16, 1.0, off)
+        assert loss2 == loss and dl2.tobytes() == dl.tobytes(), off
