@@ -37,7 +37,7 @@ struct Mi355Ctx {
     int gemm_split;            // sgemm on the bfloat16 instruction (gemm_split.h): 0 = where it pays, -1 = never, 1 / 2 =
                                // always, in tiles of 128 x 256 / 256 x 128
     int rms_cluster;           // channel split of the clustered RMSNorm: 0 = per shape, -1 = never, 2/4/8 = forced
-    int ce_resident;           // one-launch softmax-CE: -1 = never, otherwise whenever the shape allows
+    int ce_resident;           // one-launch softmax-CE: 0 = where it pays, 1 = whenever the shape allows, -1 = never
     int rms_cluster_spin;      // its bounded wait in ticks of the 100 MHz clock: 0 = 2 ms, negative = do not wait at all
     int xch_take_nothing;      // test mode of those kernels: 1 = no partner's value is taken, present or not, so every
                                // workgroup goes the way of an expired wait

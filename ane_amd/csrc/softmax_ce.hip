@@ -963,8 +963,11 @@ int ce_run(const char *who, T *dlogits, float *loss_dev, const T *logits, const 
         // recomputes a partner's partial reads the partner's logits).  One workgroup per compute unit at most, so that
         // all of them are resident at once.  Measured against the three launches, us: fp32 [1000][256] 8.6 against 20
         // (12 with one column per lane), [32000][256] 18.3 against 27, [151936][256] 65.7 against 83, [32000][1000] 71
-        // against 88; bfloat16 [32000][200] 15.3 against 31.6, [151936][256] 49 against 88.  Only a single strip of a
-        // large vocabulary, which occupies 64 of the compute units, is close: fp32 [151936][63] 42 against 38.
+        // against 88; bfloat16 [32000][200] 15.3 against 31.6, [151936][256] 49 against 88.
+        // Not for a single strip of fp32 whose members have more than 14 row steps (V > 57344 in 64 members): its 64
+        // workgroups leave three quarters of the chip idle.  [50000][63] 19.0 against 20.0, [65536][63] 20.8 against 20.3,
+        // [90000][64] 28.5 against 23.9, [151936][63] 44.5 against 34.5, [151936][4] 41 against 23.  (bfloat16, whose three
+        // launches convert twice: [151936][63] 44 against 56; two strips: [151936][65] 46 against 50.)
         typedef typename std::conditional<std::is_same<T, float>::value, CrF32, CrBf16>::type ST;
         const int cu = g_ctx.num_cu > 0 ? g_ctx.num_cu : 256;
         const int strips_r = (int)ceil_div((size_t)S, (size_t)CR_W);
@@ -979,7 +982,8 @@ int ce_run(const char *who, T *dlogits, float *loss_dev, const T *logits, const 
             const int csplit = cu / strips_r < CR_MAX_SPLIT ? cu / strips_r : CR_MAX_SPLIT;
             const int Rm = csplit > 0 ? (int)ceil_div((size_t)V, (size_t)csplit) : 0;
             const int K = (int)ceil_div((size_t)Rm, (size_t)CR_RPS);
-            if (csplit >= 2 && csplit * strips_r <= CR_MAX_WG && csplit * strips_r <= cu && K <= CR_MAX_STEPS) {
+            if (csplit >= 2 && csplit * strips_r <= CR_MAX_WG && csplit * strips_r <= cu && K <= CR_MAX_STEPS &&
+                !(std::is_same<T, float>::value && strips_r == 1 && K > 14 && g_ctx.ce_resident == 0)) {
                 CeXch xch;
                 xch.slots = (unsigned long long *)(base + CE_SCRATCH_BYTES);
                 xch.cnt = (unsigned *)(base + CE_SCRATCH_BYTES + (size_t)CR_MAX_WG * CR_STRIDE * 8);
@@ -1044,17 +1048,18 @@ int ce_run(const char *who, T *dlogits, float *loss_dev, const T *logits, const 
 
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const size_t part_b = al((size_t)nblk * S * sizeof(float)), col_b = al((size_t)S * sizeof(float));
-    char *ws;
-    if (no_alloc) {
-        if (2 * part_b + 3 * col_b > CE_SCRATCH_BYTES)
+    // The fixed scratch array where it is large enough (it always is for the single strips above, which therefore can be
+    // recorded without a call that sizes the workspace), else the workspace.
+    char *ws = (g_ctx.device >= 0 && g_ctx.device < CE_MAX_DEVICES) ? (char *)g_scratch_ptr[g_ctx.device] : nullptr;
+    if (no_alloc && !ws) return mi355_fail("%s: the scratch array was not located at init", who);
+    if (2 * part_b + 3 * col_b > CE_SCRATCH_BYTES) {
+        if (no_alloc)
             return mi355_fail("%s: V=%d S=%d needs %zu bytes of scratch, the fixed scratch holds %zu "
                               "(use mi355_softmax_ce_dev, whose workspace grows)", who, V, S, 2 * part_b + 3 * col_b,
                               CE_SCRATCH_BYTES);
-        ws = (g_ctx.device >= 0 && g_ctx.device < CE_MAX_DEVICES) ? (char *)g_scratch_ptr[g_ctx.device] : nullptr;
-        if (!ws) return mi355_fail("%s: the scratch array was not located at init", who);
-    } else {
-        ws = (char *)mi355_ws(2 * part_b + 3 * col_b);
+        ws = nullptr;
     }
+    if (!ws) ws = (char *)mi355_ws(2 * part_b + 3 * col_b);
     if (!ws) return -1;
     float *pm = (float *)ws, *pl = (float *)(ws + part_b);
     float *colM = (float *)(ws + 2 * part_b), *colInv = (float *)(ws + 2 * part_b + col_b);

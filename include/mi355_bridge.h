@@ -66,7 +66,7 @@ size_t mi355_workspace_size(void);
  * 0 = a multiple of 128 bytes that rotates from one allocation to the next, 1..8 = always (value-1)*128),
  * "rms_cluster" (channel split of the RMSNorm over cooperating workgroups: -1 = never, and mi355_int8_scale_dev and
  * mi355_int8_quantize_dynamic_dev then run as two launches each; 2/4/8 = forced),
- * "ce_resident" (one-launch softmax-CE: -1 = never), "rms_cluster_spin" (how long a workgroup of those
+ * "ce_resident" (one-launch softmax-CE: -1 = never, 1 = whenever the shape allows), "rms_cluster_spin" (how long a workgroup of those
  * kernels and of mi355_int8_scale_dev waits for a partner's partial result before it computes it itself, in ticks
  * of 10 ns: 0 = 2 ms; -1 = do not wait), "xch_take_nothing" (1: those kernels take no partner's value at
  * all, present or not, so every workgroup goes the way of an expired wait).  The last two settings are for tests: the
@@ -303,9 +303,10 @@ int mi355_embed_scatter_add_form(int V, int D, int S, int batch, int aligned);
  * Logits of 4 to 1024 columns that are not overwritten in place run as ONE launch
  * that keeps the logits in registers and LDS between the two passes (one workgroup per compute unit; partial
  * sums exchanged inside the launch through a device array of the library, bounded wait as for the RMSNorm); every
- * other call runs as three launches that read the logits twice.  Both forms are deterministic; they sum in
- * different orders, so their results differ in the last bits.  Tuning knob "ce_resident": 0 or 1 = as described,
- * -1 = never the one-launch form. */
+ * other call runs as three launches that read the logits twice, and so do fp32 logits of at most 64 columns and more than
+ * 57344 rows, which would keep only 64 of the compute units busy.  Both forms are deterministic; they sum in
+ * different orders, so their results differ in the last bits.  Tuning knob "ce_resident": 0 = as described, 1 = one launch
+ * for the latter too, -1 = never the one-launch form. */
 int mi355_softmax_ce_dev(float *dlogits, float *loss_dev, const float *logits,
                          const int32_t *targets, int V, int S, float grad_scale);
 

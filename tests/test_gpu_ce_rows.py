@@ -10,14 +10,18 @@ import oracle as O
 pytestmark = pytest.mark.gpu
 
 
-def run(br, logits, tgt, bf16, scale, off=0):
-    """off: elements between the start of an allocation and the tensor, on both sides"""
+def run(br, logits, tgt, bf16, scale, off=0, one_launch=1):
+    """off: elements between the start of an allocation and the tensor, on both sides; one_launch: the knob's value"""
     dt = np.uint16 if bf16 else np.float32
     raw = O.cvt_f32_bf16(logits) if bf16 else logits
     ld = br.DevArray.from_numpy(np.concatenate([np.zeros(off, dt), raw.ravel()]))
     td, dl, loss = br.DevArray.from_numpy(tgt), br.DevArray(off + logits.size, dt), br.DevArray(1)
     fn, at = br.lib.mi355_softmax_ce_bf16_dev if bf16 else br.lib.mi355_softmax_ce_dev, off * dt().itemsize
-    br.check(fn(dl.ptr + at, loss.ptr, ld.ptr + at, td.ptr, logits.shape[0], logits.shape[1], scale))
+    br.tune("ce_resident", one_launch)
+    try:
+        br.check(fn(dl.ptr + at, loss.ptr, ld.ptr + at, td.ptr, logits.shape[0], logits.shape[1], scale))
+    finally:
+        br.tune("ce_resident", 0)
     return loss.numpy().tobytes(), dl.numpy()[off:].reshape(logits.shape)
 
 
@@ -63,3 +67,42 @@ def test_rows_of_whole_lines_at_any_element(br, V, S, bf16):
     for off in (1, 4, 16, 64):
         loss2, dl2 = run(br, logits, tgt, bf16, 1.0, off)
         assert loss2 == loss and dl2.tobytes() == dl.tobytes(), off
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("S", [37, 64])
+def test_a_single_strip_of_a_large_vocabulary_takes_three_launches(br, S, bf16):
+    """14 row steps of 64 rows in 64 members are the last that one launch takes there (fp32), and the other form needs no
+    call that sizes a workspace before a graph is recorded, as the one launch does not."""
+    for V in (57344, 57345):
+        logits = H.normal(404, (V, S), 0, 2.0)
+        tgt = np.random.default_rng(405).integers(0, V, S).astype(np.int32)
+        want = run(br, logits, tgt, bf16, 1.0, 0, 0)
+        rl, rd = O.cross_entropy(O.cvt_bf16_f32(O.cvt_f32_bf16(logits)) if bf16 else logits, tgt, 1.0)
+        assert H.rel_err(O.cvt_bf16_f32(want[1]) if bf16 else want[1], rd) <= (5e-3 if bf16 else 1e-5)
+        assert abs(float(np.frombuffer(want[0], np.float32)[0]) - rl) <= 1e-5 * abs(rl)
+        expired = br.exchange_fallbacks()[1]
+        try:
+            br.tune("xch_take_nothing", 1)                    # counted by the one launch only
+            got = run(br, logits, tgt, bf16, 1.0, 0, 0)
+        finally:
+            br.tune("xch_take_nothing", 0)
+        assert (br.exchange_fallbacks()[1] > expired) == (bf16 or V == 57344)
+        assert got[0] == want[0] and got[1].tobytes() == want[1].tobytes()
+    if bf16:
+        return
+    L = br.lib
+    ld, td, dl, loss = br.DevArray.from_numpy(logits), br.DevArray.from_numpy(tgt), br.DevArray((V, S)), br.DevArray(1)
+    ws = L.mi355_workspace_size()
+    br.check(L.mi355_graph_begin())
+    br.check(L.mi355_softmax_ce_dev(dl.ptr, loss.ptr, ld.ptr, td.ptr, V, S, 1.0))
+    g = L.mi355_graph_end()
+    assert g, br.last_error()
+    assert L.mi355_workspace_size() == ws
+    for _ in range(3):
+        br.check(L.mi355_graph_launch(g))
+        assert loss.numpy().tobytes() == want[0] and dl.numpy().tobytes() == want[1].tobytes()
+        run(br, logits[:40000], np.zeros(S, np.int32), False, 2.0, 0, -1)         # other values in the scratch
+        br.check(L.mi355_buf_zero(dl.handle))
+        br.sync()
+    L.mi355_graph_free(g)
