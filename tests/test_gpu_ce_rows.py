@@ -106,3 +106,23 @@ def test_a_single_strip_of_a_large_vocabulary_takes_three_launches(br, S, bf16):
         br.check(L.mi355_buf_zero(dl.handle))
         br.sync()
     L.mi355_graph_free(g)
+
+
+@pytest.mark.parametrize("V,S,bf16", [(65536, 1000, False), (262144, 5, True)])
+def test_one_launch_up_to_64_row_steps(br, V, S, bf16):
+    """16 members at S = 1000, 64 at S = 5: the last V that one launch takes, and the next, which are three; the two forms
+    sum in different orders and agree within the parity bar."""
+    for v, one in ((V, True), (V + 1, False)):
+        logits = np.random.default_rng(406).standard_normal((v, S), dtype=np.float32)
+        tgt = np.random.default_rng(407).integers(0, v, S).astype(np.int32)
+        loss, dl = run(br, logits, tgt, bf16, 1.0, 0, -1)
+        try:
+            br.tune("xch_take_nothing", 1)                    # counted by the one launch only
+            expired = br.exchange_fallbacks()[1]
+            loss1, dl1 = run(br, logits, tgt, bf16, 1.0, 0, 0)
+        finally:
+            br.tune("xch_take_nothing", 0)
+        assert (br.exchange_fallbacks()[1] > expired) == one
+        assert abs(np.frombuffer(loss1, np.float32)[0] / np.frombuffer(loss, np.float32)[0] - 1) <= 1e-5
+        a, b = (O.cvt_bf16_f32(d) if bf16 else d for d in (dl1, dl))
+        assert np.max(np.abs(a - b) / np.maximum(np.abs(b), np.float32(1e-3 / v / S))) <= (2.0 ** -7 if bf16 else 1e-5)
