@@ -912,7 +912,7 @@ MI355_API int mi355_qknorm_rope_fwd_bf16_dev(uint16_t *q_out, uint16_t *k_out, c
     if (!cos_dev || !sin_dev || (heads > 0 && (!q_out || !q || !wq)) || (kv_heads > 0 && (!k_out || !k || !wk)))
         return mi355_fail("qknorm_rope_fwd_bf16: NULL pointer");
     QkBf cfg;
-    if (!pick_qk_bf(hd, S, q_out == q || k_out == k, false, cfg))
+    if (!pick_qk_bf(hd, S, (heads > 0 && q_out == q) || (kv_heads > 0 && k_out == k), false, cfg))
         return mi355_fail("qknorm_rope_fwd_bf16: head size %d does not fit the register tile for this layout", hd);
     const int strips = (int)ceil_div((size_t)S, (size_t)cfg.lpr * cfg.vec);
     const int nq = batch * heads * strips, nk = batch * kv_heads * strips;
@@ -934,7 +934,7 @@ MI355_API int mi355_qknorm_rope_bwd_bf16_dev(uint16_t *dq, uint16_t *dk, float *
         (kv_heads > 0 && (!dk || !dwk || !dk_out || !k || !wk)))
         return mi355_fail("qknorm_rope_bwd_bf16: NULL pointer");
     QkBf cfg;
-    if (!pick_qk_bf(hd, S, dq == dq_out || dk == dk_out, true, cfg))
+    if (!pick_qk_bf(hd, S, (heads > 0 && dq == dq_out) || (kv_heads > 0 && dk == dk_out), true, cfg))
         return mi355_fail("qknorm_rope_bwd_bf16: head size %d does not fit the register tile for this layout", hd);
     const int strips = (int)ceil_div((size_t)S, (size_t)cfg.lpr * cfg.vec);
     const int nq = batch * heads * strips, nk = batch * kv_heads * strips;

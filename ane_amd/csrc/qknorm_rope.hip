@@ -241,7 +241,7 @@ MI355_API int mi355_qknorm_rope_fwd_dev(float *q_out, float *k_out, const float 
     if (!cos_dev || !sin_dev || (heads > 0 && (!q_out || !q || !wq)) || (kv_heads > 0 && (!k_out || !k || !wk)))
         return mi355_fail("qknorm_rope_fwd: NULL pointer");
     QkCfg cfg;
-    if (!pick_qk(hd, S, q_out == q || k_out == k, cfg, false)) {
+    if (!pick_qk(hd, S, (heads > 0 && q_out == q) || (kv_heads > 0 && k_out == k), cfg, false)) {
         // unfused composition: per-head norm (heads folded into the batch), then the rotation in place
         if (heads > 0 && mi355_rmsnorm_fwd_dev(q_out, q, wq, hd, S, batch * heads, eps)) return -1;
         if (kv_heads > 0 && mi355_rmsnorm_fwd_dev(k_out, k, wk, hd, S, batch * kv_heads, eps)) return -1;
@@ -266,7 +266,7 @@ MI355_API int mi355_qknorm_rope_bwd_dev(float *dq, float *dk, float *dwq, float 
         (kv_heads > 0 && (!dk || !dwk || !dk_out || !k || !wk)))
         return mi355_fail("qknorm_rope_bwd: NULL pointer");
     QkCfg cfg;
-    if (!pick_qk(hd, S, dq == dq_out || dk == dk_out, cfg, true)) {
+    if (!pick_qk(hd, S, (heads > 0 && dq == dq_out) || (kv_heads > 0 && dk == dk_out), cfg, true)) {
         // unfused composition: inverse rotation into dq/dk, then the per-head norm backward in place
         if (mi355_rope_dev(dq, dk, dq_out, dk_out, heads, kv_heads, hd, S, batch, cos_dev, sin_dev, -1)) return -1;
         if (heads > 0 && mi355_rmsnorm_bwd_dev(dq, dwq, dq, q, wq, hd, S, batch * heads, eps, variant)) return -1;

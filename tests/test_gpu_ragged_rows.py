@@ -111,3 +111,23 @@ def test_rope_and_qknorm_on_rows_of_any_length(br, B, heads, kvh, hd, S, bf16):
                                           B, cd, sd, 1e-5, 0))
         assert H.rel_err(st.get(dq, q.shape), rdq) <= tol and H.rel_err(st.get(dk, k.shape), rdk) <= tol
         assert H.rel_err(dwq.numpy(), rdwq) <= TOL and H.rel_err(dwk.numpy(), rdwk) <= TOL
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("which", ["q", "k"])
+def test_qknorm_of_one_operand_alone_is_not_in_place(br, which, bf16):
+    """heads = 0 or kv_heads = 0 with NULL for what is absent: those equal pointers are no call in place, whose rows of this
+    length go one column per lane, which holds no head of 256."""
+    B, n, hd, S = 1, 2, 256, 257
+    st = Store(br, bf16, 0)
+    x, g, w = st.values(H.normal(350, (B, n * hd, S))), st.values(H.normal(351, (B, n * hd, S))), H.normal(352, hd, 1.0, 0.02)
+    wd, xd, gd, dw = br.DevArray.from_numpy(w), st.put(x), st.put(g), br.DevArray(hd)
+    cd, sd = br.rope_tables_dev(S, hd, 1e4)
+    both = lambda a: (a, None) if which == "q" else (None, a)
+    counts = (n, 0) if which == "q" else (0, n)
+    y, dx = st.new(x.shape), st.new(x.shape)
+    br.check(st.fn("qknorm_rope_fwd")(*both(y), *both(xd), *both(wd.ptr), *counts, hd, S, B, cd, sd, 1e-5))
+    assert H.rel_err(st.get(y, x.shape), O.qknorm_rope_fwd(x, w, hd, 1e4)) <= st.tol
+    br.check(st.fn("qknorm_rope_bwd")(*both(dx), *both(dw.ptr), *both(gd), *both(xd), *both(wd.ptr), *counts, hd, S, B, cd, sd, 1e-5, 0))
+    rdx, rdw = O.qknorm_rope_bwd(g, x, w, hd, 1e4)
+    assert H.rel_err(st.get(dx, x.shape), rdx) <= st.tol and H.rel_err(dw.numpy(), rdw) <= TOL
