@@ -561,21 +561,39 @@ struct QkBf {
     int vec, lpr, threads, cap;
 };
 
-// Widest strip whose row pairs fit the (packed) register tile: 16 lanes x 8 columns = 256-byte row segments first;
-// 64-byte segments run at little more than half the rate.  One-column lanes (rows of fewer than eight columns, in-place
-// calls whose short last group of columns would be shared by two workgroups) hold at most four pairs.
-bool pick_qk_bf(int hd, int S, bool in_place, bool backward, QkBf &cfg) {
+// The tile for `slabs` head slabs of [hd][S].  Small tensors take one column per lane on 1024 threads: with few strips to
+// go round, waves count for more than bytes per access.  us, one column per lane / eight:
+//   hd 128, 24 heads   fwd  [1][257] 5.0 / 9.8   [4][257] 7.4 / 9.5    [8][257] 12.0 / 11.8   [8][500] 18.2 / 15.1
+//                      bwd       9.7 / 13.7          15.7 / 16.0            25.9 / 23.1            39.0 / 31.5
+//   hd 64, 24 heads    fwd  [4][197] 5.2 / 6.6   [8][197] 7.3 / 7.6    [16][197] 12.1 / 9.5
+//                      bwd      11.1 / 12.6          15.0 / 13.6             25.4 / 17.1
+// The line lies between [8][197] and [8][250] of hd 64 and between [4][257] and [8][129] of hd 128; shorter heads leave the
+// 64 pairs of the former mostly empty (hd 32 fwd [4][257] 5.0 / 6.2, [16][77] 5.9 / 5.1).  Eight columns per lane:
+// 16 lanes to a row, with two row pairs per lane where that takes 256 or 512 threads (hd 128 forward on 256 threads with
+// four pairs: [8][257] 14.6 for 11.8; hd 64 backward on 512 with one: [8][257] 25.7 for 16.2); 8 lanes where 16 would leave
+// most of a strip empty (rows of up to 64 columns: fwd hd 128 [32][33] 8.0 for 10.0; in the backward of long heads from a
+// sixth on: [8][257] 23.1 for 28.8, [16][197] 37.3 for 30.6).
+// Rows of fewer than eight columns, and in-place calls whose short last group of columns would be shared by two workgroups,
+// have no choice; a lane of one column holds at most four pairs, one of eight columns what fits 16, 8 or 4 lanes.
+bool pick_qk_bf(int hd, int S, size_t slabs, bool in_place, bool backward, QkBf &cfg) {
     const int half = hd / 2;
-    auto fits = [&](int lpr, int threads, int cap) {
-        cfg = QkBf{8, lpr, threads, cap};
-        return (threads / lpr) * cap >= half && (!in_place || tail_in_strip(S, lpr * 8, 8));
+    const bool small = slabs * hd * S < (half <= 16 ? 800000u : half <= 32 ? 2500000u : 3200000u);
+    const auto padded = [S](int w) { return (S + w - 1) / w * w; };
+    auto fits = [&](int lpr, int threads) {
+        for (int cap : {1, 2, 4}) {
+            cfg = QkBf{8, lpr, threads, cap};
+            if ((threads / lpr) * cap >= half) return !in_place || tail_in_strip(S, lpr * 8, 8);
+        }
+        return false;
     };
-    if (S >= 8) {
-        const int thr = backward ? 512 : 256;
+    if (S >= 8 && half <= 64 && !small) {
+        const bool narrow = S <= 64 || (backward && half > 32 && 5 * padded(128) >= 6 * padded(64));
+        if (fits(narrow ? 8 : 16, narrow || half <= 32 ? 256 : 512)) return true;
+    }
+    if (S >= 8 && (half > 64 || !small)) {              // long heads, and in-place calls for which that strip is too narrow
         for (int lpr : {16, 8, 4})
-            for (int cap : {1, 2, 4})
-                if (fits(lpr, thr, cap)) return true;
-        if (fits(4, 1024, 2)) return true;
+            if (fits(lpr, backward ? 512 : 256)) return true;
+        if (fits(4, 1024)) return true;
     }
     cfg = QkBf{1, 64, 1024, 4};
     return half <= 64;
@@ -912,7 +930,7 @@ MI355_API int mi355_qknorm_rope_fwd_bf16_dev(uint16_t *q_out, uint16_t *k_out, c
     if (!cos_dev || !sin_dev || (heads > 0 && (!q_out || !q || !wq)) || (kv_heads > 0 && (!k_out || !k || !wk)))
         return mi355_fail("qknorm_rope_fwd_bf16: NULL pointer");
     QkBf cfg;
-    if (!pick_qk_bf(hd, S, (heads > 0 && q_out == q) || (kv_heads > 0 && k_out == k), false, cfg))
+    if (!pick_qk_bf(hd, S, (size_t)batch * (heads + kv_heads), (heads > 0 && q_out == q) || (kv_heads > 0 && k_out == k), false, cfg))
         return mi355_fail("qknorm_rope_fwd_bf16: head size %d does not fit the register tile for this layout", hd);
     const int strips = (int)ceil_div((size_t)S, (size_t)cfg.lpr * cfg.vec);
     const int nq = batch * heads * strips, nk = batch * kv_heads * strips;
@@ -934,7 +952,7 @@ MI355_API int mi355_qknorm_rope_bwd_bf16_dev(uint16_t *dq, uint16_t *dk, float *
         (kv_heads > 0 && (!dk || !dwk || !dk_out || !k || !wk)))
         return mi355_fail("qknorm_rope_bwd_bf16: NULL pointer");
     QkBf cfg;
-    if (!pick_qk_bf(hd, S, (heads > 0 && dq == dq_out) || (kv_heads > 0 && dk == dk_out), true, cfg))
+    if (!pick_qk_bf(hd, S, (size_t)batch * (heads + kv_heads), (heads > 0 && dq == dq_out) || (kv_heads > 0 && dk == dk_out), true, cfg))
         return mi355_fail("qknorm_rope_bwd_bf16: head size %d does not fit the register tile for this layout", hd);
     const int strips = (int)ceil_div((size_t)S, (size_t)cfg.lpr * cfg.vec);
     const int nq = batch * heads * strips, nk = batch * kv_heads * strips;

@@ -82,7 +82,10 @@ def test_rmsnorm_family_on_rows_of_any_length(br, B, C, S, bf16, off):
 
 
 @pytest.mark.parametrize("bf16", [False, True])
-@pytest.mark.parametrize("B,heads,kvh,hd,S", [(2, 4, 2, 128, 197), (1, 2, 1, 64, 65), (1, 3, 3, 16, 257), (2, 2, 1, 128, 9), (1, 2, 2, 32, 4)])
+@pytest.mark.parametrize("B,heads,kvh,hd,S", [(2, 4, 2, 128, 197), (1, 2, 1, 64, 65), (1, 3, 3, 16, 257), (2, 2, 1, 128, 9), (1, 2, 2, 32, 4),
+                                                # large enough for eight columns per lane: 16 and 8 lanes, 256 and 512 threads
+                                                (9, 12, 12, 64, 197), (52, 12, 12, 64, 33), (6, 16, 8, 128, 197),
+                                                (6, 16, 8, 128, 257), (32, 16, 8, 128, 33), (40, 12, 12, 32, 100)])
 def test_rope_and_qknorm_on_rows_of_any_length(br, B, heads, kvh, hd, S, bf16):
     print("[case] ragged rope B=%d heads=%d/%d hd=%d S=%d bf16=%d" % (B, heads, kvh, hd, S, bf16), flush=True)
     st = Store(br, bf16, 1)
