@@ -895,8 +895,7 @@ unsigned long long *scatter_report_word(int N, int D) {
 // ids itself (the library sort is slower and cannot be recorded).
 int scatter_form(int N, int D, bool cols_ok, bool whole, bool rows_recordable) {
     if (!cols_ok) return -1;
-    if (g_ctx.capturing && !rows_recordable) return whole || N <= COL_SMALL ? 1 : -1;
-    if (g_ctx.scatter_cols > 0) return 1;
+    if (g_ctx.scatter_cols > 0 || (g_ctx.capturing && !rows_recordable)) return 1;
     const int cu = g_ctx.num_cu > 0 ? g_ctx.num_cu : 256;
     if (N > COLS_MAX_N || (int)ceil_div((size_t)D, cols_per_workgroup(D)) > cu) return -1;
     if (N <= COL_SMALL) return 1;

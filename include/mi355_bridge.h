@@ -284,8 +284,9 @@ int mi355_embed_gather_dev(float *x, const float *E, const int32_t *ids, int V, 
  * a word of pinned host memory, and the next call with the same number of positions and D (up to 65536) takes the form
  * that it makes the faster: same bits, only the time differs.  Without such a word the first form is taken up to 16384
  * positions in sequences of a multiple of 4 (of any length up to 512 positions), else the second.
- * While a graph is recorded, inputs beyond 16384 positions (S a multiple of 4, dx 16-byte aligned) take the first form too
- * (the library sort of the second cannot be recorded). */
+ * The words of eight shapes are kept; two that share one leave each other without.  While a graph is recorded, inputs
+ * beyond 16384 positions or with a vocabulary of 2^18 and more take the first form (the library sort of the second cannot
+ * be recorded); V >= 2^19 is refused. */
 int mi355_embed_scatter_add_dev(float *dE, const float *dx, const int32_t *ids, int V, int D,
                                 int S, int batch);
 /* Which form the next mi355_embed_scatter_add_dev call of this shape would take under the current knobs and the last

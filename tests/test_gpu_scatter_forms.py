@@ -92,3 +92,33 @@ def test_graph_records_a_short_sequence_of_any_length_into_a_large_vocabulary(br
             assert dEd.numpy().tobytes() == want.tobytes()
     finally:
         if g: L.mi355_graph_free(g)
+
+
+@pytest.mark.parametrize("V,D,B,S,shift", [(300000, 8, 5, 197, 1), (3000, 12, 27, 607, 0)])    # 985 positions; 16389
+def test_graph_records_sequences_of_any_length_that_the_library_would_sort(br, V, D, B, S, shift):
+    """The column form reads sequences of any length at any element, so it stands in for the library sort there too."""
+    L = br.lib
+    ids = H.zipf_ids(18, B * S, V).astype(np.int32).reshape(B, S)
+    dx = H.normal(19, (B, D, S)); dE0 = H.normal(20, (V, D))
+    dEd, idd = br.DevArray.from_numpy(dE0), br.DevArray.from_numpy(ids)
+    dxd = br.DevArray.from_numpy(np.concatenate([np.zeros(shift, np.float32), dx.ravel()]))
+    call = lambda e: L.mi355_embed_scatter_add_dev(e.ptr, dxd.ptr + 4 * shift, idd.ptr, V, D, S, B)
+    eager = br.DevArray.from_numpy(dE0)
+    br.check(call(eager))                               # also sizes the workspace
+    br.sync()
+    br.check(L.mi355_graph_begin())
+    got = call(dEd)
+    why = br.last_error()
+    g = L.mi355_graph_end()
+    try:
+        assert got == 0 and g, why
+        want = dE0
+        for _ in range(3):
+            br.check(L.mi355_graph_launch(g))
+            want = O.embed_backward(want, dx, ids)
+            assert dEd.numpy().tobytes() == want.tobytes()
+            br.check(call(eager))                       # the program's own eager work between replays
+            br.sync()
+        assert eager.numpy().tobytes() == O.embed_backward(want, dx, ids).tobytes()
+    finally:
+        if g: L.mi355_graph_free(g)
