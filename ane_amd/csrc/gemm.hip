@@ -297,19 +297,9 @@ GemmPlan plan_gemm(int M, int N, int K, bool reads_c, int lda, int ldb) {
     return best;
 }
 
-}   // namespace
-
-MI355_API int mi355_sgemm_dev(int trans_a, int trans_b, int M, int N, int K, float alpha, const float *A, int lda,
-                              const float *B, int ldb, float beta, float *C, int ldc) {
-    if (!mi355_ready("sgemm")) return -1;
-    if (!mi355_outside_capture("sgemm (its K slices may need workspace)")) return -1;
-    if (!A || !B || !C) return mi355_fail("sgemm: NULL pointer");
-    const int ta = trans_flag(trans_a), tb = trans_flag(trans_b);
-    if (ta < 0 || tb < 0) return mi355_fail("sgemm: transpose flags must be 0/1 (or CblasNoTrans/CblasTrans)");
-    if (M <= 0 || N <= 0 || K <= 0) return mi355_fail("sgemm: bad shape M=%d N=%d K=%d", M, N, K);
-    // row-major leading dimensions: A is M x K (or K x M when transposed), B is K x N (or N x K), C is M x N
-    if (lda < (ta ? M : K) || ldb < (tb ? K : N) || ldc < N)
-        return mi355_fail("sgemm: leading dimension too small (lda=%d ldb=%d ldc=%d)", lda, ldb, ldc);
+// The product within the limits of one launch: M, K <= 2^30, fewer than 2^24 workgroups (the caller cuts larger ones).
+int sgemm_piece(int ta, int tb, int M, int N, int K, float alpha, const float *A, int lda, const float *B, int ldb, float beta,
+                float *C, int ldc) {
     const GemmPlan p = plan_gemm(M, N, K, beta != 0.f, lda, ldb);
     float *part = nullptr;
     if (p.slices > 1) {
@@ -353,5 +343,37 @@ MI355_API int mi355_sgemm_dev(int trans_a, int trans_b, int M, int N, int K, flo
                            part, p.slices, M, N, alpha, beta);
         LAUNCH_OK("sgemm slice sum");
     }
+    return 0;
+}
+
+}   // namespace
+
+MI355_API int mi355_sgemm_dev(int trans_a, int trans_b, int M, int N, int K, float alpha, const float *A, int lda,
+                              const float *B, int ldb, float beta, float *C, int ldc) {
+    if (!mi355_ready("sgemm")) return -1;
+    if (!mi355_outside_capture("sgemm (its K slices may need workspace)")) return -1;
+    if (!A || !B || !C) return mi355_fail("sgemm: NULL pointer");
+    const int ta = trans_flag(trans_a), tb = trans_flag(trans_b);
+    if (ta < 0 || tb < 0) return mi355_fail("sgemm: transpose flags must be 0/1 (or CblasNoTrans/CblasTrans)");
+    if (M <= 0 || N <= 0 || K <= 0) return mi355_fail("sgemm: bad shape M=%d N=%d K=%d", M, N, K);
+    // row-major leading dimensions: A is M x K (or K x M when transposed), B is K x N (or N x K), C is M x N
+    if (lda < (ta ? M : K) || ldb < (tb ? K : N) || ldc < N)
+        return mi355_fail("sgemm: leading dimension too small (lda=%d ldb=%d ldc=%d)", lda, ldb, ldc);
+    // Pieces of what a launch can number and 32-bit arithmetic on rows and k can hold: 2^30 values of k, 2^26 rows, and as many
+    // columns as make 2^23 tiles of 64 x 64.  All but thin or long products beyond a billion rows or columns are one piece.
+    constexpr int KC = 1 << 30, MC = 1 << 26;
+    const int mc = M < MC ? M : MC;
+    const size_t tiles_n = ((size_t)1 << 23) / ceil_div((size_t)mc, 64);
+    const int nc = (size_t)N > 64 * tiles_n ? (int)(64 * tiles_n) : N;
+    for (long long m = 0; m < M; m += mc)
+        for (long long n = 0; n < N; n += nc)
+            for (long long k = 0; k < K; k += KC) {
+                const int pm = (int)(M - m < mc ? M - m : mc), pn = (int)(N - n < nc ? N - n : nc);
+                const int pk = (int)(K - k < KC ? K - k : KC);
+                if (sgemm_piece(ta, tb, pm, pn, pk, alpha, A + (ta ? m + k * lda : m * lda + k), lda,
+                                B + (tb ? n * ldb + k : n + k * ldb), ldb, k == 0 ? beta : 1.0f, C + m * ldc + n, ldc))
+                    return -1;
+                if (alpha == 0.f) break;
+            }
     return 0;
 }
