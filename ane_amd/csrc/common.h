@@ -34,8 +34,8 @@ struct Mi355Ctx {
     int rms_lpr, rms_threads, ew_unroll, ce_rows, ce_rows2, qk_lpr, qk_threads, gemm_splitk, scatter_tree, buf_phase;
     int scatter_cols;          // ordered scatter-add with the columns of dE dealt out to the workgroups: 0 = where it pays,
                                // 1 = whenever the shape allows, -1 = never
-    int gemm_split;            // sgemm on the bfloat16 instruction (gemm_split.h): 0 = where it pays, -1 = never, 1 / 2 =
-                               // always, in tiles of 128 x 256 / 256 x 128
+    int gemm_split;            // sgemm on the bfloat16 instruction (gemm_split.h): 0 = where it pays, -1 = never, 1 / 2 / 3 / 4 =
+                               // always, in tiles of 128 x 256 / 256 x 128 / 64 x 64 with one / two groups of waves
     int rms_cluster;           // channel split of the clustered RMSNorm: 0 = per shape, -1 = never, 2/4/8 = forced
     int ce_resident;           // one-launch softmax-CE: 0 = where it pays, 1 = whenever the shape allows, -1 = never
     int rms_cluster_spin;      // its bounded wait in ticks of the 100 MHz clock: 0 = 2 ms, negative = do not wait at all

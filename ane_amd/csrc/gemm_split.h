@@ -5,7 +5,8 @@
 // 2^-16 of the first are taken (hh, hm, mh, hl, lh, mm), each with an exact fp32 product and fp32 sums in
 // v_mfma_f32_16x16x32_bf16; what is left out is below 2^-24 of a term.  Six instructions of 32 terms stand for eight of
 // v_mfma_f32_16x16x4_f32, take 6 x 16 cycles instead of 8 x 32, and round a sum six times where those round it eight
-// times and more: the error against 64 bits is smaller (see the figures at plan_gemm).
+// times.  Against 64 bits the error of the large tiles is smaller from K = 80 on, that of the small ones, which keep a sum of
+// their own for the hh products, a third at any K (figures at plan_gemm).
 // A split is not exact where l leaves bfloat16 (values below 2^-109), and h + m + l of an infinity or of a value that
 // rounds to one is a NaN.  Both are seen: the first in the low half of l's pattern, the second in the result, which is
 // then not finite.  A workgroup that saw either computes its tile again with the fp32 instruction, straight from memory
@@ -34,20 +35,23 @@ __device__ __forceinline__ int split_chunk(int slot, int c) {
     const int a = slot >> 2, g = ((a >> 1) & 1) | (((a ^ (a >> 1)) & 1) << 1);
     return c ^ g ^ ((slot >> 4) & 3);
 }
-// row 4i + j of a group of 64 lies at 16j + i
-__device__ __forceinline__ int split_slot(int x) { return (x & ~63) | ((x & 3) << 4) | ((x >> 2) & 15); }
-__device__ __forceinline__ int split_row(int slot) { return (slot & ~63) | ((slot & 15) << 2) | ((slot >> 4) & 3); }
+// F fragments (16 rows each) to a wave: row F*i + j of a group of 16*F lies at 16j + i
+template <int F>
+__device__ __forceinline__ int split_slot(int x) { return (x & ~(16 * F - 1)) | (x & (F - 1)) << 4 | ((x / F) & 15); }
+template <int F>
+__device__ __forceinline__ int split_row(int slot) { return (slot & ~(16 * F - 1)) | (slot & 15) * F | ((slot >> 4) & (F - 1)); }
 
 struct Planes { v4u h, m, l; };
 
 // One operand tile of BX rows (of M or N) by SK: global -> registers -> three planes in LDS.  KC: k is the contiguous index.
-template <int BX, bool KC>
+// THREADS: of the group of waves that loads it, tid() a thread's number in the group; groups take the steps in turn.
+template <int BX, bool KC, int THREADS, int F>
 struct SplitOperand {
     static constexpr int PIECES = BX * (SK / 8);                             // eight values of k of one row
-    static constexpr int NP = PIECES / S_THREADS;                            // per thread
+    static constexpr int NP = PIECES / THREADS;                              // per thread
     static constexpr int W = NP;                                             // K strided: columns of one load
     static constexpr int PLANE = BX * SK * 2;                                // bytes
-    static_assert(PIECES % S_THREADS == 0 && (W == 1 || W == 2), "whole pieces, units of W columns");
+    static_assert(PIECES % THREADS == 0 && (W == 1 || W == 2), "whole pieces, units of W columns");
     const char *base;           // the step at hand (the same for the whole workgroup)
     size_t ahead;               // bytes from one step to the next
     size_t row;                 // K strided: bytes from one k to the next
@@ -56,33 +60,34 @@ struct SplitOperand {
     float r[NP][8];
 
     // K contiguous: four threads to a row.  K strided: sixteen threads cover 16 columns and W chunks of k.
+    static __device__ __forceinline__ int tid() { return threadIdx.x % THREADS; }
     static __device__ __forceinline__ int unit_x() {
-        const int g = threadIdx.x >> 4;
-        return g % (BX / 16) * 16 + (threadIdx.x & 15) % (16 / W) * W;
+        const int g = tid() >> 4;
+        return g % (BX / 16) * 16 + (tid() & 15) % (16 / W) * W;
     }
     static __device__ __forceinline__ int piece_slot(int p) {
-        return KC ? (threadIdx.x >> 2) + p * (S_THREADS / 4) : split_slot(unit_x() + p);
+        return KC ? (tid() >> 2) + p * (THREADS / 4) : split_slot<F>(unit_x() + p);
     }
 
     // rows past the end are read from the last one; what they multiply is never stored
-    __device__ __forceinline__ void start(const float *__restrict__ p, int ld, int x0, int X, int k0) {
+    __device__ __forceinline__ void start(const float *__restrict__ p, int ld, int x0, int X, int k0, int groups = 1) {
         if constexpr (KC) {
-            kc = threadIdx.x & 3;
+            kc = tid() & 3;
 #pragma unroll
             for (int i = 0; i < NP; i++) {
-                const int x = min(x0 + split_row(piece_slot(i)), X - 1) - x0;
+                const int x = min(x0 + split_row<F>(piece_slot(i)), X - 1) - x0;
                 off[i] = ((unsigned)x * (unsigned)ld + 8 * kc) * 4;
             }
             base = (const char *)(p + (size_t)x0 * ld + k0);
-            ahead = SK * 4;
+            ahead = (size_t)SK * 4 * groups;
             row = 4;
         } else {
-            kc = (threadIdx.x >> 4) / (BX / 16) * W + (threadIdx.x & 15) / (16 / W);
+            kc = (tid() >> 4) / (BX / 16) * W + (tid() & 15) / (16 / W);
 #pragma unroll
             for (int i = 0; i < NP; i++)
                 off[i] = ((unsigned)(8 * kc) * (unsigned)ld + (unsigned)(min(x0 + unit_x() + i, X - 1) - x0)) * 4;
             base = (const char *)(p + (size_t)k0 * ld + x0);
-            ahead = (size_t)SK * ld * 4;
+            ahead = (size_t)SK * ld * 4 * groups;
             row = (size_t)ld * 4;
         }
     }
@@ -144,6 +149,92 @@ struct SplitOperand {
     }
 };
 
+// The end of a tile: the wave's fragments at rows m0.. and columns n0.., computed again where values called for it
+// (`left`: what the splits could not hold), scaled and stored; part: where the bare product of the slice goes, or NULL;
+// mine: this wave finishes them.
+// Register e of a lane's fragment i, j: row FM * (4 * quarter + e) + i, column FN * li + j.
+template <int FM, int FN, bool TA, bool TB>
+__device__ __forceinline__ void split_finish(v4f (&acc)[FM][FN], unsigned left, const float *__restrict__ A, int lda,
+                                             const float *__restrict__ B, int ldb, float *C, int ldc, int M, int N, int m0,
+                                             int n0, int k_beg, int k_end, float alpha, float beta, float *__restrict__ part,
+                                             bool mine = true) {
+    typedef float vec __attribute__((ext_vector_type(FN), aligned(4)));
+    const int lane = threadIdx.x & 63, quarter = lane >> 4, li = lane & 15;
+    const int n = n0 + FN * li;
+    bool again = (left & 0xffffu) != 0;
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) again |= (__float_as_uint(acc[i][j][e]) & 0x7f800000u) == 0x7f800000u;
+    const bool bad = __syncthreads_or(again);
+    if (!mine) return;
+    if (bad) {
+        const float *pa[FM], *pb[FN];
+#pragma unroll
+        for (int i = 0; i < FM; i++) {
+#pragma unroll
+            for (int j = 0; j < FN; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+            const int m = min(m0 + FM * li + i, M - 1);
+            pa[i] = TA ? A + m : A + (size_t)m * lda;
+        }
+#pragma unroll
+        for (int j = 0; j < FN; j++) {
+            const int nn = min(n + j, N - 1);
+            pb[j] = TB ? B + (size_t)nn * ldb : B + nn;
+        }
+        for (int k0 = k_beg; k0 < k_end; k0 += 4) {
+            const int k = k0 + quarter;
+            float va[FM], vb[FN];
+#pragma unroll
+            for (int i = 0; i < FM; i++) va[i] = k < k_end ? pa[i][TA ? (size_t)k * lda : (size_t)k] : 0.f;
+#pragma unroll
+            for (int j = 0; j < FN; j++) vb[j] = k < k_end ? pb[j][TB ? (size_t)k : (size_t)k * ldb] : 0.f;
+#pragma unroll
+            for (int i = 0; i < FM; i++)
+#pragma unroll
+                for (int j = 0; j < FN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[i], vb[j], acc[i][j], 0, 0, 0);
+        }
+    }
+
+    float *out = part ? part : C;
+    const int ldo = part ? N : ldc;
+    const bool read = !part && beta != 0.f;             // beta == 0 does not read C (cblas semantics)
+    vec c[FM][4];                                       // all of the old values are asked for before the first store
+    auto each = [&](auto fn) {
+#pragma unroll
+        for (int i = 0; i < FM; i++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int m = m0 + FM * (4 * quarter + e) + i;
+                if (m < M) fn(i, e, out + (size_t)m * ldo + n);
+            }
+    };
+    if (read)
+        each([&](int i, int e, const float *o) {
+            if (n + FN <= N) {
+                c[i][e] = *reinterpret_cast<const vec *>(o);
+            } else {
+#pragma unroll
+                for (int j = 0; j < FN; j++) c[i][e][j] = n + j < N ? o[j] : 0.f;
+            }
+        });
+    each([&](int i, int e, float *o) {
+        vec v;
+#pragma unroll
+        for (int j = 0; j < FN; j++) v[j] = part ? acc[i][j][e] : acc[i][j][e] * alpha;
+        if (read) v += beta * c[i][e];
+        if (n + FN <= N) {
+            *reinterpret_cast<vec *>(o) = v;
+        } else {
+#pragma unroll
+            for (int j = 0; j < FN; j++)
+                if (n + j < N) o[j] = v[j];
+        }
+    });
+}
+
 // C = alpha * op(A) . op(B) + beta * C for one K slice; part != NULL: the bare product of the slice goes to part[slice].
 // Workgroup order as sgemm_kernel's.  lda, ldb < 2^22: the lanes' offsets into a tile are 32 bits of bytes.
 template <int BM, int BN, bool TA, bool TB>
@@ -151,9 +242,9 @@ __global__ __launch_bounds__(S_THREADS) void sgemm_split_kernel(const float *__r
                                                                 const float *__restrict__ B, int ldb, float *C, int ldc,
                                                                 int M, int N, int K, int k_slice, int tiles_n, int tiles,
                                                                 float alpha, float beta, float *__restrict__ part) {
-    typedef SplitOperand<BM, !TA> OpA;
-    typedef SplitOperand<BN, TB> OpB;
     constexpr int WM = 64, WN = 64, FM = WM / 16, FN = WN / 16;
+    typedef SplitOperand<BM, !TA, S_THREADS, FM> OpA;
+    typedef SplitOperand<BN, TB, S_THREADS, FN> OpB;
     static_assert((BM / WM) * (BN / WN) == S_THREADS / 64, "eight waves cover the tile");
     __shared__ __align__(16) char lds[2][3 * (OpA::PLANE + OpB::PLANE)];
     const int logical = xcd_remap(blockIdx.x, gridDim.x);
@@ -272,62 +363,135 @@ __global__ __launch_bounds__(S_THREADS) void sgemm_split_kernel(const float *__r
         }
     }
 
-    // register e of a lane's block i, j: row(i, e), column 4 * li + j of the wave's 64
-    auto row = [&](int i, int e) { return m0 + wm + 16 * quarter + 4 * e + i; };
-    const int n = n0 + wn + 4 * li;
-    bool again = (left & 0xffffu) != 0;
+    split_finish<FM, FN, TA, TB>(acc, left, A, lda, B, ldb, C, ldc, M, N, m0 + wm, n0 + wn, k_beg, k_end, alpha, beta,
+                                 part ? part + (size_t)slice * M * N : nullptr);
+}
+
+// The same for outputs with few tiles of 128 x 256: KS groups of four waves own a tile of 64 x 64 (a wave 32 x 32) and take the
+// steps in turn.  One group: three workgroups share a compute unit (49 KB each) and one splits, loads or stores while another
+// multiplies; [3072][256] . [256][1024] += 18.0 us (fp32 64 x 64 20.1, 128 x 256 27), [9001][768] . [768][197] 35 (49, 43).
+// Two groups: where there is one tile to a compute unit, whose four waves would wait for each other (1024 x 1024 x 1024
+// 27.8 with one group, 21.6 with two).  What bounds it is the splitting, done again by every tile: at 64 x 64 as many vector
+// cycles as half of the matrix cycles, and the LDS reads, as many cycles as the products.  A second step on its way to
+// registers changed nothing (12.7 and 12.7 at [2048][256] . [256][768]), nor did tiles of 64 x 128 (13.4).
+// The hh products of a term have sums of their own, so a sum of full size is rounded once per 32 values of k, and the five
+// small products, below 2^-8 of it, beside it.
+constexpr int SS_THREADS = 256;        // of a group
+template <int BM, int BN, int WM, int WN, int KS, bool TA, bool TB>
+__global__ __launch_bounds__(SS_THREADS * KS) void sgemm_split_small_kernel(const float *__restrict__ A, int lda,
+                                                                            const float *__restrict__ B, int ldb, float *C,
+                                                                            int ldc, int M, int N, int K, int k_slice,
+                                                                            int tiles_n, int tiles, float alpha, float beta,
+                                                                            float *__restrict__ part) {
+    constexpr int FM = WM / 16, FN = WN / 16;
+    typedef SplitOperand<BM, !TA, SS_THREADS, FM> OpA;
+    typedef SplitOperand<BN, TB, SS_THREADS, FN> OpB;
+    static_assert((BM / WM) * (BN / WN) == SS_THREADS / 64, "four waves cover the tile");
+    __shared__ __align__(16) char lds[KS][2][3 * (OpA::PLANE + OpB::PLANE)];
+    const int logical = xcd_remap(blockIdx.x, gridDim.x);
+    const int slice = logical / tiles, tile = logical - slice * tiles;
+    const int m0 = tile / tiles_n * BM, n0 = tile % tiles_n * BN;
+    const int k_beg = slice * k_slice, k_end = min(K, k_beg + k_slice);
+    const int steps = (k_end - k_beg) / SK, rest = (k_end - k_beg) % SK, all = steps + (rest > 0);
+    const bool edge_m = m0 + BM > M, edge_n = n0 + BN > N;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, quarter = lane >> 4, li = lane & 15;
+    const int group = wave / 4, ww = wave % 4;
+    const int wm = ww / (BN / WN) * WM, wn = ww % (BN / WN) * WN;
+
+    v4f acc[FM][FN], low[FM][FN];
 #pragma unroll
     for (int i = 0; i < FM; i++)
 #pragma unroll
-        for (int j = 0; j < FN; j++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) again |= (__float_as_uint(acc[i][j][e]) & 0x7f800000u) == 0x7f800000u;
-    if (__syncthreads_or(again)) {
-        clear();
-        const float *pa[FM], *pb[FN];
-#pragma unroll
-        for (int i = 0; i < FM; i++) {
-            const int m = min(m0 + wm + 4 * li + i, M - 1);
-            pa[i] = TA ? A + m : A + (size_t)m * lda;
+        for (int j = 0; j < FN; j++) acc[i][j] = low[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+    unsigned left = 0;
+    OpA oa;
+    OpB ob;
+    oa.start(A, lda, m0, M, k_beg + SK * group, KS);
+    ob.start(B, ldb, n0, N, k_beg + SK * group, KS);
+    // step t of the group is step KS * t + group of the tile; where that is past the end it is all zeros
+    const int rounds = (all + KS - 1) / KS;
+    auto fetch = [&](int t) {
+        const int s = KS * t + group;
+        if (s < steps) { oa.fetch(edge_m); ob.fetch(edge_n); }
+        else { oa.fetch_tail(s == steps ? rest : 0); ob.fetch_tail(s == steps ? rest : 0); }
+    };
+    constexpr int NPA = OpA::NP, NPB = OpB::NP;
+    auto piece = [&](int p, char *to) {
+        Planes o;
+        if (p < NPA) {
+            oa.split(p < NPA ? p : 0, 0, 4, o, left);
+            oa.write(p < NPA ? p : 0, o, to);
+        } else {
+            ob.split(p < NPA ? 0 : p - NPA, 0, 4, o, left);
+            ob.write(p < NPA ? 0 : p - NPA, o, to + 3 * OpA::PLANE);
         }
+    };
+    fetch(0);
 #pragma unroll
-        for (int j = 0; j < FN; j++) {
-            const int nn = min(n + j, N - 1);
-            pb[j] = TB ? B + (size_t)nn * ldb : B + nn;
+    for (int p = 0; p < NPA + NPB; p++) piece(p, lds[group][0]);
+    if (rounds > 1) fetch(1);
+    __syncthreads();
+    int fa[FM], fb[FN];                                  // where this lane's fragments lie in a plane
+#pragma unroll
+    for (int i = 0; i < FM; i++) {
+        const int slot = wm + 16 * i + li;
+        fa[i] = slot * (SK * 2) + split_chunk(slot, quarter) * 16;
+    }
+#pragma unroll
+    for (int j = 0; j < FN; j++) {
+        const int slot = wn + 16 * j + li;
+        fb[j] = slot * (SK * 2) + split_chunk(slot, quarter) * 16 + 3 * OpA::PLANE;
+    }
+    for (int t = 0; t < rounds; t++) {
+        const char *cur = lds[group][t & 1];
+        bf8_t a[FM][3], b[FN][3];
+#pragma unroll
+        for (int q = 0; q < 3; q++) {
+#pragma unroll
+            for (int i = 0; i < FM; i++) a[i][q] = *reinterpret_cast<const bf8_t *>(cur + fa[i] + q * OpA::PLANE);
+#pragma unroll
+            for (int j = 0; j < FN; j++) b[j][q] = *reinterpret_cast<const bf8_t *>(cur + fb[j] + q * OpB::PLANE);
         }
-        for (int k0 = k_beg; k0 < k_end; k0 += 4) {
-            const int k = k0 + quarter;
-            float va[FM], vb[FN];
+        const bool more = t + 1 < rounds;
+        constexpr int P[6][2] = {{0, 0}, {0, 1}, {1, 0}, {1, 1}, {0, 2}, {2, 0}};
 #pragma unroll
-            for (int i = 0; i < FM; i++) va[i] = k < k_end ? pa[i][TA ? (size_t)k * lda : (size_t)k] : 0.f;
-#pragma unroll
-            for (int j = 0; j < FN; j++) vb[j] = k < k_end ? pb[j][TB ? (size_t)k : (size_t)k * ldb] : 0.f;
+        for (int p = 0; p < 6; p++) {
 #pragma unroll
             for (int i = 0; i < FM; i++)
 #pragma unroll
-                for (int j = 0; j < FN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[i], vb[j], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < FN; j++) {
+                    v4f &s = p == 0 ? acc[i][j] : low[i][j];
+                    s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i][P[p][0]], b[j][P[p][1]], s, 0, 0, 0);
+                }
+            if (more && p < NPA + NPB) piece(p, lds[group][(t + 1) & 1]);
+        }
+        if (more) {
+            if (t + 2 < rounds) fetch(t + 2);
+            __syncthreads();
         }
     }
-
-    float *out = part ? part + (size_t)slice * M * N : C;
-    const int ldo = part ? N : ldc;
-    const bool read = !part && beta != 0.f;             // beta == 0 does not read C (cblas semantics)
 #pragma unroll
     for (int i = 0; i < FM; i++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int m = row(i, e);
-            if (m >= M) continue;
-            float *o = out + (size_t)m * ldo + n;
-            v4f v = {acc[i][0][e], acc[i][1][e], acc[i][2][e], acc[i][3][e]};
-            if (!part) v *= alpha;
-            if (n + 4 <= N) {
-                if (read) v += beta * ld4(o);
-                st4(o, v);
-            } else {
+        for (int j = 0; j < FN; j++) acc[i][j] += low[i][j];
+    if constexpr (KS > 1) {
+        // the other groups' sums, added in group order by the first; they leave with it at the next barrier
+        static_assert((KS - 1) * BM * BN * 4 <= (int)sizeof(lds), "the sums fit the buffers");
+        v4f *x = reinterpret_cast<v4f *>(&lds[0][0][0]);
+        auto at = [&](int g, int f) { return ((g - 1) * FM * FN + f) * SS_THREADS + ww * 64 + lane; };
+        __syncthreads();
+        if (group > 0) {
 #pragma unroll
-                for (int j = 0; j < 4; j++)
-                    if (n + j < N) o[j] = read ? v[j] + beta * o[j] : v[j];
-            }
+            for (int f = 0; f < FM * FN; f++) x[at(group, f)] = acc[f / FN][f % FN];
         }
+        __syncthreads();
+        if (group == 0) {
+#pragma unroll
+            for (int g = 1; g < KS; g++)
+#pragma unroll
+                for (int f = 0; f < FM * FN; f++) acc[f / FN][f % FN] += x[at(g, f)];
+        }
+    }
+    split_finish<FM, FN, TA, TB>(acc, left, A, lda, B, ldb, C, ldc, M, N, m0 + wm, n0 + wn, k_beg, k_end, alpha, beta,
+                                 part ? part + (size_t)slice * M * N : nullptr, group == 0);
 }

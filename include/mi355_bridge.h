@@ -56,8 +56,9 @@ size_t mi355_workspace_size(void);
  * "rms_lpr" (lanes per strip row, 4/8/16) and "rms_threads" (256/512/1024) of the RMSNorm tiles, "qk_lpr" and
  * "qk_threads" (256/512) of the QK-norm + RoPE tiles, "ew_unroll" (accesses per lane of the streaming ops, 1/2/4),
  * "ce_rows" / "ce_rows2" (rows of logits per workgroup in the first / second pass of softmax-CE),
- * "gemm_splitk" (K slices of mi355_sgemm_dev; 1 = never split), "gemm_split" (its kernel that multiplies fp32 values as
- * sums of three bfloat16 values: 0 = where it pays, -1 = never, 1 / 2 = always, in tiles of 128 x 256 / 256 x 128),
+ * "gemm_splitk" (K slices of mi355_sgemm_dev; 1 = never split), "gemm_split" (its kernels that multiply fp32 values as
+ * sums of three bfloat16 values: 0 = where they pay, -1 = never, 1 / 2 = always, in tiles of 128 x 256 / 256 x 128,
+ * 3 / 4 = always, in tiles of 64 x 64 with one / two groups of waves),
  * "scatter_tree" (1: mi355_embed_scatter_add_dev sums long segments by a fixed tree instead of the reference's
  * sequential order: still deterministic and within 1e-5 of each row's scale, faster, no longer bit-identical to
  * the CPU loop), "scatter_cols" (the form of mi355_embed_scatter_add_dev in which every workgroup owns a few columns
@@ -408,7 +409,10 @@ int mi355_attn_grads_finish_dev(float *dq, float *dk, float *dv, const void *dq_
  * the classifier products training/training_dynamic/train.m:490-491 (logits), :501-502 (dy), :507-508 (gcembed +=)
  * and the weight-gradient products :577-581, :613, :681-685.  Same argument order and meaning as the cblas call
  * without the layout argument (always row-major); trans flags take 0/1 or CblasNoTrans/CblasTrans (111/112).
- * fp32 products and sums on the matrix cores, deterministic (K slices are added in order). */
+ * fp32 operands, sums and results on the matrix cores, deterministic (K slices are added in a fixed order).  Where it pays a product
+ * is formed from operands split exactly into three bfloat16 values each, six of their nine products: what is left out
+ * is below 2^-24 of a term, and the result as close to the exact one as with fp32 products.  Infinities, NaNs and values too
+ * small to split give what fp32 products give. */
 int mi355_sgemm_dev(int trans_a, int trans_b, int M, int N, int K, float alpha, const float *A, int lda,
                     const float *B, int ldb, float beta, float *C, int ldc);
 

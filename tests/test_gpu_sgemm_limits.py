@@ -29,7 +29,7 @@ class Sparse:
         self.br.lib.mi355_buf_free(self.handle)
 
 
-@pytest.mark.parametrize("knob", [-1, 1])
+@pytest.mark.parametrize("knob", [-1, 1, 4])
 @pytest.mark.parametrize("K", [BIG, 2 ** 30 + 5])
 def test_k(br, K, knob):
     print("[case] sgemm K=%d knob=%d" % (K, knob), flush=True)
@@ -49,7 +49,7 @@ def test_k(br, K, knob):
         for t in (a, b, c): t.free()
 
 
-@pytest.mark.parametrize("knob", [-1, 1])
+@pytest.mark.parametrize("knob", [-1, 1, 4])
 @pytest.mark.parametrize("rows", [True, False])
 def test_rows_and_columns(br, rows, knob):
     print("[case] sgemm %s=%d knob=%d" % ("M" if rows else "N", BIG, knob), flush=True)

@@ -23,7 +23,7 @@ def product(br, knob, A, B, ta, tb, alpha=1.0, beta=0.0, C0=None, off=0):
         br.tune("gemm_split", 0)
 
 
-@pytest.mark.parametrize("knob", [1, 2])
+@pytest.mark.parametrize("knob", [1, 2, 3, 4])
 @pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (0, 1), (1, 1)])
 @pytest.mark.parametrize("M,N,K", [(1, 1, 1), (127, 257, 31), (129, 255, 33), (256, 256, 64), (300, 130, 97), (70, 3, 700)])
 def test_split_tile_edges(br, M, N, K, ta, tb, knob):
@@ -50,7 +50,7 @@ def test_split_gives_infinities_and_nans_of_fp32(br, ta, tb):
     B[64, 260] = np.inf; B[1, 17] = 0.0; B[5, 4] = 0.0
     As, Bs = np.ascontiguousarray(A.T if ta else A), np.ascontiguousarray(B.T if tb else B)
     want = product(br, -1, As, Bs, ta, tb)
-    for knob in (1, 2):
+    for knob in (1, 2, 3, 4):
         got = product(br, knob, As, Bs, ta, tb)
         assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
         assert np.array_equal(np.sign(got[np.isinf(got)]), np.sign(want[np.isinf(want)]))
@@ -70,14 +70,14 @@ def test_split_keeps_values_near_the_smallest(br, scale):
     A[100:, 0] = np.float32(2.0 ** -115 * (1 + 2.0 ** -9 + 2.0 ** -17))
     B = H.normal(621, (K, N))
     ref = A.astype(np.float64) @ B.astype(np.float64); mag = np.abs(A.astype(np.float64)) @ np.abs(B.astype(np.float64))
-    for knob in (1, 2):
+    for knob in (1, 2, 3, 4):
         got = product(br, knob, A, B, 0, 0).astype(np.float64)
         assert np.all(np.abs(got - ref) <= (K + 1) * 2.0 ** -23 * mag + K * 2.0 ** -149)
 
 
 def test_alpha_zero_reads_no_operand(br):
     A = np.full((40, 300), np.nan, np.float32); B = np.full((300, 50), np.inf, np.float32); C0 = H.normal(630, (40, 50))
-    for knob in (-1, 1):
+    for knob in (-1, 1, 3, 4):
         assert np.array_equal(product(br, knob, A, B, 0, 0, alpha=0.0, beta=2.0, C0=C0), 2.0 * C0)
         assert not np.any(product(br, knob, A, B, 0, 0, alpha=0.0))
 
