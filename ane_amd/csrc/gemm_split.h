@@ -21,7 +21,7 @@
 // A step takes 2.45 us where its instructions take 1.28 at 2.4 GHz; the chip runs this kernel at 1.8 GHz, so the matrix
 // cores are busy 70 % of the time.  The splitting (6 vector instructions per value) is a third of the matrix time and runs
 // in the shadow of the other wave of the SIMD; with the whole splitting at the end of a step and the barrier behind it,
-// 4096 x 4096 x 4096 took 667 us, in this order 640 (215 TFLOP/s; the fp32 instruction 1118 us).
+// 4096 x 4096 x 4096 took 667 us, in this order 640 (215 TFLOP/s; the fp32 instruction 1145 us).
 #pragma once
 
 typedef __bf16 bf8_t __attribute__((ext_vector_type(8)));

@@ -303,9 +303,9 @@ int mi355_embed_scatter_add_form(int V, int D, int S, int batch, int aligned);
  * (stories_cpu_ops.h:98).  dlogits may alias logits.
  * A column that holds a NaN or +inf, or -inf alone, is NaN throughout, and so is the loss that counts it.
  * Logits of 4 to 1024 columns and at most 4096 * min(64, compute units / ceil(S / 64)) rows (262144 up to 256 columns,
- * 65536 at 1000, on 256 compute units) that are not overwritten in place run as ONE launch that keeps the logits in registers and LDS between the two passes (one workgroup per compute unit; partial
- * sums exchanged inside the launch through a device array of the library, bounded wait as for the RMSNorm); every
- * other call runs as three launches that read the logits twice, and so do fp32 logits of at most 64 columns and more than
+ * 65536 at 1000, on 256 compute units) that are not overwritten in place run as ONE launch that keeps the logits in
+ * registers and LDS between the two passes (one workgroup per compute unit; partial sums exchanged inside the launch
+ * through a device array of the library, bounded wait as for the RMSNorm); every other call runs as three launches that read the logits twice, and so do fp32 logits of at most 64 columns and more than
  * 57344 rows, which would keep only 64 of the compute units busy.  Both forms are deterministic; they sum in
  * different orders, so their results differ in the last bits.  Tuning knob "ce_resident": 0 = as described, 1 = one launch
  * for the latter too, -1 = never the one-launch form. */
@@ -316,8 +316,8 @@ int mi355_softmax_ce_dev(float *dlogits, float *loss_dev, const float *logits,
  * harnesses that forbid hipMalloc).  No counterpart in the reference.  Same arguments, same kernels and the same
  * bits out, but the scratch lives in a fixed 3 MiB device array of the library, located once by mi355_init (call
  * it first): the call performs no hipMalloc, no hipFree and no workspace growth.  The array holds the exchange
- * slots of the one-launch form (which mi355_softmax_ce_dev uses from there as well) and 2 MiB for the three-launch
- * form's first-pass partials and per-column max / sum / loss.
+ * slots of the one-launch form and 2 MiB for the three-launch form's first-pass partials and per-column max / sum / loss;
+ * mi355_softmax_ce_dev uses both as well, and its workspace only for what does not fit.
  * Limit, for calls that take the three-launch form: 2 * ceil(V / rows per workgroup) * S * 4 + 3 * S * 4 bytes
  * (rounded up to 256 each) must fit 2 MiB, otherwise the call fails with a message and launches nothing.  Every
  * call on a GPU shares that GPU's array: calls that overlap on one GPU (two streams, two threads) race. */
