@@ -51,7 +51,7 @@ def short(name):
 
 
 def skipped(name):
-    return name.startswith("__amd") or name.startswith("fill_")
+    return name.startswith("__amd") or name.startswith("fill_") or name.startswith("at::native")
 
 
 def find_csv(directory, suffix):
@@ -74,8 +74,7 @@ def write_stats(directory, out_md, cmd, title, note):
         lines.append("| `%s` | %s | %.1f | %.1f | %.1f | %.2f |" % (n, r["Calls"], float(r["AverageNs"]) / 1e3,
                                                                   float(r["MinNs"]) / 1e3, float(r["MaxNs"]) / 1e3,
                                                                   float(r["Percentage"])))
-    lines += ["", "`__amd_rocclr_fillBufferAligned` and `fill_*` kernels (buffer zeroing and synthetic-input generation "
-                  "before the timed region) are omitted."]
+    lines += ["", "Buffer zeroing and the making of the inputs (`__amd_*`, `fill_*`, torch's kernels) are omitted."]
     open(os.path.join(PROFILES, out_md), "w").write("\n".join(lines) + "\n")
 
 

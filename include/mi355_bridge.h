@@ -305,10 +305,10 @@ int mi355_embed_scatter_add_form(int V, int D, int S, int batch, int aligned);
  * Logits of 4 to 1024 columns and at most 4096 * min(64, compute units / ceil(S / 64)) rows (262144 up to 256 columns,
  * 65536 at 1000, on 256 compute units) that are not overwritten in place run as ONE launch that keeps the logits in
  * registers and LDS between the two passes (one workgroup per compute unit; partial sums exchanged inside the launch
- * through a device array of the library, bounded wait as for the RMSNorm); every other call runs as three launches that read the logits twice, and so do fp32 logits of at most 64 columns and more than
- * 57344 rows, which would keep only 64 of the compute units busy.  Both forms are deterministic; they sum in
- * different orders, so their results differ in the last bits.  Tuning knob "ce_resident": 0 = as described, 1 = one launch
- * for the latter too, -1 = never the one-launch form. */
+ * through a device array of the library, bounded wait as for the RMSNorm); every other call runs as three launches that
+ * read the logits twice, and so do fp32 logits of at most 64 columns and more than 57344 rows, which would keep only 64 of
+ * the compute units busy.  Both forms are deterministic; they sum in different orders, so their results differ in the last
+ * bits.  Tuning knob "ce_resident": 0 = as described, 1 = one launch for the latter too, -1 = never the one-launch form. */
 int mi355_softmax_ce_dev(float *dlogits, float *loss_dev, const float *logits,
                          const int32_t *targets, int V, int S, float grad_scale);
 
