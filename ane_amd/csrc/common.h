@@ -35,7 +35,8 @@ struct Mi355Ctx {
     int scatter_cols;          // ordered scatter-add with the columns of dE dealt out to the workgroups: 0 = where it pays,
                                // 1 = whenever the shape allows, -1 = never
     int gemm_split;            // sgemm on the bfloat16 instruction (gemm_split.h): 0 = where it pays, -1 = never, 1 / 2 / 3 / 4 =
-                               // always, in tiles of 128 x 256 / 256 x 128 / 64 x 64 with one / two groups of waves
+                               // always, in tiles of 128 x 256 / 256 x 128 / 64 x 64 with one / two groups of waves, 5 / 6 / 7 / 8 =
+                               // with B split ahead (gemm_planes.h): tiles of 96 / 64 x 256, whole rows of A, 96 / 64 of them
     int rms_cluster;           // channel split of the clustered RMSNorm: 0 = per shape, -1 = never, 2/4/8 = forced
     int ce_resident;           // one-launch softmax-CE: 0 = where it pays, 1 = whenever the shape allows, -1 = never
     int rms_cluster_spin;      // its bounded wait in ticks of the 100 MHz clock: 0 = 2 ms, negative = do not wait at all

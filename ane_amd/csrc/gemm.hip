@@ -5,7 +5,8 @@
 // gcembed += dlogits . x_final^T (:507-508), and the dW products of each layer (:577-581, :613, :681-685).
 //
 // Large products and many of middle size go through the bfloat16 matrix instruction, each fp32 value as a sum of three
-// (gemm_split.h); the kernel in this file takes the others (plan_gemm).
+// (gemm_split.h; gemm_planes.h where one operand is small enough to be split ahead); the kernel in this file takes the others
+// (plan_gemm).
 //
 // fp32 products on the fp32 matrix instruction (v_mfma_f32_16x16x4_f32: fp32 products and sums, 157 TFLOP/s on the
 // chip).  An instruction takes 32 cycles of its SIMD for two registers of operands, so neither LDS nor memory is close to
@@ -34,6 +35,8 @@
 
 #include <algorithm>
 #include <type_traits>
+
+void mi355_free_planes(void);
 
 namespace {
 
@@ -260,6 +263,7 @@ __global__ __launch_bounds__(64 * KS * (BM / WM) * (BN / WN), KS > 1 ? 6 : 1) vo
 }
 
 #include "gemm_split.h"
+#include "gemm_planes.h"
 
 // C = alpha * sum_s part[s] + beta * C.  GROUPS threads to an element: thread g adds the slices g, g + GROUPS, ... in order,
 // then the groups' sums are added in order.  One thread to an element waits for slices / 4 trips to memory one after the
@@ -295,9 +299,10 @@ int trans_flag(int t) {
     return -1;
 }
 
-// split: the bfloat16 instruction (gemm_split.h); groups of waves
+// split: the bfloat16 instruction, 1 with both operands split by every tile (gemm_split.h), 2 and 3 with B split ahead
+// (gemm_planes.h: sgemm_planes_kernel, sgemm_rows_kernel); groups of waves; ranges of columns (3)
 struct GemmPlan {
-    int split, groups, bm, bn, slices, k_slice;
+    int split, groups, bm, bn, slices, k_slice, ranges;
 };
 constexpr int gemm_key(int split, int groups, int bm, int bn) { return ((split * 10 + groups) * 1000 + bm) * 1000 + bn; }
 
@@ -312,45 +317,58 @@ constexpr GemmKernel GEMM_KERNELS[] = {
     {0, 4, 64, 32, 64, 3, 0.67, 0.66, 0.27}, {0, 4, 32, 64, 64, 3, 0.67, 0.66, 0.27},
     {1, 1, 128, 256, 32, 1, 2.3, 2.6, 4.2},  {1, 1, 256, 128, 32, 1, 2.3, 2.6, 4.2},
     {1, 1, 64, 64, 32, 3, 0.93, 0.43, 2.1},  {1, 2, 64, 64, 64, 1, 0.91, 0.91, 2.7},
+    {2, 1, 96, 256, 64, 1, 3.7, 3.7, 4.4},   {2, 1, 64, 256, 64, 1, 2.6, 2.6, 4.4},
 };
 // The kernel and number of K slices with the least estimated time: a launch, the longer of the work of the busiest compute
 // unit and the bytes from memory at 5.6 TB/s or from the L2s at 21, and a quarter of the shorter one, which do not overlap
 // better than that.  fp32 operands whose k is strided take a sixth longer (their fragments are read a float at a time).
-// Slices cost a launch and the way of their partial products through memory.  The numbers are fitted to 210 products of
-// every transpose case (vocabularies of 2000 to 24573 rows by 32 to 512 columns, the weight gradients of a layer, squares,
-// thin and long ones) in every kernel and number of slices: what is chosen takes 0.5 % more than the best on the average and
-// 14 % at worst; tiles of 128 x 64 and 64 x 128 were never the best and are gone.
+// Slices cost a launch and the way of their partial products through memory, an operand split ahead a launch and its way at
+// the rate of the last-level cache.  The numbers are fitted to 210 products of every transpose case (vocabularies of 2000 to
+// 24573 rows by 32 to 512 columns, the weight gradients of a layer, squares, thin and long ones) in every kernel and number of
+// slices, those of gemm_planes.h to 153 of them: what is chosen takes 0.7 % more than the best on the average and 14 % at worst;
+// tiles of 128 x 64 and 64 x 128 were never the best and are gone.
 // Measured, us; the chosen kernel first (in brackets the library that stood here before):
-//   [32000][768] . [768][256]          split 128 x 256 71, 64 x 64 92, fp32 64 x 64 113                        (105)
-//   [768][32000] . [32000][256]        split 128 x 256 in 32 slices 92, fp32 64 x 64 119                       (328)
-//   [32000][256] . [256][768] +=       split 128 x 256 88, 64 x 64 107, fp32 64 x 64 119                       (112)
-//   [9001][768] . [768][197]           split 64 x 64 35, 256 x 128 39, fp32 64 x 32 41                         (42)
-//   [2048][256] . [256][768] +=        fp32 32 x 64 11.8, 64 x 64 13.1, split 64 x 64 13.6, 128 x 256 24       (10.9)
-//   [3072][256] . [256][1024] +=       split 64 x 64 18.0, fp32 64 x 64 20.1, split 128 x 256 27               (16.3)
-//   [24573][64] . [64][1024] +=        fp32 64 x 64 50, split 128 x 256 52, 64 x 64 54                         (42)
+//   [24573][1024] . [1024][256]        planes 96 x 256 71, split 256 x 128 90, 64 x 64 100, fp32 124
+//   [24573][256] . [256][1024] +=      rows of 96 68, split 128 x 256 94, 64 x 64 107, fp32 123
+//   [32000][256] . [256][768] +=       rows of 64 73, of 96 82, split 128 x 256 90, fp32 121                   (112)
+//   [32000][768] . [768][256]          split 128 x 256 68, planes 64 x 256 78, 96 x 256 92, fp32 115           (105)
+//   [768][32000] . [32000][256]        split 128 x 256 in 32 slices 80, planes 96 x 256 84, fp32 120           (328)
+//   [9001][768] . [768][197]           split 64 x 64 35, planes 64 x 256 37, fp32 64 x 32 41                   (42)
+//   [14000][768] . [768][256]          planes 64 x 256 39, split 256 x 128 48, 64 x 64 52, fp32 61
+//   [14000][256] . [256][768] +=       rows of 64 37, of 96 43, split 64 x 64 51, fp32 58
+//   [24573][64] . [64][1024] +=        rows of 96 41, fp32 64 x 64 55, split 128 x 256 56, 64 x 64 59          (42)
+//   [2048][256] . [256][768] +=        fp32 32 x 64 11.8, 64 x 64 13.1, split 64 x 64 13.6, rows of 64 20      (10.9)
+//   [3072][256] . [256][1024] +=       split 64 x 64 18.0, fp32 64 x 64 20.1, rows of 64 24, split 128 x 256 27 (16.3)
+//   [4096][1024] . [1024][3072]        planes 64 x 256 140, split 128 x 256 168, 64 x 64 181, fp32 228
 //   [1024][1024] . [1024][1024]        split 64 x 64 in two groups 21.6, fp32 64 x 32 23.5, 64 x 64 23.7       (19.9)
 //   [2048][768] . [768][256]           fp32 64 x 32 10.9, split 64 x 64 in two groups 15.4, fp32 64 x 64 17    (13.8)
 //   [24573][1024] . [1024][1]          fp32 64 x 32 24.5, split 64 x 64 32, fp32 64 x 64 38                    (72)
 //   [32][100000] . [100000][32]        fp32 32 x 64 in 256 slices 12.7                                         (28)
 //   [1][1000000] . [1000000][1]        fp32 32 x 64 in 256 slices 45, all of it for one element of a tile      (32)
 // Relative error against 64 bits (2-norms, normal operands):
-//   K       fp32, one group     two / four groups         split 64 x 64    split 128 x 256    (library)
-//   32           1.03e-7            0.8e-7 / 0.8e-7          0.39e-7           1.17e-7          1.03e-7
-//   64           1.44e-7            1.1e-7 / 0.8e-7          0.50e-7           1.46e-7          1.44e-7
-//   80           1.61e-7            1.2e-7 / 1.0e-7          0.54e-7           1.56e-7          1.61e-7
-//   256          2.87e-7            2.1e-7 / 1.5e-7          0.89e-7           2.57e-7          2.87e-7 (2.06e-7 in slices)
-//   1024         5.72e-7            4.1e-7 / 2.9e-7          1.86e-7           5.0e-7           5.72e-7
+//   K       fp32, one group     two / four groups      split 64 x 64  split 128 x 256  planes   rows     (library)
+//   32           1.03e-7            0.8e-7 / 0.8e-7       0.39e-7        1.17e-7       0.4e-7   0.4e-7   1.03e-7
+//   64           1.44e-7            1.1e-7 / 0.8e-7       0.50e-7        1.46e-7       0.53e-7  0.53e-7  1.44e-7
+//   80           1.61e-7            1.2e-7 / 1.0e-7       0.54e-7        1.56e-7       0.55e-7  0.57e-7  1.61e-7
+//   256          2.87e-7            2.1e-7 / 1.5e-7       0.93e-7        2.57e-7       0.69e-7  0.74e-7  2.87e-7 (2.06e-7 in slices)
+//   1024         5.72e-7            4.1e-7 / 2.9e-7       1.86e-7        5.0e-7        0.97e-7     -     5.72e-7
 // so the large split tiles, whose hh products and small ones share a sum, are not taken below K = 80.
-GemmPlan plan_gemm(int ta, int tb, int M, int N, int K, bool reads_c, int lda, int ldb) {
+// ahead: B may be split ahead (there is memory for its planes).
+GemmPlan plan_gemm(int ta, int tb, int M, int N, int K, bool reads_c, int lda, int ldb, int ldc, bool ahead) {
     const int cus = g_ctx.num_cu > 0 ? g_ctx.num_cu : 256;
-    GemmPlan best = {0, 1, 64, 64, 1, K};
+    GemmPlan best = {0, 1, 64, 64, 1, K, 1};
     double best_us = -1.0;
     const bool can = lda < (1 << 22) && ldb < (1 << 22);        // (32-bit offsets of the lanes)
     const int knob = can ? g_ctx.gemm_split : -1;
     const auto up = [](double x) { return (double)(long)(x + 0.999999); };
+    const double planes = (double)plane_bytes(N, K);
+    const bool planes_ok = can && ahead && planes <= (double)P_MAX_BYTES;
+    const double split_us = 1.9 + (4.0 * N * K + planes) / 15.4e6;         // the launch that splits B
+    const double c_times = reads_c ? 2 : 1;
     for (const GemmKernel &t : GEMM_KERNELS) {
-        const int id = !t.split ? -1 : t.bm == 64 ? 2 + t.groups : t.bm / 128;         // as the knob numbers them
-        if (knob ? (knob < 0 ? t.split != 0 : id != knob) : t.bm * t.bn > 64 * 64 && K < 80) continue;
+        const int id = !t.split ? -1 : t.split == 2 ? (t.bm == 96 ? 5 : 6) : t.bm == 64 ? 2 + t.groups : t.bm / 128;         // as the knob numbers them
+        if (t.split == 2 && !planes_ok) continue;
+        if (knob ? (knob < 0 ? t.split != 0 : id != knob) : t.split != 2 && t.bm * t.bn > 64 * 64 && K < 80) continue;
         const double tiles_m = (double)ceil_div((size_t)M, (size_t)t.bm), tiles_n = (double)ceil_div((size_t)N, (size_t)t.bn);
         const double slow = t.split ? 1.0 : 1.0 + 0.16 * ((ta ? 1 : 0) + (tb ? 0 : 1));
         // slices: a few, and what fills every compute unit once, twice and three times
@@ -363,21 +381,60 @@ GemmPlan plan_gemm(int ta, int tb, int M, int N, int K, bool reads_c, int lda, i
             if (want > 1 && !g_ctx.gemm_splitk && (k_slice < 128 || slices * out > 64e6)) continue;
             const double n = up(tiles_m * tiles_n * slices / cus);                      // workgroups of the busiest compute unit
             const double work = steps * std::max(t.alone, n * t.shared) * slow + t.fixed * up(n / t.resident);
-            const double hbm = 4.0 * ((double)M * K + (double)N * K + out * (slices > 1 ? slices : reads_c ? 2 : 1));
-            const double l2 = 4.0 * K * (M * tiles_n + N * tiles_m);
+            const double hbm = 4.0 * ((double)M * K + out * (slices > 1 ? slices : c_times)) + (t.split == 2 ? planes : 4.0 * N * K);
+            const double l2 = t.split == 2 ? 0.0 : 4.0 * K * (M * tiles_n + N * tiles_m);
             const double mem = std::max(hbm / 5.6e6, l2 / 21e6);
             double us = 3.4 + std::max(work, mem) + 0.23 * std::min(work, mem);
             if (slices > 1) us += 5.4 + slices * out * 4.0 / 5.6e6;
-            if (best_us < 0.0 || us < best_us) { best_us = us; best = GemmPlan{t.split, t.groups, t.bm, t.bn, slices, k_slice}; }
+            if (t.split == 2) us += split_us;
+            if (best_us < 0.0 || us < best_us) { best_us = us; best = GemmPlan{t.split, t.groups, t.bm, t.bn, slices, k_slice, 1}; }
+        }
+    }
+    // Rows of A held whole, 96 or 64 of them: the columns dealt out over a few ranges, each with a workgroup of its own per block
+    // of rows, where the blocks alone leave compute units idle.
+    for (int fm : {6, 4}) {
+        if (knob ? knob != (fm == 6 ? 7 : 8) : g_ctx.gemm_splitk > 1) continue;
+        if (!planes_ok || plane_steps(K) > rows_steps(fm) || ldc >= (1 << 22)) continue;        // (32-bit offsets into C)
+        const int units = (int)ceil_div((size_t)N, 32), waves = R_THREADS / 64;
+        const double blocks = (double)ceil_div((size_t)M, 16 * (size_t)fm);
+        for (int want = 1; want <= 8 && waves * (want - 1) < units; want++) {
+            const int per = (int)ceil_div((size_t)units, (size_t)want), ranges = (int)ceil_div((size_t)units, (size_t)per);
+            if (per > R_UNITS) continue;
+            const double work = up(blocks * ranges / cus) * (5.5 + up((double)per / waves) * (0.55 + plane_steps(K) * fm * 0.357));
+            const double mem = (4.0 * ((double)M * K * ranges + (double)M * N * c_times) + planes) / 5.6e6;
+            const double us = 3.4 + split_us + std::max(work, mem) + 0.21 * std::min(work, mem);
+            if (best_us < 0.0 || us < best_us) { best_us = us; best = GemmPlan{3, 1, 16 * fm, 32 * per, 1, K, ranges}; }
         }
     }
     return best;
 }
 
+// Where the planes of an operand lie: grow-only, at most P_MAX_BYTES and the flags, freed with the caches.  Not the workspace: a
+// product is never recorded, so no graph holds this address and none goes stale when a product needs more of it.  NULL where
+// there is no memory for it (the other kernels then take the product).
+char *g_planes = nullptr;
+size_t g_planes_bytes = 0;
+char *plane_space(size_t bytes) {
+    if (bytes <= g_planes_bytes) return g_planes;
+    mi355_free_planes();
+    const size_t want = (bytes + 0xFFFFF) & ~(size_t)0xFFFFF;   // 1 MiB granules
+    void *p = nullptr;
+    if (hipMalloc(&p, want) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    g_planes = (char *)p;
+    g_planes_bytes = want;
+    return g_planes;
+}
+
 // The product within the limits of one launch: M, N, K <= 2^30 and 2^21 tiles of 64 x 64 (the caller cuts larger ones).
 int sgemm_piece(int ta, int tb, int M, int N, int K, float alpha, const float *A, int lda, const float *B, int ldb, float beta,
                 float *C, int ldc) {
-    const GemmPlan p = plan_gemm(ta, tb, M, N, K, beta != 0.f, lda, ldb);
+    // (alpha == 0 reads neither operand: nothing is split ahead)
+    GemmPlan p = plan_gemm(ta, tb, M, N, K, beta != 0.f, lda, ldb, ldc, alpha != 0.f);
+    char *planes = nullptr;
+    if (p.split >= 2 && !(planes = plane_space(plane_bytes(N, K)))) p = plan_gemm(ta, tb, M, N, K, beta != 0.f, lda, ldb, ldc, false);
     float *part = nullptr;
     if (p.slices > 1) {
         part = (float *)mi355_ws((size_t)p.slices * M * N * sizeof(float));
@@ -389,6 +446,20 @@ int sgemm_piece(int ta, int tb, int M, int N, int K, float alpha, const float *A
     auto launch = [&](auto kernel, int threads) {
         hipLaunchKernelGGL(kernel, dim3((unsigned)tiles * p.slices), dim3(threads), 0, g_ctx.stream, A, lda, B, ldb, C, ldc, M, N,
                            k_all, p.k_slice, tiles_n, tiles, alpha, beta, part);
+    };
+    const int psteps = plane_steps(K);
+    int *inexact = nullptr;
+    if (p.split >= 2) {
+        const int units = plane_cols(N) * psteps;               // (P_MAX_BYTES keeps it small)
+        inexact = (int *)(planes + (size_t)units * P_UNIT);
+        const dim3 grid((unsigned)ceil_div((size_t)units, 4));
+        if (tb) hipLaunchKernelGGL(split_planes_kernel<true>, grid, dim3(256), 0, g_ctx.stream, planes, inexact, B, ldb, N, K, psteps, units);
+        else hipLaunchKernelGGL(split_planes_kernel<false>, grid, dim3(256), 0, g_ctx.stream, planes, inexact, B, ldb, N, K, psteps, units);
+        LAUNCH_OK("sgemm planes");
+    }
+    auto launch_planes = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)tiles * p.slices), dim3(P_THREADS), 0, g_ctx.stream, A, lda, B, ldb, C, ldc, M, N,
+                           k_all, p.k_slice, tiles_n, tiles, alpha, beta, part, (const char *)planes, (const int *)inexact, psteps);
     };
 #define GEMM_CASE(BM, BN, WM, WN, KS)                                                                                 \
     case gemm_key(0, KS, BM, BN): {                                                                                   \
@@ -413,6 +484,27 @@ int sgemm_piece(int ta, int tb, int M, int N, int K, float alpha, const float *A
         else if (!tb) launch(sgemm_split_kernel<BM, BN, true, false>, S_THREADS);                                 \
         else launch(sgemm_split_kernel<BM, BN, true, true>, S_THREADS);                                           \
         break;
+    auto launch_rows = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(ceil_div((size_t)M, (size_t)p.bm) * p.ranges)), dim3(R_THREADS), 0, g_ctx.stream, A, lda,
+                           B, ldb, C, ldc, M, N, K, p.bn / 32, p.ranges, alpha, beta, (const char *)planes,
+                           (const int *)inexact, psteps);
+    };
+#define ROWS_CASE(FM)                                                                                                 \
+    if (p.split == 3 && p.bm == 16 * FM) {                                                                            \
+        if (!ta && !tb) launch_rows(sgemm_rows_kernel<FM, false, false>);                                             \
+        else if (!ta) launch_rows(sgemm_rows_kernel<FM, false, true>);                                                \
+        else if (!tb) launch_rows(sgemm_rows_kernel<FM, true, false>);                                                \
+        else launch_rows(sgemm_rows_kernel<FM, true, true>);                                                          \
+    } else
+#define PLANES_CASE(BM)                                                                                               \
+    case gemm_key(2, 1, BM, PN):                                                                                      \
+        if (!ta && !tb) launch_planes(sgemm_planes_kernel<BM, false, false>);                                         \
+        else if (!ta) launch_planes(sgemm_planes_kernel<BM, false, true>);                                            \
+        else if (!tb) launch_planes(sgemm_planes_kernel<BM, true, false>);                                            \
+        else launch_planes(sgemm_planes_kernel<BM, true, true>);                                                      \
+        break;
+    ROWS_CASE(6)
+    ROWS_CASE(4)
     switch (gemm_key(p.split, p.groups, p.bm, p.bn)) {
         GEMM_CASE(64, 64, 32, 32, 1)
         GEMM_CASE(64, 64, 32, 32, 2)
@@ -422,11 +514,15 @@ int sgemm_piece(int ta, int tb, int M, int N, int K, float alpha, const float *A
         SMALL_CASE(64, 64, 32, 32, 2)
         SPLIT_CASE(128, 256)
         SPLIT_CASE(256, 128)
+        PLANES_CASE(96)
+        PLANES_CASE(64)
         default: return mi355_fail("sgemm: no kernel for a tile of %d x %d", p.bm, p.bn);
     }
 #undef GEMM_CASE
 #undef SMALL_CASE
 #undef SPLIT_CASE
+#undef PLANES_CASE
+#undef ROWS_CASE
     LAUNCH_OK("sgemm");
     if (part) {
         auto sum = [&](auto kernel, int groups) {
@@ -441,6 +537,14 @@ int sgemm_piece(int ta, int tb, int M, int N, int K, float alpha, const float *A
 }
 
 }   // namespace
+
+void mi355_free_planes(void) {
+    if (!g_planes) return;
+    (void)hipStreamSynchronize(g_ctx.stream);
+    (void)hipFree(g_planes);
+    g_planes = nullptr;
+    g_planes_bytes = 0;
+}
 
 MI355_API int mi355_sgemm_dev(int trans_a, int trans_b, int M, int N, int K, float alpha, const float *A, int lda,
                               const float *B, int ldb, float beta, float *C, int ldc) {

@@ -42,6 +42,21 @@ template <int F>
 __device__ __forceinline__ int split_row(int slot) { return (slot & ~(16 * F - 1)) | (slot & 15) * F | ((slot >> 4) & (F - 1)); }
 
 struct Planes { v4u h, m, l; };
+// splits values 2 j0 .. 2 j1 - 1 of a piece; the low half of `left` takes what a split could not hold
+__device__ __forceinline__ void split_eight(const float (&r)[8], int j0, int j1, Planes &o, unsigned &left) {
+#pragma unroll
+    for (int j = j0; j < j1; j++) {
+        float a = r[2 * j], b = r[2 * j + 1];
+        o.h[j] = f2_to_bf2(a, b);
+        a -= bf_to_f(o.h[j]);
+        b -= __uint_as_float(o.h[j] & 0xffff0000u);
+        o.m[j] = f2_to_bf2(a, b);
+        a -= bf_to_f(o.m[j]);
+        b -= __uint_as_float(o.m[j] & 0xffff0000u);
+        o.l[j] = f2_to_bf2(a, b);
+        left |= __float_as_uint(a) | __float_as_uint(b);
+    }
+}
 
 // One operand tile of BX rows (of M or N) by SK: global -> registers -> three planes in LDS.  KC: k is the contiguous index.
 // THREADS: of the group of waves that loads it, tid() a thread's number in the group; groups take the steps in turn.
@@ -125,20 +140,8 @@ struct SplitOperand {
 #pragma unroll
             for (int k = 0; k < 8; k++) r[i][k] = 8 * kc + k < n ? *(const float *)(base + k * row + off[i]) : 0.f;
     }
-    // splits values 2 j0 .. 2 j1 - 1 of piece p; the low half of `left` takes what a split could not hold
     __device__ __forceinline__ void split(int p, int j0, int j1, Planes &o, unsigned &left) const {
-#pragma unroll
-        for (int j = j0; j < j1; j++) {
-            float a = r[p][2 * j], b = r[p][2 * j + 1];
-            o.h[j] = f2_to_bf2(a, b);
-            a -= bf_to_f(o.h[j]);
-            b -= __uint_as_float(o.h[j] & 0xffff0000u);
-            o.m[j] = f2_to_bf2(a, b);
-            a -= bf_to_f(o.m[j]);
-            b -= __uint_as_float(o.m[j] & 0xffff0000u);
-            o.l[j] = f2_to_bf2(a, b);
-            left |= __float_as_uint(a) | __float_as_uint(b);
-        }
+        split_eight(r[p], j0, j1, o, left);
     }
     __device__ __forceinline__ void write(int p, const Planes &o, char *lds) const {
         const int slot = piece_slot(p);
@@ -149,11 +152,55 @@ struct SplitOperand {
     }
 };
 
+// The wave's fragments at rows m0.. and columns n0.., over k_beg .. k_end, again with the fp32 instruction.
+// Register e of a lane's fragment i, j: row FM * (4 * quarter + e) + i, column FN * li + j; ROWS16: row 16 * i + 4 * quarter + e.
+template <int FM, int FN, bool TA, bool TB, bool ROWS16>
+__device__ __forceinline__ void split_again(v4f (&acc)[FM][FN], const float *__restrict__ A, int lda,
+                                            const float *__restrict__ B, int ldb, int M, int N, int m0, int n0, int k_beg,
+                                            int k_end) {
+    const int lane = threadIdx.x & 63, quarter = lane >> 4, li = lane & 15;
+    const float *pa[FM], *pb[FN];
+#pragma unroll
+    for (int i = 0; i < FM; i++) {
+#pragma unroll
+        for (int j = 0; j < FN; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+        const int m = min(m0 + (ROWS16 ? 16 * i + li : FM * li + i), M - 1);
+        pa[i] = TA ? A + m : A + (size_t)m * lda;
+    }
+#pragma unroll
+    for (int j = 0; j < FN; j++) {
+        const int nn = min(n0 + FN * li + j, N - 1);
+        pb[j] = TB ? B + (size_t)nn * ldb : B + nn;
+    }
+    for (int k0 = k_beg; k0 < k_end; k0 += 4) {
+        const int k = k0 + quarter;
+        float va[FM], vb[FN];
+#pragma unroll
+        for (int i = 0; i < FM; i++) va[i] = k < k_end ? pa[i][TA ? (size_t)k * lda : (size_t)k] : 0.f;
+#pragma unroll
+        for (int j = 0; j < FN; j++) vb[j] = k < k_end ? pb[j][TB ? (size_t)k : (size_t)k * ldb] : 0.f;
+#pragma unroll
+        for (int i = 0; i < FM; i++)
+#pragma unroll
+            for (int j = 0; j < FN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[i], vb[j], acc[i][j], 0, 0, 0);
+    }
+}
+template <int FM, int FN>
+__device__ __forceinline__ bool split_not_finite(const v4f (&acc)[FM][FN]) {
+    bool again = false;
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) again |= (__float_as_uint(acc[i][j][e]) & 0x7f800000u) == 0x7f800000u;
+    return again;
+}
+
 // The end of a tile: the wave's fragments at rows m0.. and columns n0.., computed again where values called for it
 // (`left`: what the splits could not hold), scaled and stored; part: where the bare product of the slice goes, or NULL;
 // mine: this wave finishes them.
-// Register e of a lane's fragment i, j: row FM * (4 * quarter + e) + i, column FN * li + j.
-template <int FM, int FN, bool TA, bool TB>
+template <int FM, int FN, bool TA, bool TB, bool ROWS16 = false>
 __device__ __forceinline__ void split_finish(v4f (&acc)[FM][FN], unsigned left, const float *__restrict__ A, int lda,
                                              const float *__restrict__ B, int ldb, float *C, int ldc, int M, int N, int m0,
                                              int n0, int k_beg, int k_end, float alpha, float beta, float *__restrict__ part,
@@ -161,42 +208,9 @@ __device__ __forceinline__ void split_finish(v4f (&acc)[FM][FN], unsigned left, 
     typedef float vec __attribute__((ext_vector_type(FN), aligned(4)));
     const int lane = threadIdx.x & 63, quarter = lane >> 4, li = lane & 15;
     const int n = n0 + FN * li;
-    bool again = (left & 0xffffu) != 0;
-#pragma unroll
-    for (int i = 0; i < FM; i++)
-#pragma unroll
-        for (int j = 0; j < FN; j++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) again |= (__float_as_uint(acc[i][j][e]) & 0x7f800000u) == 0x7f800000u;
-    const bool bad = __syncthreads_or(again);
+    const bool bad = __syncthreads_or((left & 0xffffu) != 0 || split_not_finite<FM, FN>(acc));
     if (!mine) return;
-    if (bad) {
-        const float *pa[FM], *pb[FN];
-#pragma unroll
-        for (int i = 0; i < FM; i++) {
-#pragma unroll
-            for (int j = 0; j < FN; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-            const int m = min(m0 + FM * li + i, M - 1);
-            pa[i] = TA ? A + m : A + (size_t)m * lda;
-        }
-#pragma unroll
-        for (int j = 0; j < FN; j++) {
-            const int nn = min(n + j, N - 1);
-            pb[j] = TB ? B + (size_t)nn * ldb : B + nn;
-        }
-        for (int k0 = k_beg; k0 < k_end; k0 += 4) {
-            const int k = k0 + quarter;
-            float va[FM], vb[FN];
-#pragma unroll
-            for (int i = 0; i < FM; i++) va[i] = k < k_end ? pa[i][TA ? (size_t)k * lda : (size_t)k] : 0.f;
-#pragma unroll
-            for (int j = 0; j < FN; j++) vb[j] = k < k_end ? pb[j][TB ? (size_t)k : (size_t)k * ldb] : 0.f;
-#pragma unroll
-            for (int i = 0; i < FM; i++)
-#pragma unroll
-                for (int j = 0; j < FN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[i], vb[j], acc[i][j], 0, 0, 0);
-        }
-    }
+    if (bad) split_again<FM, FN, TA, TB, ROWS16>(acc, A, lda, B, ldb, M, N, m0, n0, k_beg, k_end);
 
     float *out = part ? part : C;
     const int ldo = part ? N : ldc;
@@ -207,7 +221,7 @@ __device__ __forceinline__ void split_finish(v4f (&acc)[FM][FN], unsigned left, 
         for (int i = 0; i < FM; i++)
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                const int m = m0 + FM * (4 * quarter + e) + i;
+                const int m = m0 + (ROWS16 ? 16 * i + 4 * quarter + e : FM * (4 * quarter + e) + i);
                 if (m < M) fn(i, e, out + (size_t)m * ldo + n);
             }
     };

@@ -112,6 +112,7 @@ Table *resident_table(const char *who, const float *embed, int vocab, int dim) {
 
 void mi355_free_rope_cache(void);
 void mi355_free_scatter_report(void);
+void mi355_free_planes(void);
 
 void mi355_free_caches(void) {
     for (auto &s : g_slot) { if (s.dev) (void)hipFree(s.dev); s = Slot{}; }
@@ -119,6 +120,7 @@ void mi355_free_caches(void) {
     g_tab_n = 0;
     mi355_free_rope_cache();
     mi355_free_scatter_report();
+    mi355_free_planes();
 }
 
 MI355_API void mi355_rmsnorm(float *out, const float *x, const float *w, int d, int S) {

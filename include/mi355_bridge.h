@@ -58,7 +58,8 @@ size_t mi355_workspace_size(void);
  * "ce_rows" / "ce_rows2" (rows of logits per workgroup in the first / second pass of softmax-CE),
  * "gemm_splitk" (K slices of mi355_sgemm_dev; 1 = never split), "gemm_split" (its kernels that multiply fp32 values as
  * sums of three bfloat16 values: 0 = where they pay, -1 = never, 1 / 2 = always, in tiles of 128 x 256 / 256 x 128,
- * 3 / 4 = always, in tiles of 64 x 64 with one / two groups of waves),
+ * 3 / 4 = always, in tiles of 64 x 64 with one / two groups of waves, 5 / 6 = B split by a launch of its own, tiles of 96 x 256 /
+ * 64 x 256, 7 / 8 = the same with 96 / 64 whole rows of A in LDS, for K up to 256 / 384),
  * "scatter_tree" (1: mi355_embed_scatter_add_dev sums long segments by a fixed tree instead of the reference's
  * sequential order: still deterministic and within 1e-5 of each row's scale, faster, no longer bit-identical to
  * the CPU loop), "scatter_cols" (the form of mi355_embed_scatter_add_dev in which every workgroup owns a few columns
