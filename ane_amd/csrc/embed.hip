@@ -4,8 +4,8 @@
 // training/training_dynamic/cpu_ops.h:150-156) and embed_backward (stories_cpu_ops.h:123-131;
 // cpu_ops.h:158-164).  The table E is [V][D] row-major, activations are [batch][D][S].
 //
-// Gather: a 64-token x 64-dim tile goes through LDS so that both sides are coalesced — table
-// rows are read along d (256 B runs), the channel-first output is written along t (256 B runs).
+// Gather: a tile of tokens x dims goes through LDS so that both sides are coalesced — table rows are read along d, the
+// channel-first output is written along t.
 //
 // Scatter-add: the reference adds dx[:,t] into dE[tok_t] for t ascending, so each (row, d) sum has
 // a fixed order.  To reproduce it bit for bit:
@@ -38,15 +38,23 @@ constexpr int STAGE_ROWS = 15 * ROWS_PER_WAVE;    // two buffers of 240 rows x 1
 // ---------------------------------------------------------------------------------------------
 // Gather
 // ---------------------------------------------------------------------------------------------
-template <bool VEC_D>
+// A tile of GT positions by GD dims goes through LDS.  What bounds it is the way of the output: pieces of GT floats of rows of S
+// floats.  Where rows are whole 128-byte lines, 64 x 64 writes whole lines ([64][768][256] 11.4 us; 256 x 32 12.7).  Otherwise a piece
+// begins and ends inside a line whose other part belongs to the next tile: longer pieces have fewer such lines, and tiles next to each
+// other along the positions run on one XCD, whose L2 puts the parts together ([40][1024][1000], 164 MB: 64 x 64 in the order of
+// the grid 71 us, in this order 53, 256 x 32 41.5).  Four positions of one sequence are stored as one access at any
+// alignment ([37][768][333] 21.5 -> 14.3 us).
+template <bool VEC_D, int GT, int GD>
 __global__ __launch_bounds__(256) void gather_kernel(float *__restrict__ x, const float *__restrict__ E,
                                                      const int32_t *__restrict__ ids, int V, int D, int S, int N) {
-    __shared__ float tile[TT][TD + 1];
-    __shared__ int tok[TT];
-    const int n0 = blockIdx.x * TT;            // 64 consecutive positions, of one or several sequences
-    const int d0 = blockIdx.y * TD;
+    __shared__ float tile[GT][GD + 1];
+    __shared__ int tok[GT];
+    const int tiles_n = (N + GT - 1) / GT;
+    const int logical = xcd_remap(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
+    const int n0 = logical % tiles_n * GT;     // consecutive positions, of one or several sequences
+    const int d0 = logical / tiles_n * GD;
     const int tid = threadIdx.x;
-    if (tid < TT) {
+    if (tid < GT) {
         const int n = n0 + tid;
         int id = -1;
         if (n < N) {
@@ -58,43 +66,46 @@ __global__ __launch_bounds__(256) void gather_kernel(float *__restrict__ x, cons
     __syncthreads();
     // phase 1: table rows -> LDS, lanes along d
     {
-        const int dq = tid & 15, r0 = tid >> 4;
+        constexpr int LANES = GD / 4, ROWS = 256 / LANES;
+        const int dq = tid % LANES, r0 = tid / LANES, d = d0 + 4 * dq;
+        v4f v[GT / ROWS];
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const int r = r0 + 16 * k;
-            const int id = tok[r];
-            const int d = d0 + 4 * dq;
+        for (int k = 0; k < GT / ROWS; k++) {
+            const int id = tok[r0 + ROWS * k];
+            v[k] = v4f{0.f, 0.f, 0.f, 0.f};
             if (id >= 0) {
                 const float *src = E + (size_t)id * D + d;
                 if (VEC_D && d + 3 < D) {
-                    v4f v = ld4(src);
-                    tile[r][4 * dq + 0] = v.x; tile[r][4 * dq + 1] = v.y;
-                    tile[r][4 * dq + 2] = v.z; tile[r][4 * dq + 3] = v.w;
+                    v[k] = ld4(src);
                 } else {
 #pragma unroll
                     for (int j = 0; j < 4; j++)
-                        if (d + j < D) tile[r][4 * dq + j] = src[j];
+                        if (d + j < D) v[k][j] = src[j];
                 }
             }
         }
+#pragma unroll
+        for (int k = 0; k < GT / ROWS; k++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) tile[r0 + ROWS * k][4 * dq + j] = v[k][j];
     }
     __syncthreads();
-    // phase 2: LDS -> channel-first output, lanes along positions; four consecutive positions lie in one sequence
-    // when S is a multiple of 4
+    // phase 2: LDS -> channel-first output, lanes along positions; four consecutive positions of one sequence at a time
     {
-        const int tq = tid & 15, r0 = tid >> 4;
+        constexpr int LANES = GT / 4, ROWS = 256 / LANES;
+        const int tq = tid % LANES, r0 = tid / LANES;
         const int n4 = n0 + 4 * tq;
-        const int i0 = tok[4 * tq], i1 = tok[4 * tq + 1], i2 = tok[4 * tq + 2], i3 = tok[4 * tq + 3];
-        const bool all = (i0 >= 0) & (i1 >= 0) & (i2 >= 0) & (i3 >= 0) & ((S & 3) == 0) & (((uintptr_t)x & 15u) == 0);
+        const bool all = (tok[4 * tq] >= 0) & (tok[4 * tq + 1] >= 0) & (tok[4 * tq + 2] >= 0) & (tok[4 * tq + 3] >= 0);
         const int b4 = n4 / S, t4 = n4 - b4 * S;
+        const bool whole = all && t4 + 4 <= S;
+        float *to = x + ((size_t)b4 * D + d0) * S + t4;
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const int dl = r0 + 16 * k;
-            const int d = d0 + dl;
+        for (int k = 0; k < GD / ROWS; k++) {
+            const int dl = r0 + ROWS * k, d = d0 + dl;
             if (d >= D) continue;
-            if (all) {
-                v4f v = {tile[4 * tq][dl], tile[4 * tq + 1][dl], tile[4 * tq + 2][dl], tile[4 * tq + 3][dl]};
-                st4(x + ((size_t)b4 * D + d) * S + t4, v);
+            if (whole) {
+                const v4f v = {tile[4 * tq][dl], tile[4 * tq + 1][dl], tile[4 * tq + 2][dl], tile[4 * tq + 3][dl]};
+                st4_nt(to + (size_t)dl * S, v);
             } else {
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
@@ -105,6 +116,18 @@ __global__ __launch_bounds__(256) void gather_kernel(float *__restrict__ x, cons
             }
         }
     }
+}
+
+template <int GT, int GD>
+int launch_gather(float *x, const float *E, const int32_t *ids, int V, int D, int S, int N) {
+    const size_t tiles_n = ceil_div((size_t)N, GT), tiles_d = ceil_div((size_t)D, GD), tiles = tiles_n * tiles_d;
+    // (a grid dimension holds 2^32 threads)
+    const dim3 grid = tiles < ((size_t)1 << 24) ? dim3((unsigned)tiles) : dim3((unsigned)tiles_n, (unsigned)tiles_d);
+    if (grid.y > 65535) return mi355_fail("embed_gather: D too large");
+    if (D % 4 == 0) hipLaunchKernelGGL((gather_kernel<true, GT, GD>), grid, dim3(256), 0, g_ctx.stream, x, E, ids, V, D, S, N);
+    else hipLaunchKernelGGL((gather_kernel<false, GT, GD>), grid, dim3(256), 0, g_ctx.stream, x, E, ids, V, D, S, N);
+    LAUNCH_OK("embed_gather");
+    return 0;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -838,13 +861,13 @@ MI355_API int mi355_embed_gather_dev(float *x, const float *E, const int32_t *id
     if (V <= 0 || D <= 0 || S <= 0 || batch <= 0) return mi355_fail("embed_gather: bad shape V=%d D=%d S=%d batch=%d", V, D, S, batch);
     if ((size_t)batch * S > (size_t)1 << 30) return mi355_fail("embed_gather: more than 2^30 positions");
     const int N = batch * S;
-    const dim3 grid((unsigned)ceil_div((size_t)N, TT), (unsigned)ceil_div((size_t)D, TD));
-    if (grid.y > 65535) return mi355_fail("embed_gather: D too large");
-    const bool vec_d = (D % 4 == 0) && aligned16(E) && aligned16(x);
-    if (vec_d) hipLaunchKernelGGL((gather_kernel<true>), grid, dim3(256), 0, g_ctx.stream, x, E, ids, V, D, S, N);
-    else hipLaunchKernelGGL((gather_kernel<false>), grid, dim3(256), 0, g_ctx.stream, x, E, ids, V, D, S, N);
-    LAUNCH_OK("embed_gather");
-    return 0;
+    // Rows of whole lines: see gather_kernel.  Others: 256 x 32, or 256 x 16 where that leaves fewer than eight workgroups to a
+    // compute unit ([37][768][333] 14.3 us with 16 dims, 16.4 with 32; [40][1024][1000] 43.4 and 41.5).
+    const size_t wide = ceil_div((size_t)N, 256) * ceil_div((size_t)D, 32);
+    const size_t cus = g_ctx.num_cu > 0 ? g_ctx.num_cu : 256;
+    if ((S % 32 == 0 && ((uintptr_t)x & 127u) == 0) || wide >= ((size_t)1 << 23)) return launch_gather<64, 64>(x, E, ids, V, D, S, N);
+    if (wide >= 8 * cus) return launch_gather<256, 32>(x, E, ids, V, D, S, N);
+    return launch_gather<256, 16>(x, E, ids, V, D, S, N);
 }
 
 // Which form takes an input of N positions and row width D.  Both forms give the same bits, so the choice is only a
