@@ -1,7 +1,6 @@
 // host_dropins.hip — host-pointer entry points with the reference's own signatures.
 //
-// Each stages its operands through cached device buffers (H2D, kernels, D2H) and returns when the
-// result is in host memory, so a caller of the reference's CPU ops swaps the symbol only:
+// Each brings its operands to the device, runs the kernels and returns when the result is in host memory (host_stage.h), so a caller of the reference's CPU ops swaps the symbol only:
 //   rmsnorm / rmsnorm_bwd            training/stories_cpu_ops.h:6-53
 //   cross_entropy_loss               training/stories_cpu_ops.h:71-108, training/training_dynamic/cpu_ops.h:68-93
 //   embed_lookup / embed_backward    training/stories_cpu_ops.h:112-131
@@ -9,8 +8,14 @@
 // Failures print one "mi355_bridge: ..." line and leave the outputs untouched.
 #include "common.h"
 
+#include <emmintrin.h>
+#include <pthread.h>
+#include <sched.h>
+#include <signal.h>
 #include <stdlib.h>
+#include <unistd.h>
 #include <algorithm>
+#include <atomic>
 #include <vector>
 
 namespace {
@@ -48,6 +53,14 @@ bool d2h(void *dst, const void *src, size_t bytes) {
     if (e == hipSuccess) e = hipStreamSynchronize(g_ctx.stream);
     if (e != hipSuccess) { mi355_fail("D2H copy: %s", hipGetErrorString(e)); return false; }
     return true;
+}
+
+#include "host_stage.h"
+
+// A device call of a drop-in that failed: its inputs may still be on their way.
+bool ran(int rc) {
+    if (rc) (void)hipStreamSynchronize(g_ctx.stream);
+    return rc == 0;
 }
 
 // resident embedding tables, keyed by host address
@@ -115,6 +128,7 @@ void mi355_free_scatter_report(void);
 void mi355_free_planes(void);
 
 void mi355_free_caches(void) {
+    free_stage();
     for (auto &s : g_slot) { if (s.dev) (void)hipFree(s.dev); s = Slot{}; }
     for (int i = 0; i < g_tab_n; i++) if (g_tab[i].dev) (void)hipFree(g_tab[i].dev);
     g_tab_n = 0;
@@ -127,44 +141,42 @@ MI355_API void mi355_rmsnorm(float *out, const float *x, const float *w, int d, 
     if (!host_ready("rmsnorm")) return;
     if (!out || !x || !w || d <= 0 || S <= 0) { mi355_fail("rmsnorm: bad arguments"); return; }
     const size_t nb = (size_t)d * S * sizeof(float);
-    float *dx = (float *)slot(0, nb), *dy = (float *)slot(1, nb), *dw = (float *)slot(2, (size_t)d * sizeof(float));
-    if (!dx || !dy || !dw) return;
-    if (!h2d(dx, x, nb) || !h2d(dw, w, (size_t)d * sizeof(float))) return;
-    if (mi355_rmsnorm_fwd_dev(dy, dx, dw, d, S, 1, 1e-5f)) return;
-    d2h(out, dy, nb);
+    Stage st;
+    const int ix = st.in(x, nb), iw = st.in(w, (size_t)d * sizeof(float)), iy = st.out(out, nb);
+    if (!st.send()) return;
+    if (!ran(mi355_rmsnorm_fwd_dev(st.dev<float>(iy), st.dev<float>(ix), st.dev<float>(iw), d, S, 1, 1e-5f))) return;
+    st.receive();
 }
 
 MI355_API void mi355_rmsnorm_bwd(float *dx, float *dw, const float *dy, const float *x, const float *w, int d, int S) {
     if (!host_ready("rmsnorm_bwd")) return;
     if (!dx || !dw || !dy || !x || !w || d <= 0 || S <= 0) { mi355_fail("rmsnorm_bwd: bad arguments"); return; }
     const size_t nb = (size_t)d * S * sizeof(float), wb = (size_t)d * sizeof(float);
-    float *x_d = (float *)slot(0, nb), *dy_d = (float *)slot(1, nb), *w_d = (float *)slot(2, wb);
-    float *dx_d = (float *)slot(3, nb), *dw_d = (float *)slot(4, wb);
-    if (!x_d || !dy_d || !w_d || !dx_d || !dw_d) return;
-    if (!h2d(x_d, x, nb) || !h2d(dy_d, dy, nb) || !h2d(w_d, w, wb) || !h2d(dw_d, dw, wb)) return;
-    if (mi355_rmsnorm_bwd_dev(dx_d, dw_d, dy_d, x_d, w_d, d, S, 1, 1e-5f, 0)) return;
-    std::vector<float> dw_new(d);
-    if (!d2h(dw_new.data(), dw_d, wb)) return;
-    if (!d2h(dx, dx_d, nb)) return;
-    memcpy(dw, dw_new.data(), wb);
+    Stage st;
+    const int ix = st.in(x, nb), iy = st.in(dy, nb), iw = st.in(w, wb), id = st.inout(dw, wb), io = st.out(dx, nb);
+    if (!st.send()) return;
+    if (!ran(mi355_rmsnorm_bwd_dev(st.dev<float>(io), st.dev<float>(id), st.dev<float>(iy), st.dev<float>(ix), st.dev<float>(iw), d, S,
+                                   1, 1e-5f, 0)))
+        return;
+    // (a queued reduction of dw would not be in time for the copy)
+    if (!ran(mi355_dw_flush())) return;
+    st.receive();
 }
 
 MI355_API float mi355_cross_entropy_loss(float *dlogits, const float *logits, const uint16_t *targets, int V, int S) {
     if (!host_ready("cross_entropy_loss")) return NAN;
     if (!dlogits || !logits || !targets || V <= 0 || S <= 0) { mi355_fail("cross_entropy_loss: bad arguments"); return NAN; }
     const size_t nb = (size_t)V * S * sizeof(float);
-    float *l_d = (float *)slot(0, nb);
-    int32_t *t_d = (int32_t *)slot(1, (size_t)S * sizeof(int32_t));
-    float *loss_d = (float *)slot(2, 256);
-    if (!l_d || !t_d || !loss_d) return NAN;
     std::vector<int32_t> t32(S);
     for (int t = 0; t < S; t++) t32[t] = targets[t];
-    if (!h2d(l_d, logits, nb) || !h2d(t_d, t32.data(), (size_t)S * sizeof(int32_t))) return NAN;
-    // the copy of t32 must finish before the vector dies; the loss read-back below synchronises
-    if (mi355_softmax_ce_dev(l_d, loss_d, l_d, t_d, V, S, 1.0f)) { (void)hipStreamSynchronize(g_ctx.stream); return NAN; }
     float loss = NAN;
-    if (!d2h(&loss, loss_d, sizeof(float))) return NAN;
-    if (!d2h(dlogits, l_d, nb)) return NAN;
+    Stage st;
+    // (the gradient takes the logits' place on the device, and has an array of its own on the host)
+    const int io = st.out(&loss, sizeof(float)), il = st.in(logits, nb), it = st.in(t32.data(), (size_t)S * sizeof(int32_t));
+    if (!st.send()) return NAN;
+    if (!ran(mi355_softmax_ce_dev(st.dev<float>(il), st.dev<float>(io), st.dev<float>(il), st.dev<int32_t>(it), V, S, 1.0f))) return NAN;
+    st.becomes(il, dlogits);
+    if (!st.receive()) return NAN;
     for (int t = 0; t < S; t++)
         if (targets[t] >= V)
             fprintf(stderr, "WARN: target token %d out of vocab range [0,%d), skipping\n", (int)targets[t], V);
@@ -221,19 +233,12 @@ MI355_API void mi355_embed_backward(float *d_embed, const float *dx, const uint1
         if (tokens[t] < vocab) cid[t] = (int32_t)(std::lower_bound(uniq.begin(), uniq.end(), (int)tokens[t]) - uniq.begin());
         else cid[t] = -1;
     }
-    const size_t rb = (size_t)dim * sizeof(float);
-    std::vector<float> rows((size_t)U * dim);
-    for (int u = 0; u < U; u++) memcpy(&rows[(size_t)u * dim], d_embed + (size_t)uniq[u] * dim, rb);
-    const size_t xb = (size_t)dim * seq * sizeof(float);
-    float *dx_d = (float *)slot(0, xb), *rows_d = (float *)slot(3, (size_t)U * rb);
-    int32_t *t_d = (int32_t *)slot(1, (size_t)seq * sizeof(int32_t));
-    if (!dx_d || !rows_d || !t_d) return;
-    bool ok = h2d(dx_d, dx, xb) && h2d(rows_d, rows.data(), (size_t)U * rb) &&
-              h2d(t_d, cid.data(), (size_t)seq * sizeof(int32_t));
-    if (ok) ok = mi355_embed_scatter_add_dev(rows_d, dx_d, t_d, U, dim, seq, 1) == 0;
-    if (!ok) { (void)hipStreamSynchronize(g_ctx.stream); return; }
-    if (!d2h(rows.data(), rows_d, (size_t)U * rb)) return;
-    for (int u = 0; u < U; u++) memcpy(d_embed + (size_t)uniq[u] * dim, &rows[(size_t)u * dim], rb);
+    Stage st;
+    const int ix = st.in(dx, (size_t)dim * seq * sizeof(float)), it = st.in(cid.data(), (size_t)seq * sizeof(int32_t));
+    const int ir = st.rows_inout(d_embed, uniq.data(), U, (size_t)dim * sizeof(float));
+    if (!st.send()) return;
+    if (!ran(mi355_embed_scatter_add_dev(st.dev<float>(ir), st.dev<float>(ix), st.dev<int32_t>(it), U, dim, seq, 1))) return;
+    st.receive();
 }
 
 MI355_API void mi355_rope_backward_inplace(float *dx, int seq, int dim, int hd) {
@@ -241,12 +246,11 @@ MI355_API void mi355_rope_backward_inplace(float *dx, int seq, int dim, int hd) 
     if (!dx || seq <= 0 || dim <= 0 || hd <= 0 || (hd & 1) || dim % hd) { mi355_fail("rope_backward_inplace: bad arguments"); return; }
     const float *c_d, *s_d;
     if (mi355_rope_tables_dev(&c_d, &s_d, seq, hd, 10000.0f)) return;
-    const size_t nb = (size_t)dim * seq * sizeof(float);
-    float *x_d = (float *)slot(0, nb);
-    if (!x_d) return;
-    if (!h2d(x_d, dx, nb)) return;
-    if (mi355_rope_dev(x_d, nullptr, x_d, nullptr, dim / hd, 0, hd, seq, 1, c_d, s_d, -1)) return;
-    d2h(dx, x_d, nb);
+    Stage st;
+    const int ix = st.inout(dx, (size_t)dim * seq * sizeof(float));
+    if (!st.send()) return;
+    if (!ran(mi355_rope_dev(st.dev<float>(ix), nullptr, st.dev<float>(ix), nullptr, dim / hd, 0, hd, seq, 1, c_d, s_d, -1))) return;
+    st.receive();
 }
 
 // SiLU-gate backward as one call: the 13 vDSP/vForce calls of training/training_dynamic/train.m:537-554.
@@ -254,13 +258,11 @@ MI355_API void mi355_swiglu_bwd(float *dh1, float *dh3, const float *dsilu, cons
     if (!host_ready("swiglu_bwd")) return;
     if (!dh1 || !dh3 || !dsilu || !h1 || !h3 || n == 0) { mi355_fail("swiglu_bwd: bad arguments"); return; }
     const size_t nb = n * sizeof(float);
-    float *d = (float *)slot(0, nb), *a = (float *)slot(1, nb), *b = (float *)slot(2, nb);
-    float *o1 = (float *)slot(3, nb), *o3 = (float *)slot(4, nb);
-    if (!d || !a || !b || !o1 || !o3) return;
-    if (!h2d(d, dsilu, nb) || !h2d(a, h1, nb) || !h2d(b, h3, nb)) return;
-    if (mi355_swiglu_bwd_dev(o1, o3, d, a, b, n)) return;
-    if (!d2h(dh1, o1, nb)) return;
-    d2h(dh3, o3, nb);
+    Stage st;
+    const int id = st.in(dsilu, nb), i1 = st.in(h1, nb), i3 = st.in(h3, nb), o1 = st.out(dh1, nb), o3 = st.out(dh3, nb);
+    if (!st.send()) return;
+    if (!ran(mi355_swiglu_bwd_dev(st.dev<float>(o1), st.dev<float>(o3), st.dev<float>(id), st.dev<float>(i1), st.dev<float>(i3), n))) return;
+    st.receive();
 }
 
 // SiLU-gate forward: out = (h1*sigmoid(h1))*h3 (training/forward.h:101,149-151).
@@ -268,11 +270,11 @@ MI355_API void mi355_swiglu_fwd(float *out, const float *h1, const float *h3, si
     if (!host_ready("swiglu_fwd")) return;
     if (!out || !h1 || !h3 || n == 0) { mi355_fail("swiglu_fwd: bad arguments"); return; }
     const size_t nb = n * sizeof(float);
-    float *a = (float *)slot(0, nb), *b = (float *)slot(1, nb), *o = (float *)slot(2, nb);
-    if (!a || !b || !o) return;
-    if (!h2d(a, h1, nb) || !h2d(b, h3, nb)) return;
-    if (mi355_swiglu_fwd_dev(o, a, b, n)) return;
-    d2h(out, o, nb);
+    Stage st;
+    const int i1 = st.in(h1, nb), i3 = st.in(h3, nb), io = st.out(out, nb);
+    if (!st.send()) return;
+    if (!ran(mi355_swiglu_fwd_dev(st.dev<float>(io), st.dev<float>(i1), st.dev<float>(i3), n))) return;
+    st.receive();
 }
 
 // Residual family on host pointers: vDSP_vsma / vDSP_vsmul / vDSP_vadd
@@ -281,12 +283,11 @@ MI355_API void mi355_axpby(float *y, const float *a, const float *b, float alpha
     if (!host_ready("axpby")) return;
     if (!y || !a || (mode != 1 && !b) || n == 0 || mode < 0 || mode > 2) { mi355_fail("axpby: bad arguments"); return; }
     const size_t nb = n * sizeof(float);
-    float *ad = (float *)slot(0, nb), *bd = (float *)slot(1, nb), *yd = (float *)slot(2, nb);
-    if (!ad || !bd || !yd) return;
-    if (!h2d(ad, a, nb)) return;
-    if (mode != 1 && !h2d(bd, b, nb)) return;
-    if (mi355_axpby_dev(yd, ad, mode != 1 ? bd : nullptr, alpha, n, mode)) return;
-    d2h(y, yd, nb);
+    Stage st;
+    const int ia = st.in(a, nb), ib = mode != 1 ? st.in(b, nb) : -1, iy = st.out(y, nb);
+    if (!st.send()) return;
+    if (!ran(mi355_axpby_dev(st.dev<float>(iy), st.dev<float>(ia), mode != 1 ? st.dev<float>(ib) : nullptr, alpha, n, mode))) return;
+    st.receive();
 }
 
 // adam_update (training/training_dynamic/cpu_ops.h:56-64) on host arrays.
@@ -295,16 +296,27 @@ MI355_API void mi355_adam_update(float *w, const float *g, float *m, float *v, s
     if (!host_ready("adam_update")) return;
     if (!w || !g || !m || !v || n == 0 || t < 1) { mi355_fail("adam_update: bad arguments"); return; }
     const size_t nb = n * sizeof(float);
-    float *wd_ = (float *)slot(0, nb), *gd = (float *)slot(1, nb), *md = (float *)slot(2, nb), *vd = (float *)slot(3, nb);
-    if (!wd_ || !gd || !md || !vd) return;
-    if (!h2d(wd_, w, nb) || !h2d(gd, g, nb) || !h2d(md, m, nb) || !h2d(vd, v, nb)) return;
-    if (mi355_adam_update_dev(wd_, gd, md, vd, n, t, lr, b1, b2, eps, wd, 1.0f, nullptr, 0)) return;
-    std::vector<float> w2(n), m2(n);
-    if (!d2h(w2.data(), wd_, nb) || !d2h(m2.data(), md, nb)) return;
-    if (!d2h(v, vd, nb)) return;
-    memcpy(w, w2.data(), nb);
-    memcpy(m, m2.data(), nb);
-    host_written_from(w, wd_, nb);      // a resident embedding table that lives in w follows on the device
+    Stage st;
+    const int ig = st.in(g, nb), iw = st.inout(w, nb), im = st.inout(m, nb), iv = st.inout(v, nb);
+    if (!st.send()) return;
+    if (!ran(mi355_adam_update_dev(st.dev<float>(iw), st.dev<float>(ig), st.dev<float>(im), st.dev<float>(iv), n, t, lr, b1, b2, eps, wd,
+                                   1.0f, nullptr, 0)))
+        return;
+    // Small arrays change together: w and m when v is there.
+    std::vector<float> w2, m2;
+    const bool small = nb <= PIECE;
+    if (small) {
+        w2.resize(n);
+        m2.resize(n);
+        st.becomes(iw, w2.data());
+        st.becomes(im, m2.data());
+    }
+    if (!st.receive()) return;
+    if (small) {
+        memcpy(w, w2.data(), nb);
+        memcpy(m, m2.data(), nb);
+    }
+    host_written_from(w, st.dev<float>(iw), nb);      // a resident embedding table that lives in w follows on the device
 }
 
 // ---- vocabulary compaction on host arrays: training/training_dynamic/cpu_ops.h:96-148 ----

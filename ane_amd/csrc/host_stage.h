@@ -1,0 +1,394 @@
+// host_stage.h — how the drop-ins on host arrays bring their operands to the device and their results back.
+// Included by host_dropins.hip inside its unnamed namespace.
+//
+// A copy from or to ordinary host memory goes through the runtime's own staging, one block after the other: 256 KB 106 us,
+// 4 MB 153 us in and 245 us out, where the same from pinned memory takes 12.6 and 81 us (55 GB/s and 6 us).  The caller's
+// arrays cannot be pinned, so a call packs its inputs into a pinned block of the library's own, in the order they have on the
+// device, and sends it in a few copies that grow (256 KB, 512 KB, ... 4 MB): while one travels the next is filled.  Results
+// come back the same way in copies that shrink, each unpacked while the next travels.  One thread moves 30 GB/s of memory
+// that is in no cache, so HELPERS threads of the library pack and unpack beside the caller's (1, 2, 3 and 6: 3.5, 2.5, 2.4 and
+// 2.5 ms for the nine calls of a layer, a loss and an update; 4.9 through the runtime).  What bounds it: the link, in one
+// direction at a time (88 MB, 1.6 ms).
+//
+// The helpers touch nothing but memory: they are given pieces of at most 64 KB, take them by counting up one number, and
+// mark each when it is done.  The caller takes pieces as well and waits only for pieces that somebody has taken, so a
+// helper that is asleep, late or was never created (no more processors, no threads left, a forked child) costs time and nothing
+// else.  Between calls they look for work for 100 us and then sleep.
+#pragma once
+
+constexpr int HELPERS = 3;
+constexpr size_t PIECE = (size_t)64 << 10;
+constexpr size_t PIN_MAX = (size_t)32 << 20;         // pinned bytes at most; longer transfers go in rounds of this
+constexpr int MAX_PIECES = (int)(PIN_MAX / PIECE) + 64;
+constexpr size_t SEND_MIN = (size_t)256 << 10, SEND_MAX = (size_t)4 << 20;
+constexpr int MAX_SENDS = 32;                        // copies of a round
+
+// A host array of a call and where it lies in the call's block.  rows: the array is `rows`[i] * row_bytes behind host for i =
+// 0 .., row_bytes each, and contiguous in the block.
+struct Part {
+    char *host;
+    size_t at, bytes;
+    const int *rows;
+    size_t row_bytes;
+};
+
+// memcpy past the caches: what the device reads next, or results that are larger than a cache (18.9 MB unpacked in 344 us, with
+// memcpy 450)
+void copy_past(char *to, const char *from, size_t n) {
+    if (n < 256) { memcpy(to, from, n); return; }
+    const size_t head = (16 - ((uintptr_t)to & 15)) & 15;
+    memcpy(to, from, head);
+    to += head;
+    from += head;
+    n -= head;
+    for (; n >= 64; n -= 64, to += 64, from += 64) {
+        __m128i v[4];
+        for (int i = 0; i < 4; i++) v[i] = _mm_loadu_si128((const __m128i *)(from + 16 * i));
+        for (int i = 0; i < 4; i++) _mm_stream_si128((__m128i *)(to + 16 * i), v[i]);
+    }
+    memcpy(to, from, n);
+    _mm_sfence();
+}
+
+// `bytes` bytes from byte `from` of a part on; to the block or back
+void move_part(const Part &p, size_t from, size_t bytes, char *block, bool in, bool past) {
+    const auto copy = [past](char *to, const char *from, size_t n) {
+        if (past) copy_past(to, from, n);
+        else memcpy(to, from, n);
+    };
+    if (!p.rows) {
+        if (in) copy(block, p.host + from, bytes);
+        else copy(p.host + from, block, bytes);
+        return;
+    }
+    while (bytes) {
+        const size_t r = from / p.row_bytes, o = from - r * p.row_bytes, n = p.row_bytes - o < bytes ? p.row_bytes - o : bytes;
+        char *h = p.host + (size_t)p.rows[r] * p.row_bytes + o;
+        if (in) copy(block, h, n);
+        else copy(h, block, n);
+        block += n;
+        from += n;
+        bytes -= n;
+    }
+}
+
+struct Piece {
+    const Part *part;
+    size_t from, bytes;
+    char *block;
+};
+
+struct Helpers {
+    pthread_t thread[HELPERS];
+    int n;                                // created
+    pid_t pid;                            // of the process that created them
+    pthread_mutex_t lock;
+    pthread_cond_t wake;
+    bool stop;                            // under the lock
+    std::atomic<int> asleep;
+    std::atomic<unsigned> calls;          // goes up with each round of pieces: a helper that has slept looks again
+    // the round at hand: pieces below `ready` may be taken; `next` counts them out (its upper half is the round's number, so that
+    // a helper that was late for a round takes nothing of the one behind it)
+    std::atomic<unsigned long long> next;
+    std::atomic<int> ready;
+    std::atomic<int> active;              // between the start of a round and its end
+    bool in, past;
+    Piece piece[MAX_PIECES];
+    std::atomic<unsigned char> done[MAX_PIECES];
+};
+Helpers *g_helpers = nullptr;
+
+// takes and moves one piece of the round; false if there is none to take
+bool one_piece(Helpers *h) {
+    unsigned long long n = h->next.load(std::memory_order_acquire);
+    for (;;) {
+        if ((int)(n & 0xffffffffu) >= h->ready.load(std::memory_order_acquire)) return false;
+        if (h->next.compare_exchange_weak(n, n + 1, std::memory_order_acq_rel, std::memory_order_acquire)) break;
+    }
+    const int i = (int)(n & 0xffffffffu);
+    const Piece &p = h->piece[i];
+    move_part(*p.part, p.from, p.bytes, p.block, h->in, h->past);
+    h->done[i].store(1, std::memory_order_release);
+    return true;
+}
+
+void *helper_main(void *arg) {
+    Helpers *h = (Helpers *)arg;
+    unsigned seen = h->calls.load(std::memory_order_acquire);
+    int idle = 0;
+    for (;;) {
+        if (one_piece(h)) { idle = 0; continue; }
+        if (h->active.load(std::memory_order_acquire)) idle = 0;           // pieces of this round are still to come
+        if (++idle < 800) {                               // about 100 us
+            for (int i = 0; i < 8; i++) __builtin_ia32_pause();
+            continue;
+        }
+        idle = 0;
+        pthread_mutex_lock(&h->lock);
+        h->asleep.fetch_add(1);
+        while (!h->stop && h->calls.load() == seen) pthread_cond_wait(&h->wake, &h->lock);
+        seen = h->calls.load();
+        h->asleep.fetch_sub(1);
+        const bool stop = h->stop;
+        pthread_mutex_unlock(&h->lock);
+        if (stop) return nullptr;
+    }
+}
+
+// The helpers' state, created with its threads on first use; NULL without memory for it.
+Helpers *helpers() {
+    if (g_helpers) return g_helpers;
+    Helpers *h = (Helpers *)calloc(1, sizeof(Helpers));
+    if (!h) return nullptr;
+    pthread_mutex_init(&h->lock, nullptr);
+    pthread_cond_init(&h->wake, nullptr);
+    h->pid = getpid();
+    cpu_set_t cpus;
+    const int have = sched_getaffinity(0, sizeof(cpus), &cpus) == 0 ? CPU_COUNT(&cpus) : 1;
+    sigset_t all, old;                                    // the program's signals are not for them
+    sigfillset(&all);
+    pthread_sigmask(SIG_SETMASK, &all, &old);
+    while (h->n < HELPERS && h->n + 1 < have && pthread_create(&h->thread[h->n], nullptr, helper_main, h) == 0) h->n++;
+    pthread_sigmask(SIG_SETMASK, &old, nullptr);
+    return g_helpers = h;
+}
+
+void stop_helpers() {
+    Helpers *h = g_helpers;
+    if (!h || h->pid != getpid()) return;                 // (a forked child has no threads to stop)
+    pthread_mutex_lock(&h->lock);
+    h->stop = true;
+    pthread_cond_broadcast(&h->wake);
+    pthread_mutex_unlock(&h->lock);
+    for (int i = 0; i < h->n; i++) pthread_join(h->thread[i], nullptr);
+    pthread_cond_destroy(&h->wake);
+    pthread_mutex_destroy(&h->lock);
+    free(h);
+    g_helpers = nullptr;
+}
+// (threads that run when the library's code goes away would crash)
+__attribute__((destructor)) void stop_helpers_at_exit() { stop_helpers(); }
+
+// ---- the blocks ----
+char *g_pin = nullptr, *g_pin_dev = nullptr;         // the host's address of it and the device's
+size_t g_pin_bytes = 0;
+hipEvent_t g_sent[MAX_SENDS] = {};
+
+// pinned memory for min(bytes, PIN_MAX) and the events of a round; NULL where there is none
+char *pinned(size_t bytes) {
+    if (!g_sent[MAX_SENDS - 1])
+        for (auto &e : g_sent)
+            if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) { e = nullptr; (void)hipGetLastError(); return nullptr; }
+    size_t want = (size_t)1 << 20;
+    while (want < bytes && want < PIN_MAX) want *= 2;
+    if (g_pin && g_pin_bytes >= want) return g_pin;
+    if (g_pin) (void)hipHostFree(g_pin);                   // (between calls nothing travels)
+    g_pin = nullptr;
+    g_pin_bytes = 0;
+    void *p = nullptr;
+    if (hipHostMalloc(&p, want, hipHostMallocMapped) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
+    void *d = nullptr;
+    if (hipHostGetDevicePointer(&d, p, 0) != hipSuccess) { (void)hipGetLastError(); (void)hipHostFree(p); return nullptr; }
+    g_pin_bytes = want;
+    g_pin_dev = (char *)d;
+    return g_pin = (char *)p;
+}
+
+// A copy between the pinned block and the device's: 16 bytes at a time, over the link at 50 GB/s from 1 MB on.  By a kernel, not
+// a copy engine: the engine waits 9 us for the kernel before it and lets the one behind it wait as long (16 MB in pieces of 1 MB:
+// 442 us in and 440 out, by kernels 375 and 332).
+__global__ __launch_bounds__(256) void stage_copy_kernel(v4i *__restrict__ to, const v4i *__restrict__ from, unsigned n) {
+    for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256)
+        __builtin_nontemporal_store(__builtin_nontemporal_load(from + i), to + i);
+}
+hipError_t stage_copy(char *to, const char *from, size_t bytes) {
+    const unsigned n = (unsigned)ceil_div(bytes, 16);
+    hipLaunchKernelGGL(stage_copy_kernel, dim3(std::min(512u, (n + 255) / 256)), dim3(256), 0, g_ctx.stream, (v4i *)to, (const v4i *)from, n);
+    return hipGetLastError();
+}
+
+void free_stage() {
+    stop_helpers();
+    if (g_pin) (void)hipHostFree(g_pin);
+    g_pin = g_pin_dev = nullptr;
+    g_pin_bytes = 0;
+    for (auto &e : g_sent) { if (e) (void)hipEventDestroy(e); e = nullptr; }
+}
+
+// The operands of one call: laid out one behind the other in a block of device memory, in the order in which they are added.
+// The inputs have to be neighbours, and the results (what lies between two of them travels with them).
+class Stage {
+public:
+    // each returns the part's number
+    int in(const void *host, size_t bytes) { return add((void *)host, bytes, true, false); }
+    int out(void *host, size_t bytes) { return add(host, bytes, false, true); }
+    int inout(void *host, size_t bytes) { return add(host, bytes, true, true); }
+    int rows_inout(void *host, const int *rows, size_t n, size_t row_bytes) {
+        const int i = add(host, n * row_bytes, true, true);
+        p_[i].rows = rows;
+        p_[i].row_bytes = row_bytes;
+        return i;
+    }
+    template <typename T>
+    T *dev(int i) const { return (T *)(dev_ + p_[i].at); }
+
+    // the part is a result from here on, and belongs to this array
+    void becomes(int i, void *host) { p_[i].host = (char *)host; in_[i] = false; out_[i] = true; }
+
+    // device memory, and the inputs on their way to it
+    bool send() {
+        dev_ = (char *)slot(0, total_);
+        if (!dev_) return false;
+        return move(true);
+    }
+    // brings the results to their arrays, which are untouched if the kernels failed
+    bool receive() { return move(false); }
+
+private:
+    static constexpr int MAX = 8;
+    Part p_[MAX];
+    bool in_[MAX], out_[MAX];
+    int n_ = 0;
+    size_t total_ = 0;
+    char *dev_ = nullptr;
+
+    int add(void *host, size_t bytes, bool in, bool out) {
+        p_[n_] = Part{(char *)host, total_, bytes, nullptr, 0};
+        in_[n_] = in;
+        out_[n_] = out;
+        total_ += (bytes + 255) & ~(size_t)255;
+        return n_++;
+    }
+    bool fail(const char *what, hipError_t e) const {
+        mi355_fail("%s copy: %s", what, hipGetErrorString(e));
+        (void)hipStreamSynchronize(g_ctx.stream);          // nothing of the call is in the blocks any more
+        return false;
+    }
+
+    bool move(bool in) {
+        const char *what = in ? "H2D" : "D2H";
+        size_t lo = total_, hi = 0;
+        for (int i = 0; i < n_; i++)
+            if (in ? in_[i] : out_[i]) {
+                lo = std::min(lo, p_[i].at);
+                hi = std::max(hi, p_[i].at + p_[i].bytes);
+            }
+        if (lo >= hi) return true;
+        char *pin = pinned(total_);                        // (as large for both directions: it does not move while inputs travel)
+        Helpers *h = helpers();
+        if (!pin || !h) return move_unpinned(in, what);
+        for (size_t beg = lo; beg < hi; beg += g_pin_bytes) {
+            if (in && beg > lo) {                          // the block is filled again: the last round has to have left it
+                const hipError_t e = hipStreamSynchronize(g_ctx.stream);
+                if (e != hipSuccess) return fail(what, e);
+            }
+            if (!round(in, what, h, pin, beg, std::min(hi, beg + g_pin_bytes))) return false;
+        }
+        return true;
+    }
+
+    // bytes beg .. end - 1 of the device block, through the pinned one
+    bool round(bool in, const char *what, Helpers *h, char *pin, size_t beg, size_t end) {
+        // the ends of the copies
+        size_t cut[MAX_SENDS];
+        int sends = 0;
+        for (size_t at = beg, c = SEND_MIN; at < end; sends++) {
+            if (in) {
+                at += c;
+                c = std::min(2 * c, SEND_MAX);
+            } else {
+                at += std::min(SEND_MAX, std::max(SEND_MIN, ((end - at) / 2 + 0xffff) & ~(size_t)0xffff));
+            }
+            if (at > end || sends + 1 == MAX_SENDS) at = end;
+            cut[sends] = at;
+        }
+        // the pieces, none across the end of a copy; last[s]: pieces up to the end of copy s
+        int pieces = 0, last[MAX_SENDS], s = 0;
+        for (int i = 0; i < n_; i++) {
+            if (!(in ? in_[i] : out_[i])) continue;
+            size_t at = std::max(p_[i].at, beg);
+            const size_t stop = std::min(p_[i].at + p_[i].bytes, end);
+            while (at < stop) {
+                while (at >= cut[s]) last[s++] = pieces;
+                const size_t n = std::min(std::min(stop, cut[s]) - at, PIECE);
+                h->done[pieces].store(0, std::memory_order_relaxed);
+                h->piece[pieces++] = Piece{&p_[i], at - p_[i].at, n, pin + (at - beg)};
+                at += n;
+            }
+        }
+        while (s < sends) last[s++] = pieces;
+        // no helper may still be looking at the round before
+        const unsigned long long number = (h->next.load(std::memory_order_relaxed) >> 32) + 1;
+        h->ready.store(0, std::memory_order_seq_cst);
+        h->in = in;
+        h->past = in || end - beg > (size_t)1 << 20;           // (small results stay in the caches for their reader)
+        h->next.store(number << 32, std::memory_order_seq_cst);
+        if (in) h->ready.store(pieces, std::memory_order_seq_cst);
+        if (pieces > 4 && h->n > 0) {
+            h->active.store(1);
+            h->calls.fetch_add(1);
+            if (h->asleep.load() > 0) {
+                pthread_mutex_lock(&h->lock);
+                pthread_cond_broadcast(&h->wake);
+                pthread_mutex_unlock(&h->lock);
+            }
+        }
+        hipError_t e = hipSuccess;
+        if (in) {
+            int ok = 0;
+            size_t from = beg;
+            for (s = 0; s < sends;) {
+                while (ok < pieces && h->done[ok].load(std::memory_order_acquire)) ok++;
+                if (ok >= last[s]) {
+                    e = stage_copy(dev_ + from, g_pin_dev + (from - beg), cut[s] - from);
+                    if (e != hipSuccess) break;
+                    from = cut[s++];
+                } else if (!one_piece(h)) {
+                    __builtin_ia32_pause();
+                }
+            }
+        } else {
+            size_t from = beg;
+            for (s = 0; s < sends && e == hipSuccess; s++) {
+                e = stage_copy(g_pin_dev + (from - beg), dev_ + from, cut[s] - from);
+                if (e == hipSuccess) e = hipEventRecord(g_sent[s], g_ctx.stream);
+                from = cut[s];
+            }
+            for (s = 0; s < sends && e == hipSuccess;) {
+                e = hipEventQuery(g_sent[s]);
+                if (e == hipSuccess) {
+                    h->ready.store(last[s++], std::memory_order_release);
+                } else if (e == hipErrorNotReady) {
+                    (void)hipGetLastError();
+                    e = hipSuccess;
+                    if (!one_piece(h)) __builtin_ia32_pause();
+                }
+            }
+        }
+        // what is left to take (after an error nothing more is), and then the pieces that helpers have taken
+        int taken = pieces;
+        if (e == hipSuccess) while (one_piece(h)) { }
+        else taken = std::min(pieces, (int)(h->next.exchange((number << 32) | 0x7fffffffu) & 0x7fffffffu));
+        for (int i = 0; i < taken; i++)
+            while (!h->done[i].load(std::memory_order_acquire)) __builtin_ia32_pause();
+        h->active.store(0);
+        return e == hipSuccess || fail(what, e);
+    }
+
+    // without pinned memory: each array by itself, through the runtime's staging
+    bool move_unpinned(bool in, const char *what) {
+        for (int i = 0; i < n_; i++) {
+            if (!(in ? in_[i] : out_[i])) continue;
+            const Part &p = p_[i];
+            const size_t step = p.rows ? p.row_bytes : p.bytes;
+            for (size_t r = 0; r * step < p.bytes; r++) {
+                char *host = p.host + (p.rows ? (size_t)p.rows[r] * step : 0), *dev = dev_ + p.at + r * step;
+                hipError_t e = in ? hipMemcpyAsync(dev, host, step, hipMemcpyHostToDevice, g_ctx.stream)
+                                  : hipMemcpyAsync(host, dev, step, hipMemcpyDeviceToHost, g_ctx.stream);
+                if (e == hipSuccess && !in) e = hipStreamSynchronize(g_ctx.stream);
+                if (e != hipSuccess) return fail(what, e);
+            }
+        }
+        return true;
+    }
+};
