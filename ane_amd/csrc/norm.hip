@@ -517,11 +517,9 @@ void launch_bwd_cluster_as(const ClusterPlan &cp, float *dx, float *part, const 
 template <bool RES>
 void launch_bwd_cluster(const ClusterPlan &cp, float *dx, float *part, const float *dy, const float *x, const float *w,
                         int C, int S, float eps, int variant, const float *res, float *dx2, float alpha2) {
-    // (with the residual's rows the unmasked variant would need more than the 128 registers a lane has)
-    if constexpr (!RES) {
-        if (cp.exact) { launch_bwd_cluster_as<false, true>(cp, dx, part, dy, x, w, C, S, eps, variant, res, dx2, alpha2); return; }
-    }
-    launch_bwd_cluster_as<RES, false>(cp, dx, part, dy, x, w, C, S, eps, variant, res, dx2, alpha2);
+    // (with the residual 126 of the 128 registers a lane has; [16][1024][256] 15.4 -> 14.7 us)
+    if (cp.exact) launch_bwd_cluster_as<RES, true>(cp, dx, part, dy, x, w, C, S, eps, variant, res, dx2, alpha2);
+    else launch_bwd_cluster_as<RES, false>(cp, dx, part, dy, x, w, C, S, eps, variant, res, dx2, alpha2);
 }
 
 }   // namespace

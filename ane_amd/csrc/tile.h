@@ -171,10 +171,14 @@ __device__ __forceinline__ typename RawT<VEC>::type raw_zero() {
 
 // Sum acc[q][j] over all threads of the block that share the same lane column (tid % LPR).
 // Every thread ends with the full per-column totals.  lds: NW*NV*LPR*VEC floats.
+// Across the waves a column is added up by one thread, and every thread then reads its totals: with every thread adding up its
+// own columns' waves, 32 reads of 16 bytes and 128 additions for the bfloat16 QK-norm backward on 512 threads, that kernel
+// took 3.5 us of its 26 for it ([16][24 x 128][256]).
 template <int VEC, int LPR, int THREADS, int NV>
 __device__ __forceinline__ void strip_reduce(float (&acc)[NV][VEC], float *lds) {
     constexpr int NW = THREADS / 64;
     constexpr int WLPR = LPR < 64 ? LPR : 64;
+    constexpr int TOTALS = NV * WLPR * VEC;
 #pragma unroll
     for (int q = 0; q < NV; q++)
 #pragma unroll
@@ -189,15 +193,17 @@ __device__ __forceinline__ void strip_reduce(float (&acc)[NV][VEC], float *lds) 
                 for (int j = 0; j < VEC; j++) lds[((wave * NV + q) * WLPR + lane) * VEC + j] = acc[q][j];
         }
         __syncthreads();
+        for (int i = threadIdx.x; i < TOTALS; i += THREADS) {
+            float s = 0.f;
+#pragma unroll
+            for (int wv = 0; wv < NW; wv++) s += lds[wv * TOTALS + i];
+            lds[i] = s;                     // (wave 0's place, which nobody else reads before the barrier)
+        }
+        __syncthreads();
 #pragma unroll
         for (int q = 0; q < NV; q++)
 #pragma unroll
-            for (int j = 0; j < VEC; j++) {
-                float s = 0.f;
-#pragma unroll
-                for (int wv = 0; wv < NW; wv++) s += lds[((wv * NV + q) * WLPR + (lc & (WLPR - 1))) * VEC + j];
-                acc[q][j] = s;
-            }
+            for (int j = 0; j < VEC; j++) acc[q][j] = lds[(q * WLPR + (lc & (WLPR - 1))) * VEC + j];
     }
 }
 

@@ -1,0 +1,79 @@
+"""QK-norm + RoPE and the RMSNorm backward with the residual where a tile is whole (every row pair of a head, every column of a
+strip) and one step beside it (one column more, a head size that leaves rows of the tile empty), fp32 and bfloat16."""
+import numpy as np
+import pytest
+
+import helpers as H
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def br():
+    import ane_amd.bridge as b
+    b.init()
+    return b
+
+
+def to_bf(x):
+    return O.cvt_f32_bf16(np.ascontiguousarray(x, np.float32)).reshape(x.shape)
+
+
+def widen(h):
+    return O.cvt_bf16_f32(np.ascontiguousarray(h)).reshape(h.shape)
+
+
+def err(a, r):
+    """Largest difference over the value, or over the root mean square where that is larger."""
+    r = r.astype(np.float64)
+    return float(np.max(np.abs(a - r) / np.maximum(np.abs(r), np.sqrt(np.mean(r * r)))))
+
+
+# hd 128 and 64 fill the tiles; batches beyond the line below which bfloat16 takes one column per lane
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("hd,heads,kv,B,S", [(128, 16, 8, 9, 128), (128, 16, 8, 5, 256), (128, 16, 8, 5, 257), (64, 12, 12, 14, 256), (64, 12, 12, 14, 255),
+                                             (96, 8, 8, 9, 256), (128, 3, 1, 2, 64)])
+def test_qknorm_rope_whole_and_ragged_tiles(br, hd, heads, kv, B, S, bf16):
+    print("[case] qk tiles hd=%d heads=%d kv=%d B=%d S=%d bf16=%d" % (hd, heads, kv, B, S, bf16), flush=True)
+    theta, eps = 1e6, 1e-5
+    end = "_bf16_dev" if bf16 else "_dev"
+    enc, dec = (to_bf, widen) if bf16 else (lambda a: np.array(a), lambda a: a)
+    D = br.DevArray.from_numpy
+    cos, sin = br.rope_tables_dev(S, hd, theta)
+    wq, wk = H.normal(960, hd, 1.0, 0.02), H.normal(961, hd, 1.0, 0.02)
+    q, k = enc(H.normal(962, (B, heads * hd, S))), enc(H.normal(963, (B, kv * hd, S)))
+    gq, gk = enc(H.normal(964, (B, heads * hd, S))), enc(H.normal(965, (B, kv * hd, S)))
+    qd, kd, gqd, gkd, wqd, wkd = (D(a) for a in (q, k, gq, gk, wq, wk))
+    qo, ko, dq, dk = (br.DevArray(a.shape, a.dtype) for a in (q, k, q, k))
+    dwq, dwk = br.DevArray(hd), br.DevArray(hd)
+    br.check(getattr(br.lib, "mi355_qknorm_rope_fwd" + end)(qo.ptr, ko.ptr, qd.ptr, kd.ptr, wqd.ptr, wkd.ptr, heads, kv, hd, S, B, cos, sin, eps))
+    br.check(getattr(br.lib, "mi355_qknorm_rope_bwd" + end)(dq.ptr, dk.ptr, dwq.ptr, dwk.ptr, gqd.ptr, gkd.ptr, qd.ptr, kd.ptr, wqd.ptr, wkd.ptr,
+                                                            heads, kv, hd, S, B, cos, sin, eps, 0))
+    # one rounding to 8 bits on store, relative to the value (2^-8); fp32: as the other QK-norm tests
+    tol, tol_w = (2.0 ** -8 * 1.01, 1e-5) if bf16 else (1e-5, 1e-5)
+    for x, g, w, out, dx, dw in ((q, gq, wq, qo, dq, dwq), (k, gk, wk, ko, dk, dwk)):
+        y = O.qknorm_rope_fwd(dec(x), w, hd, theta, eps)
+        rdx, rdw = O.qknorm_rope_bwd(dec(g), dec(x), w, hd, theta, eps)
+        assert err(dec(out.numpy()), y) <= tol
+        assert err(dec(dx.numpy()), rdx) <= tol
+        assert err(dw.numpy(), rdw) <= tol_w
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("C,S,B", [(1024, 256, 16), (1024, 128, 3), (1024, 255, 16), (512, 256, 4), (768, 256, 8)])
+def test_rmsnorm_bwd_residual_whole_and_ragged_tiles(br, C, S, B, bf16):
+    print("[case] rmsnorm_bwd_residual C=%d S=%d B=%d bf16=%d" % (C, S, B, bf16), flush=True)
+    end = "_bf16_dev" if bf16 else "_dev"
+    enc, dec = (to_bf, widen) if bf16 else (lambda a: np.array(a), lambda a: a)
+    x, dy, res = (enc(H.normal(970 + i, (B, C, S))) for i in range(3))
+    w = H.normal(973, C, 1.0, 0.02)
+    xd, dyd, rd, wd = (br.DevArray.from_numpy(a) for a in (x, dy, res, w))
+    dx, dx2, dw = br.DevArray(x.shape, x.dtype), br.DevArray(x.shape, x.dtype), br.DevArray(C)
+    br.check(getattr(br.lib, "mi355_rmsnorm_bwd_residual" + end)(dx.ptr, dx2.ptr, dw.ptr, dyd.ptr, xd.ptr, wd.ptr, rd.ptr, 0.25, C, S, B, 1e-5, 0))
+    rdx, rdw = O.rmsnorm_bwd(dec(dy), dec(x), w)
+    want = rdx.reshape(x.shape) + dec(res)
+    tol = 2.0 ** -8 * 1.01 if bf16 else 1e-5
+    assert err(dec(dx.numpy()), want) <= tol
+    assert err(dec(dx2.numpy()), want * np.float32(0.25)) <= tol
+    assert err(dw.numpy(), rdw) <= 1e-5
