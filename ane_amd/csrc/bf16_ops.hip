@@ -10,6 +10,7 @@
 #include "common.h"
 #include "tile.h"
 #include "norm_cluster.h"
+#include "rope.h"
 
 #include <math.h>
 
@@ -324,50 +325,6 @@ __device__ __forceinline__ void ldtab(float (&r)[VEC], const float *p) {
     } else {
         r[0] = *p;
     }
-}
-
-// one lane = one interleaved row pair of one head x VEC columns; Q pair rows first, then K
-template <int VEC>
-__global__ __launch_bounds__(BT) void rope_bf16_kernel(bf16_t *q_out, bf16_t *k_out, const bf16_t *q_in,
-                                                       const bf16_t *k_in, int heads, int /*kv_heads*/, int hd, int S,
-                                                       int batch, const float *__restrict__ cos_t,
-                                                       const float *__restrict__ sin_t, float sgn, size_t total) {
-    const size_t idx = (size_t)blockIdx.x * BT + threadIdx.x;
-    if (idx >= total) return;
-    const int cols = (S + VEC - 1) / VEC;
-    const int cg = (int)(idx % cols);
-    size_t pr = idx / cols;
-    const int half = hd >> 1;
-    const size_t q_rows = (size_t)batch * heads * half;
-    const bf16_t *in = q_in;
-    bf16_t *out = q_out;
-    if (pr >= q_rows) { pr -= q_rows; in = k_in; out = k_out; }
-    const int i = (int)(pr % half);
-    const size_t row = (pr / half) * hd + 2 * i;
-    const int s = cg * VEC;
-    const size_t o0 = row * S + s;
-    if (VEC > 1 && s + VEC > S) {        // the short last group of a row of any length
-        for (int j = 0; j < S - s; j++) {
-            const float a = bf_to_f(in[o0 + j]), b = bf_to_f(in[o0 + S + j]);
-            const float c = cos_t[(size_t)i * S + s + j], sj = sin_t[(size_t)i * S + s + j] * sgn;
-            out[o0 + j] = (bf16_t)f_to_bf(a * c - b * sj);
-            out[o0 + S + j] = (bf16_t)f_to_bf(a * sj + b * c);
-        }
-        return;
-    }
-    float v0[VEC], v1[VEC], c[VEC], sn[VEC], r0[VEC], r1[VEC];
-    ldb<VEC, true>(v0, in + o0);
-    ldb<VEC, true>(v1, in + o0 + S);
-    ldtab<VEC>(c, cos_t + (size_t)i * S + s);
-    ldtab<VEC>(sn, sin_t + (size_t)i * S + s);
-#pragma unroll
-    for (int j = 0; j < VEC; j++) {
-        const float sj = sn[j] * sgn;
-        r0[j] = v0[j] * c[j] - v1[j] * sj;
-        r1[j] = v0[j] * sj + v1[j] * c[j];
-    }
-    stb<VEC>(out + o0, r0);
-    stb<VEC>(out + o0 + S, r1);
 }
 
 // Products and sums of these two kernels that belong together are fused multiply-adds: a rounding fewer each, and a third fewer
@@ -944,9 +901,7 @@ MI355_API int mi355_rope_bf16_dev(uint16_t *q_out, uint16_t *k_out, const uint16
     if (!cos_dev || !sin_dev || (heads > 0 && (!q_out || !q_in)) || (kv_heads > 0 && (!k_out || !k_in)))
         return mi355_fail("rope_bf16: NULL pointer");
     if (dir != 1 && dir != -1) return mi355_fail("rope_bf16: dir must be +1 or -1");
-    const size_t pair_rows = (size_t)batch * (heads + kv_heads) * (hd / 2);
-    const size_t total = pair_rows * ceil_div((size_t)S, 8);
-    hipLaunchKernelGGL(rope_bf16_kernel<8>, dim3(blocks_for(total)), dim3(BT), 0, g_ctx.stream, q_out, k_out, q_in, k_in, heads, kv_heads, hd, S, batch, cos_dev, sin_dev, (float)dir, total);
+    launch_rope<bf16_t>(q_out, k_out, q_in, k_in, heads, kv_heads, hd, S, batch, cos_dev, sin_dev, dir);
     LAUNCH_OK("rope_bf16");
     return 0;
 }

@@ -5,6 +5,7 @@
 // 1 KiB run, UNROLL independent loads in flight per lane before the first use, and enough
 // workgroups (one pass, no grid-stride loop) to cover the 256 compute units many times over.
 #include "common.h"
+#include "rope.h"
 
 #include <math.h>
 
@@ -139,54 +140,6 @@ __global__ void axpby_scalar(float *y, const float *a, const float *b, float alp
         if (MODE == 0) y[i] = b[i] * alpha + a[i];
         else if (MODE == 1) y[i] = a[i] * alpha;
         else y[i] = a[i] + b[i];
-    }
-}
-
-// ---- RoPE on interleaved row pairs; one thread = one pair of rows x 4 columns ----
-// rows: all (batch, head, pair) triples of Q then of K; tables [hd/2][S].
-__global__ __launch_bounds__(EW_THREADS) void rope_kernel(float *q_out, float *k_out, const float *q_in,
-                                                          const float *k_in, int heads, int /*kv_heads*/, int hd, int S,
-                                                          int batch, const float *__restrict__ cos_t,
-                                                          const float *__restrict__ sin_t, float sgn, size_t total) {
-    const int cols = (S + 3) / 4;   // column groups per row
-    const size_t idx = (size_t)blockIdx.x * EW_THREADS + threadIdx.x;
-    if (idx >= total) return;
-    const int cg = (int)(idx % cols);
-    size_t pr = idx / cols;   // pair-row index
-    const int half = hd >> 1;
-    const size_t q_rows = (size_t)batch * heads * half;
-    const float *in;
-    float *out;
-    int i;
-    size_t row;
-    if (pr < q_rows) {
-        i = (int)(pr % half);
-        row = (pr / half) * hd + 2 * i;   // (b*heads + h)*hd + 2i
-        in = q_in; out = q_out;
-    } else {
-        pr -= q_rows;
-        i = (int)(pr % half);
-        row = (pr / half) * hd + 2 * i;
-        in = k_in; out = k_out;
-    }
-    const int s = cg * 4;
-    const size_t o0 = row * S + s, o1 = o0 + S;
-    const size_t t = (size_t)i * S + s;
-    if (s + 4 <= S) {
-        v4f v0 = ld4(in + o0), v1 = ld4(in + o1);
-        v4f c = ld4(cos_t + t), sn = ld4(sin_t + t) * sgn;
-        // forward (sgn=+1): x0*c - x1*s, x0*s + x1*c ; backward (sgn=-1): x0*c + x1*s, -x0*s + x1*c
-        v4f r0 = v0 * c - v1 * sn;
-        v4f r1 = v0 * sn + v1 * c;
-        st4(out + o0, r0);
-        st4(out + o1, r1);
-    } else {                                // the short last group of a row of any length
-        for (int j = 0; j < S - s; j++) {
-            const float v0 = in[o0 + j], v1 = in[o1 + j];
-            const float c = cos_t[t + j], sn = sin_t[t + j] * sgn;
-            out[o0 + j] = v0 * c - v1 * sn;
-            out[o1 + j] = v0 * sn + v1 * c;
-        }
     }
 }
 
@@ -781,9 +734,7 @@ MI355_API int mi355_rope_dev(float *q_out, float *k_out, const float *q_in, cons
         return mi355_fail("rope: bad shape heads=%d kv_heads=%d hd=%d S=%d batch=%d", heads, kv_heads, hd, S, batch);
     if ((heads > 0 && (!q_out || !q_in)) || (kv_heads > 0 && (!k_out || !k_in))) return mi355_fail("rope: NULL pointer");
     if (dir != 1 && dir != -1) return mi355_fail("rope: dir must be +1 or -1");
-    const size_t total = (size_t)batch * (heads + kv_heads) * (hd / 2) * ceil_div((size_t)S, 4);
-    hipLaunchKernelGGL(rope_kernel, dim3((unsigned)ceil_div(total, EW_THREADS)), dim3(EW_THREADS), 0, g_ctx.stream, q_out,
-                       k_out, q_in, k_in, heads, kv_heads, hd, S, batch, cos_dev, sin_dev, (float)dir, total);
+    launch_rope<float>(q_out, k_out, q_in, k_in, heads, kv_heads, hd, S, batch, cos_dev, sin_dev, dir);
     LAUNCH_OK("rope");
     return 0;
 }
