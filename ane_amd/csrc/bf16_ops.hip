@@ -134,7 +134,7 @@ __global__ __launch_bounds__(THREADS) void rms_fwd_bf16_kernel(bf16_t *__restric
         for (int k = 0; k < CAP; k++) {
             const int c = row0 + k * RPS;
             const bool ok = c < C && col_ok;
-            xr[k] = ok ? ld_raw<VEC, true>(x + base + (size_t)c * S) : raw_zero<VEC>();
+            xr[k] = ok ? ld_raw<VEC, false>(x + base + (size_t)c * S) : raw_zero<VEC>();
             wv[k] = ok ? w[c] : 0.f;
         }
 #pragma unroll
@@ -246,8 +246,8 @@ __global__ __launch_bounds__(THREADS) void rms_bwd_bf16_kernel(bf16_t *dx, float
         for (int k = 0; k < CAP; k++) {
             const int c = row0 + k * RPS;
             const bool ok = c < C && col_ok;
-            xr[k] = ok ? ld_raw<VEC, true>(x + base + (size_t)c * S) : raw_zero<VEC>();
-            dr[k] = ok ? ld_raw<VEC, true>(dy + base + (size_t)c * S) : raw_zero<VEC>();
+            xr[k] = ok ? ld_raw<VEC, false>(x + base + (size_t)c * S) : raw_zero<VEC>();
+            dr[k] = ok ? ld_raw<VEC, false>(dy + base + (size_t)c * S) : raw_zero<VEC>();
             wv[k] = ok ? w[c] : 0.f;
         }
 #pragma unroll
@@ -329,9 +329,14 @@ __device__ __forceinline__ void ldtab(float (&r)[VEC], const float *p) {
 
 // Products and sums of these two kernels that belong together are fused multiply-adds: a rounding fewer each, and a third fewer
 // vector instructions (backward of [16][24 x 128][256] 26.7 -> 25.7 us).
-// EXACT: the tile holds every row pair of the head and nothing else, and every strip is whole.  Then no load or store is behind
-// a condition (forward 12.0 -> 10.4 us, backward 22.9 -> 20.0).
-template <int VEC, int LPR, int THREADS, int CAP, bool EXACT>
+enum { QK_SOME, QK_ROWS, QK_ALL };
+// WHOLE = QK_ALL: the tile holds every row pair of the head and nothing else, and every strip is whole.  Then no load or store is
+// behind a condition (forward 12.0 -> 10.4 us, backward 22.9 -> 20.0).  QK_ROWS: the same but for the columns; lanes past the end
+// of a row load its last columns again, and only the stores are conditional ([22][24 x 128][147] forward 18.1 -> 15.6, backward
+// 28.0 -> 24.3; [5][570] 13.0 -> 12.1 and 21.8 -> 17.6).
+// Loads leave a row's lines in the caches: rows of any length ask for most lines twice ([22][24 x 128][147] 21.5 -> 18.1 and
+// 32.7 -> 28.9 us), and whole lines come no faster past them ([16][24 x 128][256] 10.0 either way, 18.7 -> 16.7).
+template <int VEC, int LPR, int THREADS, int CAP, int WHOLE>
 __global__ __launch_bounds__(THREADS) void qknorm_rope_fwd_bf16_kernel(
     bf16_t *__restrict__ q_out, bf16_t *__restrict__ k_out, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k,
     const float *__restrict__ wq, const float *__restrict__ wk, int hd, int S, int strips, int nq,
@@ -346,7 +351,8 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_fwd_bf16_kernel(
     if (blk >= nq) { blk -= nq; in = k; out = k_out; w = wk; }
     const int slab = blk / strips, strip = blk - slab * strips;
     const int lc = threadIdx.x % LPR, p0 = threadIdx.x / LPR;
-    const LaneCols mine = lane_cols<VEC>((strip * LPR + lc) * VEC, S);
+    const int nominal = (strip * LPR + lc) * VEC;
+    const LaneCols mine = WHOLE == QK_ROWS ? lane_cols_inside<VEC, LPR * VEC>(nominal, S) : lane_cols<VEC>(nominal, S);
     const int col = mine.col;
     const bool col_ok = mine.ok;
     const int half = hd >> 1;
@@ -359,9 +365,9 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_fwd_bf16_kernel(
 #pragma unroll
     for (int kk = 0; kk < CAP; kk++) {
         const int rp = p0 + kk * PPS;
-        const bool ok = EXACT || (rp < half && col_ok);
-        r0[kk] = ok ? ld_raw<VEC, true>(in + base + (size_t)(2 * rp) * S) : raw_zero<VEC>();
-        r1[kk] = ok ? ld_raw<VEC, true>(in + base + (size_t)(2 * rp + 1) * S) : raw_zero<VEC>();
+        const bool ok = WHOLE || (rp < half && col_ok);
+        r0[kk] = ok ? ld_raw<VEC, false>(in + base + (size_t)(2 * rp) * S) : raw_zero<VEC>();
+        r1[kk] = ok ? ld_raw<VEC, false>(in + base + (size_t)(2 * rp + 1) * S) : raw_zero<VEC>();
         w0[kk] = ok ? w[2 * rp] : 0.f;
         w1[kk] = ok ? w[2 * rp + 1] : 0.f;
         float x0[VEC], x1[VEC];
@@ -382,7 +388,7 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_fwd_bf16_kernel(
 #pragma unroll
     for (int kk = 0; kk < CAP; kk++) {
         const int rp = p0 + kk * PPS;
-        if (EXACT || (rp < half && col_ok)) {
+        if (WHOLE || (rp < half && col_ok)) {
             float x0[VEC], x1[VEC], cs[VEC], sn[VEC], o0[VEC], o1[VEC];
             unpack<VEC>(x0, r0[kk]);
             unpack<VEC>(x1, r1[kk]);
@@ -394,15 +400,17 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_fwd_bf16_kernel(
                 o0[j] = __builtin_fmaf(y0, cs[j], -(y1 * sn[j]));
                 o1[j] = __builtin_fmaf(y0, sn[j], y1 * cs[j]);
             }
-            stb<VEC>(out + base + (size_t)(2 * rp) * S, o0);
-            stb<VEC>(out + base + (size_t)(2 * rp + 1) * S, o1);
+            if (WHOLE != QK_ROWS || col_ok) {
+                stb<VEC>(out + base + (size_t)(2 * rp) * S, o0);
+                stb<VEC>(out + base + (size_t)(2 * rp + 1) * S, o1);
+            }
         }
     }
 }
 
 // Where a lane has one or two row pairs it keeps their un-rotated gradients across the reduction, in place of the packed upstream
-// ones: the table is read once and the rotation undone once (24.2 -> 22.9 us; with whole tiles 22.0 -> 20.0, 123 registers).
-template <int VEC, int LPR, int THREADS, int CAP, bool EXACT>
+// ones: the table is read once and the rotation undone once (24.2 -> 22.9 us; with whole tiles 22.0 -> 20.0, with loads through the caches 16.7; 123 registers).
+template <int VEC, int LPR, int THREADS, int CAP, int WHOLE>
 __global__ __launch_bounds__(THREADS) void qknorm_rope_bwd_bf16_kernel(
     bf16_t *dq, bf16_t *dk, float *__restrict__ part, const bf16_t *dq_out, const bf16_t *dk_out,
     const bf16_t *__restrict__ q, const bf16_t *__restrict__ k, const float *__restrict__ wq,
@@ -420,7 +428,8 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_bwd_bf16_kernel(
     if (blk >= nq) { blk -= nq; gin = dk_out; xin = k; out = dk; w = wk; }
     const int slab = blk / strips, strip = blk - slab * strips;
     const int lc = threadIdx.x % LPR, p0 = threadIdx.x / LPR;
-    const LaneCols mine = lane_cols<VEC>((strip * LPR + lc) * VEC, S);
+    const int nominal = (strip * LPR + lc) * VEC;
+    const LaneCols mine = WHOLE == QK_ROWS ? lane_cols_inside<VEC, LPR * VEC>(nominal, S) : lane_cols<VEC>(nominal, S);
     const int col = mine.col;
     const bool col_ok = mine.ok;
     const int half = hd >> 1;
@@ -440,7 +449,7 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_bwd_bf16_kernel(
         unpack<VEC>(g1, rg1[kk]);
         // (from a valid address in every lane: with the loads under a branch the compiler merges the two paths through
         // scratch memory, and a kernel with scratch is dispatched later; a masked lane's gradients are zero)
-        const size_t to = EXACT || (rp < half && col_ok) ? (size_t)rp * S + col : 0;
+        const size_t to = WHOLE || (rp < half && col_ok) ? (size_t)rp * S + col : 0;
         ldtab<VEC>(c, cos_t + to);
         ldtab<VEC>(sn, sin_t + to);
 #pragma unroll
@@ -453,12 +462,12 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_bwd_bf16_kernel(
 #pragma unroll
     for (int kk = 0; kk < CAP; kk++) {
         const int rp = p0 + kk * PPS;
-        const bool ok = EXACT || (rp < half && col_ok);
+        const bool ok = WHOLE || (rp < half && col_ok);
         const size_t o = base + (size_t)(2 * rp) * S;
-        rx0[kk] = ok ? ld_raw<VEC, true>(xin + o) : raw_zero<VEC>();
-        rx1[kk] = ok ? ld_raw<VEC, true>(xin + o + S) : raw_zero<VEC>();
-        rg0[kk] = ok ? ld_raw<VEC, true>(gin + o) : raw_zero<VEC>();
-        rg1[kk] = ok ? ld_raw<VEC, true>(gin + o + S) : raw_zero<VEC>();
+        rx0[kk] = ok ? ld_raw<VEC, false>(xin + o) : raw_zero<VEC>();
+        rx1[kk] = ok ? ld_raw<VEC, false>(xin + o + S) : raw_zero<VEC>();
+        rg0[kk] = ok ? ld_raw<VEC, false>(gin + o) : raw_zero<VEC>();
+        rg1[kk] = ok ? ld_raw<VEC, false>(gin + o + S) : raw_zero<VEC>();
         w0[kk] = ok ? w[2 * rp] : 0.f;
         w1[kk] = ok ? w[2 * rp + 1] : 0.f;
         float x0[VEC], x1[VEC], d0[VEC], d1[VEC];
@@ -489,7 +498,7 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_bwd_bf16_kernel(
 #pragma unroll
     for (int kk = 0; kk < CAP; kk++) {
         const int rp = p0 + kk * PPS;
-        if (EXACT || rp < half) {   // uniform over each group of LPR lanes
+        if (WHOLE || rp < half) {   // uniform over each group of LPR lanes
             float x0[VEC], x1[VEC], d0[VEC], d1[VEC], o0[VEC], o1[VEC];
             unpack<VEC>(x0, rx0[kk]);
             unpack<VEC>(x1, rx1[kk]);
@@ -500,7 +509,7 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_bwd_bf16_kernel(
                 unrotate(kk, rp, d0, d1);
             }
             float s0 = 0.f, s1 = 0.f;
-            if constexpr (EXACT) {
+            if constexpr (WHOLE == QK_ALL) {
 #pragma unroll
                 for (int j = 0; j < VEC; j++) {
                     s0 = __builtin_fmaf(d0[j] * x0[j], rr[j], s0);
@@ -520,7 +529,7 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_bwd_bf16_kernel(
                     o1[j] = (d1[j] * w1[kk]) * rr[j] - (x1[j] * dotn[j]) * rr[j];
                 }
             }
-            if (EXACT || col_ok) {
+            if (WHOLE == QK_ALL || col_ok) {
                 stb<VEC>(out + base + (size_t)(2 * rp) * S, o0);
                 stb<VEC>(out + base + (size_t)(2 * rp + 1) * S, o1);
             }
@@ -540,22 +549,23 @@ struct QkBf {
 
 // The tile for `slabs` head slabs of [hd][S].  Small tensors take one column per lane on 1024 threads: with few strips to
 // go round, waves count for more than bytes per access.  us, one column per lane / eight:
-//   hd 128, 24 heads   fwd  [1][257] 5.0 / 9.8   [4][257] 7.4 / 9.5    [8][257] 12.0 / 11.8   [8][500] 18.2 / 15.1
-//                      bwd       9.7 / 13.7          15.7 / 16.0            25.9 / 23.1            39.0 / 31.5
-//   hd 64, 24 heads    fwd  [4][197] 5.2 / 6.6   [8][197] 7.3 / 7.6    [16][197] 12.1 / 9.5
-//                      bwd      11.1 / 12.6          15.0 / 13.6             25.4 / 17.1
-// The line lies between [8][197] and [8][250] of hd 64 and between [4][257] and [8][129] of hd 128; shorter heads leave the
-// 64 pairs of the former mostly empty (hd 32 fwd [4][257] 5.0 / 6.2, [16][77] 5.9 / 5.1).  Eight columns per lane:
+//   hd 128, 24 heads   fwd  [1][257] 4.5 / 6.0   [4][197] 6.5 / 6.0    [4][257] 6.6 / 7.5     [8][147] 9.0 / 7.5   [8][257] 11.8 / 9.8
+//                      bwd       9.2 / 9.4           12.4 / 9.9            13.5 / 13.0            16.6 / 12.8          23.2 / 18.6
+//   hd 64, 24 heads    fwd  [4][257] 5.1 / 5.8   [8][147] 6.4 / 5.7    [8][257] 7.9 / 6.5
+//                      bwd       10.0 / 9.8          12.0 / 9.8            14.8 / 11.5
+// The line lies between [8][197] and [8][250] of hd 64; of hd 128 between [4][257] and [8][129], and below [4][197] where strips
+// of 128 columns are at least three quarters full; shorter heads leave the 64 pairs of the former mostly empty (hd 32 fwd [4][257]
+// 5.0 / 6.2, [16][77] 5.9 / 5.1).  Eight columns per lane:
 // 16 lanes to a row, with two row pairs per lane where that takes 256 or 512 threads (hd 128 forward on 256 threads with
-// four pairs: [8][257] 14.6 for 11.8; hd 64 backward on 512 with one: [8][257] 25.7 for 16.2); 8 lanes where 16 would leave
-// most of a strip empty (rows of up to 64 columns: fwd hd 128 [32][33] 8.0 for 10.0; in the backward of long heads from a
-// sixth on: [8][257] 23.1 for 28.8, [16][197] 37.3 for 30.6).
+// four pairs: [8][257] 14.6 for 11.8; hd 64 backward on 512 with one: [8][257] 25.7 for 16.2); 8 lanes for rows of up to 64
+// columns, where 16 would leave half a strip empty (fwd hd 128 [32][33] 8.0 for 10.0).  For longer rows 16 even where the last
+// strip holds one column: backward of hd 128 [20][130] 21.4 for 26.0, [12][257] 24.1 for 27.6, forward 14.9 for 19.4.
 // Rows of fewer than eight columns, and in-place calls whose short last group of columns would be shared by two workgroups,
 // have no choice; a lane of one column holds at most four pairs, one of eight columns what fits 16, 8 or 4 lanes.
 bool pick_qk_bf(int hd, int S, size_t slabs, bool in_place, bool backward, QkBf &cfg) {
     const int half = hd / 2;
-    const bool small = slabs * hd * S < (half <= 16 ? 800000u : half <= 32 ? 2500000u : 3200000u);
-    const auto padded = [S](int w) { return (S + w - 1) / w * w; };
+    const bool full = (S + 127) / 128 * 128 * 3 <= S * 4;          // strips, on average
+    const bool small = slabs * hd * S < (half <= 16 ? 800000u : half <= 32 ? 2500000u : full ? 2200000u : 3200000u);
     auto fits = [&](int lpr, int threads) {
         for (int cap : {1, 2, 4}) {
             cfg = QkBf{8, lpr, threads, cap};
@@ -564,7 +574,7 @@ bool pick_qk_bf(int hd, int S, size_t slabs, bool in_place, bool backward, QkBf 
         return false;
     };
     if (S >= 8 && half <= 64 && !small) {
-        const bool narrow = S <= 64 || (backward && half > 32 && 5 * padded(128) >= 6 * padded(64));
+        const bool narrow = S <= 64;
         if (fits(narrow ? 8 : 16, narrow || half <= 32 ? 256 : 512)) return true;
     }
     if (S >= 8 && (half > 64 || !small)) {              // long heads, and in-place calls for which that strip is too narrow
@@ -578,15 +588,17 @@ bool pick_qk_bf(int hd, int S, size_t slabs, bool in_place, bool backward, QkBf 
 
 #define QKBF_CASE(KERNEL, V, L, T, CP, grid, ...)                                                                    \
     case (V) * 1000000 + (L) * 10000 + ((T) / 256) * 100 + (CP):                                                     \
-        hipLaunchKernelGGL((KERNEL<V, L, T, CP, false>), grid, dim3(T), 0, g_ctx.stream, __VA_ARGS__);               \
+        hipLaunchKernelGGL((KERNEL<V, L, T, CP, QK_SOME>), grid, dim3(T), 0, g_ctx.stream, __VA_ARGS__);             \
         break;
-// tiles that a head size of 64 or 128 fills
+// tiles that a head size of 64 or 128 fills (more than one column per lane: QK_ROWS needs rows of a whole group)
 #define QKBF_CASE_EXACT(KERNEL, V, L, T, CP, grid, ...)                                                              \
     case (V) * 1000000 + (L) * 10000 + ((T) / 256) * 100 + (CP):                                                     \
         if ((T) / (L) * (CP) == hd / 2 && S % ((L) * (V)) == 0)                                                      \
-            hipLaunchKernelGGL((KERNEL<V, L, T, CP, true>), grid, dim3(T), 0, g_ctx.stream, __VA_ARGS__);            \
+            hipLaunchKernelGGL((KERNEL<V, L, T, CP, QK_ALL>), grid, dim3(T), 0, g_ctx.stream, __VA_ARGS__);          \
+        else if ((T) / (L) * (CP) == hd / 2)                                                                         \
+            hipLaunchKernelGGL((KERNEL<V, L, T, CP, QK_ROWS>), grid, dim3(T), 0, g_ctx.stream, __VA_ARGS__);         \
         else                                                                                                         \
-            hipLaunchKernelGGL((KERNEL<V, L, T, CP, false>), grid, dim3(T), 0, g_ctx.stream, __VA_ARGS__);           \
+            hipLaunchKernelGGL((KERNEL<V, L, T, CP, QK_SOME>), grid, dim3(T), 0, g_ctx.stream, __VA_ARGS__);         \
         break;
 #define QKBF_DISPATCH(KERNEL, cfg, grid, ...)                                                                        \
     do {                                                                                                             \
@@ -595,7 +607,7 @@ bool pick_qk_bf(int hd, int S, size_t slabs, bool in_place, bool backward, QkBf 
             QKBF_CASE(KERNEL, 8, 16, 256, 1, grid, __VA_ARGS__) QKBF_CASE_EXACT(KERNEL, 8, 16, 256, 2, grid, __VA_ARGS__)  \
             QKBF_CASE(KERNEL, 8, 16, 256, 4, grid, __VA_ARGS__) QKBF_CASE(KERNEL, 8, 16, 512, 1, grid, __VA_ARGS__)  \
             QKBF_CASE_EXACT(KERNEL, 8, 16, 512, 2, grid, __VA_ARGS__) QKBF_CASE(KERNEL, 8, 16, 512, 4, grid, __VA_ARGS__)  \
-            QKBF_CASE(KERNEL, 8, 8, 256, 1, grid, __VA_ARGS__) QKBF_CASE(KERNEL, 8, 8, 256, 2, grid, __VA_ARGS__)    \
+            QKBF_CASE(KERNEL, 8, 8, 256, 1, grid, __VA_ARGS__) QKBF_CASE_EXACT(KERNEL, 8, 8, 256, 2, grid, __VA_ARGS__)    \
             QKBF_CASE(KERNEL, 8, 8, 256, 4, grid, __VA_ARGS__) QKBF_CASE(KERNEL, 8, 8, 512, 1, grid, __VA_ARGS__)    \
             QKBF_CASE(KERNEL, 8, 8, 512, 2, grid, __VA_ARGS__) QKBF_CASE(KERNEL, 8, 8, 512, 4, grid, __VA_ARGS__)    \
             QKBF_CASE(KERNEL, 8, 4, 256, 1, grid, __VA_ARGS__) QKBF_CASE(KERNEL, 8, 4, 256, 2, grid, __VA_ARGS__)    \

@@ -48,7 +48,7 @@ __global__ __launch_bounds__(THREADS) void rms_fwd_kernel(float *__restrict__ y,
         for (int k = 0; k < CAP; k++) {
             const int c = row0 + k * RPS;
             if (c < C && col_ok) {
-                ldv_nt<VEC>(xv[k], xs + (size_t)c * S);
+                ldv<VEC>(xv[k], xs + (size_t)c * S);
                 wv[k] = w[c];
             } else {
 #pragma unroll
@@ -165,9 +165,9 @@ __device__ __forceinline__ void rms_bwd_body(float *dx, float *__restrict__ dw_p
         for (int k = 0; k < CAP; k++) {
             const int c = row0 + k * RPS;
             if (c < C && col_ok) {
-                ldv_nt<VEC>(xv[k], xs + (size_t)c * S);
-                ldv_nt<VEC>(dv[k], dys + (size_t)c * S);
-                if constexpr (RES) ldv_nt<VEC>(rv[k], ress + (size_t)c * S);
+                ldv<VEC>(xv[k], xs + (size_t)c * S);
+                ldv<VEC>(dv[k], dys + (size_t)c * S);
+                if constexpr (RES) ldv<VEC>(rv[k], ress + (size_t)c * S);
                 wv[k] = w[c];
             } else {
 #pragma unroll
@@ -278,8 +278,8 @@ __global__ __launch_bounds__(THREADS) void res_rms_fwd_kernel(float *y, float *_
             const int c = row0 + k * RPS;
             if (c < C && col_ok) {
                 float bv[VEC];
-                ldv_nt<VEC>(yv[k], a + base + (size_t)c * S);
-                ldv_nt<VEC>(bv, b + base + (size_t)c * S);
+                ldv<VEC>(yv[k], a + base + (size_t)c * S);
+                ldv<VEC>(bv, b + base + (size_t)c * S);
 #pragma unroll
                 for (int j = 0; j < VEC; j++) yv[k][j] = bv[j] * alpha + yv[k][j];
                 wv[k] = w[c];

@@ -74,6 +74,16 @@ struct StoreBf16 {
 };
 static_assert(CL_SLOT_STRIDE >= 2 * CL_LPR * StoreBf16::VEC, "two quantities per column must fit a workgroup's slots");
 
+// The first read of an operand's rows.  A cache line that holds the end of one row piece and the start of another is asked for
+// twice, and again by the workgroup of the next strip, so the loads leave it in the caches: nontemporal ones took, for the
+// backward of fp32 [22][1024][147] and [115][768][54], 18.5 and 27.3 us for 15.2 and 21.7, of bfloat16 [8][768][197] 10.8 for
+// 10.0, and of fp32 [16][1024][256], where pieces are whole lines, no less either (11.7, 11.6).  Whole pieces of bfloat16 alone
+// are read past the caches ([16][1024][256] 12.8 for 13.2 us, forward 7.1 for 7.2).
+template <typename ST, bool EXACT>
+__device__ __forceinline__ typename ST::Raw cluster_load(const typename ST::T *p) {
+    return EXACT && sizeof(typename ST::T) == 2 ? ST::load_nt(p) : ST::load(p);
+}
+
 // Per-thread partial sums acc[q][j] (q < NV quantities, j < VEC columns of this lane) -> per-column sums of the
 // workgroup in wsum[q*W + column], valid for all threads after the barrier.  lds: NW*NV*W floats.
 template <int THREADS, int NV, int VEC>
@@ -177,7 +187,9 @@ __device__ __forceinline__ ClusterGeo cluster_geo(int nblk, int csplit, int stri
 // RMSNorm that follows it (training/training_dynamic/train.m:460-461).  Otherwise x = a and b, y_res are unused.
 // EXACT: every member holds exactly RPS*RPT rows and every strip is whole.  Then no row or column needs a mask and
 // the loads of the tile are issued back to back without branches, which is worth 0.45 us of the 8 us that the
-// forward kernel takes on fp32 [16][1024][256]; other shapes take the masked loads.
+// forward kernel takes on fp32 [16][1024][256].  In other shapes lanes without a row or without columns load valid ones and
+// only their values are dropped, which is still quicker than branches: bfloat16 [5][1024][570] forward 8.0 -> 7.6, with the
+// residual 10.7 -> 10.4, backward 12.2 -> 12.0, with it 14.0 -> 13.7; fp32 [115][768][54] with the residual 21.2 -> 20.1.
 template <typename ST, int RPT, int THREADS, bool FUSE, bool EXACT>
 __global__ __launch_bounds__(THREADS) void rms_fwd_cluster_kernel(typename ST::T *__restrict__ yn, typename ST::T *y_res,
                                                                   const typename ST::T *a, const typename ST::T *b,
@@ -195,7 +207,7 @@ __global__ __launch_bounds__(THREADS) void rms_fwd_cluster_kernel(typename ST::T
     __shared__ int failed;
     const ClusterGeo g = cluster_geo(nblk, csplit, strips);
     const int lc = threadIdx.x % CL_LPR, row0 = threadIdx.x / CL_LPR;
-    const LaneCols mine = lane_cols<VEC>(g.strip * W + lc * VEC, S);
+    const LaneCols mine = lane_cols_inside<VEC, W>(g.strip * W + lc * VEC, S);
     const int col = mine.col;
     const bool col_ok = mine.ok;
     const size_t slab_base = (size_t)g.slab * C * S + col;
@@ -205,19 +217,20 @@ __global__ __launch_bounds__(THREADS) void rms_fwd_cluster_kernel(typename ST::T
 
     // rows of member m held by this thread: c = m*rows_pm + row0 + k*RPS, valid while below (m+1)*rows_pm and C
     auto row_of = [&](int m, int k) { return m * rows_pm + row0 + k * RPS; };
-    auto row_ok = [&](int m, int k) { return row0 + k * RPS < rows_pm && row_of(m, k) < C && col_ok; };
+    auto row_live = [&](int m, int k) { return row0 + k * RPS < rows_pm && row_of(m, k) < C; };
+    auto row_ok = [&](int m, int k) { return row_live(m, k) && col_ok; };
     // one row piece of x (FUSE: of y = a + alpha*b, rounded to the storage type as the stored y is)
-    auto load_row = [&](int c, bool streaming) -> typename ST::Raw {
+    auto load_row = [&](int c, bool first) -> typename ST::Raw {
         const size_t off = slab_base + (size_t)c * S;
         if constexpr (FUSE) {
             float av[VEC], bv[VEC], v[VEC];
-            ST::widen(av, streaming ? ST::load_nt(a + off) : ST::load(a + off));
-            ST::widen(bv, streaming ? ST::load_nt(b + off) : ST::load(b + off));
+            ST::widen(av, first ? cluster_load<ST, EXACT>(a + off) : ST::load(a + off));
+            ST::widen(bv, first ? cluster_load<ST, EXACT>(b + off) : ST::load(b + off));
 #pragma unroll
             for (int j = 0; j < VEC; j++) v[j] = bv[j] * alpha + av[j];
             return ST::pack(v);
         } else {
-            return streaming ? ST::load_nt(a + off) : ST::load(a + off);
+            return first ? cluster_load<ST, EXACT>(a + off) : ST::load(a + off);
         }
     };
 
@@ -225,13 +238,11 @@ __global__ __launch_bounds__(THREADS) void rms_fwd_cluster_kernel(typename ST::T
     float wv[RPT];
 #pragma unroll
     for (int k = 0; k < RPT; k++) {
-        if (EXACT || row_ok(g.member, k)) {
-            xr[k] = load_row(row_of(g.member, k), true);
-            wv[k] = w[row_of(g.member, k)];
-        } else {
-            xr[k] = ST::zero();
-            wv[k] = 0.f;
-        }
+        const bool live = EXACT || row_live(g.member, k);
+        const int c = live ? row_of(g.member, k) : 0;
+        xr[k] = load_row(c, true);
+        wv[k] = w[c];
+        if (!live) xr[k] = ST::zero();
     }
     float acc[1][VEC];
 #pragma unroll
@@ -313,7 +324,7 @@ __global__ __launch_bounds__(THREADS) void rms_bwd_cluster_kernel(typename ST::T
     __shared__ int failed;
     const ClusterGeo g = cluster_geo(nblk, csplit, strips);
     const int lc = threadIdx.x % CL_LPR, row0 = threadIdx.x / CL_LPR;
-    const LaneCols mine = lane_cols<VEC>(g.strip * W + lc * VEC, S);
+    const LaneCols mine = lane_cols_inside<VEC, W>(g.strip * W + lc * VEC, S);
     const int col = mine.col;
     const bool col_ok = mine.ok;
     const size_t slab_base = (size_t)g.slab * C * S + col;
@@ -322,23 +333,21 @@ __global__ __launch_bounds__(THREADS) void rms_bwd_cluster_kernel(typename ST::T
     cluster_tags<THREADS, 2, VEC>(my_tag, want_tag, g.blk, g.cluster, csplit, ws);
 
     auto row_of = [&](int m, int k) { return m * rows_pm + row0 + k * RPS; };
-    auto row_ok = [&](int m, int k) { return row0 + k * RPS < rows_pm && row_of(m, k) < C && col_ok; };
+    auto row_live = [&](int m, int k) { return row0 + k * RPS < rows_pm && row_of(m, k) < C; };
+    auto row_ok = [&](int m, int k) { return row_live(m, k) && col_ok; };
 
     typename ST::Raw xr[RPT], dr[RPT], rr_res[RES ? RPT : 1];
     float wv[RPT];
 #pragma unroll
     for (int k = 0; k < RPT; k++) {
-        if (EXACT || row_ok(g.member, k)) {
-            const size_t off = slab_base + (size_t)row_of(g.member, k) * S;
-            xr[k] = ST::load_nt(x + off);
-            dr[k] = ST::load_nt(dy + off);
-            if constexpr (RES) rr_res[k] = ST::load_nt(res + off);
-            wv[k] = w[row_of(g.member, k)];
-        } else {
-            xr[k] = dr[k] = ST::zero();
-            if constexpr (RES) rr_res[k] = ST::zero();
-            wv[k] = 0.f;
-        }
+        const bool live = EXACT || row_live(g.member, k);
+        const int c = live ? row_of(g.member, k) : 0;
+        const size_t off = slab_base + (size_t)c * S;
+        xr[k] = cluster_load<ST, EXACT>(x + off);
+        dr[k] = cluster_load<ST, EXACT>(dy + off);
+        if constexpr (RES) rr_res[k] = cluster_load<ST, EXACT>(res + off);
+        wv[k] = w[c];
+        if (!live) xr[k] = ST::zero();
     }
     float acc[2][VEC];      // [0] = sum x^2, [1] = sum (dy*x)*w
 #pragma unroll

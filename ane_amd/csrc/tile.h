@@ -76,6 +76,17 @@ __device__ __forceinline__ LaneCols lane_cols(int nominal, int S) {
     l.ragged = VEC > 1 && S % VEC != 0;
     return l;
 }
+// The same, where a lane whose strip gives it no columns at all reads the row's last VEC too: every load is in bounds, none
+// behind a condition.  All its columns are duplicates (S >= VEC > 1).
+template <int VEC, int W>
+__device__ __forceinline__ LaneCols lane_cols_inside(int nominal, int S) {
+    LaneCols l;
+    l.ok = nominal < S;
+    l.col = min(nominal, S - VEC);
+    l.dup = min(nominal - l.col, VEC);
+    l.ragged = S % W != 0;      // strips are W columns wide
+    return l;
+}
 // Whether an operand may be overwritten in place by a kernel that holds whole tiles in registers: a duplicated column
 // must not be written by one workgroup before another has read it, so the short group and its neighbour have to lie in
 // the same strip of W columns.
