@@ -13,7 +13,7 @@
 //
 // Three launches (one, col_sum_small_kernel, up to 512 positions):
 //   1. chunk_sort_blk_kernel: every 256 consecutive (token, position-in-block) words sorted by counting.
-//   2. block_rank_kernel: the sorted chunks of a block merged by rank (16 lanes per position, a binary search per
+//   2. block_rank_kernel: the sorted chunks of a block merged by rank (16 lanes per one or two positions, a binary search per
 //      chunk): rk[position] = its rank within the block, and the block's runs {token, first rank, length}, long runs
 //      listed from the front of the block's task array, short ones from its back.
 //   3. col_sum_kernel<K>: per block, every thread writes its values of dx (fetched into registers while the previous
@@ -31,6 +31,7 @@ constexpr int CB_CHUNKS = CB / CHUNK;       // sorted chunks per block
 constexpr int CB_CPL = CB_CHUNKS / 16;      // chunks searched by one lane
 constexpr int COL_LONG = 16;                // runs of at least this many positions go to the long-run waves
 constexpr int COL_CARRY = 256;              // entries of the token-indexed table that carries long runs' sums to the next block
+constexpr int RANK_ONE = 32768;             // up to here block_rank_kernel ranks 64 positions per workgroup: two on each of 256 compute units
 constexpr int COL_PPT = CB / 1024;          // positions of a block per thread
 static_assert(CB_CPL >= 1 && COL_PPT % 4 == 0, "block size");
 
@@ -64,17 +65,22 @@ __global__ __launch_bounds__(CHUNK) void chunk_sort_blk_kernel(unsigned *__restr
     sorted_chunks[blockIdx.x * CHUNK + r] = w;
 }
 
-// One workgroup = 64 consecutive positions of one block, 16 lanes per position, one chunk of the block per lane.
+// One workgroup = 64*P consecutive positions of one block, 16 lanes per position, one chunk of the block per lane.
 // rk[position] = its rank within its block.
 // tasks[block][...] = {token, start | length << 16}; cnt[block] = number of long runs (low word) and of short runs.
+// A workgroup's time is the fill of its LDS and a chain of searches, whatever P is; two fit a compute unit.  With P = 1 a launch
+// of 625 is a round and a fifth: 40000 positions 15.0 us, with P = 2 10.7 (the whole call 102.6 -> 98.3); 16384 positions
+// take as long with either, 5796 and 10240 1 us longer with P = 2.
+template <int P>
 __global__ __launch_bounds__(1024) void block_rank_kernel(uint16_t *__restrict__ rk, v2u *__restrict__ tasks,
                                                           unsigned long long *__restrict__ cnt,
                                                           const unsigned *__restrict__ sorted_chunks,
                                                           const int32_t *__restrict__ ids, int N, int V, int nchunks) {
     __shared__ unsigned sc[CB_CHUNKS * CHUNK_PITCH];
     __shared__ int n_long, n_short, base_long, base_short;
+    static_assert(CB % (64 * P) == 0, "a workgroup's positions lie in one block");
     const int t = threadIdx.x;
-    const int n0 = blockIdx.x * 64, blk = n0 >> CB_BITS, c0 = blk * CB_CHUNKS;
+    const int n0 = blockIdx.x * (64 * P), blk = n0 >> CB_BITS, c0 = blk * CB_CHUNKS;
 #pragma unroll
     for (int i = 0; i < CB / 4096; i++) {
         const int j = i * 4096 + 4 * t;
@@ -84,10 +90,9 @@ __global__ __launch_bounds__(1024) void block_rank_kernel(uint16_t *__restrict__
         dst[0] = q.x; dst[1] = q.y; dst[2] = q.z; dst[3] = q.w;
     }
     const int k = t & 15, tl = t >> 4;
-    const int e = n0 + tl;
-    const bool live = e < N;
-    const unsigned w = pack_word_blk(ids, e, N, V);
-    const unsigned key = w >> CB_BITS;
+    unsigned w[P];
+#pragma unroll
+    for (int u = 0; u < P; u++) w[u] = pack_word_blk(ids, n0 + tl + 64 * u, N, V);
     if (t == 0) n_long = n_short = 0;
     __syncthreads();
     // a lane's chunks: k, k + 16, ...; one past the end is searched as chunk 0 and not counted.  The searches of a
@@ -99,48 +104,65 @@ __global__ __launch_bounds__(1024) void block_rank_kernel(uint16_t *__restrict__
         okc[m] = c0 + k + 16 * m < nchunks;
         chp[m] = sc + (okc[m] ? k + 16 * m : 0) * CHUNK_PITCH;
     }
-    auto count_below = [&](unsigned x, int (&p)[CB_CPL]) {       // per chunk: number of words < x
+    auto count_below = [&](const unsigned (&x)[P], int (&p)[P][CB_CPL]) {       // per chunk: number of words < x
 #pragma unroll
-        for (int m = 0; m < CB_CPL; m++) p[m] = 0;
+        for (int u = 0; u < P; u++)
+#pragma unroll
+            for (int m = 0; m < CB_CPL; m++) p[u][m] = 0;
 #pragma unroll
         for (int st = CHUNK / 2; st >= 1; st >>= 1) {
 #pragma unroll
-            for (int m = 0; m < CB_CPL; m++)
-                if (chp[m][p[m] + st - 1] < x) p[m] += st;
+            for (int u = 0; u < P; u++)
+#pragma unroll
+                for (int m = 0; m < CB_CPL; m++)
+                    if (chp[m][p[u][m] + st - 1] < x[u]) p[u][m] += st;
         }
 #pragma unroll
-        for (int m = 0; m < CB_CPL; m++) p[m] += chp[m][p[m]] < x ? 1 : 0;
+        for (int u = 0; u < P; u++)
+#pragma unroll
+            for (int m = 0; m < CB_CPL; m++) p[u][m] += chp[m][p[u][m]] < x[u] ? 1 : 0;
     };
-    int p[CB_CPL];
-    int below = 0;
-    unsigned pred1 = 0;                                         // largest smaller word + 1, or 0 if there is none
+    int p[P][CB_CPL], below[P], upto[P], idx[P];
+    unsigned pred1[P], next[P];                                 // pred1: largest smaller word + 1, or 0 if there is none
+    bool first[P], any_first = false;
     count_below(w, p);
 #pragma unroll
-    for (int m = 0; m < CB_CPL; m++)
-        if (okc[m]) {
-            below += p[m];
-            if (p[m] > 0) pred1 = max(pred1, chp[m][p[m] - 1] + 1u);
+    for (int u = 0; u < P; u++) {
+        below[u] = 0;
+        pred1[u] = 0;
+#pragma unroll
+        for (int m = 0; m < CB_CPL; m++)
+            if (okc[m]) {
+                below[u] += p[u][m];
+                if (p[u][m] > 0) pred1[u] = max(pred1[u], chp[m][p[u][m] - 1] + 1u);
+            }
+#pragma unroll
+        for (int m = 1; m < 16; m <<= 1) {
+            below[u] += __shfl_xor(below[u], m, 64);
+            pred1[u] = max(pred1[u], (unsigned)__shfl_xor((int)pred1[u], m, 64));
         }
-#pragma unroll
-    for (int m = 1; m < 16; m <<= 1) {
-        below += __shfl_xor(below, m, 64);
-        pred1 = max(pred1, (unsigned)__shfl_xor((int)pred1, m, 64));
+        const unsigned key = w[u] >> CB_BITS;
+        first[u] = n0 + tl + 64 * u < N && key < (unsigned)V && (pred1[u] == 0 || ((pred1[u] - 1u) >> CB_BITS) != key);
+        next[u] = (key + 1u) << CB_BITS;                        // no overflow where first: key < V < 2^(32 - CB_BITS)
+        any_first |= first[u];
+        upto[u] = 0;
     }
-    const bool first = live && key < (unsigned)V && (pred1 == 0 || ((pred1 - 1u) >> CB_BITS) != key);
-    int upto = 0;
-    if (first) {                                                // uniform over the 16 lanes of a position
-        count_below((key + 1u) << CB_BITS, p);                  // no overflow: key < V < 2^(32 - CB_BITS)
+    if (any_first) {                                            // uniform over the 16 lanes of the positions
+        count_below(next, p);
 #pragma unroll
-        for (int m = 0; m < CB_CPL; m++) upto += okc[m] ? p[m] : 0;
+        for (int u = 0; u < P; u++) {
 #pragma unroll
-        for (int m = 1; m < 16; m <<= 1) upto += __shfl_xor(upto, m, 64);
+            for (int m = 0; m < CB_CPL; m++) upto[u] += okc[m] ? p[u][m] : 0;
+#pragma unroll
+            for (int m = 1; m < 16; m <<= 1) upto[u] += __shfl_xor(upto[u], m, 64);
+        }
     }
-    const bool head = k == 0 && first;
-    const int len = upto - below;
-    const bool is_long = head && len >= COL_LONG;
-    int idx = 0;
-    if (head) idx = atomicAdd(is_long ? &n_long : &n_short, 1);
-    if (k == 0 && live) rk[e] = (uint16_t)below;
+    const auto is_long = [&](int u) { return upto[u] - below[u] >= COL_LONG; };
+#pragma unroll
+    for (int u = 0; u < P; u++) {
+        if (k == 0 && first[u]) idx[u] = atomicAdd(is_long(u) ? &n_long : &n_short, 1);
+        if (k == 0 && n0 + tl + 64 * u < N) rk[n0 + tl + 64 * u] = (uint16_t)below[u];
+    }
     __syncthreads();
     if (t == 0) {
         unsigned long long old = 0;
@@ -150,10 +172,12 @@ __global__ __launch_bounds__(1024) void block_rank_kernel(uint16_t *__restrict__
         base_short = (int)(old >> 32);
     }
     __syncthreads();
-    if (head) {
-        const v2u entry = {key, (unsigned)below | ((unsigned)len << 16)};
-        tasks[(size_t)blk * CB + (is_long ? base_long + idx : CB - 1 - (base_short + idx))] = entry;
-    }
+#pragma unroll
+    for (int u = 0; u < P; u++)
+        if (k == 0 && first[u]) {
+            const v2u entry = {w[u] >> CB_BITS, (unsigned)below[u] | ((unsigned)(upto[u] - below[u]) << 16)};
+            tasks[(size_t)blk * CB + (is_long(u) ? base_long + idx[u] : CB - 1 - (base_short + idx[u]))] = entry;
+        }
 }
 
 
@@ -547,8 +571,12 @@ int scatter_add_cols(float *dE, const float *dx, const int32_t *ids, int V, int 
     v2u *tasks = (v2u *)(ws + off_tasks);
     hipLaunchKernelGGL(chunk_sort_blk_kernel, dim3(nchunks), dim3(CHUNK), 0, g_ctx.stream, sorted_chunks, cnt, nblk, ids,
                        N, V);
-    hipLaunchKernelGGL(block_rank_kernel, dim3((unsigned)ceil_div((size_t)N, 64)), dim3(1024), 0, g_ctx.stream, rk, tasks,
-                       cnt, sorted_chunks, ids, N, V, nchunks);
+    auto rank = [&](auto kernel, int per) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)ceil_div((size_t)N, (size_t)per)), dim3(1024), 0, g_ctx.stream, rk, tasks, cnt,
+                           sorted_chunks, ids, N, V, nchunks);
+    };
+    if (N <= RANK_ONE) rank(block_rank_kernel<1>, 64);
+    else rank(block_rank_kernel<2>, 128);
     LAUNCH_OK("embed_scatter_add plan");
     const bool any = S % 4 != 0 || !aligned16(dx);
     auto launch = [&](auto kernel) {
