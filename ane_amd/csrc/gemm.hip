@@ -316,7 +316,7 @@ constexpr GemmKernel GEMM_KERNELS[] = {
     {0, 1, 64, 64, 16, 4, 0.41, 0.30, 0.14}, {0, 2, 64, 64, 32, 3, 0.48, 0.49, 1.7},
     {0, 4, 64, 32, 64, 3, 0.67, 0.66, 0.27}, {0, 4, 32, 64, 64, 3, 0.67, 0.66, 0.27},
     {1, 1, 128, 256, 32, 1, 2.3, 2.6, 4.2},  {1, 1, 256, 128, 32, 1, 2.3, 2.6, 4.2},
-    {1, 1, 64, 64, 32, 3, 0.93, 0.43, 2.1},  {1, 2, 64, 64, 64, 1, 0.91, 0.91, 2.7},
+    {1, 1, 64, 64, 32, 3, 0.93, 0.43, 2.1},  {1, 2, 64, 64, 64, 1, 0.86, 0.86, 2.7},
     {2, 1, 96, 256, 64, 1, 3.7, 3.7, 4.4},   {2, 1, 64, 256, 64, 1, 2.6, 2.6, 4.4},
 };
 // The kernel and number of K slices with the least estimated time: a launch, the longer of the work of the busiest compute

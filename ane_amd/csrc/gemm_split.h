@@ -385,7 +385,10 @@ __global__ __launch_bounds__(S_THREADS) void sgemm_split_kernel(const float *__r
 // steps in turn.  One group: three workgroups share a compute unit (49 KB each) and one splits, loads or stores while another
 // multiplies; [3072][256] . [256][1024] += 18.0 us (fp32 64 x 64 20.1, 128 x 256 27), [9001][768] . [768][197] 35 (49, 43).
 // Two groups: where there is one tile to a compute unit, whose four waves would wait for each other (1024 x 1024 x 1024
-// 27.8 with one group, 21.6 with two).  What bounds it is the splitting, done again by every tile: at 64 x 64 as many vector
+// 27.8 with one group, 21.6 with two).  There the steps up to the last few know that there is another behind them: a step
+// without branches can be scheduled as one ([3563][1024] . [1024][256] 22.0 -> 20.1 us, [256][768] of 2657 rows 16.7 -> 14.9); with one
+// group, where other workgroups fill in, that changes nothing or costs
+// ([9001][1024] . [1024][256] 44 -> 50).  What bounds it is the splitting, done again by every tile: at 64 x 64 as many vector
 // cycles as half of the matrix cycles, and the LDS reads, as many cycles as the products.  A second step on its way to
 // registers changed nothing (12.7 and 12.7 at [2048][256] . [256][768]), nor did tiles of 64 x 128 (13.4).
 // The hh products of a term have sums of their own, so a sum of full size is rounded once per 32 values of k, and the five
@@ -456,7 +459,7 @@ __global__ __launch_bounds__(SS_THREADS * KS) void sgemm_split_small_kernel(cons
         const int slot = wn + 16 * j + li;
         fb[j] = slot * (SK * 2) + split_chunk(slot, quarter) * 16 + 3 * OpA::PLANE;
     }
-    for (int t = 0; t < rounds; t++) {
+    auto step = [&](auto steady, int t) __attribute__((always_inline)) {
         const char *cur = lds[group][t & 1];
         bf8_t a[FM][3], b[FN][3];
 #pragma unroll
@@ -466,7 +469,7 @@ __global__ __launch_bounds__(SS_THREADS * KS) void sgemm_split_small_kernel(cons
 #pragma unroll
             for (int j = 0; j < FN; j++) b[j][q] = *reinterpret_cast<const bf8_t *>(cur + fb[j] + q * OpB::PLANE);
         }
-        const bool more = t + 1 < rounds;
+        const bool more = decltype(steady)::value || t + 1 < rounds;
         constexpr int P[6][2] = {{0, 0}, {0, 1}, {1, 0}, {1, 1}, {0, 2}, {2, 0}};
 #pragma unroll
         for (int p = 0; p < 6; p++) {
@@ -479,11 +482,14 @@ __global__ __launch_bounds__(SS_THREADS * KS) void sgemm_split_small_kernel(cons
                 }
             if (more && p < NPA + NPB) piece(p, lds[group][(t + 1) & 1]);
         }
-        if (more) {
-            if (t + 2 < rounds) fetch(t + 2);
-            __syncthreads();
-        }
-    }
+        if (decltype(steady)::value) { oa.fetch(edge_m); ob.fetch(edge_n); }
+        else if (t + 2 < rounds) fetch(t + 2);
+        if (more) __syncthreads();
+    };
+    int t = 0;
+    if constexpr (KS > 1)
+        for (; KS * (t + 2) + KS - 1 < steps; t++) step(std::true_type(), t);
+    for (; t < rounds; t++) step(std::false_type(), t);
 #pragma unroll
     for (int i = 0; i < FM; i++)
 #pragma unroll
