@@ -386,7 +386,7 @@ __global__ __launch_bounds__(S_THREADS) void sgemm_split_kernel(const float *__r
 // multiplies; [3072][256] . [256][1024] += 18.0 us (fp32 64 x 64 20.1, 128 x 256 27), [9001][768] . [768][197] 35 (49, 43).
 // Two groups: where there is one tile to a compute unit, whose four waves would wait for each other (1024 x 1024 x 1024
 // 27.8 with one group, 21.6 with two).  There the steps up to the last few know that there is another behind them: a step
-// without branches can be scheduled as one ([3563][1024] . [1024][256] 22.0 -> 20.1 us, [256][768] of 2657 rows 16.7 -> 14.9); with one
+// without branches can be scheduled as one ([3563][1024] . [1024][256] 22.0 -> 20.1 us, [2657][768] . [768][256] 16.7 -> 14.9); with one
 // group, where other workgroups fill in, that changes nothing or costs
 // ([9001][1024] . [1024][256] 44 -> 50).  What bounds it is the splitting, done again by every tile: at 64 x 64 as many vector
 // cycles as half of the matrix cycles, and the LDS reads, as many cycles as the products.  A second step on its way to

@@ -17,6 +17,7 @@
 #include "tile.h"
 
 #include <math.h>
+#include <algorithm>
 #include <type_traits>
 
 namespace {
@@ -362,7 +363,7 @@ constexpr int CR_THREADS = 1024;
 constexpr int CR_W = 64;                     // columns per strip
 constexpr int CR_RPS = CR_THREADS / 16;      // rows per step: 16 lanes x 16 B per row piece
 constexpr int CR_NW = CR_THREADS / 64;
-constexpr int CR_MAX_SPLIT = 64;             // members per strip
+constexpr int CR_MAX_SPLIT = 128;            // members per strip
 constexpr int CR_MAX_STRIPS = 16;
 constexpr int CR_LOSS_SLOT = 2 * CR_W;       // after the 64 maxima and 64 sums
 constexpr int CR_STRIDE = 136;               // slots per workgroup number
@@ -620,20 +621,19 @@ __device__ __forceinline__ void cr_member_partial(const CrGeo<typename ST::T> &g
     __syncthreads();
 }
 
-constexpr int CR_MPG = CR_MAX_SPLIT / CR_NW;     // members per group of 64 threads (thread = group, slot)
-
-// The members' partials, four members per thread (pm, pl: member grp * mpg + q of slot c) -> the strip's column maxima
+// The members' partials, MPG members per thread (pm, pl: member grp * mpg + q of slot c) -> the strip's column maxima
 // and the reciprocals of its sums, in fM and fInv (valid after the barrier): first within the sixteen groups, then the
 // groups.
-__device__ __forceinline__ void cr_merge_members(const float (&pm)[CR_MPG], const float (&pl)[CR_MPG], float (*wm)[CR_P],
+template <int MPG>
+__device__ __forceinline__ void cr_merge_members(const float (&pm)[MPG], const float (&pl)[MPG], float (*wm)[CR_P],
                                                  float (*wl)[CR_P], float *fM, float *fInv) {
     const int c = threadIdx.x & 63, grp = threadIdx.x >> 6;
     float M = pm[0];
 #pragma unroll
-    for (int q = 1; q < CR_MPG; q++) M = fmaxf(M, pm[q]);
+    for (int q = 1; q < MPG; q++) M = fmaxf(M, pm[q]);
     float L = 0.f;
 #pragma unroll
-    for (int q = 0; q < CR_MPG; q++) L += pl[q] * exp_neg(pm[q] - M);      // a member that is absent has sum 0
+    for (int q = 0; q < MPG; q++) L += pl[q] * exp_neg(pm[q] - M);      // a member that is absent has sum 0
     wm[grp][c] = M;
     wl[grp][c] = L;
     __syncthreads();
@@ -681,10 +681,12 @@ __device__ __forceinline__ bool cr_wait_slot(const unsigned long long *sp, unsig
 // the code of a step is written out once for each, 60 KB (fp32) and 83 KB (bfloat16) for the largest, and a launch that
 // runs through it once per wave waits for instructions: with one row step per workgroup ([1000][256]) a launch took
 // 12.8 us, 4.8 of them before its partial was ready.
+// MEMBERS: the most a strip may have.  128 take a thread 32 registers more for the slots it fetches, so the variants for them hold
+// eight row steps in registers and the others in LDS.
 // NT: rows are read and written past the caches where their pieces are whole 128-byte lines; where two strips share
 // the lines at their border the caches have to put the pieces together ([151936][200] fp32 102 us past them, 77 with
 // them; [151936][256] 68 and 94).
-template <typename ST, int K_REG, int K_LDS, bool NT>
+template <typename ST, int K_REG, int K_LDS, bool NT, int MEMBERS = CR_MAX_SPLIT / 2>
 __global__ __launch_bounds__(CR_THREADS) void ce_resident_kernel(typename ST::T *__restrict__ dlogits,
                                                                  const typename ST::T *__restrict__ logits,
                                                                  const int32_t *__restrict__ targets, int V, int S,
@@ -692,13 +694,14 @@ __global__ __launch_bounds__(CR_THREADS) void ce_resident_kernel(typename ST::T 
                                                                  float grad_scale, float *__restrict__ loss_out, CeXch ws,
                                                                  int spin_ticks, int take_nothing) {
     typedef typename ST::Raw Raw;
+    constexpr int MPG = MEMBERS / CR_NW;           // members per group of 64 threads (thread = group, slot)
     __shared__ Raw lrow[K_LDS > 0 ? K_LDS : 1][K_LDS > 0 ? CR_THREADS : 1];
     __shared__ float wm[CR_NW][CR_P], wl[CR_NW][CR_P];
     __shared__ float fb[2][CR_W];                  // one member's partial on its way to the threads that hold it
     __shared__ float fM[CR_W], fInv[CR_W];
     __shared__ float strip_loss[CR_MAX_STRIPS];
-    __shared__ unsigned want[CR_MAX_SPLIT];
-    __shared__ int failed[CR_MAX_SPLIT], failed_loss[CR_MAX_STRIPS];
+    __shared__ unsigned want[MEMBERS];
+    __shared__ int failed[MEMBERS], failed_loss[CR_MAX_STRIPS];
     __shared__ int any_failed, any_failed_loss;
     const int tid = threadIdx.x;
     auto rows_of = [&]() { return (Raw (*)[CR_THREADS])lrow; };
@@ -732,15 +735,15 @@ __global__ __launch_bounds__(CR_THREADS) void ce_resident_kernel(typename ST::T 
     const float my_logit = cr_slot_logit(g, strip, my_tgt);         // (in flight while the partners' partials are awaited)
     __syncthreads();
     // ---- every member's partial.  Thread (group, slot) fetches the (max, sum) slots of the group's members for
-    // its slot: eight of them.  The loads of a round go out together, so a round costs one trip to the memory side
-    // however many of the eight are still missing.
+    // its slot: eight of them (sixteen with 128 members).  The loads of a round go out together, so a round costs one trip
+    // to the memory side however many of them are still missing.
     const int mc = tid & 63, mgrp = tid >> 6;
-    const int mpg = (csplit + CR_NW - 1) / CR_NW;                      // members per group, at most CR_MPG
-    float pm[CR_MPG], pl[CR_MPG];
+    const int mpg = (csplit + CR_NW - 1) / CR_NW;                      // members per group, at most MPG
+    float pm[MPG], pl[MPG];
     {
         unsigned pend = 0;
 #pragma unroll
-        for (int q = 0; q < CR_MPG; q++) {
+        for (int q = 0; q < MPG; q++) {
             pm[q] = NO_MAX;
             pl[q] = 0.f;
             if (q < mpg && mgrp * mpg + q < csplit) pend |= 3u << (2 * q);
@@ -748,22 +751,22 @@ __global__ __launch_bounds__(CR_THREADS) void ce_resident_kernel(typename ST::T 
         const long long t0 = wall_clock64();
         if (take_nothing) {                    // test mode: every partner counts as late, whatever its slots hold
 #pragma unroll
-            for (int f = 0; f < 2 * CR_MPG; f++)
+            for (int f = 0; f < 2 * MPG; f++)
                 if ((pend >> f) & 1u) failed[mgrp * mpg + (f >> 1)] = 1;
             any_failed = 1;
             pend = 0;
         }
         while (pend) {
-            unsigned long long pk[2 * CR_MPG];
+            unsigned long long pk[2 * MPG];
 #pragma unroll
-            for (int f = 0; f < 2 * CR_MPG; f++) {
+            for (int f = 0; f < 2 * MPG; f++) {
                 const int p = mgrp * mpg + (f >> 1);
                 if ((pend >> f) & 1u)
                     pk[f] = __hip_atomic_load(ws.slots + (size_t)(p * strips + strip) * CR_STRIDE + (f & 1) * CR_W + mc,
                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
 #pragma unroll
-            for (int f = 0; f < 2 * CR_MPG; f++) {
+            for (int f = 0; f < 2 * MPG; f++) {
                 const int p = mgrp * mpg + (f >> 1);
                 if (((pend >> f) & 1u) && (unsigned)(pk[f] >> 32) == want[p]) {
                     if (f & 1) pl[f >> 1] = __uint_as_float((unsigned)pk[f]);
@@ -774,7 +777,7 @@ __global__ __launch_bounds__(CR_THREADS) void ce_resident_kernel(typename ST::T 
             if (pend) {
                 if (wall_clock64() - t0 >= (long long)spin_ticks) {
 #pragma unroll
-                    for (int f = 0; f < 2 * CR_MPG; f++)
+                    for (int f = 0; f < 2 * MPG; f++)
                         if ((pend >> f) & 1u) failed[mgrp * mpg + (f >> 1)] = 1;
                     any_failed = 1;
                     break;
@@ -784,13 +787,13 @@ __global__ __launch_bounds__(CR_THREADS) void ce_resident_kernel(typename ST::T 
         }
     }
     // one member's partial from memory, into the threads that hold it
-    auto recompute = [&](int s2, int p, float (&qm)[CR_MPG], float (&ql)[CR_MPG]) {
+    auto recompute = [&](int s2, int p, float (&qm)[MPG], float (&ql)[MPG]) {
         float M2 = NO_MAX, L2 = 0.f;
         cr_member_partial<ST, K_REG, K_LDS, false, NT>(g, s2, p, xr, rows_of(), wm, wl, M2, L2);
         if (tid < 4 * CR_W && (tid & 3) == 0) { fb[0][tid >> 2] = M2; fb[1][tid >> 2] = L2; }
         __syncthreads();
 #pragma unroll
-        for (int q = 0; q < CR_MPG; q++)
+        for (int q = 0; q < MPG; q++)
             if (q < mpg && mgrp * mpg + q == p) { qm[q] = fb[0][mc]; ql[q] = fb[1][mc]; }
         __syncthreads();
     };
@@ -901,9 +904,9 @@ __global__ __launch_bounds__(CR_THREADS) void ce_resident_kernel(typename ST::T 
         if (any_failed_loss) {
             for (int s2 = 1; s2 < strips; s2++) {
                 if (failed_loss[s2]) {
-                    float qm[CR_MPG], ql[CR_MPG];
+                    float qm[MPG], ql[MPG];
 #pragma unroll
-                    for (int q = 0; q < CR_MPG; q++) { qm[q] = NO_MAX; ql[q] = 0.f; }
+                    for (int q = 0; q < MPG; q++) { qm[q] = NO_MAX; ql[q] = 0.f; }
                     for (int p = 0; p < csplit; p++) recompute(s2, p, qm, ql);
                     cr_merge_members(qm, ql, wm, wl, fM, fInv);
                     if (tid < CR_W) {
@@ -967,7 +970,8 @@ int ce_run(const char *who, T *dlogits, float *loss_dev, const T *logits, const 
         // Not for a single strip of fp32 whose members have more than 14 row steps (V > 57344 in 64 members): its 64
         // workgroups leave three quarters of the chip idle.  [50000][63] 19.0 against 20.0, [65536][63] 20.8 against 20.3,
         // [90000][64] 28.5 against 23.9, [151936][63] 44.5 against 34.5, [151936][4] 41 against 23.  (bfloat16, whose three
-        // launches convert twice: [151936][63] 44 against 56; two strips: [151936][65] 46 against 50.)
+        // launches convert twice: [151936][63] 44 against 56; two strips: [151936][65] 46 against 50.)  The line is drawn by what 64
+        // members take and left there: with the 128 below one launch would be ahead from it on ([120000][33] 21.5 against 24.4).
         typedef typename std::conditional<std::is_same<T, float>::value, CrF32, CrBf16>::type ST;
         const int cu = g_ctx.num_cu > 0 ? g_ctx.num_cu : 256;
         const int strips_r = (int)ceil_div((size_t)S, (size_t)CR_W);
@@ -979,11 +983,22 @@ int ce_run(const char *who, T *dlogits, float *loss_dev, const T *logits, const 
         const int sw = lines ? CR_W : 4 * (int)ceil_div((size_t)S, 4 * (size_t)strips_r);
         unsigned char *base = (g_ctx.device >= 0 && g_ctx.device < CE_MAX_DEVICES) ? g_scratch_ptr[g_ctx.device] : nullptr;
         if (g_ctx.ce_resident >= 0 && base && S >= 4 && strips_r <= CR_MAX_STRIPS && (const void *)dlogits != (const void *)logits) {
-            const int csplit = cu / strips_r < CR_MAX_SPLIT ? cu / strips_r : CR_MAX_SPLIT;
-            const int Rm = csplit > 0 ? (int)ceil_div((size_t)V, (size_t)csplit) : 0;
-            const int K = (int)ceil_div((size_t)Rm, (size_t)CR_RPS);
-            if (csplit >= 2 && csplit * strips_r <= CR_MAX_WG && csplit * strips_r <= cu && K <= CR_MAX_STEPS &&
-                !(std::is_same<T, float>::value && strips_r == 1 && K > 14 && g_ctx.ce_resident == 0)) {
+            int csplit = std::min(cu / strips_r, CR_MAX_SPLIT / 2);
+            const auto rows = [&]() { return csplit > 0 ? (int)ceil_div((size_t)V, (size_t)csplit) : 0; };
+            const auto row_steps = [&]() { return (int)ceil_div((size_t)rows(), (size_t)CR_RPS); };
+            if (csplit >= 2 && csplit * strips_r <= CR_MAX_WG && csplit * strips_r <= cu && row_steps() <= CR_MAX_STEPS &&
+                !(std::is_same<T, float>::value && strips_r == 1 && row_steps() > 14 && g_ctx.ce_resident == 0)) {
+                // Few strips: 64 members each leave compute units idle, and twice as many halve their rows for 1.7 us more of
+                // exchange.  us, 64 / 128 members: fp32 [16000][64] 10.1 / 11.1, [32000][64] 13.3 / 12.4, [28673][123] 14.4 / 14.7, [86946][128] 25.9 / 23.7,
+                // [151936][128] 44.7 / 37.9; bfloat16 [32000][64] 14.0 / 13.0, [86946][64] 31.3 / 18.4, [151936][128] 46.6 / 27.0,
+                // [202000][33] 53 / 32.  Three strips, 64 / 80 members (a multiple of 8 keeps a strip's workgroups on their XCD; with
+                // 85 [120000][150] takes 58 for 47): bfloat16 [32000][150] 14.6 / 14.9, [64000][192] 23.3 / 20.4, [151936][150] 49.6 /
+                // 41.6; fp32 [64000][150] 23.5 / 22.4, [151936][192] 52.6 / 53.2, left as it is.
+                // (fp32 strips that take three launches keep 64 members where one is forced: the form that the line above compares.)
+                const int many = std::min(cu / strips_r, CR_MAX_SPLIT) & ~7, steps = row_steps();
+                const bool few = sizeof(T) == 2 ? strips_r <= 2 || (strips_r == 3 && steps > 12) : (strips_r == 2 && steps > 8) || (strips_r == 1 && steps <= 14);
+                if (many > csplit && few && steps > 7) csplit = many;
+                const int Rm = rows(), K = row_steps();
                 CeXch xch;
                 xch.slots = (unsigned long long *)(base + CE_SCRATCH_BYTES);
                 xch.cnt = (unsigned *)(base + CE_SCRATCH_BYTES + (size_t)CR_MAX_WG * CR_STRIDE * 8);
@@ -994,7 +1009,14 @@ int ce_run(const char *who, T *dlogits, float *loss_dev, const T *logits, const 
                                        logits, targets, V, S, strips_r, sw, csplit, Rm, 1.0f / (float)S, grad_scale, loss_dev,
                                        xch, spin < 0 ? 0 : spin, g_ctx.xch_take_nothing > 0 ? 1 : 0);
                 };
-                if (K <= 8) { if (lines) launch(ce_resident_kernel<ST, 8, 0, true>); else launch(ce_resident_kernel<ST, 8, 0, false>); }
+                if (csplit > CR_MAX_SPLIT / 2 && K <= 8) {
+                    if (lines) launch(ce_resident_kernel<ST, 8, 0, true, CR_MAX_SPLIT>);
+                    else launch(ce_resident_kernel<ST, 8, 0, false, CR_MAX_SPLIT>);
+                } else if (csplit > CR_MAX_SPLIT / 2) {
+                    if (lines) launch(ce_resident_kernel<ST, 8, ST::K_LDS, true, CR_MAX_SPLIT>);
+                    else launch(ce_resident_kernel<ST, 8, ST::K_LDS, false, CR_MAX_SPLIT>);
+                }
+                else if (K <= 8) { if (lines) launch(ce_resident_kernel<ST, 8, 0, true>); else launch(ce_resident_kernel<ST, 8, 0, false>); }
                 else if (K <= 16) { if (lines) launch(ce_resident_kernel<ST, 16, 0, true>); else launch(ce_resident_kernel<ST, 16, 0, false>); }
                 else if (lines) launch(ce_resident_kernel<ST, ST::K_REG, ST::K_LDS, true>);
                 else launch(ce_resident_kernel<ST, ST::K_REG, ST::K_LDS, false>);
