@@ -130,13 +130,15 @@ __global__ __launch_bounds__(THREADS) void rms_fwd_bf16_kernel(bf16_t *__restric
     if constexpr (CAP > 0) {
         typename RawT<VEC>::type xr[CAP];
         float wv[CAP];
+        first_loads(S % 64 == 0, [&](auto lines) __attribute__((always_inline)) {
 #pragma unroll
-        for (int k = 0; k < CAP; k++) {
-            const int c = row0 + k * RPS;
-            const bool ok = c < C && col_ok;
-            xr[k] = ok ? ld_raw<VEC, false>(x + base + (size_t)c * S) : raw_zero<VEC>();
-            wv[k] = ok ? w[c] : 0.f;
-        }
+            for (int k = 0; k < CAP; k++) {
+                const int c = row0 + k * RPS;
+                const bool ok = c < C && col_ok;
+                xr[k] = ok ? ld_raw<VEC, decltype(lines)::value>(x + base + (size_t)c * S) : raw_zero<VEC>();
+                wv[k] = ok ? w[c] : 0.f;
+            }
+        });
 #pragma unroll
         for (int k = 0; k < CAP; k++) {
             float xv[VEC];
@@ -242,14 +244,16 @@ __global__ __launch_bounds__(THREADS) void rms_bwd_bf16_kernel(bf16_t *dx, float
     if constexpr (CAP > 0) {
         typename RawT<VEC>::type xr[CAP], dr[CAP];
         float wv[CAP];
+        first_loads(S % 64 == 0, [&](auto lines) __attribute__((always_inline)) {
 #pragma unroll
-        for (int k = 0; k < CAP; k++) {
-            const int c = row0 + k * RPS;
-            const bool ok = c < C && col_ok;
-            xr[k] = ok ? ld_raw<VEC, false>(x + base + (size_t)c * S) : raw_zero<VEC>();
-            dr[k] = ok ? ld_raw<VEC, false>(dy + base + (size_t)c * S) : raw_zero<VEC>();
-            wv[k] = ok ? w[c] : 0.f;
-        }
+            for (int k = 0; k < CAP; k++) {
+                const int c = row0 + k * RPS;
+                const bool ok = c < C && col_ok;
+                xr[k] = ok ? ld_raw<VEC, decltype(lines)::value>(x + base + (size_t)c * S) : raw_zero<VEC>();
+                dr[k] = ok ? ld_raw<VEC, decltype(lines)::value>(dy + base + (size_t)c * S) : raw_zero<VEC>();
+                wv[k] = ok ? w[c] : 0.f;
+            }
+        });
 #pragma unroll
         for (int k = 0; k < CAP; k++) {
             float xv[VEC], dv[VEC];
@@ -658,13 +662,13 @@ ClusterPlan plan_cluster_bf(int C, int S, int batch, bool vec_ok) {
     if (g_ctx.rms_lpr || g_ctx.rms_threads) return NO_CLUSTER;
     return cluster_plan(C, S, batch, vec_ok, StoreBf16::VEC, 2, 4, 1);
 }
-#define BF_CLUSTER_FWD(RPT, EXACT)                                                                                   \
-    hipLaunchKernelGGL((rms_fwd_cluster_kernel<StoreBf16, RPT, 1024, false, EXACT>), dim3(cp.nblk), dim3(1024), 0,   \
+#define BF_CLUSTER_FWD(RPT, WHOLE)                                                                                   \
+    hipLaunchKernelGGL((rms_fwd_cluster_kernel<StoreBf16, RPT, 1024, false, WHOLE>), dim3(cp.nblk), dim3(1024), 0,   \
                        g_ctx.stream, y, (uint16_t *)nullptr, x, (const uint16_t *)nullptr, 0.f, w, C, S, cp.strips,  \
                        cp.nblk, cp.csplit, cp.rows_pm, eps, 1.0f / (float)C, g_bf_cluster_ws,                        \
                        mi355_exchange_spin_ticks())
-#define BF_CLUSTER_BWD(RPT, EXACT)                                                                                   \
-    hipLaunchKernelGGL((rms_bwd_cluster_kernel<StoreBf16, RPT, 1024, false, EXACT>), dim3(cp.nblk), dim3(1024), 0,   \
+#define BF_CLUSTER_BWD(RPT, WHOLE)                                                                                   \
+    hipLaunchKernelGGL((rms_bwd_cluster_kernel<StoreBf16, RPT, 1024, false, WHOLE>), dim3(cp.nblk), dim3(1024), 0,   \
                        g_ctx.stream, dx, part, dy, x, w, C, S, cp.strips, cp.nblk, cp.csplit, cp.rows_pm, eps,       \
                        1.0f / (float)C, variant, (const uint16_t *)nullptr, (uint16_t *)nullptr, 0.f,                \
                        g_bf_cluster_ws, mi355_exchange_spin_ticks())
@@ -782,10 +786,11 @@ MI355_API int mi355_rmsnorm_fwd_bf16_dev(uint16_t *y, const uint16_t *x, const f
     const ClusterPlan cp = y == x ? NO_CLUSTER : plan_cluster_bf(C, S, batch, vec_ok);
     if (cp.csplit) {
         if (!mi355_exchange(&g_bf_cluster_ws)) return -1;
-        if (cp.rpt == 2 && cp.exact) BF_CLUSTER_FWD(2, true);
-        else if (cp.rpt == 2) BF_CLUSTER_FWD(2, false);
-        else if (cp.exact) BF_CLUSTER_FWD(4, true);
-        else BF_CLUSTER_FWD(4, false);
+        cluster_whole(cp, [&](auto whole) {
+            constexpr int WHOLE = decltype(whole)::value;
+            if (cp.rpt == 2) BF_CLUSTER_FWD(2, WHOLE);
+            else BF_CLUSTER_FWD(4, WHOLE);
+        });
         LAUNCH_OK("rmsnorm_fwd_bf16");
         return 0;
     }
@@ -812,9 +817,11 @@ MI355_API int mi355_rmsnorm_bwd_bf16_dev(uint16_t *dx, float *dw, const uint16_t
         float *part = mi355_dw_partials((size_t)nrows * C, dw, nullptr);
         if (!part) return -1;
         // (four rows per lane without the masks would need more than the 128 registers a lane has)
-        if (cp.rpt == 2 && cp.exact) BF_CLUSTER_BWD(2, true);
-        else if (cp.rpt == 2) BF_CLUSTER_BWD(2, false);
-        else BF_CLUSTER_BWD(4, false);
+        cluster_whole(cp, [&](auto whole) {
+            constexpr int WHOLE = decltype(whole)::value;
+            if (cp.rpt == 2) BF_CLUSTER_BWD(2, WHOLE);
+            else BF_CLUSTER_BWD(4, WHOLE == CL_EXACT ? CL_LINES : WHOLE);
+        });
         LAUNCH_OK("rmsnorm_bwd_bf16");
         if (mi355_dw_submit(dw, part, nrows, C)) return -1;
         return mi355_dw_op_end();
@@ -845,14 +852,15 @@ MI355_API int mi355_residual_rmsnorm_fwd_bf16_dev(uint16_t *y, uint16_t *yn, con
     const ClusterPlan cp = (y == a || y == b) ? NO_CLUSTER : plan_cluster_bf(C, S, batch, vec_ok);
     if (cp.csplit) {
         if (!mi355_exchange(&g_bf_cluster_ws)) return -1;
-#define BF_CLUSTER_RES_FWD(RPT, EXACT)                                                                               \
-    hipLaunchKernelGGL((rms_fwd_cluster_kernel<StoreBf16, RPT, 1024, true, EXACT>), dim3(cp.nblk), dim3(1024), 0,    \
+#define BF_CLUSTER_RES_FWD(RPT, WHOLE)                                                                               \
+    hipLaunchKernelGGL((rms_fwd_cluster_kernel<StoreBf16, RPT, 1024, true, WHOLE>), dim3(cp.nblk), dim3(1024), 0,    \
                        g_ctx.stream, yn, y, a, b, alpha, w, C, S, cp.strips, cp.nblk, cp.csplit, cp.rows_pm, eps,    \
                        1.0f / (float)C, g_bf_cluster_ws, mi355_exchange_spin_ticks())
-        if (cp.rpt == 2 && cp.exact) BF_CLUSTER_RES_FWD(2, true);
-        else if (cp.rpt == 2) BF_CLUSTER_RES_FWD(2, false);
-        else if (cp.exact) BF_CLUSTER_RES_FWD(4, true);
-        else BF_CLUSTER_RES_FWD(4, false);
+        cluster_whole(cp, [&](auto whole) {
+            constexpr int WHOLE = decltype(whole)::value;
+            if (cp.rpt == 2) BF_CLUSTER_RES_FWD(2, WHOLE);
+            else BF_CLUSTER_RES_FWD(4, WHOLE);
+        });
 #undef BF_CLUSTER_RES_FWD
         LAUNCH_OK("residual_rmsnorm_fwd_bf16");
         return 0;
@@ -881,13 +889,15 @@ MI355_API int mi355_rmsnorm_bwd_residual_bf16_dev(uint16_t *dx, uint16_t *dx_sca
         const int nrows = cp.nblk / cp.csplit;
         float *part = mi355_dw_partials((size_t)nrows * C, dw, nullptr);
         if (!part) return -1;
-#define BF_CLUSTER_RES_BWD(RPT, EXACT)                                                                               \
-    hipLaunchKernelGGL((rms_bwd_cluster_kernel<StoreBf16, RPT, 1024, true, EXACT>), dim3(cp.nblk), dim3(1024), 0,    \
+#define BF_CLUSTER_RES_BWD(RPT, WHOLE)                                                                               \
+    hipLaunchKernelGGL((rms_bwd_cluster_kernel<StoreBf16, RPT, 1024, true, WHOLE>), dim3(cp.nblk), dim3(1024), 0,    \
                        g_ctx.stream, dx, part, dy, x, w, C, S, cp.strips, cp.nblk, cp.csplit, cp.rows_pm, eps,       \
                        1.0f / (float)C, variant, res, dx_scaled, alpha, g_bf_cluster_ws, mi355_exchange_spin_ticks())
-        if (cp.rpt == 2 && cp.exact) BF_CLUSTER_RES_BWD(2, true);
-        else if (cp.rpt == 2) BF_CLUSTER_RES_BWD(2, false);
-        else BF_CLUSTER_RES_BWD(4, false);
+        cluster_whole(cp, [&](auto whole) {
+            constexpr int WHOLE = decltype(whole)::value;
+            if (cp.rpt == 2) BF_CLUSTER_RES_BWD(2, WHOLE);
+            else BF_CLUSTER_RES_BWD(4, WHOLE == CL_EXACT ? CL_LINES : WHOLE);
+        });
 #undef BF_CLUSTER_RES_BWD
         LAUNCH_OK("rmsnorm_bwd_residual_bf16");
         if (mi355_dw_submit(dw, part, nrows, C)) return -1;

@@ -48,7 +48,7 @@ __global__ __launch_bounds__(THREADS) void rms_fwd_kernel(float *__restrict__ y,
         for (int k = 0; k < CAP; k++) {
             const int c = row0 + k * RPS;
             if (c < C && col_ok) {
-                ldv<VEC>(xv[k], xs + (size_t)c * S);
+                ldv_nt<VEC>(xv[k], xs + (size_t)c * S);
                 wv[k] = w[c];
             } else {
 #pragma unroll
@@ -161,24 +161,28 @@ __device__ __forceinline__ void rms_bwd_body(float *dx, float *__restrict__ dw_p
 
     if constexpr (CAP > 0) {
         float xv[CAP][VEC], dv[CAP][VEC], wv[CAP], rv[RES ? CAP : 1][VEC];
+        auto first = [&](auto lines) __attribute__((always_inline)) {
 #pragma unroll
-        for (int k = 0; k < CAP; k++) {
-            const int c = row0 + k * RPS;
-            if (c < C && col_ok) {
-                ldv<VEC>(xv[k], xs + (size_t)c * S);
-                ldv<VEC>(dv[k], dys + (size_t)c * S);
-                if constexpr (RES) ldv<VEC>(rv[k], ress + (size_t)c * S);
-                wv[k] = w[c];
-            } else {
+            for (int k = 0; k < CAP; k++) {
+                const int c = row0 + k * RPS;
+                if (c < C && col_ok) {
+                    ldv_first<VEC, decltype(lines)::value>(xv[k], xs + (size_t)c * S);
+                    ldv_first<VEC, decltype(lines)::value>(dv[k], dys + (size_t)c * S);
+                    if constexpr (RES) ldv_first<VEC, decltype(lines)::value>(rv[k], ress + (size_t)c * S);
+                    wv[k] = w[c];
+                } else {
 #pragma unroll
-                for (int j = 0; j < VEC; j++) xv[k][j] = dv[k][j] = 0.f;
-                if constexpr (RES) {
+                    for (int j = 0; j < VEC; j++) xv[k][j] = dv[k][j] = 0.f;
+                    if constexpr (RES) {
 #pragma unroll
-                    for (int j = 0; j < VEC; j++) rv[k][j] = 0.f;
+                        for (int j = 0; j < VEC; j++) rv[k][j] = 0.f;
+                    }
+                    wv[k] = 0.f;
                 }
-                wv[k] = 0.f;
             }
-        }
+        };
+        if constexpr (RES) first(std::true_type());
+        else first_loads(S % 32 == 0, first);
 #pragma unroll
         for (int k = 0; k < CAP; k++)
 #pragma unroll
@@ -278,8 +282,8 @@ __global__ __launch_bounds__(THREADS) void res_rms_fwd_kernel(float *y, float *_
             const int c = row0 + k * RPS;
             if (c < C && col_ok) {
                 float bv[VEC];
-                ldv<VEC>(yv[k], a + base + (size_t)c * S);
-                ldv<VEC>(bv, b + base + (size_t)c * S);
+                ldv_nt<VEC>(yv[k], a + base + (size_t)c * S);
+                ldv_nt<VEC>(bv, b + base + (size_t)c * S);
 #pragma unroll
                 for (int j = 0; j < VEC; j++) yv[k][j] = bv[j] * alpha + yv[k][j];
                 wv[k] = w[c];
@@ -488,10 +492,10 @@ ClusterPlan plan_cluster(int C, int S, int batch, bool vec_ok, int max_rpt, int 
     return cluster_plan(C, S, batch, vec_ok, StoreF32::VEC, 4, max_rpt, rounds);
 }
 
-template <int RPT, bool FUSE, bool EXACT>
+template <int RPT, bool FUSE, int WHOLE>
 void launch_fwd_cluster_as(const ClusterPlan &cp, float *yn, float *y_res, const float *a, const float *b, float alpha,
                            const float *w, int C, int S, float eps) {
-    hipLaunchKernelGGL((rms_fwd_cluster_kernel<StoreF32, RPT, 1024, FUSE, EXACT>), dim3(cp.nblk), dim3(1024), 0, g_ctx.stream, yn,
+    hipLaunchKernelGGL((rms_fwd_cluster_kernel<StoreF32, RPT, 1024, FUSE, WHOLE>), dim3(cp.nblk), dim3(1024), 0, g_ctx.stream, yn,
                        y_res, a, b, alpha, w, C, S, cp.strips, cp.nblk, cp.csplit, cp.rows_pm, eps, 1.0f / (float)C,
                        g_cluster_ws, cluster_spin_ticks());
 }
@@ -499,17 +503,18 @@ void launch_fwd_cluster_as(const ClusterPlan &cp, float *yn, float *y_res, const
 template <bool FUSE>
 void launch_fwd_cluster(const ClusterPlan &cp, float *yn, float *y_res, const float *a, const float *b, float alpha,
                         const float *w, int C, int S, float eps) {
-    if (cp.rpt == 4 && cp.exact) launch_fwd_cluster_as<4, FUSE, true>(cp, yn, y_res, a, b, alpha, w, C, S, eps);
-    else if (cp.rpt == 4) launch_fwd_cluster_as<4, FUSE, false>(cp, yn, y_res, a, b, alpha, w, C, S, eps);
-    else if (cp.exact) launch_fwd_cluster_as<8, FUSE, true>(cp, yn, y_res, a, b, alpha, w, C, S, eps);
-    else launch_fwd_cluster_as<8, FUSE, false>(cp, yn, y_res, a, b, alpha, w, C, S, eps);
+    cluster_whole(cp, [&](auto whole) {
+        constexpr int WHOLE = decltype(whole)::value;
+        if (cp.rpt == 4) launch_fwd_cluster_as<4, FUSE, WHOLE>(cp, yn, y_res, a, b, alpha, w, C, S, eps);
+        else launch_fwd_cluster_as<8, FUSE, WHOLE>(cp, yn, y_res, a, b, alpha, w, C, S, eps);
+    });
 }
 
 // The backward tiles hold two (with the residual three) operands per row: four rows per lane fill the registers.
-template <bool RES, bool EXACT>
+template <bool RES, int WHOLE>
 void launch_bwd_cluster_as(const ClusterPlan &cp, float *dx, float *part, const float *dy, const float *x, const float *w,
                            int C, int S, float eps, int variant, const float *res, float *dx2, float alpha2) {
-    hipLaunchKernelGGL((rms_bwd_cluster_kernel<StoreF32, 4, 1024, RES, EXACT>), dim3(cp.nblk), dim3(1024), 0, g_ctx.stream, dx, part,
+    hipLaunchKernelGGL((rms_bwd_cluster_kernel<StoreF32, 4, 1024, RES, WHOLE>), dim3(cp.nblk), dim3(1024), 0, g_ctx.stream, dx, part,
                        dy, x, w, C, S, cp.strips, cp.nblk, cp.csplit, cp.rows_pm, eps, 1.0f / (float)C, variant, res, dx2,
                        alpha2, g_cluster_ws, cluster_spin_ticks());
 }
@@ -518,8 +523,10 @@ template <bool RES>
 void launch_bwd_cluster(const ClusterPlan &cp, float *dx, float *part, const float *dy, const float *x, const float *w,
                         int C, int S, float eps, int variant, const float *res, float *dx2, float alpha2) {
     // (with the residual 126 of the 128 registers a lane has; [16][1024][256] 15.4 -> 14.7 us)
-    if (cp.exact) launch_bwd_cluster_as<RES, true>(cp, dx, part, dy, x, w, C, S, eps, variant, res, dx2, alpha2);
-    else launch_bwd_cluster_as<RES, false>(cp, dx, part, dy, x, w, C, S, eps, variant, res, dx2, alpha2);
+    // (CL_EXACT with the residual: 126 of the 128 registers a lane has; [16][1024][256] 15.4 -> 14.7 us)
+    cluster_whole(cp, [&](auto whole) {
+        launch_bwd_cluster_as<RES, decltype(whole)::value>(cp, dx, part, dy, x, w, C, S, eps, variant, res, dx2, alpha2);
+    });
 }
 
 }   // namespace

@@ -74,15 +74,16 @@ struct StoreBf16 {
 };
 static_assert(CL_SLOT_STRIDE >= 2 * CL_LPR * StoreBf16::VEC, "two quantities per column must fit a workgroup's slots");
 
-// The first read of an operand's rows.  A cache line that holds the end of one row piece and the start of another is asked for
-// twice, and again by the workgroup of the next strip, so the loads leave it in the caches: nontemporal ones took, for the
-// backward of fp32 [22][1024][147] and [115][768][54], 18.5 and 27.3 us for 15.2 and 21.7, of bfloat16 [8][768][197] 10.8 for
-// 10.0, and of fp32 [16][1024][256], where pieces are whole lines, no less either (11.7, 11.6).  Whole pieces of bfloat16 alone
-// are read past the caches ([16][1024][256] 12.8 for 13.2 us, forward 7.1 for 7.2).
-template <typename ST, bool EXACT>
-__device__ __forceinline__ typename ST::Raw cluster_load(const typename ST::T *p) {
-    return EXACT && sizeof(typename ST::T) == 2 ? ST::load_nt(p) : ST::load(p);
-}
+// The first read of an operand's rows: past the caches where rows are whole 128-byte lines, through them otherwise (first_loads in
+// tile.h).  Cold operands, us, past / through: backward of fp32 [16][1024][256] 11.4 / 12.0, [32][1024][256] 23.5 / 25.2, with the
+// residual 34.8 / 36.4, [32][768][256] with it 25.6 / 28.0; [22][1024][147] 18.0 / 15.9, [8][768][197] 9.2 / 8.3, with the residual
+// 10.3 / 9.2, [115][768][54] with it 21.4 / 22.5 (20.1 of operands that the last-level cache holds); bfloat16 [32][768][256] with the
+// residual 17.1 / 19.9, [22][1024][147] 14.4 / 12.6.
+// CL_EXACT: every member holds exactly RPS*RPT rows and every strip is whole; CL_LINES: rows are whole lines; CL_ANY: neither.  (One
+// kernel with the loads written twice behind a branch took 27.9 us for the 25.4 of [32][768][256].)
+enum { CL_ANY, CL_LINES, CL_EXACT };
+template <typename ST, int WHOLE>
+__device__ __forceinline__ typename ST::Raw cluster_load(const typename ST::T *p) { return WHOLE != CL_ANY ? ST::load_nt(p) : ST::load(p); }
 
 // Per-thread partial sums acc[q][j] (q < NV quantities, j < VEC columns of this lane) -> per-column sums of the
 // workgroup in wsum[q*W + column], valid for all threads after the barrier.  lds: NW*NV*W floats.
@@ -185,18 +186,19 @@ __device__ __forceinline__ ClusterGeo cluster_geo(int nblk, int csplit, int stri
 
 // FUSE: y = a + alpha*b is formed first (and stored), and the norm is taken of it — the residual add and the
 // RMSNorm that follows it (training/training_dynamic/train.m:460-461).  Otherwise x = a and b, y_res are unused.
-// EXACT: every member holds exactly RPS*RPT rows and every strip is whole.  Then no row or column needs a mask and
+// WHOLE = CL_EXACT: every member holds exactly RPS*RPT rows and every strip is whole.  Then no row or column needs a mask and
 // the loads of the tile are issued back to back without branches, which is worth 0.45 us of the 8 us that the
 // forward kernel takes on fp32 [16][1024][256].  In other shapes lanes without a row or without columns load valid ones and
 // only their values are dropped, which is still quicker than branches: bfloat16 [5][1024][570] forward 8.0 -> 7.6, with the
 // residual 10.7 -> 10.4, backward 12.2 -> 12.0, with it 14.0 -> 13.7; fp32 [115][768][54] with the residual 21.2 -> 20.1.
-template <typename ST, int RPT, int THREADS, bool FUSE, bool EXACT>
+template <typename ST, int RPT, int THREADS, bool FUSE, int WHOLE>
 __global__ __launch_bounds__(THREADS) void rms_fwd_cluster_kernel(typename ST::T *__restrict__ yn, typename ST::T *y_res,
                                                                   const typename ST::T *a, const typename ST::T *b,
                                                                   float alpha, const float *__restrict__ w, int C,
                                                                   int S, int strips, int nblk, int csplit, int rows_pm,
                                                                   float eps, float invC, ClusterWs ws,
                                                                   int spin_ticks) {
+    constexpr bool EXACT = WHOLE == CL_EXACT;
     constexpr int VEC = ST::VEC;
     constexpr int W = CL_LPR * VEC;
     constexpr int RPS = THREADS / CL_LPR;
@@ -224,13 +226,13 @@ __global__ __launch_bounds__(THREADS) void rms_fwd_cluster_kernel(typename ST::T
         const size_t off = slab_base + (size_t)c * S;
         if constexpr (FUSE) {
             float av[VEC], bv[VEC], v[VEC];
-            ST::widen(av, first ? cluster_load<ST, EXACT>(a + off) : ST::load(a + off));
-            ST::widen(bv, first ? cluster_load<ST, EXACT>(b + off) : ST::load(b + off));
+            ST::widen(av, first ? cluster_load<ST, WHOLE>(a + off) : ST::load(a + off));
+            ST::widen(bv, first ? cluster_load<ST, WHOLE>(b + off) : ST::load(b + off));
 #pragma unroll
             for (int j = 0; j < VEC; j++) v[j] = bv[j] * alpha + av[j];
             return ST::pack(v);
         } else {
-            return first ? cluster_load<ST, EXACT>(a + off) : ST::load(a + off);
+            return first ? cluster_load<ST, WHOLE>(a + off) : ST::load(a + off);
         }
     };
 
@@ -305,7 +307,7 @@ __global__ __launch_bounds__(THREADS) void rms_fwd_cluster_kernel(typename ST::T
 
 // RES: dx = rmsnorm_bwd(dy, x, w) + res and optionally dx2 = alpha2*dx (training/training_dynamic/train.m:586-595,
 // :714-721), as rms_bwd_res_kernel of norm.hip.  dw partials: part[cluster][c], one row per cluster.
-template <typename ST, int RPT, int THREADS, bool RES, bool EXACT>
+template <typename ST, int RPT, int THREADS, bool RES, int WHOLE>
 __global__ __launch_bounds__(THREADS) void rms_bwd_cluster_kernel(typename ST::T *dx, float *__restrict__ dw_part,
                                                                   const typename ST::T *dy,
                                                                   const typename ST::T *__restrict__ x,
@@ -314,6 +316,7 @@ __global__ __launch_bounds__(THREADS) void rms_bwd_cluster_kernel(typename ST::T
                                                                   float eps, float invC, int variant,
                                                                   const typename ST::T *res, typename ST::T *dx2,
                                                                   float alpha2, ClusterWs ws, int spin_ticks) {
+    constexpr bool EXACT = WHOLE == CL_EXACT;
     constexpr int VEC = ST::VEC;
     constexpr int W = CL_LPR * VEC;
     constexpr int RPS = THREADS / CL_LPR;
@@ -343,9 +346,9 @@ __global__ __launch_bounds__(THREADS) void rms_bwd_cluster_kernel(typename ST::T
         const bool live = EXACT || row_live(g.member, k);
         const int c = live ? row_of(g.member, k) : 0;
         const size_t off = slab_base + (size_t)c * S;
-        xr[k] = cluster_load<ST, EXACT>(x + off);
-        dr[k] = cluster_load<ST, EXACT>(dy + off);
-        if constexpr (RES) rr_res[k] = cluster_load<ST, EXACT>(res + off);
+        xr[k] = cluster_load<ST, WHOLE>(x + off);
+        dr[k] = cluster_load<ST, WHOLE>(dy + off);
+        if constexpr (RES) rr_res[k] = cluster_load<ST, WHOLE>(res + off);
         wv[k] = w[c];
         if (!live) xr[k] = ST::zero();
     }
@@ -458,9 +461,9 @@ __global__ __launch_bounds__(THREADS) void rms_bwd_cluster_kernel(typename ST::T
 // How a shape is split: csplit members of rows_pm rows each; rpt rows per lane.  csplit = 0: not clustered.
 struct ClusterPlan {
     int csplit, rows_pm, rpt, threads, strips, nblk;
-    bool exact;        // every member holds exactly rps*rpt rows and every strip is whole: the unmasked kernels
+    int whole;         // which kernel: CL_EXACT, CL_LINES or CL_ANY
 };
-constexpr ClusterPlan NO_CLUSTER = {0, 0, 0, 0, 0, 0, false};
+constexpr ClusterPlan NO_CLUSTER = {0, 0, 0, 0, 0, 0, CL_ANY};
 
 // Clustering pays when whole-C strips of 256 bytes would leave most compute units idle: tall tensors
 // (C >= 512) whose strips number fewer than the compute units.  Measured at C = 1024, fp32, with 32 x 256 and
@@ -497,8 +500,14 @@ ClusterPlan cluster_plan(int C, int S, int batch, bool vec_ok, int vec, int rpt_
     p.threads = threads;
     p.strips = (int)strips;
     p.nblk = (int)(clusters * split);
-    p.exact = rows == rps * rpt && rows * split == C && S % w == 0;
+    p.whole = rows == rps * rpt && rows * split == C && S % w == 0 ? CL_EXACT : S % (w / 2) == 0 ? CL_LINES : CL_ANY;
     return p;
+}
+template <typename F>
+void cluster_whole(const ClusterPlan &p, F as) {
+    if (p.whole == CL_EXACT) as(std::integral_constant<int, CL_EXACT>());
+    else if (p.whole == CL_LINES) as(std::integral_constant<int, CL_LINES>());
+    else as(std::integral_constant<int, CL_ANY>());
 }
 
 }   // namespace

@@ -2,6 +2,8 @@
 #pragma once
 #include "common.h"
 
+#include <type_traits>
+
 template <int VEC>
 __device__ __forceinline__ void ldv(float (&r)[VEC], const float *p) {
     if constexpr (VEC == 4) {
@@ -38,6 +40,22 @@ __device__ __forceinline__ void stv(float *p, const float (&r)[VEC]) {
     } else {
         *p = r[0];
     }
+}
+
+// The first loads of a tile that one workgroup holds: past the caches where rows are whole 128-byte lines, through them where a line
+// that holds the end of one row piece and the start of another is asked for twice.  RMSNorm of cold operands, past the caches
+// always / this: bfloat16 [115][768][54] forward 9.0 / 8.1 us, backward 13.2 / 11.5, with the residual 19.3 / 17.5, [64][1024][256]
+// 15.4 / 13.8, 25.0 / 22.8, 42.2 / 39.4; fp32 backward [115][768][54] 27.2 / 25.7, [22][1024][147] 18.0 / 16.1.  The other fp32 tiles
+// stay past the caches: forward no difference, with the residual [115][768][54] 21.5 / 24.2.
+template <typename F>
+__device__ __forceinline__ void first_loads(bool lines, F load) {
+    if (lines) load(std::true_type());
+    else load(std::false_type());
+}
+template <int VEC, bool LINES>
+__device__ __forceinline__ void ldv_first(float (&r)[VEC], const float *p) {
+    if constexpr (LINES) ldv_nt<VEC>(r, p);
+    else ldv<VEC>(r, p);
 }
 
 // The columns of a lane whose strip gives it columns nominal .. nominal+VEC-1 of rows of S columns (S >= VEC).  Where

@@ -35,17 +35,17 @@ STREAM_LAUNCH_MS, STREAM_RATE_BYTES_PER_MS = 0.0035, 6.97e9      # measured: one
 # here; this file holds none of them.  An op's traffic is the sum over the kernels it launches, each with a weight
 # (the weight-gradient reduction is shared by the two backward ops that queue it).
 OP_KERNELS = {
-    "rmsnorm_fwd": [("rms_fwd_cluster_kernel<StoreF32, 4, 1024, false, true>", 1.0)],
-    "rmsnorm_bwd": [("rms_bwd_cluster_kernel<StoreF32, 4, 1024, false, true>", 1.0), ("reduce_jobs_kernel", 0.5)],
+    "rmsnorm_fwd": [("rms_fwd_cluster_kernel<StoreF32, 4, 1024, false, 2>", 1.0)],
+    "rmsnorm_bwd": [("rms_bwd_cluster_kernel<StoreF32, 4, 1024, false, 2>", 1.0), ("reduce_jobs_kernel", 0.5)],
     "qknorm_rope_fwd": [("qknorm_rope_fwd_kernel<16, 256, 4>", 1.0)],
-    "qknorm_rope_bwd": [("qknorm_rope_bwd_kernel<16, 512, 2>", 1.0)],
+    "qknorm_rope_bwd": [("qknorm_rope_bwd_kernel<16, 512, 2, true>", 1.0)],
     "swiglu_fwd": [("swiglu_fwd_kernel<1>", 1.0)],
     "swiglu_bwd": [("swiglu_bwd_kernel<1>", 1.0)],
     "residual": [("axpby_kernel<0, 1>", 1.0)],
-    "residual_rmsnorm_fwd": [("rms_fwd_cluster_kernel<StoreF32, 4, 1024, true, true>", 1.0)],
-    "rmsnorm_bwd_residual": [("rms_bwd_cluster_kernel<StoreF32, 4, 1024, true, false>", 1.0)],
+    "residual_rmsnorm_fwd": [("rms_fwd_cluster_kernel<StoreF32, 4, 1024, true, 2>", 1.0)],
+    "rmsnorm_bwd_residual": [("rms_bwd_cluster_kernel<StoreF32, 4, 1024, true, 2>", 1.0)],
     "scale_copy": [("axpby_kernel<1, 1>", 1.0)],
-    "softmax_ce": [("ce_resident_kernel<CrF32, 16, 9, true>", 1.0)],
+    "softmax_ce": [("ce_resident_kernel<CrF32, 16, 9, true, 64>", 1.0)],
     "int8_scale": [("absmax_scale_kernel", 1.0)],
     "int8_quant": [("quant_kernel<1>", 1.0)],
     "int8_dequant": [("dequant_kernel<1>", 1.0)],
@@ -54,9 +54,9 @@ OP_KERNELS = {
 # the three launches of the ordered scatter-add in its column form and in its row form, and
 # the gather
 EMBED_KERNELS = {
-    "scatter_cols": [("chunk_sort_blk_kernel", 1.0), ("block_rank_kernel", 1.0), ("col_sum_kernel<3, true, false>", 1.0)],
+    "scatter_cols": [("chunk_sort_blk_kernel", 1.0), ("block_rank_kernel<1>", 1.0), ("col_sum_kernel<3, true, false>", 1.0)],
     "scatter_rows": [("chunk_sort_kernel", 1.0), ("rank_transpose_kernel", 1.0), ("seg_sum_kernel<false>", 1.0)],
-    "gather": [("gather_kernel<true>", 1.0)],
+    "gather": [("gather_kernel<true, 64, 64>", 1.0)],
 }
 
 
