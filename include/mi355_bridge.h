@@ -471,8 +471,8 @@ int mi355_vocab_scatter_grads_dev(float *full_grad, const float *compact_grad, c
 
 /* ------------------------------------------------------------------------------------------
  * Host-pointer drop-ins: the reference signatures verbatim (host float* in, host float* out),
- * so a caller swaps the symbol only.  Each call stages through cached device buffers
- * (H2D, kernel, D2H) and returns when the result is in host memory.  On failure they print one
+ * so a caller swaps the symbol only.  Each call stages through a pinned block of at most 32 MB, which three threads of the
+ * library help to fill and empty, and cached device buffers (H2D, kernel, D2H) and returns when the result is in host memory.  On failure they print one
  * line to stderr and leave the outputs untouched.
  * ---------------------------------------------------------------------------------------- */
 /* rmsnorm — training/stories_cpu_ops.h:6 */
