@@ -14,7 +14,14 @@
 
 namespace {
 
-template <int LPR, int THREADS, int CAP>
+// ROWS: the tile holds every row pair of the head and nothing else; rows are not whole cache lines.  Then lanes past the end of a row
+// load its last columns again, no load is behind a condition, and lines that two pieces share stay in the caches.  us, before / with:
+// [22][24 x 128][147] forward 29.5 / 23.7 (cold operands 30.1 / 27.8), backward 41.1 / 32.6 (40.3 / 33.9); [5][570] 25.2 / 19.8 (25.3 /
+// 22.7) and 32.7 / 26.3 (32.0 / 28.8); [2][197] 7.7 / 5.4 and 8.5 / 7.3.
+template <bool ROWS>
+__device__ __forceinline__ v4f qk_load(const float *p) { return ROWS ? ld4(p) : ld4_nt(p); }
+
+template <int LPR, int THREADS, int CAP, bool ROWS = false>
 __global__ __launch_bounds__(THREADS) void qknorm_rope_fwd_kernel(
     float *__restrict__ q_out, float *__restrict__ k_out, const float *__restrict__ q, const float *__restrict__ k,
     const float *__restrict__ wq, const float *__restrict__ wk, int hd, int S, int strips, int nq,
@@ -30,7 +37,7 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_fwd_kernel(
     else { blk -= nq; in = k; out = k_out; w = wk; }
     const int slab = blk / strips, strip = blk - slab * strips;
     const int lc = threadIdx.x % LPR, p0 = threadIdx.x / LPR;
-    const LaneCols mine = lane_cols<4>(strip * W + lc * 4, S);
+    const LaneCols mine = ROWS ? lane_cols_inside<4, W>(strip * W + lc * 4, S) : lane_cols<4>(strip * W + lc * 4, S);
     const int col = mine.col;
     const bool col_ok = mine.ok;
     const int half = hd >> 1;
@@ -42,10 +49,10 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_fwd_kernel(
 #pragma unroll
     for (int kk = 0; kk < CAP; kk++) {
         const int rp = p0 + kk * PPS;
-        if (rp < half && col_ok) {
+        if (ROWS || (rp < half && col_ok)) {
             const float *px = in + base + (size_t)(2 * rp) * S;
-            x0[kk] = ld4_nt(px);
-            x1[kk] = ld4_nt(px + S);
+            x0[kk] = qk_load<ROWS>(px);
+            x1[kk] = qk_load<ROWS>(px + S);
             w0[kk] = w[2 * rp];
             w1[kk] = w[2 * rp + 1];
         } else {
@@ -68,27 +75,31 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_fwd_kernel(
 #pragma unroll
     for (int kk = 0; kk < CAP; kk++) {
         const int rp = p0 + kk * PPS;
-        if (rp < half && col_ok) {
+        if (ROWS || (rp < half && col_ok)) {
             // the tables are shared by every head and sequence (cache-resident): read here, after the reduction,
             // rather than held in registers across it
             const v4f cs = ld4(cos_t + (size_t)rp * S + col), sn = ld4(sin_t + (size_t)rp * S + col);
             const v4f y0 = (x0[kk] * rr) * w0[kk];
             const v4f y1 = (x1[kk] * rr) * w1[kk];
             float *po = out + base + (size_t)(2 * rp) * S;
-            st4_nt(po, y0 * cs - y1 * sn);
-            st4_nt(po + S, y0 * sn + y1 * cs);
+            if (!ROWS || col_ok) {
+                st4_nt(po, y0 * cs - y1 * sn);
+                st4_nt(po + S, y0 * sn + y1 * cs);
+            }
         }
     }
 }
 
+enum { QK_SOME, QK_ROWS, QK_ALL };
 // EXACT: the tile holds every row pair of the head and nothing else, every strip is whole: no load or store is behind a condition
 // ([16][24 x 128][256] 32.4 -> 31.5 us).  (The forward is slower so, 20.3 -> 21.5: fewer registers, more workgroups at a time.)
-template <int LPR, int THREADS, int CAP, bool EXACT = false>
+template <int LPR, int THREADS, int CAP, int WHOLE = QK_SOME>
 __global__ __launch_bounds__(THREADS) void qknorm_rope_bwd_kernel(
     float *dq, float *dk, float *__restrict__ part, const float *dq_out, const float *dk_out,
     const float *__restrict__ q, const float *__restrict__ k, const float *__restrict__ wq,
     const float *__restrict__ wk, int hd, int S, int strips, int nq, const float *__restrict__ cos_t,
     const float *__restrict__ sin_t, float eps, float invhd, int variant) {
+    constexpr bool EXACT = WHOLE == QK_ALL, ROWS = WHOLE == QK_ROWS;
     constexpr int PPS = THREADS / LPR;
     constexpr int W = LPR * 4;
     constexpr int NW = THREADS / 64;
@@ -101,7 +112,7 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_bwd_kernel(
     else { blk -= nq; gin = dk_out; xin = k; out = dk; w = wk; }
     const int slab = blk / strips, strip = blk - slab * strips;
     const int lc = threadIdx.x % LPR, p0 = threadIdx.x / LPR;
-    const LaneCols mine = lane_cols<4>(strip * W + lc * 4, S);
+    const LaneCols mine = ROWS ? lane_cols_inside<4, W>(strip * W + lc * 4, S) : lane_cols<4>(strip * W + lc * 4, S);
     const int col = mine.col;
     const bool col_ok = mine.ok;
     const int half = hd >> 1;
@@ -113,11 +124,11 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_bwd_kernel(
 #pragma unroll
     for (int kk = 0; kk < CAP; kk++) {
         const int rp = p0 + kk * PPS;
-        if (EXACT || (rp < half && col_ok)) {
+        if (EXACT || ROWS || (rp < half && col_ok)) {
             const size_t o = base + (size_t)(2 * rp) * S;
-            x0[kk] = ld4_nt(xin + o);
-            x1[kk] = ld4_nt(xin + o + S);
-            const v4f g0 = ld4_nt(gin + o), g1 = ld4_nt(gin + o + S);
+            x0[kk] = qk_load<ROWS>(xin + o);
+            x1[kk] = qk_load<ROWS>(xin + o + S);
+            const v4f g0 = qk_load<ROWS>(gin + o), g1 = qk_load<ROWS>(gin + o + S);
             const v4f c = ld4(cos_t + (size_t)rp * S + col), s = ld4(sin_t + (size_t)rp * S + col);
             d0[kk] = g0 * c + g1 * s;        // inverse rotation (cpu_ops.h:179-180)
             d1[kk] = (-g0) * s + g1 * c;
@@ -148,7 +159,7 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_bwd_kernel(
 #pragma unroll
     for (int kk = 0; kk < CAP; kk++) {
         const int rp = p0 + kk * PPS;
-        if (EXACT || rp < half) {   // uniform over each group of LPR lanes
+        if (EXACT || ROWS || rp < half) {   // uniform over each group of LPR lanes
             v4f o0, o1;
             if (variant == 0) {
                 o0 = ((d0[kk] - x0[kk] * dotn) * rr) * w0[kk];
@@ -227,6 +238,9 @@ bool pick_qk(int hd, int S, bool in_place, QkCfg &cfg, bool backward) {
         }                                                                                                     \
     } while (0)
 
+// Rows that are not whole 128-byte lines, on a tile that the head's row pairs fill (hd 128 and 64): the ROWS kernels.
+bool whole_rows(const QkCfg &cfg, int hd, int S) { return S % 32 != 0 && cfg.lpr == 16 && cfg.threads / 16 * cfg.cap * 2 == hd; }
+
 int check_shape(const char *who, int heads, int kv_heads, int hd, int S, int batch) {
     if (hd <= 0 || (hd & 1) || S <= 0 || batch <= 0 || heads < 0 || kv_heads < 0 || heads + kv_heads == 0)
         return mi355_fail("%s: bad shape heads=%d kv_heads=%d hd=%d S=%d batch=%d", who, heads, kv_heads, hd, S, batch);
@@ -251,8 +265,16 @@ MI355_API int mi355_qknorm_rope_fwd_dev(float *q_out, float *k_out, const float 
     }
     const int strips = (int)ceil_div((size_t)S, (size_t)cfg.lpr * 4);
     const int nq = batch * heads * strips, nk = batch * kv_heads * strips;
-    QK_DISPATCH(qknorm_rope_fwd_kernel, cfg, dim3(nq + nk), q_out, k_out, q, k, wq, wk, hd, S, strips, nq, cos_dev,
-                sin_dev, eps, 1.0f / (float)hd);
+    auto launch = [&](auto kernel, int threads) {
+        hipLaunchKernelGGL(kernel, dim3(nq + nk), dim3(threads), 0, g_ctx.stream, q_out, k_out, q, k, wq, wk, hd, S, strips, nq, cos_dev,
+                           sin_dev, eps, 1.0f / (float)hd);
+    };
+    const bool rows = whole_rows(cfg, hd, S);
+    if (rows && cfg.threads == 256 && cfg.cap == 4) launch(qknorm_rope_fwd_kernel<16, 256, 4, true>, 256);
+    else if (rows && cfg.threads == 256 && cfg.cap == 2) launch(qknorm_rope_fwd_kernel<16, 256, 2, true>, 256);
+    else
+        QK_DISPATCH(qknorm_rope_fwd_kernel, cfg, dim3(nq + nk), q_out, k_out, q, k, wq, wk, hd, S, strips, nq, cos_dev,
+                    sin_dev, eps, 1.0f / (float)hd);
     LAUNCH_OK("qknorm_rope_fwd");
     return 0;
 }
@@ -279,9 +301,15 @@ MI355_API int mi355_qknorm_rope_bwd_dev(float *dq, float *dk, float *dwq, float 
     const int nq = batch * heads * strips, nk = batch * kv_heads * strips;
     float *part = mi355_dw_partials((size_t)(nq + nk) * hd, nq > 0 ? dwq : nullptr, nk > 0 ? dwk : nullptr);
     if (!part) return -1;
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(nq + nk), dim3(512), 0, g_ctx.stream, dq, dk, part, dq_out, dk_out, q, k, wq, wk, hd, S, strips, nq,
+                           cos_dev, sin_dev, eps, 1.0f / (float)hd, variant);
+    };
+    const bool rows = whole_rows(cfg, hd, S);
     if (cfg.lpr == 16 && cfg.threads == 512 && cfg.cap == 2 && hd == 128 && S % 64 == 0)
-        hipLaunchKernelGGL((qknorm_rope_bwd_kernel<16, 512, 2, true>), dim3(nq + nk), dim3(512), 0, g_ctx.stream, dq, dk, part, dq_out,
-                           dk_out, q, k, wq, wk, hd, S, strips, nq, cos_dev, sin_dev, eps, 1.0f / (float)hd, variant);
+        launch(qknorm_rope_bwd_kernel<16, 512, 2, QK_ALL>);
+    else if (rows && cfg.threads == 512 && cfg.cap == 2) launch(qknorm_rope_bwd_kernel<16, 512, 2, QK_ROWS>);
+    else if (rows && cfg.threads == 512 && cfg.cap == 1) launch(qknorm_rope_bwd_kernel<16, 512, 1, QK_ROWS>);
     else
         QK_DISPATCH(qknorm_rope_bwd_kernel, cfg, dim3(nq + nk), dq, dk, part, dq_out, dk_out, q, k, wq, wk, hd, S, strips,
                     nq, cos_dev, sin_dev, eps, 1.0f / (float)hd, variant);

@@ -81,35 +81,38 @@ def test_rmsnorm_bwd_residual_whole_and_ragged_tiles(br, C, S, B, bf16):
 
 # whole rows of a tile beside columns that are not: one column in the last strip, the last group moved back over a strip's edge,
 # strips that end inside a group; in place where the tile allows it and where another takes over (S % 128 < 8)
+@pytest.mark.parametrize("bf16", [True, False])
 @pytest.mark.parametrize("hd,heads,kv,B,S", [(128, 16, 8, 9, 129), (128, 16, 8, 8, 147), (128, 16, 8, 4, 197), (128, 16, 8, 40, 33), (128, 16, 8, 60, 15),
                                              (64, 12, 12, 30, 131), (64, 12, 12, 30, 136), (128, 16, 8, 100, 8)])
-def test_qknorm_rope_bf16_ragged_strips(br, hd, heads, kv, B, S):
-    print("[case] qk strips hd=%d heads=%d kv=%d B=%d S=%d" % (hd, heads, kv, B, S), flush=True)
+def test_qknorm_rope_ragged_strips(br, hd, heads, kv, B, S, bf16):
+    print("[case] qk strips hd=%d heads=%d kv=%d B=%d S=%d bf16=%d" % (hd, heads, kv, B, S, bf16), flush=True)
+    end = "_bf16_dev" if bf16 else "_dev"
+    enc, dec = (to_bf, widen) if bf16 else (lambda a: np.array(a), lambda a: a)
     theta, eps = 1e6, 1e-5
     D = br.DevArray.from_numpy
     cos, sin = br.rope_tables_dev(S, hd, theta)
     wq, wk = H.normal(980, hd, 1.0, 0.02), H.normal(981, hd, 1.0, 0.02)
-    q, k = to_bf(H.normal(982, (B, heads * hd, S))), to_bf(H.normal(983, (B, kv * hd, S)))
-    gq, gk = to_bf(H.normal(984, (B, heads * hd, S))), to_bf(H.normal(985, (B, kv * hd, S)))
+    q, k = enc(H.normal(982, (B, heads * hd, S))), enc(H.normal(983, (B, kv * hd, S)))
+    gq, gk = enc(H.normal(984, (B, heads * hd, S))), enc(H.normal(985, (B, kv * hd, S)))
     qd, kd, wqd, wkd = (D(a) for a in (q, k, wq, wk))
-    guard = lambda a: D(np.concatenate([a.ravel(), np.full(64, 7, np.uint16)]))
-    tol = 2.0 ** -8 * 1.01          # one rounding to 8 bits on store
+    guard = lambda a: D(np.concatenate([a.ravel(), np.full(64, 7, a.dtype)]))
+    tol = 2.0 ** -8 * 1.01 if bf16 else 1e-5          # one rounding to 8 bits on store
     qo, ko = guard(np.zeros_like(q)), guard(np.zeros_like(k))
-    br.check(br.lib.mi355_qknorm_rope_fwd_bf16_dev(qo.ptr, ko.ptr, qd.ptr, kd.ptr, wqd.ptr, wkd.ptr, heads, kv, hd, S, B, cos, sin, eps))
+    br.check(getattr(br.lib, "mi355_qknorm_rope_fwd" + end)(qo.ptr, ko.ptr, qd.ptr, kd.ptr, wqd.ptr, wkd.ptr, heads, kv, hd, S, B, cos, sin, eps))
     for x, w, o in ((q, wq, qo), (k, wk, ko)):
         got = o.numpy()
-        assert err(widen(got[:x.size].reshape(x.shape)), O.qknorm_rope_fwd(widen(x), w, hd, theta, eps)) <= tol
+        assert err(dec(got[:x.size].reshape(x.shape)), O.qknorm_rope_fwd(dec(x), w, hd, theta, eps)) <= tol
         assert np.all(got[x.size:] == 7)
     for in_place in (False, True):
         gqd, gkd = guard(gq), guard(gk)
         dq, dk = (gqd, gkd) if in_place else (guard(np.zeros_like(q)), guard(np.zeros_like(k)))
         dwq, dwk = br.DevArray(hd), br.DevArray(hd)
-        br.check(br.lib.mi355_qknorm_rope_bwd_bf16_dev(dq.ptr, dk.ptr, dwq.ptr, dwk.ptr, gqd.ptr, gkd.ptr, qd.ptr, kd.ptr, wqd.ptr, wkd.ptr,
+        br.check(getattr(br.lib, "mi355_qknorm_rope_bwd" + end)(dq.ptr, dk.ptr, dwq.ptr, dwk.ptr, gqd.ptr, gkd.ptr, qd.ptr, kd.ptr, wqd.ptr, wkd.ptr,
                                                        heads, kv, hd, S, B, cos, sin, eps, 0))
         for x, g, w, dx, dw in ((q, gq, wq, dq, dwq), (k, gk, wk, dk, dwk)):
-            rdx, rdw = O.qknorm_rope_bwd(widen(g), widen(x), w, hd, theta, eps)
+            rdx, rdw = O.qknorm_rope_bwd(dec(g), dec(x), w, hd, theta, eps)
             got = dx.numpy()
-            assert err(widen(got[:x.size].reshape(x.shape)), rdx) <= tol
+            assert err(dec(got[:x.size].reshape(x.shape)), rdx) <= tol
             assert np.all(got[x.size:] == 7)
             assert err(dw.numpy(), rdw) <= 1e-5
 
