@@ -358,7 +358,10 @@ __global__ __launch_bounds__(THREADS) void rms_bwd_cluster_kernel(typename ST::T
         dr[k] = cluster_load<ST, WHOLE>(dy + off);
         if constexpr (RES) rr_res[k] = cluster_load<ST, WHOLE>(res + off);
         wv[k] = w[c];
-        if (!live) xr[k] = ST::zero();
+        if (!live) {                  // (all three: an infinity in the row read instead would make 0 * inf of the sum)
+            xr[k] = dr[k] = ST::zero();
+            wv[k] = 0.f;
+        }
     }
     float acc[2][VEC];      // [0] = sum x^2, [1] = sum (dy*x)*w
 #pragma unroll

@@ -148,3 +148,29 @@ def test_rmsnorm_ragged_clusters(br, C, S, B, bf16):
     rdx, rdw = O.rmsnorm_bwd(dec(dy), dec(x), w)
     check(dx, rdx.reshape(x.shape))
     assert err(dw.numpy(), rdw) <= 1e-5
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("res", [False, True])
+@pytest.mark.parametrize("C,S,B", [(768, 129, 3), (768, 256, 2), (513, 131, 2)])
+def test_rmsnorm_bwd_clusters_pass_infinities_on(br, C, S, B, res, bf16):
+    """Lanes without a row read row 0: an infinity there must not become a NaN in a sum that it would only make infinite."""
+    print("[case] rmsnorm_bwd infinities C=%d S=%d B=%d res=%d bf16=%d" % (C, S, B, res, bf16), flush=True)
+    end = "_bf16_dev" if bf16 else "_dev"
+    enc, dec = (to_bf, widen) if bf16 else (lambda a: np.array(a), lambda a: a)
+    x, dy, r = (enc(H.normal(995 + i, (B, C, S))) for i in range(3))
+    dy[0, 0, 5] = enc(np.array([np.inf], np.float32))[0]
+    dy[B - 1, 0, S - 1] = enc(np.array([-np.inf], np.float32))[0]
+    w = H.normal(998, C, 1.0, 0.02)
+    D = br.DevArray.from_numpy
+    xd, dyd, rd, wd, dx, dw = D(x), D(dy), D(r), D(w), br.DevArray(x.shape, x.dtype), br.DevArray(C)
+    if res:
+        br.check(getattr(br.lib, "mi355_rmsnorm_bwd_residual" + end)(dx.ptr, None, dw.ptr, dyd.ptr, xd.ptr, wd.ptr, rd.ptr, 0.25, C, S, B, 1e-5, 0))
+    else:
+        br.check(getattr(br.lib, "mi355_rmsnorm_bwd" + end)(dx.ptr, dw.ptr, dyd.ptr, xd.ptr, wd.ptr, C, S, B, 1e-5, 0))
+    with np.errstate(invalid="ignore"):
+        rdx, _ = O.rmsnorm_bwd(dec(dy), dec(x), w)
+        want = rdx.reshape(x.shape) + (dec(r) if res else np.float32(0))
+    got = dec(dx.numpy())
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isposinf(got), np.isposinf(want))
+    assert np.array_equal(np.isneginf(got), np.isneginf(want))
