@@ -407,7 +407,10 @@ __global__ __launch_bounds__(R_THREADS) void sgemm_rows_kernel(const float *__re
     auto read_a = [&](int ks, int i, int q) {
         a[q] = *reinterpret_cast<const bf8_t *>(lds + (size_t)ks * (FM * 3 * P_FRAG) + slot(ks, quarter, li) + (i * 3 + q) * P_FRAG);
     };
-    // (rows and columns past the end are out of the buffer's range: not read, not written)
+    // Rows and columns past the end are out of the buffer's range: not read, not written.  The range check compares the vector
+    // offset, so the row is part of that; whether the scalar offset counts too is not the same in every description of it.
+    // (96 rows of 2^22 columns end below 2^31, and 2^31 and a row more stays below 2^32.)
+    auto row = [&](int i, int e) { return (unsigned)((16 * i + e) * ldc) * 4u; };
     auto finish = [&](int u) __attribute__((always_inline)) {
         const int n = u * 32 + FN * li;
         const unsigned at = n + 1 < N ? (unsigned)(4 * quarter * ldc + n) * 4u : 1u << 31;
@@ -417,13 +420,13 @@ __global__ __launch_bounds__(R_THREADS) void sgemm_rows_kernel(const float *__re
             if (read) {
 #pragma unroll
                 for (int e = 0; e < 4; e++)
-                    c[e] = __builtin_bit_cast(v2f, __builtin_amdgcn_raw_buffer_load_b64(out, at, (16 * i + e) * ldc * 4, 0));
+                    c[e] = __builtin_bit_cast(v2f, __builtin_amdgcn_raw_buffer_load_b64(out, at + row(i, e), 0, 0));
             }
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 v2f v = {acc[i][0][e] * alpha, acc[i][1][e] * alpha};
                 if (read) v += beta * c[e];
-                __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u, v), out, at, (16 * i + e) * ldc * 4, 0);
+                __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u, v), out, at + row(i, e), 0, 0);
             }
         }
         if ((N & 1) && u * 32 + 32 > N) {                        // a last column without a neighbour
@@ -433,8 +436,8 @@ __global__ __launch_bounds__(R_THREADS) void sgemm_rows_kernel(const float *__re
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     float v = acc[i][0][e] * alpha;
-                    if (read) v += beta * __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(out, last, (16 * i + e) * ldc * 4, 0));
-                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), out, last, (16 * i + e) * ldc * 4, 0);
+                    if (read) v += beta * __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(out, last + row(i, e), 0, 0));
+                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), out, last + row(i, e), 0, 0);
                 }
         }
     };

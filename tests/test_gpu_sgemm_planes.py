@@ -135,3 +135,32 @@ def test_many_columns_in_ranges(br):
     for knob in (7, 8):
         got = product(br, knob, A, B, 0, 0, 1.0, 0.5, C0)
         assert np.all(np.abs(got - want) <= 7 * 5 * 2.0 ** -23 * mag + 3 * 2.0 ** -24 * (np.abs(want) + np.abs(C0)))
+
+
+@pytest.mark.parametrize("knob", KNOBS)
+@pytest.mark.parametrize("M", [1, 2, 65, 66, 97, 98, 127, 191])
+def test_planes_write_nothing_outside_c(br, M, knob):
+    """Last blocks of 1, 2, 63 and 95 rows: a whole block of rows in front of C and one behind its last row keep their values, and
+    what lies there is not read either (it would make a NaN of a sum)."""
+    for N, beta, pad in ((70, 0.0, 0), (70, 1.5, 3), (33, 1.5, 0), (300, 0.0, 5)):
+        K, ldc, guard = 100, N + pad, 96 * (N + pad)
+        print("[case] sgemm planes guards M=%d N=%d knob=%d beta=%g pad=%d" % (M, N, knob, beta, pad), flush=True)
+        A = H.normal(760, (M, K)); B = H.normal(761, (K, N)); C0 = H.normal(762, (M, N))
+        inside = np.full((M, ldc), np.nan, np.float32)
+        inside[:, :N] = C0 if beta else np.nan
+        fence = np.full(guard, np.nan, np.float32)
+        buf = br.DevArray.from_numpy(np.concatenate([fence, inside.ravel(), fence]))
+        ad, bd = br.DevArray.from_numpy(A), br.DevArray.from_numpy(B)
+        br.tune("gemm_split", knob)
+        try:
+            br.check(br.lib.mi355_sgemm_dev(0, 0, M, N, K, 1.0, ad.ptr, K, bd.ptr, N, beta, buf.ptr + 4 * guard, ldc))
+            got = buf.numpy()
+        finally:
+            br.tune("gemm_split", 0)
+        same = lambda a: np.array_equal(a.view(np.uint32), np.full(a.size, fence[:1].view(np.uint32)[0]))
+        out = got[guard:guard + M * ldc].reshape(M, ldc)
+        assert same(got[:guard]) and same(got[guard + M * ldc:]) and same(np.ascontiguousarray(out[:, N:]).ravel())
+        mag = np.abs(A.astype(np.float64)) @ np.abs(B.astype(np.float64))
+        want = A.astype(np.float64) @ B.astype(np.float64) + beta * C0
+        bound = (7 * (K // 32 + 2) + 2) * 2.0 ** -23 * mag + 3 * 2.0 ** -24 * (np.abs(want) + beta * np.abs(C0))
+        assert np.all(np.abs(out[:, :N] - want) <= bound)
