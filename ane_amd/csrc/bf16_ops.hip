@@ -452,14 +452,16 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_bwd_bf16_kernel(
         unpack<VEC>(g0, rg0[kk]);
         unpack<VEC>(g1, rg1[kk]);
         // (from a valid address in every lane: with the loads under a branch the compiler merges the two paths through
-        // scratch memory, and a kernel with scratch is dispatched later; a masked lane's gradients are zero)
-        const size_t to = WHOLE || (rp < half && col_ok) ? (size_t)rp * S + col : 0;
+        // scratch memory, and a kernel with scratch is dispatched later; what a masked lane makes of it is dropped, since zero
+        // times an infinity of the table is a NaN)
+        const bool ok = WHOLE || (rp < half && col_ok);
+        const size_t to = ok ? (size_t)rp * S + col : 0;
         ldtab<VEC>(c, cos_t + to);
         ldtab<VEC>(sn, sin_t + to);
 #pragma unroll
         for (int j = 0; j < VEC; j++) {
-            d0[j] = __builtin_fmaf(g0[j], c[j], g1[j] * sn[j]);
-            d1[j] = __builtin_fmaf(-g0[j], sn[j], g1[j] * c[j]);
+            d0[j] = ok ? __builtin_fmaf(g0[j], c[j], g1[j] * sn[j]) : 0.f;
+            d1[j] = ok ? __builtin_fmaf(-g0[j], sn[j], g1[j] * c[j]) : 0.f;
         }
     };
 

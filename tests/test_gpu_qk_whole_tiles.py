@@ -174,3 +174,32 @@ def test_rmsnorm_bwd_clusters_pass_infinities_on(br, C, S, B, res, bf16):
     got = dec(dx.numpy())
     assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isposinf(got), np.isposinf(want))
     assert np.array_equal(np.isneginf(got), np.isneginf(want))
+
+
+# an infinity in the table's first value reaches the column and the row pair that it belongs to, also where lanes without a row pair or
+# without columns (heads and strips that do not fill the tile) load the table's first values in place of none
+@pytest.mark.parametrize("bf16", [True, False])
+@pytest.mark.parametrize("hd,heads,kv,B,S", [(96, 8, 8, 9, 256), (96, 8, 8, 9, 100), (40, 8, 4, 9, 200), (192, 4, 4, 9, 72), (128, 2, 1, 1, 33), (128, 16, 8, 9, 129), (6, 3, 1, 2, 9)])
+def test_qknorm_rope_bwd_infinite_table_value_stays_in_its_column(br, hd, heads, kv, B, S, bf16):
+    print("[case] qk table hd=%d heads=%d kv=%d B=%d S=%d bf16=%d" % (hd, heads, kv, B, S, bf16), flush=True)
+    end = "_bf16_dev" if bf16 else "_dev"
+    enc, dec = (to_bf, widen) if bf16 else (lambda a: np.array(a), lambda a: a)
+    D = br.DevArray.from_numpy
+    angle = H.normal(990, (hd // 2, S))
+    wq, wk = H.normal(991, hd, 1.0, 0.02), H.normal(992, hd, 1.0, 0.02)
+    ops = [enc(H.normal(993 + i, (B, n * hd, S))) for i, n in enumerate((heads, kv, heads, kv))]
+    gq, gk, q, k = ops
+    gqd, gkd, qd, kd, wqd, wkd = (D(a) for a in (gq, gk, q, k, wq, wk))
+    res = []
+    for first in (np.float32(0.5), np.float32(np.inf)):
+        cos, sin = np.cos(angle).astype(np.float32), np.sin(angle).astype(np.float32)
+        cos[0, 0] = first
+        cd, sd = D(cos), D(sin)
+        dq, dk, dwq, dwk = br.DevArray(q.shape, q.dtype), br.DevArray(k.shape, k.dtype), br.DevArray(hd), br.DevArray(hd)
+        br.check(getattr(br.lib, "mi355_qknorm_rope_bwd" + end)(dq.ptr, dk.ptr, dwq.ptr, dwk.ptr, gqd.ptr, gkd.ptr, qd.ptr, kd.ptr, wqd.ptr, wkd.ptr,
+                                                                heads, kv, hd, S, B, cd.ptr, sd.ptr, 1e-5, 0))
+        res.append([a.numpy() for a in (dq, dk, dwq, dwk)])
+    for i in (0, 1):
+        assert res[0][i][..., 1:].tobytes() == res[1][i][..., 1:].tobytes()
+        assert res[0][2 + i][2:].tobytes() == res[1][2 + i][2:].tobytes()
+        assert np.all(np.isfinite(res[0][2 + i])) and not np.any(np.isfinite(dec(res[1][i][..., 0])))
