@@ -236,6 +236,7 @@ MI355_API int mi355_tune_set(const char *key, int value) {
         {"gemm_splitk", &g_ctx.gemm_splitk}, {"gemm_split", &g_ctx.gemm_split}, {"scatter_tree", &g_ctx.scatter_tree}, {"scatter_cols", &g_ctx.scatter_cols},
         {"rms_cluster", &g_ctx.rms_cluster}, {"rms_cluster_spin", &g_ctx.rms_cluster_spin},
         {"ce_resident", &g_ctx.ce_resident}, {"xch_take_nothing", &g_ctx.xch_take_nothing},
+        {"host_stage", &g_ctx.host_stage}, {"host_stage_fail", &g_ctx.host_stage_fail},
     };
     for (auto &t : tab)
         if (strcmp(t.k, key) == 0) { *t.v = value; g_coop_rebase = true; return 0; }

@@ -1,11 +1,13 @@
 // host_dropins.hip — host-pointer entry points with the reference's own signatures.
 //
-// Each brings its operands to the device, runs the kernels and returns when the result is in host memory (host_stage.h), so a caller of the reference's CPU ops swaps the symbol only:
+// Each brings its operands to the device, runs the kernels and returns when the result is in host memory
+// (host_stage.h), so a caller of the reference's CPU ops swaps the symbol only:
 //   rmsnorm / rmsnorm_bwd            training/stories_cpu_ops.h:6-53
 //   cross_entropy_loss               training/stories_cpu_ops.h:71-108, training/training_dynamic/cpu_ops.h:68-93
 //   embed_lookup / embed_backward    training/stories_cpu_ops.h:112-131
 //   rope_backward_inplace            training/training_dynamic/cpu_ops.h:168-184
-// Failures print one "mi355_bridge: ..." line and leave the outputs untouched.
+// Failures print one "mi355_bridge: ..." line and leave arrays that are updated in place untouched, and all others unless it was
+// the copy back that failed.
 #include "common.h"
 
 #include <emmintrin.h>
@@ -302,20 +304,7 @@ MI355_API void mi355_adam_update(float *w, const float *g, float *m, float *v, s
     if (!ran(mi355_adam_update_dev(st.dev<float>(iw), st.dev<float>(ig), st.dev<float>(im), st.dev<float>(iv), n, t, lr, b1, b2, eps, wd,
                                    1.0f, nullptr, 0)))
         return;
-    // Small arrays change together: w and m when v is there.
-    std::vector<float> w2, m2;
-    const bool small = nb <= PIECE;
-    if (small) {
-        w2.resize(n);
-        m2.resize(n);
-        st.becomes(iw, w2.data());
-        st.becomes(im, m2.data());
-    }
     if (!st.receive()) return;
-    if (small) {
-        memcpy(w, w2.data(), nb);
-        memcpy(m, m2.data(), nb);
-    }
     host_written_from(w, st.dev<float>(iw), nb);      // a resident embedding table that lives in w follows on the device
 }
 

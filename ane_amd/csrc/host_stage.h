@@ -14,6 +14,10 @@
 // mark each when it is done.  The caller takes pieces as well and waits only for pieces that somebody has taken, so a
 // helper that is asleep, late or was never created (no more processors, no threads left, a forked child) costs time and nothing
 // else.  Between calls they look for work for 100 us and then sleep.
+//
+// A call that fails leaves the arrays that it updates in place as they were, so that it can be made again: they are unpacked behind the
+// last copy of all results, and where one round cannot hold those, from memory of their own.  Arrays that it only writes
+// are unpacked as their bytes arrive.
 #pragma once
 
 constexpr int HELPERS = 3;
@@ -81,6 +85,7 @@ struct Piece {
 struct Helpers {
     pthread_t thread[HELPERS];
     int n;                                // created
+    int mode;                             // g_ctx.host_stage at the time
     pid_t pid;                            // of the process that created them
     pthread_mutex_t lock;
     pthread_cond_t wake;
@@ -112,6 +117,37 @@ bool one_piece(Helpers *h) {
     return true;
 }
 
+// The pieces 0 .. pieces - 1 become a round, of which the first `ready` may be taken; the round's number.
+unsigned long long start_pieces(Helpers *h, int pieces, int ready, bool in, bool past) {
+    // no helper may still be looking at the round before
+    const unsigned long long number = (h->next.load(std::memory_order_relaxed) >> 32) + 1;
+    h->ready.store(0, std::memory_order_seq_cst);
+    h->in = in;
+    h->past = past;
+    h->next.store(number << 32, std::memory_order_seq_cst);
+    h->ready.store(ready, std::memory_order_seq_cst);
+    if (pieces > 4 && h->n > 0) {
+        h->active.store(1);
+        h->calls.fetch_add(1);
+        if (h->asleep.load() > 0) {
+            pthread_mutex_lock(&h->lock);
+            pthread_cond_broadcast(&h->wake);
+            pthread_mutex_unlock(&h->lock);
+        }
+    }
+    return number;
+}
+
+// Takes what is left of a round (after an error nothing more is), and waits for the pieces that helpers have taken.
+void end_pieces(Helpers *h, int pieces, unsigned long long number, bool ok) {
+    int taken = pieces;
+    if (ok) while (one_piece(h)) { }
+    else taken = std::min(pieces, (int)(h->next.exchange((number << 32) | 0x7fffffffu) & 0x7fffffffu));
+    for (int i = 0; i < taken; i++)
+        while (!h->done[i].load(std::memory_order_acquire)) __builtin_ia32_pause();
+    h->active.store(0);
+}
+
 void *helper_main(void *arg) {
     Helpers *h = (Helpers *)arg;
     unsigned seen = h->calls.load(std::memory_order_acquire);
@@ -135,24 +171,6 @@ void *helper_main(void *arg) {
     }
 }
 
-// The helpers' state, created with its threads on first use; NULL without memory for it.
-Helpers *helpers() {
-    if (g_helpers) return g_helpers;
-    Helpers *h = (Helpers *)calloc(1, sizeof(Helpers));
-    if (!h) return nullptr;
-    pthread_mutex_init(&h->lock, nullptr);
-    pthread_cond_init(&h->wake, nullptr);
-    h->pid = getpid();
-    cpu_set_t cpus;
-    const int have = sched_getaffinity(0, sizeof(cpus), &cpus) == 0 ? CPU_COUNT(&cpus) : 1;
-    sigset_t all, old;                                    // the program's signals are not for them
-    sigfillset(&all);
-    pthread_sigmask(SIG_SETMASK, &all, &old);
-    while (h->n < HELPERS && h->n + 1 < have && pthread_create(&h->thread[h->n], nullptr, helper_main, h) == 0) h->n++;
-    pthread_sigmask(SIG_SETMASK, &old, nullptr);
-    return g_helpers = h;
-}
-
 void stop_helpers() {
     Helpers *h = g_helpers;
     if (!h || h->pid != getpid()) return;                 // (a forked child has no threads to stop)
@@ -169,6 +187,26 @@ void stop_helpers() {
 // (threads that run when the library's code goes away would crash)
 __attribute__((destructor)) void stop_helpers_at_exit() { stop_helpers(); }
 
+// The helpers' state, created with its threads on first use; NULL without memory for it.
+Helpers *helpers() {
+    if (g_helpers && g_helpers->mode != g_ctx.host_stage) stop_helpers();
+    if (g_helpers) return g_helpers;
+    Helpers *h = (Helpers *)calloc(1, sizeof(Helpers));
+    if (!h) return nullptr;
+    pthread_mutex_init(&h->lock, nullptr);
+    pthread_cond_init(&h->wake, nullptr);
+    h->pid = getpid();
+    h->mode = g_ctx.host_stage;
+    cpu_set_t cpus;
+    const int have = sched_getaffinity(0, sizeof(cpus), &cpus) == 0 ? CPU_COUNT(&cpus) : 1;
+    sigset_t all, old;                                    // the program's signals are not for them
+    sigfillset(&all);
+    pthread_sigmask(SIG_SETMASK, &all, &old);
+    while (h->mode != 1 && h->n < HELPERS && h->n + 1 < have && pthread_create(&h->thread[h->n], nullptr, helper_main, h) == 0) h->n++;
+    pthread_sigmask(SIG_SETMASK, &old, nullptr);
+    return g_helpers = h;
+}
+
 // ---- the blocks ----
 char *g_pin = nullptr, *g_pin_dev = nullptr;         // the host's address of it and the device's
 size_t g_pin_bytes = 0;
@@ -176,6 +214,7 @@ hipEvent_t g_sent[MAX_SENDS] = {};
 
 // pinned memory for min(bytes, PIN_MAX) and the events of a round; NULL where there is none
 char *pinned(size_t bytes) {
+    if (g_ctx.host_stage == 2) return nullptr;
     if (!g_sent[MAX_SENDS - 1])
         for (auto &e : g_sent)
             if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) { e = nullptr; (void)hipGetLastError(); return nullptr; }
@@ -241,7 +280,7 @@ public:
         if (!dev_) return false;
         return move(true);
     }
-    // brings the results to their arrays, which are untouched if the kernels failed
+    // brings the results to their arrays; those that are inputs too are untouched unless it returns true
     bool receive() { return move(false); }
 
 private:
@@ -251,6 +290,8 @@ private:
     int n_ = 0;
     size_t total_ = 0;
     char *dev_ = nullptr;
+    bool late_[MAX] = {};       // in place: unpacked when every copy of the round has arrived
+    int copies_ = 0;            // of this receive()
 
     int add(void *host, size_t bytes, bool in, bool out) {
         p_[n_] = Part{(char *)host, total_, bytes, nullptr, 0};
@@ -276,6 +317,43 @@ private:
         if (lo >= hi) return true;
         char *pin = pinned(total_);                        // (as large for both directions: it does not move while inputs travel)
         Helpers *h = helpers();
+        if (in) return move_range(in, what, h, pin, lo, hi);
+        copies_ = 0;
+        const bool one_round = pin && h && hi - lo <= g_pin_bytes;
+        size_t updated = 0;
+        for (int i = 0; i < n_; i++) {
+            const bool both = in_[i] && out_[i];
+            late_[i] = both && one_round;
+            if (both && !one_round) updated += p_[i].bytes;
+        }
+        if (updated == 0) return move_range(in, what, h, pin, lo, hi);
+        char *const hold = (char *)malloc(updated);
+        if (!hold) {
+            mi355_fail("no host memory for %zu bytes of results", updated);
+            (void)hipStreamSynchronize(g_ctx.stream);
+            return false;
+        }
+        Part own[MAX];
+        char *to = hold;
+        for (int i = 0; i < n_; i++) {
+            own[i] = p_[i];
+            if (!in_[i] || !out_[i]) continue;
+            p_[i].host = to;
+            p_[i].rows = nullptr;
+            to += p_[i].bytes;
+        }
+        const bool ok = move_range(in, what, h, pin, lo, hi);
+        for (int i = 0; i < n_; i++) {
+            const char *from = p_[i].host;
+            p_[i] = own[i];
+            if (ok && in_[i] && out_[i]) unpack(h, p_[i], (char *)from);
+        }
+        free(hold);
+        return ok;
+    }
+
+    // the bytes lo .. hi - 1 of the device block
+    bool move_range(bool in, const char *what, Helpers *h, char *pin, size_t lo, size_t hi) {
         if (!pin || !h) return move_unpinned(in, what);
         for (size_t beg = lo; beg < hi; beg += g_pin_bytes) {
             if (in && beg > lo) {                          // the block is filled again: the last round has to have left it
@@ -286,6 +364,22 @@ private:
         }
         return true;
     }
+
+    // a whole part from host memory at `from` to its array
+    static void unpack(Helpers *h, const Part &p, char *from) {
+        if (!h) { move_part(p, 0, p.bytes, from, false, true); return; }
+        for (size_t at = 0; at < p.bytes;) {
+            int pieces = 0;
+            for (; pieces < MAX_PIECES && at < p.bytes; at += PIECE) {
+                h->done[pieces].store(0, std::memory_order_relaxed);
+                h->piece[pieces++] = Piece{&p, at, std::min(p.bytes - at, PIECE), from + at};
+            }
+            end_pieces(h, pieces, start_pieces(h, pieces, pieces, false, true), true);
+        }
+    }
+
+    // a copy on its way back, or what g_ctx.host_stage_fail makes of it
+    hipError_t back(hipError_t e) { return e == hipSuccess && ++copies_ == g_ctx.host_stage_fail ? hipErrorUnknown : e; }
 
     // bytes beg .. end - 1 of the device block, through the pinned one
     bool round(bool in, const char *what, Helpers *h, char *pin, size_t beg, size_t end) {
@@ -302,10 +396,10 @@ private:
             if (at > end || sends + 1 == MAX_SENDS) at = end;
             cut[sends] = at;
         }
-        // the pieces, none across the end of a copy; last[s]: pieces up to the end of copy s
+        // the pieces, none across the end of a copy; last[s]: pieces up to the end of copy s.  Behind them those that wait for all.
         int pieces = 0, last[MAX_SENDS], s = 0;
         for (int i = 0; i < n_; i++) {
-            if (!(in ? in_[i] : out_[i])) continue;
+            if (!(in ? in_[i] : out_[i]) || (!in && late_[i])) continue;
             size_t at = std::max(p_[i].at, beg);
             const size_t stop = std::min(p_[i].at + p_[i].bytes, end);
             while (at < stop) {
@@ -317,22 +411,14 @@ private:
             }
         }
         while (s < sends) last[s++] = pieces;
-        // no helper may still be looking at the round before
-        const unsigned long long number = (h->next.load(std::memory_order_relaxed) >> 32) + 1;
-        h->ready.store(0, std::memory_order_seq_cst);
-        h->in = in;
-        h->past = in || end - beg > (size_t)1 << 20;           // (small results stay in the caches for their reader)
-        h->next.store(number << 32, std::memory_order_seq_cst);
-        if (in) h->ready.store(pieces, std::memory_order_seq_cst);
-        if (pieces > 4 && h->n > 0) {
-            h->active.store(1);
-            h->calls.fetch_add(1);
-            if (h->asleep.load() > 0) {
-                pthread_mutex_lock(&h->lock);
-                pthread_cond_broadcast(&h->wake);
-                pthread_mutex_unlock(&h->lock);
-            }
-        }
+        if (!in)
+            for (int i = 0; i < n_; i++)
+                for (size_t at = 0; late_[i] && at < p_[i].bytes; at += PIECE) {
+                    h->done[pieces].store(0, std::memory_order_relaxed);
+                    h->piece[pieces++] = Piece{&p_[i], at, std::min(p_[i].bytes - at, PIECE), pin + (p_[i].at + at - beg)};
+                }
+        // (small results stay in the caches for their reader)
+        const unsigned long long number = start_pieces(h, pieces, in ? pieces : 0, in, in || end - beg > (size_t)1 << 20);
         hipError_t e = hipSuccess;
         if (in) {
             int ok = 0;
@@ -350,7 +436,7 @@ private:
         } else {
             size_t from = beg;
             for (s = 0; s < sends && e == hipSuccess; s++) {
-                e = stage_copy(g_pin_dev + (from - beg), dev_ + from, cut[s] - from);
+                e = back(stage_copy(g_pin_dev + (from - beg), dev_ + from, cut[s] - from));
                 if (e == hipSuccess) e = hipEventRecord(g_sent[s], g_ctx.stream);
                 from = cut[s];
             }
@@ -364,14 +450,9 @@ private:
                     if (!one_piece(h)) __builtin_ia32_pause();
                 }
             }
+            if (e == hipSuccess) h->ready.store(pieces, std::memory_order_release);
         }
-        // what is left to take (after an error nothing more is), and then the pieces that helpers have taken
-        int taken = pieces;
-        if (e == hipSuccess) while (one_piece(h)) { }
-        else taken = std::min(pieces, (int)(h->next.exchange((number << 32) | 0x7fffffffu) & 0x7fffffffu));
-        for (int i = 0; i < taken; i++)
-            while (!h->done[i].load(std::memory_order_acquire)) __builtin_ia32_pause();
-        h->active.store(0);
+        end_pieces(h, pieces, number, e == hipSuccess);
         return e == hipSuccess || fail(what, e);
     }
 
@@ -385,6 +466,7 @@ private:
                 char *host = p.host + (p.rows ? (size_t)p.rows[r] * step : 0), *dev = dev_ + p.at + r * step;
                 hipError_t e = in ? hipMemcpyAsync(dev, host, step, hipMemcpyHostToDevice, g_ctx.stream)
                                   : hipMemcpyAsync(host, dev, step, hipMemcpyDeviceToHost, g_ctx.stream);
+                if (!in) e = back(e);
                 if (e == hipSuccess && !in) e = hipStreamSynchronize(g_ctx.stream);
                 if (e != hipSuccess) return fail(what, e);
             }
