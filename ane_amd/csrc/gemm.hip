@@ -314,7 +314,7 @@ struct GemmKernel {
 };
 constexpr GemmKernel GEMM_KERNELS[] = {
     {0, 1, 64, 64, 16, 4, 0.41, 0.30, 0.14}, {0, 2, 64, 64, 32, 3, 0.48, 0.49, 1.7},
-    {0, 4, 64, 32, 64, 3, 0.67, 0.66, 0.27}, {0, 4, 32, 64, 64, 3, 0.67, 0.66, 0.27},
+    {0, 4, 64, 32, 64, 3, 0.66, 0.66, 0.27}, {0, 4, 32, 64, 64, 3, 0.66, 0.66, 0.27},
     {1, 1, 128, 256, 32, 1, 2.3, 2.6, 4.2},  {1, 1, 256, 128, 32, 1, 2.3, 2.6, 4.2},
     {1, 1, 64, 64, 32, 3, 0.93, 0.43, 2.1},  {1, 2, 64, 64, 64, 1, 0.86, 0.86, 2.7},
     {2, 1, 96, 256, 64, 1, 3.7, 3.7, 4.4},   {2, 1, 64, 256, 64, 1, 2.6, 2.6, 4.4},
@@ -326,8 +326,13 @@ constexpr GemmKernel GEMM_KERNELS[] = {
 // the rate of the last-level cache.  The numbers are fitted to 210 products of every transpose case (vocabularies of 2000 to
 // 24573 rows by 32 to 512 columns, the weight gradients of a layer, squares, thin and long ones) in every kernel and number of
 // slices, those of gemm_planes.h to 153 of them: what is chosen takes 0.7 % more than the best on the average and 14 % at worst;
-// tiles of 128 x 64 and 64 x 128 were never the best and are gone.
-// Measured, us; the chosen kernel first (in brackets the library that stood here before):
+// tiles of 128 x 64 and 64 x 128 were never the best and are gone.  On 380 other products, odd sizes among them, whose operands
+// no cache holds, it takes 2.2 % more than the best of the kernels on the average, 5 % more in 57 and 58 % more at worst ([1000][768]^T
+// . [1000][500], fp32 32 x 64 27.9, split 64 x 64 in two groups 17.7).
+// Measured on operands that the caches hold, us; the chosen kernel first (in brackets the library that stood here before).  Where
+// they do not, the same ones are ahead: [24573][1024] . [1024][256] 72, split 256 x 128 91; [24573][256] . [256][1024] += 82, 105;
+// [32000][256] . [256][768] += 90, 104; [32000][768] . [768][256] 75, planes 64 x 256 81; [768][32000] . [32000][256] 82, planes 87;
+// [14000][768] . [768][256] 43, 52; [14000][256] . [256][768] += 45, split 64 x 64 58; [24573][64] . [64][1024] += 58, fp32 66.
 //   [24573][1024] . [1024][256]        planes 96 x 256 71, split 256 x 128 90, 64 x 64 100, fp32 124
 //   [24573][256] . [256][1024] +=      rows of 96 68, split 128 x 256 94, 64 x 64 107, fp32 123
 //   [32000][256] . [256][768] +=       rows of 64 73, of 96 82, split 128 x 256 90, fp32 121                   (112)
@@ -340,6 +345,8 @@ constexpr GemmKernel GEMM_KERNELS[] = {
 //   [2048][256] . [256][768] +=        fp32 32 x 64 11.8, 64 x 64 13.1, split 64 x 64 13.6, rows of 64 20      (10.9)
 //   [3072][256] . [256][1024] +=       split 64 x 64 18.0, fp32 64 x 64 20.1, rows of 64 24, split 128 x 256 27 (16.3)
 //   [4096][1024] . [1024][3072]        planes 64 x 256 140, split 128 x 256 168, 64 x 64 181, fp32 228
+//   [4096][4096] . [4096][4096]        split 128 x 256 691, planes 96 x 256 725, 64 x 256 760 (6.4 GB of planes from the L2s), fp32 1183
+//   [256][4096] . [4096][256]          fp32 32 x 64 12.5, split 64 x 64 in two groups 15.6
 //   [1024][1024] . [1024][1024]        split 64 x 64 in two groups 21.6, fp32 64 x 32 23.5, 64 x 64 23.7       (19.9)
 //   [2048][768] . [768][256]           fp32 64 x 32 10.9, split 64 x 64 in two groups 15.4, fp32 64 x 64 17    (13.8)
 //   [24573][1024] . [1024][1]          fp32 64 x 32 24.5, split 64 x 64 32, fp32 64 x 64 38                    (72)
@@ -382,7 +389,8 @@ GemmPlan plan_gemm(int ta, int tb, int M, int N, int K, bool reads_c, int lda, i
             const double n = up(tiles_m * tiles_n * slices / cus);                      // workgroups of the busiest compute unit
             const double work = steps * std::max(t.alone, n * t.shared) * slow + t.fixed * up(n / t.resident);
             const double hbm = 4.0 * ((double)M * K + out * (slices > 1 ? slices : c_times)) + (t.split == 2 ? planes : 4.0 * N * K);
-            const double l2 = t.split == 2 ? 0.0 : 4.0 * K * (M * tiles_n + N * tiles_m);
+            // (a value of B's planes has six bytes; these kernels ask for them and for A a step ahead, so half of it counts)
+            const double l2 = t.split == 2 ? K * (2.0 * M * tiles_n + 3.0 * N * tiles_m) : 4.0 * K * (M * tiles_n + N * tiles_m);
             const double mem = std::max(hbm / 5.6e6, l2 / 21e6);
             double us = 3.4 + std::max(work, mem) + 0.23 * std::min(work, mem);
             if (slices > 1) us += 5.4 + slices * out * 4.0 / 5.6e6;

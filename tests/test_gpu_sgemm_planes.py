@@ -164,3 +164,13 @@ def test_planes_write_nothing_outside_c(br, M, knob):
         want = A.astype(np.float64) @ B.astype(np.float64) + beta * C0
         bound = (7 * (K // 32 + 2) + 2) * 2.0 ** -23 * mag + 3 * 2.0 ** -24 * (np.abs(want) + beta * np.abs(C0))
         assert np.all(np.abs(out[:, :N] - want) <= bound)
+
+
+@pytest.mark.parametrize("M,N,K,knob", [(4096, 4096, 4096, 1), (256, 256, 4096, -1), (24573, 256, 1024, 5)])
+def test_the_quickest_kernel_is_chosen(br, M, N, K, knob):
+    """Planes of a large operand that every tile reads again, many slices of a small output, and the classifier's logits: the choice
+    is seen by the bits, which differ between the kernels."""
+    print("[case] sgemm choice M=%d N=%d K=%d knob=%d" % (M, N, K, knob), flush=True)
+    A, B = H.normal(770, (M, K)), H.normal(771, (K, N))
+    got = {k: product(br, k, A, B, 0, 0).tobytes() for k in (0, -1, 1, 4, 5)}
+    assert got[0] == got[knob] and all(got[0] != got[k] for k in (-1, 1, 4, 5) if k != knob)
