@@ -44,15 +44,22 @@ constexpr int STAGE_ROWS = 15 * ROWS_PER_WAVE;    // two buffers of 240 rows x 1
 // other along the positions run on one XCD, whose L2 puts the parts together ([40][1024][1000], 164 MB: 64 x 64 in the order of
 // the grid 71 us, in this order 53, 256 x 32 41.5).  Four positions of one sequence are stored as one access at any
 // alignment ([37][768][333] 21.5 -> 14.3 us).
-template <bool VEC_D, int GT, int GD>
+// REMAP: tiles are dealt out by XCD.  Finding its tile costs a workgroup 0.2 us, and where a compute unit has few of them that is
+// what a launch takes longer (one to eight sequences of 512 4.7 us, with the grid's own order 4.45).
+template <bool VEC_D, int GT, int GD, bool REMAP>
 __global__ __launch_bounds__(256) void gather_kernel(float *__restrict__ x, const float *__restrict__ E,
                                                      const int32_t *__restrict__ ids, int V, int D, int S, int N) {
     __shared__ float tile[GT][GD + 1];
     __shared__ int tok[GT];
-    const int tiles_n = (N + GT - 1) / GT;
-    const int logical = xcd_remap(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
-    const int n0 = logical % tiles_n * GT;     // consecutive positions, of one or several sequences
-    const int d0 = logical / tiles_n * GD;
+    int tile_n = blockIdx.x, tile_d = blockIdx.y;
+    if constexpr (REMAP) {
+        const int tiles_n = (N + GT - 1) / GT;
+        const int logical = xcd_remap(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
+        tile_n = logical % tiles_n;
+        tile_d = logical / tiles_n;
+    }
+    const int n0 = tile_n * GT;                // consecutive positions, of one or several sequences
+    const int d0 = tile_d * GD;
     const int tid = threadIdx.x;
     if (tid < GT) {
         const int n = n0 + tid;
@@ -118,14 +125,14 @@ __global__ __launch_bounds__(256) void gather_kernel(float *__restrict__ x, cons
     }
 }
 
-template <int GT, int GD>
+template <int GT, int GD, bool REMAP = true>
 int launch_gather(float *x, const float *E, const int32_t *ids, int V, int D, int S, int N) {
     const size_t tiles_n = ceil_div((size_t)N, GT), tiles_d = ceil_div((size_t)D, GD), tiles = tiles_n * tiles_d;
     // (a grid dimension holds 2^32 threads)
-    const dim3 grid = tiles < ((size_t)1 << 24) ? dim3((unsigned)tiles) : dim3((unsigned)tiles_n, (unsigned)tiles_d);
+    const dim3 grid = REMAP && tiles < ((size_t)1 << 24) ? dim3((unsigned)tiles) : dim3((unsigned)tiles_n, (unsigned)tiles_d);
     if (grid.y > 65535) return mi355_fail("embed_gather: D too large");
-    if (D % 4 == 0) hipLaunchKernelGGL((gather_kernel<true, GT, GD>), grid, dim3(256), 0, g_ctx.stream, x, E, ids, V, D, S, N);
-    else hipLaunchKernelGGL((gather_kernel<false, GT, GD>), grid, dim3(256), 0, g_ctx.stream, x, E, ids, V, D, S, N);
+    if (D % 4 == 0) hipLaunchKernelGGL((gather_kernel<true, GT, GD, REMAP>), grid, dim3(256), 0, g_ctx.stream, x, E, ids, V, D, S, N);
+    else hipLaunchKernelGGL((gather_kernel<false, GT, GD, REMAP>), grid, dim3(256), 0, g_ctx.stream, x, E, ids, V, D, S, N);
     LAUNCH_OK("embed_gather");
     return 0;
 }
@@ -862,10 +869,17 @@ MI355_API int mi355_embed_gather_dev(float *x, const float *E, const int32_t *id
     if ((size_t)batch * S > (size_t)1 << 30) return mi355_fail("embed_gather: more than 2^30 positions");
     const int N = batch * S;
     // Rows of whole lines: see gather_kernel.  Others: 256 x 32, or 256 x 16 where that leaves fewer than eight workgroups to a
-    // compute unit ([37][768][333] 14.3 us with 16 dims, 16.4 with 32; [40][1024][1000] 43.4 and 41.5).
+    // compute unit ([37][768][333] 14.3 us with 16 dims, 16.4 with 32; [40][1024][1000] 43.4 and 41.5).  Few positions: 64 x 32,
+    // since a workgroup's loads and stores one behind the other are most of the time: on the average 4.5 us for up to 512 tiles of
+    // rows of any length (256 x 16: 5.2) and 4.4 for 1024 to 2048 of whole lines (64 x 64: 4.6; from 4096 on 8.3, and 9.1 with
+    // 64 x 32); by XCD from 512 on where lines are shared, 5.7 (6.3, the grid's own order 6.6) up to 2048, 9.5 (9.0) beyond.
+    const size_t small = ceil_div((size_t)N, 64) * ceil_div((size_t)D, 32);
+    const bool lines = S % 32 == 0 && ((uintptr_t)x & 127u) == 0;
     const size_t wide = ceil_div((size_t)N, 256) * ceil_div((size_t)D, 32);
     const size_t cus = g_ctx.num_cu > 0 ? g_ctx.num_cu : 256;
-    if ((S % 32 == 0 && ((uintptr_t)x & 127u) == 0) || wide >= ((size_t)1 << 23)) return launch_gather<64, 64>(x, E, ids, V, D, S, N);
+    if (small < (lines ? 16 : 2) * cus) return launch_gather<64, 32, false>(x, E, ids, V, D, S, N);
+    if (!lines && small < 8 * cus) return launch_gather<64, 32>(x, E, ids, V, D, S, N);
+    if (lines || wide >= ((size_t)1 << 23)) return launch_gather<64, 64>(x, E, ids, V, D, S, N);
     if (wide >= 8 * cus) return launch_gather<256, 32>(x, E, ids, V, D, S, N);
     return launch_gather<256, 16>(x, E, ids, V, D, S, N);
 }

@@ -1,5 +1,5 @@
-"""mi355_embed_gather_dev at the edges of its tiles: 64 x 64 for rows of whole 128-byte lines, 256 x 32 and 256 x 16 for others, x
-and the table at any float, positions of several sequences in a tile, ids out of range."""
+"""mi355_embed_gather_dev at the edges of its tiles: 64 x 32 for few positions, in the order of the grid and by XCD, 64 x 64 for rows of
+whole 128-byte lines, 256 x 32 and 256 x 16 for others, x and the table at any float, positions of several sequences in a tile, ids out of range."""
 import numpy as np
 import pytest
 
@@ -18,7 +18,8 @@ def br():
 
 @pytest.mark.parametrize("off", [0, 1])
 @pytest.mark.parametrize("V,D,B,S,oob", [(50, 65, 2, 32, 3), (50, 64, 1, 64, 0), (300, 68, 3, 96, 0), (300, 17, 1, 255, 5), (300, 16, 1, 256, 0),
-                                         (300, 33, 1, 257, 1), (300, 15, 5, 3, 2), (700, 1023, 130, 127, 9), (700, 1028, 66, 250, 0), (9, 1, 7, 73, 0)])
+                                         (300, 33, 1, 257, 1), (300, 15, 5, 3, 2), (700, 1023, 130, 127, 9), (700, 1028, 66, 250, 0), (9, 1, 7, 73, 0),
+                                         (300, 260, 33, 130, 4), (300, 515, 34, 250, 3), (300, 513, 64, 256, 2)])
 def test_gather_tiles(br, V, D, B, S, oob, off):
     print("[case] gather tiles V=%d D=%d B=%d S=%d off=%d" % (V, D, B, S, off), flush=True)
     rng = np.random.default_rng(800)
