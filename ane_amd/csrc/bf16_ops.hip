@@ -791,7 +791,7 @@ MI355_API int mi355_rmsnorm_fwd_bf16_dev(uint16_t *y, const uint16_t *x, const f
         cluster_whole(cp, [&](auto whole) {
             constexpr int WHOLE = decltype(whole)::value;
             if (cp.rpt == 2) BF_CLUSTER_FWD(2, WHOLE);
-            else BF_CLUSTER_FWD(4, WHOLE);
+            else BF_CLUSTER_FWD(4, WHOLE % CL_FEW);
         });
         LAUNCH_OK("rmsnorm_fwd_bf16");
         return 0;
@@ -822,7 +822,7 @@ MI355_API int mi355_rmsnorm_bwd_bf16_dev(uint16_t *dx, float *dw, const uint16_t
         cluster_whole(cp, [&](auto whole) {
             constexpr int WHOLE = decltype(whole)::value;
             if (cp.rpt == 2) BF_CLUSTER_BWD(2, WHOLE);
-            else BF_CLUSTER_BWD(4, WHOLE == CL_EXACT ? CL_LINES : WHOLE);
+            else BF_CLUSTER_BWD(4, WHOLE == CL_EXACT ? CL_LINES : WHOLE % CL_FEW);
         });
         LAUNCH_OK("rmsnorm_bwd_bf16");
         if (mi355_dw_submit(dw, part, nrows, C)) return -1;
@@ -861,7 +861,7 @@ MI355_API int mi355_residual_rmsnorm_fwd_bf16_dev(uint16_t *y, uint16_t *yn, con
         cluster_whole(cp, [&](auto whole) {
             constexpr int WHOLE = decltype(whole)::value;
             if (cp.rpt == 2) BF_CLUSTER_RES_FWD(2, WHOLE);
-            else BF_CLUSTER_RES_FWD(4, WHOLE);
+            else BF_CLUSTER_RES_FWD(4, WHOLE % CL_FEW);
         });
 #undef BF_CLUSTER_RES_FWD
         LAUNCH_OK("residual_rmsnorm_fwd_bf16");
@@ -898,7 +898,7 @@ MI355_API int mi355_rmsnorm_bwd_residual_bf16_dev(uint16_t *dx, uint16_t *dx_sca
         cluster_whole(cp, [&](auto whole) {
             constexpr int WHOLE = decltype(whole)::value;
             if (cp.rpt == 2) BF_CLUSTER_RES_BWD(2, WHOLE);
-            else BF_CLUSTER_RES_BWD(4, WHOLE == CL_EXACT ? CL_LINES : WHOLE);
+            else BF_CLUSTER_RES_BWD(4, WHOLE == CL_EXACT ? CL_LINES : WHOLE % CL_FEW);
         });
 #undef BF_CLUSTER_RES_BWD
         LAUNCH_OK("rmsnorm_bwd_residual_bf16");

@@ -506,7 +506,7 @@ void launch_fwd_cluster(const ClusterPlan &cp, float *yn, float *y_res, const fl
     cluster_whole(cp, [&](auto whole) {
         constexpr int WHOLE = decltype(whole)::value;
         if (cp.rpt == 4) launch_fwd_cluster_as<4, FUSE, WHOLE>(cp, yn, y_res, a, b, alpha, w, C, S, eps);
-        else launch_fwd_cluster_as<8, FUSE, WHOLE>(cp, yn, y_res, a, b, alpha, w, C, S, eps);
+        else launch_fwd_cluster_as<8, FUSE, WHOLE % CL_FEW>(cp, yn, y_res, a, b, alpha, w, C, S, eps);
     });
 }
 
@@ -522,7 +522,6 @@ void launch_bwd_cluster_as(const ClusterPlan &cp, float *dx, float *part, const 
 template <bool RES>
 void launch_bwd_cluster(const ClusterPlan &cp, float *dx, float *part, const float *dy, const float *x, const float *w,
                         int C, int S, float eps, int variant, const float *res, float *dx2, float alpha2) {
-    // (with the residual 126 of the 128 registers a lane has; [16][1024][256] 15.4 -> 14.7 us)
     // (CL_EXACT with the residual: 126 of the 128 registers a lane has; [16][1024][256] 15.4 -> 14.7 us)
     cluster_whole(cp, [&](auto whole) {
         launch_bwd_cluster_as<RES, decltype(whole)::value>(cp, dx, part, dy, x, w, C, S, eps, variant, res, dx2, alpha2);

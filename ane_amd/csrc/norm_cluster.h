@@ -81,9 +81,14 @@ static_assert(CL_SLOT_STRIDE >= 2 * CL_LPR * StoreBf16::VEC, "two quantities per
 // residual 17.1 / 19.9, [22][1024][147] 14.4 / 12.6.
 // CL_EXACT: every member holds exactly RPS*RPT rows and every strip is whole; CL_LINES: rows are whole lines; CL_ANY: neither.  (One
 // kernel with the loads written twice behind a branch took 27.9 us for the 25.4 of [32][768][256].)
-enum { CL_ANY, CL_LINES, CL_EXACT };
+// CL_FEW, with one of the latter two: the members' rows fill at most half of their tiles.  Then the row steps in which no lane has a row
+// are passed over; elsewhere that costs more than it saves.  fp32 backward with the residual, us, loaded all the same / passed over:
+// [1][512][32] 8.8 / 7.9, [8][512][54] 9.4 / 8.4, [16][512][147] 18.0 / 17.2; bfloat16 [4][512][33] 11.7 / 10.9 (12.1 / 12.6 for
+// [4][1024][54], where they fill it).
+enum { CL_ANY, CL_LINES, CL_EXACT, CL_FEW };
+constexpr bool cl_lines(int whole) { return whole == CL_EXACT || whole % CL_FEW == CL_LINES; }
 template <typename ST, int WHOLE>
-__device__ __forceinline__ typename ST::Raw cluster_load(const typename ST::T *p) { return WHOLE != CL_ANY ? ST::load_nt(p) : ST::load(p); }
+__device__ __forceinline__ typename ST::Raw cluster_load(const typename ST::T *p) { return cl_lines(WHOLE) ? ST::load_nt(p) : ST::load(p); }
 
 // Per-thread partial sums acc[q][j] (q < NV quantities, j < VEC columns of this lane) -> per-column sums of the
 // workgroup in wsum[q*W + column], valid for all threads after the barrier.  lds: NW*NV*W floats.
@@ -240,6 +245,11 @@ __global__ __launch_bounds__(THREADS) void rms_fwd_cluster_kernel(typename ST::T
     float wv[RPT];
 #pragma unroll
     for (int k = 0; k < RPT; k++) {
+        if (WHOLE >= CL_FEW && k * RPS >= rows_pm) {
+            xr[k] = ST::zero();
+            wv[k] = 0.f;
+            continue;
+        }
         const bool live = EXACT || row_live(g.member, k);
         const int c = live ? row_of(g.member, k) : 0;
         xr[k] = load_row(c, true);
@@ -318,8 +328,8 @@ __global__ __launch_bounds__(THREADS) void rms_bwd_cluster_kernel(typename ST::T
                                                                   float alpha2, ClusterWs ws, int spin_ticks) {
     // without the residual, rows of whole lines keep the branch: [4][768][256] 8.1 us with it, 8.6 without ([8][768][256] with the
     // residual 10.0 and 9.1)
-    constexpr bool INSIDE = RES || WHOLE != CL_LINES;
     constexpr bool EXACT = WHOLE == CL_EXACT;
+    constexpr bool INSIDE = RES || EXACT || !cl_lines(WHOLE);
     constexpr int VEC = ST::VEC;
     constexpr int W = CL_LPR * VEC;
     constexpr int RPS = THREADS / CL_LPR;
@@ -346,8 +356,9 @@ __global__ __launch_bounds__(THREADS) void rms_bwd_cluster_kernel(typename ST::T
     float wv[RPT];
 #pragma unroll
     for (int k = 0; k < RPT; k++) {
-        if (!INSIDE && !row_live(g.member, k)) {
+        if (INSIDE ? WHOLE >= CL_FEW && k * RPS >= rows_pm : !row_live(g.member, k)) {
             xr[k] = dr[k] = ST::zero();
+            if constexpr (RES) rr_res[k] = ST::zero();
             wv[k] = 0.f;
             continue;
         }
@@ -472,7 +483,7 @@ __global__ __launch_bounds__(THREADS) void rms_bwd_cluster_kernel(typename ST::T
 // How a shape is split: csplit members of rows_pm rows each; rpt rows per lane.  csplit = 0: not clustered.
 struct ClusterPlan {
     int csplit, rows_pm, rpt, threads, strips, nblk;
-    int whole;         // which kernel: CL_EXACT, CL_LINES or CL_ANY
+    int whole;         // which kernel: CL_EXACT, or CL_LINES or CL_ANY, with or without CL_FEW
 };
 constexpr ClusterPlan NO_CLUSTER = {0, 0, 0, 0, 0, 0, CL_ANY};
 
@@ -511,13 +522,16 @@ ClusterPlan cluster_plan(int C, int S, int batch, bool vec_ok, int vec, int rpt_
     p.threads = threads;
     p.strips = (int)strips;
     p.nblk = (int)(clusters * split);
-    p.whole = rows == rps * rpt && rows * split == C && S % w == 0 ? CL_EXACT : S % (w / 2) == 0 ? CL_LINES : CL_ANY;
+    p.whole = rows == rps * rpt && rows * split == C && S % w == 0 ? CL_EXACT : (S % (w / 2) == 0 ? CL_LINES : CL_ANY) + (2 * rows <= rps * rpt ? CL_FEW : 0);
     return p;
 }
+// (a tile of more than the fewest rows per lane is at least half full: no CL_FEW there)
 template <typename F>
 void cluster_whole(const ClusterPlan &p, F as) {
     if (p.whole == CL_EXACT) as(std::integral_constant<int, CL_EXACT>());
     else if (p.whole == CL_LINES) as(std::integral_constant<int, CL_LINES>());
+    else if (p.whole == CL_LINES + CL_FEW) as(std::integral_constant<int, CL_LINES + CL_FEW>());
+    else if (p.whole == CL_ANY + CL_FEW) as(std::integral_constant<int, CL_ANY + CL_FEW>());
     else as(std::integral_constant<int, CL_ANY>());
 }
 

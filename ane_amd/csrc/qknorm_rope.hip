@@ -91,7 +91,7 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_fwd_kernel(
 }
 
 enum { QK_SOME, QK_ROWS, QK_ALL };
-// EXACT: the tile holds every row pair of the head and nothing else, every strip is whole: no load or store is behind a condition
+// WHOLE = QK_ALL: the tile holds every row pair of the head and nothing else, every strip is whole: no load or store is behind a condition
 // ([16][24 x 128][256] 32.4 -> 31.5 us).  (The forward is slower so, 20.3 -> 21.5: fewer registers, more workgroups at a time.)
 template <int LPR, int THREADS, int CAP, int WHOLE = QK_SOME>
 __global__ __launch_bounds__(THREADS) void qknorm_rope_bwd_kernel(
@@ -240,6 +240,15 @@ bool pick_qk(int hd, int S, bool in_place, QkCfg &cfg, bool backward) {
 
 // Rows that are not whole 128-byte lines, on a tile that the head's row pairs fill (hd 128 and 64): the ROWS kernels.
 bool whole_rows(const QkCfg &cfg, int hd, int S) { return S % 32 != 0 && cfg.lpr == 16 && cfg.threads / 16 * cfg.cap * 2 == hd; }
+// Where the forward is quicker with them, by the workgroups to a compute unit.  The other kernel does best just before its workgroups
+// need another round: hd 64 from four to five of them ([12][24 x 64][197] 10.5 us, ROWS 12.3; with eight 15.4 and 14.0), hd 128 from
+// three to four ([12][24 x 128][147] 16.0, 17.1; with three 13.5, 13.0).  And lanes past the end of a row ask again for what others
+// have: in a single strip that costs more than it saves from three on ([64][24 x 64][54] 9.7, 11.3; [32][24 x 128][54] 9.2, 10.7;
+// [4][24 x 128][54] 6.2, 4.4), and in two of which the second is nearly empty from six on ([30][24 x 64][70] 1.15 times as long).
+bool forward_rows(int hd, int S, size_t workgroups) {
+    const size_t cus = g_ctx.num_cu > 0 ? g_ctx.num_cu : 256, round = ceil_div(workgroups, cus);
+    return round != (hd == 128 ? 4 : 5) && (S >= 80 || round <= (S <= 64 ? 2 : 5));
+}
 
 int check_shape(const char *who, int heads, int kv_heads, int hd, int S, int batch) {
     if (hd <= 0 || (hd & 1) || S <= 0 || batch <= 0 || heads < 0 || kv_heads < 0 || heads + kv_heads == 0)
@@ -269,7 +278,7 @@ MI355_API int mi355_qknorm_rope_fwd_dev(float *q_out, float *k_out, const float 
         hipLaunchKernelGGL(kernel, dim3(nq + nk), dim3(threads), 0, g_ctx.stream, q_out, k_out, q, k, wq, wk, hd, S, strips, nq, cos_dev,
                            sin_dev, eps, 1.0f / (float)hd);
     };
-    const bool rows = whole_rows(cfg, hd, S);
+    const bool rows = whole_rows(cfg, hd, S) && forward_rows(hd, S, (size_t)(nq + nk));
     if (rows && cfg.threads == 256 && cfg.cap == 4) launch(qknorm_rope_fwd_kernel<16, 256, 4, true>, 256);
     else if (rows && cfg.threads == 256 && cfg.cap == 2) launch(qknorm_rope_fwd_kernel<16, 256, 2, true>, 256);
     else
