@@ -1489,8 +1489,8 @@ def test_host_vocab_dropins_and_table_coherence(br):
     assert xo.tobytes() == O.embed_lookup(E, tok.astype(np.int32))[0][0].tobytes()
     big = np.concatenate([E.ravel(), np.zeros(D, np.float32)]); E2 = big[:V * D].reshape(V, D)
     br.lib.mi355_embed_lookup(_p(xo), _p(E2), _p(tok), V, D, S)                         # a second resident table
-    tail = big[(V - 3) * D:]; zt = np.zeros_like(tail)
-    br.lib.mi355_adam_update(_p(tail), _p(np.ones_like(tail)), _p(zt), _p(zt.copy()), tail.size, 1, 1e-2, 0.9, 0.95, 1e-8, 0.0)
+    tail = big[(V - 3) * D:]; gt, mt, vt = np.ones_like(tail), np.zeros_like(tail), np.zeros_like(tail)
+    br.lib.mi355_adam_update(_p(tail), _p(gt), _p(mt), _p(vt), tail.size, 1, 1e-2, 0.9, 0.95, 1e-8, 0.0)
     tok2 = np.full(S, V - 1, np.uint16)
     br.lib.mi355_embed_lookup(_p(xo), _p(E2), _p(tok2), V, D, S)
     assert xo.tobytes() == O.embed_lookup(E2, tok2.astype(np.int32))[0][0].tobytes()
