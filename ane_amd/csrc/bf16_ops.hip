@@ -660,9 +660,9 @@ BfCfg pick_bf(int C, bool vec_ok, int S, int batch) {
 // Clustered variants (norm_cluster.h, bf16 storage: strips of 128 columns, 2 or 4 rows per lane).  Not when the
 // single-workgroup tile is chosen by hand through the rms_lpr / rms_threads knobs.
 Mi355Exchange g_bf_cluster_ws = {nullptr, nullptr, nullptr};
-ClusterPlan plan_cluster_bf(int C, int S, int batch, bool vec_ok) {
+ClusterPlan plan_cluster_bf(int C, int S, int batch, bool vec_ok, bool residual_bwd = false) {
     if (g_ctx.rms_lpr || g_ctx.rms_threads) return NO_CLUSTER;
-    return cluster_plan(C, S, batch, vec_ok, StoreBf16::VEC, 2, 4, 1);
+    return cluster_plan(C, S, batch, vec_ok, StoreBf16::VEC, 2, 4, 1, residual_bwd ? 32 : CL_MAX_BLOCKS);
 }
 #define BF_CLUSTER_FWD(RPT, WHOLE)                                                                                   \
     hipLaunchKernelGGL((rms_fwd_cluster_kernel<StoreBf16, RPT, 1024, false, WHOLE>), dim3(cp.nblk), dim3(1024), 0,   \
@@ -885,7 +885,7 @@ MI355_API int mi355_rmsnorm_bwd_residual_bf16_dev(uint16_t *dx, uint16_t *dx_sca
     if (dx == x) return mi355_fail("rmsnorm_bwd_residual_bf16: dx must not alias x (dx may alias res or dy)");
     const bool vec_ok = S >= 8;
     const bool apart = dx != res || tail_in_strip(S, CL_LPR * StoreBf16::VEC, StoreBf16::VEC);
-    const ClusterPlan cp = dx == dy || !apart ? NO_CLUSTER : plan_cluster_bf(C, S, batch, vec_ok);
+    const ClusterPlan cp = dx == dy || !apart ? NO_CLUSTER : plan_cluster_bf(C, S, batch, vec_ok, true);
     if (cp.csplit) {
         if (!mi355_exchange(&g_bf_cluster_ws)) return -1;
         const int nrows = cp.nblk / cp.csplit;

@@ -487,9 +487,9 @@ ClusterWs g_cluster_ws = {nullptr, nullptr, nullptr};
 bool cluster_ws_ready(void) { return mi355_exchange(&g_cluster_ws); }
 
 // The single-workgroup tiles are chosen by hand (knobs) or the shape does not cluster: csplit == 0.
-ClusterPlan plan_cluster(int C, int S, int batch, bool vec_ok, int max_rpt, int rounds = 1) {
+ClusterPlan plan_cluster(int C, int S, int batch, bool vec_ok, int max_rpt, int rounds = 1) {      // max_rpt: 8 forward, 4 backward
     if (g_ctx.rms_lpr || g_ctx.rms_threads) return NO_CLUSTER;
-    return cluster_plan(C, S, batch, vec_ok, StoreF32::VEC, 4, max_rpt, rounds);
+    return cluster_plan(C, S, batch, vec_ok, StoreF32::VEC, 4, max_rpt, rounds, max_rpt == 8 ? CL_MAX_BLOCKS : 24);
 }
 
 template <int RPT, bool FUSE, int WHOLE>
