@@ -37,8 +37,8 @@ STREAM_LAUNCH_MS, STREAM_RATE_BYTES_PER_MS = 0.0035, 6.97e9      # measured: one
 OP_KERNELS = {
     "rmsnorm_fwd": [("rms_fwd_cluster_kernel<StoreF32, 4, 1024, false, 2>", 1.0)],
     "rmsnorm_bwd": [("rms_bwd_cluster_kernel<StoreF32, 4, 1024, false, 2>", 1.0), ("reduce_jobs_kernel", 0.5)],
-    "qknorm_rope_fwd": [("qknorm_rope_fwd_kernel<16, 256, 4>", 1.0)],
-    "qknorm_rope_bwd": [("qknorm_rope_bwd_kernel<16, 512, 2, true>", 1.0)],
+    "qknorm_rope_fwd": [("qknorm_rope_fwd_kernel<16, 256, 4, false>", 1.0)],
+    "qknorm_rope_bwd": [("qknorm_rope_bwd_kernel<16, 512, 2, 2>", 1.0)],
     "swiglu_fwd": [("swiglu_fwd_kernel<1>", 1.0)],
     "swiglu_bwd": [("swiglu_bwd_kernel<1>", 1.0)],
     "residual": [("axpby_kernel<0, 1>", 1.0)],
@@ -56,7 +56,7 @@ OP_KERNELS = {
 EMBED_KERNELS = {
     "scatter_cols": [("chunk_sort_blk_kernel", 1.0), ("block_rank_kernel<1>", 1.0), ("col_sum_kernel<3, true, false>", 1.0)],
     "scatter_rows": [("chunk_sort_kernel", 1.0), ("rank_transpose_kernel", 1.0), ("seg_sum_kernel<false>", 1.0)],
-    "gather": [("gather_kernel<true, 64, 64>", 1.0)],
+    "gather": [("gather_kernel<true, 64, 64, true>", 1.0)],
 }
 
 
@@ -64,7 +64,10 @@ def traffic_bytes(profile_key, kernels):
     """HBM-side bytes of one op from profiles/traffic.json, or None when the file or a kernel's row is missing."""
     from ane_amd.profile_summary import load_traffic
     rows = load_traffic().get(profile_key, {}).get("kernels", {})
-    if any(k not in rows for k, _ in kernels):
+    missing = [k for k, _ in kernels if k not in rows]
+    if missing:
+        print("bench.py: profiles/traffic.json has no %s row of %s: no traffic is reported for it" % (profile_key, ", ".join(missing)),
+              file=sys.stderr)
         return None
     return sum(rows[k]["traffic_mb"] * wgt for k, wgt in kernels) * 1e6
 
@@ -914,8 +917,8 @@ def main():
                                                                ("softmax_ce", "int8_scale", "int8_quant", "int8_dequant", "int8_quantize_dynamic") else 1))
     roofline = dict(bound="hbm", kernel=dom["op"], achieved=dom["gbs"], peak=PEAK_HBM_GBS, unit="GB/s",
                     frac=dom["gbs"] / PEAK_HBM_GBS,
-                    traffic=(traffic_bytes("qwen3_sweep", OP_KERNELS.get(dom["op"], [("-", 1.0)]))
-                             if (cfg["name"], cfg["batch"], bf16) == ("qwen3-0.6b", 16, False) else None),
+                    traffic=(traffic_bytes("qwen3_sweep", OP_KERNELS[dom["op"]])
+                             if (cfg["name"], cfg["batch"], bf16) == ("qwen3-0.6b", 16, False) and dom["op"] in OP_KERNELS else None),
                     traffic_source="profiles/traffic.json (qwen3_sweep)", alg_bytes_per_launch=ab[dom["op"]],
                     avg_launch_ms=dom["ms"])
 

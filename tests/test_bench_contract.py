@@ -42,3 +42,17 @@ def test_traffic_figures_come_from_the_tracked_profile_summaries():
                 assert abs(float(m.group(3)) - rows[k]["traffic_mb"]) <= 0.011, (key, k)
     src = open(os.path.join(ROOT, "bench.py")).read()
     assert not re.search(r"TRAFFIC_BYTES\s*=", src)
+
+
+def test_priced_kernels_are_kernels_of_the_library():
+    """A kernel whose template arguments change leaves its old name in the profiles, and its op would be priced by what no longer runs:
+    every name that bench.py prices is a kernel of the built library."""
+    sys.path.insert(0, ROOT)
+    import bench
+    from ane_amd.profile_summary import short
+    out = subprocess.run(["nm", "-C", os.path.join(ROOT, "ane_amd", "libmi355_ops.so")], capture_output=True, text=True, check=True).stdout
+    have = {short(line.split(" ", 2)[2]) for line in out.splitlines() if line.count(" ") >= 2}
+    for ops in (bench.OP_KERNELS, bench.EMBED_KERNELS):
+        for op, kernels in ops.items():
+            for k, _ in kernels:
+                assert k in have, (op, k)
