@@ -16,9 +16,9 @@
 // else.  Between calls they look for work for 100 us and then sleep.
 //
 // Results are unpacked as their bytes arrive.  A call that fails leaves the arrays that it updates in place as they were, so that
-// it can be made again: their results come back through a block of their own, and when a copy fails they are filled again from
-// the inputs' block, which still holds what was packed from them (unpacked behind the last copy instead, the nine calls took
-// 2.59 ms for 2.37).  Where one round cannot hold the inputs, such results wait in ordinary memory for the last copy.
+// it can be made again: a piece of such an array is copied to a log as it is packed, while the link is busy, and when a
+// copy back fails the arrays are filled again from there.  (Unpacked behind the last copy instead, the nine calls took 2.59 ms
+// for 2.37, and an Adam step of 3.1 M values, whose results came back in two rounds and waited in ordinary memory, 4.4 ms longer.)
 #pragma once
 
 constexpr int HELPERS = 3;
@@ -35,6 +35,7 @@ struct Part {
     size_t at, bytes;
     const int *rows;
     size_t row_bytes;
+    char *log;                           // what the array held before the call, or NULL
 };
 
 // memcpy past the caches: what the device reads next, or results that are larger than a cache (18.9 MB unpacked in 344 us, with
@@ -114,6 +115,7 @@ bool one_piece(Helpers *h) {
     const int i = (int)(n & 0xffffffffu);
     const Piece &p = h->piece[i];
     move_part(*p.part, p.from, p.bytes, p.block, h->in, h->past);
+    if (h->in && p.part->log) move_part(*p.part, p.from, p.bytes, p.part->log + p.from, true, true);
     h->done[i].store(1, std::memory_order_release);
     return true;
 }
@@ -209,29 +211,46 @@ Helpers *helpers() {
 }
 
 // ---- the blocks ----
-struct Pinned {
-    char *host, *dev;                                // its address here and on the device
-    size_t bytes;
-};
-Pinned g_pin = {}, g_pin_back = {};                  // the second for results of calls that update arrays in place
+char *g_pin = nullptr, *g_pin_dev = nullptr;         // the host's address of it and the device's
+size_t g_pin_bytes = 0;
 hipEvent_t g_sent[MAX_SENDS] = {};
+char *g_log = nullptr;                               // old values of arrays that a call updates
+size_t g_log_bytes = 0;
+constexpr size_t LOG_KEPT = (size_t)256 << 20;       // a longer one does not outlive its call
 
-// pinned memory for min(bytes, PIN_MAX) and the events of a round; false where there is none
-bool pinned(Pinned &p, size_t bytes) {
-    if (g_ctx.host_stage == 2) return false;
+// pinned memory for min(bytes, PIN_MAX) and the events of a round; NULL where there is none
+char *pinned(size_t bytes) {
+    if (g_ctx.host_stage == 2) return nullptr;
     if (!g_sent[MAX_SENDS - 1])
         for (auto &e : g_sent)
-            if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) { e = nullptr; (void)hipGetLastError(); return false; }
+            if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) { e = nullptr; (void)hipGetLastError(); return nullptr; }
     size_t want = (size_t)1 << 20;
     while (want < bytes && want < PIN_MAX) want *= 2;
-    if (p.host && p.bytes >= want) return true;
-    if (p.host) (void)hipHostFree(p.host);                 // (between calls nothing travels)
-    p = Pinned{};
-    void *h = nullptr, *d = nullptr;
-    if (hipHostMalloc(&h, want, hipHostMallocMapped) != hipSuccess) { (void)hipGetLastError(); return false; }
-    if (hipHostGetDevicePointer(&d, h, 0) != hipSuccess) { (void)hipGetLastError(); (void)hipHostFree(h); return false; }
-    p = Pinned{(char *)h, (char *)d, want};
-    return true;
+    if (g_pin && g_pin_bytes >= want) return g_pin;
+    if (g_pin) (void)hipHostFree(g_pin);                   // (between calls nothing travels)
+    g_pin = nullptr;
+    g_pin_bytes = 0;
+    void *p = nullptr;
+    if (hipHostMalloc(&p, want, hipHostMallocMapped) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
+    void *d = nullptr;
+    if (hipHostGetDevicePointer(&d, p, 0) != hipSuccess) { (void)hipGetLastError(); (void)hipHostFree(p); return nullptr; }
+    g_pin_bytes = want;
+    g_pin_dev = (char *)d;
+    return g_pin = (char *)p;
+}
+
+char *log_space(size_t bytes) {
+    if (bytes <= g_log_bytes) return g_log;
+    free(g_log);
+    g_log = (char *)malloc(bytes);
+    g_log_bytes = g_log ? bytes : 0;
+    if (!g_log) mi355_fail("no host memory for %zu bytes of old values", bytes);
+    return g_log;
+}
+void free_log() {
+    free(g_log);
+    g_log = nullptr;
+    g_log_bytes = 0;
 }
 
 // A copy between the pinned block and the device's: 16 bytes at a time, over the link at 50 GB/s from 1 MB on.  By a kernel, not
@@ -249,10 +268,10 @@ hipError_t stage_copy(char *to, const char *from, size_t bytes) {
 
 void free_stage() {
     stop_helpers();
-    for (Pinned *p : {&g_pin, &g_pin_back}) {
-        if (p->host) (void)hipHostFree(p->host);
-        *p = Pinned{};
-    }
+    if (g_pin) (void)hipHostFree(g_pin);
+    g_pin = g_pin_dev = nullptr;
+    g_pin_bytes = 0;
+    free_log();
     for (auto &e : g_sent) { if (e) (void)hipEventDestroy(e); e = nullptr; }
 }
 
@@ -276,14 +295,32 @@ public:
     // the part is a result from here on, and belongs to this array
     void becomes(int i, void *host) { p_[i].host = (char *)host; in_[i] = false; out_[i] = true; }
 
+    ~Stage() { if (g_log_bytes > LOG_KEPT) free_log(); }
+
     // device memory, and the inputs on their way to it
     bool send() {
         dev_ = (char *)slot(0, total_);
         if (!dev_) return false;
+        size_t updated = 0;
+        for (int i = 0; i < n_; i++)
+            if (in_[i] && out_[i]) updated += p_[i].bytes;
+        char *log = updated ? log_space(updated) : nullptr;
+        if (updated && !log) return false;
+        for (int i = 0; i < n_; i++)
+            if (in_[i] && out_[i]) {
+                p_[i].log = log;
+                log += p_[i].bytes;
+            }
         return move(true);
     }
-    // brings the results to their arrays; those that are inputs too are untouched unless it returns true
-    bool receive() { return move(false); }
+    // brings the results to their arrays; those that are inputs too are as before the call unless it returns true
+    bool receive() {
+        copies_ = 0;
+        if (move(false)) return true;
+        for (int i = 0; i < n_; i++)
+            if (p_[i].log) unpack(helpers(), p_[i], p_[i].log);
+        return false;
+    }
 
 private:
     static constexpr int MAX = 8;
@@ -292,12 +329,10 @@ private:
     int n_ = 0;
     size_t total_ = 0;
     char *dev_ = nullptr;
-    size_t sent_ = 0;           // where the inputs begin
-    bool packed_ = false;       // the pinned block holds all of them
     int copies_ = 0;            // of this receive()
 
     int add(void *host, size_t bytes, bool in, bool out) {
-        p_[n_] = Part{(char *)host, total_, bytes, nullptr, 0};
+        p_[n_] = Part{(char *)host, total_, bytes, nullptr, 0, nullptr};
         in_[n_] = in;
         out_[n_] = out;
         total_ += (bytes + 255) & ~(size_t)255;
@@ -318,58 +353,15 @@ private:
                 hi = std::max(hi, p_[i].at + p_[i].bytes);
             }
         if (lo >= hi) return true;
+        char *pin = pinned(total_);                        // (as large for both directions: it does not move while inputs travel)
         Helpers *h = helpers();
-        const bool pin = pinned(g_pin, total_) && h;       // (as large for both directions: it does not move while inputs travel)
-        if (in) {
-            sent_ = lo;
-            packed_ = pin && hi - lo <= g_pin.bytes;
-            return move_range(in, what, h, pin ? &g_pin : nullptr, lo, hi);
-        }
-        copies_ = 0;
-        size_t updated = 0;
-        for (int i = 0; i < n_; i++)
-            if (in_[i] && out_[i]) updated += p_[i].bytes;
-        if (updated == 0) return move_range(in, what, h, pin ? &g_pin : nullptr, lo, hi);
-        if (pin && packed_ && pinned(g_pin_back, hi - lo)) {
-            if (move_range(in, what, h, &g_pin_back, lo, hi)) return true;
-            for (int i = 0; i < n_; i++)
-                if (in_[i] && out_[i]) unpack(h, p_[i], g_pin.host + (p_[i].at - sent_));
-            return false;
-        }
-        char *const hold = (char *)malloc(updated);
-        if (!hold) {
-            mi355_fail("no host memory for %zu bytes of results", updated);
-            (void)hipStreamSynchronize(g_ctx.stream);
-            return false;
-        }
-        Part own[MAX];
-        char *to = hold;
-        for (int i = 0; i < n_; i++) {
-            own[i] = p_[i];
-            if (!in_[i] || !out_[i]) continue;
-            p_[i].host = to;
-            p_[i].rows = nullptr;
-            to += p_[i].bytes;
-        }
-        const bool ok = move_range(in, what, h, pin ? &g_pin : nullptr, lo, hi);
-        for (int i = 0; i < n_; i++) {
-            const char *from = p_[i].host;
-            p_[i] = own[i];
-            if (ok && in_[i] && out_[i]) unpack(h, p_[i], (char *)from);
-        }
-        free(hold);
-        return ok;
-    }
-
-    // the bytes lo .. hi - 1 of the device block, through a pinned one if there is one
-    bool move_range(bool in, const char *what, Helpers *h, const Pinned *pin, size_t lo, size_t hi) {
-        if (!pin) return move_unpinned(in, what);
-        for (size_t beg = lo; beg < hi; beg += pin->bytes) {
+        if (!pin || !h) return move_unpinned(in, what);
+        for (size_t beg = lo; beg < hi; beg += g_pin_bytes) {
             if (in && beg > lo) {                          // the block is filled again: the last round has to have left it
                 const hipError_t e = hipStreamSynchronize(g_ctx.stream);
                 if (e != hipSuccess) return fail(what, e);
             }
-            if (!round(in, what, h, *pin, beg, std::min(hi, beg + pin->bytes))) return false;
+            if (!round(in, what, h, pin, beg, std::min(hi, beg + g_pin_bytes))) return false;
         }
         return true;
     }
@@ -391,7 +383,7 @@ private:
     hipError_t back(hipError_t e) { return e == hipSuccess && ++copies_ == g_ctx.host_stage_fail ? hipErrorUnknown : e; }
 
     // bytes beg .. end - 1 of the device block, through the pinned one
-    bool round(bool in, const char *what, Helpers *h, const Pinned &pin, size_t beg, size_t end) {
+    bool round(bool in, const char *what, Helpers *h, char *pin, size_t beg, size_t end) {
         // the ends of the copies
         size_t cut[MAX_SENDS];
         int sends = 0;
@@ -415,7 +407,7 @@ private:
                 while (at >= cut[s]) last[s++] = pieces;
                 const size_t n = std::min(std::min(stop, cut[s]) - at, PIECE);
                 h->done[pieces].store(0, std::memory_order_relaxed);
-                h->piece[pieces++] = Piece{&p_[i], at - p_[i].at, n, pin.host + (at - beg)};
+                h->piece[pieces++] = Piece{&p_[i], at - p_[i].at, n, pin + (at - beg)};
                 at += n;
             }
         }
@@ -429,7 +421,7 @@ private:
             for (s = 0; s < sends;) {
                 while (ok < pieces && h->done[ok].load(std::memory_order_acquire)) ok++;
                 if (ok >= last[s]) {
-                    e = stage_copy(dev_ + from, pin.dev + (from - beg), cut[s] - from);
+                    e = stage_copy(dev_ + from, g_pin_dev + (from - beg), cut[s] - from);
                     if (e != hipSuccess) break;
                     from = cut[s++];
                 } else if (!one_piece(h)) {
@@ -439,7 +431,7 @@ private:
         } else {
             size_t from = beg;
             for (s = 0; s < sends && e == hipSuccess; s++) {
-                e = stage_copy(pin.dev + (from - beg), dev_ + from, cut[s] - from);
+                e = stage_copy(g_pin_dev + (from - beg), dev_ + from, cut[s] - from);
                 if (e == hipSuccess) e = hipEventRecord(g_sent[s], g_ctx.stream);
                 from = cut[s];
             }
@@ -463,6 +455,7 @@ private:
         for (int i = 0; i < n_; i++) {
             if (!(in ? in_[i] : out_[i])) continue;
             const Part &p = p_[i];
+            if (in && p.log) move_part(p, 0, p.bytes, p.log, true, true);
             const size_t step = p.rows ? p.row_bytes : p.bytes;
             for (size_t r = 0; r * step < p.bytes; r++) {
                 char *host = p.host + (p.rows ? (size_t)p.rows[r] * step : 0), *dev = dev_ + p.at + r * step;
