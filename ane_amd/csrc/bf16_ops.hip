@@ -662,7 +662,7 @@ BfCfg pick_bf(int C, bool vec_ok, int S, int batch) {
 Mi355Exchange g_bf_cluster_ws = {nullptr, nullptr, nullptr};
 ClusterPlan plan_cluster_bf(int C, int S, int batch, bool vec_ok, bool residual_bwd = false) {
     if (g_ctx.rms_lpr || g_ctx.rms_threads) return NO_CLUSTER;
-    return cluster_plan(C, S, batch, vec_ok, StoreBf16::VEC, 2, 4, 1, residual_bwd ? 32 : CL_MAX_BLOCKS);
+    return cluster_plan(C, S, batch, vec_ok, StoreBf16::VEC, 2, 4, 1, residual_bwd ? 3000000 : 0);
 }
 #define BF_CLUSTER_FWD(RPT, WHOLE)                                                                                   \
     hipLaunchKernelGGL((rms_fwd_cluster_kernel<StoreBf16, RPT, 1024, false, WHOLE>), dim3(cp.nblk), dim3(1024), 0,   \

@@ -487,9 +487,9 @@ ClusterWs g_cluster_ws = {nullptr, nullptr, nullptr};
 bool cluster_ws_ready(void) { return mi355_exchange(&g_cluster_ws); }
 
 // The single-workgroup tiles are chosen by hand (knobs) or the shape does not cluster: csplit == 0.
-ClusterPlan plan_cluster(int C, int S, int batch, bool vec_ok, int max_rpt, int rounds = 1) {      // max_rpt: 8 forward, 4 backward
+ClusterPlan plan_cluster(int C, int S, int batch, bool vec_ok, int max_rpt, int rounds = 1, size_t past = 0) {
     if (g_ctx.rms_lpr || g_ctx.rms_threads) return NO_CLUSTER;
-    return cluster_plan(C, S, batch, vec_ok, StoreF32::VEC, 4, max_rpt, rounds, max_rpt == 8 ? CL_MAX_BLOCKS : 24);
+    return cluster_plan(C, S, batch, vec_ok, StoreF32::VEC, 4, max_rpt, rounds, past);
 }
 
 template <int RPT, bool FUSE, int WHOLE>
@@ -578,7 +578,7 @@ MI355_API int mi355_rmsnorm_bwd_dev(float *dx, float *dw, const float *dy, const
     const bool vec_ok = S >= 4;
     // in place on dy the single-workgroup tile is used: a cluster member that has to recompute another member's
     // sums (its bounded wait expired) would read rows that their owner has already overwritten
-    const ClusterPlan cp = dx == dy ? NO_CLUSTER : plan_cluster(C, S, batch, vec_ok, 4);
+    const ClusterPlan cp = dx == dy ? NO_CLUSTER : plan_cluster(C, S, batch, vec_ok, 4, 1, 3000000);
     if (cp.csplit) {
         if (!cluster_ws_ready()) return -1;
         const int nrows = cp.nblk / cp.csplit;
@@ -613,7 +613,7 @@ MI355_API int mi355_rmsnorm_bwd_residual_dev(float *dx, float *dx_scaled, float 
     if (dx == x) return mi355_fail("rmsnorm_bwd_residual: dx must not alias x (dx may alias res or dy)");
     const bool vec_ok = S >= 4;
     const bool apart = dx != res || tail_in_strip(S, CL_LPR * StoreF32::VEC, StoreF32::VEC);
-    const ClusterPlan cp = dx == dy || !apart ? NO_CLUSTER : plan_cluster(C, S, batch, vec_ok, 4, 2);
+    const ClusterPlan cp = dx == dy || !apart ? NO_CLUSTER : plan_cluster(C, S, batch, vec_ok, 4, 2, 1500000);
     if (cp.csplit) {
         if (!cluster_ws_ready()) return -1;
         const int nrows = cp.nblk / cp.csplit;

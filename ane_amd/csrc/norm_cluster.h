@@ -79,9 +79,12 @@ static_assert(CL_SLOT_STRIDE >= 2 * CL_LPR * StoreBf16::VEC, "two quantities per
 // residual 34.8 / 36.4, [32][768][256] with it 25.6 / 28.0; [22][1024][147] 18.0 / 15.9, [8][768][197] 9.2 / 8.3, with the residual
 // 10.3 / 9.2, [115][768][54] with it 21.4 / 22.5 (20.1 of operands that the last-level cache holds); bfloat16 [32][768][256] with the
 // residual 17.1 / 19.9, [22][1024][147] 14.4 / 12.6.
-// Backward kernels of many clusters are quicker past them all the same, time past them over through them at C = 512 / 768 / 1024: fp32
-// 8 clusters 0.98 / 1.01 / 1.03, with the residual 1.02 / 1.05 / 1.07; 28 0.99 / 0.96 / 0.97, 0.97 / 0.96 / 0.97; 64 0.95 / 0.94 / 0.94,
-// 0.95 / 0.96 / 0.96.  bfloat16 with the residual 8 1.01 / 1.03 / 1.05; 32 0.98 / 0.98 / 0.98; 64 0.97 / 0.96 / 0.94; without it 0.97 to 1.04.
+// Backward kernels of large tensors are quicker past them all the same, if nothing of their operands is in the last-level cache, time
+// past them over through them at C = 512 / 768 / 1024: fp32 8 clusters 0.98 / 1.01 / 1.03, with the residual 1.02 / 1.05 / 1.07; 28 0.99 / 0.96
+// / 0.97, 0.97 / 0.96 / 0.97; 64 0.95 / 0.94 / 0.94, 0.95 / 0.96 / 0.96; bfloat16 with the residual 32 0.98, 64 0.97 / 0.96 / 0.94.  In a
+// layer the operands of smaller tensors still are: fused fp32 layer of [8][768][197] (4.8 MB) 70.4 us through, 71.7 past, of [16][1024][100]
+// (6.6 MB) 106.4, 103.2, of [32][768][100] 117.6, 112.3; one call per op [32][768][100] (9.8 MB) 124.5, 125.6, [12][1024][250] (12.3 MB)
+// 185.3, 181.2; bfloat16 [40][1024][100] (8.2 MB) 129.3, 124.6.
 // CL_EXACT: every member holds exactly RPS*RPT rows and every strip is whole; CL_LINES: rows are read past the caches; CL_ANY: neither.  (One
 // kernel with the loads written twice behind a branch took 27.9 us for the 25.4 of [32][768][256].)
 // CL_FEW, with one of the latter two: the members' rows fill at most half of their tiles.  Then the row steps in which no lane has a row
@@ -498,9 +501,9 @@ constexpr ClusterPlan NO_CLUSTER = {0, 0, 0, 0, 0, 0, CL_ANY};
 // the single-workgroup tiles with 128-byte strips (forward 30.0 against 29.1 us, backward 22.3 against 19.9 us),
 // except for the backward with the residual, whose single-workgroup tile is the weakest (32.7 against 43.7 us).
 // vec: columns per lane of the storage type; rpt_lo..rpt_hi: rows per lane that are instantiated (powers of two);
-// rounds: how many workgroups per compute unit a launch may have (1: all resident at once).  past_from: clusters from which on rows
-// that are not whole lines are read past the caches as well (cluster_load).
-ClusterPlan cluster_plan(int C, int S, int batch, bool vec_ok, int vec, int rpt_lo, int rpt_hi, int rounds, int past_from = CL_MAX_BLOCKS) {
+// rounds: how many workgroups per compute unit a launch may have (1: all resident at once).  past: values of a tensor from which on
+// rows that are not whole lines are read past the caches as well (cluster_load); 0: never.
+ClusterPlan cluster_plan(int C, int S, int batch, bool vec_ok, int vec, int rpt_lo, int rpt_hi, int rounds, size_t past = 0) {
     ClusterPlan p = NO_CLUSTER;
     if (!vec_ok || C < 512 || g_ctx.rms_cluster < 0) return p;
     const int w = CL_LPR * vec;
@@ -528,7 +531,8 @@ ClusterPlan cluster_plan(int C, int S, int batch, bool vec_ok, int vec, int rpt_
     p.threads = threads;
     p.strips = (int)strips;
     p.nblk = (int)(clusters * split);
-    p.whole = rows == rps * rpt && rows * split == C && S % w == 0 ? CL_EXACT : (S % (w / 2) == 0 || clusters >= past_from ? CL_LINES : CL_ANY) + (2 * rows <= rps * rpt ? CL_FEW : 0);
+    const bool read_past = past > 0 && clusters >= 24 && (size_t)C * S * batch >= past;
+    p.whole = rows == rps * rpt && rows * split == C && S % w == 0 ? CL_EXACT : (S % (w / 2) == 0 || read_past ? CL_LINES : CL_ANY) + (2 * rows <= rps * rpt ? CL_FEW : 0);
     return p;
 }
 // (a tile of more than the fewest rows per lane is at least half full: no CL_FEW there)

@@ -1,5 +1,5 @@
 """Both sides of lines at which the clustered norms and the fp32 QK-norm + RoPE forward change their kernel: members whose rows fill
-half of a tile, a row more and fewer; clusters from which on rows of any length are read past the caches; eight rows per lane
+half of a tile, a row more and fewer; tensors from which on rows of any length are read past the caches; eight rows per lane
 with the residual; rows of a head without conditions, by the workgroups to one of 256 compute units and the fill of a strip."""
 import pytest
 
@@ -18,7 +18,8 @@ def br():
 
 @pytest.mark.parametrize("bf16", [False, True])
 @pytest.mark.parametrize("B,C,S", [(1, 512, 32), (2, 512, 33), (1, 513, 100), (3, 520, 64), (1, 1024, 54), (1, 1032, 54),     # rows of a member
-                                   (11, 512, 100), (12, 512, 100), (31, 768, 100), (32, 768, 100), (33, 520, 65),             # clusters
+                                   (11, 512, 100), (12, 512, 100), (31, 768, 100), (32, 768, 100), (33, 520, 65),             # clusters, not large enough
+                                   (15, 1000, 100), (15, 1000, 99), (30, 1000, 101), (31, 1000, 97),                          # values of a tensor
                                    (40, 1024, 100), (50, 1000, 67), (64, 768, 33)])                                           # rows per lane
 def test_norm_clusters(br, B, C, S, bf16):
     R.test_rmsnorm_family_on_rows_of_any_length(br, B, C, S, bf16, 1)
