@@ -413,7 +413,8 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_fwd_bf16_kernel(
 }
 
 // Where a lane has one or two row pairs it keeps their un-rotated gradients across the reduction, in place of the packed upstream
-// ones: the table is read once and the rotation undone once (24.2 -> 22.9 us; with whole tiles 22.0 -> 20.0, with loads through the caches 16.7; 123 registers).
+// ones: the table is read once and the rotation undone once (24.2 -> 22.9 us; with whole tiles 22.0 -> 20.0, with loads through the
+// caches 16.7; 123 registers).
 template <int VEC, int LPR, int THREADS, int CAP, int WHOLE>
 __global__ __launch_bounds__(THREADS) void qknorm_rope_bwd_bf16_kernel(
     bf16_t *dq, bf16_t *dk, float *__restrict__ part, const bf16_t *dq_out, const bf16_t *dk_out,
@@ -597,7 +598,7 @@ bool pick_qk_bf(int hd, int S, size_t slabs, bool in_place, bool backward, QkBf 
         hipLaunchKernelGGL((KERNEL<V, L, T, CP, QK_SOME>), grid, dim3(T), 0, g_ctx.stream, __VA_ARGS__);             \
         break;
 // tiles that a head size of 64 or 128 fills (more than one column per lane: QK_ROWS needs rows of a whole group)
-#define QKBF_CASE_EXACT(KERNEL, V, L, T, CP, grid, ...)                                                              \
+#define QKBF_CASE_WHOLE(KERNEL, V, L, T, CP, grid, ...)                                                              \
     case (V) * 1000000 + (L) * 10000 + ((T) / 256) * 100 + (CP):                                                     \
         if ((T) / (L) * (CP) == hd / 2 && S % ((L) * (V)) == 0)                                                      \
             hipLaunchKernelGGL((KERNEL<V, L, T, CP, QK_ALL>), grid, dim3(T), 0, g_ctx.stream, __VA_ARGS__);          \
@@ -610,10 +611,10 @@ bool pick_qk_bf(int hd, int S, size_t slabs, bool in_place, bool backward, QkBf 
     do {                                                                                                             \
         switch ((cfg).vec * 1000000 + (cfg).lpr * 10000 + ((cfg).threads / 256) * 100 + (cfg).cap) {                 \
             QKBF_CASE(KERNEL, 1, 64, 1024, 4, grid, __VA_ARGS__)                                                     \
-            QKBF_CASE(KERNEL, 8, 16, 256, 1, grid, __VA_ARGS__) QKBF_CASE_EXACT(KERNEL, 8, 16, 256, 2, grid, __VA_ARGS__)  \
+            QKBF_CASE(KERNEL, 8, 16, 256, 1, grid, __VA_ARGS__) QKBF_CASE_WHOLE(KERNEL, 8, 16, 256, 2, grid, __VA_ARGS__)  \
             QKBF_CASE(KERNEL, 8, 16, 256, 4, grid, __VA_ARGS__) QKBF_CASE(KERNEL, 8, 16, 512, 1, grid, __VA_ARGS__)  \
-            QKBF_CASE_EXACT(KERNEL, 8, 16, 512, 2, grid, __VA_ARGS__) QKBF_CASE(KERNEL, 8, 16, 512, 4, grid, __VA_ARGS__)  \
-            QKBF_CASE(KERNEL, 8, 8, 256, 1, grid, __VA_ARGS__) QKBF_CASE_EXACT(KERNEL, 8, 8, 256, 2, grid, __VA_ARGS__)    \
+            QKBF_CASE_WHOLE(KERNEL, 8, 16, 512, 2, grid, __VA_ARGS__) QKBF_CASE(KERNEL, 8, 16, 512, 4, grid, __VA_ARGS__)  \
+            QKBF_CASE(KERNEL, 8, 8, 256, 1, grid, __VA_ARGS__) QKBF_CASE_WHOLE(KERNEL, 8, 8, 256, 2, grid, __VA_ARGS__)    \
             QKBF_CASE(KERNEL, 8, 8, 256, 4, grid, __VA_ARGS__) QKBF_CASE(KERNEL, 8, 8, 512, 1, grid, __VA_ARGS__)    \
             QKBF_CASE(KERNEL, 8, 8, 512, 2, grid, __VA_ARGS__) QKBF_CASE(KERNEL, 8, 8, 512, 4, grid, __VA_ARGS__)    \
             QKBF_CASE(KERNEL, 8, 4, 256, 1, grid, __VA_ARGS__) QKBF_CASE(KERNEL, 8, 4, 256, 2, grid, __VA_ARGS__)    \

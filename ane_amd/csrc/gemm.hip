@@ -373,7 +373,8 @@ GemmPlan plan_gemm(int ta, int tb, int M, int N, int K, bool reads_c, int lda, i
     const double split_us = 1.9 + (4.0 * N * K + planes) / 15.4e6;         // the launch that splits B
     const double c_times = reads_c ? 2 : 1;
     for (const GemmKernel &t : GEMM_KERNELS) {
-        const int id = !t.split ? -1 : t.split == 2 ? (t.bm == 96 ? 5 : 6) : t.bm == 64 ? 2 + t.groups : t.bm / 128;         // as the knob numbers them
+        // as the knob numbers them
+        const int id = !t.split ? -1 : t.split == 2 ? (t.bm == 96 ? 5 : 6) : t.bm == 64 ? 2 + t.groups : t.bm / 128;
         if (t.split == 2 && !planes_ok) continue;
         if (knob ? (knob < 0 ? t.split != 0 : id != knob) : t.split != 2 && t.bm * t.bn > 64 * 64 && K < 80) continue;
         const double tiles_m = (double)ceil_div((size_t)M, (size_t)t.bm), tiles_n = (double)ceil_div((size_t)N, (size_t)t.bn);

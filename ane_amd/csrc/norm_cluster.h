@@ -79,18 +79,19 @@ static_assert(CL_SLOT_STRIDE >= 2 * CL_LPR * StoreBf16::VEC, "two quantities per
 // residual 34.8 / 36.4, [32][768][256] with it 25.6 / 28.0; [22][1024][147] 18.0 / 15.9, [8][768][197] 9.2 / 8.3, with the residual
 // 10.3 / 9.2, [115][768][54] with it 21.4 / 22.5 (20.1 of operands that the last-level cache holds); bfloat16 [32][768][256] with the
 // residual 17.1 / 19.9, [22][1024][147] 14.4 / 12.6.
-// Backward kernels of large tensors are quicker past them all the same, if nothing of their operands is in the last-level cache, time
-// past them over through them at C = 512 / 768 / 1024: fp32 8 clusters 0.98 / 1.01 / 1.03, with the residual 1.02 / 1.05 / 1.07; 28 0.99 / 0.96
-// / 0.97, 0.97 / 0.96 / 0.97; 64 0.95 / 0.94 / 0.94, 0.95 / 0.96 / 0.96; bfloat16 with the residual 32 0.98, 64 0.97 / 0.96 / 0.94.  In a
-// layer the operands of smaller tensors still are: fused fp32 layer of [8][768][197] (4.8 MB) 70.4 us through, 71.7 past, of [16][1024][100]
-// (6.6 MB) 106.4, 103.2, of [32][768][100] 117.6, 112.3; one call per op [32][768][100] (9.8 MB) 124.5, 125.6, [12][1024][250] (12.3 MB)
-// 185.3, 181.2; bfloat16 [40][1024][100] (8.2 MB) 129.3, 124.6.
-// CL_EXACT: every member holds exactly RPS*RPT rows and every strip is whole; CL_LINES: rows are read past the caches; CL_ANY: neither.  (One
-// kernel with the loads written twice behind a branch took 27.9 us for the 25.4 of [32][768][256].)
-// CL_FEW, with one of the latter two: the members' rows fill at most half of their tiles.  Then the row steps in which no lane has a row
-// are passed over; elsewhere that costs more than it saves.  fp32 backward with the residual, us, loaded all the same / passed over:
-// [1][512][32] 8.8 / 7.9, [8][512][54] 9.4 / 8.4, [16][512][147] 18.0 / 17.2; bfloat16 [4][512][33] 11.7 / 10.9 (12.1 / 12.6 for
-// [4][1024][54], where they fill it).
+// Backward kernels of large tensors are quicker past them all the same, if nothing of their operands is in the last-level cache.  Time
+// past them over through them at C = 512 / 768 / 1024: fp32, 8 clusters, 0.98 / 1.01 / 1.03, with the residual 1.02 / 1.05 / 1.07;
+// 28 clusters 0.99 / 0.96 / 0.97 and 0.97 / 0.96 / 0.97; 64 clusters 0.95 / 0.94 / 0.94 and 0.95 / 0.96 / 0.96; bfloat16 with the
+// residual, 32 clusters 0.98, 64 clusters 0.97 / 0.96 / 0.94.  In a layer the operands of smaller tensors still are: fused fp32
+// layer of [8][768][197] (4.8 MB) 70.4 us through, 71.7 past, of [16][1024][100] (6.6 MB) 106.4 and 103.2, of [32][768][100] 117.6
+// and 112.3; one call per op [32][768][100] (9.8 MB) 124.5 and 125.6, [12][1024][250] (12.3 MB) 185.3 and 181.2; bfloat16
+// [40][1024][100] (8.2 MB) 129.3 and 124.6.
+// CL_EXACT: every member holds exactly RPS*RPT rows and every strip is whole; CL_LINES: rows are read past the caches; CL_ANY:
+// neither.  (One kernel with the loads written twice behind a branch took 27.9 us for the 25.4 of [32][768][256].)
+// CL_FEW, with one of the latter two: the members' rows fill at most half of their tiles.  Then the row steps in which no lane has
+// a row are passed over; elsewhere that costs more than it saves.  Backward with the residual, us, loaded all the same / passed
+// over: fp32 [1][512][32] 8.4 / 8.0, [8][512][54] 9.3 / 8.8, [16][512][147] 18.0 / 17.3, bfloat16 [4][512][33] 11.6 / 10.9;
+// forward, bfloat16 [4][768][33], three quarters full, 6.5 / 6.7.
 enum { CL_ANY, CL_LINES, CL_EXACT, CL_FEW };
 constexpr bool cl_lines(int whole) { return whole == CL_EXACT || whole % CL_FEW == CL_LINES; }
 template <typename ST, int WHOLE>
@@ -532,7 +533,9 @@ ClusterPlan cluster_plan(int C, int S, int batch, bool vec_ok, int vec, int rpt_
     p.strips = (int)strips;
     p.nblk = (int)(clusters * split);
     const bool read_past = past > 0 && clusters >= 24 && (size_t)C * S * batch >= past;
-    p.whole = rows == rps * rpt && rows * split == C && S % w == 0 ? CL_EXACT : (S % (w / 2) == 0 || read_past ? CL_LINES : CL_ANY) + (2 * rows <= rps * rpt ? CL_FEW : 0);
+    p.whole = rows == rps * rpt && rows * split == C && S % w == 0
+                  ? CL_EXACT
+                  : (S % (w / 2) == 0 || read_past ? CL_LINES : CL_ANY) + (2 * rows <= rps * rpt ? CL_FEW : 0);
     return p;
 }
 // (a tile of more than the fewest rows per lane is at least half full: no CL_FEW there)

@@ -99,7 +99,7 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_bwd_kernel(
     const float *__restrict__ q, const float *__restrict__ k, const float *__restrict__ wq,
     const float *__restrict__ wk, int hd, int S, int strips, int nq, const float *__restrict__ cos_t,
     const float *__restrict__ sin_t, float eps, float invhd, int variant) {
-    constexpr bool EXACT = WHOLE == QK_ALL, ROWS = WHOLE == QK_ROWS;
+    constexpr bool ALL = WHOLE == QK_ALL, ROWS = WHOLE == QK_ROWS;
     constexpr int PPS = THREADS / LPR;
     constexpr int W = LPR * 4;
     constexpr int NW = THREADS / 64;
@@ -124,7 +124,7 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_bwd_kernel(
 #pragma unroll
     for (int kk = 0; kk < CAP; kk++) {
         const int rp = p0 + kk * PPS;
-        if (EXACT || ROWS || (rp < half && col_ok)) {
+        if (ALL || ROWS || (rp < half && col_ok)) {
             const size_t o = base + (size_t)(2 * rp) * S;
             x0[kk] = qk_load<ROWS>(xin + o);
             x1[kk] = qk_load<ROWS>(xin + o + S);
@@ -159,7 +159,7 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_bwd_kernel(
 #pragma unroll
     for (int kk = 0; kk < CAP; kk++) {
         const int rp = p0 + kk * PPS;
-        if (EXACT || ROWS || rp < half) {   // uniform over each group of LPR lanes
+        if (ALL || ROWS || rp < half) {   // uniform over each group of LPR lanes
             v4f o0, o1;
             if (variant == 0) {
                 o0 = ((d0[kk] - x0[kk] * dotn) * rr) * w0[kk];
@@ -168,7 +168,7 @@ __global__ __launch_bounds__(THREADS) void qknorm_rope_bwd_kernel(
                 o0 = (d0[kk] * w0[kk]) * rr - (x0[kk] * dotn) * rr;
                 o1 = (d1[kk] * w1[kk]) * rr - (x1[kk] * dotn) * rr;
             }
-            if (EXACT || col_ok) {
+            if (ALL || col_ok) {
                 float *po = out + base + (size_t)(2 * rp) * S;
                 st4_nt(po, o0);
                 st4_nt(po + S, o1);
@@ -241,8 +241,8 @@ bool pick_qk(int hd, int S, bool in_place, QkCfg &cfg, bool backward) {
 // Rows that are not whole 128-byte lines, on a tile that the head's row pairs fill (hd 128 and 64): the ROWS kernels.
 bool whole_rows(const QkCfg &cfg, int hd, int S) { return S % 32 != 0 && cfg.lpr == 16 && cfg.threads / 16 * cfg.cap * 2 == hd; }
 // Where the forward is quicker with them, by the workgroups to a compute unit.  The other kernel does best just before its workgroups
-// need another round: hd 64 from four to five of them ([12][24 x 64][197] 10.5 us, ROWS 12.3; with eight 15.4 and 14.0), hd 128 from
-// three to four ([12][24 x 128][147] 16.0, 17.1; with three 13.5, 13.0).  And lanes past the end of a row ask again for what others
+// need another round: hd 64 from four to five of them ([12][24 x 64][197] 10.5 us, ROWS 12.3; six, [16], 15.3 and 13.9), hd 128 from
+// three to four ([12][24 x 128][147] 16.0, 17.1; three, [16][24 x 128][100], 13.5, 13.0).  Lanes past the end of a row ask for what others
 // have: in a single strip that costs more than it saves from three on ([64][24 x 64][54] 9.7, 11.3; [32][24 x 128][54] 9.2, 10.7;
 // [4][24 x 128][54] 6.2, 4.4), and in two of which the second is nearly empty from six on ([30][24 x 64][70] 1.15 times as long).
 bool forward_rows(int hd, int S, size_t workgroups) {

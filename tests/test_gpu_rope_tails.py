@@ -1,5 +1,4 @@
-"""RoPE on rows whose last group of columns is short, in both storages: out of place, in place, Q rotated into K's place; rows of
-less than a group; tensors at any element.  The same products and sums as the oracle's, so the same bits."""
+"""RoPE on rows whose last group of columns is short, in both storages: out of place and in place; rows of less than a group; tensors at any element.  The same products and sums as the oracle's, so the same bits."""
 import numpy as np
 import pytest
 import torch
