@@ -16,9 +16,10 @@
 // else.  Between calls they look for work for 100 us and then sleep.
 //
 // Results are unpacked as their bytes arrive.  A call that fails leaves the arrays that it updates in place as they were, so that
-// it can be made again: a piece of such an array is copied to a log as it is packed, while the link is busy, and when a
-// copy back fails the arrays are filled again from there.  (Unpacked behind the last copy instead, the nine calls took 2.59 ms
-// for 2.37, and an Adam step of 3.1 M values, whose results came back in two rounds and waited in ordinary memory, 4.4 ms longer.)
+// it can be made again: when a copy back fails they are filled again with what they held.  Where one round holds the inputs, that
+// is still in the pinned block, and the results come back through another (unpacked behind the last copy instead, the nine calls took
+// 2.59 ms for 2.37); otherwise each piece of such an array is copied to a log as it is packed, which costs 1 to 2 %
+// (results held in ordinary memory until the last copy: nine calls 8.5 ms for 4.1).
 #pragma once
 
 constexpr int HELPERS = 3;
@@ -35,7 +36,7 @@ struct Part {
     size_t at, bytes;
     const int *rows;
     size_t row_bytes;
-    char *log;                           // what the array held before the call, or NULL
+    char *log;                           // where what the array held is copied to while it is packed, or NULL
 };
 
 // memcpy past the caches: what the device reads next, or results that are larger than a cache (18.9 MB unpacked in 344 us, with
@@ -84,6 +85,8 @@ struct Piece {
     char *block;
 };
 
+enum : unsigned char { TO_DO, PACKED, DONE };       // PACKED: may be sent, the log is still to come
+
 struct Helpers {
     pthread_t thread[HELPERS];
     int n;                                // created
@@ -115,8 +118,11 @@ bool one_piece(Helpers *h) {
     const int i = (int)(n & 0xffffffffu);
     const Piece &p = h->piece[i];
     move_part(*p.part, p.from, p.bytes, p.block, h->in, h->past);
-    if (h->in && p.part->log) move_part(*p.part, p.from, p.bytes, p.part->log + p.from, true, true);
-    h->done[i].store(1, std::memory_order_release);
+    if (h->in && p.part->log) {
+        h->done[i].store(PACKED, std::memory_order_release);
+        move_part(*p.part, p.from, p.bytes, p.part->log + p.from, true, true);
+    }
+    h->done[i].store(DONE, std::memory_order_release);
     return true;
 }
 
@@ -147,7 +153,7 @@ void end_pieces(Helpers *h, int pieces, unsigned long long number, bool ok) {
     if (ok) while (one_piece(h)) { }
     else taken = std::min(pieces, (int)(h->next.exchange((number << 32) | 0x7fffffffu) & 0x7fffffffu));
     for (int i = 0; i < taken; i++)
-        while (!h->done[i].load(std::memory_order_acquire)) __builtin_ia32_pause();
+        while (h->done[i].load(std::memory_order_acquire) != DONE) __builtin_ia32_pause();
     h->active.store(0);
 }
 
@@ -211,32 +217,32 @@ Helpers *helpers() {
 }
 
 // ---- the blocks ----
-char *g_pin = nullptr, *g_pin_dev = nullptr;         // the host's address of it and the device's
-size_t g_pin_bytes = 0;
+struct Pinned {
+    char *host, *dev;                                // its address here and on the device
+    size_t bytes;
+};
+Pinned g_pin = {}, g_pin_back = {};                  // the second for results of calls that update arrays
 hipEvent_t g_sent[MAX_SENDS] = {};
 char *g_log = nullptr;                               // old values of arrays that a call updates
 size_t g_log_bytes = 0;
 constexpr size_t LOG_KEPT = (size_t)256 << 20;       // a longer one does not outlive its call
 
-// pinned memory for min(bytes, PIN_MAX) and the events of a round; NULL where there is none
-char *pinned(size_t bytes) {
-    if (g_ctx.host_stage == 2) return nullptr;
+// pinned memory for min(bytes, PIN_MAX) and the events of a round; false where there is none
+bool pinned(Pinned &p, size_t bytes) {
+    if (g_ctx.host_stage == 2) return false;
     if (!g_sent[MAX_SENDS - 1])
         for (auto &e : g_sent)
-            if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) { e = nullptr; (void)hipGetLastError(); return nullptr; }
+            if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) { e = nullptr; (void)hipGetLastError(); return false; }
     size_t want = (size_t)1 << 20;
     while (want < bytes && want < PIN_MAX) want *= 2;
-    if (g_pin && g_pin_bytes >= want) return g_pin;
-    if (g_pin) (void)hipHostFree(g_pin);                   // (between calls nothing travels)
-    g_pin = nullptr;
-    g_pin_bytes = 0;
-    void *p = nullptr;
-    if (hipHostMalloc(&p, want, hipHostMallocMapped) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
-    void *d = nullptr;
-    if (hipHostGetDevicePointer(&d, p, 0) != hipSuccess) { (void)hipGetLastError(); (void)hipHostFree(p); return nullptr; }
-    g_pin_bytes = want;
-    g_pin_dev = (char *)d;
-    return g_pin = (char *)p;
+    if (p.host && p.bytes >= want) return true;
+    if (p.host) (void)hipHostFree(p.host);                 // (between calls nothing travels)
+    p = Pinned{};
+    void *h = nullptr, *d = nullptr;
+    if (hipHostMalloc(&h, want, hipHostMallocMapped) != hipSuccess) { (void)hipGetLastError(); return false; }
+    if (hipHostGetDevicePointer(&d, h, 0) != hipSuccess) { (void)hipGetLastError(); (void)hipHostFree(h); return false; }
+    p = Pinned{(char *)h, (char *)d, want};
+    return true;
 }
 
 char *log_space(size_t bytes) {
@@ -268,9 +274,10 @@ hipError_t stage_copy(char *to, const char *from, size_t bytes) {
 
 void free_stage() {
     stop_helpers();
-    if (g_pin) (void)hipHostFree(g_pin);
-    g_pin = g_pin_dev = nullptr;
-    g_pin_bytes = 0;
+    for (Pinned *p : {&g_pin, &g_pin_back}) {
+        if (p->host) (void)hipHostFree(p->host);
+        *p = Pinned{};
+    }
     free_log();
     for (auto &e : g_sent) { if (e) (void)hipEventDestroy(e); e = nullptr; }
 }
@@ -304,13 +311,18 @@ public:
         size_t updated = 0;
         for (int i = 0; i < n_; i++)
             if (in_[i] && out_[i]) updated += p_[i].bytes;
-        char *log = updated ? log_space(updated) : nullptr;
-        if (updated && !log) return false;
-        for (int i = 0; i < n_; i++)
-            if (in_[i] && out_[i]) {
-                p_[i].log = log;
-                log += p_[i].bytes;
-            }
+        // (no pinned memory: each array by itself, and the log)
+        pin_ = helpers() && pinned(g_pin, total_) ? &g_pin : nullptr;
+        back_ = pin_ && updated && total_ <= pin_->bytes && pinned(g_pin_back, total_) ? &g_pin_back : pin_;
+        if (updated && back_ == pin_) {
+            char *log = log_space(updated);
+            if (!log) return false;
+            for (int i = 0; i < n_; i++)
+                if (in_[i] && out_[i]) {
+                    p_[i].log = log;
+                    log += p_[i].bytes;
+                }
+        }
         return move(true);
     }
     // brings the results to their arrays; those that are inputs too are as before the call unless it returns true
@@ -318,7 +330,7 @@ public:
         copies_ = 0;
         if (move(false)) return true;
         for (int i = 0; i < n_; i++)
-            if (p_[i].log) unpack(helpers(), p_[i], p_[i].log);
+            if (in_[i] && out_[i]) unpack(helpers(), p_[i], p_[i].log ? p_[i].log : g_pin.host + (p_[i].at - sent_));
         return false;
     }
 
@@ -329,6 +341,8 @@ private:
     int n_ = 0;
     size_t total_ = 0;
     char *dev_ = nullptr;
+    const Pinned *pin_ = nullptr, *back_ = nullptr;         // what the inputs and the results go through; NULL: nothing
+    size_t sent_ = 0;           // where the inputs begin
     int copies_ = 0;            // of this receive()
 
     int add(void *host, size_t bytes, bool in, bool out) {
@@ -353,15 +367,16 @@ private:
                 hi = std::max(hi, p_[i].at + p_[i].bytes);
             }
         if (lo >= hi) return true;
-        char *pin = pinned(total_);                        // (as large for both directions: it does not move while inputs travel)
+        if (in) sent_ = lo;
+        const Pinned *pin = in ? pin_ : back_;
         Helpers *h = helpers();
         if (!pin || !h) return move_unpinned(in, what);
-        for (size_t beg = lo; beg < hi; beg += g_pin_bytes) {
+        for (size_t beg = lo; beg < hi; beg += pin->bytes) {
             if (in && beg > lo) {                          // the block is filled again: the last round has to have left it
                 const hipError_t e = hipStreamSynchronize(g_ctx.stream);
                 if (e != hipSuccess) return fail(what, e);
             }
-            if (!round(in, what, h, pin, beg, std::min(hi, beg + g_pin_bytes))) return false;
+            if (!round(in, what, h, *pin, beg, std::min(hi, beg + pin->bytes))) return false;
         }
         return true;
     }
@@ -372,7 +387,7 @@ private:
         for (size_t at = 0; at < p.bytes;) {
             int pieces = 0;
             for (; pieces < MAX_PIECES && at < p.bytes; at += PIECE) {
-                h->done[pieces].store(0, std::memory_order_relaxed);
+                h->done[pieces].store(TO_DO, std::memory_order_relaxed);
                 h->piece[pieces++] = Piece{&p, at, std::min(p.bytes - at, PIECE), from + at};
             }
             end_pieces(h, pieces, start_pieces(h, pieces, pieces, false, true), true);
@@ -383,7 +398,7 @@ private:
     hipError_t back(hipError_t e) { return e == hipSuccess && ++copies_ == g_ctx.host_stage_fail ? hipErrorUnknown : e; }
 
     // bytes beg .. end - 1 of the device block, through the pinned one
-    bool round(bool in, const char *what, Helpers *h, char *pin, size_t beg, size_t end) {
+    bool round(bool in, const char *what, Helpers *h, const Pinned &pin, size_t beg, size_t end) {
         // the ends of the copies
         size_t cut[MAX_SENDS];
         int sends = 0;
@@ -406,8 +421,8 @@ private:
             while (at < stop) {
                 while (at >= cut[s]) last[s++] = pieces;
                 const size_t n = std::min(std::min(stop, cut[s]) - at, PIECE);
-                h->done[pieces].store(0, std::memory_order_relaxed);
-                h->piece[pieces++] = Piece{&p_[i], at - p_[i].at, n, pin + (at - beg)};
+                h->done[pieces].store(TO_DO, std::memory_order_relaxed);
+                h->piece[pieces++] = Piece{&p_[i], at - p_[i].at, n, pin.host + (at - beg)};
                 at += n;
             }
         }
@@ -419,9 +434,9 @@ private:
             int ok = 0;
             size_t from = beg;
             for (s = 0; s < sends;) {
-                while (ok < pieces && h->done[ok].load(std::memory_order_acquire)) ok++;
+                while (ok < pieces && h->done[ok].load(std::memory_order_acquire) != TO_DO) ok++;
                 if (ok >= last[s]) {
-                    e = stage_copy(dev_ + from, g_pin_dev + (from - beg), cut[s] - from);
+                    e = stage_copy(dev_ + from, pin.dev + (from - beg), cut[s] - from);
                     if (e != hipSuccess) break;
                     from = cut[s++];
                 } else if (!one_piece(h)) {
@@ -431,7 +446,7 @@ private:
         } else {
             size_t from = beg;
             for (s = 0; s < sends && e == hipSuccess; s++) {
-                e = stage_copy(g_pin_dev + (from - beg), dev_ + from, cut[s] - from);
+                e = stage_copy(pin.dev + (from - beg), dev_ + from, cut[s] - from);
                 if (e == hipSuccess) e = hipEventRecord(g_sent[s], g_ctx.stream);
                 from = cut[s];
             }

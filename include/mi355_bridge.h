@@ -472,8 +472,8 @@ int mi355_vocab_scatter_grads_dev(float *full_grad, const float *compact_grad, c
 
 /* ------------------------------------------------------------------------------------------
  * Host-pointer drop-ins: the reference signatures verbatim (host float* in, host float* out),
- * so a caller swaps the symbol only.  Each call stages through a pinned block of at most 32 MB, which three threads of the
- * library help to fill and empty, and cached device buffers (H2D, kernel, D2H) and returns when the result is in host
+ * so a caller swaps the symbol only.  Each call stages through pinned blocks of at most 32 MB (a second one for the results of
+ * calls that update arrays), which three threads of the library help to fill and empty, and cached device buffers (H2D, kernel, D2H) and returns when the result is in host
  * memory.  On failure they print one line to stderr and leave the arrays that they update (dw, d_embed, w, m, v, dx of
  * mi355_rope_backward_inplace) untouched, so that the call can be made again; arrays that they only write are untouched unless
  * what failed is a copy back to the host, which may leave a part of the result in them.
