@@ -667,14 +667,14 @@ ClusterPlan plan_cluster_bf(int C, int S, int batch, bool vec_ok, bool residual_
 }
 #define BF_CLUSTER_FWD(RPT, WHOLE)                                                                                   \
     hipLaunchKernelGGL((rms_fwd_cluster_kernel<StoreBf16, RPT, 1024, false, WHOLE>), dim3(cp.nblk), dim3(1024), 0,   \
-                       g_ctx.stream, y, (uint16_t *)nullptr, x, (const uint16_t *)nullptr, 0.f, w, C, S, cp.strips,  \
-                       cp.nblk, cp.csplit, cp.rows_pm, eps, 1.0f / (float)C, g_bf_cluster_ws,                        \
-                       mi355_exchange_spin_ticks())
+                       g_ctx.stream, x, (const uint16_t *)nullptr, w, g_bf_cluster_ws.cnt, C, S, cp.word_a(),        \
+                       cp.word_b(), y, (uint16_t *)nullptr, 0.f, eps, 1.0f / (float)C, g_bf_cluster_ws.slots,        \
+                       g_bf_cluster_ws.fallbacks, mi355_exchange_spin_ticks())
 #define BF_CLUSTER_BWD(RPT, WHOLE)                                                                                   \
     hipLaunchKernelGGL((rms_bwd_cluster_kernel<StoreBf16, RPT, 1024, false, WHOLE>), dim3(cp.nblk), dim3(1024), 0,   \
-                       g_ctx.stream, dx, part, dy, x, w, C, S, cp.strips, cp.nblk, cp.csplit, cp.rows_pm, eps,       \
-                       1.0f / (float)C, variant, (const uint16_t *)nullptr, (uint16_t *)nullptr, 0.f,                \
-                       g_bf_cluster_ws, mi355_exchange_spin_ticks())
+                       g_ctx.stream, x, dy, w, g_bf_cluster_ws.cnt, C, S, cp.word_a(), cp.word_b(),                  \
+                       (const uint16_t *)nullptr, dx, part, (uint16_t *)nullptr, 0.f, eps, 1.0f / (float)C, variant, \
+                       g_bf_cluster_ws.slots, g_bf_cluster_ws.fallbacks, mi355_exchange_spin_ticks())
 
 #define BF_CASE(KERNEL, V, L, T, CP, nblk, ...)                                                                      \
     case (V) * 1000000 + (L) * 10000 + ((T) / 256) * 100 + (CP):                                                     \
@@ -857,8 +857,9 @@ MI355_API int mi355_residual_rmsnorm_fwd_bf16_dev(uint16_t *y, uint16_t *yn, con
         if (!mi355_exchange(&g_bf_cluster_ws)) return -1;
 #define BF_CLUSTER_RES_FWD(RPT, WHOLE)                                                                               \
     hipLaunchKernelGGL((rms_fwd_cluster_kernel<StoreBf16, RPT, 1024, true, WHOLE>), dim3(cp.nblk), dim3(1024), 0,    \
-                       g_ctx.stream, yn, y, a, b, alpha, w, C, S, cp.strips, cp.nblk, cp.csplit, cp.rows_pm, eps,    \
-                       1.0f / (float)C, g_bf_cluster_ws, mi355_exchange_spin_ticks())
+                       g_ctx.stream, a, b, w, g_bf_cluster_ws.cnt, C, S, cp.word_a(), cp.word_b(), yn, y, alpha,     \
+                       eps, 1.0f / (float)C, g_bf_cluster_ws.slots, g_bf_cluster_ws.fallbacks,                       \
+                       mi355_exchange_spin_ticks())
         cluster_whole(cp, [&](auto whole) {
             constexpr int WHOLE = decltype(whole)::value;
             if (cp.rpt == 2) BF_CLUSTER_RES_FWD(2, WHOLE);
@@ -894,8 +895,9 @@ MI355_API int mi355_rmsnorm_bwd_residual_bf16_dev(uint16_t *dx, uint16_t *dx_sca
         if (!part) return -1;
 #define BF_CLUSTER_RES_BWD(RPT, WHOLE)                                                                               \
     hipLaunchKernelGGL((rms_bwd_cluster_kernel<StoreBf16, RPT, 1024, true, WHOLE>), dim3(cp.nblk), dim3(1024), 0,    \
-                       g_ctx.stream, dx, part, dy, x, w, C, S, cp.strips, cp.nblk, cp.csplit, cp.rows_pm, eps,       \
-                       1.0f / (float)C, variant, res, dx_scaled, alpha, g_bf_cluster_ws, mi355_exchange_spin_ticks())
+                       g_ctx.stream, x, dy, w, g_bf_cluster_ws.cnt, C, S, cp.word_a(), cp.word_b(), res, dx, part,   \
+                       dx_scaled, alpha, eps, 1.0f / (float)C, variant, g_bf_cluster_ws.slots,                       \
+                       g_bf_cluster_ws.fallbacks, mi355_exchange_spin_ticks())
         cluster_whole(cp, [&](auto whole) {
             constexpr int WHOLE = decltype(whole)::value;
             if (cp.rpt == 2) BF_CLUSTER_RES_BWD(2, WHOLE);

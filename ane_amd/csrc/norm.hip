@@ -495,9 +495,9 @@ ClusterPlan plan_cluster(int C, int S, int batch, bool vec_ok, int max_rpt, int 
 template <int RPT, bool FUSE, int WHOLE>
 void launch_fwd_cluster_as(const ClusterPlan &cp, float *yn, float *y_res, const float *a, const float *b, float alpha,
                            const float *w, int C, int S, float eps) {
-    hipLaunchKernelGGL((rms_fwd_cluster_kernel<StoreF32, RPT, 1024, FUSE, WHOLE>), dim3(cp.nblk), dim3(1024), 0, g_ctx.stream, yn,
-                       y_res, a, b, alpha, w, C, S, cp.strips, cp.nblk, cp.csplit, cp.rows_pm, eps, 1.0f / (float)C,
-                       g_cluster_ws, cluster_spin_ticks());
+    hipLaunchKernelGGL((rms_fwd_cluster_kernel<StoreF32, RPT, 1024, FUSE, WHOLE>), dim3(cp.nblk), dim3(1024), 0, g_ctx.stream, a, b,
+                       w, g_cluster_ws.cnt, C, S, cp.word_a(), cp.word_b(), yn, y_res, alpha, eps, 1.0f / (float)C,
+                       g_cluster_ws.slots, g_cluster_ws.fallbacks, cluster_spin_ticks());
 }
 
 template <bool FUSE>
@@ -514,9 +514,9 @@ void launch_fwd_cluster(const ClusterPlan &cp, float *yn, float *y_res, const fl
 template <bool RES, int WHOLE>
 void launch_bwd_cluster_as(const ClusterPlan &cp, float *dx, float *part, const float *dy, const float *x, const float *w,
                            int C, int S, float eps, int variant, const float *res, float *dx2, float alpha2) {
-    hipLaunchKernelGGL((rms_bwd_cluster_kernel<StoreF32, 4, 1024, RES, WHOLE>), dim3(cp.nblk), dim3(1024), 0, g_ctx.stream, dx, part,
-                       dy, x, w, C, S, cp.strips, cp.nblk, cp.csplit, cp.rows_pm, eps, 1.0f / (float)C, variant, res, dx2,
-                       alpha2, g_cluster_ws, cluster_spin_ticks());
+    hipLaunchKernelGGL((rms_bwd_cluster_kernel<StoreF32, 4, 1024, RES, WHOLE>), dim3(cp.nblk), dim3(1024), 0, g_ctx.stream, x, dy,
+                       w, g_cluster_ws.cnt, C, S, cp.word_a(), cp.word_b(), res, dx, part, dx2, alpha2, eps, 1.0f / (float)C,
+                       variant, g_cluster_ws.slots, g_cluster_ws.fallbacks, cluster_spin_ticks());
 }
 
 template <bool RES>

@@ -125,74 +125,110 @@ __device__ __forceinline__ void member_sums(float (&acc)[NV][VEC], float *lds, f
     __syncthreads();
 }
 
-// slots fetched per thread: the members' NV*W column sums, THREADS at a time
-template <int THREADS, int NV, int VEC>
-constexpr int cluster_fetches() { return (CL_MAX_SPLIT * NV * CL_LPR * VEC + THREADS - 1) / THREADS; }
+// The launch counters of the cluster's members, one to a lane, and this workgroup's own.  Asked for ahead of the rows and wanted
+// only with the column sums.  (A relaxed atomic load: the compiler leaves it where it stands, an ordinary one moves to where the
+// sums are published, a trip to memory that everybody waits for.  As a load behind a condition, with one added to it at once, it
+// kept every wave from asking for its rows until it was back.)
+struct ClusterTags {
+    unsigned lanes;
+    int mine;
+    __device__ __forceinline__ unsigned of(int m) const { return __builtin_amdgcn_readlane(lanes, m) + 1u; }
+    __device__ __forceinline__ unsigned own() const { return of(mine); }
+};
+__device__ __forceinline__ ClusterTags cluster_tags(unsigned *cnt, int first, int member, int csplit) {
+    const int m = min((int)(threadIdx.x & 63), csplit - 1);
+    return {__hip_atomic_load(cnt + first + m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP), member};
+}
 
-// Publishes wsum (this member's column sums) and gathers every member's into tot[(m*NV+q)*W + column].
-// Returns false when the bounded wait expired for any slot (block-uniform).
+// Per-thread partial sums acc[q][j] -> the cluster's sum of quantity q over column c, in thread i = q*W + c < NV*W (the others
+// return at once): the waves' sums are added up and published, every other member's are fetched by the same thread, all of them
+// in flight together, and added in member order.  false: the bounded wait expired for a member of this column.  lds: NW*NV*W
+// floats; a barrier stands between the writes to it and the sums.
+// One thread has a sum from here to the end: what is formed of it (a division, a square root) is formed once and handed to the
+// lanes behind the next barrier.  With the members' sums handed on and added up again by every lane, and the division and the root
+// taken by all sixteen waves, there was a barrier more.  With that, the launch counters (cluster_tags) and the order of the loads,
+// us by the trace, before and after: with the residual, bfloat16 [16][1024][256] forward 9.9 and 8.4, backward 12.9 and 10.4, fp32
+// [8][768][197] 7.8 and 7.2, 9.8 and 8.2; without, fp32 [16][1024][256] 8.1 and 7.2, 10.8 and 10.5, [1][768][256] 5.7 and 4.8, 6.7 and 5.5.
 template <int THREADS, int NV, int VEC>
-__device__ __forceinline__ bool cluster_exchange(const float *wsum, float *tot, int *failed, int blk, int cluster,
-                                                 int csplit, const ClusterWs &ws, unsigned my_tag,
-                                                 const unsigned (&want_tag)[cluster_fetches<THREADS, NV, VEC>()],
-                                                 int spin_ticks) {
-    constexpr int NF = cluster_fetches<THREADS, NV, VEC>();
-    constexpr int PER = NV * CL_LPR * VEC;            // slots per member
-    static_assert(PER <= CL_SLOT_STRIDE && PER <= THREADS, "a member's column sums must fit its slots");
-    if (threadIdx.x < PER) {
-        const unsigned long long pk = ((unsigned long long)my_tag << 32) | __float_as_uint(wsum[threadIdx.x]);
-        __hip_atomic_store(&ws.slots[(size_t)blk * CL_SLOT_STRIDE + threadIdx.x], pk, __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-    }
-    const int nslots = csplit * PER;
+__device__ __forceinline__ bool cluster_totals(float (&acc)[NV][VEC], float *lds, int blk, int first, int member, int csplit,
+                                               unsigned long long *slots, const ClusterTags &tags, int spin_ticks,
+                                               float &total) {
+    constexpr int NW = THREADS / 64, W = CL_LPR * VEC;
+    static_assert(NV * W <= CL_SLOT_STRIDE && NV * W <= THREADS, "a member's column sums must fit its slots");
 #pragma unroll
-    for (int f = 0; f < NF; f++) {
-        const int i = threadIdx.x + f * THREADS;
-        if (i < nslots) {
-            const int m = i / PER, c = i - m * PER;
-            const unsigned long long *sp = &ws.slots[(size_t)(cluster * csplit + m) * CL_SLOT_STRIDE + c];
-            const long long t0 = wall_clock64();
-            unsigned long long pk;
-            bool ok = false;
-            for (;;) {
-                pk = __hip_atomic_load(sp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (spin_ticks < 0) break;                        // test mode: whatever the slot holds is refused
-                if ((unsigned)(pk >> 32) == want_tag[f]) { ok = true; break; }
-                if (wall_clock64() - t0 >= (long long)spin_ticks) break;
-                __builtin_amdgcn_s_sleep(2);
-            }
-            if (!ok) *failed = 1;
-            tot[i] = __uint_as_float((unsigned)pk);
-        }
+    for (int q = 0; q < NV; q++)
+#pragma unroll
+        for (int j = 0; j < VEC; j++) acc[q][j] = wave_sum_stride<CL_LPR>(acc[q][j]);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const unsigned i = threadIdx.x;
+    if (lane < CL_LPR) {
+#pragma unroll
+        for (int q = 0; q < NV; q++)
+#pragma unroll
+            for (int j = 0; j < VEC; j++) lds[(wave * NV + q) * W + lane * VEC + j] = acc[q][j];
     }
     __syncthreads();
-    return *failed == 0;
-}
-
-// The launch tags: this workgroup's own, and for every slot it will fetch the one its owner will write.
-template <int THREADS, int NV, int VEC>
-__device__ __forceinline__ void cluster_tags(unsigned &my_tag, unsigned (&want_tag)[cluster_fetches<THREADS, NV, VEC>()],
-                                             int blk, int cluster, int csplit, const ClusterWs &ws) {
-    constexpr int PER = NV * CL_LPR * VEC;
+    if (i >= NV * W) return true;
+    float own = 0.f;
 #pragma unroll
-    for (int f = 0; f < cluster_fetches<THREADS, NV, VEC>(); f++) {
-        const int i = threadIdx.x + f * THREADS;
-        want_tag[f] = i < csplit * PER ? ws.cnt[cluster * csplit + i / PER] + 1u : 0u;
+    for (int wv = 0; wv < NW; wv++) own += lds[wv * NV * W + i];
+    auto slot = [&](int b) {
+        return (unsigned long long *)((char *)(slots + (size_t)b * CL_SLOT_STRIDE) + i * (unsigned)sizeof(unsigned long long));
+    };
+    __hip_atomic_store(slot(blk), (unsigned long long)tags.own() << 32 | __float_as_uint(own), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+    unsigned long long pk[CL_MAX_SPLIT];
+    bool ok = false;
+    for (long long t0 = 0;;) {
+#pragma unroll
+        for (int m = 0; m < CL_MAX_SPLIT; m++)
+            pk[m] = __hip_atomic_load(slot(first + min(m, csplit - 1)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (spin_ticks < 0) break;                        // test mode: whatever the slots hold is refused
+        ok = true;
+#pragma unroll
+        for (int m = 0; m < CL_MAX_SPLIT; m++)
+            ok = ok & ((min(m, csplit - 1) == member) | ((unsigned)(pk[m] >> 32) == tags.of(min(m, csplit - 1))));
+        if (ok) break;
+        const long long now = wall_clock64();
+        if (t0 == 0) t0 = now;
+        if (now - t0 >= (long long)spin_ticks) break;
+        __builtin_amdgcn_s_sleep(2);
     }
-    my_tag = threadIdx.x < PER ? ws.cnt[blk] + 1u : 0u;     // used by the publishing threads and by thread 0
+    total = 0.f;
+#pragma unroll
+    for (int m = 0; m < CL_MAX_SPLIT; m++)
+        if (m < csplit) total += m == member ? own : __uint_as_float((unsigned)pk[m]);
+    return ok;
 }
 
-// Geometry shared by the kernels: workgroup number -> (slab, strip, member), rows of a member.
+// Geometry shared by the kernels: workgroup number -> (slab, strip, member), rows of a member.  It comes in two words, which with the
+// operands of the tile are the arguments that the waves find in their registers when they start (14 dwords of them): what
+// has to be loaded is not waited for until the rows have been asked for.  The number of strips comes with its reciprocal.
 struct ClusterGeo {
-    int blk, cluster, member, slab, strip;
+    int blk, first, csplit, member, slab, strip, rows_pm;
 };
-__device__ __forceinline__ ClusterGeo cluster_geo(int nblk, int csplit, int strips) {
+constexpr int CL_NBLK_BITS = 12, CL_SPLIT_BITS = 2, CL_STRIP_BITS = 11, CL_RECIP = 20;
+static_assert(CL_MAX_BLOCKS < 1 << CL_NBLK_BITS && CL_MAX_SPLIT < 1 << (1 << CL_SPLIT_BITS), "the fields hold their values");
+// cluster / strips = cluster * recip >> CL_RECIP: both are below 2^10 (at least two members to a cluster), so that the excess of
+// the reciprocal, below strips / 2^CL_RECIP, times the cluster stays below 1
+static_assert(CL_MAX_BLOCKS / 2 <= 1 << (CL_RECIP / 2) && CL_MAX_BLOCKS / 2 < 1 << CL_STRIP_BITS, "the reciprocal is exact");
+static inline unsigned cluster_word_a(int nblk, int csplit, int rows_pm) {
+    return (unsigned)nblk | (unsigned)__builtin_ctz(csplit) << CL_NBLK_BITS | (unsigned)rows_pm << (CL_NBLK_BITS + CL_SPLIT_BITS);
+}
+static inline unsigned cluster_word_b(int strips) {
+    return (unsigned)strips | (unsigned)(((1 << CL_RECIP) + strips - 1) / strips) << CL_STRIP_BITS;
+}
+__device__ __forceinline__ ClusterGeo cluster_geo(unsigned wa, unsigned wb) {
     ClusterGeo g;
-    g.blk = xcd_remap(blockIdx.x, nblk);      // the members of a cluster are neighbours on one XCD
-    g.cluster = g.blk / csplit;
-    g.member = g.blk - g.cluster * csplit;
-    g.slab = g.cluster / strips;
-    g.strip = g.cluster - g.slab * strips;
+    const int shift = wa >> CL_NBLK_BITS & ((1 << CL_SPLIT_BITS) - 1);
+    g.csplit = 1 << shift;
+    g.rows_pm = wa >> (CL_NBLK_BITS + CL_SPLIT_BITS);
+    g.blk = xcd_remap(blockIdx.x, wa & ((1 << CL_NBLK_BITS) - 1));      // the members of a cluster are neighbours on one XCD
+    const unsigned cluster = g.blk >> shift;
+    g.first = cluster << shift;
+    g.member = g.blk - g.first;
+    g.slab = cluster * (wb >> CL_STRIP_BITS) >> CL_RECIP;
+    g.strip = cluster - g.slab * (wb & ((1 << CL_STRIP_BITS) - 1));
     return g;
 }
 
@@ -204,11 +240,12 @@ __device__ __forceinline__ ClusterGeo cluster_geo(int nblk, int csplit, int stri
 // only their values are dropped, which is still quicker than branches: bfloat16 [5][1024][570] forward 8.0 -> 7.6, with the
 // residual 10.7 -> 10.4, backward 12.2 -> 12.0, with it 14.0 -> 13.7; fp32 [115][768][54] with the residual 21.2 -> 20.1.
 template <typename ST, int RPT, int THREADS, bool FUSE, int WHOLE>
-__global__ __launch_bounds__(THREADS) void rms_fwd_cluster_kernel(typename ST::T *__restrict__ yn, typename ST::T *y_res,
-                                                                  const typename ST::T *a, const typename ST::T *b,
-                                                                  float alpha, const float *__restrict__ w, int C,
-                                                                  int S, int strips, int nblk, int csplit, int rows_pm,
-                                                                  float eps, float invC, ClusterWs ws,
+__global__ __launch_bounds__(THREADS) void rms_fwd_cluster_kernel(const typename ST::T *a, const typename ST::T *b,
+                                                                  const float *__restrict__ w, unsigned *cnt, int C, int S,
+                                                                  unsigned word_a, unsigned word_b,
+                                                                  typename ST::T *__restrict__ yn, typename ST::T *y_res,
+                                                                  float alpha, float eps, float invC,
+                                                                  unsigned long long *slots, int *fallbacks,
                                                                   int spin_ticks) {
     constexpr bool EXACT = WHOLE == CL_EXACT;
     // sixteen loads ahead of the first use are more than there is room for: [12][1024][500] with the residual 30.9 us, with the branch 28.4
@@ -218,53 +255,73 @@ __global__ __launch_bounds__(THREADS) void rms_fwd_cluster_kernel(typename ST::T
     constexpr int RPS = THREADS / CL_LPR;
     constexpr int NW = THREADS / 64;
     __shared__ float lds[NW * W];
-    __shared__ float wsum[W];
-    __shared__ float tot[CL_MAX_SPLIT * W];
+    __shared__ __align__(16) float col_rr[W];
     __shared__ int failed;
-    const ClusterGeo g = cluster_geo(nblk, csplit, strips);
+    const ClusterGeo g = cluster_geo(word_a, word_b);
+    const int csplit = g.csplit, rows_pm = g.rows_pm;
     const int lc = threadIdx.x % CL_LPR, row0 = threadIdx.x / CL_LPR;
     const LaneCols mine = lane_cols_inside<VEC, W>(g.strip * W + lc * VEC, S);
     const int col = mine.col;
     const bool col_ok = mine.ok;
     const size_t slab_base = (size_t)g.slab * C * S + col;
-    if (threadIdx.x == 0) failed = 0;
-    unsigned my_tag, want_tag[cluster_fetches<THREADS, 1, VEC>()];
-    cluster_tags<THREADS, 1, VEC>(my_tag, want_tag, g.blk, g.cluster, csplit, ws);
+    const ClusterTags tags = cluster_tags(cnt, g.first, g.member, csplit);
 
     // rows of member m held by this thread: c = m*rows_pm + row0 + k*RPS, valid while below (m+1)*rows_pm and C
     auto row_of = [&](int m, int k) { return m * rows_pm + row0 + k * RPS; };
     auto row_live = [&](int m, int k) { return row0 + k * RPS < rows_pm && row_of(m, k) < C; };
     auto row_ok = [&](int m, int k) { return row_live(m, k) && col_ok; };
     // one row piece of x (FUSE: of y = a + alpha*b, rounded to the storage type as the stored y is)
+    auto sum_row = [&](const typename ST::Raw &ra, const typename ST::Raw &rb) -> typename ST::Raw {
+        float av[VEC], bv[VEC], v[VEC];
+        ST::widen(av, ra);
+        ST::widen(bv, rb);
+#pragma unroll
+        for (int j = 0; j < VEC; j++) v[j] = bv[j] * alpha + av[j];
+        return ST::pack(v);
+    };
     auto load_row = [&](int c, bool first) -> typename ST::Raw {
         const size_t off = slab_base + (size_t)c * S;
-        if constexpr (FUSE) {
-            float av[VEC], bv[VEC], v[VEC];
-            ST::widen(av, first ? cluster_load<ST, WHOLE>(a + off) : ST::load(a + off));
-            ST::widen(bv, first ? cluster_load<ST, WHOLE>(b + off) : ST::load(b + off));
-#pragma unroll
-            for (int j = 0; j < VEC; j++) v[j] = bv[j] * alpha + av[j];
-            return ST::pack(v);
-        } else {
-            return first ? cluster_load<ST, WHOLE>(a + off) : ST::load(a + off);
-        }
+        const typename ST::Raw ra = first ? cluster_load<ST, WHOLE>(a + off) : ST::load(a + off);
+        if constexpr (FUSE) return sum_row(ra, first ? cluster_load<ST, WHOLE>(b + off) : ST::load(b + off));
+        else return ra;
     };
 
-    typename ST::Raw xr[RPT];
+    typename ST::Raw xr[RPT], br[FUSE && INSIDE ? RPT : 1];
     float wv[RPT];
+    if constexpr (INSIDE) {
+        // every load first, then what depends on one: a use between them would wait for it with the others not yet asked for
+        auto row = [&](int k) { return EXACT || row_live(g.member, k) ? row_of(g.member, k) : 0; };
+        auto none = [&](int k) { return WHOLE >= CL_FEW && k * RPS >= rows_pm; };
 #pragma unroll
-    for (int k = 0; k < RPT; k++) {
-        if (INSIDE ? WHOLE >= CL_FEW && k * RPS >= rows_pm : !row_ok(g.member, k)) {
+        for (int k = 0; k < RPT; k++) {
             xr[k] = ST::zero();
-            wv[k] = 0.f;
-            continue;
+            if constexpr (FUSE) br[k] = ST::zero();
+            if (none(k)) continue;
+            const size_t off = slab_base + (size_t)row(k) * S;
+            xr[k] = cluster_load<ST, WHOLE>(a + off);
+            if constexpr (FUSE) br[k] = cluster_load<ST, WHOLE>(b + off);
         }
-        const bool live = EXACT || row_live(g.member, k);
-        const int c = live ? row_of(g.member, k) : 0;
-        xr[k] = load_row(c, true);
-        wv[k] = w[c];
-        if (!live) xr[k] = ST::zero();
+#pragma unroll
+        for (int k = 0; k < RPT; k++) wv[k] = w[row(k)];
+#pragma unroll
+        for (int k = 0; k < RPT; k++) {
+            if constexpr (FUSE) xr[k] = sum_row(xr[k], br[k]);
+            if (!EXACT && !row_live(g.member, k)) xr[k] = ST::zero();
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < RPT; k++) {
+            if (!row_ok(g.member, k)) {
+                xr[k] = ST::zero();
+                wv[k] = 0.f;
+                continue;
+            }
+            const int c = row_of(g.member, k);
+            xr[k] = load_row(c, true);
+            wv[k] = w[c];
+        }
     }
+    if (threadIdx.x == 0) failed = 0;
     float acc[1][VEC];
 #pragma unroll
     for (int j = 0; j < VEC; j++) acc[0][j] = 0.f;
@@ -277,16 +334,23 @@ __global__ __launch_bounds__(THREADS) void rms_fwd_cluster_kernel(typename ST::T
     }
 #pragma unroll
     for (int k = 0; k < RPT; k++) ST::forget(xr[k]);
-    member_sums<THREADS, 1, VEC>(acc, lds, wsum);
-    float ss[VEC];
+    float total = 0.f, rr[VEC];
+    const bool met = cluster_totals<THREADS, 1, VEC>(acc, lds, g.blk, g.first, g.member, csplit, slots, tags, spin_ticks, total);
+    auto scale = [&](float ss) { return 1.0f / sqrtf(ss * invC + eps); };
+    if (threadIdx.x < W) {
+        col_rr[threadIdx.x] = scale(total);
+        if (!met) failed = 1;
+    }
+    __syncthreads();
+    if (!failed) {
 #pragma unroll
-    for (int j = 0; j < VEC; j++) ss[j] = 0.f;
-    if (cluster_exchange<THREADS, 1, VEC>(wsum, tot, &failed, g.blk, g.cluster, csplit, ws, my_tag, want_tag, spin_ticks)) {
-        for (int m = 0; m < csplit; m++)
-#pragma unroll
-            for (int j = 0; j < VEC; j++) ss[j] += tot[m * W + lc * VEC + j];
+        for (int j = 0; j < VEC; j++) rr[j] = col_rr[lc * VEC + j];
     } else {
-        if (threadIdx.x == 0) atomicAdd(ws.fallbacks, 1);
+        __shared__ float wsum[W];
+        float ss[VEC];
+#pragma unroll
+        for (int j = 0; j < VEC; j++) ss[j] = 0.f;
+        if (threadIdx.x == 0) atomicAdd(fallbacks, 1);
         for (int m = 0; m < csplit; m++) {
             float a2[1][VEC];
 #pragma unroll
@@ -305,10 +369,9 @@ __global__ __launch_bounds__(THREADS) void rms_fwd_cluster_kernel(typename ST::T
             for (int j = 0; j < VEC; j++) ss[j] += wsum[lc * VEC + j];
             __syncthreads();
         }
-    }
-    float rr[VEC];
 #pragma unroll
-    for (int j = 0; j < VEC; j++) rr[j] = 1.0f / sqrtf(ss[j] * invC + eps);
+        for (int j = 0; j < VEC; j++) rr[j] = scale(ss[j]);
+    }
 #pragma unroll
     for (int k = 0; k < RPT; k++) {
         if (EXACT || row_ok(g.member, k)) {
@@ -321,20 +384,20 @@ __global__ __launch_bounds__(THREADS) void rms_fwd_cluster_kernel(typename ST::T
             ST::store_nt(yn + off, ST::pack(o));
         }
     }
-    if (threadIdx.x == 0) ws.cnt[g.blk] = my_tag;
+    if (threadIdx.x == 0) cnt[g.blk] = tags.own();
 }
 
 // RES: dx = rmsnorm_bwd(dy, x, w) + res and optionally dx2 = alpha2*dx (training/training_dynamic/train.m:586-595,
 // :714-721), as rms_bwd_res_kernel of norm.hip.  dw partials: part[cluster][c], one row per cluster.
 template <typename ST, int RPT, int THREADS, bool RES, int WHOLE>
-__global__ __launch_bounds__(THREADS) void rms_bwd_cluster_kernel(typename ST::T *dx, float *__restrict__ dw_part,
-                                                                  const typename ST::T *dy,
-                                                                  const typename ST::T *__restrict__ x,
-                                                                  const float *__restrict__ w, int C, int S,
-                                                                  int strips, int nblk, int csplit, int rows_pm,
-                                                                  float eps, float invC, int variant,
-                                                                  const typename ST::T *res, typename ST::T *dx2,
-                                                                  float alpha2, ClusterWs ws, int spin_ticks) {
+__global__ __launch_bounds__(THREADS) void rms_bwd_cluster_kernel(const typename ST::T *__restrict__ x,
+                                                                  const typename ST::T *dy, const float *__restrict__ w,
+                                                                  unsigned *cnt, int C, int S, unsigned word_a,
+                                                                  unsigned word_b, const typename ST::T *res,
+                                                                  typename ST::T *dx, float *__restrict__ dw_part,
+                                                                  typename ST::T *dx2, float alpha2, float eps, float invC,
+                                                                  int variant, unsigned long long *slots, int *fallbacks,
+                                                                  int spin_ticks) {
     // without the residual, rows of whole lines keep the branch: [4][768][256] 8.1 us with it, 8.6 without ([8][768][256] with the
     // residual 10.0 and 9.1)
     constexpr bool EXACT = WHOLE == CL_EXACT;
@@ -344,18 +407,16 @@ __global__ __launch_bounds__(THREADS) void rms_bwd_cluster_kernel(typename ST::T
     constexpr int RPS = THREADS / CL_LPR;
     constexpr int NW = THREADS / 64;
     __shared__ float lds[NW * 2 * W];
-    __shared__ float wsum[2 * W];
-    __shared__ float tot[CL_MAX_SPLIT * 2 * W];
+    __shared__ __align__(16) float cols[2 * W];      // 1 / rms, then sum (dy*x)*w
     __shared__ int failed;
-    const ClusterGeo g = cluster_geo(nblk, csplit, strips);
+    const ClusterGeo g = cluster_geo(word_a, word_b);
+    const int csplit = g.csplit, rows_pm = g.rows_pm;
     const int lc = threadIdx.x % CL_LPR, row0 = threadIdx.x / CL_LPR;
     const LaneCols mine = lane_cols_inside<VEC, W>(g.strip * W + lc * VEC, S);
     const int col = mine.col;
     const bool col_ok = mine.ok;
     const size_t slab_base = (size_t)g.slab * C * S + col;
-    if (threadIdx.x == 0) failed = 0;
-    unsigned my_tag, want_tag[cluster_fetches<THREADS, 2, VEC>()];
-    cluster_tags<THREADS, 2, VEC>(my_tag, want_tag, g.blk, g.cluster, csplit, ws);
+    const ClusterTags tags = cluster_tags(cnt, g.first, g.member, csplit);
 
     auto row_of = [&](int m, int k) { return m * rows_pm + row0 + k * RPS; };
     auto row_live = [&](int m, int k) { return row0 + k * RPS < rows_pm && row_of(m, k) < C; };
@@ -363,26 +424,47 @@ __global__ __launch_bounds__(THREADS) void rms_bwd_cluster_kernel(typename ST::T
 
     typename ST::Raw xr[RPT], dr[RPT], rr_res[RES ? RPT : 1];
     float wv[RPT];
+    if constexpr (INSIDE) {
+        // every load first, then what depends on one (as above); the residual, needed last, last
+        auto row = [&](int k) { return EXACT || row_live(g.member, k) ? row_of(g.member, k) : 0; };
+        auto none = [&](int k) { return WHOLE >= CL_FEW && k * RPS >= rows_pm; };
 #pragma unroll
-    for (int k = 0; k < RPT; k++) {
-        if (INSIDE ? WHOLE >= CL_FEW && k * RPS >= rows_pm : !row_live(g.member, k)) {
+        for (int k = 0; k < RPT; k++) {
             xr[k] = dr[k] = ST::zero();
-            if constexpr (RES) rr_res[k] = ST::zero();
-            wv[k] = 0.f;
-            continue;
+            if (none(k)) continue;
+            const size_t off = slab_base + (size_t)row(k) * S;
+            xr[k] = cluster_load<ST, WHOLE>(x + off);
+            dr[k] = cluster_load<ST, WHOLE>(dy + off);
         }
-        const bool live = EXACT || row_live(g.member, k);
-        const int c = live ? row_of(g.member, k) : 0;
-        const size_t off = slab_base + (size_t)c * S;
-        xr[k] = cluster_load<ST, WHOLE>(x + off);
-        dr[k] = cluster_load<ST, WHOLE>(dy + off);
-        if constexpr (RES) rr_res[k] = cluster_load<ST, WHOLE>(res + off);
-        wv[k] = w[c];
-        if (!live) {                  // (all three: an infinity in the row read instead would make 0 * inf of the sum)
+#pragma unroll
+        for (int k = 0; k < RPT; k++) wv[k] = w[row(k)];
+        if constexpr (RES) {
+#pragma unroll
+            for (int k = 0; k < RPT; k++) {
+                rr_res[k] = ST::zero();
+                if (!none(k)) rr_res[k] = cluster_load<ST, WHOLE>(res + slab_base + (size_t)row(k) * S);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < RPT; k++)
+            if (!EXACT && !row_live(g.member, k)) {  // (all three: an infinity in the row read instead would make 0 * inf of the sum)
+                xr[k] = dr[k] = ST::zero();
+                wv[k] = 0.f;
+            }
+    } else {
+#pragma unroll
+        for (int k = 0; k < RPT; k++) {
             xr[k] = dr[k] = ST::zero();
             wv[k] = 0.f;
+            if (!row_live(g.member, k)) continue;
+            const int c = row_of(g.member, k);
+            const size_t off = slab_base + (size_t)c * S;
+            xr[k] = cluster_load<ST, WHOLE>(x + off);
+            dr[k] = cluster_load<ST, WHOLE>(dy + off);
+            wv[k] = w[c];
         }
     }
+    if (threadIdx.x == 0) failed = 0;
     float acc[2][VEC];      // [0] = sum x^2, [1] = sum (dy*x)*w
 #pragma unroll
     for (int j = 0; j < VEC; j++) acc[0][j] = acc[1][j] = 0.f;
@@ -399,19 +481,27 @@ __global__ __launch_bounds__(THREADS) void rms_bwd_cluster_kernel(typename ST::T
     }
 #pragma unroll
     for (int k = 0; k < RPT; k++) { ST::forget(xr[k]); ST::forget(dr[k]); }
-    member_sums<THREADS, 2, VEC>(acc, lds, wsum);
-    float ss[VEC], sd[VEC];
+    float total = 0.f, rr[VEC], dotn[VEC];
+    const bool met = cluster_totals<THREADS, 2, VEC>(acc, lds, g.blk, g.first, g.member, csplit, slots, tags, spin_ticks, total);
+    auto scale = [&](float ss) { return 1.0f / sqrtf(ss * invC + eps); };
+    auto dot = [&](float sd, float r) { return sd * ((r * r) * invC); };
+    if (threadIdx.x < 2 * W) {
+        cols[threadIdx.x] = threadIdx.x < W ? scale(total) : total;
+        if (!met) failed = 1;
+    }
+    __syncthreads();
+    if (!failed) {
 #pragma unroll
-    for (int j = 0; j < VEC; j++) ss[j] = sd[j] = 0.f;
-    if (cluster_exchange<THREADS, 2, VEC>(wsum, tot, &failed, g.blk, g.cluster, csplit, ws, my_tag, want_tag, spin_ticks)) {
-        for (int m = 0; m < csplit; m++)
-#pragma unroll
-            for (int j = 0; j < VEC; j++) {
-                ss[j] += tot[(m * 2 + 0) * W + lc * VEC + j];
-                sd[j] += tot[(m * 2 + 1) * W + lc * VEC + j];
-            }
+        for (int j = 0; j < VEC; j++) {
+            rr[j] = cols[lc * VEC + j];
+            dotn[j] = dot(cols[W + lc * VEC + j], rr[j]);
+        }
     } else {
-        if (threadIdx.x == 0) atomicAdd(ws.fallbacks, 1);
+        __shared__ float wsum[2 * W];
+        float ss[VEC], sd[VEC];
+#pragma unroll
+        for (int j = 0; j < VEC; j++) ss[j] = sd[j] = 0.f;
+        if (threadIdx.x == 0) atomicAdd(fallbacks, 1);
         for (int m = 0; m < csplit; m++) {
             float a2[2][VEC];
 #pragma unroll
@@ -436,14 +526,10 @@ __global__ __launch_bounds__(THREADS) void rms_bwd_cluster_kernel(typename ST::T
             for (int j = 0; j < VEC; j++) { ss[j] += wsum[lc * VEC + j]; sd[j] += wsum[W + lc * VEC + j]; }
             __syncthreads();
         }
-    }
-    float rr[VEC], dotn[VEC];
 #pragma unroll
-    for (int j = 0; j < VEC; j++) {
-        rr[j] = 1.0f / sqrtf(ss[j] * invC + eps);
-        dotn[j] = sd[j] * ((rr[j] * rr[j]) * invC);
+        for (int j = 0; j < VEC; j++) { rr[j] = scale(ss[j]); dotn[j] = dot(sd[j], rr[j]); }
     }
-    float *part = dw_part + (size_t)g.cluster * C;
+    float *part = dw_part + (size_t)(g.first / csplit) * C;
 #pragma unroll
     for (int k = 0; k < RPT; k++) {
         const int c = row_of(g.member, k);
@@ -486,13 +572,15 @@ __global__ __launch_bounds__(THREADS) void rms_bwd_cluster_kernel(typename ST::T
             if (lc == 0) part[c] = p;
         }
     }
-    if (threadIdx.x == 0) ws.cnt[g.blk] = my_tag;
+    if (threadIdx.x == 0) cnt[g.blk] = tags.own();
 }
 
 // How a shape is split: csplit members of rows_pm rows each; rpt rows per lane.  csplit = 0: not clustered.
 struct ClusterPlan {
     int csplit, rows_pm, rpt, threads, strips, nblk;
     int whole;         // which kernel: CL_EXACT, or CL_LINES or CL_ANY, with or without CL_FEW
+    unsigned word_a() const { return cluster_word_a(nblk, csplit, rows_pm); }
+    unsigned word_b() const { return cluster_word_b(strips); }
 };
 constexpr ClusterPlan NO_CLUSTER = {0, 0, 0, 0, 0, 0, CL_ANY};
 
