@@ -186,17 +186,18 @@ __device__ __forceinline__ float wave_sum_far_first(float v) {
     return v;
 }
 
-// exp(d) for d <= 0 through the hardware exp2: the product d*log2(e) is carried in two floats
-// so the result keeps ~1 ulp for |d| up to ~100 (a single-float product loses |d|*2^-24).  A NaN stays one: the clamp is
-// IEEE 754-2019's maximum (v_maximum3_f32), where fmaxf would take the bound in its place.
+// exp(d) for d <= 0 through the hardware exp2: 2^h with h = d*log2(e) rounded to a float, and what h leaves of d, formed exactly
+// but for the last bits (h*ln2 in two parts), as a factor 1 + r; so the result keeps ~1 ulp for |d| up to ~100 (a single-float
+// product loses |d|*2^-24).  A NaN stays one: the clamp is IEEE 754-2019's maximum (v_maximum3_f32), where fmaxf would
+// take the bound in its place.
 __device__ __forceinline__ float exp_neg(float d) {
-    const float L2E_HI = 1.44269502162933349609375f;      // float(log2 e)
-    const float L2E_LO = 1.925963033500011e-08f;          // log2 e - L2E_HI
+    const float LN2_HI = 0.693147182464599609375f;        // float(ln 2)
+    const float LN2_LO = -1.904654290582768e-09f;         // ln 2 - LN2_HI
     d = __builtin_elementwise_maximum(d, -200.0f);        // exp2 of the product is already 0 there; keeps -inf finite
-    float hi = d * L2E_HI;
-    float lo = __builtin_fmaf(d, L2E_HI, -hi) + d * L2E_LO;
-    float e = __builtin_amdgcn_exp2f(hi);
-    return __builtin_fmaf(e, lo * 0.693147180559945f, e);
+    const float h = d * 1.44269502162933349609375f;
+    const float r = __builtin_fmaf(h, -LN2_LO, __builtin_fmaf(h, -LN2_HI, d));
+    const float e = __builtin_amdgcn_exp2f(h);
+    return __builtin_fmaf(e, r, e);
 }
 
 // exp(d) for d <= 0 with a single-float product: relative error up to |d| * 6e-8; 0 for -inf, NaN for NaN.  Used where the

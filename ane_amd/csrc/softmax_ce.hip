@@ -433,17 +433,31 @@ __device__ __forceinline__ LaneCols cr_cols(int strip, int sw, int lc, int S) {
 }
 // The rows of member p: R of them from v_lo, in K steps of CR_RPS rows.  A lane has its row of every step but the last,
 // and of that one if row0 is below `last`.
+// Addresses: row(k, from) of a step k >= 0 is inside the tensor for every lane and every member, also one without rows: a lane without a row
+// in the last step reads the member's last row, and a step behind the last one is the last again.  So no load of a tile stands
+// behind a condition.  (Behind conditions the compiler waits for each load before the next wherever it moves a value between
+// registers at their end: five of the eight loads of bfloat16 [32000][200] went one after the other, and a member's
+// partial was there 5.6 us after its start for now 4.6, of fp32 [24573][256] 6.8 for 5.3.)
 struct CrRows {
     int v_lo, K, last;
+    unsigned step, off, off_last;      // bytes: a step, this lane's row and columns of a step and of the last one
 };
 template <typename T>
-__device__ __forceinline__ CrRows cr_rows(const CrGeo<T> &g, int p) {
+__device__ __forceinline__ CrRows cr_rows(const CrGeo<T> &g, int p, int col, int row0) {
     CrRows r;
-    r.v_lo = p * g.Rm;
-    const int R = max(0, min(g.V, r.v_lo + g.Rm) - r.v_lo);
+    const int R = max(0, min(g.V - p * g.Rm, g.Rm));
+    r.v_lo = min(p * g.Rm, g.V - 1);
     r.K = (R + CR_RPS - 1) / CR_RPS;
-    r.last = R - (r.K - 1) * CR_RPS;
+    r.last = R > 0 ? R - (r.K - 1) * CR_RPS : 1;
+    r.step = (unsigned)(CR_RPS * g.S) * (unsigned)sizeof(T);
+    r.off = (unsigned)(row0 * g.S + col) * (unsigned)sizeof(T);
+    r.off_last = (unsigned)(min(row0, r.last - 1) * g.S + col) * (unsigned)sizeof(T);
     return r;
+}
+template <typename T>
+__device__ __forceinline__ T *cr_at(T *first, const CrRows &r, int k) {      // first: row v_lo
+    const int kk = max(min(k, r.K - 1), 0);
+    return (T *)((char *)first + (size_t)((unsigned)kk * r.step) + (kk >= r.K - 1 ? r.off_last : r.off));
 }
 
 // (m, l) <- (m, l) merged with N more values: the online-softmax step
@@ -481,40 +495,42 @@ __device__ __forceinline__ void cr_merge16(const float (*wm)[CR_P], const float 
 // The (max, sum exp) partial of member p of a strip over its rows, for the 64 slots of the strip: valid in the quad of
 // threads 4c .. 4c+3 of slot c on return.  Of a member's K row steps the last K_REG are the register rows, the K_LDS
 // before them the LDS rows, and the first kL = K - K_REG - K_LDS the rows that are read twice.  A lane folds its rows
-// into its running (max, sum) four at a time, in row order: the rows before the register rows, then the register rows.
-// KEEP: this workgroup's own rows; the loads run ahead of the arithmetic.  Every condition on a step is the same for the
+// into its running (max, sum) four (eight, cr_reg_sub) at a time, in row order: the rows before the register rows, then the register rows.
+// KEEP: this workgroup's own rows; the loads run ahead of the arithmetic (asked(): called when the first ones are on their way).  Every condition on a step is the same for the
 // whole workgroup (scalar branches); a lane without a row in the last step reads the member's last row and its value
-// is replaced when it is folded.
+// is replaced when it is folded, as is that of a step that the member does not have.
 // Otherwise nothing is kept: one column and one group of four rows at a time, the same operations on the same values
 // in the same order (same bits) in a handful of registers, because the caller's own rows stay live in theirs.
-template <typename ST, int K_REG, int K_LDS, bool KEEP, bool NT>
+// Register rows of the variants that have no others fold eight at a time: a group costs a maximum, an exponential and a product
+// beside its values.
+constexpr int cr_reg_sub(int k_reg, int k_lds) { return k_lds == 0 && k_reg % 8 == 0 ? 8 : CR_SUB; }
+template <typename ST, int K_REG, int K_LDS, bool KEEP, bool NT, typename Asked>
 __device__ __forceinline__ void cr_member_partial(const CrGeo<typename ST::T> &g, int strip, int p, typename ST::Raw (&xr)[K_REG],
                                                   typename ST::Raw (*lrow)[CR_THREADS],
-                                                  float (*wm)[CR_P], float (*wl)[CR_P], float &Mout, float &Lout) {
+                                                  float (*wm)[CR_P], float (*wl)[CR_P], float &Mout, float &Lout,
+                                                  Asked asked) {
     typedef typename ST::Raw Raw;
-    static_assert(K_REG % CR_SUB == 0, "the register rows fold four at a time");
+    constexpr int RSUB = cr_reg_sub(K_REG, K_LDS);
+    static_assert(K_REG % RSUB == 0, "the register rows fold in whole groups");
     const int lc = threadIdx.x & 15, row0 = threadIdx.x >> 4, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const LaneCols mine = cr_cols(strip, g.sw, lc, g.S);
-    const CrRows r = cr_rows(g, p);
+    const CrRows r = cr_rows(g, p, mine.col, row0);
     const int K = r.K, kR = max(0, K - K_REG), kL = max(0, kR - K_LDS);
     const int mineK = row0 < r.last ? K : K - 1;                  // steps in which this lane has a row
-    // a row piece = (uniform address of row v_lo + 64k) + (this lane's fixed 32-bit offset)
-    const typename ST::T *base = g.logits + (size_t)r.v_lo * g.S;
-    const unsigned loff = (unsigned)row0 * (unsigned)g.S + (unsigned)mine.col;
-    const unsigned loff_last = (unsigned)min(row0, max(r.last - 1, 0)) * (unsigned)g.S + (unsigned)mine.col;
-    const size_t step = (size_t)CR_RPS * g.S;
+    const typename ST::T *first = g.logits + (size_t)r.v_lo * g.S;
     const Raw ninf = ST::ninf();
     float m[4], l[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) { m[j] = NO_MAX; l[j] = 0.f; }
     if constexpr (KEEP) {
-        auto foldg = [&](const Raw (&t)[CR_SUB]) {
+        auto foldg = [&](auto &t) {
+            constexpr int N = sizeof(t) / sizeof(t[0]);
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                float x4[CR_SUB];
+                float xs[N];
 #pragma unroll
-                for (int u = 0; u < CR_SUB; u++) x4[u] = ST::at(t[u], j);
-                online_update<CR_SUB>(m[j], l[j], x4);
+                for (int u = 0; u < N; u++) xs[u] = ST::at(t[u], j);
+                online_update<N>(m[j], l[j], xs);
                 // a column at a time: the four in step take 13 registers more than there are ([151936][256] 73 us)
                 asm volatile("" : "+v"(m[j]), "+v"(l[j]));
             }
@@ -523,23 +539,18 @@ __device__ __forceinline__ void cr_member_partial(const CrGeo<typename ST::T> &g
         // through two groups of four.  (Rows that stay on the chip may be read past the cache.)
 #pragma unroll
         for (int i = 0; i < K_REG; i++) {
-            const int k = kR + i;
-            if (k < K) {
-                const typename ST::T *a = base + k * step + (k == K - 1 ? loff_last : loff);
-                xr[i] = NT ? ST::ld_nt(a) : ST::ld(a);
-            }
+            const typename ST::T *at = cr_at(first, r, kR + i);
+            xr[i] = NT ? ST::ld_nt(at) : ST::ld(at);
         }
+        if (K_LDS == 0 || kR == 0) asked();
         if (K_LDS > 0 && kR > 0) {
+            // (a row step behind the last of these, kR - 1, is that one again, and dropped when it is folded)
             auto loadg = [&](Raw (&t)[CR_SUB], int k0) {
 #pragma unroll
                 for (int u = 0; u < CR_SUB; u++) {
-                    const int k = k0 + u;
-                    if (k < kR) {
-                        const typename ST::T *a = base + k * step + loff;
-                        t[u] = (NT && k >= kL) ? ST::ld_nt(a) : ST::ld(a);
-                    } else {
-                        t[u] = ninf;
-                    }
+                    const int k = min(k0 + u, kR - 1);
+                    const typename ST::T *at = (const typename ST::T *)((const char *)first + (size_t)((unsigned)k * r.step) + r.off);
+                    t[u] = NT && K_LDS > 0 && k0 >= kL ? ST::ld_nt(at) : ST::ld(at);
                 }
             };
             auto keepg = [&](const Raw (&t)[CR_SUB], int k0) {
@@ -547,30 +558,40 @@ __device__ __forceinline__ void cr_member_partial(const CrGeo<typename ST::T> &g
                 for (int u = 0; u < CR_SUB; u++)
                     if (k0 + u >= kL && k0 + u < kR) lrow[k0 + u - kL][threadIdx.x] = t[u];
             };
+            auto tail = [&](Raw (&t)[CR_SUB], int k0) {
+                if (k0 + CR_SUB > kR) {
+#pragma unroll
+                    for (int u = 0; u < CR_SUB; u++)
+                        if (k0 + u >= kR) t[u] = ninf;
+                }
+            };
             Raw ta[CR_SUB], tb[CR_SUB];
             loadg(ta, 0);
             loadg(tb, CR_SUB);
+            asked();
             for (int k0 = 0; k0 < kR; k0 += 2 * CR_SUB) {
                 keepg(ta, k0);
+                tail(ta, k0);
                 foldg(ta);
                 loadg(ta, k0 + 2 * CR_SUB);
                 if (k0 + CR_SUB < kR) {
                     keepg(tb, k0 + CR_SUB);
+                    tail(tb, k0 + CR_SUB);
                     foldg(tb);
                 }
                 loadg(tb, k0 + 3 * CR_SUB);
             }
         }
 #pragma unroll
-        for (int c = 0; c < K_REG / CR_SUB; c++) {
-            const int k0 = kR + c * CR_SUB;
+        for (int c = 0; c < K_REG / RSUB; c++) {
+            const int k0 = kR + c * RSUB;
             if (k0 < K) {                                         // groups past the last step hold nothing
-                Raw t[CR_SUB];
+                Raw t[RSUB];
 #pragma unroll
-                for (int u = 0; u < CR_SUB; u++) t[u] = xr[c * CR_SUB + u];
-                if (k0 + CR_SUB >= K) {
+                for (int u = 0; u < RSUB; u++) t[u] = xr[c * RSUB + u];
+                if (k0 + RSUB >= K) {
 #pragma unroll
-                    for (int u = 0; u < CR_SUB; u++)
+                    for (int u = 0; u < RSUB; u++)
                         if (k0 + u >= mineK) t[u] = ninf;
                 }
                 foldg(t);
@@ -579,23 +600,25 @@ __device__ __forceinline__ void cr_member_partial(const CrGeo<typename ST::T> &g
 #pragma unroll
         for (int i = 0; i < K_REG; i++) ST::forget(xr[i]);
     } else {
+        const unsigned step = CR_RPS * g.S, loff = row0 * g.S + mine.col;
 #pragma unroll 1
         for (int j = 0; j < 4; j++) {
             float mj = NO_MAX, lj = 0.f;
-            auto part = [&](int kbeg, int kend) {
+            auto part = [&](auto sub, int kbeg, int kend) {
+                constexpr int N = decltype(sub)::value;
 #pragma unroll 1
-                for (int k0 = kbeg; k0 < kend; k0 += CR_SUB) {
-                    float x4[CR_SUB];
+                for (int k0 = kbeg; k0 < kend; k0 += N) {
+                    float xs[N];
 #pragma unroll
-                    for (int u = 0; u < CR_SUB; u++) {
+                    for (int u = 0; u < N; u++) {
                         const int k = k0 + u;
-                        x4[u] = k < min(kend, mineK) ? ld_one(base + k * step + loff + j) : -INFINITY;
+                        xs[u] = k < min(kend, mineK) ? ld_one(first + (size_t)k * step + loff + j) : -INFINITY;
                     }
-                    online_update<CR_SUB>(mj, lj, x4);
+                    online_update<N>(mj, lj, xs);
                 }
             };
-            part(0, kR);
-            part(kR, K);
+            part(std::integral_constant<int, CR_SUB>(), 0, kR);
+            part(std::integral_constant<int, RSUB>(), kR, K);
 #pragma unroll
             for (int q = 0; q < 4; q++)
                 if (q == j) { m[q] = mj; l[q] = lj; }
@@ -644,14 +667,16 @@ __device__ __forceinline__ void cr_merge_members(const float (&pm)[MPG], const f
     __syncthreads();
 }
 
-// The target of the column of slot threadIdx.x < 64 of a strip; -1 where the slot has no column of its own or the target
-// is out of range.
+// The target of the column of slot threadIdx.x % 64 of a strip, as it stands (asked for early), and what counts of it: -1 where
+// the slot has no column of its own or the target is out of range.
 template <typename T>
 __device__ __forceinline__ int cr_slot_target(const CrGeo<T> &g, int strip, const int32_t *targets) {
-    const LaneCols mine = cr_cols(strip, g.sw, threadIdx.x >> 2, g.S);
-    if (!mine.ok || (int)(threadIdx.x & 3) < mine.dup) return -1;
-    const int tg = targets[mine.col + (threadIdx.x & 3)];
-    return tg < g.V ? tg : -1;
+    return targets[cr_cols(strip, g.sw, (threadIdx.x & 63) >> 2, g.S).col + (threadIdx.x & 3)];
+}
+template <typename T>
+__device__ __forceinline__ int cr_own_target(const CrGeo<T> &g, int strip, int tg) {
+    const LaneCols mine = cr_cols(strip, g.sw, (threadIdx.x & 63) >> 2, g.S);
+    return mine.ok && (int)(threadIdx.x & 3) >= mine.dup && tg < g.V ? tg : -1;
 }
 template <typename T>
 __device__ __forceinline__ float cr_slot_logit(const CrGeo<T> &g, int strip, int tg) {
@@ -663,6 +688,20 @@ __device__ __forceinline__ float cr_strip_loss(int tg, float logit, float M, flo
     const float p = exp_neg(logit - M) * inv;
     return wave_sum_far_first(tg >= 0 ? -logf(p + 1e-10f) : 0.f);
 }
+
+// Strips, members and the reciprocal of the strips in one word: with the tensors, the counters and the sizes they are the arguments
+// that a wave finds in its registers (14 dwords), so that it waits for no argument before it asks for its rows.
+// n * recip >> 16 is n / strips for the workgroup numbers: the excess of the reciprocal, below strips / 2^16, times n < 2^9 stays below 1.
+struct CrWord {
+    int strips, csplit;
+    unsigned recip;
+    __device__ __forceinline__ int over_strips(int n) const { return (int)((unsigned)n * recip >> 16); }
+};
+static_assert(CR_MAX_STRIPS < 32 && CR_MAX_SPLIT < 256 && CR_MAX_WG * CR_MAX_STRIPS <= 1 << 16, "the fields and the reciprocal hold");
+static inline unsigned cr_word(int strips, int csplit) {
+    return (unsigned)strips | (unsigned)csplit << 5 | (unsigned)(((1 << 16) + strips - 1) / strips) << 13;
+}
+__device__ __forceinline__ CrWord cr_unpack(unsigned w) { return {(int)(w & 31), (int)(w >> 5 & 255), w >> 13}; }
 
 // One bounded wait for a tagged slot.  false: the tag did not arrive within spin_ticks.
 __device__ __forceinline__ bool cr_wait_slot(const unsigned long long *sp, unsigned want, int spin_ticks, float &value) {
@@ -687,109 +726,114 @@ __device__ __forceinline__ bool cr_wait_slot(const unsigned long long *sp, unsig
 // the lines at their border the caches have to put the pieces together ([151936][200] fp32 102 us past them, 77 with
 // them; [151936][256] 68 and 94).
 template <typename ST, int K_REG, int K_LDS, bool NT, int MEMBERS = CR_MAX_SPLIT / 2>
-__global__ __launch_bounds__(CR_THREADS) void ce_resident_kernel(typename ST::T *__restrict__ dlogits,
-                                                                 const typename ST::T *__restrict__ logits,
-                                                                 const int32_t *__restrict__ targets, int V, int S,
-                                                                 int strips, int sw, int csplit, int Rm, float invS,
-                                                                 float grad_scale, float *__restrict__ loss_out, CeXch ws,
-                                                                 int spin_ticks, int take_nothing) {
+__global__ __launch_bounds__(CR_THREADS) void ce_resident_kernel(const typename ST::T *__restrict__ logits,
+                                                                 const int32_t *__restrict__ targets, unsigned *cnt, int V,
+                                                                 int S, unsigned word, int sw, int Rm,
+                                                                 typename ST::T *__restrict__ dlogits, float grad_scale,
+                                                                 float invS, float *__restrict__ loss_out,
+                                                                 unsigned long long *slots, int *fallbacks, int spin_ticks,
+                                                                 int take_nothing) {
     typedef typename ST::Raw Raw;
     constexpr int MPG = MEMBERS / CR_NW;           // members per group of 64 threads (thread = group, slot)
     __shared__ Raw lrow[K_LDS > 0 ? K_LDS : 1][K_LDS > 0 ? CR_THREADS : 1];
     __shared__ float wm[CR_NW][CR_P], wl[CR_NW][CR_P];
     __shared__ float fb[2][CR_W];                  // one member's partial on its way to the threads that hold it
-    __shared__ float fM[CR_W], fInv[CR_W];
+    __shared__ __align__(16) float fM[CR_W], fInv[CR_W];
+    __shared__ __align__(16) int tgt[CR_W];        // the slots' targets as they stand
     __shared__ float strip_loss[CR_MAX_STRIPS];
-    __shared__ unsigned want[MEMBERS];
+    __shared__ unsigned want[MEMBERS], lead[CR_MAX_STRIPS];      // tags of the members, and of the strips' leaders
     __shared__ int failed[MEMBERS], failed_loss[CR_MAX_STRIPS];
     __shared__ int any_failed, any_failed_loss;
     const int tid = threadIdx.x;
     auto rows_of = [&]() { return (Raw (*)[CR_THREADS])lrow; };
     // Workgroups are dealt to the eight XCDs in turn.  The workgroups that read the pieces of one row run at the
     // same time and, where the split allows, on one XCD, so that each L2 sees whole rows.
-    int strip = blockIdx.x % strips, me = blockIdx.x / strips;
+    const CrWord cw = cr_unpack(word);
+    const int strips = cw.strips, csplit = cw.csplit;
+    int me, strip;
     if (csplit % 8 == 0) {
         const int xcd = blockIdx.x % 8, q = blockIdx.x / 8;
-        strip = q % strips;
-        me = xcd + 8 * (q / strips);
+        me = cw.over_strips(q);
+        strip = q - me * strips;
+        me = xcd + 8 * me;
+    } else {
+        me = cw.over_strips(blockIdx.x);
+        strip = blockIdx.x - me * strips;
     }
     const int b = me * strips + strip;           // the workgroup number that owns slots and counter
     const CrGeo<typename ST::T> g = {logits, V, S, strips, sw, csplit, Rm};
-    // the launch tags and the leader's targets are asked for ahead of the rows and wanted only after them
-    const unsigned t_mem = tid < csplit ? ws.cnt[tid * strips + strip] + 1u : 0u;
-    const unsigned t_lead = tid < strips ? ws.cnt[tid] + 1u : 0u;   // member 0 of strip s is workgroup s
-    const unsigned my_tag = ws.cnt[b] + 1u;
-    const int my_tgt = me == 0 && tid < CR_W ? cr_slot_target(g, strip, targets) : -1;
+    // the launch counters and the strip's targets are asked for ahead of the rows and wanted only after them (relaxed atomic
+    // loads: the compiler leaves them where they stand)
+    auto count = [&](int i) { return __hip_atomic_load(cnt + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
+    const unsigned c_mem = count(min(tid, csplit - 1) * strips + strip);
+    const unsigned c_lead = count(min(tid, strips - 1));         // member 0 of strip s is workgroup s
+    const unsigned c_own = count(b);
+    const int my_tgt = cr_slot_target(g, strip, targets);
 
     // ---- pass 1: this member's rows, kept; its partial published
     Raw xr[K_REG];
     float Mp = NO_MAX, Lp = 0.f;
-    cr_member_partial<ST, K_REG, K_LDS, true, NT>(g, strip, me, xr, rows_of(), wm, wl, Mp, Lp);
+    unsigned my_tag = 0;
+    cr_member_partial<ST, K_REG, K_LDS, true, NT>(g, strip, me, xr, rows_of(), wm, wl, Mp, Lp, [&]() {
+        my_tag = __builtin_amdgcn_readfirstlane(c_own) + 1u;
+        if (tid < csplit) { want[tid] = c_mem + 1u; failed[tid] = 0; }
+        if (tid < strips) { lead[tid] = c_lead + 1u; failed_loss[tid] = 0; }
+        if (tid < CR_W) tgt[tid] = my_tgt;
+        if (tid == 0) any_failed = any_failed_loss = 0;
+    });
     if (tid < 4 * CR_W && (tid & 3) < 2)
-        __hip_atomic_store(ws.slots + (size_t)b * CR_STRIDE + (tid & 3) * CR_W + (tid >> 2),
+        __hip_atomic_store(slots + (size_t)b * CR_STRIDE + (tid & 3) * CR_W + (tid >> 2),
                            ((unsigned long long)my_tag << 32) | __float_as_uint((tid & 3) ? Lp : Mp), __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
-    if (tid < csplit) { want[tid] = t_mem; failed[tid] = 0; }
-    if (tid < strips) failed_loss[tid] = 0;
-    if (tid == 0) any_failed = any_failed_loss = 0;
-    const float my_logit = cr_slot_logit(g, strip, my_tgt);         // (in flight while the partners' partials are awaited)
+    const int own_tgt = me == 0 && tid < CR_W ? cr_own_target(g, strip, tgt[tid]) : -1;
+    const float my_logit = cr_slot_logit(g, strip, own_tgt);        // (in flight while the partners' partials are awaited)
     __syncthreads();
     // ---- every member's partial.  Thread (group, slot) fetches the (max, sum) slots of the group's members for
     // its slot: eight of them (sixteen with 128 members).  The loads of a round go out together, so a round costs one trip
     // to the memory side however many of them are still missing.
-    const int mc = tid & 63, mgrp = tid >> 6;
+    const int mc = tid & 63, mgrp = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int mpg = (csplit + CR_NW - 1) / CR_NW;                      // members per group, at most MPG
     float pm[MPG], pl[MPG];
     {
-        unsigned pend = 0;
+        unsigned long long pk[2 * MPG];
+        unsigned tag[MPG];
+        // member q of the group; one that is not there: the last member once more
+        auto member = [&](int q) { return min(mgrp * mpg + q, csplit - 1); };
+        auto there = [&](int q) { return q < mpg && mgrp * mpg + q < csplit; };
+#pragma unroll
+        for (int q = 0; q < MPG; q++) tag[q] = __builtin_amdgcn_readfirstlane(want[member(q)]);
+        for (long long t0 = 0;;) {
+#pragma unroll
+            for (int f = 0; f < 2 * MPG; f++) {
+                const char *from = (const char *)(slots + (size_t)(member(f >> 1) * strips + strip) * CR_STRIDE + (f & 1) * CR_W);
+                pk[f] = __hip_atomic_load((const unsigned long long *)(from + (unsigned)mc * 8u), __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_AGENT);
+            }
+            bool all = true;
+#pragma unroll
+            for (int f = 0; f < 2 * MPG; f++) all = all & ((unsigned)(pk[f] >> 32) == tag[f >> 1]);
+            if (all && !take_nothing) break;
+            const long long now = wall_clock64();
+            if (t0 == 0) t0 = now;
+            if (take_nothing || now - t0 >= (long long)spin_ticks) {       // (test mode: every partner counts as late, whatever its slots hold)
+#pragma unroll
+                for (int f = 0; f < 2 * MPG; f++)
+                    if (there(f >> 1) && (take_nothing || (unsigned)(pk[f] >> 32) != tag[f >> 1])) failed[member(f >> 1)] = 1;
+                any_failed = 1;
+                break;
+            }
+            __builtin_amdgcn_s_sleep(2);
+        }
 #pragma unroll
         for (int q = 0; q < MPG; q++) {
-            pm[q] = NO_MAX;
-            pl[q] = 0.f;
-            if (q < mpg && mgrp * mpg + q < csplit) pend |= 3u << (2 * q);
-        }
-        const long long t0 = wall_clock64();
-        if (take_nothing) {                    // test mode: every partner counts as late, whatever its slots hold
-#pragma unroll
-            for (int f = 0; f < 2 * MPG; f++)
-                if ((pend >> f) & 1u) failed[mgrp * mpg + (f >> 1)] = 1;
-            any_failed = 1;
-            pend = 0;
-        }
-        while (pend) {
-            unsigned long long pk[2 * MPG];
-#pragma unroll
-            for (int f = 0; f < 2 * MPG; f++) {
-                const int p = mgrp * mpg + (f >> 1);
-                if ((pend >> f) & 1u)
-                    pk[f] = __hip_atomic_load(ws.slots + (size_t)(p * strips + strip) * CR_STRIDE + (f & 1) * CR_W + mc,
-                                              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-#pragma unroll
-            for (int f = 0; f < 2 * MPG; f++) {
-                const int p = mgrp * mpg + (f >> 1);
-                if (((pend >> f) & 1u) && (unsigned)(pk[f] >> 32) == want[p]) {
-                    if (f & 1) pl[f >> 1] = __uint_as_float((unsigned)pk[f]);
-                    else pm[f >> 1] = __uint_as_float((unsigned)pk[f]);
-                    pend &= ~(1u << f);
-                }
-            }
-            if (pend) {
-                if (wall_clock64() - t0 >= (long long)spin_ticks) {
-#pragma unroll
-                    for (int f = 0; f < 2 * MPG; f++)
-                        if ((pend >> f) & 1u) failed[mgrp * mpg + (f >> 1)] = 1;
-                    any_failed = 1;
-                    break;
-                }
-                __builtin_amdgcn_s_sleep(2);
-            }
+            pm[q] = there(q) ? __uint_as_float((unsigned)pk[2 * q]) : NO_MAX;
+            pl[q] = there(q) ? __uint_as_float((unsigned)pk[2 * q + 1]) : 0.f;
         }
     }
     // one member's partial from memory, into the threads that hold it
     auto recompute = [&](int s2, int p, float (&qm)[MPG], float (&ql)[MPG]) {
         float M2 = NO_MAX, L2 = 0.f;
-        cr_member_partial<ST, K_REG, K_LDS, false, NT>(g, s2, p, xr, rows_of(), wm, wl, M2, L2);
+        cr_member_partial<ST, K_REG, K_LDS, false, NT>(g, s2, p, xr, rows_of(), wm, wl, M2, L2, []() {});
         if (tid < 4 * CR_W && (tid & 3) == 0) { fb[0][tid >> 2] = M2; fb[1][tid >> 2] = L2; }
         __syncthreads();
 #pragma unroll
@@ -799,7 +843,7 @@ __global__ __launch_bounds__(CR_THREADS) void ce_resident_kernel(typename ST::T 
     };
     __syncthreads();
     if (any_failed) {                                                // the same for every thread: read after the barrier
-        if (tid == 0) atomicAdd(ws.fallbacks, 1);
+        if (tid == 0) atomicAdd(fallbacks, 1);
         for (int p = 0; p < csplit; p++)
             if (failed[p]) recompute(strip, p, pm, pl);
     }
@@ -807,16 +851,16 @@ __global__ __launch_bounds__(CR_THREADS) void ce_resident_kernel(typename ST::T 
     // ---- the loss: a strip's leader forms the strip's term; wave 0 of workgroup 0 adds the terms in order, before its
     // rows (behind them its loads would queue after the workgroup's stores, 2 us at the end of the launch)
     if (tid < CR_W && me == 0) {
-        const float ls = cr_strip_loss(my_tgt, my_logit, fM[tid], fInv[tid]);
+        const float ls = cr_strip_loss(own_tgt, my_logit, fM[tid], fInv[tid]);
         if (tid == 0)
-            __hip_atomic_store(ws.slots + (size_t)b * CR_STRIDE + CR_LOSS_SLOT,
+            __hip_atomic_store(slots + (size_t)b * CR_STRIDE + CR_LOSS_SLOT,
                                ((unsigned long long)my_tag << 32) | __float_as_uint(ls), __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_AGENT);
         if (strip == 0) {
             float val = ls;
             bool late = false;
             if (tid > 0 && tid < strips)
-                late = take_nothing || !cr_wait_slot(ws.slots + (size_t)tid * CR_STRIDE + CR_LOSS_SLOT, t_lead, spin_ticks, val);
+                late = take_nothing || !cr_wait_slot(slots + (size_t)tid * CR_STRIDE + CR_LOSS_SLOT, lead[tid], spin_ticks, val);
             if (tid < strips) strip_loss[tid] = val;
             if (late) { failed_loss[tid] = 1; any_failed_loss = 1; }
             float total = 0.f;
@@ -829,43 +873,55 @@ __global__ __launch_bounds__(CR_THREADS) void ce_resident_kernel(typename ST::T 
     {
         const int lc = tid & 15;
         int row0 = tid >> 4;
-        asm volatile("" : "+v"(row0));     // the row masks are formed again here instead of being kept from pass 1
+        asm volatile("" : "+v"(row0));     // the addresses are formed again here instead of being kept from pass 1
         const LaneCols mine = cr_cols(strip, sw, lc, S);
-        const CrRows r = cr_rows(g, me);
+        const CrRows r = cr_rows(g, me, mine.col, row0);
         const int K = r.K, kR = max(0, K - K_REG), kL = max(0, kR - K_LDS);
-        const int mineK = !mine.ok ? 0 : row0 < r.last ? K : K - 1;      // steps in which this lane has a row to write
         const typename ST::T *src = logits + (size_t)r.v_lo * S;
         typename ST::T *dst = dlogits + (size_t)r.v_lo * S;
-        const unsigned loff = (unsigned)row0 * (unsigned)S + (unsigned)mine.col;
-        const size_t step = (size_t)CR_RPS * S;
-        float M[4], inv[4], sc[4];
+        // A value costs the exponential and one product: f is 1/L, 1/S and the scale in one.  The targets, one or two of the rows of a
+        // workgroup, are put in by a step that knows it has one (`hot`), with 1/L by itself, so that p - 1 is what it would be.
+        // With the comparison, the subtraction and three products at every value bfloat16 [32000][200] wrote its rows in 4.1 us, now in 3.6.
+        // With the order of the loads: [32000][200] 14.7 -> 12.4 us, fp32 [151936][256] 65 -> 60.4, [24573][256] 16.3 -> 14.6.
+        float M[4], f[4];
         int tk[4];                         // the target's row is this lane's row of step k when tk == 64k
+        unsigned long long hot = 0;        // steps in which a lane of the wave has one
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             M[j] = fM[lc * 4 + j];
-            inv[j] = fInv[lc * 4 + j];
-            const int tg = targets[mine.col + j];
+            const int tg = tgt[lc * 4 + j];
             const bool ok = tg >= 0 && tg < V;
             tk[j] = ok ? tg - r.v_lo - row0 : -1;
-            sc[j] = ok ? invS : 1.0f;      // an out-of-range target leaves the column unscaled (stories_cpu_ops.h:98)
+            // an out-of-range target leaves the column unscaled (stories_cpu_ops.h:98)
+            f[j] = (fInv[lc * 4 + j] * (ok ? invS : 1.0f)) * grad_scale;
+            int k = mine.ok && tk[j] >= 0 && tk[j] % CR_RPS == 0 && tk[j] / CR_RPS < K ? tk[j] / CR_RPS : -1;
+            while (const unsigned long long some = __builtin_amdgcn_ballot_w64(k >= 0)) {
+                const int one = __builtin_amdgcn_readlane(k, __builtin_ctzll(some));
+                hot |= 1ull << one;
+                if (k == one) k = -1;
+            }
         }
         auto emit = [&](int k, const Raw &x) {
-            if (k >= mineK) return;
             float o[4];
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                float pj = exp_neg(ST::at(x, j) - M[j]) * inv[j];
-                if (tk[j] == CR_RPS * k) pj -= 1.0f;
-                o[j] = (pj * sc[j]) * grad_scale;
+            for (int j = 0; j < 4; j++) o[j] = exp_neg(ST::at(x, j) - M[j]) * f[j];
+            if ((hot >> k) & 1) {
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    if (tk[j] == CR_RPS * k) o[j] = ((exp_neg(ST::at(x, j) - M[j]) * fInv[lc * 4 + j] - 1.0f) * invS) * grad_scale;
             }
-            ST::template st<NT>(dst + k * step + loff, o);
+            if (mine.ok && (k < K - 1 || row0 < r.last))
+                ST::template st<NT>((typename ST::T *)((char *)dst + (size_t)((unsigned)k * r.step) + r.off), o);
         };
         // the rows read a second time run up to sixteen ahead of their use, in the registers that the register
         // rows leave as they are written out
         auto loadg = [&](Raw (&t)[CR_SUB], int k0) {
 #pragma unroll
             for (int u = 0; u < CR_SUB; u++)
-                if (k0 + u < kL) t[u] = NT ? ST::ld_nt(src + (k0 + u) * step + loff) : ST::ld(src + (k0 + u) * step + loff);
+                if (k0 + u < kL) {
+                    const typename ST::T *at = (const typename ST::T *)((const char *)src + (size_t)((unsigned)(k0 + u) * r.step) + r.off);
+                    t[u] = NT ? ST::ld_nt(at) : ST::ld(at);
+                }
         };
         auto emitg = [&](const Raw (&t)[CR_SUB], int k0) {
 #pragma unroll
@@ -910,7 +966,7 @@ __global__ __launch_bounds__(CR_THREADS) void ce_resident_kernel(typename ST::T 
                     for (int p = 0; p < csplit; p++) recompute(s2, p, qm, ql);
                     cr_merge_members(qm, ql, wm, wl, fM, fInv);
                     if (tid < CR_W) {
-                        const int tg = cr_slot_target(g, s2, targets);
+                        const int tg = cr_own_target(g, s2, cr_slot_target(g, s2, targets));
                         const float ls = cr_strip_loss(tg, cr_slot_logit(g, s2, tg), fM[tid], fInv[tid]);
                         if (tid == 0) strip_loss[s2] = ls;
                     }
@@ -924,7 +980,7 @@ __global__ __launch_bounds__(CR_THREADS) void ce_resident_kernel(typename ST::T 
             }
         }
     }
-    if (tid == 0) ws.cnt[b] = my_tag;
+    if (tid == 0) cnt[b] = my_tag;
 }
 
 // resident workgroups of the second pass per compute unit (asked of the runtime once per storage type)
@@ -1006,9 +1062,10 @@ int ce_run(const char *who, T *dlogits, float *loss_dev, const T *logits, const 
                 xch.fallbacks = (int *)(base + CE_SCRATCH_BYTES + (size_t)CR_MAX_WG * CR_STRIDE * 8 + (size_t)CR_MAX_WG * 4);
                 auto launch = [&](auto kernel) {
                     const int spin = mi355_exchange_spin_ticks();
-                    hipLaunchKernelGGL(kernel, dim3((unsigned)(csplit * strips_r)), dim3(CR_THREADS), 0, g_ctx.stream, dlogits,
-                                       logits, targets, V, S, strips_r, sw, csplit, Rm, 1.0f / (float)S, grad_scale, loss_dev,
-                                       xch, spin < 0 ? 0 : spin, g_ctx.xch_take_nothing > 0 ? 1 : 0);
+                    hipLaunchKernelGGL(kernel, dim3((unsigned)(csplit * strips_r)), dim3(CR_THREADS), 0, g_ctx.stream, logits,
+                                       targets, xch.cnt, V, S, cr_word(strips_r, csplit), sw, Rm, dlogits, grad_scale,
+                                       1.0f / (float)S, loss_dev, xch.slots, xch.fallbacks, spin < 0 ? 0 : spin,
+                                       g_ctx.xch_take_nothing > 0 ? 1 : 0);
                 };
                 if (csplit > CR_MAX_SPLIT / 2 && K <= 8) {
                     if (lines) launch(ce_resident_kernel<ST, 8, 0, true, CR_MAX_SPLIT>);
@@ -1017,6 +1074,7 @@ int ce_run(const char *who, T *dlogits, float *loss_dev, const T *logits, const 
                     if (lines) launch(ce_resident_kernel<ST, 8, ST::K_LDS, true, CR_MAX_SPLIT>);
                     else launch(ce_resident_kernel<ST, 8, ST::K_LDS, false, CR_MAX_SPLIT>);
                 }
+                else if (K <= 4) { if (lines) launch(ce_resident_kernel<ST, 4, 0, true>); else launch(ce_resident_kernel<ST, 4, 0, false>); }
                 else if (K <= 8) { if (lines) launch(ce_resident_kernel<ST, 8, 0, true>); else launch(ce_resident_kernel<ST, 8, 0, false>); }
                 else if (K <= 16) { if (lines) launch(ce_resident_kernel<ST, 16, 0, true>); else launch(ce_resident_kernel<ST, 16, 0, false>); }
                 else if (lines) launch(ce_resident_kernel<ST, ST::K_REG, ST::K_LDS, true>);
