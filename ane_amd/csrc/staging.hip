@@ -14,6 +14,7 @@
 #include "common.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace {
 
@@ -87,21 +88,20 @@ __global__ __launch_bounds__(ST_THREADS) void cvt_f16_f32_v1(float *__restrict__
 
 // ---- attention-gradient finish ----
 template <typename T, int VEC>
-__device__ __forceinline__ void load_cols(float (&o)[VEC], const T *p) {
-    if constexpr (VEC == 1) {
-        o[0] = (float)p[0];
-    } else if constexpr (sizeof(T) == 2) {
-        static_assert(VEC == 4, "fp16 rows are read 4 columns at a time");
-        const h4 v = __builtin_nontemporal_load(reinterpret_cast<const h4_any *>(p));
-#pragma unroll
-        for (int j = 0; j < 4; j++) o[j] = (float)v[j];
-    } else {
-        static_assert(VEC == 4, "fp32 rows are read 4 columns at a time");
-        const v4f v = ld4_nt(reinterpret_cast<const float *>(p));
-#pragma unroll
-        for (int j = 0; j < 4; j++) o[j] = v[j];
+struct Cols {
+    static_assert(VEC == 1 || VEC == 4, "rows are read 4 columns at a time");
+    typedef T Any __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+    typedef T Vec __attribute__((ext_vector_type(4)));
+    typedef typename std::conditional<VEC == 4, Vec, T>::type Raw;
+    static __device__ __forceinline__ Raw load(const T *p) {
+        if constexpr (VEC == 4) return __builtin_nontemporal_load(reinterpret_cast<const Any *>(p));
+        else return *p;
     }
-}
+    static __device__ __forceinline__ float at(const Raw &r, int j) {
+        if constexpr (VEC == 4) return (float)r[j];
+        else return (float)r;
+    }
+};
 
 // table rows are shared by every head and sequence: ordinary (cached) loads
 template <int VEC>
@@ -136,59 +136,40 @@ __device__ __forceinline__ void store_cols(float *p, const float (&o)[VEC]) {
 // lane has rotated; one column per lane there).  [8][2048][1001] fp16 in: 89.4 us with one column per lane, now 45.2.
 // Four columns per lane for fp16 too, whose stores are then whole lines: [16][2048][256] 22.4 us (117 MB: 5.2 TB/s)
 // against 25.2 with eight, [16][2048][250] 24.6 against 26.9 (48.1 with one).  Pair rows are numbered Q heads first, then K heads, then V heads.
-template <typename T, int VEC>
+// TABLE: dQ and dK are rotated back.  WAVE: rows are whole waves of columns, so that a wave has one row and what follows of its number
+// (three divisions among it) is scalar.
+template <typename T, int VEC, bool TABLE, bool WAVE>
 __global__ __launch_bounds__(ST_THREADS) void attn_grads_finish_kernel(
-    float *dq, float *__restrict__ dk, float *__restrict__ dv, const T *qf, const T *__restrict__ kf,
-    const T *__restrict__ vf, size_t sq, size_t sk, size_t sv, int heads, int kv_heads, int ratio, int hd, int S,
-    int batch, const float *__restrict__ cos_t, const float *__restrict__ sin_t, size_t total) {
+    const T *qf, const T *__restrict__ kf, const T *__restrict__ vf, int S, int hd, int heads, int kv_heads, int ratio, int batch,
+    unsigned total, const float *__restrict__ cos_t, const float *__restrict__ sin_t, size_t sq, size_t sk, size_t sv, float *dq,
+    float *__restrict__ dk, float *__restrict__ dv) {
+    typedef Cols<T, VEC> Col;
+    typedef typename Col::Raw Raw;
     const unsigned idx = blockIdx.x * ST_THREADS + threadIdx.x;
     if (idx >= total) return;
     const unsigned colg = ((unsigned)S + VEC - 1) / VEC;
-    unsigned pr = idx / colg;
+    unsigned pr, group;
+    if constexpr (WAVE) {
+        const unsigned wave = __builtin_amdgcn_readfirstlane(idx >> 6);
+        pr = wave / (colg >> 6);
+        group = ((wave - pr * (colg >> 6)) << 6) + (threadIdx.x & 63);
+    } else {
+        pr = idx / colg;
+        group = idx - pr * colg;
+    }
+    const int s = (int)last_whole((size_t)group * VEC, VEC, S);
     const unsigned half = (unsigned)hd >> 1;
-    const int s = (int)last_whole((size_t)(idx - pr * colg) * VEC, VEC, S);
     const unsigned q_rows = (unsigned)batch * heads * half, kv_rows = (unsigned)batch * kv_heads * half;
 
-    float r0[VEC], r1[VEC];
-    float *out;
-    int i;
-    bool rotate;
-    if (pr < q_rows) {
-        const unsigned bh = pr / half;               // b*heads + h
-        i = (int)(pr - bh * half);
-        const size_t b = bh / (unsigned)heads, h = bh - b * heads;
-        const T *in = qf + b * sq + (h * hd + 2 * i) * (size_t)S + s;
-        load_cols<T, VEC>(r0, in);
-        load_cols<T, VEC>(r1, in + S);
-        out = dq + ((size_t)bh * hd + 2 * i) * (size_t)S + s;
-        rotate = true;
-    } else {
-        pr -= q_rows;
-        const bool is_k = pr < kv_rows;
-        if (!is_k) pr -= kv_rows;
-        const unsigned bh = pr / half;               // b*kv_heads + kv
-        i = (int)(pr - bh * half);
-        const size_t b = bh / (unsigned)kv_heads, kv = bh - b * kv_heads;
-        const T *in = (is_k ? kf + b * sk : vf + b * sv) + ((kv * ratio) * hd + 2 * i) * (size_t)S + s;
-#pragma unroll
-        for (int j = 0; j < VEC; j++) r0[j] = r1[j] = 0.f;
-        for (int r = 0; r < ratio; r++) {            // zero, then += in query-head order (io.h:342-350)
-            float a0[VEC], a1[VEC];
-            load_cols<T, VEC>(a0, in + (size_t)r * hd * S);
-            load_cols<T, VEC>(a1, in + (size_t)r * hd * S + S);
-#pragma unroll
-            for (int j = 0; j < VEC; j++) {
-                r0[j] += a0[j];
-                r1[j] += a1[j];
-            }
-        }
-        out = (is_k ? dk : dv) + ((size_t)bh * hd + 2 * i) * (size_t)S + s;
-        rotate = is_k;
-    }
-    if (rotate && cos_t) {
-        float c[VEC], sn[VEC];
+    // Each kind of row asks for all it will read before it uses any: with the table read where the rotation is, and a query head
+    // when the one before it had been added, a K row of two heads made three trips to memory one after the other
+    // ([16][2048][256] with eight KV heads, fp16, 117 MB: 22.8 us, now 21.4 with the scalar rows).
+    float r0[VEC], r1[VEC], c[VEC], sn[VEC];
+    auto ask_table = [&](int i) {
         load_tab<VEC>(c, cos_t + (size_t)i * S + s);
         load_tab<VEC>(sn, sin_t + (size_t)i * S + s);
+    };
+    auto turn = [&]() {
 #pragma unroll
         for (int j = 0; j < VEC; j++) {
             // inverse rotation, written as the forward one with the sine negated
@@ -197,6 +178,52 @@ __global__ __launch_bounds__(ST_THREADS) void attn_grads_finish_kernel(
             r0[j] = x0 * c[j] - x1 * ns;
             r1[j] = x0 * ns + x1 * c[j];
         }
+    };
+    float *out;
+    if (pr < q_rows) {
+        const unsigned bh = pr / half;               // b*heads + h
+        const int i = (int)(pr - bh * half);
+        const size_t b = bh / (unsigned)heads, h = bh - b * heads;
+        const T *in = qf + b * sq + (h * hd + 2 * i) * (size_t)S + s;
+        out = dq + ((size_t)bh * hd + 2 * i) * (size_t)S + s;
+        if (TABLE) ask_table(i);
+        const Raw a0 = Col::load(in), a1 = Col::load(in + S);
+#pragma unroll
+        for (int j = 0; j < VEC; j++) {
+            r0[j] = Col::at(a0, j);
+            r1[j] = Col::at(a1, j);
+        }
+        if (TABLE) turn();
+    } else {
+        pr -= q_rows;
+        const bool is_k = pr < kv_rows;
+        if (!is_k) pr -= kv_rows;
+        const unsigned bh = pr / half;               // b*kv_heads + kv
+        const int i = (int)(pr - bh * half);
+        const size_t b = bh / (unsigned)kv_heads, kv = bh - b * kv_heads, head = (size_t)hd * S;
+        const T *in = (is_k ? kf + b * sk : vf + b * sv) + ((kv * ratio) * hd + 2 * i) * (size_t)S + s;
+        out = (is_k ? dk : dv) + ((size_t)bh * hd + 2 * i) * (size_t)S + s;
+        if (TABLE) ask_table(i);                     // (also for V rows, which have no use for it: no branch between the loads)
+        const T *second = in + (ratio > 1 ? head : 0);
+        const Raw a0 = Col::load(in), a1 = Col::load(in + S), b0 = Col::load(second), b1 = Col::load(second + S);
+        __builtin_amdgcn_sched_barrier(0);           // (the compiler would use the first before it asks for the others)
+        auto add = [&](const Raw &x0, const Raw &x1) {
+#pragma unroll
+            for (int j = 0; j < VEC; j++) {
+                r0[j] += Col::at(x0, j);
+                r1[j] += Col::at(x1, j);
+            }
+        };
+#pragma unroll
+        for (int j = 0; j < VEC; j++) r0[j] = r1[j] = 0.f;
+        add(a0, a1);                                 // zero, then += in query-head order (io.h:342-350)
+#pragma unroll
+        for (int j = 0; j < VEC; j++) {              // (selects: behind a branch the second head would be read there)
+            r0[j] = ratio > 1 ? r0[j] + Col::at(b0, j) : r0[j];
+            r1[j] = ratio > 1 ? r1[j] + Col::at(b1, j) : r1[j];
+        }
+        for (int r = 2; r < ratio; r++) add(Col::load(in + r * head), Col::load(in + r * head + S));
+        if (TABLE && is_k) turn();
     }
     store_cols<VEC>(out, r0);
     store_cols<VEC>(out + S, r1);
@@ -282,23 +309,25 @@ MI355_API int mi355_attn_grads_finish_dev(float *dq, float *dk, float *dv, const
         const size_t lanes = pairs * ceil_div((size_t)S, (size_t)vec);
         const int per = (int)std::min<size_t>(std::max<size_t>(ST_LANES / lanes, 1), (size_t)batch);   // sequences of one launch
         const size_t kv_full = (size_t)kv_heads * hd * S;
+        static_assert(ST_LANES < 1ull << 32, "a launch's lanes are counted in 32 bits");
         for (int b = 0; b < batch; b += std::min(per, batch - b)) {
             const int n = std::min(per, batch - b);
             hipLaunchKernelGGL(kernel, dim3((unsigned)ceil_div(lanes * n, ST_THREADS)), dim3(ST_THREADS), 0, g_ctx.stream,
-                               dq + b * full, dk + b * kv_full, dv + b * kv_full, q + b * q_stride, k + b * k_stride,
-                               v + b * v_stride, q_stride, k_stride, v_stride, heads, kv_heads, ratio, hd, S, n, cos_dev,
-                               sin_dev, lanes * n);
+                               q + b * q_stride, k + b * k_stride, v + b * v_stride, S, hd, heads, kv_heads, ratio, n,
+                               (unsigned)(lanes * n), cos_dev, sin_dev, q_stride, k_stride, v_stride, dq + b * full,
+                               dk + b * kv_full, dv + b * kv_full);
         }
     };
-#define FINISH(T, VEC)                                                                                               \
-    launch(attn_grads_finish_kernel<T, VEC>, (const T *)dq_full, (const T *)dk_full, (const T *)dv_full, VEC)
-    if (in_f16) {
-        if (S % 4 == 0 || (S > 4 && !in_place)) FINISH(_Float16, 4);
-        else FINISH(_Float16, 1);
-    } else {
-        if (S % 4 == 0 || (S > 4 && !in_place)) FINISH(float, 4);
-        else FINISH(float, 1);
-    }
+#define FINISH_AS(T, VEC, WAVE)                                                                                      \
+    if (cos_dev) launch(attn_grads_finish_kernel<T, VEC, true, WAVE>, (const T *)dq_full, (const T *)dk_full, (const T *)dv_full, VEC); \
+    else launch(attn_grads_finish_kernel<T, VEC, false, WAVE>, (const T *)dq_full, (const T *)dk_full, (const T *)dv_full, VEC)
+#define FINISH(T)                                                                                                    \
+    if (S % 256 == 0) { FINISH_AS(T, 4, true); }                                                                     \
+    else if (S % 4 == 0 || (S > 4 && !in_place)) { FINISH_AS(T, 4, false); }                                         \
+    else { FINISH_AS(T, 1, false); }
+    if (in_f16) { FINISH(_Float16) }
+    else { FINISH(float) }
+#undef FINISH_AS
 #undef FINISH
     LAUNCH_OK("attn_grads_finish");
     return 0;
