@@ -58,25 +58,25 @@ __global__ __launch_bounds__(BT) void cvt_bf16_f32_kernel(float *__restrict__ ds
 // ---- SwiGLU and the residual family ----
 __device__ __forceinline__ float sigmoid_ref(float h) { return 1.0f / (1.0f + expf(-h)); }
 
-template <int VEC>
-__global__ __launch_bounds__(BT) void swiglu_fwd_bf16_kernel(bf16_t *__restrict__ out, const bf16_t *__restrict__ h1,
+template <int VEC, int THREADS = BT>
+__global__ __launch_bounds__(THREADS) void swiglu_fwd_bf16_kernel(bf16_t *__restrict__ out, const bf16_t *__restrict__ h1,
                                                              const bf16_t *__restrict__ h3, size_t nv) {
-    const size_t i = (size_t)blockIdx.x * BT + threadIdx.x;
+    const size_t i = (size_t)blockIdx.x * THREADS + threadIdx.x;
     if (i >= nv) return;
     float a[VEC], b[VEC], o[VEC];
     ldb<VEC, true>(a, h1 + VEC * i);
     ldb<VEC, true>(b, h3 + VEC * i);
 #pragma unroll
     for (int j = 0; j < VEC; j++) o[j] = (a[j] * sigmoid_ref(a[j])) * b[j];
-    stb<VEC>(out + VEC * i, o);
+    stb<VEC, THREADS == FAR_THREADS>(out + VEC * i, o);
 }
 
-template <int VEC>
-__global__ __launch_bounds__(BT) void swiglu_bwd_bf16_kernel(bf16_t *__restrict__ dh1, bf16_t *__restrict__ dh3,
+template <int VEC, int THREADS = BT>
+__global__ __launch_bounds__(THREADS) void swiglu_bwd_bf16_kernel(bf16_t *__restrict__ dh1, bf16_t *__restrict__ dh3,
                                                              const bf16_t *__restrict__ ds,
                                                              const bf16_t *__restrict__ h1,
                                                              const bf16_t *__restrict__ h3, size_t nv) {
-    const size_t i = (size_t)blockIdx.x * BT + threadIdx.x;
+    const size_t i = (size_t)blockIdx.x * THREADS + threadIdx.x;
     if (i >= nv) return;
     float d[VEC], a[VEC], b[VEC], o1[VEC], o3[VEC];
     ldb<VEC, true>(d, ds + VEC * i);
@@ -92,21 +92,21 @@ __global__ __launch_bounds__(BT) void swiglu_bwd_bf16_kernel(bf16_t *__restrict_
         u = sig * u;
         o1[j] = (d[j] * b[j]) * u;
     }
-    stb<VEC>(dh1 + VEC * i, o1);
-    stb<VEC>(dh3 + VEC * i, o3);
+    stb<VEC, THREADS == FAR_THREADS>(dh1 + VEC * i, o1);
+    stb<VEC, THREADS == FAR_THREADS>(dh3 + VEC * i, o3);
 }
 
-template <int VEC, int MODE>
-__global__ __launch_bounds__(BT) void axpby_bf16_kernel(bf16_t *y, const bf16_t *a, const bf16_t *b, float alpha,
+template <int VEC, int MODE, int THREADS = BT>
+__global__ __launch_bounds__(THREADS) void axpby_bf16_kernel(bf16_t *y, const bf16_t *a, const bf16_t *b, float alpha,
                                                         size_t nv) {
-    const size_t i = (size_t)blockIdx.x * BT + threadIdx.x;
+    const size_t i = (size_t)blockIdx.x * THREADS + threadIdx.x;
     if (i >= nv) return;
     float x[VEC], z[VEC], o[VEC];
     ldb<VEC, true>(x, a + VEC * i);
     if (MODE != 1) ldb<VEC, true>(z, b + VEC * i);
 #pragma unroll
     for (int j = 0; j < VEC; j++) o[j] = MODE == 0 ? z[j] * alpha + x[j] : MODE == 1 ? x[j] * alpha : x[j] + z[j];
-    stb<VEC>(y + VEC * i, o);
+    stb<VEC, THREADS == FAR_THREADS>(y + VEC * i, o);
 }
 
 // ---- RMSNorm forward / backward: the fp32 tile (workgroup = all C rows x a strip of columns) with 8-column lanes ----
@@ -705,6 +705,11 @@ int cvt_check(const char *who, const void *dst, const void *src, size_t dst_ld, 
 }
 
 inline unsigned blocks_for(size_t work) { return (unsigned)ceil_div(work, (size_t)BT); }
+// streams of nv groups of eight whose results go out by st16_far: large ones that start on a line, a wave to a workgroup
+inline bool bf_far(size_t nv, const void *out, const void *out2 = nullptr) {
+    return 16 * nv >= FAR_BYTES && (((uintptr_t)out | (uintptr_t)out2) & 127u) == 0;
+}
+#define BF_FAR(nv) dim3((unsigned)ceil_div(nv, (size_t)FAR_THREADS)), dim3(FAR_THREADS), 0, g_ctx.stream
 
 }   // namespace
 
@@ -742,7 +747,9 @@ MI355_API int mi355_swiglu_fwd_bf16_dev(uint16_t *out, const uint16_t *h1, const
     if (!mi355_ready("swiglu_fwd_bf16")) return -1;
     if (!out || !h1 || !h3) return mi355_fail("swiglu_fwd_bf16: NULL pointer");
     if (n == 0) return mi355_fail("swiglu_fwd_bf16: empty tensor");
-    if (n % 8 == 0 && aligned16(out) && aligned16(h1) && aligned16(h3))
+    if (n % 8 == 0 && aligned16(h1) && aligned16(h3) && bf_far(n / 8, out))
+        hipLaunchKernelGGL((swiglu_fwd_bf16_kernel<8, FAR_THREADS>), BF_FAR(n / 8), out, h1, h3, n / 8);
+    else if (n % 8 == 0 && aligned16(out) && aligned16(h1) && aligned16(h3))
         hipLaunchKernelGGL(swiglu_fwd_bf16_kernel<8>, dim3(blocks_for(n / 8)), dim3(BT), 0, g_ctx.stream, out, h1, h3, n / 8);
     else
         hipLaunchKernelGGL(swiglu_fwd_bf16_kernel<1>, dim3(blocks_for(n)), dim3(BT), 0, g_ctx.stream, out, h1, h3, n);
@@ -755,7 +762,9 @@ MI355_API int mi355_swiglu_bwd_bf16_dev(uint16_t *dh1, uint16_t *dh3, const uint
     if (!mi355_ready("swiglu_bwd_bf16")) return -1;
     if (!dh1 || !dh3 || !dsilu || !h1 || !h3) return mi355_fail("swiglu_bwd_bf16: NULL pointer");
     if (n == 0) return mi355_fail("swiglu_bwd_bf16: empty tensor");
-    if (n % 8 == 0 && aligned16(dh1) && aligned16(dh3) && aligned16(dsilu) && aligned16(h1) && aligned16(h3))
+    if (n % 8 == 0 && aligned16(dsilu) && aligned16(h1) && aligned16(h3) && bf_far(n / 8, dh1, dh3))
+        hipLaunchKernelGGL((swiglu_bwd_bf16_kernel<8, FAR_THREADS>), BF_FAR(n / 8), dh1, dh3, dsilu, h1, h3, n / 8);
+    else if (n % 8 == 0 && aligned16(dh1) && aligned16(dh3) && aligned16(dsilu) && aligned16(h1) && aligned16(h3))
         hipLaunchKernelGGL(swiglu_bwd_bf16_kernel<8>, dim3(blocks_for(n / 8)), dim3(BT), 0, g_ctx.stream, dh1, dh3, dsilu, h1, h3, n / 8);
     else
         hipLaunchKernelGGL(swiglu_bwd_bf16_kernel<1>, dim3(blocks_for(n)), dim3(BT), 0, g_ctx.stream, dh1, dh3, dsilu, h1, h3, n);
@@ -771,9 +780,12 @@ MI355_API int mi355_axpby_bf16_dev(uint16_t *y, const uint16_t *a, const uint16_
     const bool vec = n % 8 == 0 && aligned16(y) && aligned16(a) && (mode == 1 || aligned16(b));
     const size_t nv = vec ? n / 8 : n;
 #define AX(V, M) hipLaunchKernelGGL((axpby_bf16_kernel<V, M>), dim3(blocks_for(nv)), dim3(BT), 0, g_ctx.stream, y, a, b, alpha, nv)
-    if (vec) { if (mode == 0) AX(8, 0); else if (mode == 1) AX(8, 1); else AX(8, 2); }
+#define AXF(M) hipLaunchKernelGGL((axpby_bf16_kernel<8, M, FAR_THREADS>), BF_FAR(nv), y, a, b, alpha, nv)
+    if (vec && bf_far(nv, y)) { if (mode == 0) AXF(0); else if (mode == 1) AXF(1); else AXF(2); }
+    else if (vec) { if (mode == 0) AX(8, 0); else if (mode == 1) AX(8, 1); else AX(8, 2); }
     else { if (mode == 0) AX(1, 0); else if (mode == 1) AX(1, 1); else AX(1, 2); }
 #undef AX
+#undef AXF
     LAUNCH_OK("axpby_bf16");
     return 0;
 }

@@ -115,6 +115,30 @@ __device__ __forceinline__ v4f ld4_nt(const float *p) {
     return __builtin_nontemporal_load(reinterpret_cast<const v4f_any *>(p));
 }
 
+// A streaming store that is written through to memory (scope bits of an agent store besides the streaming one), so that the
+// XCDs' L2s do not hold it back until the lines are wanted or the kernel ends.  For results of whole 128-byte lines, written
+// in the order of the grid, of FAR_BYTES and more to a tensor; the elementwise ops and the optimizer, with workgroups of one wave
+// each (FAR_THREADS), which come and go one at a time (the converts are as quick in workgroups of 256, the INT8 dequantizer, which
+// reads 4 bytes per lane, quicker: 4.2 M values 5.6 us with st4, 4.7 in waves, 4.1).  Per launch on cold operands, us, workgroups of 256 with st4_nt / this: one tensor in and one out of 48 MB 17.0 /
+// 16.2, of 24 MB 9.7 / 9.0, two in and one out of 24 MB 13.0 / 12.8, of 12 MB 7.7 / 7.3, of 4 MB 3.35 / 3.56, three in and two out of
+// 48 MB 40.4 / 39.5, of 12 MB 11.8 / 11.4, of 4 MB 4.9 / 4.9.  Pieces of lines are written one by one: rotated rows of 197 floats
+// 5.3 -> 6.2.  (Written through, but not marked as streaming, results also stay in the last-level cache, and what reads them next
+// is quicker, two in and one out of 48 MB 24 -> 19; what they push out of it is what the op after that wanted: over a layer no gain.)
+// There is no builtin for it.  The data registers of a store of 16 bytes must not be written by the next instruction, which the
+// compiler cannot know of this one: hence the s_nop.
+constexpr size_t FAR_BYTES = (size_t)8 << 20;
+constexpr int FAR_THREADS = 64;
+template <typename V>
+__device__ __forceinline__ void st16_far(void *p, V v) {
+    static_assert(sizeof(V) == 16, "one 128-bit access");
+    asm volatile("global_store_dwordx4 %0, %1, off sc1 nt\n\ts_nop 1" : : "v"(p), "v"(v) : "memory");
+}
+template <bool FAR>
+__device__ __forceinline__ void st4_stream(float *p, v4f v) {
+    if constexpr (FAR) st16_far(p, v);
+    else st4_nt(p, v);
+}
+
 // Value of lane (l ^ M) of a wave64, through the cheapest path measured for each distance: a DPP quad permute inside
 // the adder for 1 and 2, ds_bpermute for 4, 8 and 16, v_permlane32_swap for 32.  (ds_swizzle in bit-mask mode also
 // reaches 4, 8 and 16, without an address register, but the 16-wave RMSNorm tile ran 0.2-0.3 us slower with it

@@ -20,14 +20,14 @@ __device__ __forceinline__ float sigmoid_ref(float h) {
 }
 
 // ---- SwiGLU forward: out = (h1*sig(h1))*h3  (mil_dynamic.h:264-266) ----
-template <int UNROLL>
-__global__ __launch_bounds__(EW_THREADS) void swiglu_fwd_kernel(float *__restrict__ out, const float *__restrict__ h1,
+template <int UNROLL, int THREADS = EW_THREADS>
+__global__ __launch_bounds__(THREADS) void swiglu_fwd_kernel(float *__restrict__ out, const float *__restrict__ h1,
                                                                 const float *__restrict__ h3, size_t n4) {
-    const size_t base = (size_t)blockIdx.x * (EW_THREADS * UNROLL) + threadIdx.x;
+    const size_t base = (size_t)blockIdx.x * (THREADS * UNROLL) + threadIdx.x;
     v4f a[UNROLL], b[UNROLL];
 #pragma unroll
     for (int u = 0; u < UNROLL; u++) {
-        const size_t i = base + (size_t)u * EW_THREADS;
+        const size_t i = base + (size_t)u * THREADS;
         if (i < n4) {
             a[u] = ld4_nt(h1 + 4 * i);
             b[u] = ld4_nt(h3 + 4 * i);
@@ -35,12 +35,12 @@ __global__ __launch_bounds__(EW_THREADS) void swiglu_fwd_kernel(float *__restric
     }
 #pragma unroll
     for (int u = 0; u < UNROLL; u++) {
-        const size_t i = base + (size_t)u * EW_THREADS;
+        const size_t i = base + (size_t)u * THREADS;
         if (i < n4) {
             v4f o;
 #pragma unroll
             for (int j = 0; j < 4; j++) o[j] = (a[u][j] * sigmoid_ref(a[u][j])) * b[u][j];
-            st4_nt(out + 4 * i, o);
+            st4_stream<THREADS == FAR_THREADS>(out + 4 * i, o);
         }
     }
 }
@@ -61,16 +61,16 @@ __device__ __forceinline__ void swiglu_bwd_elem(float d, float h, float g, float
     dh1 = (d * g) * u;
 }
 
-template <int UNROLL>
-__global__ __launch_bounds__(EW_THREADS) void swiglu_bwd_kernel(float *__restrict__ dh1, float *__restrict__ dh3,
+template <int UNROLL, int THREADS = EW_THREADS>
+__global__ __launch_bounds__(THREADS) void swiglu_bwd_kernel(float *__restrict__ dh1, float *__restrict__ dh3,
                                                                 const float *__restrict__ ds,
                                                                 const float *__restrict__ h1,
                                                                 const float *__restrict__ h3, size_t n4) {
-    const size_t base = (size_t)blockIdx.x * (EW_THREADS * UNROLL) + threadIdx.x;
+    const size_t base = (size_t)blockIdx.x * (THREADS * UNROLL) + threadIdx.x;
     v4f a[UNROLL], b[UNROLL], d[UNROLL];
 #pragma unroll
     for (int u = 0; u < UNROLL; u++) {
-        const size_t i = base + (size_t)u * EW_THREADS;
+        const size_t i = base + (size_t)u * THREADS;
         if (i < n4) {
             d[u] = ld4_nt(ds + 4 * i);
             a[u] = ld4_nt(h1 + 4 * i);
@@ -79,7 +79,7 @@ __global__ __launch_bounds__(EW_THREADS) void swiglu_bwd_kernel(float *__restric
     }
 #pragma unroll
     for (int u = 0; u < UNROLL; u++) {
-        const size_t i = base + (size_t)u * EW_THREADS;
+        const size_t i = base + (size_t)u * THREADS;
         if (i < n4) {
             v4f o1, o3;
 #pragma unroll
@@ -89,8 +89,8 @@ __global__ __launch_bounds__(EW_THREADS) void swiglu_bwd_kernel(float *__restric
                 o1[j] = x1;
                 o3[j] = x3;
             }
-            st4_nt(dh1 + 4 * i, o1);
-            st4_nt(dh3 + 4 * i, o3);
+            st4_stream<THREADS == FAR_THREADS>(dh1 + 4 * i, o1);
+            st4_stream<THREADS == FAR_THREADS>(dh3 + 4 * i, o3);
         }
     }
 }
@@ -107,14 +107,14 @@ __global__ void swiglu_bwd_scalar(float *dh1, float *dh3, const float *ds, const
 }
 
 // ---- residual family ----
-template <int MODE, int UNROLL>
-__global__ __launch_bounds__(EW_THREADS) void axpby_kernel(float *y, const float *a, const float *b, float alpha,
+template <int MODE, int UNROLL, int THREADS = EW_THREADS>
+__global__ __launch_bounds__(THREADS) void axpby_kernel(float *y, const float *a, const float *b, float alpha,
                                                            size_t n4) {
-    const size_t base = (size_t)blockIdx.x * (EW_THREADS * UNROLL) + threadIdx.x;
+    const size_t base = (size_t)blockIdx.x * (THREADS * UNROLL) + threadIdx.x;
     v4f av[UNROLL], bv[UNROLL];
 #pragma unroll
     for (int u = 0; u < UNROLL; u++) {
-        const size_t i = base + (size_t)u * EW_THREADS;
+        const size_t i = base + (size_t)u * THREADS;
         if (i < n4) {
             av[u] = ld4_nt(a + 4 * i);
             if (MODE != 1) bv[u] = ld4_nt(b + 4 * i);
@@ -122,13 +122,13 @@ __global__ __launch_bounds__(EW_THREADS) void axpby_kernel(float *y, const float
     }
 #pragma unroll
     for (int u = 0; u < UNROLL; u++) {
-        const size_t i = base + (size_t)u * EW_THREADS;
+        const size_t i = base + (size_t)u * THREADS;
         if (i < n4) {
             v4f o;
             if (MODE == 0) o = bv[u] * alpha + av[u];
             else if (MODE == 1) o = av[u] * alpha;
             else o = av[u] + bv[u];
-            st4_nt(y + 4 * i, o);
+            st4_stream<THREADS == FAR_THREADS>(y + 4 * i, o);
         }
     }
 }
@@ -493,7 +493,7 @@ __global__ __launch_bounds__(1024) void quant_dyn_one_kernel(int *__restrict__ q
     if (t == 0) ws.cnt[blk] = my_tag;
 }
 
-template <int UNROLL>
+template <int UNROLL, bool FAR = false>
 __global__ __launch_bounds__(EW_THREADS) void dequant_kernel(float *__restrict__ x, const int *__restrict__ q4,
                                                              const float *__restrict__ scale_p, size_t n4) {
     const float scale = *scale_p;
@@ -511,7 +511,8 @@ __global__ __launch_bounds__(EW_THREADS) void dequant_kernel(float *__restrict__
             v4f o;
 #pragma unroll
             for (int j = 0; j < 4; j++) o[j] = (float)(int)(signed char)((a[u] >> (8 * j)) & 0xFF) * scale;
-            st4(x + 4 * i, o);
+            if constexpr (FAR) st16_far(x + 4 * i, o);
+            else st4(x + 4 * i, o);;
         }
     }
 }
@@ -584,6 +585,12 @@ inline int pick_unroll(size_t n4, int deflt) {
         }                                                                                                  \
     } while (0)
 
+// Streams whose results go out by st16_far: large ones that start on a line, a wave to a workgroup.
+inline bool ew_far(size_t n4, int unroll, const void *out, const void *out2 = nullptr) {
+    return unroll == 1 && 16 * n4 >= FAR_BYTES && (((uintptr_t)out | (uintptr_t)out2) & 127u) == 0;
+}
+#define EW_FAR(n4) dim3((unsigned)ceil_div(n4, (size_t)FAR_THREADS)), dim3(FAR_THREADS), 0, g_ctx.stream
+
 }   // namespace
 
 // n4 vector part + scalar tail split used by every elementwise op
@@ -600,7 +607,8 @@ MI355_API int mi355_swiglu_fwd_dev(float *out, const float *h1, const float *h3,
     split_vec(n, aligned16(out) && aligned16(h1) && aligned16(h3), n4, lo);
     if (n4) {
         const int u = pick_unroll(n4, 1);
-        EW_LAUNCH(swiglu_fwd_kernel, u, n4, out, h1, h3, n4);
+        if (ew_far(n4, u, out)) hipLaunchKernelGGL((swiglu_fwd_kernel<1, FAR_THREADS>), EW_FAR(n4), out, h1, h3, n4);
+        else EW_LAUNCH(swiglu_fwd_kernel, u, n4, out, h1, h3, n4);
         LAUNCH_OK("swiglu_fwd");
     }
     if (lo < n) {
@@ -620,7 +628,8 @@ MI355_API int mi355_swiglu_bwd_dev(float *dh1, float *dh3, const float *dsilu, c
     split_vec(n, aligned16(dh1) && aligned16(dh3) && aligned16(dsilu) && aligned16(h1) && aligned16(h3), n4, lo);
     if (n4) {
         const int u = pick_unroll(n4, 1);
-        EW_LAUNCH(swiglu_bwd_kernel, u, n4, dh1, dh3, dsilu, h1, h3, n4);
+        if (ew_far(n4, u, dh1, dh3)) hipLaunchKernelGGL((swiglu_bwd_kernel<1, FAR_THREADS>), EW_FAR(n4), dh1, dh3, dsilu, h1, h3, n4);
+        else EW_LAUNCH(swiglu_bwd_kernel, u, n4, dh1, dh3, dsilu, h1, h3, n4);
         LAUNCH_OK("swiglu_bwd");
     }
     if (lo < n) {
@@ -637,7 +646,8 @@ static int axpby_run(float *y, const float *a, const float *b, float alpha, size
     split_vec(n, aligned16(y) && aligned16(a) && (MODE == 1 || aligned16(b)), n4, lo);
     if (n4) {
         const int u = pick_unroll(n4, 1);
-        switch (u) {
+        if (ew_far(n4, u, y)) hipLaunchKernelGGL((axpby_kernel<MODE, 1, FAR_THREADS>), EW_FAR(n4), y, a, b, alpha, n4);
+        else switch (u) {
             case 8: hipLaunchKernelGGL((axpby_kernel<MODE, 8>), dim3((unsigned)ceil_div(n4, (size_t)EW_THREADS * 8)), dim3(EW_THREADS), 0, g_ctx.stream, y, a, b, alpha, n4); break;
             case 4: hipLaunchKernelGGL((axpby_kernel<MODE, 4>), dim3((unsigned)ceil_div(n4, (size_t)EW_THREADS * 4)), dim3(EW_THREADS), 0, g_ctx.stream, y, a, b, alpha, n4); break;
             case 2: hipLaunchKernelGGL((axpby_kernel<MODE, 2>), dim3((unsigned)ceil_div(n4, (size_t)EW_THREADS * 2)), dim3(EW_THREADS), 0, g_ctx.stream, y, a, b, alpha, n4); break;
@@ -884,7 +894,8 @@ MI355_API int mi355_int8_dequant_dev(float *x, const int8_t *q, const float *sca
     split_vec(n, aligned16(x) && ((uintptr_t)q & 3u) == 0, n4, lo);
     if (n4) {
         const int u = pick_unroll(n4, 1);
-        EW_LAUNCH(dequant_kernel, u, n4, x, (const int *)q, scale_dev, n4);
+        if (ew_far(n4, u, x)) hipLaunchKernelGGL((dequant_kernel<1, true>), dim3((unsigned)ceil_div(n4, (size_t)EW_THREADS)), dim3(EW_THREADS), 0, g_ctx.stream, x, (const int *)q, scale_dev, n4);
+        else EW_LAUNCH(dequant_kernel, u, n4, x, (const int *)q, scale_dev, n4);
         LAUNCH_OK("int8_dequant");
     }
     if (lo < n) {

@@ -69,15 +69,15 @@ __device__ __forceinline__ void adam1(float &w, float &m, float &v, float g, flo
     w -= lr * (mh / (sqrtf(vh) + eps) + wd * w);
 }
 
-template <bool ZERO>
-__global__ __launch_bounds__(OPT_THREADS) void adam_kernel(float *__restrict__ w, float *__restrict__ g,
+template <bool ZERO, int THREADS>
+__global__ __launch_bounds__(THREADS) void adam_kernel(float *__restrict__ w, float *__restrict__ g,
                                                            float *__restrict__ m, float *__restrict__ v, size_t n,
                                                            size_t n4, float lr, float b1, float b2, float eps,
                                                            float wd, float bc1, float bc2, float scale1,
                                                            const float *__restrict__ scale2_p, bool vec) {
     const float scale2 = scale2_p ? *scale2_p : 1.0f;
     const float omb1 = 1.0f - b1, omb2 = 1.0f - b2;
-    const size_t i = (size_t)blockIdx.x * OPT_THREADS + threadIdx.x;
+    const size_t i = (size_t)blockIdx.x * THREADS + threadIdx.x;
     if (vec) {
         if (i < n4) {
             v4f wv = ld4_nt(w + 4 * i), gv = ld4_nt(g + 4 * i), mv = ld4_nt(m + 4 * i), vv = ld4_nt(v + 4 * i);
@@ -88,10 +88,10 @@ __global__ __launch_bounds__(OPT_THREADS) void adam_kernel(float *__restrict__ w
                 adam1(a, b, c, gv[j], lr, b1, b2, omb1, omb2, eps, wd, bc1, bc2);
                 wv[j] = a; mv[j] = b; vv[j] = c;
             }
-            st4_nt(w + 4 * i, wv);
-            st4_nt(m + 4 * i, mv);
-            st4_nt(v + 4 * i, vv);
-            if (ZERO) { const v4f z = {0.f, 0.f, 0.f, 0.f}; st4_nt(g + 4 * i, z); }
+            st4_stream<THREADS == FAR_THREADS>(w + 4 * i, wv);
+            st4_stream<THREADS == FAR_THREADS>(m + 4 * i, mv);
+            st4_stream<THREADS == FAR_THREADS>(v + 4 * i, vv);
+            if (ZERO) { const v4f z = {0.f, 0.f, 0.f, 0.f}; st4_stream<THREADS == FAR_THREADS>(g + 4 * i, z); }
         }
         if (blockIdx.x == 0 && threadIdx.x < n - n4 * 4) {
             const size_t k = n4 * 4 + threadIdx.x;
@@ -177,16 +177,17 @@ __global__ __launch_bounds__(OPT_THREADS) void sumsq_partial_mt_kernel(float *__
     if (threadIdx.x == 0) part[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-// Bound by its eight streams (16 B read, 16 B written per parameter with ZERO, at the 5.6 TB/s of a copy).  1024-thread
-// workgroups 705 us, plain stores 725, g read and cleared with ordinary accesses 698 (norm + clip + update, against 650).
+// Bound by its eight streams (16 B read, 16 B written per parameter with ZERO, at the 5.7 TB/s of a copy).  Norm + clip + update of
+// the 110 M parameters: 650 us in workgroups of 256 with streaming stores (of 1024 705, plain stores 725, g read and cleared with
+// ordinary accesses 698), 620 to 630 a wave to a workgroup, which alone was worth 15 to 20 of it, with stores written through.
 template <bool ZERO>
-__global__ __launch_bounds__(OPT_THREADS) void adam_mt_kernel(MtAdam a, float lr, float b1, float b2, float eps,
+__global__ __launch_bounds__(FAR_THREADS) void adam_mt_kernel(MtAdam a, float lr, float b1, float b2, float eps,
                                                               float bc1, float bc2, float scale1,
                                                               const float *__restrict__ scale2_p) {
     const unsigned block = gridDim.x - 1 - blockIdx.x;
     const int ti = mt_owner(a.blk, block);
     const size_t n = a.n[ti], n4 = n / 4;
-    const size_t i = (size_t)(block - a.blk.first[ti]) * OPT_THREADS + threadIdx.x;
+    const size_t i = (size_t)(block - a.blk.first[ti]) * FAR_THREADS + threadIdx.x;
     float *__restrict__ w = a.w[ti], *__restrict__ g = a.g[ti];
     float *__restrict__ m = a.m[ti], *__restrict__ v = a.v[ti];
     const float wd = a.wd[ti];
@@ -201,10 +202,10 @@ __global__ __launch_bounds__(OPT_THREADS) void adam_mt_kernel(MtAdam a, float lr
             adam1(x, y, z, gv[j], lr, b1, b2, omb1, omb2, eps, wd, bc1, bc2);
             wv[j] = x; mv[j] = y; vv[j] = z;
         }
-        st4_nt(w + 4 * i, wv);
-        st4_nt(m + 4 * i, mv);
-        st4_nt(v + 4 * i, vv);
-        if (ZERO) { const v4f z4 = {0.f, 0.f, 0.f, 0.f}; st4_nt(g + 4 * i, z4); }
+        st16_far(w + 4 * i, wv);
+        st16_far(m + 4 * i, mv);
+        st16_far(v + 4 * i, vv);
+        if (ZERO) { const v4f z4 = {0.f, 0.f, 0.f, 0.f}; st16_far(g + 4 * i, z4); }
     } else if (i == n4) {
         for (size_t k = 4 * n4; k < n; k++) {                    // fewer than four are left
             const float gg = (g[k] * scale1) * scale2;
@@ -214,14 +215,14 @@ __global__ __launch_bounds__(OPT_THREADS) void adam_mt_kernel(MtAdam a, float lr
     }
 }
 
-// The block table of the first tensors of a list, `per` 128-bit groups to a block (one more group where a tensor ends
-// within one): as many as one launch holds (MT_MAX, and fewer than 2^32 threads).  Returns how many; `blocks`: theirs.
-int mt_blocks(MtFirst &f, unsigned &blocks, const size_t *n, int count, size_t per) {
+// The block table of the first tensors of a list, `per` 128-bit groups to a block of `threads` (one more group where a tensor
+// ends within one): as many as one launch holds (MT_MAX, and fewer than 2^32 threads).  Returns how many; `blocks`: theirs.
+int mt_blocks(MtFirst &f, unsigned &blocks, const size_t *n, int count, size_t per, int threads) {
     size_t total = 0;
     int k = 0;
     for (; k < count && k < MT_MAX; k++) {
         const size_t more = ceil_div(ceil_div(n[k], (size_t)4), per);
-        if (total + more >= ((size_t)1 << 32) / OPT_THREADS) break;
+        if (total + more >= ((size_t)1 << 32) / threads) break;
         f.first[k] = (unsigned)total;
         total += more;
     }
@@ -249,7 +250,7 @@ MI355_API int mi355_sumsq_accum_multi_dev(float *acc_dev, const float *const *g,
     for (int i0 = 0, k = 0; i0 < count; i0 += k) {
         MtSumsq a = {};
         unsigned blocks;
-        k = mt_blocks(a.blk, blocks, n + i0, count - i0, per);
+        k = mt_blocks(a.blk, blocks, n + i0, count - i0, per, OPT_THREADS);
         if (!k) return mi355_fail("sumsq_accum_multi: tensor %d is too large for one launch", i0);
         for (int i = 0; i < k; i++) { a.g[i] = g[i0 + i]; a.n[i] = n[i0 + i]; }
         hipLaunchKernelGGL(sumsq_partial_mt_kernel, dim3(blocks), dim3(OPT_THREADS), 0, g_ctx.stream, part + done, a, pre_scale,
@@ -274,7 +275,7 @@ MI355_API int mi355_adam_update_multi_dev(float *const *w, float *const *g, floa
     for (int i0 = 0, k = 0; i0 < count; i0 += k) {
         MtAdam a = {};
         unsigned blocks;
-        k = mt_blocks(a.blk, blocks, n + i0, count - i0, OPT_THREADS);
+        k = mt_blocks(a.blk, blocks, n + i0, count - i0, FAR_THREADS, FAR_THREADS);
         if (!k) return mi355_fail("adam_update_multi: tensor %d is too large for one launch", i0);
         const dim3 grid(blocks);
         for (int i = 0; i < k; i++) {
@@ -282,10 +283,10 @@ MI355_API int mi355_adam_update_multi_dev(float *const *w, float *const *g, floa
             a.n[i] = n[i0 + i]; a.wd[i] = wd[i0 + i];
         }
         if (zero_grad)
-            hipLaunchKernelGGL((adam_mt_kernel<true>), grid, dim3(OPT_THREADS), 0, g_ctx.stream, a, lr, b1, b2, eps, bc1,
+            hipLaunchKernelGGL((adam_mt_kernel<true>), grid, dim3(FAR_THREADS), 0, g_ctx.stream, a, lr, b1, b2, eps, bc1,
                                bc2, scale1, scale2_dev);
         else
-            hipLaunchKernelGGL((adam_mt_kernel<false>), grid, dim3(OPT_THREADS), 0, g_ctx.stream, a, lr, b1, b2, eps, bc1,
+            hipLaunchKernelGGL((adam_mt_kernel<false>), grid, dim3(FAR_THREADS), 0, g_ctx.stream, a, lr, b1, b2, eps, bc1,
                                bc2, scale1, scale2_dev);
         LAUNCH_OK("adam_update_multi");
     }
@@ -329,13 +330,13 @@ MI355_API int mi355_adam_update_dev(float *w, float *g, float *m, float *v, size
     const bool vec = aligned16(w) && aligned16(g) && aligned16(m) && aligned16(v);
     const size_t n4 = vec ? n / 4 : 0;
     const size_t work = vec ? (n4 ? n4 : 1) : n;
-    const unsigned blocks = (unsigned)ceil_div(work, (size_t)OPT_THREADS);
-    if (zero_grad)
-        hipLaunchKernelGGL((adam_kernel<true>), dim3(blocks), dim3(OPT_THREADS), 0, g_ctx.stream, w, g, m, v, n, n4, lr,
-                           b1, b2, eps, wd, bc1, bc2, scale1, scale2_dev, vec);
-    else
-        hipLaunchKernelGGL((adam_kernel<false>), dim3(blocks), dim3(OPT_THREADS), 0, g_ctx.stream, w, g, m, v, n, n4, lr,
-                           b1, b2, eps, wd, bc1, bc2, scale1, scale2_dev, vec);
+    const bool far = 16 * n4 >= FAR_BYTES && (((uintptr_t)w | (uintptr_t)g | (uintptr_t)m | (uintptr_t)v) & 127u) == 0;
+#define ADAM(ZERO, T)                                                                                                \
+    hipLaunchKernelGGL((adam_kernel<ZERO, T>), dim3((unsigned)ceil_div(work, (size_t)T)), dim3(T), 0, g_ctx.stream, w, g, m, v, n, \
+                       n4, lr, b1, b2, eps, wd, bc1, bc2, scale1, scale2_dev, vec)
+    if (far) { if (zero_grad) ADAM(true, FAR_THREADS); else ADAM(false, FAR_THREADS); }
+    else { if (zero_grad) ADAM(true, OPT_THREADS); else ADAM(false, OPT_THREADS); }
+#undef ADAM
     LAUNCH_OK("adam_update");
     return 0;
 }

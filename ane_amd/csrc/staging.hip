@@ -35,6 +35,7 @@ typedef _Float16 h8_any __attribute__((ext_vector_type(8), aligned(2)));      //
 // [24576][1001] from fp16 63.0 (26.7).  Lanes are numbered in 32 bits (a launch holds no more).
 __device__ __forceinline__ size_t last_whole(size_t c, size_t n, size_t cols) { return c + n <= cols ? c : cols - n; }
 
+template <bool FAR>
 __global__ __launch_bounds__(ST_THREADS) void cvt_f32_f16_v8(_Float16 *__restrict__ dst, size_t dst_ld,
                                                              const float *__restrict__ src, size_t src_ld,
                                                              unsigned colg, size_t cols, size_t total) {
@@ -50,9 +51,11 @@ __global__ __launch_bounds__(ST_THREADS) void cvt_f32_f16_v8(_Float16 *__restric
         o[j] = (_Float16)a[j];       // round to nearest even, overflow to infinity, subnormals kept
         o[4 + j] = (_Float16)b[j];
     }
-    __builtin_nontemporal_store(o, reinterpret_cast<h8_any *>(dst + r * dst_ld + c));
+    if constexpr (FAR) st16_far(dst + r * dst_ld + c, o);
+    else __builtin_nontemporal_store(o, reinterpret_cast<h8_any *>(dst + r * dst_ld + c));
 }
 
+template <bool FAR>
 __global__ __launch_bounds__(ST_THREADS) void cvt_f16_f32_v4(float *__restrict__ dst, size_t dst_ld,
                                                              const _Float16 *__restrict__ src, size_t src_ld,
                                                              unsigned colg, size_t cols, size_t total) {
@@ -65,7 +68,7 @@ __global__ __launch_bounds__(ST_THREADS) void cvt_f16_f32_v4(float *__restrict__
 #pragma unroll
     for (int j = 0; j < 4; j++) a[j] = (float)v[j];
     float *d = dst + r * dst_ld + c;
-    st4_nt(d, a);
+    st4_stream<FAR>(d, a);
 }
 
 __global__ __launch_bounds__(ST_THREADS) void cvt_f32_f16_v1(_Float16 *__restrict__ dst, size_t dst_ld,
@@ -118,7 +121,7 @@ __device__ __forceinline__ void load_tab(float (&o)[VEC], const float *p) {
     }
 }
 
-template <int VEC>
+template <int VEC, bool FAR>
 __device__ __forceinline__ void store_cols(float *p, const float (&o)[VEC]) {
     if constexpr (VEC == 1) {
         p[0] = o[0];
@@ -126,7 +129,7 @@ __device__ __forceinline__ void store_cols(float *p, const float (&o)[VEC]) {
 #pragma unroll
         for (int q = 0; q < VEC / 4; q++) {
             v4f v = {o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]};
-            st4_nt(p + 4 * q, v);
+            st4_stream<FAR>(p + 4 * q, v);
         }
     }
 }
@@ -138,7 +141,7 @@ __device__ __forceinline__ void store_cols(float *p, const float (&o)[VEC]) {
 // against 25.2 with eight, [16][2048][250] 24.6 against 26.9 (48.1 with one).  Pair rows are numbered Q heads first, then K heads, then V heads.
 // TABLE: dQ and dK are rotated back.  WAVE: rows are whole waves of columns, so that a wave has one row and what follows of its number
 // (three divisions among it) is scalar.
-template <typename T, int VEC, bool TABLE, bool WAVE>
+template <typename T, int VEC, bool TABLE, bool WAVE, bool FAR>
 __global__ __launch_bounds__(ST_THREADS) void attn_grads_finish_kernel(
     const T *qf, const T *__restrict__ kf, const T *__restrict__ vf, int S, int hd, int heads, int kv_heads, int ratio, int batch,
     unsigned total, const float *__restrict__ cos_t, const float *__restrict__ sin_t, size_t sq, size_t sk, size_t sv, float *dq,
@@ -225,8 +228,13 @@ __global__ __launch_bounds__(ST_THREADS) void attn_grads_finish_kernel(
         for (int r = 2; r < ratio; r++) add(Col::load(in + r * head), Col::load(in + r * head + S));
         if (TABLE && is_k) turn();
     }
-    store_cols<VEC>(out, r0);
-    store_cols<VEC>(out + S, r1);
+    store_cols<VEC, FAR>(out, r0);
+    store_cols<VEC, FAR>(out + S, r1);
+}
+
+// Results that go out by st16_far: large, and every row of them whole lines.
+bool far_rows(const void *dst, size_t pitch_bytes, size_t row_bytes, size_t rows) {
+    return row_bytes * rows >= FAR_BYTES && (((uintptr_t)dst | row_bytes | (rows > 1 ? pitch_bytes : 0)) & 127u) == 0;
 }
 
 int cvt_args(const char *who, const void *dst, const void *src, size_t dst_ld, size_t src_ld, size_t rows,
@@ -249,7 +257,8 @@ MI355_API int mi355_cvt_f32_f16_dev(uint16_t *dst, size_t dst_ld, const float *s
     if (dst_ld == cols && src_ld == cols) { cols *= rows; rows = 1; }       // no gaps: one row
     if (cols >= 8) {
         const size_t colg = ceil_div(cols, (size_t)8), total = rows * colg;
-        hipLaunchKernelGGL(cvt_f32_f16_v8, dim3((unsigned)ceil_div(total, ST_THREADS)), dim3(ST_THREADS), 0,
+        auto kernel = far_rows(d, 2 * dst_ld, 2 * cols, rows) ? cvt_f32_f16_v8<true> : cvt_f32_f16_v8<false>;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)ceil_div(total, ST_THREADS)), dim3(ST_THREADS), 0,
                            g_ctx.stream, d, dst_ld, src, src_ld, (unsigned)colg, cols, total);
     } else {
         const size_t total = rows * cols;
@@ -274,8 +283,9 @@ MI355_API int mi355_cvt_f16_f32_dev(float *dst, size_t dst_ld, const uint16_t *s
             const dim3 grid((unsigned)ceil_div(total, ST_THREADS));
             float *d = dst + r0 * dst_ld + c0;
             const _Float16 *from = s + r0 * src_ld + c0;
+            auto kernel = far_rows(d, 4 * dst_ld, 4 * n, total / colg) ? cvt_f16_f32_v4<true> : cvt_f16_f32_v4<false>;
             if (n >= 4)
-                hipLaunchKernelGGL(cvt_f16_f32_v4, grid, dim3(ST_THREADS), 0, g_ctx.stream, d, dst_ld, from, src_ld,
+                hipLaunchKernelGGL(kernel, grid, dim3(ST_THREADS), 0, g_ctx.stream, d, dst_ld, from, src_ld,
                                    (unsigned)colg, n, total);
             else
                 hipLaunchKernelGGL(cvt_f16_f32_v1, grid, dim3(ST_THREADS), 0, g_ctx.stream, d, dst_ld, from, src_ld, n, total);
@@ -318,13 +328,16 @@ MI355_API int mi355_attn_grads_finish_dev(float *dq, float *dk, float *dv, const
                                dk + b * kv_full, dv + b * kv_full);
         }
     };
-#define FINISH_AS(T, VEC, WAVE)                                                                                      \
-    if (cos_dev) launch(attn_grads_finish_kernel<T, VEC, true, WAVE>, (const T *)dq_full, (const T *)dk_full, (const T *)dv_full, VEC); \
-    else launch(attn_grads_finish_kernel<T, VEC, false, WAVE>, (const T *)dq_full, (const T *)dk_full, (const T *)dv_full, VEC)
+    const bool far = far_rows(dq, 4 * (size_t)S, 4 * (size_t)S, (size_t)batch * heads * hd) &&
+                     (((uintptr_t)dk | (uintptr_t)dv) & 127u) == 0;
+#define FINISH_AS(T, VEC, ...)                                                                                       \
+    if (cos_dev) launch(attn_grads_finish_kernel<T, VEC, true, __VA_ARGS__>, (const T *)dq_full, (const T *)dk_full, (const T *)dv_full, VEC); \
+    else launch(attn_grads_finish_kernel<T, VEC, false, __VA_ARGS__>, (const T *)dq_full, (const T *)dk_full, (const T *)dv_full, VEC)
 #define FINISH(T)                                                                                                    \
-    if (S % 256 == 0) { FINISH_AS(T, 4, true); }                                                                     \
-    else if (S % 4 == 0 || (S > 4 && !in_place)) { FINISH_AS(T, 4, false); }                                         \
-    else { FINISH_AS(T, 1, false); }
+    if (S % 256 == 0 && far) { FINISH_AS(T, 4, true, true); }                                                        \
+    else if (S % 256 == 0) { FINISH_AS(T, 4, true, false); }                                                         \
+    else if (S % 4 == 0 || (S > 4 && !in_place)) { FINISH_AS(T, 4, false, false); }                                  \
+    else { FINISH_AS(T, 1, false, false); }
     if (in_f16) { FINISH(_Float16) }
     else { FINISH(float) }
 #undef FINISH_AS

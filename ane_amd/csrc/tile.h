@@ -144,13 +144,14 @@ __device__ __forceinline__ void ldb(float (&r)[VEC], const bf16_t *p) {
         r[0] = bf_to_f(*p);
     }
 }
-template <int VEC>
+template <int VEC, bool FAR = false>
 __device__ __forceinline__ void stb(bf16_t *p, const float (&r)[VEC]) {
     if constexpr (VEC == 8) {
         v4u w;
 #pragma unroll
         for (int j = 0; j < 4; j++) w[j] = f2_to_bf2(r[2 * j], r[2 * j + 1]);
-        __builtin_nontemporal_store(w, reinterpret_cast<v4u_any *>(p));
+        if constexpr (FAR) st16_far(p, w);
+        else __builtin_nontemporal_store(w, reinterpret_cast<v4u_any *>(p));
     } else {
         *p = (bf16_t)f_to_bf(r[0]);
     }
