@@ -133,9 +133,8 @@ __device__ __forceinline__ void st16_far(void *p, V v) {
     static_assert(sizeof(V) == 16, "one 128-bit access");
     asm volatile("global_store_dwordx4 %0, %1, off sc1 nt\n\ts_nop 1" : : "v"(p), "v"(v) : "memory");
 }
-template <bool FAR>
-__device__ __forceinline__ void st4_stream(float *p, v4f v) {
-    if constexpr (FAR) st16_far(p, v);
+__device__ __forceinline__ void st4_stream(float *p, v4f v, bool far) {
+    if (far) st16_far(p, v);
     else st4_nt(p, v);
 }
 

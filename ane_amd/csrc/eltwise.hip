@@ -20,14 +20,15 @@ __device__ __forceinline__ float sigmoid_ref(float h) {
 }
 
 // ---- SwiGLU forward: out = (h1*sig(h1))*h3  (mil_dynamic.h:264-266) ----
-template <int UNROLL, int THREADS = EW_THREADS>
-__global__ __launch_bounds__(THREADS) void swiglu_fwd_kernel(float *__restrict__ out, const float *__restrict__ h1,
-                                                                const float *__restrict__ h3, size_t n4) {
-    const size_t base = (size_t)blockIdx.x * (THREADS * UNROLL) + threadIdx.x;
+template <int UNROLL>
+__global__ __launch_bounds__(EW_THREADS) void swiglu_fwd_kernel(float *__restrict__ out, const float *__restrict__ h1,
+                                                                const float *__restrict__ h3, size_t n4, bool far) {
+    const unsigned threads = far ? FAR_THREADS : EW_THREADS;
+    const size_t base = (size_t)blockIdx.x * (threads * UNROLL) + threadIdx.x;
     v4f a[UNROLL], b[UNROLL];
 #pragma unroll
     for (int u = 0; u < UNROLL; u++) {
-        const size_t i = base + (size_t)u * THREADS;
+        const size_t i = base + (size_t)u * threads;
         if (i < n4) {
             a[u] = ld4_nt(h1 + 4 * i);
             b[u] = ld4_nt(h3 + 4 * i);
@@ -35,12 +36,12 @@ __global__ __launch_bounds__(THREADS) void swiglu_fwd_kernel(float *__restrict__
     }
 #pragma unroll
     for (int u = 0; u < UNROLL; u++) {
-        const size_t i = base + (size_t)u * THREADS;
+        const size_t i = base + (size_t)u * threads;
         if (i < n4) {
             v4f o;
 #pragma unroll
             for (int j = 0; j < 4; j++) o[j] = (a[u][j] * sigmoid_ref(a[u][j])) * b[u][j];
-            st4_stream<THREADS == FAR_THREADS>(out + 4 * i, o);
+            st4_stream(out + 4 * i, o, far);
         }
     }
 }
@@ -61,16 +62,17 @@ __device__ __forceinline__ void swiglu_bwd_elem(float d, float h, float g, float
     dh1 = (d * g) * u;
 }
 
-template <int UNROLL, int THREADS = EW_THREADS>
-__global__ __launch_bounds__(THREADS) void swiglu_bwd_kernel(float *__restrict__ dh1, float *__restrict__ dh3,
+template <int UNROLL>
+__global__ __launch_bounds__(EW_THREADS) void swiglu_bwd_kernel(float *__restrict__ dh1, float *__restrict__ dh3,
                                                                 const float *__restrict__ ds,
                                                                 const float *__restrict__ h1,
-                                                                const float *__restrict__ h3, size_t n4) {
-    const size_t base = (size_t)blockIdx.x * (THREADS * UNROLL) + threadIdx.x;
+                                                                const float *__restrict__ h3, size_t n4, bool far) {
+    const unsigned threads = far ? FAR_THREADS : EW_THREADS;
+    const size_t base = (size_t)blockIdx.x * (threads * UNROLL) + threadIdx.x;
     v4f a[UNROLL], b[UNROLL], d[UNROLL];
 #pragma unroll
     for (int u = 0; u < UNROLL; u++) {
-        const size_t i = base + (size_t)u * THREADS;
+        const size_t i = base + (size_t)u * threads;
         if (i < n4) {
             d[u] = ld4_nt(ds + 4 * i);
             a[u] = ld4_nt(h1 + 4 * i);
@@ -79,7 +81,7 @@ __global__ __launch_bounds__(THREADS) void swiglu_bwd_kernel(float *__restrict__
     }
 #pragma unroll
     for (int u = 0; u < UNROLL; u++) {
-        const size_t i = base + (size_t)u * THREADS;
+        const size_t i = base + (size_t)u * threads;
         if (i < n4) {
             v4f o1, o3;
 #pragma unroll
@@ -89,8 +91,8 @@ __global__ __launch_bounds__(THREADS) void swiglu_bwd_kernel(float *__restrict__
                 o1[j] = x1;
                 o3[j] = x3;
             }
-            st4_stream<THREADS == FAR_THREADS>(dh1 + 4 * i, o1);
-            st4_stream<THREADS == FAR_THREADS>(dh3 + 4 * i, o3);
+            st4_stream(dh1 + 4 * i, o1, far);
+            st4_stream(dh3 + 4 * i, o3, far);
         }
     }
 }
@@ -107,14 +109,15 @@ __global__ void swiglu_bwd_scalar(float *dh1, float *dh3, const float *ds, const
 }
 
 // ---- residual family ----
-template <int MODE, int UNROLL, int THREADS = EW_THREADS>
-__global__ __launch_bounds__(THREADS) void axpby_kernel(float *y, const float *a, const float *b, float alpha,
-                                                           size_t n4) {
-    const size_t base = (size_t)blockIdx.x * (THREADS * UNROLL) + threadIdx.x;
+template <int MODE, int UNROLL>
+__global__ __launch_bounds__(EW_THREADS) void axpby_kernel(float *y, const float *a, const float *b, float alpha,
+                                                           size_t n4, bool far) {
+    const unsigned threads = far ? FAR_THREADS : EW_THREADS;
+    const size_t base = (size_t)blockIdx.x * (threads * UNROLL) + threadIdx.x;
     v4f av[UNROLL], bv[UNROLL];
 #pragma unroll
     for (int u = 0; u < UNROLL; u++) {
-        const size_t i = base + (size_t)u * THREADS;
+        const size_t i = base + (size_t)u * threads;
         if (i < n4) {
             av[u] = ld4_nt(a + 4 * i);
             if (MODE != 1) bv[u] = ld4_nt(b + 4 * i);
@@ -122,13 +125,13 @@ __global__ __launch_bounds__(THREADS) void axpby_kernel(float *y, const float *a
     }
 #pragma unroll
     for (int u = 0; u < UNROLL; u++) {
-        const size_t i = base + (size_t)u * THREADS;
+        const size_t i = base + (size_t)u * threads;
         if (i < n4) {
             v4f o;
             if (MODE == 0) o = bv[u] * alpha + av[u];
             else if (MODE == 1) o = av[u] * alpha;
             else o = av[u] + bv[u];
-            st4_stream<THREADS == FAR_THREADS>(y + 4 * i, o);
+            st4_stream(y + 4 * i, o, far);
         }
     }
 }
@@ -493,9 +496,9 @@ __global__ __launch_bounds__(1024) void quant_dyn_one_kernel(int *__restrict__ q
     if (t == 0) ws.cnt[blk] = my_tag;
 }
 
-template <int UNROLL, bool FAR = false>
+template <int UNROLL>
 __global__ __launch_bounds__(EW_THREADS) void dequant_kernel(float *__restrict__ x, const int *__restrict__ q4,
-                                                             const float *__restrict__ scale_p, size_t n4) {
+                                                             const float *__restrict__ scale_p, size_t n4, bool far) {
     const float scale = *scale_p;
     const size_t base = (size_t)blockIdx.x * (EW_THREADS * UNROLL) + threadIdx.x;
     int a[UNROLL];
@@ -511,7 +514,7 @@ __global__ __launch_bounds__(EW_THREADS) void dequant_kernel(float *__restrict__
             v4f o;
 #pragma unroll
             for (int j = 0; j < 4; j++) o[j] = (float)(int)(signed char)((a[u] >> (8 * j)) & 0xFF) * scale;
-            if constexpr (FAR) st16_far(x + 4 * i, o);
+            if (far) st16_far(x + 4 * i, o);
             else st4(x + 4 * i, o);;
         }
     }
@@ -607,8 +610,8 @@ MI355_API int mi355_swiglu_fwd_dev(float *out, const float *h1, const float *h3,
     split_vec(n, aligned16(out) && aligned16(h1) && aligned16(h3), n4, lo);
     if (n4) {
         const int u = pick_unroll(n4, 1);
-        if (ew_far(n4, u, out)) hipLaunchKernelGGL((swiglu_fwd_kernel<1, FAR_THREADS>), EW_FAR(n4), out, h1, h3, n4);
-        else EW_LAUNCH(swiglu_fwd_kernel, u, n4, out, h1, h3, n4);
+        if (ew_far(n4, u, out)) hipLaunchKernelGGL(swiglu_fwd_kernel<1>, EW_FAR(n4), out, h1, h3, n4, true);
+        else EW_LAUNCH(swiglu_fwd_kernel, u, n4, out, h1, h3, n4, false);
         LAUNCH_OK("swiglu_fwd");
     }
     if (lo < n) {
@@ -628,8 +631,8 @@ MI355_API int mi355_swiglu_bwd_dev(float *dh1, float *dh3, const float *dsilu, c
     split_vec(n, aligned16(dh1) && aligned16(dh3) && aligned16(dsilu) && aligned16(h1) && aligned16(h3), n4, lo);
     if (n4) {
         const int u = pick_unroll(n4, 1);
-        if (ew_far(n4, u, dh1, dh3)) hipLaunchKernelGGL((swiglu_bwd_kernel<1, FAR_THREADS>), EW_FAR(n4), dh1, dh3, dsilu, h1, h3, n4);
-        else EW_LAUNCH(swiglu_bwd_kernel, u, n4, dh1, dh3, dsilu, h1, h3, n4);
+        if (ew_far(n4, u, dh1, dh3)) hipLaunchKernelGGL(swiglu_bwd_kernel<1>, EW_FAR(n4), dh1, dh3, dsilu, h1, h3, n4, true);
+        else EW_LAUNCH(swiglu_bwd_kernel, u, n4, dh1, dh3, dsilu, h1, h3, n4, false);
         LAUNCH_OK("swiglu_bwd");
     }
     if (lo < n) {
@@ -646,12 +649,12 @@ static int axpby_run(float *y, const float *a, const float *b, float alpha, size
     split_vec(n, aligned16(y) && aligned16(a) && (MODE == 1 || aligned16(b)), n4, lo);
     if (n4) {
         const int u = pick_unroll(n4, 1);
-        if (ew_far(n4, u, y)) hipLaunchKernelGGL((axpby_kernel<MODE, 1, FAR_THREADS>), EW_FAR(n4), y, a, b, alpha, n4);
+        if (ew_far(n4, u, y)) hipLaunchKernelGGL((axpby_kernel<MODE, 1>), EW_FAR(n4), y, a, b, alpha, n4, true);
         else switch (u) {
-            case 8: hipLaunchKernelGGL((axpby_kernel<MODE, 8>), dim3((unsigned)ceil_div(n4, (size_t)EW_THREADS * 8)), dim3(EW_THREADS), 0, g_ctx.stream, y, a, b, alpha, n4); break;
-            case 4: hipLaunchKernelGGL((axpby_kernel<MODE, 4>), dim3((unsigned)ceil_div(n4, (size_t)EW_THREADS * 4)), dim3(EW_THREADS), 0, g_ctx.stream, y, a, b, alpha, n4); break;
-            case 2: hipLaunchKernelGGL((axpby_kernel<MODE, 2>), dim3((unsigned)ceil_div(n4, (size_t)EW_THREADS * 2)), dim3(EW_THREADS), 0, g_ctx.stream, y, a, b, alpha, n4); break;
-            default: hipLaunchKernelGGL((axpby_kernel<MODE, 1>), dim3((unsigned)ceil_div(n4, (size_t)EW_THREADS)), dim3(EW_THREADS), 0, g_ctx.stream, y, a, b, alpha, n4); break;
+            case 8: hipLaunchKernelGGL((axpby_kernel<MODE, 8>), dim3((unsigned)ceil_div(n4, (size_t)EW_THREADS * 8)), dim3(EW_THREADS), 0, g_ctx.stream, y, a, b, alpha, n4, false); break;
+            case 4: hipLaunchKernelGGL((axpby_kernel<MODE, 4>), dim3((unsigned)ceil_div(n4, (size_t)EW_THREADS * 4)), dim3(EW_THREADS), 0, g_ctx.stream, y, a, b, alpha, n4, false); break;
+            case 2: hipLaunchKernelGGL((axpby_kernel<MODE, 2>), dim3((unsigned)ceil_div(n4, (size_t)EW_THREADS * 2)), dim3(EW_THREADS), 0, g_ctx.stream, y, a, b, alpha, n4, false); break;
+            default: hipLaunchKernelGGL((axpby_kernel<MODE, 1>), dim3((unsigned)ceil_div(n4, (size_t)EW_THREADS)), dim3(EW_THREADS), 0, g_ctx.stream, y, a, b, alpha, n4, false); break;
         }
         LAUNCH_OK("axpby");
     }
@@ -894,8 +897,7 @@ MI355_API int mi355_int8_dequant_dev(float *x, const int8_t *q, const float *sca
     split_vec(n, aligned16(x) && ((uintptr_t)q & 3u) == 0, n4, lo);
     if (n4) {
         const int u = pick_unroll(n4, 1);
-        if (ew_far(n4, u, x)) hipLaunchKernelGGL((dequant_kernel<1, true>), dim3((unsigned)ceil_div(n4, (size_t)EW_THREADS)), dim3(EW_THREADS), 0, g_ctx.stream, x, (const int *)q, scale_dev, n4);
-        else EW_LAUNCH(dequant_kernel, u, n4, x, (const int *)q, scale_dev, n4);
+        EW_LAUNCH(dequant_kernel, u, n4, x, (const int *)q, scale_dev, n4, ew_far(n4, u, x));
         LAUNCH_OK("int8_dequant");
     }
     if (lo < n) {

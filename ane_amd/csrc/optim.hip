@@ -88,10 +88,10 @@ __global__ __launch_bounds__(THREADS) void adam_kernel(float *__restrict__ w, fl
                 adam1(a, b, c, gv[j], lr, b1, b2, omb1, omb2, eps, wd, bc1, bc2);
                 wv[j] = a; mv[j] = b; vv[j] = c;
             }
-            st4_stream<THREADS == FAR_THREADS>(w + 4 * i, wv);
-            st4_stream<THREADS == FAR_THREADS>(m + 4 * i, mv);
-            st4_stream<THREADS == FAR_THREADS>(v + 4 * i, vv);
-            if (ZERO) { const v4f z = {0.f, 0.f, 0.f, 0.f}; st4_stream<THREADS == FAR_THREADS>(g + 4 * i, z); }
+            st4_stream(w + 4 * i, wv, THREADS == FAR_THREADS);
+            st4_stream(m + 4 * i, mv, THREADS == FAR_THREADS);
+            st4_stream(v + 4 * i, vv, THREADS == FAR_THREADS);
+            if (ZERO) { const v4f z = {0.f, 0.f, 0.f, 0.f}; st4_stream(g + 4 * i, z, THREADS == FAR_THREADS); }
         }
         if (blockIdx.x == 0 && threadIdx.x < n - n4 * 4) {
             const size_t k = n4 * 4 + threadIdx.x;

@@ -68,7 +68,7 @@ __global__ __launch_bounds__(ST_THREADS) void cvt_f16_f32_v4(float *__restrict__
 #pragma unroll
     for (int j = 0; j < 4; j++) a[j] = (float)v[j];
     float *d = dst + r * dst_ld + c;
-    st4_stream<FAR>(d, a);
+    st4_stream(d, a, FAR);
 }
 
 __global__ __launch_bounds__(ST_THREADS) void cvt_f32_f16_v1(_Float16 *__restrict__ dst, size_t dst_ld,
@@ -129,7 +129,7 @@ __device__ __forceinline__ void store_cols(float *p, const float (&o)[VEC]) {
 #pragma unroll
         for (int q = 0; q < VEC / 4; q++) {
             v4f v = {o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]};
-            st4_stream<FAR>(p + 4 * q, v);
+            st4_stream(p + 4 * q, v, FAR);
         }
     }
 }
