@@ -892,11 +892,14 @@ MI355_API int mi355_embed_gather_dev(float *x, const float *E, const int32_t *id
 // long in columns.  The ids are on the device, so the library learns from the previous call of the same N and D: the last
 // kernel of either form leaves its number of runs in a word of pinned host memory, and the next call compares it with the
 // number at which the two forms cost the same.  Fitted to measurements, in us:
-//   up to 16384 positions  columns 10 + 2.5 per block + 4.9 ns per pair   rows 24 + 1.4e-6 N D
-//   with the library sort  columns  5 + 1.2e-6 N D + 5.0 ns per pair      rows 54 + 2.8e-6 N D
-// (20480 to 65536 positions, D = 768 and 1024, 14 % to 97 % pairs: [1000 x 40][1024] of 151936 Zipf-distributed ids 106
-// against 175, drawn uniformly 227 against 198).  Before the first report whole sequences of up to 16384 positions take
-// the columns, everything else the rows.  The row form reports distinct tokens, not pairs; how many pairs a token makes
+//   up to 16384 positions  columns 10 + 3.8 per block + 3.6 ns per pair   rows 23 + 1.75e-6 N D
+//   with the library sort  columns of K < 4 are ahead by 56 + 1.6e-6 N D - 5.0 ns per pair, of K = 4 (whole 16-byte pieces of dE) by
+//                          52 + 1.9e-6 N D - 3.3 ns per pair
+// (2048 to 65536 positions, D = 512, 768 and 1024, 14 % to 97 % pairs, 63 inputs; columns / rows, us: 16384 x 768, 4624 pairs of Zipf-
+// distributed ids 37 / 50, 7003 drawn uniformly 42 / 43, 8915 48 / 44; 8192 x 768, 5916 pairs 34 / 35; 12288 x 512, 3618 26 / 39, 9437
+// 38 / 34; 40000 x 1024, 13531 93 / 167, 38929 176 / 185; 32768 x 768, 17876 90 / 99, 23706 144 / 100.)  Before the first report
+// whole sequences of up to 16384 positions take the columns, everything else the rows.  The row form reports distinct tokens, not
+// pairs; how many pairs a token makes
 // is taken from the last time both forms saw this shape (1.2 until then), so that a steady input settles on one form
 // instead of alternating.
 namespace {
@@ -944,8 +947,9 @@ int scatter_form(int N, int D, bool cols_ok, bool whole, bool rows_recordable) {
     if (form == 0 || rN != N || rD != D) return unknown;
     const int nblk = (int)ceil_div((size_t)N, CB);
     const double nd = (double)N * D;
-    const double even = rows_recordable ? std::max((14.0 - 2.5 * nblk + 1.4e-6 * nd) / 4.9e-3, 0.30 * N)
-                                        : (49.0 + 1.6e-6 * nd) / 5.0e-3;
+    const double even = rows_recordable ? std::max((13.0 - 3.8 * nblk + 1.75e-6 * nd) / 3.6e-3, 0.30 * N)
+                        : cols_per_workgroup(D) < 4 ? (56.0 + 1.6e-6 * nd) / 5.0e-3
+                                                    : (52.0 + 1.9e-6 * nd) / 3.3e-3;
     if (form == 1) {
         g_cols_runs = runs; g_cols_N = N; g_cols_D = D;
         return runs <= 1.08 * even ? 1 : -1;

@@ -11,12 +11,11 @@
 // acc += x[rank] for the ranks ascending; dE = acc.  Blocks in ascending order and ranks ascending within a run are
 // the order of the reference loop, so the result is that loop's bit for bit.
 //
-// Three launches (one, col_sum_small_kernel, up to 512 positions):
-//   1. chunk_sort_blk_kernel: every 256 consecutive (token, position-in-block) words sorted by counting.
-//   2. block_rank_kernel: the sorted chunks of a block merged by rank (16 lanes per one or two positions, a binary search per
-//      chunk): rk[position] = its rank within the block, and the block's runs {token, first rank, length}, long runs
-//      listed from the front of the block's task array, short ones from its back.
-//   3. col_sum_kernel<K>: per block, every thread writes its values of dx (fetched into registers while the previous
+// Two launches (one, col_sum_small_kernel, up to 512 positions):
+//   1. block_plan_kernel: 32 or 64 workgroups to a block, each with the tokens of one hash value: rk[position] = its rank within
+//      the block, and the block's runs {token, first rank, length}, long runs listed from the front of the block's task
+//      array, short ones from its back.
+//   2. col_sum_kernel<K>: per block, every thread writes its values of dx (fetched into registers while the previous
 //      block was summed) to LDS at their ranks, so that a run is a contiguous piece of an LDS column.  Waves 0..K-1
 //      take the long runs of one column each (128-bit LDS reads issued sixteen adds ahead); the other waves take the
 //      short runs, K columns to a lane, the old sums of a lane's runs asked for before the block's values are put in
@@ -27,159 +26,179 @@
 #pragma once
 
 constexpr int CB = 8192, CB_BITS = 13;      // positions per block
-constexpr int CB_CHUNKS = CB / CHUNK;       // sorted chunks per block
-constexpr int CB_CPL = CB_CHUNKS / 16;      // chunks searched by one lane
 constexpr int COL_LONG = 16;                // runs of at least this many positions go to the long-run waves
 constexpr int COL_CARRY = 256;              // entries of the token-indexed table that carries long runs' sums to the next block
-constexpr int RANK_ONE = 32768;             // up to here block_rank_kernel ranks 64 positions per workgroup: two on each of 256 compute units
 constexpr int COL_PPT = CB / 1024;          // positions of a block per thread
-static_assert(CB_CPL >= 1 && COL_PPT % 4 == 0, "block size");
+static_assert(COL_PPT % 4 == 0 && CB / 16 / 64 == 8, "values of dx come by fours; a wave of a plan has eight times 64 ids");
 
 typedef unsigned v2u __attribute__((ext_vector_type(2)));
 
-__device__ __forceinline__ unsigned pack_word_blk(const int32_t *__restrict__ ids, int i, int N, int V) {
-    unsigned key = (unsigned)V;                             // padding and out-of-range ids sort last
-    if (i < N) {
-        const int id = ids[i];
-        if (id >= 0 && id < V) key = (unsigned)id;
-    }
-    return (key << CB_BITS) | (unsigned)(i & (CB - 1));
+constexpr int PLAN_WORKGROUPS = 256;        // of a plan, over its blocks
+constexpr int PLAN_BLOCKS = 64;             // blocks of one pair of launches; more positions are taken in several
+
+// The numbers of long (low word) and short runs of a block, a line to a block.  Two that take turns: a plan counts in one, which the
+// plan before it has cleared, and clears the other.  Whose turn it is is the last bit of plan_turn, which the sums move on, and which
+// a block's sums find beside the counts; so nothing is cleared by a launch of its own and a recorded graph can be replayed.
+struct __attribute__((aligned(128))) PlanCount {
+    unsigned long long runs[2];
+    unsigned turn;
+};
+__device__ unsigned plan_turn;
+__device__ PlanCount plan_count[PLAN_BLOCKS];
+
+// v summed over groups of 2^sh adjacent lanes (sh <= 4, the same for all lanes); every lane ends with its group's sum
+__device__ __forceinline__ int lanes_sum(int v, int sh) {
+    if (sh >= 1) v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, true);      // quad_perm:[1,0,3,2]
+    if (sh >= 2) v += __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, true);      // quad_perm:[2,3,0,1]
+    if (sh >= 3) v += __builtin_amdgcn_update_dpp(0, v, 0x141, 0xF, 0xF, true);     // half of a row mirrored
+    if (sh >= 4) v += __builtin_amdgcn_update_dpp(0, v, 0x140, 0xF, 0xF, true);     // a row mirrored
+    return v;
 }
 
-__global__ __launch_bounds__(CHUNK) void chunk_sort_blk_kernel(unsigned *__restrict__ sorted_chunks,
-                                                               unsigned long long *__restrict__ cnt, int nblk,
-                                                               const int32_t *__restrict__ ids, int N, int V) {
-    __shared__ __attribute__((aligned(16))) unsigned sw[CHUNK];
-    const int t = threadIdx.x;
-    if (blockIdx.x == 0)
-        for (int i = t; i < nblk; i += CHUNK) cnt[i] = 0ull;
-    const unsigned w = pack_word_blk(ids, blockIdx.x * CHUNK + t, N, V);
-    sw[t] = w;
+// Workgroup (block, g) of `groups` to a block ranks the positions whose token falls into group g; ids outside [0, V) count as token V,
+// which no run is listed for.  It reads all ids of the block, 512 to a wave: how many fall into the groups before g is its first
+// rank; a wave's own go to its list in order of position.  Of 64 of the list the wave finds the equal ones (a comparison with each of the
+// first FEW tokens, then a ballot per bit of the others): every distinct token of the 64 is one entry {token, which 64, how many}, and the
+// entries (50 to 120, also where one token has a thousand positions) are ranked against all others by counting, 1024 lanes at a time.
+// What the sum of the smaller entries' positions is does not depend on their order in LDS.
+// Bound by its chain of barriers and trips to memory, no part of which grows with the text; two workgroups fit a compute unit.  In
+// place of a launch that sorted chunks of 256 and one that merged them by binary search, us by the trace: 16384 positions of text 12.4,
+// now 6.9; 40000 15.3, 7.8 (of which, by the clock: 1 to start and load, 0.6 for the groups, 0.8 for the equal ones, 1.5 for the entries, 1 for the
+// counts).  `groups`: as many workgroups as compute units, 128 to a block at most (the first version, in 64 and 32: 7.8 and 9.3).
+__global__ __launch_bounds__(1024) void block_plan_kernel(uint16_t *__restrict__ rk, v2u *__restrict__ tasks,
+                                                          const int32_t *__restrict__ ids, int N, int V, int key_bits, int groups) {
+    constexpr int PER_WAVE = CB / 16, FEW = 12;
+    __shared__ __attribute__((aligned(16))) unsigned ent[CB];
+    __shared__ unsigned list[CB];                               // PER_WAVE to a wave
+    __shared__ uint16_t first_of[1024];
+    __shared__ __attribute__((aligned(16))) int wave_less[16];
+    __shared__ int n_ent, n_long, n_short, base_long, base_short;
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int blk = blockIdx.x / (unsigned)groups;
+    const unsigned g = blockIdx.x - blk * groups;
+    const int p0 = blk * CB + wave * PER_WAVE + lane;
+    int id[PER_WAVE / 64];
+#pragma unroll
+    for (int j = 0; j < PER_WAVE / 64; j++) id[j] = ids[min(p0 + 64 * j, N - 1)];
+    const unsigned turn = plan_turn;
+    if (blockIdx.x == 0 && t < PLAN_BLOCKS) plan_count[t].runs[(turn + 1) & 1] = 0ull;
+    if (g == 0 && t == 0) plan_count[blk].turn = turn;
+    if (t == 0) n_ent = n_long = n_short = 0;
+    const v4u none = {~0u, ~0u, ~0u, ~0u};                      // behind the entries: not below any
+    *reinterpret_cast<v4u *>(&ent[4 * t]) = none;
+    *reinterpret_cast<v4u *>(&ent[CB / 2 + 4 * t]) = none;
     __syncthreads();
-    int r = 0;
-#pragma unroll 8
-    for (int j = 0; j < CHUNK; j += 4) {
-        const v4u q = *reinterpret_cast<const v4u *>(&sw[j]);
-        r += (q.x < w ? 1 : 0) + (q.y < w ? 1 : 0) + (q.z < w ? 1 : 0) + (q.w < w ? 1 : 0);
-    }
-    sorted_chunks[blockIdx.x * CHUNK + r] = w;
-}
 
-// One workgroup = 64*P consecutive positions of one block, 16 lanes per position, one chunk of the block per lane.
-// rk[position] = its rank within its block.
-// tasks[block][...] = {token, start | length << 16}; cnt[block] = number of long runs (low word) and of short runs.
-// A workgroup's time is the fill of its LDS and a chain of searches, whatever P is; two fit a compute unit.  With P = 1 a launch
-// of 625 is a round and a fifth: 40000 positions 15.0 us, with P = 2 10.7 (the whole call 102.6 -> 98.3); 16384 positions
-// take as long with either, 5796 and 10240 1 us longer with P = 2.
-template <int P>
-__global__ __launch_bounds__(1024) void block_rank_kernel(uint16_t *__restrict__ rk, v2u *__restrict__ tasks,
-                                                          unsigned long long *__restrict__ cnt,
-                                                          const unsigned *__restrict__ sorted_chunks,
-                                                          const int32_t *__restrict__ ids, int N, int V, int nchunks) {
-    __shared__ unsigned sc[CB_CHUNKS * CHUNK_PITCH];
-    __shared__ int n_long, n_short, base_long, base_short;
-    static_assert(CB % (64 * P) == 0, "a workgroup's positions lie in one block");
-    const int t = threadIdx.x;
-    const int n0 = blockIdx.x * (64 * P), blk = n0 >> CB_BITS, c0 = blk * CB_CHUNKS;
+    unsigned *mine = list + wave * PER_WAVE;
+    int n = 0, less = 0;                                        // positions of this wave in group g, and in the groups before it
+    const bool whole = (blk + 1) * CB <= N;
 #pragma unroll
-    for (int i = 0; i < CB / 4096; i++) {
-        const int j = i * 4096 + 4 * t;
-        const v4u q = (c0 + j / CHUNK < nchunks) ? *reinterpret_cast<const v4u *>(&sorted_chunks[(size_t)c0 * CHUNK + j])
-                                                 : v4u{0, 0, 0, 0};
-        unsigned *dst = sc + (j / CHUNK) * CHUNK_PITCH + (j % CHUNK);
-        dst[0] = q.x; dst[1] = q.y; dst[2] = q.z; dst[3] = q.w;
+    for (int j = 0; j < PER_WAVE / 64; j++) {
+        const unsigned key = min((unsigned)id[j], (unsigned)V);
+        // 16 bits of a product of 24-bit factors, scaled to the number of groups
+        unsigned h = (__umul24(__umul24(key, 0x9E3779u) >> 8 & 0xffffu, groups)) >> 16;
+        if (!whole && p0 + 64 * j >= N) h = ~0u;
+        const unsigned long long owns = __builtin_amdgcn_ballot_w64(h == g);
+        if (h == g) mine[n + __builtin_amdgcn_mbcnt_hi((unsigned)(owns >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)owns, 0u))] =
+            key << CB_BITS | (unsigned)(wave * PER_WAVE + 64 * j + lane);
+        n += __builtin_popcountll(owns);
+        less += __builtin_popcountll(__builtin_amdgcn_ballot_w64(h < g));
     }
-    const int k = t & 15, tl = t >> 4;
-    unsigned w[P];
-#pragma unroll
-    for (int u = 0; u < P; u++) w[u] = pack_word_blk(ids, n0 + tl + 64 * u, N, V);
-    if (t == 0) n_long = n_short = 0;
-    __syncthreads();
-    // a lane's chunks: k, k + 16, ...; one past the end is searched as chunk 0 and not counted.  The searches of a
-    // lane are independent chains of LDS reads and run interleaved.
-    const unsigned *chp[CB_CPL];
-    bool okc[CB_CPL];
-#pragma unroll
-    for (int m = 0; m < CB_CPL; m++) {
-        okc[m] = c0 + k + 16 * m < nchunks;
-        chp[m] = sc + (okc[m] ? k + 16 * m : 0) * CHUNK_PITCH;
-    }
-    auto count_below = [&](const unsigned (&x)[P], int (&p)[P][CB_CPL]) {       // per chunk: number of words < x
-#pragma unroll
-        for (int u = 0; u < P; u++)
-#pragma unroll
-            for (int m = 0; m < CB_CPL; m++) p[u][m] = 0;
-#pragma unroll
-        for (int st = CHUNK / 2; st >= 1; st >>= 1) {
-#pragma unroll
-            for (int u = 0; u < P; u++)
-#pragma unroll
-                for (int m = 0; m < CB_CPL; m++)
-                    if (chp[m][p[u][m] + st - 1] < x[u]) p[u][m] += st;
+    if (lane == 0) wave_less[wave] = less;
+    for (int c = 0; 64 * c < n; c++) {                          // (a wave's own list: its writes are in order with its reads)
+        const int i = 64 * c + lane;
+        const bool live = i < n;
+        const unsigned w = live ? mine[i] : 0u, k = w >> CB_BITS;
+        unsigned long long same = 0, rest = __builtin_amdgcn_ballot_w64(live);
+        const unsigned long long all = rest;
+        for (int j = 0; j < FEW && rest; j++) {                 // the first tokens one by one: a frequent one is among them
+            const unsigned kj = __builtin_amdgcn_readlane(k, __builtin_ctzll(rest));
+            const unsigned long long m = __builtin_amdgcn_ballot_w64(k == kj) & all;
+            same = k == kj ? m : same;
+            rest &= ~m;
         }
-#pragma unroll
-        for (int u = 0; u < P; u++)
-#pragma unroll
-            for (int m = 0; m < CB_CPL; m++) p[u][m] += chp[m][p[u][m]] < x[u] ? 1 : 0;
-    };
-    int p[P][CB_CPL], below[P], upto[P], idx[P];
-    unsigned pred1[P], next[P];                                 // pred1: largest smaller word + 1, or 0 if there is none
-    bool first[P], any_first = false;
-    count_below(w, p);
-#pragma unroll
-    for (int u = 0; u < P; u++) {
-        below[u] = 0;
-        pred1[u] = 0;
-#pragma unroll
-        for (int m = 0; m < CB_CPL; m++)
-            if (okc[m]) {
-                below[u] += p[u][m];
-                if (p[u][m] > 0) pred1[u] = max(pred1[u], chp[m][p[u][m] - 1] + 1u);
+        if (rest) {
+            unsigned long long eq = rest;
+            for (int b = 0; b < key_bits; b++) {
+                const unsigned long long ones = __builtin_amdgcn_ballot_w64((k >> b & 1u) != 0);
+                const unsigned one = (unsigned)((int)(k << (31 - b)) >> 31);            // all ones where the bit is set
+                const unsigned lo = (unsigned)eq & ~((unsigned)ones ^ one), hi = (unsigned)(eq >> 32) & ~((unsigned)(ones >> 32) ^ one);
+                eq = (unsigned long long)hi << 32 | lo;
             }
-#pragma unroll
-        for (int m = 1; m < 16; m <<= 1) {
-            below[u] += __shfl_xor(below[u], m, 64);
-            pred1[u] = max(pred1[u], (unsigned)__shfl_xor((int)pred1[u], m, 64));
+            if (rest >> lane & 1ull) same = eq;
         }
-        const unsigned key = w[u] >> CB_BITS;
-        first[u] = n0 + tl + 64 * u < N && key < (unsigned)V && (pred1[u] == 0 || ((pred1[u] - 1u) >> CB_BITS) != key);
-        next[u] = (key + 1u) << CB_BITS;                        // no overflow where first: key < V < 2^(32 - CB_BITS)
-        any_first |= first[u];
-        upto[u] = 0;
-    }
-    if (any_first) {                                            // uniform over the 16 lanes of the positions
-        count_below(next, p);
-#pragma unroll
-        for (int u = 0; u < P; u++) {
-#pragma unroll
-            for (int m = 0; m < CB_CPL; m++) upto[u] += okc[m] ? p[u][m] : 0;
-#pragma unroll
-            for (int m = 1; m < 16; m <<= 1) upto[u] += __shfl_xor(upto[u], m, 64);
+        const int idx = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(same >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)same, 0u));
+        const bool head = live && idx == 0;
+        const unsigned long long heads = __builtin_amdgcn_ballot_w64(head);
+        int e0 = 0;
+        if (lane == 0) e0 = atomicAdd(&n_ent, __builtin_popcountll(heads));
+        e0 = __builtin_amdgcn_readfirstlane(e0);
+        if (live) {
+            const int e = e0 + __builtin_popcountll(heads & ((same & -same) - 1ull));       // (the heads ahead of its own)
+            if (head) ent[e] = k << CB_BITS | (unsigned)(8 * wave + c) << 6 | (unsigned)(__builtin_popcountll(same) - 1);
+            mine[i] = (w & (CB - 1)) | (unsigned)idx << CB_BITS | (unsigned)e << (CB_BITS + 6);
         }
-    }
-    const auto is_long = [&](int u) { return upto[u] - below[u] >= COL_LONG; };
-#pragma unroll
-    for (int u = 0; u < P; u++) {
-        if (k == 0 && first[u]) idx[u] = atomicAdd(is_long(u) ? &n_long : &n_short, 1);
-        if (k == 0 && n0 + tl + 64 * u < N) rk[n0 + tl + 64 * u] = (uint16_t)below[u];
     }
     __syncthreads();
-    if (t == 0) {
-        unsigned long long old = 0;
-        if (n_long | n_short)
-            old = atomicAdd(&cnt[blk], ((unsigned long long)(unsigned)n_short << 32) | (unsigned)n_long);
-        base_long = (int)(old & 0xffffffffu);
-        base_short = (int)(old >> 32);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < P; u++)
-        if (k == 0 && first[u]) {
-            const v2u entry = {w[u] >> CB_BITS, (unsigned)below[u] | ((unsigned)(upto[u] - below[u]) << 16)};
-            tasks[(size_t)blk * CB + (is_long(u) ? base_long + idx[u] : CB - 1 - (base_short + idx[u]))] = entry;
-        }
-}
 
+    const int ne = n_ent;
+    const int sh = ne <= 64 ? 4 : ne <= 128 ? 3 : ne <= 256 ? 2 : ne <= 512 ? 1 : 0;       // 2^sh lanes to an entry
+    for (int e1 = 0; e1 < ne; e1 += 1024 >> sh) {
+        const int e = e1 + (t >> sh), part = t & ((1 << sh) - 1);
+        const unsigned w = ent[min(e, CB - 1)], lo = w & ~(CB - 1u), hi = lo + CB;
+        int s = 0, upto = 0;                                    // positions of the entries below, and of those up to the token's last
+        bool again = false;                                     // the token has an entry below
+        if (e < ne)                                             // (the same for the lanes of an entry)
+            for (int j = 4 * part; j < ne; j += 4 << sh) {
+                const v4u x = *reinterpret_cast<const v4u *>(&ent[j]);
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const int m = (int)(x[u] & 63u) + 1;
+                    s += x[u] < w ? m : 0;
+                    upto += x[u] < hi ? m : 0;
+                    again |= x[u] < w && x[u] >= lo;
+                }
+            }
+        s = lanes_sum(s, sh);
+        upto = lanes_sum(upto, sh);
+        const bool mine_e = e < ne && part == 0, run = lanes_sum(again, sh) == 0 && mine_e && w >> CB_BITS < (unsigned)V;
+        const bool is_long = run && upto - s >= COL_LONG;
+        if (mine_e) first_of[e - e1] = (uint16_t)s;
+        const unsigned long long longs = __builtin_amdgcn_ballot_w64(is_long), shorts = __builtin_amdgcn_ballot_w64(run && !is_long);
+        int il = 0, is = 0;
+        if (lane == 0 && longs) il = atomicAdd(&n_long, __builtin_popcountll(longs));
+        if (lane == 0 && shorts) is = atomicAdd(&n_short, __builtin_popcountll(shorts));
+        __syncthreads();
+        // the place in the block's lists is a trip to memory; the ranks are written meanwhile
+        unsigned long long old = 0;
+        if (t == 0 && (n_long | n_short))
+            old = atomicAdd(&plan_count[blk].runs[turn & 1], (unsigned long long)(unsigned)n_short << 32 | (unsigned)n_long);
+        int rank0 = 0;
+#pragma unroll
+        for (int v = 0; v < 16; v++) rank0 += wave_less[v];
+        for (int i = lane; i < n; i += 64) {
+            const unsigned x = mine[i];
+            const int ex = (int)(x >> (CB_BITS + 6)) - e1;
+            if (ex >= 0 && ex < 1024 >> sh)
+                rk[(size_t)blk * CB + (x & (CB - 1))] = (uint16_t)(rank0 + first_of[ex] + (x >> CB_BITS & 63u));
+        }
+        if (t == 0) {
+            base_long = (int)(old & 0xffffffffu);
+            base_short = (int)(old >> 32);
+            n_long = n_short = 0;
+        }
+        __syncthreads();
+        il = __builtin_amdgcn_readfirstlane(il);
+        is = __builtin_amdgcn_readfirstlane(is);
+        if (run) {
+            const unsigned long long below = (1ull << lane) - 1ull;
+            const int slot = is_long ? base_long + il + __builtin_popcountll(longs & below)
+                                     : CB - 1 - (base_short + is + __builtin_popcountll(shorts & below));
+            const v2u entry = {w >> CB_BITS, (unsigned)(rank0 + s) | (unsigned)(upto - s) << 16};
+            tasks[(size_t)blk * CB + slot] = entry;
+        }
+    }
+}
 
 // acc + x[start] + x[start+1] + ... + x[start+len-1], in that order, from one LDS column.  The column is read in
 // aligned groups of eight; what lies outside the run in the first and in the last groups is replaced by -0, which
@@ -240,8 +259,7 @@ struct __attribute__((packed, aligned(4))) ColVec { float f[K]; };
 template <int K, bool FULL, bool ANY>
 __global__ __launch_bounds__(1024) void col_sum_kernel(float *dE, const float *__restrict__ dx,
                                                        const v2u *__restrict__ tasks,
-                                                       const unsigned long long *__restrict__ cnt,
-                                                       const uint16_t *__restrict__ rk, int N, int D, int S, int nblk,
+                                                       const uint16_t *__restrict__ rk, int first, int N, int D, int S, int nblk,
                                                        unsigned long long *report) {
     constexpr int XP = CB + 48;                                 // a column in LDS, with room for the reads issued ahead
     constexpr int NSL = (16 - K) * 64;                          // lanes that take short runs
@@ -263,14 +281,17 @@ __global__ __launch_bounds__(1024) void col_sum_kernel(float *dE, const float *_
         v2u pd[RPL];
     };
     Pre o;
+    unsigned turn;
     auto fetch_runs = [&](Pre &o, int blk) __attribute__((always_inline)) {
         const v2u *tb = tasks + (size_t)blk * CB;
-        o.pc = cnt[blk];
+        const PlanCount c = plan_count[blk];
+        turn = c.turn;
+        o.pc = turn & 1 ? c.runs[1] : c.runs[0];
 #pragma unroll
         for (int i = 0; i < RPL; i++) o.pd[i] = tb[hot ? lane + 64 * i : CB - 1 - (sl + NSL * i)];
     };
     auto fetch_values = [&](Pre &o, int blk) __attribute__((always_inline)) {
-        const int p0 = blk * CB + COL_PPT * t;
+        const int p0 = first + blk * CB + COL_PPT * t;
 #pragma unroll
         for (int q = 0; q < COL_PPT / 4; q++) {
             const int p = p0 + 4 * q < N ? p0 + 4 * q : 0;       // (past the end: any address; the values are not used)
@@ -362,7 +383,7 @@ __global__ __launch_bounds__(1024) void col_sum_kernel(float *dE, const float *_
 #pragma unroll
         for (int q = 0; q < COL_PPT; q++) {
             const int r = (o.prk[q / 2] >> (16 * (q & 1))) & 0xffff;
-            if (blk * CB + COL_PPT * t + q < N) {
+            if (first + blk * CB + COL_PPT * t + q < N) {
 #pragma unroll
                 for (int d = 0; d < K; d++) xs[d][r] = o.px[d][q / 4][q & 3];
             }
@@ -444,6 +465,7 @@ __global__ __launch_bounds__(1024) void col_sum_kernel(float *dE, const float *_
         }
     }
     // what the host looks at before it picks a form for the next call of this shape (one 8-byte store to host memory)
+    if (blockIdx.x == 0 && t == 0) plan_turn = turn + 1;
     if (report && blockIdx.x == 0 && t == 0) *report = scatter_report(runs, N, D, 1);
 }
 
@@ -552,36 +574,30 @@ int scatter_add_cols(float *dE, const float *dx, const int32_t *ids, int V, int 
         LAUNCH_OK("embed_scatter_add column sums");
         return 0;
     }
-    const int nchunks = (int)ceil_div((size_t)N, CHUNK), nblk = (int)ceil_div((size_t)N, CB);
+    constexpr int MOST = PLAN_BLOCKS * CB;
+    const int most_blocks = (int)ceil_div((size_t)std::min(N, MOST), CB);
     size_t total = 0;
     auto take = [&total](size_t bytes) {
         const size_t off = total;
         total += (bytes + 255) & ~(size_t)255;
         return off;
     };
-    const size_t off_chunks = take((size_t)nchunks * CHUNK * sizeof(unsigned));
-    const size_t off_cnt = take((size_t)nblk * sizeof(unsigned long long));
-    const size_t off_rk = take((size_t)nblk * CB * sizeof(uint16_t));
-    const size_t off_tasks = take((size_t)nblk * CB * sizeof(v2u));
+    const size_t off_rk = take((size_t)most_blocks * CB * sizeof(uint16_t));
+    const size_t off_tasks = take((size_t)most_blocks * CB * sizeof(v2u));
     char *ws = (char *)mi355_ws(total);
     if (!ws) return -1;
-    unsigned *sorted_chunks = (unsigned *)(ws + off_chunks);
-    unsigned long long *cnt = (unsigned long long *)(ws + off_cnt);
     uint16_t *rk = (uint16_t *)(ws + off_rk);
     v2u *tasks = (v2u *)(ws + off_tasks);
-    hipLaunchKernelGGL(chunk_sort_blk_kernel, dim3(nchunks), dim3(CHUNK), 0, g_ctx.stream, sorted_chunks, cnt, nblk, ids,
-                       N, V);
-    auto rank = [&](auto kernel, int per) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned)ceil_div((size_t)N, (size_t)per)), dim3(1024), 0, g_ctx.stream, rk, tasks, cnt,
-                           sorted_chunks, ids, N, V, nchunks);
-    };
-    if (N <= RANK_ONE) rank(block_rank_kernel<1>, 64);
-    else rank(block_rank_kernel<2>, 128);
-    LAUNCH_OK("embed_scatter_add plan");
     const bool any = S % 4 != 0 || !aligned16(dx);
-    auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, grid, dim3(1024), 0, g_ctx.stream, dE, dx, tasks, cnt, rk, N, D, S, nblk, report);
-    };
+    for (int first = 0; first < N; first += std::min(MOST, N - first)) {
+        const int n = std::min(MOST, N - first), nblk = (int)ceil_div((size_t)n, CB);
+        const int groups = std::max(16, std::min(128, PLAN_WORKGROUPS / nblk));
+        hipLaunchKernelGGL(block_plan_kernel, dim3(nblk * groups), dim3(1024), 0, g_ctx.stream, rk, tasks, ids + first, n, V,
+                           32 - __builtin_clz((unsigned)V), groups);
+        LAUNCH_OK("embed_scatter_add plan");
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, dim3(1024), 0, g_ctx.stream, dE, dx, tasks, rk, first, N, D, S, nblk, report);
+        };
 #define COL_LAUNCH(KK)                                                     \
     case KK:                                                               \
         if (D % KK == 0 && !any) launch(col_sum_kernel<KK, true, false>);  \
@@ -589,11 +605,12 @@ int scatter_add_cols(float *dE, const float *dx, const int32_t *ids, int V, int 
         else if (!any) launch(col_sum_kernel<KK, false, false>);           \
         else launch(col_sum_kernel<KK, false, true>);                      \
         break;
-    switch (K) {
-        COL_LAUNCH(1) COL_LAUNCH(2) COL_LAUNCH(3) COL_LAUNCH(4)
-    default: return mi355_fail("embed_scatter_add: no kernel for %d columns per workgroup", K);
-    }
+        switch (K) {
+            COL_LAUNCH(1) COL_LAUNCH(2) COL_LAUNCH(3) COL_LAUNCH(4)
+        default: return mi355_fail("embed_scatter_add: no kernel for %d columns per workgroup", K);
+        }
 #undef COL_LAUNCH
-    LAUNCH_OK("embed_scatter_add column sums");
+        LAUNCH_OK("embed_scatter_add column sums");
+    }
     return 0;
 }

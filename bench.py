@@ -51,10 +51,10 @@ OP_KERNELS = {
     "int8_dequant": [("dequant_kernel<1>", 1.0)],
     "int8_quantize_dynamic": [("quant_dyn_one_kernel<4>", 1.0)],
 }
-# the three launches of the ordered scatter-add in its column form and in its row form, and
+# the launches of the ordered scatter-add in its column form and in its row form, and
 # the gather
 EMBED_KERNELS = {
-    "scatter_cols": [("chunk_sort_blk_kernel", 1.0), ("block_rank_kernel<1>", 1.0), ("col_sum_kernel<3, true, false>", 1.0)],
+    "scatter_cols": [("block_plan_kernel", 1.0), ("col_sum_kernel<3, true, false>", 1.0)],
     "scatter_rows": [("chunk_sort_kernel", 1.0), ("rank_transpose_kernel", 1.0), ("seg_sum_kernel<false>", 1.0)],
     "gather": [("gather_kernel<true, 64, 64, true>", 1.0)],
 }
