@@ -461,9 +461,8 @@ int sgemm_piece(int ta, int tb, int M, int N, int K, float alpha, const float *A
     if (p.split >= 2) {
         const int units = plane_cols(N) * psteps;               // (P_MAX_BYTES keeps it small)
         inexact = (int *)(planes + (size_t)units * P_UNIT);
-        const dim3 grid((unsigned)ceil_div((size_t)units, 4));
-        if (tb) hipLaunchKernelGGL(split_planes_kernel<true>, grid, dim3(256), 0, g_ctx.stream, planes, inexact, B, ldb, N, K, psteps, units);
-        else hipLaunchKernelGGL(split_planes_kernel<false>, grid, dim3(256), 0, g_ctx.stream, planes, inexact, B, ldb, N, K, psteps, units);
+        if (tb) hipLaunchKernelGGL(split_planes_kernel<true>, dim3(units), dim3(64), 0, g_ctx.stream, planes, inexact, B, ldb, N, K, psteps);
+        else hipLaunchKernelGGL(split_planes_kernel<false>, dim3(units), dim3(64), 0, g_ctx.stream, planes, inexact, B, ldb, N, K, psteps);
         LAUNCH_OK("sgemm planes");
     }
     auto launch_planes = [&](auto kernel) {
