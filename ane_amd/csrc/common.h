@@ -74,6 +74,9 @@ bool mi355_exchange(Mi355Exchange *out);
 int mi355_exchange_spin_ticks(void);
 // Device address of the expired-wait counter of the one-launch cross-entropy (softmax_ce.hip), NULL before init.
 int *mi355_ce_fallbacks_dev(void);
+// adam_update_dev from arrays (16-byte aligned) to others, the gradient as it is (optim.hip).
+int mi355_adam_between(float *w_out, float *m_out, float *v_out, const float *w, const float *g, const float *m, const float *v, size_t n,
+                       int t, float lr, float b1, float b2, float eps, float wd);
 // Runs every queued weight-gradient reduction (dw_reduce.hip).
 extern "C" int mi355_dw_flush(void);
 

@@ -7,7 +7,7 @@
 //   embed_lookup / embed_backward    training/stories_cpu_ops.h:112-131
 //   rope_backward_inplace            training/training_dynamic/cpu_ops.h:168-184
 // Failures print one "mi355_bridge: ..." line and leave arrays that are updated in place untouched, and all others unless it was
-// the copy back that failed.
+// the copy back that failed, or a later chunk of an elementwise call.
 #include "common.h"
 
 #include <emmintrin.h>
@@ -100,6 +100,15 @@ void host_written_from(const void *p, const void *dev_src, size_t bytes) {
             continue;
         g_tab[i].dirty = true;
     }
+}
+
+// Whether a resident table holds some of the host range [p, p+bytes).
+bool in_a_table(const void *p, size_t bytes) {
+    for (int i = 0; i < g_tab_n; i++) {
+        const char *t = (const char *)g_tab[i].host;
+        if ((const char *)p < t + (size_t)g_tab[i].V * g_tab[i].D * sizeof(float) && t < (const char *)p + bytes) return true;
+    }
+    return false;
 }
 
 // The device copy of the host table `embed` [vocab][dim], uploaded if new or stale.  NULL on failure.
@@ -262,6 +271,7 @@ MI355_API void mi355_swiglu_bwd(float *dh1, float *dh3, const float *dsilu, cons
     const size_t nb = n * sizeof(float);
     Stage st;
     const int id = st.in(dsilu, nb), i1 = st.in(h1, nb), i3 = st.in(h3, nb), o1 = st.out(dh1, nb), o3 = st.out(dh3, nb);
+    if (st.stream(n, [&](float **x, float **y, size_t k) { return mi355_swiglu_bwd_dev(y[o1], y[o3], x[id], x[i1], x[i3], k); })) return;
     if (!st.send()) return;
     if (!ran(mi355_swiglu_bwd_dev(st.dev<float>(o1), st.dev<float>(o3), st.dev<float>(id), st.dev<float>(i1), st.dev<float>(i3), n))) return;
     st.receive();
@@ -274,6 +284,7 @@ MI355_API void mi355_swiglu_fwd(float *out, const float *h1, const float *h3, si
     const size_t nb = n * sizeof(float);
     Stage st;
     const int i1 = st.in(h1, nb), i3 = st.in(h3, nb), io = st.out(out, nb);
+    if (st.stream(n, [&](float **x, float **y, size_t k) { return mi355_swiglu_fwd_dev(y[io], x[i1], x[i3], k); })) return;
     if (!st.send()) return;
     if (!ran(mi355_swiglu_fwd_dev(st.dev<float>(io), st.dev<float>(i1), st.dev<float>(i3), n))) return;
     st.receive();
@@ -287,6 +298,8 @@ MI355_API void mi355_axpby(float *y, const float *a, const float *b, float alpha
     const size_t nb = n * sizeof(float);
     Stage st;
     const int ia = st.in(a, nb), ib = mode != 1 ? st.in(b, nb) : -1, iy = st.out(y, nb);
+    if (st.stream(n, [&](float **p, float **r, size_t k) { return mi355_axpby_dev(r[iy], p[ia], mode != 1 ? p[ib] : nullptr, alpha, k, mode); }))
+        return;
     if (!st.send()) return;
     if (!ran(mi355_axpby_dev(st.dev<float>(iy), st.dev<float>(ia), mode != 1 ? st.dev<float>(ib) : nullptr, alpha, n, mode))) return;
     st.receive();
@@ -300,6 +313,10 @@ MI355_API void mi355_adam_update(float *w, const float *g, float *m, float *v, s
     const size_t nb = n * sizeof(float);
     Stage st;
     const int ig = st.in(g, nb), iw = st.inout(w, nb), im = st.inout(m, nb), iv = st.inout(v, nb);
+    if (!in_a_table(w, nb) && st.stream(n, [&](float **x, float **y, size_t k) {
+            return mi355_adam_between(y[iw], y[im], y[iv], x[iw], x[ig], x[im], x[iv], k, t, lr, b1, b2, eps, wd);
+        }))
+        return;
     if (!st.send()) return;
     if (!ran(mi355_adam_update_dev(st.dev<float>(iw), st.dev<float>(ig), st.dev<float>(im), st.dev<float>(iv), n, t, lr, b1, b2, eps, wd,
                                    1.0f, nullptr, 0)))

@@ -25,7 +25,7 @@
 constexpr int HELPERS = 3;
 constexpr size_t PIECE = (size_t)64 << 10;
 constexpr size_t PIN_MAX = (size_t)32 << 20;         // bytes of a pinned block at most; longer transfers go in rounds of this
-constexpr int MAX_PIECES = (int)(PIN_MAX / PIECE) + 64;
+constexpr int MAX_PIECES = 2 * (int)(PIN_MAX / PIECE) + 256;
 constexpr size_t SEND_MIN = (size_t)256 << 10, SEND_MAX = (size_t)4 << 20;
 constexpr int MAX_SENDS = 32;                        // copies of a round
 
@@ -83,6 +83,7 @@ struct Piece {
     const Part *part;
     size_t from, bytes;
     char *block;
+    bool in, past;                       // to the block or back; past the caches
 };
 
 enum : unsigned char { TO_DO, PACKED, DONE };       // PACKED: may be sent, the log is still to come
@@ -102,7 +103,6 @@ struct Helpers {
     std::atomic<unsigned long long> next;
     std::atomic<int> ready;
     std::atomic<int> active;              // between the start of a round and its end
-    bool in, past;
     Piece piece[MAX_PIECES];
     std::atomic<unsigned char> done[MAX_PIECES];
 };
@@ -117,8 +117,8 @@ bool one_piece(Helpers *h) {
     }
     const int i = (int)(n & 0xffffffffu);
     const Piece &p = h->piece[i];
-    move_part(*p.part, p.from, p.bytes, p.block, h->in, h->past);
-    if (h->in && p.part->log) {
+    move_part(*p.part, p.from, p.bytes, p.block, p.in, p.past);
+    if (p.in && p.part->log) {
         h->done[i].store(PACKED, std::memory_order_release);
         move_part(*p.part, p.from, p.bytes, p.part->log + p.from, true, true);
     }
@@ -127,12 +127,10 @@ bool one_piece(Helpers *h) {
 }
 
 // The pieces 0 .. pieces - 1 become a round, of which the first `ready` may be taken; the round's number.
-unsigned long long start_pieces(Helpers *h, int pieces, int ready, bool in, bool past) {
+unsigned long long start_pieces(Helpers *h, int pieces, int ready) {
     // no helper may still be looking at the round before
     const unsigned long long number = (h->next.load(std::memory_order_relaxed) >> 32) + 1;
     h->ready.store(0, std::memory_order_seq_cst);
-    h->in = in;
-    h->past = past;
     h->next.store(number << 32, std::memory_order_seq_cst);
     h->ready.store(ready, std::memory_order_seq_cst);
     if (pieces > 4 && h->n > 0) {
@@ -334,6 +332,140 @@ public:
         return false;
     }
 
+    // Elementwise calls on parts of n floats: the arrays go through in chunks of values, and the kernel of a chunk reads the pinned block
+    // of the inputs and writes that of the results itself, one launch in the place of a copy, the operation and a copy; what has come
+    // back is unpacked while later chunks are packed and travel.  chunk(in, out, count): in[i], out[i] are the addresses of
+    // part i's values; 0 if it was launched.  Longer arrays than a block holds go in rounds.
+    // 1: done.  0: nothing has been done (no pinned memory, or arrays that overlap other than value by value); the call takes
+    // the other way.  -1: failed; the parts that are inputs and results are as before the call.
+    // us, by way of the device / so: Adam step of [2048][768] 968 / 887, of [3072][1024] 2030 / 1800, SwiGLU backward of [2048][256] 281 /
+    // 252, forward 187 / 171, axpby of [768][256] 92 / 82.  Bound by the link, whose 57 GB/s are those of both directions together (two
+    // copies of 64 MB, one each way, take as long at once as one after the other), and by 7 us between the kernels of two chunks.
+    template <typename F>
+    int stream(size_t n, const F &chunk) {
+        int ins = 0;
+        size_t updated = 0;
+        for (int i = 0; i < n_; i++) {
+            if (p_[i].rows || p_[i].bytes != n * sizeof(float)) return 0;
+            ins += in_[i];
+            if (in_[i] && out_[i]) updated += p_[i].bytes;
+            for (int j = 0; j < n_; j++) {
+                if (i == j || !out_[j]) continue;
+                const char *a = p_[i].host, *b = p_[j].host;
+                if (a == b ? out_[i] : a < b + p_[j].bytes && b < a + p_[i].bytes) return 0;
+            }
+        }
+        Helpers *h = helpers();
+        if (!h) return 0;
+        const size_t most = PIN_MAX / (sizeof(float) * n_) & ~(size_t)4095;
+        const size_t len = std::min(most, (n + 63) & ~(size_t)63), stride = len * sizeof(float);     // values of a round
+        if (!pinned(g_pin, stride * n_) || !pinned(g_pin_back, stride * n_)) return 0;
+        const bool logged = updated && len < n;
+        if (logged) {
+            char *log = log_space(updated);
+            if (!log) return -1;
+            for (int i = 0; i < n_; i++)
+                if (in_[i] && out_[i]) {
+                    p_[i].log = log;
+                    log += p_[i].bytes;
+                }
+        }
+        copies_ = 0;
+        for (size_t r0 = 0; r0 < n; r0 += len) {
+            const size_t cnt = std::min(len, n - r0);
+            // the ends of the chunks: they grow, and shrink again
+            size_t cut[MAX_SENDS];
+            int sends = 0;
+            const size_t least = SEND_MIN / sizeof(float) / ins, largest = SEND_MAX / sizeof(float) / ins;
+            for (size_t at = 0, c = least; at < cnt; sends++) {
+                at += std::min(std::min(c, largest), std::max(least, (cnt - at) / 2)) & ~(size_t)1023;
+                c *= 2;
+                if (at > cnt || sends + 1 == MAX_SENDS) at = cnt;
+                cut[sends] = at;
+            }
+            // the pieces in the order in which they are taken: a chunk's results LAG chunks behind its inputs
+            constexpr int LAG = 2;
+            int pieces = 0, packed[MAX_SENDS], last[MAX_SENDS], back_from[MAX_SENDS];       // first and last + 1 to pack, first to unpack
+            auto add_pieces = [&](int s, bool in) {
+                const size_t from = s ? cut[s - 1] : 0;
+                for (int i = 0; i < n_; i++) {
+                    if (!(in ? in_[i] : out_[i])) continue;
+                    for (size_t at = from * sizeof(float); at < cut[s] * sizeof(float); at += PIECE) {
+                        h->done[pieces].store(TO_DO, std::memory_order_relaxed);
+                        h->piece[pieces++] = Piece{&p_[i], r0 * sizeof(float) + at, std::min(cut[s] * sizeof(float) - at, PIECE),
+                                                   (in ? g_pin.host : g_pin_back.host) + i * stride + at, in, in || p_[i].bytes > (size_t)1 << 20};
+                    }
+                }
+            };
+            for (int s = 0; s < sends + LAG; s++) {
+                if (s < sends) {
+                    packed[s] = pieces;
+                    add_pieces(s, true);
+                    last[s] = pieces;
+                }
+                if (s >= LAG) {
+                    back_from[s - LAG] = pieces;
+                    add_pieces(s - LAG, false);
+                }
+            }
+            const unsigned long long number = start_pieces(h, pieces, back_from[0]);
+            hipError_t e = hipSuccess;
+            int rc = 0, sent = 0, come = 0, ok = 0;
+            while (come < sends && e == hipSuccess && rc == 0) {
+                bool idle = true;
+                if (sent < sends) {
+                    ok = std::max(ok, packed[sent]);
+                    // (an array's old values are in the log before any of it is written again)
+                    while (ok < last[sent]) {
+                        const unsigned char d = h->done[ok].load(std::memory_order_acquire);
+                        if (d == TO_DO || (logged && d != DONE)) break;
+                        ok++;
+                    }
+                    if (ok == last[sent]) {
+                        const size_t from = sent ? cut[sent - 1] : 0;
+                        float *in[MAX], *out[MAX];
+                        for (int i = 0; i < n_; i++) {
+                            in[i] = (float *)(g_pin.dev + i * stride) + from;
+                            out[i] = (float *)(g_pin_back.dev + i * stride) + from;
+                        }
+                        rc = chunk(in, out, cut[sent] - from);
+                        if (rc == 0) e = hipEventRecord(g_sent[sent], g_ctx.stream);
+                        sent++;
+                        idle = false;
+                    }
+                }
+                if (e == hipSuccess && come < sent) {
+                    const hipError_t q = hipEventQuery(g_sent[come]);
+                    if (q == hipErrorNotReady) {
+                        (void)hipGetLastError();
+                    } else {
+                        e = back(q);
+                        if (e == hipSuccess) {
+                            come++;
+                            h->ready.store(come < sends ? back_from[come] : pieces, std::memory_order_release);
+                        }
+                        idle = false;
+                    }
+                }
+                if (idle && !one_piece(h)) __builtin_ia32_pause();
+            }
+            const bool good = e == hipSuccess && rc == 0;
+            end_pieces(h, pieces, number, good);
+            if (good) continue;
+            if (e != hipSuccess) fail("D2H", e);
+            else (void)hipStreamSynchronize(g_ctx.stream);
+            const size_t written = (r0 + (come ? cut[come - 1] : 0)) * sizeof(float);
+            for (int i = 0; i < n_; i++)
+                if (in_[i] && out_[i]) {
+                    Part p = p_[i];
+                    p.bytes = written;
+                    unpack(h, p, logged ? p.log : g_pin.host + i * stride);
+                }
+            return -1;
+        }
+        return 1;
+    }
+
 private:
     static constexpr int MAX = 8;
     Part p_[MAX];
@@ -388,9 +520,9 @@ private:
             int pieces = 0;
             for (; pieces < MAX_PIECES && at < p.bytes; at += PIECE) {
                 h->done[pieces].store(TO_DO, std::memory_order_relaxed);
-                h->piece[pieces++] = Piece{&p, at, std::min(p.bytes - at, PIECE), from + at};
+                h->piece[pieces++] = Piece{&p, at, std::min(p.bytes - at, PIECE), from + at, false, true};
             }
-            end_pieces(h, pieces, start_pieces(h, pieces, pieces, false, true), true);
+            end_pieces(h, pieces, start_pieces(h, pieces, pieces), true);
         }
     }
 
@@ -412,6 +544,7 @@ private:
             if (at > end || sends + 1 == MAX_SENDS) at = end;
             cut[sends] = at;
         }
+        const bool past = in || end - beg > (size_t)1 << 20;        // (small results stay in the caches for their reader)
         // the pieces, none across the end of a copy; last[s]: pieces up to the end of copy s
         int pieces = 0, last[MAX_SENDS], s = 0;
         for (int i = 0; i < n_; i++) {
@@ -422,13 +555,12 @@ private:
                 while (at >= cut[s]) last[s++] = pieces;
                 const size_t n = std::min(std::min(stop, cut[s]) - at, PIECE);
                 h->done[pieces].store(TO_DO, std::memory_order_relaxed);
-                h->piece[pieces++] = Piece{&p_[i], at - p_[i].at, n, pin.host + (at - beg)};
+                h->piece[pieces++] = Piece{&p_[i], at - p_[i].at, n, pin.host + (at - beg), in, past};
                 at += n;
             }
         }
         while (s < sends) last[s++] = pieces;
-        // (small results stay in the caches for their reader)
-        const unsigned long long number = start_pieces(h, pieces, in ? pieces : 0, in, in || end - beg > (size_t)1 << 20);
+        const unsigned long long number = start_pieces(h, pieces, in ? pieces : 0);
         hipError_t e = hipSuccess;
         if (in) {
             int ok = 0;

@@ -106,6 +106,35 @@ __global__ __launch_bounds__(THREADS) void adam_kernel(float *__restrict__ w, fl
     }
 }
 
+// The same update from arrays to others: from the pinned block of a call on host arrays to that of its results, over the link (stream()
+// in host_stage.h has the times).
+__global__ __launch_bounds__(OPT_THREADS) void adam_between_kernel(float *__restrict__ wo, float *__restrict__ mo, float *__restrict__ vo,
+                                                                   const float *__restrict__ w, const float *__restrict__ g,
+                                                                   const float *__restrict__ m, const float *__restrict__ v, size_t n,
+                                                                   size_t n4, float lr, float b1, float b2, float eps, float wd,
+                                                                   float bc1, float bc2) {
+    const float omb1 = 1.0f - b1, omb2 = 1.0f - b2;
+    const size_t i = (size_t)blockIdx.x * OPT_THREADS + threadIdx.x;
+    if (i < n4) {
+        v4f wv = ld4_nt(w + 4 * i), gv = ld4_nt(g + 4 * i), mv = ld4_nt(m + 4 * i), vv = ld4_nt(v + 4 * i);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            float a = wv[j], b = mv[j], c = vv[j];
+            adam1(a, b, c, gv[j], lr, b1, b2, omb1, omb2, eps, wd, bc1, bc2);
+            wv[j] = a; mv[j] = b; vv[j] = c;
+        }
+        st4_nt(wo + 4 * i, wv);
+        st4_nt(mo + 4 * i, mv);
+        st4_nt(vo + 4 * i, vv);
+    }
+    if (blockIdx.x == 0 && threadIdx.x < n - n4 * 4) {
+        const size_t k = n4 * 4 + threadIdx.x;
+        float a = w[k], b = m[k], c = v[k];
+        adam1(a, b, c, g[k], lr, b1, b2, omb1, omb2, eps, wd, bc1, bc2);
+        wo[k] = a; mo[k] = b; vo[k] = c;
+    }
+}
+
 // ---- many tensors per launch ----
 // The blocks of all tensors of a launch are numbered through: tensor i owns the blocks first[i] .. first[i + 1] - 1.
 // A grid of (blocks of the largest tensor) x (tensors) is mostly empty workgroups where sizes differ: the 110 M
@@ -337,6 +366,16 @@ MI355_API int mi355_adam_update_dev(float *w, float *g, float *m, float *v, size
     if (far) { if (zero_grad) ADAM(true, FAR_THREADS); else ADAM(false, FAR_THREADS); }
     else { if (zero_grad) ADAM(true, OPT_THREADS); else ADAM(false, OPT_THREADS); }
 #undef ADAM
+    LAUNCH_OK("adam_update");
+    return 0;
+}
+
+int mi355_adam_between(float *wo, float *mo, float *vo, const float *w, const float *g, const float *m, const float *v, size_t n, int t,
+                       float lr, float b1, float b2, float eps, float wd) {
+    const float bc1 = 1.0f - powf(b1, (float)t), bc2 = 1.0f - powf(b2, (float)t);
+    const size_t n4 = n / 4, blocks = std::max<size_t>(ceil_div(n4, (size_t)OPT_THREADS), 1);
+    hipLaunchKernelGGL(adam_between_kernel, dim3((unsigned)blocks), dim3(OPT_THREADS), 0, g_ctx.stream, wo, mo, vo, w, g, m, v, n, n4, lr,
+                       b1, b2, eps, wd, bc1, bc2);
     LAUNCH_OK("adam_update");
     return 0;
 }

@@ -1,0 +1,90 @@
+"""Elementwise calls on host arrays, whose chunks are packed, computed over the link and unpacked at the same time: sizes at the ends of
+chunks (16384, 21504, 32768 values ...) and of a round, results over their own inputs, arrays that overlap otherwise or lie
+in a resident table (which take the other way), and what lies beside the arrays.  The bytes are those of the device call."""
+import numpy as np
+import pytest
+
+import helpers as H
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def br():
+    import ane_amd.bridge as b
+    b.init()
+    return b
+
+
+def guarded(n):
+    buf = np.full(n + 2, 3.0, np.float32)
+    return buf[1:-1], lambda: buf[0] == 3.0 and buf[-1] == 3.0
+
+
+def on_device(br, name, outs, ins, *rest):
+    o, i = [br.DevArray(ins[0].size) for _ in range(outs)], [br.DevArray.from_numpy(x) for x in ins]
+    br.check(getattr(br.lib, name)(*[x.ptr for x in o + i], *rest))
+    return [x.numpy() for x in o]
+
+
+SIZES = [1, 3, 1023, 16384, 21504, 32769, 65536 + 1024, 131071, 700001, (2 << 20) + 1, (2796202 & ~4095) + 1]
+
+
+@pytest.mark.parametrize("n", SIZES)
+def test_results_in_arrays_of_their_own(br, n):
+    print("[case] host stream n=%d" % n, flush=True)
+    a, b, c = H.normal(960, n), H.normal(961, n), H.normal(962, n)
+    p = lambda x: x.ctypes.data
+    (y, y_ok), (z, z_ok) = guarded(n), guarded(n)
+    br.lib.mi355_swiglu_fwd(p(y), p(a), p(b), n)
+    assert y.tobytes() == on_device(br, "mi355_swiglu_fwd_dev", 1, [a, b], n)[0].tobytes() and y_ok()
+    br.lib.mi355_swiglu_bwd(p(y), p(z), p(a), p(b), p(c), n)
+    want = on_device(br, "mi355_swiglu_bwd_dev", 2, [a, b, c], n)
+    assert y.tobytes() == want[0].tobytes() and z.tobytes() == want[1].tobytes() and y_ok() and z_ok()
+    for mode in range(3):
+        br.lib.mi355_axpby(p(y), p(a), p(b), 0.3, n, mode)
+        assert y.tobytes() == on_device(br, "mi355_axpby_dev", 1, [a, b], 0.3, n, mode)[0].tobytes() and y_ok()
+
+
+@pytest.mark.parametrize("n", SIZES)
+def test_adam(br, n):
+    print("[case] host stream adam n=%d" % n, flush=True)
+    arrays = [guarded(n) for _ in range(4)]
+    for k, (x, _) in enumerate(arrays):
+        x[...] = H.normal(970 + k, n)
+    arrays[3][0][...] **= 2
+    dev = [br.DevArray.from_numpy(x) for x, _ in arrays]
+    rest = (n, 7, 3e-4, 0.9, 0.95, 1e-8, 0.1)
+    br.check(br.lib.mi355_adam_update_dev(*[d.ptr for d in dev], *rest, 1.0, None, 0))
+    br.lib.mi355_adam_update(*[x.ctypes.data for x, _ in arrays], *rest)
+    for (x, ok), d in zip(arrays, dev):
+        assert x.tobytes() == d.numpy().tobytes() and ok()
+
+
+@pytest.mark.parametrize("shift", [0, 1, -1, 40000, -40000])
+def test_results_over_inputs(br, shift):
+    """y = 0.3 b + a with y `shift` values behind a or b: every input is read before any result is written"""
+    n = 300007
+    for over in (0, 1):
+        buf = H.normal(980, n + 80000)
+        x, other = buf[40000:40000 + n], H.normal(981, n)
+        y = buf[40000 + shift:40000 + shift + n]
+        a, b = (x, other) if over == 0 else (other, x)
+        want = b * np.float32(0.3) + a
+        br.lib.mi355_axpby(y.ctypes.data, a.ctypes.data, b.ctypes.data, 0.3, n, 0)
+        assert y.tobytes() == want.tobytes()
+
+
+def test_weights_that_a_table_holds(br):
+    """the table that an update steps is looked up on the device afterwards, with the values that the update left"""
+    V, D, S = 300, 64, 50
+    w, g, m, v = H.normal(990, (V, D)), H.normal(991, (V, D)), H.normal(992, (V, D)), H.normal(993, (V, D)) ** 2
+    tok = np.random.default_rng(994).integers(0, V, S).astype(np.uint16)
+    x = np.zeros((D, S), np.float32)
+    for _ in range(2):
+        br.lib.mi355_embed_lookup(x.ctypes.data, w.ctypes.data, tok.ctypes.data, V, D, S)
+        assert x.tobytes() == np.ascontiguousarray(w[tok].T).tobytes()
+        br.lib.mi355_adam_update(w.ctypes.data, g.ctypes.data, m.ctypes.data, v.ctypes.data, V * D, 3, 3e-4, 0.9, 0.95, 1e-8, 0.1)
+    br.lib.mi355_embed_lookup(x.ctypes.data, w.ctypes.data, tok.ctypes.data, V, D, S)
+    assert x.tobytes() == np.ascontiguousarray(w[tok].T).tobytes()
+    br.lib.mi355_host_table_invalidate(w.ctypes.data)
