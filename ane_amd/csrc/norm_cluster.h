@@ -337,6 +337,13 @@ __global__ __launch_bounds__(THREADS) void rms_fwd_cluster_kernel(const typename
     float total = 0.f, rr[VEC];
     const bool met = cluster_totals<THREADS, 1, VEC>(acc, lds, g.blk, g.first, g.member, csplit, slots, tags, spin_ticks, total);
     auto scale = [&](float ss) { return 1.0f / sqrtf(ss * invC + eps); };
+    if constexpr (FUSE) {
+        // the residual goes out while the waves that hold the column sums wait for their partners' (no member that would have to read
+        // its rows again finds them overwritten: calls in place take other kernels): odd layer of [8][768][197] 64.4 -> 63.8 us
+#pragma unroll
+        for (int k = 0; k < RPT; k++)
+            if (EXACT || row_ok(g.member, k)) ST::store_nt(y_res + slab_base + (size_t)row_of(g.member, k) * S, xr[k]);
+    }
     if (threadIdx.x < W) {
         col_rr[threadIdx.x] = scale(total);
         if (!met) failed = 1;
@@ -376,7 +383,6 @@ __global__ __launch_bounds__(THREADS) void rms_fwd_cluster_kernel(const typename
     for (int k = 0; k < RPT; k++) {
         if (EXACT || row_ok(g.member, k)) {
             const size_t off = slab_base + (size_t)row_of(g.member, k) * S;
-            if constexpr (FUSE) ST::store_nt(y_res + off, xr[k]);
             float xv[VEC], o[VEC];
             ST::widen(xv, xr[k]);
 #pragma unroll
