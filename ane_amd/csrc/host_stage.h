@@ -337,7 +337,7 @@ public:
     // back is unpacked while later chunks are packed and travel.  chunk(in, out, count): in[i], out[i] are the addresses of
     // part i's values; 0 if it was launched.  Longer arrays than a block holds go in rounds.
     // 1: done.  0: nothing has been done (no pinned memory, or arrays that overlap other than value by value); the call takes
-    // the other way.  -1: failed; the parts that are inputs and results are as before the call.
+    // the other way.  -1: failed; the arrays that are inputs and results, of one part or of two, are as before the call.
     // us, by way of the device / so: Adam step of [2048][768] 968 / 887, of [3072][1024] 2030 / 1800, SwiGLU backward of [2048][256] 281 /
     // 252, forward 187 / 171, axpby of [768][256] 92 / 82.  Bound by the link, whose 57 GB/s are those of both directions together (two
     // copies of 64 MB, one each way, take as long at once as one after the other), and by 7 us between the kernels of two chunks.
@@ -345,15 +345,18 @@ public:
     int stream(size_t n, const F &chunk) {
         int ins = 0;
         size_t updated = 0;
+        bool old[MAX];                    // inputs that results are written over
         for (int i = 0; i < n_; i++) {
             if (p_[i].rows || p_[i].bytes != n * sizeof(float)) return 0;
             ins += in_[i];
-            if (in_[i] && out_[i]) updated += p_[i].bytes;
+            old[i] = in_[i] && out_[i];
             for (int j = 0; j < n_; j++) {
                 if (i == j || !out_[j]) continue;
                 const char *a = p_[i].host, *b = p_[j].host;
                 if (a == b ? out_[i] : a < b + p_[j].bytes && b < a + p_[i].bytes) return 0;
+                old[i] |= a == b;
             }
+            if (old[i]) updated += p_[i].bytes;
         }
         Helpers *h = helpers();
         if (!h) return 0;
@@ -365,7 +368,7 @@ public:
             char *log = log_space(updated);
             if (!log) return -1;
             for (int i = 0; i < n_; i++)
-                if (in_[i] && out_[i]) {
+                if (old[i]) {
                     p_[i].log = log;
                     log += p_[i].bytes;
                 }
@@ -456,7 +459,7 @@ public:
             else (void)hipStreamSynchronize(g_ctx.stream);
             const size_t written = (r0 + (come ? cut[come - 1] : 0)) * sizeof(float);
             for (int i = 0; i < n_; i++)
-                if (in_[i] && out_[i]) {
+                if (old[i]) {
                     Part p = p_[i];
                     p.bytes = written;
                     unpack(h, p, logged ? p.log : g_pin.host + i * stride);

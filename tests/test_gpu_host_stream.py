@@ -75,6 +75,22 @@ def test_results_over_inputs(br, shift):
         assert y.tobytes() == want.tobytes()
 
 
+@pytest.mark.parametrize("n", [300007, (3 << 20) + 5])       # several chunks of one round, two rounds
+@pytest.mark.parametrize("fail", [1, 2, 4])
+def test_results_over_inputs_stay_when_a_chunk_does_not_come_back(br, n, fail):
+    x, other, h1, h3 = H.normal(985, n), H.normal(986, n), H.normal(987, n), H.normal(988, n)
+    was = [a.copy() for a in (x, h1, h3)]
+    p = lambda a: a.ctypes.data
+    try:
+        br.tune("host_stage_fail", fail)
+        br.lib.mi355_axpby(p(x), p(x), p(other), 0.3, n, 0)
+        br.lib.mi355_swiglu_bwd(p(h1), p(h3), p(other), p(h1), p(h3), n)
+    finally:
+        br.tune("host_stage_fail", 0)
+    for a, b in zip((x, h1, h3), was):
+        assert a.tobytes() == b.tobytes()
+
+
 def test_weights_that_a_table_holds(br):
     """the table that an update steps is looked up on the device afterwards, with the values that the update left"""
     V, D, S = 300, 64, 50
