@@ -12,7 +12,7 @@
 // the order of the reference loop, so the result is that loop's bit for bit.
 //
 // Two launches (one, col_sum_small_kernel, up to 512 positions):
-//   1. block_plan_kernel: 32 or 64 workgroups to a block, each with the tokens of one hash value: rk[position] = its rank within
+//   1. block_plan_kernel: 16 to 128 workgroups to a block, each with the tokens of one hash value: rk[position] = its rank within
 //      the block, and the block's runs {token, first rank, length}, long runs listed from the front of the block's task
 //      array, short ones from its back.
 //   2. col_sum_kernel<K>: per block, every thread writes its values of dx (fetched into registers while the previous
