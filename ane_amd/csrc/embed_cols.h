@@ -36,14 +36,15 @@ typedef unsigned v2u __attribute__((ext_vector_type(2)));
 constexpr int PLAN_WORKGROUPS = 256;        // of a plan, over its blocks
 constexpr int PLAN_BLOCKS = 64;             // blocks of one pair of launches; more positions are taken in several
 
-// The numbers of long (low word) and short runs of a block, a line to a block.  Two that take turns: a plan counts in one, which the
-// plan before it has cleared, and clears the other.  Whose turn it is is the last bit of plan_turn, which the sums move on, and which
-// a block's sums find beside the counts; so nothing is cleared by a launch of its own and a recorded graph can be replayed.
+// The numbers of long (bits 0 to 15) and short runs (from bit 32) of a block, a line to a block.  Two that take turns: a plan counts in
+// one, which the plan before it has cleared, and clears the other.  Bits 16 to 31 count the workgroups that have come with their first
+// runs, and the last of them, which all the others have read `turn` before, moves it on.  So nothing is cleared by a launch of
+// its own, a recorded graph can be replayed, and a plan leaves a cleared count to the next one whether or not its sums are
+// launched (with the turn moved on by the sums, a call that ended between the two left its runs to be counted on top of).
 struct __attribute__((aligned(128))) PlanCount {
     unsigned long long runs[2];
     unsigned turn;
 };
-__device__ unsigned plan_turn;
 __device__ PlanCount plan_count[PLAN_BLOCKS];
 
 // v summed over groups of 2^sh adjacent lanes (sh <= 4, the same for all lanes); every lane ends with its group's sum
@@ -80,9 +81,8 @@ __global__ __launch_bounds__(1024) void block_plan_kernel(uint16_t *__restrict__
     int id[PER_WAVE / 64];
 #pragma unroll
     for (int j = 0; j < PER_WAVE / 64; j++) id[j] = ids[min(p0 + 64 * j, N - 1)];
-    const unsigned turn = plan_turn;
-    if (blockIdx.x == 0 && t < PLAN_BLOCKS) plan_count[t].runs[(turn + 1) & 1] = 0ull;
-    if (g == 0 && t == 0) plan_count[blk].turn = turn;
+    // (an atomic load: it stands where it is, ahead of the counting)
+    const unsigned turn = __hip_atomic_load(&plan_count[blk].turn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     if (t == 0) n_ent = n_long = n_short = 0;
     const v4u none = {~0u, ~0u, ~0u, ~0u};                      // behind the entries: not below any
     *reinterpret_cast<v4u *>(&ent[4 * t]) = none;
@@ -141,9 +141,11 @@ __global__ __launch_bounds__(1024) void block_plan_kernel(uint16_t *__restrict__
     }
     __syncthreads();
 
+    if (g == 0 && t == 0) plan_count[blk].runs[(turn + 1) & 1] = 0ull;
     const int ne = n_ent;
     const int sh = ne <= 64 ? 4 : ne <= 128 ? 3 : ne <= 256 ? 2 : ne <= 512 ? 1 : 0;       // 2^sh lanes to an entry
-    for (int e1 = 0; e1 < ne; e1 += 1024 >> sh) {
+    int e1 = 0;
+    do {                                                        // (also without an entry: every workgroup counts itself)
         const int e = e1 + (t >> sh), part = t & ((1 << sh) - 1);
         const unsigned w = ent[min(e, CB - 1)], lo = w & ~(CB - 1u), hi = lo + CB;
         int s = 0, upto = 0;                                    // positions of the entries below, and of those up to the token's last
@@ -171,8 +173,9 @@ __global__ __launch_bounds__(1024) void block_plan_kernel(uint16_t *__restrict__
         __syncthreads();
         // the place in the block's lists is a trip to memory; the ranks are written meanwhile
         unsigned long long old = 0;
-        if (t == 0 && (n_long | n_short))
-            old = atomicAdd(&plan_count[blk].runs[turn & 1], (unsigned long long)(unsigned)n_short << 32 | (unsigned)n_long);
+        if (t == 0 && (n_long | n_short | (e1 == 0)))
+            old = atomicAdd(&plan_count[blk].runs[turn & 1],
+                            (unsigned long long)(unsigned)n_short << 32 | (e1 == 0 ? 1u << 16 : 0u) | (unsigned)n_long);
         int rank0 = 0;
 #pragma unroll
         for (int v = 0; v < 16; v++) rank0 += wave_less[v];
@@ -183,8 +186,10 @@ __global__ __launch_bounds__(1024) void block_plan_kernel(uint16_t *__restrict__
                 rk[(size_t)blk * CB + (x & (CB - 1))] = (uint16_t)(rank0 + first_of[ex] + (x >> CB_BITS & 63u));
         }
         if (t == 0) {
-            base_long = (int)(old & 0xffffffffu);
+            base_long = (int)(old & 0xffffu);
             base_short = (int)(old >> 32);
+            if (e1 == 0 && (int)(old >> 16 & 0xffffu) == groups - 1)
+                __hip_atomic_store(&plan_count[blk].turn, turn + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             n_long = n_short = 0;
         }
         __syncthreads();
@@ -197,7 +202,8 @@ __global__ __launch_bounds__(1024) void block_plan_kernel(uint16_t *__restrict__
             const v2u entry = {w >> CB_BITS, (unsigned)(rank0 + s) | (unsigned)(upto - s) << 16};
             tasks[(size_t)blk * CB + slot] = entry;
         }
-    }
+        e1 += 1024 >> sh;
+    } while (e1 < ne);
 }
 
 // acc + x[start] + x[start+1] + ... + x[start+len-1], in that order, from one LDS column.  The column is read in
@@ -284,12 +290,10 @@ __global__ __launch_bounds__(1024) void col_sum_kernel(float *dE, const float *_
         v2u pd[RPL];
     };
     Pre o;
-    unsigned turn;
     auto fetch_runs = [&](Pre &o, int blk) __attribute__((always_inline)) {
         const v2u *tb = tasks + (size_t)blk * CB;
         const PlanCount c = plan_count[blk];
-        turn = c.turn;
-        o.pc = turn & 1 ? c.runs[1] : c.runs[0];
+        o.pc = (c.turn & 1 ? c.runs[0] : c.runs[1]) & ~0xffff0000ull;       // (the plan has moved its turn on)
 #pragma unroll
         for (int i = 0; i < RPL; i++) o.pd[i] = tb[hot ? lane + 64 * i : CB - 1 - (sl + NSL * i)];
     };
@@ -472,7 +476,6 @@ __global__ __launch_bounds__(1024) void col_sum_kernel(float *dE, const float *_
         }
     }
     // what the host looks at before it picks a form for the next call of this shape (one 8-byte store to host memory)
-    if (blockIdx.x == 0 && t == 0) plan_turn = turn + 1;
     if (report && blockIdx.x == 0 && t == 0) *report = scatter_report(runs, N, D, 1);
 }
 

@@ -73,3 +73,31 @@ def test_more_blocks_than_a_launch_takes(br):
     rng = np.random.default_rng(64)
     for N in (64 * BLOCK, 64 * BLOCK + 5, 700, 66 * BLOCK + 4099, 3 * BLOCK):
         scatter(br, np.minimum(rng.zipf(1.2, N) - 1, 9999), 10000, D=1)
+
+
+@pytest.mark.parametrize("recorded", [False, True])
+@pytest.mark.parametrize("nblk", [1, 3])
+def test_a_plan_whose_sums_are_not_launched(br, nblk, recorded):
+    """An error that another call has left behind ends a call between its plan and its sums; the calls after it start from cleared counts."""
+    rng, V = np.random.default_rng(nblk), 5000
+    N = nblk * BLOCK - 3
+    texts = [np.minimum(rng.zipf(1.2, N) - 1, V - 1) for _ in range(3)]
+    for ids in texts:
+        scatter(br, ids, V)
+    Ed, xd, idd = br.DevArray((V, 2)), br.DevArray((2, N)), br.DevArray.from_numpy(texts[0].astype(np.int32))
+    unrecorded = [br.Event(), br.Event()]
+    for times in range(1, 4):
+        if recorded:
+            br.check(br.lib.mi355_graph_begin())
+        for _ in range(times):
+            assert br.lib.mi355_event_elapsed_ms(unrecorded[0].handle, unrecorded[1].handle) < 0
+            assert br.lib.mi355_embed_scatter_add_dev(Ed.ptr, xd.ptr, idd.ptr, V, 2, N, 1) == -1 and "plan" in br.last_error()
+        if recorded:
+            graph = br.lib.mi355_graph_end()
+            assert graph
+            for _ in range(3):
+                br.check(br.lib.mi355_graph_launch(graph))
+                scatter(br, texts[times - 1], V)
+            br.lib.mi355_graph_free(graph)
+        for ids in texts:
+            scatter(br, ids, V)
