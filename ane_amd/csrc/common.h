@@ -39,7 +39,7 @@ struct Mi355Ctx {
                                // with B split ahead (gemm_planes.h): tiles of 96 / 64 x 256, whole rows of A, 96 / 64 of them
     int host_stage;            // drop-ins on host arrays (host_stage.h): 0 = as the machine allows, 1 = without helper threads, 2 = without
                                // pinned memory
-    int host_stage_fail;       // n > 0: their n-th copy back counts as failed
+    int host_stage_fail;       // n > 0: their n-th copy back counts as failed; n < 0: the -n-th chunk of an elementwise call is not launched
     int rms_cluster;           // channel split of the clustered RMSNorm: 0 = per shape, -1 = never, 2/4/8 = forced
     int ce_resident;           // one-launch softmax-CE: 0 = where it pays, 1 = whenever the shape allows, -1 = never
     int rms_cluster_spin;      // its bounded wait in ticks of the 100 MHz clock: 0 = 2 ms, negative = do not wait at all

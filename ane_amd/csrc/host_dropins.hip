@@ -7,7 +7,7 @@
 //   embed_lookup / embed_backward    training/stories_cpu_ops.h:112-131
 //   rope_backward_inplace            training/training_dynamic/cpu_ops.h:168-184
 // Failures print one "mi355_bridge: ..." line and leave arrays that are updated in place untouched, and all others unless it was
-// the copy back that failed, or a later chunk of an elementwise call.
+// the copy back that failed.
 #include "common.h"
 
 #include <emmintrin.h>

@@ -219,7 +219,7 @@ struct Pinned {
     char *host, *dev;                                // its address here and on the device
     size_t bytes;
 };
-Pinned g_pin = {}, g_pin_back = {};                  // the second for results of calls that update arrays
+Pinned g_pin = {}, g_pin_back = {};                  // the second for results of elementwise calls and of calls that update arrays
 hipEvent_t g_sent[MAX_SENDS] = {};
 char *g_log = nullptr;                               // old values of arrays that a call updates
 size_t g_log_bytes = 0;
@@ -337,7 +337,11 @@ public:
     // back is unpacked while later chunks are packed and travel.  chunk(in, out, count): in[i], out[i] are the addresses of
     // part i's values; 0 if it was launched.  Longer arrays than a block holds go in rounds.
     // 1: done.  0: nothing has been done (no pinned memory, or arrays that overlap other than value by value); the call takes
-    // the other way.  -1: failed; the arrays that are inputs and results, of one part or of two, are as before the call.
+    // the other way.  -1: failed; the arrays that are inputs and results, of one part or of two, are as before the call, and so
+    // are those that it only writes unless every chunk was launched and the results of one did not come back.
+    // Of arrays that are only written nothing is kept that could be put back.  Where a call has any, nothing is unpacked before the
+    // last chunk is launched; what that takes from the overlap the threads spend on packing, which is then done sooner.  Longer ones than a block
+    // holds would be written in one round with the chunks of the next still to be launched: those take the other way.
     // us, by way of the device / so: Adam step of [2048][768] 968 / 887, of [3072][1024] 2030 / 1800, SwiGLU backward of [2048][256] 281 /
     // 252, forward 187 / 171, axpby of [768][256] 92 / 82.  Bound by the link, whose 57 GB/s are those of both directions together (two
     // copies of 64 MB, one each way, take as long at once as one after the other), and by 7 us between the kernels of two chunks.
@@ -346,6 +350,7 @@ public:
         int ins = 0;
         size_t updated = 0;
         bool old[MAX];                    // inputs that results are written over
+        bool only = false;                // a result that lies over no input
         for (int i = 0; i < n_; i++) {
             if (p_[i].rows || p_[i].bytes != n * sizeof(float)) return 0;
             ins += in_[i];
@@ -357,11 +362,15 @@ public:
                 old[i] |= a == b;
             }
             if (old[i]) updated += p_[i].bytes;
+            bool over = in_[i];
+            for (int j = 0; j < n_; j++) over |= in_[j] && p_[j].host == p_[i].host;
+            only |= out_[i] && !over;
         }
         Helpers *h = helpers();
         if (!h) return 0;
         const size_t most = PIN_MAX / (sizeof(float) * n_) & ~(size_t)4095;
         const size_t len = std::min(most, (n + 63) & ~(size_t)63), stride = len * sizeof(float);     // values of a round
+        if (only && len < n) return 0;
         if (!pinned(g_pin, stride * n_) || !pinned(g_pin_back, stride * n_)) return 0;
         const bool logged = updated && len < n;
         if (logged) {
@@ -374,6 +383,7 @@ public:
                 }
         }
         copies_ = 0;
+        int chunks = 0;
         for (size_t r0 = 0; r0 < n; r0 += len) {
             const size_t cnt = std::min(len, n - r0);
             // the ends of the chunks: they grow, and shrink again
@@ -386,8 +396,8 @@ public:
                 if (at > cnt || sends + 1 == MAX_SENDS) at = cnt;
                 cut[sends] = at;
             }
-            // the pieces in the order in which they are taken: a chunk's results LAG chunks behind its inputs
-            constexpr int LAG = 2;
+            // the pieces in the order in which they are taken: a chunk's results two chunks behind its inputs, or behind all inputs
+            const int lag = only ? sends : 2;
             int pieces = 0, packed[MAX_SENDS], last[MAX_SENDS], back_from[MAX_SENDS];       // first and last + 1 to pack, first to unpack
             auto add_pieces = [&](int s, bool in) {
                 const size_t from = s ? cut[s - 1] : 0;
@@ -400,15 +410,15 @@ public:
                     }
                 }
             };
-            for (int s = 0; s < sends + LAG; s++) {
+            for (int s = 0; s < sends + lag; s++) {
                 if (s < sends) {
                     packed[s] = pieces;
                     add_pieces(s, true);
                     last[s] = pieces;
                 }
-                if (s >= LAG) {
-                    back_from[s - LAG] = pieces;
-                    add_pieces(s - LAG, false);
+                if (s >= lag) {
+                    back_from[s - lag] = pieces;
+                    add_pieces(s - lag, false);
                 }
             }
             const unsigned long long number = start_pieces(h, pieces, back_from[0]);
@@ -431,13 +441,14 @@ public:
                             in[i] = (float *)(g_pin.dev + i * stride) + from;
                             out[i] = (float *)(g_pin_back.dev + i * stride) + from;
                         }
-                        rc = chunk(in, out, cut[sent] - from);
+                        // (or what g_ctx.host_stage_fail makes of it)
+                        rc = ++chunks == -g_ctx.host_stage_fail ? mi355_fail("chunk %d launch: refused", chunks) : chunk(in, out, cut[sent] - from);
                         if (rc == 0) e = hipEventRecord(g_sent[sent], g_ctx.stream);
                         sent++;
                         idle = false;
                     }
                 }
-                if (e == hipSuccess && come < sent) {
+                if (e == hipSuccess && rc == 0 && come < (only && sent < sends ? 0 : sent)) {
                     const hipError_t q = hipEventQuery(g_sent[come]);
                     if (q == hipErrorNotReady) {
                         (void)hipGetLastError();

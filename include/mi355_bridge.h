@@ -73,7 +73,8 @@ size_t mi355_workspace_size(void);
  * of 10 ns: 0 = 2 ms; -1 = do not wait), "xch_take_nothing" (1: those kernels take no partner's value at
  * all, present or not, so every workgroup goes the way of an expired wait), "host_stage" (the drop-ins on host arrays:
  * 1 = without helper threads, 2 = without pinned memory).  The last three settings are for tests: the results are the same to
- * the bit.  So is "host_stage_fail" (n: the n-th copy back of such a call counts as failed). */
+ * the bit.  So is "host_stage_fail" (n > 0: the n-th copy back of such a call counts as failed; n < 0: the -n-th chunk of an elementwise one is
+ * not launched). */
 int mi355_tune_set(const char *key, int value);
 
 /* How often, since the library was loaded, a workgroup of a kernel whose workgroups hand partial results to one
@@ -473,10 +474,11 @@ int mi355_vocab_scatter_grads_dev(float *full_grad, const float *compact_grad, c
 /* ------------------------------------------------------------------------------------------
  * Host-pointer drop-ins: the reference signatures verbatim (host float* in, host float* out),
  * so a caller swaps the symbol only.  Each call stages through pinned blocks of at most 32 MB (a second one for the results of
- * calls that update arrays), which three threads of the library help to fill and empty, and cached device buffers (H2D, kernel, D2H) and returns when the result is in host
- * memory.  On failure they print one line to stderr and leave the arrays that they update (dw, d_embed, w, m, v, dx of
- * mi355_rope_backward_inplace) untouched, so that the call can be made again; arrays that they only write are untouched unless
- * what failed is a copy back to the host, which may leave a part of the result in them.
+ * elementwise calls and of calls that update arrays), which three threads of the library help to fill and empty, and cached
+ * device buffers (H2D, kernel, D2H; the kernels of elementwise calls work on the pinned blocks, chunk by chunk) and returns when
+ * the result is in host memory.  On failure they print one line to stderr and leave the arrays that they update (dw, d_embed, w, m,
+ * v, dx of mi355_rope_backward_inplace) untouched, so that the call can be made again; arrays that they only write are untouched
+ * unless all was launched and a result did not come back to the host, which may leave a part of it in them.
  * ---------------------------------------------------------------------------------------- */
 /* rmsnorm — training/stories_cpu_ops.h:6 */
 void mi355_rmsnorm(float *out, const float *x, const float *w, int d, int S);

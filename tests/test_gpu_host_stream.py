@@ -91,6 +91,28 @@ def test_results_over_inputs_stay_when_a_chunk_does_not_come_back(br, n, fail):
         assert a.tobytes() == b.tobytes()
 
 
+@pytest.mark.parametrize("fail", [1, 2, 5])
+def test_nothing_is_written_when_a_chunk_is_not_launched(br, fail):
+    """results over inputs and results in arrays of their own alike"""
+    n = 700001
+    a, b, c = H.normal(1000, n), H.normal(1001, n), H.normal(1002, n) ** 2
+    p = lambda x: x.ctypes.data
+    y, z = np.full(n, 3.0, np.float32), np.full(n, 4.0, np.float32)
+    calls = [lambda: br.lib.mi355_axpby(p(y), p(a), p(b), 0.3, n, 0), lambda: br.lib.mi355_axpby(p(y), p(a), None, 0.3, n, 1),
+             lambda: br.lib.mi355_axpby(p(a), p(a), p(b), 0.3, n, 0), lambda: br.lib.mi355_swiglu_fwd(p(y), p(a), p(b), n),
+             lambda: br.lib.mi355_swiglu_bwd(p(y), p(z), p(a), p(b), p(c), n), lambda: br.lib.mi355_swiglu_bwd(p(b), p(z), p(a), p(b), p(c), n),
+             lambda: br.lib.mi355_adam_update(p(a), p(b), p(y), p(c), n, 7, 3e-4, 0.9, 0.95, 1e-8, 0.1)]
+    was = [x.tobytes() for x in (a, b, c, y, z)]
+    try:
+        br.tune("host_stage_fail", -fail)
+        for k, call in enumerate(calls):
+            call()
+            assert "refused" in br.last_error() and [x.tobytes() for x in (a, b, c, y, z)] == was, k
+            br.lib.mi355_axpby(None, None, None, 0.3, n, 0)                       # (another error's text)
+    finally:
+        br.tune("host_stage_fail", 0)
+
+
 def test_weights_that_a_table_holds(br):
     """the table that an update steps is looked up on the device afterwards, with the values that the update left"""
     V, D, S = 300, 64, 50
