@@ -120,10 +120,11 @@ __device__ __forceinline__ v4f ld4_nt(const float *p) {
 
 // A streaming store that is written through to memory (scope bits of an agent store besides the streaming one), so that the
 // XCDs' L2s do not hold it back until the lines are wanted or the kernel ends.  For results of whole 128-byte lines, written
-// in the order of the grid, of FAR_BYTES and more to a tensor; the elementwise ops and the optimizer, with workgroups of one wave
-// each (FAR_THREADS), which come and go one at a time (the converts are as quick in workgroups of 256, the INT8 dequantizer, which
-// reads 4 bytes per lane, quicker: 4.2 M values 5.6 us with st4, 4.7 in waves, 4.1).  Per launch on cold operands, us, workgroups of 256 with st4_nt / this: one tensor in and one out of 48 MB 17.0 /
-// 16.2, of 24 MB 9.7 / 9.0, two in and one out of 24 MB 13.0 / 12.8, of 12 MB 7.7 / 7.3, of 4 MB 3.35 / 3.56, three in and two out of
+// in the order of the grid, of FAR_BYTES and more to a tensor (to a launch of the many-tensor update: MT_FAR in optim.hip); the
+// elementwise ops and the optimizer, with workgroups of one wave each (FAR_THREADS), which come and go one at a time (the converts are
+// as quick in workgroups of 256, the INT8 dequantizer, which reads 4 bytes per lane, quicker: 4.2 M values 5.6 us with st4, 4.7 in
+// waves, 4.1).  Per launch on cold operands, us, workgroups of 256 with st4_nt / this: one tensor in and one out of 48 MB 17.0 / 16.2,
+// of 24 MB 9.7 / 9.0, two in and one out of 24 MB 13.0 / 12.8, of 12 MB 7.7 / 7.3, of 4 MB 3.35 / 3.56, three in and two out of
 // 48 MB 40.4 / 39.5, of 12 MB 11.8 / 11.4, of 4 MB 4.9 / 4.9.  Pieces of lines are written one by one: rotated rows of 197 floats
 // 5.3 -> 6.2.  (Written through, but not marked as streaming, results also stay in the last-level cache, and what reads them next
 // is quicker, two in and one out of 48 MB 24 -> 19; what they push out of it is what the op after that wanted: over a layer no gain.)

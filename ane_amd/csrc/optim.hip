@@ -208,15 +208,20 @@ __global__ __launch_bounds__(OPT_THREADS) void sumsq_partial_mt_kernel(float *__
 
 // Bound by its eight streams (16 B read, 16 B written per parameter with ZERO, at the 5.7 TB/s of a copy).  Norm + clip + update of
 // the 110 M parameters: 650 us in workgroups of 256 with streaming stores (of 1024 705, plain stores 725, g read and cleared with
-// ordinary accesses 698), 620 to 630 a wave to a workgroup, which alone was worth 15 to 20 of it, with stores written through.
-template <bool ZERO>
-__global__ __launch_bounds__(FAR_THREADS) void adam_mt_kernel(MtAdam a, float lr, float b1, float b2, float eps,
+// ordinary accesses 698), 630 a wave to a workgroup with stores written through.
+// THREADS == FAR_THREADS: that form, for launches of MT_FAR parameters and more whose tensors all start on a line.  The update alone, us,
+// in workgroups of 256 / so: 110 M with the embedding 605 / 576, layers of 7.1 M parameters without it, seven 280 / 270, three 117 / 115,
+// one 40.5 / 40.7 (with g kept instead of cleared 35 / 35, 97 / 98, seven 227 / 229), 64 tensors of 64 K 25.4 / 26.5.  Starts
+// 16 bytes into a line, whose lines a wave writes in two pieces: 110 M 703 / 766, two tensors of 8 M 103 / 118, 64 of 64 K 27.7 / 32.
+constexpr size_t MT_FAR = (size_t)16 << 20;
+template <bool ZERO, int THREADS>
+__global__ __launch_bounds__(THREADS) void adam_mt_kernel(MtAdam a, float lr, float b1, float b2, float eps,
                                                               float bc1, float bc2, float scale1,
                                                               const float *__restrict__ scale2_p) {
     const unsigned block = gridDim.x - 1 - blockIdx.x;
     const int ti = mt_owner(a.blk, block);
     const size_t n = a.n[ti], n4 = n / 4;
-    const size_t i = (size_t)(block - a.blk.first[ti]) * FAR_THREADS + threadIdx.x;
+    const size_t i = (size_t)(block - a.blk.first[ti]) * THREADS + threadIdx.x;
     float *__restrict__ w = a.w[ti], *__restrict__ g = a.g[ti];
     float *__restrict__ m = a.m[ti], *__restrict__ v = a.v[ti];
     const float wd = a.wd[ti];
@@ -231,10 +236,10 @@ __global__ __launch_bounds__(FAR_THREADS) void adam_mt_kernel(MtAdam a, float lr
             adam1(x, y, z, gv[j], lr, b1, b2, omb1, omb2, eps, wd, bc1, bc2);
             wv[j] = x; mv[j] = y; vv[j] = z;
         }
-        st16_far(w + 4 * i, wv);
-        st16_far(m + 4 * i, mv);
-        st16_far(v + 4 * i, vv);
-        if (ZERO) { const v4f z4 = {0.f, 0.f, 0.f, 0.f}; st16_far(g + 4 * i, z4); }
+        st4_stream(w + 4 * i, wv, THREADS == FAR_THREADS);
+        st4_stream(m + 4 * i, mv, THREADS == FAR_THREADS);
+        st4_stream(v + 4 * i, vv, THREADS == FAR_THREADS);
+        if (ZERO) { const v4f z4 = {0.f, 0.f, 0.f, 0.f}; st4_stream(g + 4 * i, z4, THREADS == FAR_THREADS); }
     } else if (i == n4) {
         for (size_t k = 4 * n4; k < n; k++) {                    // fewer than four are left
             const float gg = (g[k] * scale1) * scale2;
@@ -304,19 +309,26 @@ MI355_API int mi355_adam_update_multi_dev(float *const *w, float *const *g, floa
     for (int i0 = 0, k = 0; i0 < count; i0 += k) {
         MtAdam a = {};
         unsigned blocks;
-        k = mt_blocks(a.blk, blocks, n + i0, count - i0, FAR_THREADS, FAR_THREADS);
+        k = mt_blocks(a.blk, blocks, n + i0, count - i0, OPT_THREADS, OPT_THREADS);
+        size_t all = 0;
+        uintptr_t starts = 0;
+        for (int i = i0; i < i0 + k; i++) {
+            all += n[i];
+            starts |= (uintptr_t)w[i] | (uintptr_t)g[i] | (uintptr_t)m[i] | (uintptr_t)v[i];
+        }
+        const bool far = all >= MT_FAR && (starts & 127u) == 0;
+        if (far) k = mt_blocks(a.blk, blocks, n + i0, count - i0, FAR_THREADS, FAR_THREADS);
         if (!k) return mi355_fail("adam_update_multi: tensor %d is too large for one launch", i0);
-        const dim3 grid(blocks);
         for (int i = 0; i < k; i++) {
             a.w[i] = w[i0 + i]; a.g[i] = g[i0 + i]; a.m[i] = m[i0 + i]; a.v[i] = v[i0 + i];
             a.n[i] = n[i0 + i]; a.wd[i] = wd[i0 + i];
         }
-        if (zero_grad)
-            hipLaunchKernelGGL((adam_mt_kernel<true>), grid, dim3(FAR_THREADS), 0, g_ctx.stream, a, lr, b1, b2, eps, bc1,
-                               bc2, scale1, scale2_dev);
-        else
-            hipLaunchKernelGGL((adam_mt_kernel<false>), grid, dim3(FAR_THREADS), 0, g_ctx.stream, a, lr, b1, b2, eps, bc1,
-                               bc2, scale1, scale2_dev);
+#define ADAM_MT(ZERO, T)                                                                                             \
+    hipLaunchKernelGGL((adam_mt_kernel<ZERO, T>), dim3(blocks), dim3(T), 0, g_ctx.stream, a, lr, b1, b2, eps, bc1, bc2, scale1, \
+                       scale2_dev)
+        if (far) { if (zero_grad) ADAM_MT(true, FAR_THREADS); else ADAM_MT(false, FAR_THREADS); }
+        else { if (zero_grad) ADAM_MT(true, OPT_THREADS); else ADAM_MT(false, OPT_THREADS); }
+#undef ADAM_MT
         LAUNCH_OK("adam_update_multi");
     }
     return 0;

@@ -72,9 +72,10 @@ def test_bf16_elementwise(br, n, off):
 
 
 @pytest.mark.parametrize("zero", [0, 1])
-@pytest.mark.parametrize("n,off", SIZES)
+@pytest.mark.parametrize("n,off", SIZES + [(8 * LINE - 1, 0), (8 * LINE + 36, 32), (8 * LINE + 11, 8)])
 def test_adam(br, n, off, zero):
-    """one tensor as a whole, one tensor in pieces, and the many-tensor launch (always written through) over the pieces"""
+    """one tensor as a whole, one tensor in pieces, and the many-tensor launch over the pieces, which is written through from 16 M
+    parameters (8 * LINE) on where all pieces start on a line"""
     import ctypes
     rng = np.random.default_rng(n + off)
     host = [rng.standard_normal(n, dtype=np.float32) for _ in range(4)]
