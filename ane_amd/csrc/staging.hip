@@ -140,8 +140,8 @@ __device__ __forceinline__ void store_cols(float *p, const float (&o)[VEC]) {
 // Four columns per lane for fp16 too, whose stores are then whole lines: [16][2048][256] 22.4 us (117 MB: 5.2 TB/s)
 // against 25.2 with eight, [16][2048][250] 24.6 against 26.9 (48.1 with one).  Pair rows are numbered Q heads first, then K heads, then V heads.
 // TABLE: dQ and dK are rotated back.  WAVE: rows are whole waves of columns, so that a wave has one row and what follows of its number
-// (three divisions among it) is scalar.
-template <typename T, int VEC, bool TABLE, bool WAVE, bool FAR>
+// (three divisions among it) is scalar.  ONE: one query head to a KV head, whose K and V rows read only what they use.
+template <typename T, int VEC, bool TABLE, bool ONE, bool WAVE, bool FAR>
 __global__ __launch_bounds__(ST_THREADS) void attn_grads_finish_kernel(
     const T *qf, const T *__restrict__ kf, const T *__restrict__ vf, int S, int hd, int heads, int kv_heads, int ratio, int batch,
     unsigned total, const float *__restrict__ cos_t, const float *__restrict__ sin_t, size_t sq, size_t sk, size_t sv, float *dq,
@@ -166,7 +166,9 @@ __global__ __launch_bounds__(ST_THREADS) void attn_grads_finish_kernel(
 
     // Each kind of row asks for all it will read before it uses any: with the table read where the rotation is, and a query head
     // when the one before it had been added, a K row of two heads made three trips to memory one after the other
-    // ([16][2048][256] with eight KV heads, fp16, 117 MB: 22.8 us, now 21.4 with the scalar rows).
+    // ([16][2048][256] with eight KV heads, fp16, 117 MB: 22.8 us, now 21.4 with the scalar rows).  With one head to a KV head there is no
+    // second to ask for, and V rows do without the table (read like the others: [16][2048][256] from fp16 29.1 us, so 26.2;
+    // [8][768][197] 7.8 and 6.9; from fp32 36.2 and 33.2, 8.7 and 7.7).
     float r0[VEC], r1[VEC], c[VEC], sn[VEC];
     auto ask_table = [&](int i) {
         load_tab<VEC>(c, cos_t + (size_t)i * S + s);
@@ -206,10 +208,8 @@ __global__ __launch_bounds__(ST_THREADS) void attn_grads_finish_kernel(
         const size_t b = bh / (unsigned)kv_heads, kv = bh - b * kv_heads, head = (size_t)hd * S;
         const T *in = (is_k ? kf + b * sk : vf + b * sv) + ((kv * ratio) * hd + 2 * i) * (size_t)S + s;
         out = (is_k ? dk : dv) + ((size_t)bh * hd + 2 * i) * (size_t)S + s;
-        if (TABLE) ask_table(i);                     // (also for V rows, which have no use for it: no branch between the loads)
-        const T *second = in + (ratio > 1 ? head : 0);
-        const Raw a0 = Col::load(in), a1 = Col::load(in + S), b0 = Col::load(second), b1 = Col::load(second + S);
-        __builtin_amdgcn_sched_barrier(0);           // (the compiler would use the first before it asks for the others)
+        const bool rotated = TABLE && is_k;
+        if (ONE ? rotated : TABLE) ask_table(i);     // (for several heads also for V rows: no branch between the loads)
         auto add = [&](const Raw &x0, const Raw &x1) {
 #pragma unroll
             for (int j = 0; j < VEC; j++) {
@@ -219,14 +219,17 @@ __global__ __launch_bounds__(ST_THREADS) void attn_grads_finish_kernel(
         };
 #pragma unroll
         for (int j = 0; j < VEC; j++) r0[j] = r1[j] = 0.f;
-        add(a0, a1);                                 // zero, then += in query-head order (io.h:342-350)
-#pragma unroll
-        for (int j = 0; j < VEC; j++) {              // (selects: behind a branch the second head would be read there)
-            r0[j] = ratio > 1 ? r0[j] + Col::at(b0, j) : r0[j];
-            r1[j] = ratio > 1 ? r1[j] + Col::at(b1, j) : r1[j];
+        const Raw a0 = Col::load(in), a1 = Col::load(in + S);
+        if constexpr (ONE) {
+            add(a0, a1);
+        } else {
+            const Raw b0 = Col::load(in + head), b1 = Col::load(in + head + S);
+            __builtin_amdgcn_sched_barrier(0);       // (the compiler would use the first before it asks for the others)
+            add(a0, a1);                             // zero, then += in query-head order (io.h:342-350)
+            add(b0, b1);
+            for (int r = 2; r < ratio; r++) add(Col::load(in + r * head), Col::load(in + r * head + S));
         }
-        for (int r = 2; r < ratio; r++) add(Col::load(in + r * head), Col::load(in + r * head + S));
-        if (TABLE && is_k) turn();
+        if (rotated) turn();
     }
     store_cols<VEC, FAR>(out, r0);
     store_cols<VEC, FAR>(out + S, r1);
@@ -328,20 +331,29 @@ MI355_API int mi355_attn_grads_finish_dev(float *dq, float *dk, float *dv, const
                                dk + b * kv_full, dv + b * kv_full);
         }
     };
+    // fp32 without the tables is written as quickly or quicker with streaming stores where three heads and more go into one
+    // ([16][2048][256], 16 heads to a KV head, 35 and 27 us, eight heads 29.3 and 26.6; with the tables 25.7 and 25.4, from fp16 21.2 and 21.3)
     const bool far = far_rows(dq, 4 * (size_t)S, 4 * (size_t)S, (size_t)batch * heads * hd) &&
-                     (((uintptr_t)dk | (uintptr_t)dv) & 127u) == 0;
-#define FINISH_AS(T, VEC, ...)                                                                                       \
-    if (cos_dev) launch(attn_grads_finish_kernel<T, VEC, true, __VA_ARGS__>, (const T *)dq_full, (const T *)dk_full, (const T *)dv_full, VEC); \
-    else launch(attn_grads_finish_kernel<T, VEC, false, __VA_ARGS__>, (const T *)dq_full, (const T *)dk_full, (const T *)dv_full, VEC)
-#define FINISH(T)                                                                                                    \
-    if (S % 256 == 0 && far) { FINISH_AS(T, 4, true, true); }                                                        \
-    else if (S % 256 == 0) { FINISH_AS(T, 4, true, false); }                                                         \
-    else if (S % 4 == 0 || (S > 4 && !in_place)) { FINISH_AS(T, 4, false, false); }                                  \
-    else { FINISH_AS(T, 1, false, false); }
-    if (in_f16) { FINISH(_Float16) }
-    else { FINISH(float) }
-#undef FINISH_AS
-#undef FINISH
+                     (((uintptr_t)dk | (uintptr_t)dv) & 127u) == 0 && (in_f16 || cos_dev || ratio <= 2);
+    auto finish = [&](auto vec, auto wave, auto written_through, auto *q, auto *k, auto *v) {
+        typedef typename std::remove_const<typename std::remove_pointer<decltype(q)>::type>::type T;
+        constexpr int VEC = decltype(vec)::value;
+        constexpr bool WAVE = decltype(wave)::value, FAR = decltype(written_through)::value;
+        if (cos_dev && ratio == 1) launch(attn_grads_finish_kernel<T, VEC, true, true, WAVE, FAR>, q, k, v, VEC);
+        else if (cos_dev) launch(attn_grads_finish_kernel<T, VEC, true, false, WAVE, FAR>, q, k, v, VEC);
+        else if (ratio == 1) launch(attn_grads_finish_kernel<T, VEC, false, true, WAVE, FAR>, q, k, v, VEC);
+        else launch(attn_grads_finish_kernel<T, VEC, false, false, WAVE, FAR>, q, k, v, VEC);
+    };
+    auto pick = [&](auto *q, auto *k, auto *v) {
+        const std::integral_constant<int, 4> four;
+        const std::integral_constant<int, 1> one;
+        if (S % 256 == 0 && far) finish(four, std::true_type(), std::true_type(), q, k, v);
+        else if (S % 256 == 0) finish(four, std::true_type(), std::false_type(), q, k, v);
+        else if (S % 4 == 0 || (S > 4 && !in_place)) finish(four, std::false_type(), std::false_type(), q, k, v);
+        else finish(one, std::false_type(), std::false_type(), q, k, v);
+    };
+    if (in_f16) pick((const _Float16 *)dq_full, (const _Float16 *)dk_full, (const _Float16 *)dv_full);
+    else pick((const float *)dq_full, (const float *)dk_full, (const float *)dv_full);
     LAUNCH_OK("attn_grads_finish");
     return 0;
 }

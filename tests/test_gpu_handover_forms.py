@@ -61,3 +61,33 @@ def test_quantize_by_its_own_scale(br, n, top, rounding):
                                               (2, 3, 1, 4, 9)])
 def test_attention_gradients(br, B, heads, kvh, hd, S, in_f16):
     P.test_attn_grads_finish_equals_separate_steps(br, B, heads, kvh, hd, S, in_f16)
+
+
+@pytest.mark.parametrize("rotate", [False, True])
+@pytest.mark.parametrize("in_f16", [0, 1])
+@pytest.mark.parametrize("ratio", [1, 2, 3, 4])
+@pytest.mark.parametrize("S", [256, 260, 9, 3])
+def test_heads_to_a_kv_head(br, S, ratio, in_f16, rotate):
+    """one head and more, with and without the tables, zeros of either sign and infinities among the gradients; dQ, and for one head
+    dK and dV, over their inputs where these are fp32"""
+    B, kvh, hd, theta = 2, 3, 4, 1e4
+    shape = (B, kvh * ratio * hd, S)
+    src = [P.H.normal(1010 + i, shape) for i in range(3)]
+    for k, a in enumerate(src):
+        a.ravel()[k::7] = 0.0
+        a.ravel()[k + 1::7] = -0.0
+        a.ravel()[k + 5::97] = np.inf
+    ins = [O.cvt_f32_f16(a) for a in src] if in_f16 else src
+    cos, sin = br.rope_tables_dev(S, hd, theta) if rotate else (None, None)
+    with np.errstate(invalid="ignore"):
+        want = P._finish_reference(*ins, kvh * ratio, kvh, hd, theta, in_f16, rotate=rotate)
+    for in_place in (False, True)[:1 if in_f16 else 2]:
+        ind = [br.DevArray.from_numpy(a) for a in ins]
+        outs = [br.DevArray(shape)] + [br.DevArray((B, kvh * hd, S)) for _ in range(2)]
+        if in_place:
+            outs = [ind[0]] + (ind[1:] if ratio == 1 else outs[1:])
+        br.check(br.lib.mi355_attn_grads_finish_dev(*[o.ptr for o in outs], *[i.ptr for i in ind], in_f16, 0, 0, 0, kvh * ratio, kvh, hd, S, B, cos, sin))
+        for got, ref in zip(outs, want):
+            got = got.numpy().reshape(ref.shape)
+            bits = got.view(np.uint32) == ref.astype(np.float32).view(np.uint32)
+            assert np.all(bits | (np.isnan(got) & np.isnan(ref)))

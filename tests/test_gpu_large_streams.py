@@ -122,15 +122,16 @@ def test_fp16_rectangles(br, cols, ld, rows, off):
 
 
 @pytest.mark.parametrize("in_f16", [0, 1])
-@pytest.mark.parametrize("S,heads,kvh,off", [(256, 16, 8, 0), (768, 6, 2, 0), (256, 16, 16, 4)])
-def test_attention_gradients(br, in_f16, S, heads, kvh, off):
+@pytest.mark.parametrize("table", [True, False])
+@pytest.mark.parametrize("S,heads,kvh,off", [(256, 16, 8, 0), (768, 6, 2, 0), (256, 16, 16, 4), (256, 12, 12, 0), (256, 16, 4, 0)])
+def test_attention_gradients(br, in_f16, S, heads, kvh, off, table):
     """a batch at once against one sequence after the other; off: results that do not start on a line"""
     hd, rng = 64, np.random.default_rng(S + heads)
     B = -(-LINE // (heads * hd * S)) + 1
     full, kv = heads * hd * S, kvh * hd * S
     t = np.float16 if in_f16 else np.float32
     ins = [br.DevArray.from_numpy(rng.standard_normal(B * full, dtype=np.float32).astype(t)) for _ in range(3)]
-    cos, sin = br.rope_tables_dev(S, hd, 1e4)
+    cos, sin = br.rope_tables_dev(S, hd, 1e4) if table else (None, None)
     got = []
     for step in (B, 1):
         outs = [br.DevArray.from_numpy(np.full(B * k + off, 7, np.float32)) for k in (full, kv, kv)]
