@@ -91,6 +91,39 @@ def test_results_over_inputs_stay_when_a_chunk_does_not_come_back(br, n, fail):
         assert a.tobytes() == b.tobytes()
 
 
+def test_results_over_inputs_stay_whichever_chunk_does_not_come_back(br):
+    """Every chunk of a call of one round and of two, the second round's among them, whose inputs stand where the first one has written
+    its results by then: the old values come from the log."""
+    p = lambda a: a.ctypes.data
+
+    def calls(n):
+        x, y, z, w = H.normal(1020, n), H.normal(1021, n), H.normal(1022, n), H.normal(1023, n) ** 2
+        yield [x], lambda: br.lib.mi355_axpby(p(x), p(x), p(y), 0.3, n, 0)
+        yield [x, z], lambda: br.lib.mi355_swiglu_bwd(p(x), p(z), p(y), p(x), p(z), n)
+        yield [x, y, w], lambda: br.lib.mi355_adam_update(p(x), p(z), p(y), p(w), n, 7, 3e-4, 0.9, 0.95, 1e-8, 0.1)
+
+    chunks = {}
+    try:
+        # values of the round of a pinned block of 32 MB, by the arrays of the calls
+        for n in (None, (3 << 20) + 5):
+            for k, parts in enumerate((3, 5, 4)):
+                m = n or ((32 << 20) // (4 * parts) & ~4095)
+                arrays, call = list(calls(m))[k]
+                was = [a.tobytes() for a in arrays]
+                fail = 0
+                while [a.tobytes() for a in arrays] == was:
+                    fail += 1
+                    assert fail <= 100
+                    br.tune("host_stage_fail", fail)
+                    call()
+                chunks[n, k] = fail - 1
+    finally:
+        br.tune("host_stage_fail", 0)
+    for k in range(3):
+        print("[case] chunks of a round, of two: %d %d" % (chunks[None, k], chunks[(3 << 20) + 5, k]), flush=True)
+        assert 2 < chunks[None, k] <= 32 and chunks[(3 << 20) + 5, k] > chunks[None, k]
+
+
 @pytest.mark.parametrize("fail", [1, 2, 5])
 def test_nothing_is_written_when_a_chunk_is_not_launched(br, fail):
     """results over inputs and results in arrays of their own alike"""
