@@ -28,6 +28,7 @@
 //
 // Reference ops: rmsnorm and rmsnorm_bwd, training/stories_cpu_ops.h:6-53.
 #pragma once
+#include "cluster_words.h"
 #include "common.h"
 #include "tile.h"
 
@@ -201,35 +202,12 @@ __device__ __forceinline__ bool cluster_totals(float (&acc)[NV][VEC], float *lds
     return ok;
 }
 
-// Geometry shared by the kernels: workgroup number -> (slab, strip, member), rows of a member.  It comes in two words, which with the
-// operands of the tile are the arguments that the waves find in their registers when they start (14 dwords of them): what
-// has to be loaded is not waited for until the rows have been asked for.  The number of strips comes with its reciprocal.
-struct ClusterGeo {
-    int blk, first, csplit, member, slab, strip, rows_pm;
-};
-constexpr int CL_NBLK_BITS = 12, CL_SPLIT_BITS = 2, CL_STRIP_BITS = 11, CL_RECIP = 20;
 static_assert(CL_MAX_BLOCKS < 1 << CL_NBLK_BITS && CL_MAX_SPLIT < 1 << (1 << CL_SPLIT_BITS), "the fields hold their values");
 // cluster / strips = cluster * recip >> CL_RECIP: both are below 2^10 (at least two members to a cluster), so that the excess of
 // the reciprocal, below strips / 2^CL_RECIP, times the cluster stays below 1
 static_assert(CL_MAX_BLOCKS / 2 <= 1 << (CL_RECIP / 2) && CL_MAX_BLOCKS / 2 < 1 << CL_STRIP_BITS, "the reciprocal is exact");
-static inline unsigned cluster_word_a(int nblk, int csplit, int rows_pm) {
-    return (unsigned)nblk | (unsigned)__builtin_ctz(csplit) << CL_NBLK_BITS | (unsigned)rows_pm << (CL_NBLK_BITS + CL_SPLIT_BITS);
-}
-static inline unsigned cluster_word_b(int strips) {
-    return (unsigned)strips | (unsigned)(((1 << CL_RECIP) + strips - 1) / strips) << CL_STRIP_BITS;
-}
 __device__ __forceinline__ ClusterGeo cluster_geo(unsigned wa, unsigned wb) {
-    ClusterGeo g;
-    const int shift = wa >> CL_NBLK_BITS & ((1 << CL_SPLIT_BITS) - 1);
-    g.csplit = 1 << shift;
-    g.rows_pm = wa >> (CL_NBLK_BITS + CL_SPLIT_BITS);
-    g.blk = xcd_remap(blockIdx.x, wa & ((1 << CL_NBLK_BITS) - 1));      // the members of a cluster are neighbours on one XCD
-    const unsigned cluster = g.blk >> shift;
-    g.first = cluster << shift;
-    g.member = g.blk - g.first;
-    g.slab = cluster * (wb >> CL_STRIP_BITS) >> CL_RECIP;
-    g.strip = cluster - g.slab * (wb & ((1 << CL_STRIP_BITS) - 1));
-    return g;
+    return cluster_of(wa, wb, xcd_remap(blockIdx.x, cluster_nblk(wa)));      // the members of a cluster are neighbours on one XCD
 }
 
 // FUSE: y = a + alpha*b is formed first (and stored), and the norm is taken of it — the residual add and the
