@@ -1048,11 +1048,12 @@ int ce_run(const char *who, T *dlogits, float *loss_dev, const T *logits, const 
                 // exchange.  us, 64 / 128 members: fp32 [16000][64] 10.1 / 11.1, [32000][64] 13.3 / 12.4, [28673][123] 14.4 / 14.7,
                 // [86946][128] 25.9 / 23.7, [151936][128] 44.7 / 37.9; bfloat16 [32000][64] 14.0 / 13.0, [86946][64] 31.3 / 18.4, [151936][128] 46.6 / 27.0,
                 // [202000][33] 53 / 32.  Three strips, 64 / 80 members (a multiple of 8 keeps a strip's workgroups on their XCD; with
-                // 85 [120000][150] takes 58 for 47): bfloat16 [32000][150] 14.6 / 14.9, [64000][192] 23.3 / 20.4, [151936][150] 49.6 /
-                // 41.6; fp32 [64000][150] 23.5 / 22.4, [151936][192] 52.6 / 53.2, left as it is.
+                // 85 [120000][150] takes 39 for 32): bfloat16 from the step on from which 64 hold rows elsewhere than in registers:
+                // [50000][150] 17.5 / 20.8, [100000][192] 25.8 / 26.1, [130000][192] 28.5 / 31, [140000][192] 33.6 / 32.1, [151936][130] 38.6 / 37.6, [202000][150]
+                // 51 / 45.5; fp32 [64000][150] 24.9 / 28.1, [151936][192] 50.4 / 51.1, left as it is.
                 // (fp32 strips that take three launches keep 64 members where one is forced: the form that the line above compares.)
                 const int many = std::min(cu / strips_r, CR_MAX_SPLIT) & ~7, steps = row_steps();
-                const bool few = sizeof(T) == 2 ? strips_r <= 2 || (strips_r == 3 && steps > 12)
+                const bool few = sizeof(T) == 2 ? strips_r <= 2 || (strips_r == 3 && steps > ST::K_REG)
                                                 : (strips_r == 2 && steps > 8) || (strips_r == 1 && steps <= 14);
                 if (many > csplit && few && steps > 7) csplit = many;
                 const int Rm = rows(), K = row_steps();

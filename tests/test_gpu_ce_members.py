@@ -18,7 +18,7 @@ def br():
 
 
 @pytest.mark.parametrize("V,S,bf16", [(28672, 64, False), (28673, 64, False), (57344, 37, False), (65536, 65, False), (65537, 128, False), (140001, 68, False),
-                                      (28673, 5, True), (65536, 64, True), (65537, 127, True), (213001, 6, True), (49152, 192, True), (49153, 192, True), (50001, 133, True)])
+                                      (28673, 5, True), (65536, 64, True), (65537, 127, True), (213001, 6, True), (49152, 192, True), (49153, 192, True), (50001, 133, True), (131072, 192, True), (131073, 192, True), (140001, 133, True)])
 def test_members(br, V, S, bf16):
     print("[case] ce members V=%d S=%d bf16=%d" % (V, S, bf16), flush=True)
     logits = np.random.default_rng(830).standard_normal((V, S), dtype=np.float32) * np.float32(2.0)
