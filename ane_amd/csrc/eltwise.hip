@@ -515,7 +515,7 @@ __global__ __launch_bounds__(EW_THREADS) void dequant_kernel(float *__restrict__
 #pragma unroll
             for (int j = 0; j < 4; j++) o[j] = (float)(int)(signed char)((a[u] >> (8 * j)) & 0xFF) * scale;
             if (far) st16_far(x + 4 * i, o);
-            else st4(x + 4 * i, o);;
+            else st4(x + 4 * i, o);
         }
     }
 }

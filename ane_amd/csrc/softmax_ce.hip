@@ -353,8 +353,8 @@ __global__ __launch_bounds__(256) void nll_grad_kernel(float *dlogits, const flo
 // with ONE workgroup of 1024 threads per compute unit can read most rows once: a workgroup owns a block of rows of
 // one 64-column strip (256-byte row pieces), keeps its last 16 row steps in registers and the 9 before them in LDS
 // (25 of the 38 steps of the Qwen3 vocabulary; all of them for 32000 rows, and for bfloat16 storage, whose rows take
-// half the space), and reads only the remainder a second time.  Measured at [151936][256]: 66 us against 83 us for
-// the three launches (bfloat16: 49 against 88).  The (max, sum exp) partials of the workgroups of a strip (its members)
+// half the space), and reads only the remainder a second time.  Measured at [151936][256]: 63 us against 84 us for
+// the three launches (bfloat16: 40 against 87).  The (max, sum exp) partials of the workgroups of a strip (its members)
 // are exchanged through tagged 8-byte slots as in the clustered RMSNorm (norm_cluster.h): one relaxed agent-scope
 // atomic {fp32 value, launch tag} per slot, a launch counter per workgroup number, nothing to clear, a bounded
 // wait.  A member whose wait for a partner expires recomputes that partner's partial from memory with the same
@@ -433,7 +433,7 @@ __device__ __forceinline__ LaneCols cr_cols(int strip, int sw, int lc, int S) {
 }
 // The rows of member p: R of them from v_lo, in K steps of CR_RPS rows.  A lane has its row of every step but the last,
 // and of that one if row0 is below `last`.
-// Addresses: row(k, from) of a step k >= 0 is inside the tensor for every lane and every member, also one without rows: a lane without a row
+// Addresses: cr_at() of a step k >= 0 is inside the tensor for every lane and every member, also one without rows: a lane without a row
 // in the last step reads the member's last row, and a step behind the last one is the last again.  So no load of a tile stands
 // behind a condition.  (Behind conditions the compiler waits for each load before the next wherever it moves a value between
 // registers at their end: five of the eight loads of bfloat16 [32000][200] went one after the other, and a member's
@@ -531,7 +531,7 @@ __device__ __forceinline__ void cr_member_partial(const CrGeo<typename ST::T> &g
 #pragma unroll
                 for (int u = 0; u < N; u++) xs[u] = ST::at(t[u], j);
                 online_update<N>(m[j], l[j], xs);
-                // a column at a time: the four in step take 13 registers more than there are ([151936][256] 73 us)
+                // a column at a time: the four in step take 13 registers more than there are ([151936][256] 73 us for 66)
                 asm volatile("" : "+v"(m[j]), "+v"(l[j]));
             }
         };
@@ -723,8 +723,8 @@ __device__ __forceinline__ bool cr_wait_slot(const unsigned long long *sp, unsig
 // MEMBERS: the most a strip may have.  128 take a thread 32 registers more for the slots it fetches, so the variants for them hold
 // eight row steps in registers and the others in LDS.
 // NT: rows are read and written past the caches where their pieces are whole 128-byte lines; where two strips share
-// the lines at their border the caches have to put the pieces together ([151936][200] fp32 102 us past them, 77 with
-// them; [151936][256] 68 and 94).
+// the lines at their border the caches have to put the pieces together ([151936][200] fp32 82 us past them, 75 with
+// them; [151936][256] 62 and 88).
 template <typename ST, int K_REG, int K_LDS, bool NT, int MEMBERS = CR_MAX_SPLIT / 2>
 __global__ __launch_bounds__(CR_THREADS) void ce_resident_kernel(const typename ST::T *__restrict__ logits,
                                                                  const int32_t *__restrict__ targets, unsigned *cnt, int V,
@@ -885,6 +885,7 @@ __global__ __launch_bounds__(CR_THREADS) void ce_resident_kernel(const typename 
         // With the order of the loads: [32000][200] 14.7 -> 12.4 us, fp32 [151936][256] 65 -> 60.4, [24573][256] 16.3 -> 14.6.
         float M[4], f[4];
         int tk[4];                         // the target's row is this lane's row of step k when tk == 64k
+        static_assert(CR_MAX_STEPS <= 64, "a bit for each step");
         unsigned long long hot = 0;        // steps in which a lane of the wave has one
 #pragma unroll
         for (int j = 0; j < 4; j++) {
@@ -1020,21 +1021,21 @@ int ce_run(const char *who, T *dlogits, float *loss_dev, const T *logits, const 
     {
         // The one-launch form: rows of 4 to 1024 columns, split into strips of at most 64, out of place (a member that
         // recomputes a partner's partial reads the partner's logits).  One workgroup per compute unit at most, so that
-        // all of them are resident at once.  Measured against the three launches, us: fp32 [1000][256] 8.6 against 20
-        // (12 with one column per lane), [32000][256] 18.3 against 27, [151936][256] 65.7 against 83, [32000][1000] 71
-        // against 88; bfloat16 [32000][200] 15.3 against 31.6, [151936][256] 49 against 88.
+        // all of them are resident at once.  Measured against the three launches, us: fp32 [1000][256] 9.0 against 12 (with one
+        // column per lane), [32000][256] 16.7 against 25.7, [151936][256] 63 against 84, [32000][1000] 73 against 88; bfloat16
+        // [32000][200] 13.9 against 30.5, [151936][256] 40 against 87.
         // Not for a single strip of fp32 whose members have more than 14 row steps (V > 57344 in 64 members): its 64
-        // workgroups leave three quarters of the chip idle.  [50000][63] 19.0 against 20.0, [65536][63] 20.8 against 20.3,
-        // [90000][64] 28.5 against 23.9, [151936][63] 44.5 against 34.5, [151936][4] 41 against 23.  (bfloat16, whose three
-        // launches convert twice: [151936][63] 44 against 56; two strips: [151936][65] 46 against 50.)  The line is drawn by what 64
-        // members take and left there: with the 128 below one launch would be ahead from it on ([120000][33] 21.5 against 24.4).
+        // workgroups leave three quarters of the chip idle.  The line lies where an earlier one-launch kernel lost ([50000][63]
+        // 19.0 against 20.0, [65536][63] 20.8 against 20.3); with the present one 64 members are ahead beyond it still ([65536][63] 17.2 against
+        // 20.7, [90000][64] 22.1 and 25.1, [151936][63] 37.5 and 37.7) except for few columns ([120000][33] 27.5 and 25.4, [151936][4] 28.2
+        // and 24.8).  (bfloat16, whose three launches convert twice: [151936][63] 28 against 67; two strips: [151936][65] 28 against 74.)
         typedef typename std::conditional<std::is_same<T, float>::value, CrF32, CrBf16>::type ST;
         const int cu = g_ctx.num_cu > 0 ? g_ctx.num_cu : 256;
         const int strips_r = (int)ceil_div((size_t)S, (size_t)CR_W);
         // rows of whole 128-byte lines: strips of 64 columns past the caches; other rows: strips of equal width through them.
-        // Tensors that start within a line have all their strips share lines; past the caches [151936][256] fp32 took
-        // 127 us at an odd element against 103 through them, bfloat16 81 against 58.  From a half line on, whose 64 bytes
-        // are what the memory moves, past the caches is the faster: 93 against 101 at 64 bytes, [90000][256] 44 against 53.
+        // Tensors that start within a line have all their strips share lines; past the caches [151936][256] fp32 takes
+        // 121 us at an odd element against 101 through them, bfloat16 75 against 48.  From a half line on, whose 64 bytes
+        // are what the memory moves, past the caches is the faster: 90 against 97 at 64 bytes, [90000][256] 44 against 53.
         const bool lines = ((size_t)S * sizeof(T)) % 128 == 0 && (((uintptr_t)logits | (uintptr_t)dlogits) & 63) == 0;
         const int sw = lines ? CR_W : 4 * (int)ceil_div((size_t)S, 4 * (size_t)strips_r);
         unsigned char *base = (g_ctx.device >= 0 && g_ctx.device < CE_MAX_DEVICES) ? g_scratch_ptr[g_ctx.device] : nullptr;
@@ -1044,10 +1045,12 @@ int ce_run(const char *who, T *dlogits, float *loss_dev, const T *logits, const 
             const auto row_steps = [&]() { return (int)ceil_div((size_t)rows(), (size_t)CR_RPS); };
             if (csplit >= 2 && csplit * strips_r <= CR_MAX_WG && csplit * strips_r <= cu && row_steps() <= CR_MAX_STEPS &&
                 !(std::is_same<T, float>::value && strips_r == 1 && row_steps() > 14 && g_ctx.ce_resident == 0)) {
-                // Few strips: 64 members each leave compute units idle, and twice as many halve their rows for 1.7 us more of
-                // exchange.  us, 64 / 128 members: fp32 [16000][64] 10.1 / 11.1, [32000][64] 13.3 / 12.4, [28673][123] 14.4 / 14.7,
-                // [86946][128] 25.9 / 23.7, [151936][128] 44.7 / 37.9; bfloat16 [32000][64] 14.0 / 13.0, [86946][64] 31.3 / 18.4, [151936][128] 46.6 / 27.0,
-                // [202000][33] 53 / 32.  Three strips, 64 / 80 members (a multiple of 8 keeps a strip's workgroups on their XCD; with
+                // Few strips: 64 members each leave compute units idle, and twice as many halve their rows for 1 us and more of
+                // exchange.  us, 64 / 128 members: fp32 [28672][64] 11.1 / 12.3, [32000][64] 11.4 / 12.3, [40000][64] 14.0 / 12.7, [28673][123] 14.5 / 15.1,
+                // [33000][123] 15.8 / 15.0, [86946][128] 25.4 / 24.3, [151936][128] 39.4 / 35.7; bfloat16 [24000][64] 10.9 / 11.9, [32000][64] 11.5 / 12.3,
+                // [50000][100] 16.5 / 15.4, [86946][64] 20.9 / 18.3, [151936][128] 33.9 / 26.0, [202000][33] 45 / 31.  (The lines lie at 8 and 9 steps; at 8, the last
+                // that a variant without LDS rows takes, 64 are the quicker by 0.8 where the line is before it.)
+                // Three strips, 64 / 80 members (a multiple of 8 keeps a strip's workgroups on their XCD; with
                 // 85 [120000][150] takes 39 for 32): bfloat16 from the step on from which 64 hold rows elsewhere than in registers:
                 // [50000][150] 17.5 / 20.8, [100000][192] 25.8 / 26.1, [130000][192] 28.5 / 31, [140000][192] 33.6 / 32.1, [151936][130] 38.6 / 37.6, [202000][150]
                 // 51 / 45.5; fp32 [64000][150] 24.9 / 28.1, [151936][192] 50.4 / 51.1, left as it is.
